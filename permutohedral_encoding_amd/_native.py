@@ -111,6 +111,25 @@ def lib():
     return _lib
 
 
+_bridge = None
+
+
+def bridge():
+    """The native path from the module and the optimizers to the library (``csrc/penc_torch.cpp``), loaded once
+    and bound to the library ``lib()`` has loaded; raises if it has not been built."""
+    global _bridge
+    if _bridge is None:
+        lib()
+        try:
+            from . import _penc_torch
+        except ImportError as e:
+            raise RuntimeError("the extension _penc_torch is missing: build it with `python -m permutohedral_encoding_amd.build` "
+                               f"(there is no fallback implementation): {e}")
+        _penc_torch.bind(LIB_PATH)
+        _bridge = _penc_torch
+    return _bridge
+
+
 def _check(status, what):
     if status != 0:
         msg = lib().penc_status_string(status).decode()
@@ -293,6 +312,9 @@ class EncodingFixedParams:
         self.m_scale_factor = torch.from_numpy(sf).to(random_shift_per_level.device)
 
 
+_WRAPPER_CALLS = frozenset(("forward", "backward", "double_backward_from_positions"))
+
+
 class EncodingWrapper:
     """The native encoding object (reference: ``EncodingWrapper``, Encoding.cuh:162-188)."""
 
@@ -308,6 +330,20 @@ class EncodingWrapper:
     @staticmethod
     def create(pos_dim, nr_feat_per_level, fixed_params):
         return EncodingWrapper(pos_dim, nr_feat_per_level, fixed_params)
+
+    def calls_replaced(self):
+        """Whether one of the three calls below is not this class's own (a subclass, an instrumented instance): the
+        module then goes through the autograd functions of ``funcs.py``, which make those calls."""
+        return type(self) is not EncodingWrapper or not _WRAPPER_CALLS.isdisjoint(self.__dict__)
+
+    def encode(self, lattice_values, positions, anneal_window):
+        """-> the encoding (N, F(L+E)) of ``positions``, differentiable as ``funcs.py`` makes it, natively:
+        one call into the extension, whose autograd nodes reach the library without entering the interpreter."""
+        fp = self.fixed_params
+        return (_bridge or bridge()).encode(
+            lattice_values, lattice_values if self.half_table is None else self.gather_table(lattice_values), positions,
+            anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,
+            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES)
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table

@@ -1,4 +1,4 @@
-"""Builds the HIP library in-tree (``permutohedral_encoding_amd/libpenc_hip.so``) with hipcc for gfx950."""
+"""Builds the HIP library (``libpenc_hip.so``, hipcc for gfx950) and its PyTorch bridge (``_penc_torch.so``) in-tree."""
 import os
 import subprocess
 
@@ -9,7 +9,7 @@ LIB_PATH = os.path.join(_HERE, "libpenc_hip.so")
 
 def build_library(force=True, verbose=False):
     """Runs ``make`` in ``csrc/``; with ``force`` the library is rebuilt even if it is up to date."""
-    cmd = ["make", "-C", CSRC]
+    cmd = ["make", "-j4", "-C", CSRC]
     if force:
         cmd.append("-B")
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -1,0 +1,616 @@
+// The path from PermutoEncoding.forward() to the kernels and back through autograd, in native code.
+//
+// What bounds a call on a small batch is not the kernels (4 us for a thousand points) but what the host does
+// around them: argument checks, output and workspace allocation, stream look-up and foreign-function
+// calls cost 20 us per call when they run in the interpreter, and every backward node written in Python
+// has to take the interpreter lock on the autograd thread besides.  Here the module makes one call into
+// this extension; the two differentiable steps are autograd nodes of their own (EncodeNode for the
+// slicing, EncodeBackNode for its gradients, which makes them differentiable once more), so a backward pass never enters
+// the interpreter.  The kernels are reached through the C ABI of include/penc.h, from the library the
+// Python side has loaded (bind()).
+//
+// The nodes follow the pair of autograd functions in funcs.py (reference: src/pytorch_modules/funcs.py), with one
+// difference in form: the result is the (N, F(L+E)) view the module hands out rather than the (L+E, F, N)
+// array behind it (reference: src/pytorch_modules/modules.py:87), so that the permute and reshape need no nodes.
+#include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <Python.h>
+#include <c10/core/DeviceGuard.h>
+#include <dlfcn.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/grad_mode.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/variable.h>
+
+#include <memory>
+#include <mutex>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/penc.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::variable_list;
+
+// ------------------------------------------------------------------------------------------
+// the C ABI
+
+struct Api {
+#define PENC_FN(name) decltype(&penc_##name) name = nullptr
+    PENC_FN(status_string);
+    PENC_FN(extra_levels);
+    PENC_FN(forward);
+    PENC_FN(forward_half);
+    PENC_FN(forward_rowmajor);
+    PENC_FN(forward_rowmajor_workspace_bytes);
+    PENC_FN(scatter_workspace_bytes);
+    PENC_FN(positions_workspace_bytes);
+    PENC_FN(backward);
+    PENC_FN(backward_half);
+    PENC_FN(backward_rowmajor);
+    PENC_FN(backward_sparse);
+    PENC_FN(double_backward_from_positions);
+    PENC_FN(double_backward_from_positions_half);
+    PENC_FN(double_backward_from_positions_rowmajor);
+    PENC_FN(double_backward_from_positions_sparse);
+    PENC_FN(adamw_step);
+    PENC_FN(adamw_step_sparse);
+    PENC_FN(transpose);
+#undef PENC_FN
+} api;
+
+void check(int status, const char* what) {
+    if (status != PENC_OK) TORCH_CHECK(false, what, ": ", api.status_string(status), " (status ", status, ")");
+}
+
+#define PENC_REQUIRE(cond, ...) TORCH_CHECK_VALUE(cond, __VA_ARGS__)
+
+void require_f32_gpu(const Tensor& t, const char* name, int64_t ndim) {
+    PENC_REQUIRE(t.is_cuda(), name, " should be in GPU memory. Please call .cuda() on the tensor");
+    PENC_REQUIRE(t.scalar_type() == at::kFloat, name, " should be of type float");
+    PENC_REQUIRE(t.dim() == ndim, name, " should have ", ndim, " dimensions, however it has sizes ", t.sizes());
+}
+
+void* current_stream(const at::Device& device) {
+    return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream();
+}
+
+const float* data(const Tensor& t) { return static_cast<const float*>(t.const_data_ptr()); }
+float* mutable_data(const Tensor& t) { return t.defined() ? static_cast<float*>(t.mutable_data_ptr()) : nullptr; }
+
+// ------------------------------------------------------------------------------------------
+// what one call of the encoding and its derivatives share
+
+// A reference to a Python object that native code may drop from any thread.
+struct PyRef {
+    explicit PyRef(PyObject* o) : object(o) { Py_XINCREF(object); }
+    PyRef(const PyRef&) = delete;
+    PyRef& operator=(const PyRef&) = delete;
+    ~PyRef() {
+        if (object == nullptr || !Py_IsInitialized()) return;
+        const PyGILState_STATE gil = PyGILState_Ensure();
+        Py_DECREF(object);
+        PyGILState_Release(gil);
+    }
+    PyObject* object;
+};
+
+struct Call {
+    int pos_dim, feat, levels, capacity, extra, concat;
+    float scaling;
+    int table_format;  // 0: fp32, else PENC_TABLE_FP16 / PENC_TABLE_BF16
+    bool rows_output;
+    int64_t n, levels_per_pass, max_workspace;  // the binding's LEVELS_PER_PASS, MAX_WORKSPACE_BYTES (< 0: no cap)
+    Tensor positions;                           // contiguous
+    Tensor table;                               // what the kernels gather from: the parameter or its 16-bit copy
+    Tensor lattice_values;                      // the parameter
+    Tensor scale_factor, shift, window;
+    std::shared_ptr<PyRef> sparse_owner;  // the wrapper that keeps the sparse table gradient; null: dense gradients
+    bool want_table, want_positions;
+
+    int64_t columns() const { return static_cast<int64_t>(feat) * (levels + extra); }
+    at::Device device() const { return positions.device(); }
+};
+
+// An (N, F(L+E)) array in [L+E][F][N] order: the result of the slicing, and the gradient w.r.t. an upstream gradient.
+Tensor level_major_array(const Call& c) {
+    return at::empty_strided({c.n, c.columns()}, {1, c.n}, c.positions.options().dtype(at::kFloat));
+}
+
+Tensor bytes(const Call& c, size_t n) { return at::empty({static_cast<int64_t>(n)}, c.positions.options().dtype(at::kByte)); }
+
+// The sparse table gradient of the call's wrapper (created there by the first gradient call): gradient and map.
+std::pair<Tensor, Tensor> sparse_gradient(const Call& c) {
+    const PyGILState_STATE gil = PyGILState_Ensure();
+    Tensor grad, touched;
+    PyObject* const lv = THPVariable_Wrap(c.lattice_values);
+    PyObject* const sparse = PyObject_CallMethod(c.sparse_owner->object, "sparse_grad_for", "O", lv);
+    if (sparse != nullptr) {
+        PyObject* const g = PyObject_GetAttrString(sparse, "grad");
+        PyObject* const t = PyObject_GetAttrString(sparse, "touched");
+        if (g != nullptr && t != nullptr && THPVariable_Check(g) && THPVariable_Check(t)) {
+            grad = THPVariable_Unpack(g);
+            touched = THPVariable_Unpack(t);
+        }
+        Py_XDECREF(g);
+        Py_XDECREF(t);
+        Py_DECREF(sparse);
+    }
+    Py_XDECREF(lv);
+    if (PyErr_Occurred()) PyErr_Clear();
+    PyGILState_Release(gil);
+    TORCH_CHECK(grad.defined() && touched.defined(), "the sparse table gradient could not be created");
+    return {grad, touched};
+}
+
+// The upstream gradient as the kernels take it: rows of `row_stride` floats, or (row_stride == 0) the [L+E][F][N] array.
+struct Upstream {
+    Tensor values;
+    int64_t row_stride = 0;
+};
+
+Upstream upstream_of(const Call& c, const Tensor& grad) {
+    require_f32_gpu(grad, "grad_sliced_values_monolithic", 2);
+    PENC_REQUIRE(grad.size(0) == c.n && grad.size(1) == c.columns(),
+                 "grad_sliced_values_monolithic should be nr_resolutions x val_dim x nr_positions");
+    PENC_REQUIRE(grad.device() == c.device(), "grad_sliced_values_monolithic must be on the same device as positions");
+    const int64_t s_point = grad.stride(0), s_col = grad.stride(1);
+    if (s_point == 1 && s_col == c.n) return {grad, 0};
+    const auto rows = [&](const Tensor& t) {
+        const int64_t s = t.stride(0);
+        return t.stride(1) == 1 && s >= c.columns() && s % 2 == 0 && (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 7u) == 0 &&
+               s * c.n < (int64_t{1} << 31);
+    };
+    if (rows(grad)) return {grad, s_point};
+    const Tensor dense = grad.contiguous();  // any other layout: rows are what it is brought into (a streaming copy)
+    if (rows(dense)) return {dense, dense.stride(0)};
+    Tensor level_major = level_major_array(c);
+    level_major.copy_(dense);
+    return {level_major, 0};
+}
+
+// Scratch memory of one gradient call, undefined when the library would not use any.  The scatter counts every
+// pair of features as a level.  `copy_bytes`: the level-major copy of a row-major upstream gradient, which the call
+// cannot do without.  A request over the cap, or one the allocator cannot serve, is made again for fewer levels per
+// pass and in the end without the scatter's part (the library then adds directly): _native.scatter_workspace.
+Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t copy_bytes) {
+    if (c.levels_per_pass < 0 && copy_bytes == 0) return {};
+    int64_t pos_bytes = positions ? static_cast<int64_t>(api.positions_workspace_bytes(c.pos_dim, c.n, c.levels)) : 0;
+    const int64_t pair_levels = static_cast<int64_t>(c.levels) * (c.feat / 2);
+    int64_t per_pass = c.levels_per_pass <= 0 ? pair_levels : std::min(c.levels_per_pass, pair_levels);
+    if (!table || c.levels_per_pass < 0) per_pass = 0;
+    while (true) {
+        int64_t want = per_pass > 0 ? static_cast<int64_t>(api.scatter_workspace_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels),
+                                                                                      c.capacity, static_cast<int>(per_pass)))
+                                    : 0;
+        want = std::max(want, pos_bytes) + copy_bytes;
+        if (c.max_workspace < 0 || want <= c.max_workspace) {
+            if (want == 0) return {};
+            try {
+                return bytes(c, static_cast<size_t>(want));
+            } catch (const c10::OutOfMemoryError&) {
+            }
+        }
+        if (per_pass > 1) {
+            per_pass /= 2;
+        } else if (per_pass == 1 || pos_bytes > 0) {
+            per_pass = pos_bytes = 0;
+        } else if (copy_bytes > 0) {
+            return bytes(c, static_cast<size_t>(copy_bytes));  // throws if even that fails
+        } else {
+            return {};
+        }
+    }
+}
+
+void* workspace_of(const Tensor& ws) { return ws.defined() ? ws.mutable_data_ptr() : nullptr; }
+size_t workspace_size(const Tensor& ws) { return ws.defined() ? static_cast<size_t>(ws.numel()) : 0; }
+
+// ------------------------------------------------------------------------------------------
+// the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
+
+Tensor compute_forward(const Call& c) {
+    void* const stream = current_stream(c.device());
+    if (c.rows_output && c.table_format == 0 && c.columns() <= 255) {
+        Tensor rows = at::empty({c.n, c.columns()}, c.positions.options());
+        const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
+        check(api.forward_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
+                                   data(c.shift), data(c.window), mutable_data(rows), c.columns(), c.concat, c.scaling,
+                                   workspace_of(ws), workspace_size(ws), stream),
+              "forward_rowmajor");
+        return rows;
+    }
+    Tensor out = level_major_array(c);
+    if (c.table_format != 0)
+        check(api.forward_half(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                               data(c.scale_factor), data(c.shift), data(c.window), mutable_data(out), c.concat, c.scaling, stream),
+              "forward");
+    else
+        check(api.forward(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
+                          data(c.shift), data(c.window), mutable_data(out), c.concat, c.scaling, stream),
+              "forward");
+    return out;
+}
+
+struct Gradients {
+    Tensor table, positions;  // undefined: not wanted (or, for the table, added into the sparse gradient)
+};
+
+Gradients compute_backward(const Call& c, const Upstream& up, bool want_table, bool want_positions) {
+    Gradients g;
+    if (!want_table && !want_positions) return g;
+    void* const stream = current_stream(c.device());
+    const bool sparse = want_table && c.sparse_owner != nullptr;
+    if (want_positions) g.positions = at::empty({c.n, c.pos_dim}, c.positions.options());
+    if (want_table && !sparse) g.table = at::empty(c.lattice_values.sizes(), c.positions.options());
+    const bool rows = up.row_stride != 0;
+    const int64_t copy_bytes = rows && want_positions ? 4 * static_cast<int64_t>(c.feat) * c.levels * c.n + 512 : 0;
+    const Tensor ws = gradient_workspace(c, want_table, want_positions, copy_bytes);
+    float* const tg = mutable_data(g.table);
+    float* const pg = mutable_data(g.positions);
+    if (sparse) {
+        PENC_REQUIRE(c.table_format == 0, "sparse_table_grad needs an fp32 table");
+        const auto [grad, touched] = sparse_gradient(c);
+        check(api.backward_sparse(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
+                                  data(c.shift), data(c.window), data(up.values), up.row_stride, mutable_data(grad),
+                                  static_cast<uint32_t*>(touched.mutable_data_ptr()), pg, workspace_of(ws), workspace_size(ws), stream),
+              "backward_sparse");
+    } else if (c.table_format != 0) {
+        check(api.backward_half(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                                data(c.scale_factor), data(c.shift), data(c.window), data(up.values), up.row_stride, tg, pg,
+                                workspace_of(ws), workspace_size(ws), stream),
+              "backward");
+    } else if (rows) {
+        check(api.backward_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
+                                    data(c.shift), data(c.window), data(up.values), up.row_stride, tg, pg, workspace_of(ws),
+                                    workspace_size(ws), stream),
+              "backward");
+    } else {
+        check(api.backward(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
+                           data(c.shift), data(c.window), data(up.values), tg, pg, workspace_of(ws), workspace_size(ws), stream),
+              "backward");
+    }
+    return g;
+}
+
+struct SecondOrder {
+    Tensor table, upstream;  // gradients w.r.t. the table (undefined as above) and w.r.t. the upstream gradient
+};
+
+SecondOrder compute_double_backward(const Call& c, const Tensor& double_positions_grad, const Upstream& up, bool want_table) {
+    require_f32_gpu(double_positions_grad, "double_positions_grad", 2);
+    PENC_REQUIRE(double_positions_grad.size(0) == c.n && double_positions_grad.size(1) == c.pos_dim,
+                 "double_positions_grad should be nr_positions x pos_dim");
+    const Tensor dpos = double_positions_grad.contiguous();
+    void* const stream = current_stream(c.device());
+    SecondOrder s;
+    s.upstream = level_major_array(c);
+    const bool sparse = want_table && c.sparse_owner != nullptr;
+    if (want_table && !sparse) s.table = at::empty(c.lattice_values.sizes(), c.positions.options());
+    const Tensor ws = want_table ? gradient_workspace(c, true, false, 0) : Tensor();
+    float* const tg = mutable_data(s.table);
+    float* const gg = mutable_data(s.upstream);
+    if (sparse) {
+        PENC_REQUIRE(c.table_format == 0, "sparse_table_grad needs an fp32 table");
+        const auto [grad, touched] = sparse_gradient(c);
+        check(api.double_backward_from_positions_sparse(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table),
+                                                        data(c.scale_factor), data(c.shift), data(c.window), data(dpos), data(up.values),
+                                                        up.row_stride, mutable_data(grad),
+                                                        static_cast<uint32_t*>(touched.mutable_data_ptr()), gg, c.concat,
+                                                        workspace_of(ws), workspace_size(ws), stream),
+              "double_backward_from_positions_sparse");
+    } else if (c.table_format != 0) {
+        check(api.double_backward_from_positions_half(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions),
+                                                      c.table.const_data_ptr(), c.table_format, data(c.scale_factor), data(c.shift),
+                                                      data(c.window), data(dpos), data(up.values), up.row_stride, tg, gg, c.concat,
+                                                      workspace_of(ws), workspace_size(ws), stream),
+              "double_backward_from_positions");
+    } else if (up.row_stride != 0) {
+        check(api.double_backward_from_positions_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table),
+                                                          data(c.scale_factor), data(c.shift), data(c.window), data(dpos),
+                                                          data(up.values), up.row_stride, tg, gg, c.concat, workspace_of(ws),
+                                                          workspace_size(ws), stream),
+              "double_backward_from_positions");
+    } else {
+        check(api.double_backward_from_positions(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table),
+                                                 data(c.scale_factor), data(c.shift), data(c.window), data(dpos), data(up.values), tg, gg,
+                                                 c.concat, workspace_of(ws), workspace_size(ws), stream),
+              "double_backward_from_positions");
+    }
+    return s;
+}
+
+// ------------------------------------------------------------------------------------------
+// autograd
+
+constexpr const char* kSecondTime =
+    "Trying to backward through the graph a second time (or directly access saved tensors after they have already been freed). "
+    "Specify retain_graph=True if you need to backward through the graph a second time.";
+
+struct EncodeNode;
+
+// Gradient of the gradients of the slicing.  Inputs (in the graph's sense): what EncodeNode produced, i.e. the
+// gradients w.r.t. the table and w.r.t. the positions; only the path through the latter is differentiated (as in the
+// reference, funcs.py:57-72).  Outputs: gradients w.r.t. the upstream gradient, w.r.t. the table, and nothing for the
+// slicing, whose node is named so that a pass through both runs it after this one.
+struct EncodeBackNode : public Node {
+    std::shared_ptr<const Call> call;
+    Upstream upstream;
+    bool released = false;
+
+    std::string name() const override { return "PermutoEncodingBackward2"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        upstream.values.reset();
+        released = true;
+    }
+    variable_list apply(variable_list&& grads) override {
+        variable_list out(3);
+        if (grads.size() < 2 || !grads[1].defined()) return out;
+        Upstream up;
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            TORCH_CHECK(!released, kSecondTime);
+            up = upstream;
+        }
+        const Call& c = *call;
+        at::NoGradGuard no_grad;
+        const c10::DeviceGuard device(c.device());
+        SecondOrder s = compute_double_backward(c, grads[1], up, c.want_table && task_should_compute_output(1));
+        out[0] = std::move(s.upstream);
+        out[1] = std::move(s.table);
+        return out;
+    }
+};
+
+// Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
+// consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
+// table scatter.
+struct EncodeNode : public Node {
+    std::shared_ptr<const Call> call;
+
+    std::string name() const override { return "PermutoEncodingBackward"; }
+    variable_list apply(variable_list&& grads) override {
+        variable_list out(2);
+        if (grads.empty() || !grads[0].defined()) return out;  // reached through a double backward alone
+        const Call& c = *call;
+        const bool want_table = c.want_table && task_should_compute_output(0);
+        const bool want_positions = c.want_positions && task_should_compute_output(1);
+        if (!want_table && !want_positions) return out;
+        const bool differentiable = c10::GradMode::is_enabled();
+        Upstream up;
+        Gradients g;
+        {
+            at::NoGradGuard no_grad;
+            const c10::DeviceGuard device(c.device());
+            up = upstream_of(c, grads[0].detach());
+            g = compute_backward(c, up, want_table, want_positions);
+        }
+        if (differentiable) {
+            auto back = std::shared_ptr<EncodeBackNode>(new EncodeBackNode(), torch::autograd::deleteNode);
+            back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
+            back->add_next_edge(torch::autograd::Edge(shared_from_this(), 0));
+            back->call = call;
+            back->upstream = std::move(up);
+            torch::autograd::set_history(g.table, back);
+            torch::autograd::set_history(g.positions, back);
+        }
+        out[0] = std::move(g.table);
+        out[1] = std::move(g.positions);
+        return out;
+    }
+};
+
+// ------------------------------------------------------------------------------------------
+// Python
+
+const Tensor& tensor_arg(PyObject* o, const char* name) {
+    PENC_REQUIRE(THPVariable_Check(o), name, " must be a torch.Tensor");
+    return THPVariable_Unpack(o);
+}
+
+// Runs `body` with C++ exceptions turned into Python ones.
+template <typename F>
+PyObject* guarded(F&& body) {
+    try {
+        return body();
+    } catch (const c10::ValueError& e) {
+        PyErr_SetString(PyExc_ValueError, e.what_without_backtrace());
+    } catch (const c10::OutOfMemoryError& e) {
+        PyObject* const torch_module = PyImport_ImportModule("torch");
+        PyObject* const type = torch_module != nullptr ? PyObject_GetAttrString(torch_module, "OutOfMemoryError") : nullptr;
+        PyErr_SetString(type != nullptr ? type : PyExc_RuntimeError, e.what_without_backtrace());
+        Py_XDECREF(type);
+        Py_XDECREF(torch_module);
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+// The checks of a call, in the order and with the words of _native.EncodingWrapper (reference: src/Encoding.cu:38-45, 57-66).
+void prepare_call(Call& c, const Tensor& positions, const Tensor& window) {
+    require_f32_gpu(positions, "positions", 2);
+    PENC_REQUIRE(positions.size(0) != 0, "Why do we have 0 points");
+    PENC_REQUIRE(positions.size(1) == c.pos_dim,
+                 "Pos dim for the lattice doesn't correspond with the position of the points. Lattice was initialized with ", c.pos_dim,
+                 " and points have pos dim ", positions.size(1));
+    const auto type = c.table.scalar_type();
+    if (type == at::kHalf || type == at::kBFloat16) {
+        PENC_REQUIRE(c.table.is_cuda(), "lattice_values should be in GPU memory. Please call .cuda() on the tensor");
+        PENC_REQUIRE(c.table.dim() == 3, "lattice_values should have 3 dimensions, however it has sizes ", c.table.sizes());
+        c.table_format = type == at::kHalf ? PENC_TABLE_FP16 : PENC_TABLE_BF16;
+    } else {
+        require_f32_gpu(c.table, "lattice_values", 3);
+        c.table_format = 0;
+    }
+    PENC_REQUIRE(c.table.is_contiguous(), "lattice_values must be contiguous (a slot is loaded at a time)");
+    PENC_REQUIRE(c.table.size(2) == c.feat, "lattice_values should be nr_levels x capacity x ", c.feat);
+    const int64_t levels = c.table.size(0), lim = (int64_t{1} << 31) - 1;
+    PENC_REQUIRE(levels <= lim && c.table.size(1) <= lim, "lattice_values is too large");
+    require_f32_gpu(c.shift, "random_shift_per_level", 2);
+    PENC_REQUIRE(c.shift.size(0) == levels, "Random shift should have the first dimension the same as the nr of resolutions");
+    PENC_REQUIRE(c.shift.size(1) == c.pos_dim, "Random shift should have the second dimension the same as the pos dim");
+    require_f32_gpu(window, "anneal_window", 1);
+    PENC_REQUIRE(window.size(0) == levels, "anneal_window should have the first dimension the same as the nr of resolutions");
+    PENC_REQUIRE(c.scale_factor.dim() == 2 && c.scale_factor.size(0) == levels && c.scale_factor.size(1) == c.pos_dim,
+                 "scale list should have one entry per level");
+    const at::Device dev = positions.device();
+    PENC_REQUIRE(c.table.device() == dev, "lattice_values must be on the same device as positions");
+    PENC_REQUIRE(c.shift.device() == dev, "random_shift_per_level must be on the same device as positions");
+    PENC_REQUIRE(window.device() == dev, "anneal_window must be on the same device as positions");
+    if (c.scale_factor.device() != dev) c.scale_factor = c.scale_factor.to(dev);
+    c.positions = positions.contiguous();
+    c.shift = c.shift.contiguous();
+    c.window = window.contiguous();
+    c.levels = static_cast<int>(levels);
+    c.capacity = static_cast<int>(c.table.size(1));
+    c.n = positions.size(0);
+    c.extra = api.extra_levels(c.pos_dim, c.feat, c.concat);
+}
+
+// encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
+//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None) -> (N, F(L+E))
+PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 14, "encode takes 14 arguments");
+        TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
+        const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
+        const Tensor& positions = tensor_arg(args[2], "positions");
+        auto call = std::make_shared<Call>();
+        Call& c = *call;
+        c.lattice_values = lattice_values;
+        c.table = tensor_arg(args[1], "lattice_values");
+        Tensor window = tensor_arg(args[3], "anneal_window");
+        c.shift = tensor_arg(args[4], "random_shift_per_level");
+        c.scale_factor = tensor_arg(args[5], "scale list");
+        c.pos_dim = static_cast<int>(PyLong_AsLong(args[6]));
+        c.feat = static_cast<int>(PyLong_AsLong(args[7]));
+        c.concat = PyObject_IsTrue(args[8]);
+        c.scaling = static_cast<float>(PyFloat_AsDouble(args[9]));
+        c.rows_output = PyObject_IsTrue(args[11]);
+        c.levels_per_pass = PyLong_AsLongLong(args[12]);
+        c.max_workspace = args[13] == Py_None ? -1 : PyLong_AsLongLong(args[13]);
+        if (PyErr_Occurred()) return nullptr;
+        const bool grad_mode = c10::GradMode::is_enabled();
+        c.want_table = grad_mode && lattice_values.requires_grad();
+        c.want_positions = grad_mode && positions.requires_grad();
+        if (args[10] != Py_None && (c.want_table || c.want_positions)) c.sparse_owner = std::make_shared<PyRef>(args[10]);
+        Tensor out;
+        {
+            NoGil no_gil;
+            at::NoGradGuard no_grad;
+            if (positions.is_cuda()) window = window.to(positions.device(), at::kFloat);
+            prepare_call(c, positions, window);
+            const c10::DeviceGuard device(c.device());
+            out = compute_forward(c);
+        }
+        if (c.want_table || c.want_positions) {
+            auto node = std::shared_ptr<EncodeNode>(new EncodeNode(), torch::autograd::deleteNode);
+            node->set_next_edges(torch::autograd::collect_next_edges(lattice_values, positions));
+            node->call = std::move(call);
+            torch::autograd::set_history(out, node);
+        }
+        return THPVariable_Wrap(std::move(out));
+    });
+}
+
+// adamw_step(param, grad, exp_avg, exp_avg_sq, lr, beta1, beta2, eps, weight_decay, step, skip_zero_gradients)
+// adamw_step_sparse(param, grad, exp_avg, exp_avg_sq, touched, lr, beta1, beta2, eps, weight_decay, step): update, clear, unmark
+// The kernels write through raw pointers: the in-place change is recorded for autograd's version checks and for the
+// 16-bit copy a module keeps of its table.
+PyObject* adamw(PyObject* const* args, Py_ssize_t n_args, bool sparse) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 11, "adamw_step takes 11 arguments");
+        TORCH_CHECK(api.adamw_step != nullptr, "bind() has not been called");
+        const Tensor& p = tensor_arg(args[0], "param");
+        const Tensor& g = tensor_arg(args[1], "grad");
+        const Tensor& m = tensor_arg(args[2], "exp_avg");
+        const Tensor& v = tensor_arg(args[3], "exp_avg_sq");
+        const int first = sparse ? 5 : 4;
+        double x[5];
+        for (int i = 0; i < 5; ++i) x[i] = PyFloat_AsDouble(args[first + i]);
+        const int64_t step = PyLong_AsLongLong(args[first + 5]);
+        if (PyErr_Occurred()) return nullptr;
+        for (const Tensor* t : {&p, &g, &m, &v})
+            TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kFloat && t->is_contiguous() && t->numel() == p.numel() && t->device() == p.device(),
+                        "AdamW: parameter, gradient and moments must be contiguous float32 tensors of one size in the memory of one GPU");
+        const c10::DeviceGuard device(p.device());
+        void* const stream = current_stream(p.device());
+        if (sparse) {
+            const Tensor& touched = tensor_arg(args[4], "touched");
+            TORCH_CHECK(p.dim() == 3 && touched.is_cuda() && touched.scalar_type() == at::kInt, "AdamW: bad table or map");
+            check(api.adamw_step_sparse(mutable_data(p), mutable_data(g), mutable_data(m), mutable_data(v), static_cast<int>(p.size(2)),
+                                        static_cast<int>(p.size(0)), static_cast<int>(p.size(1)),
+                                        static_cast<uint32_t*>(touched.mutable_data_ptr()), x[0], x[1], x[2], x[3], x[4], step, 1, stream),
+                  "adamw_step_sparse");
+        } else {
+            check(api.adamw_step(mutable_data(p), data(g), mutable_data(m), mutable_data(v), p.numel(), x[0], x[1], x[2], x[3], x[4], step,
+                                 PyObject_IsTrue(args[10]), stream),
+                  "adamw_step");
+        }
+        p.unsafeGetTensorImpl()->bump_version();
+        Py_RETURN_NONE;
+    });
+}
+PyObject* py_adamw_step(PyObject*, PyObject* const* args, Py_ssize_t n) { return adamw(args, n, false); }
+PyObject* py_adamw_step_sparse(PyObject*, PyObject* const* args, Py_ssize_t n) { return adamw(args, n, true); }
+
+// bind(path): takes the entry points from the library at `path` (already loaded by the Python side; loading it again is a reference).
+PyObject* py_bind(PyObject*, PyObject* path) {
+    return guarded([&]() -> PyObject* {
+        const char* const name = PyUnicode_AsUTF8(path);
+        if (name == nullptr) return nullptr;
+        void* const lib = dlopen(name, RTLD_NOW | RTLD_LOCAL);
+        TORCH_CHECK(lib != nullptr, "cannot load ", name, ": ", dlerror());
+#define PENC_FN(fn)                                                                \
+    api.fn = reinterpret_cast<decltype(api.fn)>(dlsym(lib, "penc_" #fn));          \
+    TORCH_CHECK(api.fn != nullptr, name, " does not export penc_" #fn)
+        PENC_FN(status_string);
+        PENC_FN(extra_levels);
+        PENC_FN(forward);
+        PENC_FN(forward_half);
+        PENC_FN(forward_rowmajor);
+        PENC_FN(forward_rowmajor_workspace_bytes);
+        PENC_FN(scatter_workspace_bytes);
+        PENC_FN(positions_workspace_bytes);
+        PENC_FN(backward);
+        PENC_FN(backward_half);
+        PENC_FN(backward_rowmajor);
+        PENC_FN(backward_sparse);
+        PENC_FN(double_backward_from_positions);
+        PENC_FN(double_backward_from_positions_half);
+        PENC_FN(double_backward_from_positions_rowmajor);
+        PENC_FN(double_backward_from_positions_sparse);
+        PENC_FN(adamw_step);
+        PENC_FN(adamw_step_sparse);
+        PENC_FN(transpose);
+#undef PENC_FN
+        Py_RETURN_NONE;
+    });
+}
+
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
+    {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"adamw_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step)), METH_FASTCALL, "one AdamW step"},
+    {"adamw_step_sparse", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step_sparse)), METH_FASTCALL,
+     "one AdamW step on the touched slot ranges"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_penc_torch", "native autograd path of the encoding", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__penc_torch() { return PyModule_Create(&module); }

@@ -48,14 +48,10 @@ class AdamW(torch.optim.Optimizer):
                     state["exp_avg"] = torch.zeros_like(p, memory_format=torch.contiguous_format)
                     state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.contiguous_format)
                 state["step"] += 1
-                with torch.cuda.device(p.device):
-                    _native._check(_native.lib().penc_adamw_step(
-                        p.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(), p.numel(),
-                        float(group["lr"]), float(beta1), float(beta2), float(group["eps"]), float(group["weight_decay"]),
-                        int(state["step"]), int(group["skip_zero_gradients"]), _native._stream()), "adamw_step")
-                # the kernel wrote through a raw pointer: record the in-place change for autograd's version
-                # checks and for the half-precision copy the module keeps of its table
-                torch.autograd.graph.increment_version(p)
+                # (records the in-place change for autograd's version checks and the half-precision copy a module keeps)
+                _native.bridge().adamw_step(p, grad, state["exp_avg"], state["exp_avg_sq"], float(group["lr"]), float(beta1),
+                                            float(beta2), float(group["eps"]), float(group["weight_decay"]), int(state["step"]),
+                                            group["skip_zero_gradients"])
         return loss
 
 
@@ -103,11 +99,7 @@ class SparseTableAdamW(torch.optim.Optimizer):
                     state["exp_avg"] = torch.zeros_like(p, memory_format=torch.contiguous_format)
                     state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.contiguous_format)
                 state["step"] += 1
-                with torch.cuda.device(p.device):
-                    _native._check(_native.lib().penc_adamw_step_sparse(
-                        p.data_ptr(), sparse.grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
-                        sparse.nr_feat, sparse.nr_levels, sparse.capacity, sparse.touched.data_ptr(), float(group["lr"]),
-                        float(beta1), float(beta2), float(group["eps"]), float(group["weight_decay"]), int(state["step"]), 1,
-                        _native._stream()), "adamw_step_sparse")
-                torch.autograd.graph.increment_version(p)
+                _native.bridge().adamw_step_sparse(p, sparse.grad, state["exp_avg"], state["exp_avg_sq"], sparse.touched,
+                                                   float(group["lr"]), float(beta1), float(beta2), float(group["eps"]),
+                                                   float(group["weight_decay"]), int(state["step"]))
         return loss
