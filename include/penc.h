@@ -282,6 +282,21 @@ int penc_adamw_step_sparse(float* params, float* grads, float* exp_avg, float* e
                            double weight_decay, int64_t step, int clear, void* stream);
 int penc_clear_touched(float* grads, int nr_feat, int nr_levels, int capacity, uint32_t* touched, void* stream);
 
+/* The two table gradients of a training step on an SDF in one pass: that of a loss on the encoded values, whose
+ * upstream gradient is `grad` (grad_row_stride 0 or a row stride, as in penc_backward_half), plus that of a loss on the position
+ * gradient a first backward has returned (double_positions_grad; `first_grad` [L+E][F][N] is what that backward was
+ * given).  Both add to the slots of the same simplices, so one scatter serves both; the results are those of
+ * penc_backward and penc_double_backward_from_positions summed.  positions_grad (optional) is that of `grad`.
+ * table_format: 0 for an fp32 table, else as in the *_half entry points.  touched: NULL, or the map of
+ * penc_backward_sparse (nothing is cleared then, the sums are added).
+ * Replaces: backward_gpu and double_backward_from_positions_gpu_1 (EncodingGPU.cuh:259-414, 1016-1257) launched for
+ * the two losses one after the other, and autograd's dense sum of what they return. */
+int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                              const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                              const float* random_shift, const float* anneal_window, const float* grad, int64_t grad_row_stride,
+                              const float* double_positions_grad, const float* first_grad, float* lattice_values_grad,
+                              uint32_t* touched, float* positions_grad, void* workspace, size_t workspace_bytes, void* stream);
+
 /* dst[c][r] = src[r][c] for a dense row-major rows x cols matrix with cols <= 255 (2 * levels):
  * turns the row-major upstream gradient (N, 2(L+E)) into the grad_sliced_values layout
  * [L+E][2][N] at streaming speed.

@@ -180,6 +180,8 @@ constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_b
     return pos_dim <= 4 || (pos_dim == 5 && !second_order) ? 6 : 4;
 }
 
+constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins) { return pos_dim <= 3 && !wide_bins ? 6 : 4; }
+
 // kRowMajor: the upstream gradient is read as rows grad[n][2*level + feature] of `grad_row_stride`
 // floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
 // all levels of a group of points back to back, so the rows mostly come from L2 (measured: fetched
@@ -187,7 +189,7 @@ constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_b
 // With `grad_level_major` the kernel also leaves the values it read in [level][feature][n] order
 // (for the position-gradient kernel, which gathers level by level and wants its upstream gradient
 // coalesced): the layout change rides on reads this kernel makes anyway.
-// kSecondOrder: the table-gradient half of the double backward (EncodingGPU.cuh:1016-1257): the
+// Second order: the table-gradient half of the double backward (EncodingGPU.cuh:1016-1257): the
 // vertex weights are the derivatives of the barycentric weights along `double_pos_grad` instead of
 // the barycentric weights themselves; everything else is the same scatter.
 // feat_pairs: with four or eight features per level the pairs (0,1), (2,3), ... are scattered like levels that
@@ -197,15 +199,21 @@ constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_b
 // kWideBins: the bins span more than kBinSlots slots (tables above 2^22 slots).  A parameter of the kernel
 // rather than a value read from its arguments, because with the bin width a variable the usual instances
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
-template <int D, bool kRowMajor, bool kSecondOrder, bool kWideBins>
-__global__ void __launch_bounds__(kScatterBlock, scatter_waves_per_simd(D, kSecondOrder, kWideBins))
-backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
-                      uint32_t capacity, uint32_t cap_mask,
-                      const float* __restrict__ positions, const float* __restrict__ scale_factor,
-                      const float* __restrict__ random_shift, const float* __restrict__ window,
-                      const float* __restrict__ grad_sliced, int64_t grad_row_stride,
-                      const float* __restrict__ double_pos_grad, float* __restrict__ table_grad,
-                      float* __restrict__ grad_level_major, BinTarget pass_bins) {
+// kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
+// a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
+// gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
+// reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
+enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
+template <int D, bool kRowMajor, int kOrder, bool kWideBins>
+__device__ __forceinline__ void
+scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
+                        uint32_t capacity, uint32_t cap_mask,
+                        const float* __restrict__ positions, const float* __restrict__ scale_factor,
+                        const float* __restrict__ random_shift, const float* __restrict__ window,
+                        const float* __restrict__ grad_sliced, int64_t grad_row_stride,
+                        const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
+                        float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
+    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
     __shared__ ScatterStateT<stage_chunk(D)> state;
     // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
     // workgroup of a die takes level j % levels of one group of points: a die works through all
@@ -230,7 +238,7 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
     // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets.
     const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);
     const float* const group_positions = positions + group_base * D;
-    const float* const group_q = kSecondOrder ? double_pos_grad + group_base * D : nullptr;
+    const float* const group_q = kNeedsQ ? double_pos_grad + group_base * D : nullptr;
     const float* const group_grad0 =
         kRowMajor ? grad_sliced + group_base * grad_row_stride + 2 * pair_level
                   : grad_sliced + (static_cast<size_t>(pair_level) * 2) * n_points + group_base;
@@ -245,6 +253,8 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
             g1 = group_grad1[i];
         }
     };
+    const float* const group_second0 = kBoth ? second_grad + (static_cast<size_t>(pair_level) * 2) * n_points + group_base : nullptr;
+    const float* const group_second1 = group_second0 + n_points;
     const auto load_group_point = [&](const float* base, uint32_t i) {
         fvec<D> v;
         static_for<D>(PENC_BODY(k) {
@@ -260,9 +270,14 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
     uint32_t nn = point_of(0);
     fvec<D> pos = load_group_point(group_positions, nn);
     fvec<D> q = 0.0f;
-    if constexpr (kSecondOrder) q = load_group_point(group_q, nn);
+    if constexpr (kNeedsQ) q = load_group_point(group_q, nn);
     float g0, g1;
     load_grad(nn, g0, g1);
+    float s0 = 0.0f, s1 = 0.0f;
+    if constexpr (kBoth) {
+        s0 = group_second0[nn];
+        s1 = group_second1[nn];
+    }
     int mode = kModeCache;
     uint32_t id_bits = 0;
     for (int t = 0; t < tiles_per_group; ++t) {
@@ -272,9 +287,14 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
         const uint32_t nn_next = point_of(t + 1);
         const fvec<D> pos_next = load_group_point(group_positions, nn_next);
         fvec<D> q_next = 0.0f;
-        if constexpr (kSecondOrder) q_next = load_group_point(group_q, nn_next);
+        if constexpr (kNeedsQ) q_next = load_group_point(group_q, nn_next);
         float g0_next, g1_next;
         load_grad(nn_next, g0_next, g1_next);
+        float s0_next = 0.0f, s1_next = 0.0f;
+        if constexpr (kBoth) {
+            s0_next = group_second0[nn_next];
+            s1_next = group_second1[nn_next];
+        }
         if constexpr (kRowMajor) {
             if (grad_level_major != nullptr && active) {
                 float* out = grad_level_major + (static_cast<size_t>(pair_level) * 2) * n_points + tile_base + threadIdx.x;
@@ -284,7 +304,8 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
         }
         const Located<D> s = locate<D>(pos, random_shift + level * D, scale_factor + level * D);
         uvec<D + 1> h;
-        fvec<D + 1> w;  // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
+        fvec<D + 1> w;   // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
+        fvec<D + 1> w2;  // kBoth: the latter
         bool via_lds = false;
         if constexpr (D > kWorkgroupSortMaxDim) {
             // Once the workgroup streams with every wave sorting on its own (stream_tile_wave), a wave's staging
@@ -298,7 +319,13 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
             static_assert((D + 1) * 64 <= kSliceCells, "a wave's staging slice holds a column of D+1 cells per lane");
             uint2* const column = reinterpret_cast<uint2*>(state.val) + (threadIdx.x >> 6) * kSliceCells + (threadIdx.x & 63);
             fvec<D + 1> sorted;
-            if constexpr (kSecondOrder) {
+            if constexpr (kBoth) {
+                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
+                w = barycentric_of_sorted<D>(sorted) * w_level;
+                wave_lds_fence();
+                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
+                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
+            } else if constexpr (kOrder == kSecondOrder) {
                 sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
                 w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
             } else {
@@ -308,7 +335,10 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
             wave_lds_fence();  // the slice is staging space again from here on
         } else {
             h = vertex_hashes<D>(s.rank, s.hash0);
-            if constexpr (kSecondOrder) {
+            if constexpr (kBoth) {
+                w = barycentric<D>(s.rank, s.delta) * w_level;
+                w2 = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
+            } else if constexpr (kOrder == kSecondOrder) {
                 w = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
             } else {
                 w = barycentric<D>(s.rank, s.delta) * w_level;
@@ -335,17 +365,45 @@ backward_table_kernel(int n_points, int first_level, uint32_t n_pass_levels, uin
             const bool next_active = tile_base + kScatterBlock + threadIdx.x < n_points && tiles_per_group > 1;
             mode = scatter_mode_decide<D>(state, bins, active, slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
         }
-        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t),
-                                              mode, id_bits, slot, w * g0, w * g1);  // g_f * (b_r * w_level), :405-410
+        fvec<D + 1> a0 = w * g0, a1 = w * g1;  // g_f * (b_r * w_level), :405-410
+        if constexpr (kBoth) {
+            a0 += w2 * s0;
+            a1 += w2 * s1;
+        }
+        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1);
         // the first tile finds the lines its own look-up has claimed: no evidence of reuse
         if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
         pos = pos_next;
         q = q_next;
         g0 = g0_next;
         g1 = g1_next;
+        s0 = s0_next;
+        s1 = s1_next;
     }
     scatter_end(state, level_grad, bins, group, mode, id_bits);
 }
+
+#define PENC_TABLE_PARAMETERS                                                                                                          \
+    int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group, uint32_t capacity, \
+        uint32_t cap_mask, const float *__restrict__ positions, const float *__restrict__ scale_factor,                                \
+        const float *__restrict__ random_shift, const float *__restrict__ window, const float *__restrict__ grad_sliced,               \
+        int64_t grad_row_stride, const float *__restrict__ double_pos_grad, const float *__restrict__ second_grad,                     \
+        float *__restrict__ table_grad, float *__restrict__ grad_level_major, BinTarget pass_bins
+#define PENC_TABLE_ARGUMENTS                                                                                                        \
+    n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
+        random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
+template <int D, bool kRowMajor, bool kSecond, bool kWideBins>
+__global__ void __launch_bounds__(kScatterBlock, scatter_waves_per_simd(D, kSecond, kWideBins))
+backward_table_kernel(PENC_TABLE_PARAMETERS) {
+    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins>(PENC_TABLE_ARGUMENTS);
+}
+template <int D, bool kRowMajor, bool kWideBins>
+__global__ void __launch_bounds__(kScatterBlock, both_orders_waves_per_simd(D, kWideBins))
+backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
+    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins>(PENC_TABLE_ARGUMENTS);
+}
+#undef PENC_TABLE_PARAMETERS
+#undef PENC_TABLE_ARGUMENTS
 
 // ------------------------------------------------------------------------------------------
 // backward w.r.t. positions (EncodingGPU.cuh:530-769)
@@ -981,6 +1039,14 @@ inline uint32_t dies_of_current_device() {
 
 using namespace penc;
 
+// The part of a table gradient that comes through the position gradient: nothing, the whole of it (double_pos_grad alone;
+// `grad` is then the upstream gradient of the first backward), or one of two summands (with `upstream`, [L][F][N]: the upstream
+// gradient of the first backward; `grad` is that of the encoded values).
+struct SecondGradient {
+    const float* double_pos_grad = nullptr;
+    const float* upstream = nullptr;
+};
+
 // The table gradient of penc_backward / penc_backward_table_rowmajor: clear, scatter, reduce the
 // bins, in as many passes over the levels as the workspace asks for.  grad_row_stride == 0 means
 // the [level][feature][n] layout, otherwise the gradient is rows of that many floats.  With
@@ -991,7 +1057,7 @@ using namespace penc;
 // that hold anything; it takes the place of the workspace's flags of direct adds.
 static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
                           const float* scale_factor, const float* random_shift, const float* anneal_window,
-                          const float* grad, int64_t grad_row_stride, const float* double_pos_grad,
+                          const float* grad, int64_t grad_row_stride, const SecondGradient& second,
                           float* lattice_values_grad, float* grad_level_major, void* workspace, size_t workspace_bytes,
                           hipStream_t st, uint32_t* touched = nullptr) {
     const int n = static_cast<int>(nr_positions);
@@ -1021,30 +1087,39 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
         const dim3 grid(padded_groups * static_cast<unsigned>(count));
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
-#define PENC_LAUNCH_TABLE_(ROW_MAJOR, SECOND_ORDER, WIDE)                                                                  \
-    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((backward_table_kernel<DD, ROW_MAJOR, SECOND_ORDER, WIDE>), grid,            \
-                                                dim3(kScatterBlock), 0, st, n, first, static_cast<uint32_t>(count),          \
-                                                feat_pairs, dies, tiles_per_group, cap, mask, positions, scale_factor,       \
-                                                random_shift, anneal_window, grad, grad_row_stride, double_pos_grad,         \
-                                                lattice_values_grad, grad_level_major, plan.target))
-#define PENC_LAUNCH_TABLE(ROW_MAJOR, SECOND_ORDER)       \
-    if (wide_bins) {                                     \
-        PENC_LAUNCH_TABLE_(ROW_MAJOR, SECOND_ORDER, true);  \
-    } else {                                             \
-        PENC_LAUNCH_TABLE_(ROW_MAJOR, SECOND_ORDER, false); \
+#define PENC_LAUNCH_TABLE(...)                                                                                             \
+    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(kScatterBlock), 0, st, n, first,                    \
+                                                static_cast<uint32_t>(count), feat_pairs, dies, tiles_per_group, cap, mask,  \
+                                                positions, scale_factor, random_shift, anneal_window, grad, grad_row_stride, \
+                                                second.double_pos_grad, second.upstream, lattice_values_grad,                \
+                                                grad_level_major, plan.target))
+#define PENC_LAUNCH_TABLE_WIDTH(KERNEL, ...)                \
+    if (wide_bins) {                                        \
+        PENC_LAUNCH_TABLE(KERNEL<DD, __VA_ARGS__, true>);   \
+    } else {                                                \
+        PENC_LAUNCH_TABLE(KERNEL<DD, __VA_ARGS__, false>);  \
     }
         const bool wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
-        if (double_pos_grad != nullptr && grad_row_stride != 0) {
-            PENC_LAUNCH_TABLE(true, true);
-        } else if (double_pos_grad != nullptr) {
-            PENC_LAUNCH_TABLE(false, true);
-        } else if (grad_row_stride != 0) {
-            PENC_LAUNCH_TABLE(true, false);
+        const bool rows = grad_row_stride != 0;
+        if (second.upstream != nullptr) {
+            if (rows) {
+                PENC_LAUNCH_TABLE_WIDTH(backward_table_both_kernel, true);
+            } else {
+                PENC_LAUNCH_TABLE_WIDTH(backward_table_both_kernel, false);
+            }
+        } else if (second.double_pos_grad != nullptr) {
+            if (rows) {
+                PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, true, true);
+            } else {
+                PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, false, true);
+            }
+        } else if (rows) {
+            PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, true, false);
         } else {
-            PENC_LAUNCH_TABLE(false, false);
+            PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, false, false);
         }
+#undef PENC_LAUNCH_TABLE_WIDTH
 #undef PENC_LAUNCH_TABLE
-#undef PENC_LAUNCH_TABLE_
         if (int rc = check_launch()) return rc;
         if (plan.enabled)
             if (int rc = reduce_bins(plan, anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
@@ -1109,7 +1184,8 @@ static int backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
                          const float* positions, const TableRef& table, const float* scale_factor,
                          const float* random_shift, const float* anneal_window,
                          const float* grad_sliced_values, float* lattice_values_grad, float* positions_grad,
-                         void* workspace, size_t workspace_bytes, void* stream, uint32_t* touched = nullptr) {
+                         void* workspace, size_t workspace_bytes, void* stream, uint32_t* touched = nullptr,
+                         const SecondGradient& second = {}) {
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0)) return rc;
     if (!positions || !scale_factor || !random_shift || !anneal_window || !grad_sliced_values)
         return PENC_ERR_NULL_POINTER;
@@ -1119,7 +1195,7 @@ static int backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (lattice_values_grad)
         if (int rc = table_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, scale_factor, random_shift,
-                                    anneal_window, grad_sliced_values, 0, nullptr, lattice_values_grad, nullptr, workspace,
+                                    anneal_window, grad_sliced_values, 0, second, lattice_values_grad, nullptr, workspace,
                                     workspace_bytes, st, touched))
             return rc;
     if (positions_grad)
@@ -1310,7 +1386,8 @@ static int backward_rowmajor_impl(int pos_dim, int nr_feat, int64_t nr_positions
                                   const float* positions, const TableRef& table, const float* scale_factor,
                                   const float* random_shift, const float* anneal_window, const float* grad_rows,
                                   int64_t grad_row_stride, float* lattice_values_grad, float* positions_grad,
-                                  void* workspace, size_t workspace_bytes, void* stream, uint32_t* touched = nullptr) {
+                                  void* workspace, size_t workspace_bytes, void* stream, uint32_t* touched = nullptr,
+                                  const SecondGradient& second = {}) {
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0)) return rc;
     if (!positions || !scale_factor || !random_shift || !anneal_window) return PENC_ERR_NULL_POINTER;
     if (!lattice_values_grad && !positions_grad) return PENC_ERR_NULL_POINTER;
@@ -1320,7 +1397,7 @@ static int backward_rowmajor_impl(int pos_dim, int nr_feat, int64_t nr_positions
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!positions_grad)
         return table_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, scale_factor, random_shift,
-                              anneal_window, grad_rows, grad_row_stride, nullptr, lattice_values_grad, nullptr, workspace,
+                              anneal_window, grad_rows, grad_row_stride, second, lattice_values_grad, nullptr, workspace,
                               workspace_bytes, st, touched);
     // The position gradient gathers level by level and reads its upstream gradient as [level][feature][n]:
     // that copy lives at the front of the workspace; the rest serves the scatter and then the partial sums.
@@ -1335,7 +1412,7 @@ static int backward_rowmajor_impl(int pos_dim, int nr_feat, int64_t nr_positions
     if (lattice_values_grad) {
         // the scattering kernel reads every (point, level) pair of the rows anyway and leaves the copy behind
         if (int rc = table_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, scale_factor, random_shift,
-                                    anneal_window, grad_rows, grad_row_stride, nullptr, lattice_values_grad, level_major,
+                                    anneal_window, grad_rows, grad_row_stride, second, lattice_values_grad, level_major,
                                     rest, rest_bytes, st, touched))
             return rc;
     } else {
@@ -1408,7 +1485,7 @@ static int double_backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, 
     }
     if (!lattice_values_grad) return PENC_OK;
     return table_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, scale_factor, random_shift, anneal_window,
-                          grad, grad_row_stride, double_positions_grad, lattice_values_grad, nullptr, workspace,
+                          grad, grad_row_stride, SecondGradient{double_positions_grad, nullptr}, lattice_values_grad, nullptr, workspace,
                           workspace_bytes, st, touched);
 }
 
@@ -1456,6 +1533,24 @@ int penc_double_backward_from_positions_half(int pos_dim, int nr_feat, int64_t n
                                 TableRef{lattice_values_half, table_format}, scale_factor, random_shift, anneal_window,
                                 double_positions_grad, grad, grad_row_stride, lattice_values_grad, grad_grad_sliced_values,
                                 concat_points, workspace, workspace_bytes, stream);
+}
+
+int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                              const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                              const float* random_shift, const float* anneal_window, const float* grad, int64_t grad_row_stride,
+                              const float* double_positions_grad, const float* first_grad, float* lattice_values_grad,
+                              uint32_t* touched, float* positions_grad, void* workspace, size_t workspace_bytes, void* stream) {
+    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!lattice_values_grad || !double_positions_grad || !first_grad) return PENC_ERR_NULL_POINTER;
+    const TableRef table{lattice_values, table_format};
+    const SecondGradient second{double_positions_grad, first_grad};
+    if (grad_row_stride != 0)
+        return backward_rowmajor_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
+                                      random_shift, anneal_window, grad, grad_row_stride, lattice_values_grad, positions_grad,
+                                      workspace, workspace_bytes, stream, touched, second);
+    return backward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
+                         anneal_window, grad, lattice_values_grad, positions_grad, workspace, workspace_bytes, stream, touched,
+                         second);
 }
 
 // The scalars of one AdamW step as torch.optim.AdamW forms them (in double), rounded once for the kernel.

@@ -18,6 +18,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <dlfcn.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -54,6 +55,7 @@ struct Api {
     PENC_FN(backward_half);
     PENC_FN(backward_rowmajor);
     PENC_FN(backward_sparse);
+    PENC_FN(backward_both_orders);
     PENC_FN(double_backward_from_positions);
     PENC_FN(double_backward_from_positions_half);
     PENC_FN(double_backward_from_positions_rowmajor);
@@ -152,6 +154,14 @@ std::pair<Tensor, Tensor> sparse_gradient(const Call& c) {
 struct Upstream {
     Tensor values;
     int64_t row_stride = 0;
+    int64_t version = -1;  // of the values when they were kept for a later pass
+
+    void keep() { version = values.is_inference() ? -1 : static_cast<int64_t>(values._version()); }
+    void check_unmodified() const {
+        TORCH_CHECK(version < 0 || version == static_cast<int64_t>(values._version()),
+                    "one of the variables needed for gradient computation has been modified by an inplace operation: the upstream gradient "
+                    "of the encoding is at version ", values._version(), "; expected version ", version, " instead");
+    }
 };
 
 Upstream upstream_of(const Call& c, const Tensor& grad) {
@@ -241,11 +251,19 @@ struct Gradients {
     Tensor table, positions;  // undefined: not wanted (or, for the table, added into the sparse gradient)
 };
 
-Gradients compute_backward(const Call& c, const Upstream& up, bool want_table, bool want_positions) {
+// The table gradient that comes through a position gradient, handed on by the node that met it (see EncodeNode).
+struct SecondOrderTerm {
+    int task = -1;                  // the graph task it belongs to
+    Tensor double_positions_grad;   // contiguous
+    Upstream upstream;              // level-major
+};
+
+Gradients compute_backward(const Call& c, const Upstream& up, bool want_table, bool want_positions, const SecondOrderTerm* second = nullptr) {
     Gradients g;
     if (!want_table && !want_positions) return g;
     void* const stream = current_stream(c.device());
     const bool sparse = want_table && c.sparse_owner != nullptr;
+    PENC_REQUIRE(!sparse || c.table_format == 0, "sparse_table_grad needs an fp32 table");
     if (want_positions) g.positions = at::empty({c.n, c.pos_dim}, c.positions.options());
     if (want_table && !sparse) g.table = at::empty(c.lattice_values.sizes(), c.positions.options());
     const bool rows = up.row_stride != 0;
@@ -253,8 +271,17 @@ Gradients compute_backward(const Call& c, const Upstream& up, bool want_table, b
     const Tensor ws = gradient_workspace(c, want_table, want_positions, copy_bytes);
     float* const tg = mutable_data(g.table);
     float* const pg = mutable_data(g.positions);
-    if (sparse) {
-        PENC_REQUIRE(c.table_format == 0, "sparse_table_grad needs an fp32 table");
+    if (want_table && second != nullptr) {
+        std::pair<Tensor, Tensor> kept;
+        if (sparse) kept = sparse_gradient(c);
+        check(api.backward_both_orders(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(),
+                                       c.table_format, data(c.scale_factor), data(c.shift), data(c.window), data(up.values), up.row_stride,
+                                       data(second->double_positions_grad), data(second->upstream.values),
+                                       sparse ? mutable_data(kept.first) : tg,
+                                       sparse ? static_cast<uint32_t*>(kept.second.mutable_data_ptr()) : nullptr, pg, workspace_of(ws),
+                                       workspace_size(ws), stream),
+              "backward_both_orders");
+    } else if (sparse) {
         const auto [grad, touched] = sparse_gradient(c);
         check(api.backward_sparse(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
                                   data(c.shift), data(c.window), data(up.values), up.row_stride, mutable_data(grad),
@@ -282,14 +309,15 @@ struct SecondOrder {
     Tensor table, upstream;  // gradients w.r.t. the table (undefined as above) and w.r.t. the upstream gradient
 };
 
-SecondOrder compute_double_backward(const Call& c, const Tensor& double_positions_grad, const Upstream& up, bool want_table) {
+SecondOrder compute_double_backward(const Call& c, const Tensor& double_positions_grad, const Upstream& up, bool want_table,
+                                    bool want_upstream) {
     require_f32_gpu(double_positions_grad, "double_positions_grad", 2);
     PENC_REQUIRE(double_positions_grad.size(0) == c.n && double_positions_grad.size(1) == c.pos_dim,
                  "double_positions_grad should be nr_positions x pos_dim");
     const Tensor dpos = double_positions_grad.contiguous();
     void* const stream = current_stream(c.device());
     SecondOrder s;
-    s.upstream = level_major_array(c);
+    if (want_upstream) s.upstream = level_major_array(c);
     const bool sparse = want_table && c.sparse_owner != nullptr;
     if (want_table && !sparse) s.table = at::empty(c.lattice_values.sizes(), c.positions.options());
     const Tensor ws = want_table ? gradient_workspace(c, true, false, 0) : Tensor();
@@ -332,7 +360,34 @@ constexpr const char* kSecondTime =
     "Trying to backward through the graph a second time (or directly access saved tensors after they have already been freed). "
     "Specify retain_graph=True if you need to backward through the graph a second time.";
 
-struct EncodeNode;
+// Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
+// consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
+// table scatter.
+struct EncodeNode : public Node {
+    std::shared_ptr<const Call> call;
+    void* forward_stream = nullptr;
+
+    // A training step on an SDF asks for two table gradients in one pass, through the encoded values and through the
+    // position gradient.  The node that meets the second one (EncodeBackNode) runs first, because it names this node as one
+    // of its outputs, and leaves it here; this node then computes both in one scatter, where two would each clear, bin
+    // and reduce a gradient of the table's size and autograd would add the two.
+    std::vector<SecondOrderTerm> second_order;
+
+    std::string name() const override { return "PermutoEncodingBackward"; }
+
+    void leave(SecondOrderTerm term) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        second_order.push_back(std::move(term));
+    }
+    std::vector<SecondOrderTerm> take(int task) {
+        std::vector<SecondOrderTerm> mine, others;
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SecondOrderTerm& t : second_order) (t.task == task ? mine : others).push_back(std::move(t));
+        second_order = std::move(others);
+        return mine;
+    }
+    variable_list apply(variable_list&& grads) override;
+};
 
 // Gradient of the gradients of the slicing.  Inputs (in the graph's sense): what EncodeNode produced, i.e. the
 // gradients w.r.t. the table and w.r.t. the positions; only the path through the latter is differentiated (as in the
@@ -340,6 +395,7 @@ struct EncodeNode;
 // slicing, whose node is named so that a pass through both runs it after this one.
 struct EncodeBackNode : public Node {
     std::shared_ptr<const Call> call;
+    std::shared_ptr<EncodeNode> slicing;
     Upstream upstream;
     bool released = false;
 
@@ -358,53 +414,79 @@ struct EncodeBackNode : public Node {
             TORCH_CHECK(!released, kSecondTime);
             up = upstream;
         }
+        up.check_unmodified();
         const Call& c = *call;
+        const bool grad_mode = c10::GradMode::is_enabled();
         at::NoGradGuard no_grad;
         const c10::DeviceGuard device(c.device());
-        SecondOrder s = compute_double_backward(c, grads[1], up, c.want_table && task_should_compute_output(1));
+        bool want_table = c.want_table && task_should_compute_output(1);
+        // (with create_graph the pass stays as it is written: EncodeNode's gradients are then differentiated once more, this one's not)
+        if (want_table && !grad_mode && up.row_stride == 0 && task_should_compute_output(2) &&
+            current_stream(c.device()) == slicing->forward_stream) {
+            slicing->leave({torch::autograd::get_current_graph_task_id(), grads[1].detach().contiguous(), up});
+            want_table = false;
+        }
+        const bool want_upstream = task_should_compute_output(0);
+        if (!want_table && !want_upstream) return out;
+        SecondOrder s = compute_double_backward(c, grads[1].detach(), up, want_table, want_upstream);
         out[0] = std::move(s.upstream);
         out[1] = std::move(s.table);
         return out;
     }
 };
 
-// Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
-// consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
-// table scatter.
-struct EncodeNode : public Node {
-    std::shared_ptr<const Call> call;
-
-    std::string name() const override { return "PermutoEncodingBackward"; }
-    variable_list apply(variable_list&& grads) override {
-        variable_list out(2);
-        if (grads.empty() || !grads[0].defined()) return out;  // reached through a double backward alone
-        const Call& c = *call;
-        const bool want_table = c.want_table && task_should_compute_output(0);
-        const bool want_positions = c.want_positions && task_should_compute_output(1);
-        if (!want_table && !want_positions) return out;
-        const bool differentiable = c10::GradMode::is_enabled();
-        Upstream up;
-        Gradients g;
-        {
-            at::NoGradGuard no_grad;
-            const c10::DeviceGuard device(c.device());
+variable_list EncodeNode::apply(variable_list&& grads) {
+    variable_list out(2);
+    const Call& c = *call;
+    std::vector<SecondOrderTerm> terms = take(torch::autograd::get_current_graph_task_id());
+    const bool first_order = !grads.empty() && grads[0].defined();  // undefined: reached through a double backward alone
+    const bool want_table = c.want_table && task_should_compute_output(0);
+    const bool want_positions = first_order && c.want_positions && task_should_compute_output(1);
+    if (!want_table && !want_positions) return out;
+    if (!first_order && terms.empty()) return out;
+    const bool differentiable = c10::GradMode::is_enabled();
+    Upstream up;
+    Gradients g;
+    {
+        at::NoGradGuard no_grad;
+        const c10::DeviceGuard device(c.device());
+        const SecondOrderTerm* fused = nullptr;
+        if (first_order) {
             up = upstream_of(c, grads[0].detach());
-            g = compute_backward(c, up, want_table, want_positions);
+            if (differentiable && want_positions && up.row_stride == c.columns() && c.columns() <= 255) {
+                // The position gradient needs its upstream gradient level by level; that copy outlives the call, so that the
+                // double backward's scatter reads it too (coalesced, where rows cost it a sixth of its time) and can be deferred.
+                Tensor level_major = level_major_array(c);
+                check(api.transpose(data(up.values), mutable_data(level_major), c.n, static_cast<int>(c.columns()), current_stream(c.device())),
+                      "transpose");
+                up = {level_major, 0};
+            }
+            if (want_table && !terms.empty()) fused = &terms.back();
+            g = compute_backward(c, up, want_table, want_positions, fused);
         }
-        if (differentiable) {
-            auto back = std::shared_ptr<EncodeBackNode>(new EncodeBackNode(), torch::autograd::deleteNode);
-            back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
-            back->add_next_edge(torch::autograd::Edge(shared_from_this(), 0));
-            back->call = call;
-            back->upstream = std::move(up);
-            torch::autograd::set_history(g.table, back);
-            torch::autograd::set_history(g.positions, back);
+        for (const SecondOrderTerm& t : terms) {
+            if (&t == fused || !want_table) continue;
+            Tensor more = compute_double_backward(c, t.double_positions_grad, t.upstream, true, false).table;
+            if (!more.defined()) continue;  // added into the sparse gradient
+            if (g.table.defined()) g.table.add_(more);
+            else g.table = std::move(more);
         }
-        out[0] = std::move(g.table);
-        out[1] = std::move(g.positions);
-        return out;
     }
-};
+    if (differentiable && first_order) {
+        auto back = std::shared_ptr<EncodeBackNode>(new EncodeBackNode(), torch::autograd::deleteNode);
+        back->slicing = std::static_pointer_cast<EncodeNode>(shared_from_this());
+        back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
+        back->add_next_edge(torch::autograd::Edge(back->slicing, 0));
+        back->call = call;
+        back->upstream = std::move(up);
+        back->upstream.keep();
+        torch::autograd::set_history(g.table, back);
+        torch::autograd::set_history(g.positions, back);
+    }
+    out[0] = std::move(g.table);
+    out[1] = std::move(g.positions);
+    return out;
+}
 
 // ------------------------------------------------------------------------------------------
 // Python
@@ -520,6 +602,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         if (c.want_table || c.want_positions) {
             auto node = std::shared_ptr<EncodeNode>(new EncodeNode(), torch::autograd::deleteNode);
             node->set_next_edges(torch::autograd::collect_next_edges(lattice_values, positions));
+            node->forward_stream = current_stream(call->device());
             node->call = std::move(call);
             torch::autograd::set_history(out, node);
         }
@@ -590,6 +673,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(backward_half);
         PENC_FN(backward_rowmajor);
         PENC_FN(backward_sparse);
+        PENC_FN(backward_both_orders);
         PENC_FN(double_backward_from_positions);
         PENC_FN(double_backward_from_positions_half);
         PENC_FN(double_backward_from_positions_rowmajor);

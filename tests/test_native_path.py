@@ -102,3 +102,69 @@ def test_native_path_graph_rules():
         native(pts.double())
     with pytest.raises(ValueError, match="anneal_window"):
         native(pts, torch.ones(3))
+
+
+@pytest.mark.parametrize("kw,normals", [({}, 1), (dict(sparse_table_grad=True), 1), (dict(lattice_half_precision=torch.bfloat16), 1),
+                                        (dict(contiguous_output=True, concat_points=True), 1), ({}, 2), (dict(sparse_table_grad=True), 2)])
+def test_losses_on_values_and_on_position_gradients_in_one_pass(kw, normals):
+    """loss(values) + loss(normals) in one backward pass, which computes both table gradients in one scatter (one more for
+    every further set of normals), against the autograd functions, which compute one after the other."""
+    native, python = modules(levels=6, **kw)
+    n = 3001
+    pts = torch.rand(n, 3, device="cuda")
+    ups = [torch.randn(n, native.output_dims(), device="cuda") for _ in range(normals)]
+    qs = [torch.randn(n, 3, device="cuda") for _ in range(normals)]
+    g = torch.randn(n, native.output_dims(), device="cuda")
+    results = []
+    for m in (native, python):
+        p = pts.clone().requires_grad_(True)
+        us = [u.clone().requires_grad_(True) for u in ups]
+        out = m(p)
+        grads = [torch.autograd.grad(out, p, u, create_graph=True)[0] for u in us]
+        torch.autograd.backward([out] + grads, [g] + qs)
+        table = m.table_grad.grad if m.sparse_table_grad else m.lattice_values.grad
+        assert m.sparse_table_grad == (m.lattice_values.grad is None)
+        results.append((table.clone(), p.grad, [u.grad for u in us]))
+    (ta, pa, ua), (tb, pb, ub) = results
+    close_sums(ta, tb)
+    assert torch.equal(pa, pb) and all(torch.equal(x, y) for x, y in zip(ua, ub))
+
+
+def test_upstream_gradient_modified_before_the_double_backward_is_refused():
+    native, _ = modules()
+    p = torch.rand(100, 3, device="cuda", requires_grad=True)
+    up = torch.randn(native.output_dims(), 100, device="cuda").t()  # level-major: kept as it is
+    normal, = torch.autograd.grad(native(p), p, up, create_graph=True)
+    up.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        normal.sum().backward()
+
+
+@pytest.mark.parametrize("d,n,levels,cap,rows,feat", [(2, 1, 3, 64, False, 2), (3, 511, 4, 1 << 12, True, 2), (3, 4097, 3, 1 << 20, False, 4), (4, 9000, 5, 50000, True, 2),
+                                                      (5, 1025, 2, 1 << 14, False, 2), (6, 700, 2, 1 << 12, True, 2), (8, 5000, 3, 1 << 13, False, 2),
+                                                      (3, 600000, 1, (1 << 22) + 5, True, 2)])
+def test_both_orders_in_one_scatter_match_the_oracle(d, n, levels, cap, rows, feat):
+    """penc_backward_both_orders at edges of tiles, groups and bin widths (more than 2^22 slots: wide bins) against the sum of the
+    oracle's two table gradients, within the bound of any sum in another order: 1e-4 of the sum of magnitudes."""
+    from helpers import assert_sum_close, make_encoding, random_problem, to_gpu
+    from oracle import api as orc
+    from permutohedral_encoding_amd import _native
+    p = random_problem(d, n, levels, cap, seed=60 + d, sigma_range=(1.0, 1e-3), nr_feat=feat)
+    first = np.random.default_rng(3).standard_normal((levels, feat, n)).astype(np.float32)
+    enc, fp = make_encoding(d, p["sigmas"], p["shift"], nr_feat=feat)
+    table, pos, win, dpos, first_t = (to_gpu(x) for x in (p["table"], p["pos"], p["window"], p["dpos"], first))
+    grad = to_gpu(p["grad"].transpose(2, 0, 1).reshape(n, -1) if rows else p["grad"])
+    lib = _native.lib()
+    ws = torch.empty(lib.penc_scatter_workspace_bytes(d, n, levels * feat // 2, cap, 0) + 4 * feat * levels * n + 1024, dtype=torch.uint8, device="cuda")
+    tg, pg = torch.full_like(table, float("nan")), torch.empty_like(pos)
+    rc = lib.penc_backward_both_orders(d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr(), 0, fp.m_scale_factor.data_ptr(),
+                                       fp.m_random_shift_per_level.data_ptr(), win.data_ptr(), grad.data_ptr(), feat * levels if rows else 0,
+                                       dpos.data_ptr(), first_t.data_ptr(), tg.data_ptr(), None, pg.data_ptr(), ws.data_ptr(), ws.numel(),
+                                       torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    sf = orc.scale_factors(d, p["sigmas"])
+    a = orc.backward_table(p["pos"], sf, p["shift"], p["window"], p["grad"], cap, want_abs=True)
+    b = orc.double_backward(p["pos"], p["table"], sf, p["shift"], p["window"], p["dpos"], first, want_abs=True)
+    assert_sum_close(tg.cpu().numpy(), a["grad64"] + b["grad64"], a["abs64"] + b["abs64"], 1e-4, "both table gradients")
+    wp = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], p["window"], p["grad"])
+    assert np.all(np.abs(pg.cpu().numpy() - wp["grad64"]) <= 1e-6 * wp["abs64"] + 1e-30)
