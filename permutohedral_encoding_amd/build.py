@@ -9,7 +9,7 @@ LIB_PATH = os.path.join(_HERE, "libpenc_hip.so")
 
 def build_library(force=True, verbose=False):
     """Runs ``make`` in ``csrc/``; with ``force`` the library is rebuilt even if it is up to date."""
-    cmd = ["make", "-j4", "-C", CSRC]
+    cmd = ["make", "-j8", "-C", CSRC]
     if force:
         cmd.append("-B")
     res = subprocess.run(cmd, capture_output=True, text=True)

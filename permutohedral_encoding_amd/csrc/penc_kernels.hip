@@ -23,7 +23,9 @@
 
 #include "../../include/penc.h"
 #include "penc_lattice.hpp"
+#include "penc_reduce.hpp"
 #include "penc_scatter.hpp"
+#include "penc_table_backward.hpp"
 
 namespace penc {
 
@@ -98,6 +100,37 @@ __device__ __forceinline__ Vertices<D, F> load_vertices(const T* __restrict__ le
 }
 
 // ------------------------------------------------------------------------------------------
+// which (tile of points, row of levels) a workgroup of a gathering kernel takes
+//
+// A row is one level, or two levels `rows` apart: with the usual coarse-to-fine level list a level whose gathers hit the
+// first-level cache with one that waits for the L2.  Each die has an L2 of its own, and workgroup i runs on die i % dies.
+// With the grid as (tile, row) every die gathers from every level, so each of the eight L2s fetches the whole table: 400 MB
+// for 24 slices of 2 MiB, 10 us whatever the number of points, a third of the forward of 2^16 points.  With `segment` != 0
+// the (row, tile) pairs, row by row, are cut into rounds * dies segments and a die takes one segment of each round, in
+// alternating directions (the dies' shares of coarse and fine rows then even out); a table slice is fetched by one or two dies.
+// Measured, forward, D = 3, 24 levels of 2^18 slots (before -> after): 2^13 points 10.3 -> 5.3 us, 2^15 22.2 -> 12.6,
+// 2^16 33.3 -> 23.4, 2^18 85.6 -> 76.4, 2^20 289 -> 283.
+struct LevelMap {
+    uint32_t tiles;    // workgroups per row
+    uint32_t rows;
+    uint32_t segment;  // (row, tile) pairs per segment; 0: the grid is (tile, row)
+    uint32_t dies;
+};
+__device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile, uint32_t& row) {
+    if (map.segment == 0u) {
+        tile = blockIdx.x;
+        row = blockIdx.y;
+        return true;
+    }
+    const uint32_t die = blockIdx.x % map.dies, j = blockIdx.x / map.dies;
+    const uint32_t round = j / map.segment;
+    const uint32_t at = (round * map.dies + ((round & 1u) ? map.dies - 1u - die : die)) * map.segment + j % map.segment;
+    row = at / map.tiles;
+    tile = at % map.tiles;
+    return row < map.rows;
+}
+
+// ------------------------------------------------------------------------------------------
 // forward (EncodingGPU.cuh:68-256)
 //
 // One thread per point and one or two levels (the host says which).  Measured alternatives, all
@@ -111,31 +144,30 @@ __device__ __forceinline__ Vertices<D, F> load_vertices(const T* __restrict__ le
 
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-forward_kernel(int n_points, int n_levels, int n_all_levels, int levels_per_thread, uint32_t capacity, uint32_t cap_mask,
+forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
                const float* __restrict__ positions, const T* __restrict__ table,
                const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                const float* __restrict__ window, float* __restrict__ sliced, float points_scaling) {
-    const int n = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t tile, row;
+    if (!locate_work(map, tile, row)) return;
+    const int n = tile * kBlock + threadIdx.x;
     if (n >= n_points) return;
     __shared__ uint2 columns[(D + 1) * kBlock];
     const fvec<D> point = load_point<D>(positions, n);
-    // The levels of a thread are `gridDim.y` apart: with the usual coarse-to-fine level list a thread that
-    // takes two pairs a level whose gathers hit the first-level cache with one that waits for the L2.
-#pragma unroll 1
-    for (int k2 = 0; k2 < levels_per_thread; ++k2) {
-        const int level = static_cast<int>(blockIdx.y) + k2 * static_cast<int>(gridDim.y);
-        if (level >= n_all_levels) break;
-        float* out = sliced + (static_cast<size_t>(level) * F) * n_points + n;  // feature k at out[k * n_points]
-
-        if (level >= n_levels) {  // extra levels carrying the raw positions (:106-121)
+    if (row == 0u) {  // extra levels carrying the raw positions (:106-121)
+        for (int level = n_levels; level < n_all_levels; ++level) {
+            float* out = sliced + (static_cast<size_t>(level) * F) * n_points + n;
             const int src = (level - n_levels) * F;
             const float* p = positions + static_cast<size_t>(n) * D;
             static_for<F>(PENC_BODY(k) {
                 PENC_INDEX(k);
                 out[static_cast<size_t>(k) * n_points] = src + k < D ? p[src + k] * points_scaling : 0.0f;
             });
-            continue;
         }
+    }
+#pragma unroll 1
+    for (int level = static_cast<int>(row); level < n_levels; level += static_cast<int>(map.rows)) {
+        float* out = sliced + (static_cast<size_t>(level) * F) * n_points + n;  // feature k at out[k * n_points]
         const float w_level = window[level];
         if (w_level == 0.0f) {
             static_for<F>(PENC_BODY(k) {
@@ -166,246 +198,6 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, int levels_per_thre
 }
 
 // ------------------------------------------------------------------------------------------
-// backward w.r.t. the table (EncodingGPU.cuh:259-414)
-
-// Wavefronts per SIMD the scattering kernel is compiled for: six (three workgroups per compute unit, at
-// most 80 vector registers) where that costs a few spilled registers at most, else four (two
-// workgroups, 128 registers).  Measured at 2^19 points, 24 levels: table backward 0.367 -> 0.338 ms
-// at D = 4 (84 -> 80 registers, 3 spilled), 0.458 -> 0.424 ms at D = 5; the second-order kernel
-// 0.577 -> 0.552 ms at D = 4, but 0.735 -> 0.754 ms at D = 5 (11 spilled), which therefore stays at
-// four; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
-// unit: held to 128, 1.334 -> 1.113 ms.
-constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins) {
-    if (wide_bins) return pos_dim <= 3 ? 6 : 4;  // (a variable bin width takes six to eight more registers: up to 30 spilled at D = 4)
-    return pos_dim <= 4 || (pos_dim == 5 && !second_order) ? 6 : 4;
-}
-
-constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins) { return pos_dim <= 3 && !wide_bins ? 6 : 4; }
-
-// kRowMajor: the upstream gradient is read as rows grad[n][2*level + feature] of `grad_row_stride`
-// floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
-// all levels of a group of points back to back, so the rows mostly come from L2 (measured: fetched
-// from memory 2.7 times, not once per level) although every level only uses 8 bytes of each.
-// With `grad_level_major` the kernel also leaves the values it read in [level][feature][n] order
-// (for the position-gradient kernel, which gathers level by level and wants its upstream gradient
-// coalesced): the layout change rides on reads this kernel makes anyway.
-// Second order: the table-gradient half of the double backward (EncodingGPU.cuh:1016-1257): the
-// vertex weights are the derivatives of the barycentric weights along `double_pos_grad` instead of
-// the barycentric weights themselves; everything else is the same scatter.
-// feat_pairs: with four or eight features per level the pairs (0,1), (2,3), ... are scattered like levels that
-// share their geometry: "levels" below (first_level, n_pass_levels, the grid, the bins) count pairs,
-// `pair_level` = level * feat_pairs + pair.  The upstream gradient needs no special case: [L][F][N]
-// is [L * F/2][2][N], and in a row the pair sits at column 2 * pair_level.
-// kWideBins: the bins span more than kBinSlots slots (tables above 2^22 slots).  A parameter of the kernel
-// rather than a value read from its arguments, because with the bin width a variable the usual instances
-// need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
-// kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
-// a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
-// gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
-// reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
-enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
-template <int D, bool kRowMajor, int kOrder, bool kWideBins>
-__device__ __forceinline__ void
-scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
-                        uint32_t capacity, uint32_t cap_mask,
-                        const float* __restrict__ positions, const float* __restrict__ scale_factor,
-                        const float* __restrict__ random_shift, const float* __restrict__ window,
-                        const float* __restrict__ grad_sliced, int64_t grad_row_stride,
-                        const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
-                        float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
-    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
-    __shared__ ScatterStateT<stage_chunk(D)> state;
-    // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
-    // workgroup of a die takes level j % levels of one group of points: a die works through all
-    // levels of a group before the next group, so the points are fetched from memory once, and
-    // compute-bound coarse levels and store-bound fine levels share the chip at all times (this
-    // kernel never reads the table: there is no slice to keep cache-resident by running a level at
-    // a time).
-    const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
-    const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
-    const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kScatterBlock;
-    if (group_base >= n_points) return;
-    const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;
-    const int level = static_cast<int>(pair_level / feat_pairs);  // the geometry's level
-    const float w_level = window[level];
-    if (w_level == 0.0f) return;
-    scatter_begin(state);
-    BinTarget bins = bins_of_level(pass_bins, level_in_pass);
-    if constexpr (!kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
-    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
-                               2 * feat_pairs, bins.direct, bins.bin_shift};
-    // Everything a thread reads lies within its group of at most 16 x 512 points, so the addresses are
-    // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets.
-    const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);
-    const float* const group_positions = positions + group_base * D;
-    const float* const group_q = kNeedsQ ? double_pos_grad + group_base * D : nullptr;
-    const float* const group_grad0 =
-        kRowMajor ? grad_sliced + group_base * grad_row_stride + 2 * pair_level
-                  : grad_sliced + (static_cast<size_t>(pair_level) * 2) * n_points + group_base;
-    const float* const group_grad1 = group_grad0 + n_points;
-    const auto load_grad = [&](uint32_t i, float& g0, float& g1) {
-        if constexpr (kRowMajor) {
-            const float2 g = *reinterpret_cast<const float2*>(group_grad0 + static_cast<int64_t>(i) * grad_row_stride);
-            g0 = g.x;
-            g1 = g.y;
-        } else {
-            g0 = group_grad0[i];
-            g1 = group_grad1[i];
-        }
-    };
-    const float* const group_second0 = kBoth ? second_grad + (static_cast<size_t>(pair_level) * 2) * n_points + group_base : nullptr;
-    const float* const group_second1 = group_second0 + n_points;
-    const auto load_group_point = [&](const float* base, uint32_t i) {
-        fvec<D> v;
-        static_for<D>(PENC_BODY(k) {
-            PENC_INDEX(k); v[k] = base[i * static_cast<uint32_t>(D) + k]; });
-        return v;
-    };
-    // A tile's inputs are fetched one tile ahead: their latency then overlaps the previous tile's
-    // scatter instead of stalling the wave at the top of every iteration.
-    const auto point_of = [&](int t) {  // the point this thread handles in tile t, within the group (clamped: the tail re-reads the last point)
-        const uint32_t i = static_cast<uint32_t>(t) * kScatterBlock + threadIdx.x;
-        return i < last_in_group ? i : last_in_group;
-    };
-    uint32_t nn = point_of(0);
-    fvec<D> pos = load_group_point(group_positions, nn);
-    fvec<D> q = 0.0f;
-    if constexpr (kNeedsQ) q = load_group_point(group_q, nn);
-    float g0, g1;
-    load_grad(nn, g0, g1);
-    float s0 = 0.0f, s1 = 0.0f;
-    if constexpr (kBoth) {
-        s0 = group_second0[nn];
-        s1 = group_second1[nn];
-    }
-    int mode = kModeCache;
-    uint32_t id_bits = 0;
-    for (int t = 0; t < tiles_per_group; ++t) {
-        const int64_t tile_base = group_base + static_cast<int64_t>(t) * kScatterBlock;
-        if (tile_base >= n_points) break;
-        const bool active = tile_base + threadIdx.x < n_points;
-        const uint32_t nn_next = point_of(t + 1);
-        const fvec<D> pos_next = load_group_point(group_positions, nn_next);
-        fvec<D> q_next = 0.0f;
-        if constexpr (kNeedsQ) q_next = load_group_point(group_q, nn_next);
-        float g0_next, g1_next;
-        load_grad(nn_next, g0_next, g1_next);
-        float s0_next = 0.0f, s1_next = 0.0f;
-        if constexpr (kBoth) {
-            s0_next = group_second0[nn_next];
-            s1_next = group_second1[nn_next];
-        }
-        if constexpr (kRowMajor) {
-            if (grad_level_major != nullptr && active) {
-                float* out = grad_level_major + (static_cast<size_t>(pair_level) * 2) * n_points + tile_base + threadIdx.x;
-                out[0] = g0;
-                out[n_points] = g1;
-            }
-        }
-        const Located<D> s = locate<D>(pos, random_shift + level * D, scale_factor + level * D);
-        uvec<D + 1> h;
-        fvec<D + 1> w;   // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
-        fvec<D + 1> w2;  // kBoth: the latter
-        bool via_lds = false;
-        if constexpr (D > kWorkgroupSortMaxDim) {
-            // Once the workgroup streams with every wave sorting on its own (stream_tile_wave), a wave's staging
-            // slice is idle between its tiles and nobody else touches it: it serves as the thread-private
-            // columns that put residuals and hash steps into rank order, in place of D(D+1) selects each
-            // (at D = 8 about 270 of 1350 vector instructions per point and level).
-            via_lds = mode == kModeStream && bins.n_bins <= static_cast<uint32_t>(kStageBins);
-        }
-        if (via_lds) {
-            constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D)>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
-            static_assert((D + 1) * 64 <= kSliceCells, "a wave's staging slice holds a column of D+1 cells per lane");
-            uint2* const column = reinterpret_cast<uint2*>(state.val) + (threadIdx.x >> 6) * kSliceCells + (threadIdx.x & 63);
-            fvec<D + 1> sorted;
-            if constexpr (kBoth) {
-                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-                wave_lds_fence();
-                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else if constexpr (kOrder == kSecondOrder) {
-                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else {
-                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-            }
-            wave_lds_fence();  // the slice is staging space again from here on
-        } else {
-            h = vertex_hashes<D>(s.rank, s.hash0);
-            if constexpr (kBoth) {
-                w = barycentric<D>(s.rank, s.delta) * w_level;
-                w2 = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
-            } else if constexpr (kOrder == kSecondOrder) {
-                w = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
-            } else {
-                w = barycentric<D>(s.rank, s.delta) * w_level;
-            }
-        }
-        uvec<D + 1> slot;
-        static_for<D + 1>(PENC_BODY(r) {
-            PENC_INDEX(r);
-            slot[r] = to_slot(h[r], capacity, cap_mask);
-        });
-        if (t == 0) {
-            // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
-            // (its point is already here)
-            const auto slots_of_next_tile = [&]() {
-                const Located<D> s1 = locate<D>(pos_next, random_shift + level * D, scale_factor + level * D);
-                const uvec<D + 1> h1 = vertex_hashes<D>(s1.rank, s1.hash0);
-                uvec<D + 1> slot1;
-                static_for<D + 1>(PENC_BODY(r) {
-                    PENC_INDEX(r);
-                    slot1[r] = to_slot(h1[r], capacity, cap_mask);
-                });
-                return slot1;
-            };
-            const bool next_active = tile_base + kScatterBlock + threadIdx.x < n_points && tiles_per_group > 1;
-            mode = scatter_mode_decide<D>(state, bins, active, slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
-        }
-        fvec<D + 1> a0 = w * g0, a1 = w * g1;  // g_f * (b_r * w_level), :405-410
-        if constexpr (kBoth) {
-            a0 += w2 * s0;
-            a1 += w2 * s1;
-        }
-        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1);
-        // the first tile finds the lines its own look-up has claimed: no evidence of reuse
-        if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
-        pos = pos_next;
-        q = q_next;
-        g0 = g0_next;
-        g1 = g1_next;
-        s0 = s0_next;
-        s1 = s1_next;
-    }
-    scatter_end(state, level_grad, bins, group, mode, id_bits);
-}
-
-#define PENC_TABLE_PARAMETERS                                                                                                          \
-    int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group, uint32_t capacity, \
-        uint32_t cap_mask, const float *__restrict__ positions, const float *__restrict__ scale_factor,                                \
-        const float *__restrict__ random_shift, const float *__restrict__ window, const float *__restrict__ grad_sliced,               \
-        int64_t grad_row_stride, const float *__restrict__ double_pos_grad, const float *__restrict__ second_grad,                     \
-        float *__restrict__ table_grad, float *__restrict__ grad_level_major, BinTarget pass_bins
-#define PENC_TABLE_ARGUMENTS                                                                                                        \
-    n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
-        random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
-template <int D, bool kRowMajor, bool kSecond, bool kWideBins>
-__global__ void __launch_bounds__(kScatterBlock, scatter_waves_per_simd(D, kSecond, kWideBins))
-backward_table_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins>(PENC_TABLE_ARGUMENTS);
-}
-template <int D, bool kRowMajor, bool kWideBins>
-__global__ void __launch_bounds__(kScatterBlock, both_orders_waves_per_simd(D, kWideBins))
-backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins>(PENC_TABLE_ARGUMENTS);
-}
-#undef PENC_TABLE_PARAMETERS
-#undef PENC_TABLE_ARGUMENTS
-
-// ------------------------------------------------------------------------------------------
 // backward w.r.t. positions (EncodingGPU.cuh:530-769)
 
 // One thread per (point, group of levels): the levels of the group are summed in
@@ -417,22 +209,22 @@ backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
 // kernel's rank permutations through LDS, as the forward does, was measured: no gain.)
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-backward_pos_kernel(int n_points, int n_levels, int levels_per_group, uint32_t capacity, uint32_t cap_mask,
+backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
                     const float* __restrict__ positions, const T* __restrict__ table,
                     const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                     const float* __restrict__ window, const float* __restrict__ grad_sliced,
                     float* __restrict__ out) {
-    const int n = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t tile, row;
+    if (!locate_work(map, tile, row)) return;
+    const int n = tile * kBlock + threadIdx.x;
     if (n >= n_points) return;
     const fvec<D> pos = load_point<D>(positions, n);
     fvec<D> total = 0.0f;
-    // The levels of a group are `gridDim.y` apart, not adjacent: with the usual coarse-to-fine level list a
+    // The levels of a group are `rows` apart, not adjacent: with the usual coarse-to-fine level list a
     // group then pairs a coarse level, whose points share few slots, with a fine one, and the table slices
-    // the whole chip gathers from at any time fit the L2 (two adjacent fine levels are 4 MiB at 2^18 slots,
+    // a die gathers from at any time fit its L2 (two adjacent fine levels are 4 MiB at 2^18 slots,
     // an L2's whole capacity).
-    for (int k = 0; k < levels_per_group; ++k) {
-        const int level = static_cast<int>(blockIdx.y) + k * static_cast<int>(gridDim.y);
-        if (level >= n_levels) break;
+    for (int level = static_cast<int>(row); level < n_levels; level += static_cast<int>(map.rows)) {
         const float w_level = window[level];
         if (w_level == 0.0f) continue;
         const float* sf = scale_factor + level * D;
@@ -449,7 +241,7 @@ backward_pos_kernel(int n_points, int n_levels, int levels_per_group, uint32_t c
         });
         total += bary_grad_to_pos_grad<D>(s.rank, dB, sf);
     }
-    float* o = out + (static_cast<size_t>(blockIdx.y) * n_points + n) * D;
+    float* o = out + (static_cast<size_t>(row) * n_points + n) * D;
     static_for<D>(PENC_BODY(i) {
         PENC_INDEX(i);
         o[i] = total[i];
@@ -476,22 +268,24 @@ reduce_level_groups_kernel(const float* __restrict__ partial, int n_groups, size
 
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-grad_grad_kernel(int n_points, int n_levels, int n_all_levels, int levels_per_thread, uint32_t capacity, uint32_t cap_mask,
+grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
                  const float* __restrict__ positions, const T* __restrict__ table,
                  const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                  const float* __restrict__ window, const float* __restrict__ double_pos_grad,
                  float* __restrict__ grad_grad_sliced) {
-    const int n = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t tile, row;
+    if (!locate_work(map, tile, row)) return;
+    const int n = tile * kBlock + threadIdx.x;
     if (n >= n_points) return;
     __shared__ uint2 columns[(D + 1) * kBlock];
     const fvec<D> point = load_point<D>(positions, n), q = load_point<D>(double_pos_grad, n);
-    // the levels of a thread are `gridDim.y` apart, as in the forward
+    if (row == 0u) {  // concat levels: zeros (:1290-1295)
+        for (size_t k = static_cast<size_t>(n_levels) * F; k < static_cast<size_t>(n_all_levels) * F; ++k) grad_grad_sliced[k * n_points + n] = 0.0f;
+    }
 #pragma unroll 1
-    for (int k2 = 0; k2 < levels_per_thread; ++k2) {
-        const int level = static_cast<int>(blockIdx.y) + k2 * static_cast<int>(gridDim.y);
-        if (level >= n_all_levels) break;
+    for (int level = static_cast<int>(row); level < n_levels; level += static_cast<int>(map.rows)) {
         float* o = grad_grad_sliced + (static_cast<size_t>(level) * F) * n_points + n;
-        const float w_level = level < n_levels ? window[level] : 0.0f;  // concat levels: zeros (:1290-1295)
+        const float w_level = window[level];
         if (w_level == 0.0f) {
             static_for<F>(PENC_BODY(k) {
                 PENC_INDEX(k); o[static_cast<size_t>(k) * n_points] = 0.0f; });
@@ -991,11 +785,6 @@ inline int reduce_bins(const BinPlan& p, const float* window, int first_level, i
 
 inline unsigned tiles(int64_t n) { return static_cast<unsigned>((n + kBlock - 1) / kBlock); }
 
-// Levels a thread of the forward and of the gathering half of the double backward takes: two up to
-// pos_dim 4 (measured on the forward at 2^20 points, 24 levels: 0.310 -> 0.302 ms at pos_dim 3, 0.275 -> 0.259 ms with a
-// 2^22-slot table, 0.396 -> 0.392 ms at pos_dim 4; at pos_dim 8 0.283 -> 0.298 ms).
-inline int gather_levels_per_thread(int pos_dim) { return pos_dim <= 4 ? 2 : 1; }
-
 // Device address of this GPU's copy of `scratch`, looked up on the first call with that GPU
 // current and kept for the life of the process.  Returns nullptr when the lookup fails.
 constexpr int kMaxDevices = 64;
@@ -1033,6 +822,55 @@ inline uint32_t dies_of_current_device() {
         dies[device] = n >= 1 && n <= 64 ? static_cast<uint32_t>(n) : kDefaultDies;
     }
     return dies[device];
+}
+
+// Levels a thread of the forward and of the gathering half of the double backward takes: two up to
+// pos_dim 4 (measured on the forward at 2^20 points, 24 levels: 0.310 -> 0.302 ms at pos_dim 3, 0.275 -> 0.259 ms with a
+// 2^22-slot table, 0.396 -> 0.392 ms at pos_dim 4; at pos_dim 8 0.283 -> 0.298 ms) and once the launch fills the chip twice
+// over with pairs (eight workgroups of four wavefronts per compute unit; 2^15 points: 12.6 us with single levels, 15.9 with
+// pairs, 2^16 23.4 and 24.8, 131 k 31.4 and 30.5).
+constexpr int64_t kPairsMinWorkgroups = 4096;
+inline int gather_levels_per_thread(int pos_dim, int64_t n, int levels) {
+    return pos_dim <= 4 && static_cast<int64_t>(tiles(n)) * ((levels + 1) / 2) >= kPairsMinWorkgroups ? 2 : 1;
+}
+
+// The largest table slice (bytes of one level) a die keeps to itself.  Up to here several slices at once fit the memory-side
+// cache; with 32 MiB slices on every die that cache thrashes (2^22 slots: the forward 251 us with all dies on the same
+// rows, 325 with segments; 2^20 slots: 138.5 and 135.5).
+constexpr size_t kMaxSegmentSliceBytes = size_t{8} << 20;
+
+// The map of a launch over `levels` levels, `levels_per_row` to a thread, and its grid.  Rounds: few rounds mean few fetches of
+// each slice, more of them a more even share of the coarse and the fine rows for every die (a fine row costs up to five
+// coarse ones).  Rows of two levels are even in themselves: three rounds, four where there are fewer rows than dies.  Rows of
+// one level: three rounds while the launch is small and the fetches are a good part of it, then eight (forward, D = 6, 16 levels,
+// 2^18 points: 92.5 us without segments, 94.1 / 91.2 / 91.2 with 3 / 5 / 8 rounds; D = 8, 24 levels, 20000 points: 31.4, then
+// 18.1 / 21.0 / 22.4), and none for launches so large that the fetches no longer matter but the dies' unequal ends do
+// (D = 5, 2^20 points: 289 and 295 us; position backward, D = 3, samples along rays, 2^20 points: 287 and 295 us).
+struct GatherLaunch {
+    LevelMap map;
+    dim3 grid;
+};
+constexpr uint64_t kSmallGather = 8192, kLargeGather = 65536;  // (row, tile) pairs
+inline GatherLaunch plan_gather(int64_t n, int levels, int levels_per_row, size_t slice_bytes, uint64_t most_pairs = uint64_t{1} << 30) {
+    GatherLaunch g;
+    g.map.tiles = tiles(n);
+    g.map.rows = static_cast<uint32_t>((levels + levels_per_row - 1) / levels_per_row);
+    g.map.segment = 0;
+    g.map.dies = dies_of_current_device();
+    g.grid = dim3(g.map.tiles, g.map.rows);
+    const uint64_t work = static_cast<uint64_t>(g.map.tiles) * g.map.rows;
+    // (with fewer single levels than dies the shares cannot be evened out: 6 levels of 300 k points 30.4 -> 33.1 us)
+    if (g.map.dies < 2 || g.map.rows < (levels_per_row > 1 ? 2u : g.map.dies) || slice_bytes > kMaxSegmentSliceBytes ||
+        work >= (levels_per_row > 1 ? most_pairs : kLargeGather))
+        return g;
+    const uint32_t rounds = levels_per_row > 1 ? (g.map.rows >= g.map.dies ? 3 : 4) : (work < kSmallGather ? 3 : 8);
+    const uint64_t segments = static_cast<uint64_t>(rounds) * g.map.dies;
+    g.map.segment = static_cast<uint32_t>((work + segments - 1) / segments);
+    g.grid = dim3(static_cast<uint32_t>(segments * g.map.segment));
+    return g;
+}
+inline size_t slice_bytes(int capacity, int nr_feat, const int format) {
+    return static_cast<size_t>(capacity) * nr_feat * (format != 0 ? 2 : 4);
 }
 
 }  // namespace penc
@@ -1085,41 +923,33 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     for (int first = 0; first < pair_levels; first += per_pass) {
         const int count = pair_levels - first < per_pass ? pair_levels - first : per_pass;
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
-        const dim3 grid(padded_groups * static_cast<unsigned>(count));
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
-#define PENC_LAUNCH_TABLE(...)                                                                                             \
-    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(kScatterBlock), 0, st, n, first,                    \
-                                                static_cast<uint32_t>(count), feat_pairs, dies, tiles_per_group, cap, mask,  \
-                                                positions, scale_factor, random_shift, anneal_window, grad, grad_row_stride, \
-                                                second.double_pos_grad, second.upstream, lattice_values_grad,                \
-                                                grad_level_major, plan.target))
-#define PENC_LAUNCH_TABLE_WIDTH(KERNEL, ...)                \
-    if (wide_bins) {                                        \
-        PENC_LAUNCH_TABLE(KERNEL<DD, __VA_ARGS__, true>);   \
-    } else {                                                \
-        PENC_LAUNCH_TABLE(KERNEL<DD, __VA_ARGS__, false>);  \
-    }
-        const bool wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
-        const bool rows = grad_row_stride != 0;
-        if (second.upstream != nullptr) {
-            if (rows) {
-                PENC_LAUNCH_TABLE_WIDTH(backward_table_both_kernel, true);
-            } else {
-                PENC_LAUNCH_TABLE_WIDTH(backward_table_both_kernel, false);
-            }
-        } else if (second.double_pos_grad != nullptr) {
-            if (rows) {
-                PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, true, true);
-            } else {
-                PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, false, true);
-            }
-        } else if (rows) {
-            PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, true, false);
-        } else {
-            PENC_LAUNCH_TABLE_WIDTH(backward_table_kernel, false, false);
-        }
-#undef PENC_LAUNCH_TABLE_WIDTH
-#undef PENC_LAUNCH_TABLE
+        TableLaunch t{};
+        t.grid = dim3(padded_groups * static_cast<unsigned>(count));
+        t.stream = st;
+        t.rows = grad_row_stride != 0;
+        t.second_order = second.double_pos_grad != nullptr;
+        t.wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
+        t.n_points = n;
+        t.first_level = first;
+        t.n_pass_levels = static_cast<uint32_t>(count);
+        t.feat_pairs = feat_pairs;
+        t.dies = dies;
+        t.tiles_per_group = tiles_per_group;
+        t.capacity = cap;
+        t.cap_mask = mask;
+        t.positions = positions;
+        t.scale_factor = scale_factor;
+        t.random_shift = random_shift;
+        t.window = anneal_window;
+        t.grad = grad;
+        t.grad_row_stride = grad_row_stride;
+        t.double_pos_grad = second.double_pos_grad;
+        t.second_grad = second.upstream;
+        t.table_grad = lattice_values_grad;
+        t.grad_level_major = grad_level_major;
+        t.bins = plan.target;
+        PENC_DISPATCH_D(pos_dim, launch_table_backward<DD>(t));
         if (int rc = check_launch()) return rc;
         if (plan.enabled)
             if (int rc = reduce_bins(plan, anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
@@ -1147,9 +977,9 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
         groups = want_groups;
         partial = reinterpret_cast<float*>(ws);
     }
+    const GatherLaunch g = plan_gather(nr_positions, nr_levels, per_group, slice_bytes(capacity, nr_feat, table.format), kLargeGather / 2);
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), dim3(tiles(nr_positions), groups), dim3(kBlock), 0,
-                                         st, n, nr_levels, per_group, cap, mask, positions,
+                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st, n, nr_levels, g.map, cap, mask, positions,
                                          static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
                                          grad_level_major, partial));
     if (int rc = check_launch()) return rc;
@@ -1214,11 +1044,11 @@ static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_l
         return PENC_ERR_NULL_POINTER;
     if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int per_thread = gather_levels_per_thread(pos_dim);
-    const dim3 grid(tiles(nr_positions), (nr_levels + extra + per_thread - 1) / per_thread);
+    const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
+                                       slice_bytes(capacity, nr_feat, table.format));
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((forward_kernel<DD, FF, TT>), grid, dim3(kBlock), 0, st,
-                                         static_cast<int>(nr_positions), nr_levels, nr_levels + extra, per_thread, static_cast<uint32_t>(capacity),
+                      hipLaunchKernelGGL((forward_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st,
+                                         static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity),
                                          mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,
                                          random_shift, anneal_window, sliced_values, points_scaling));
     return check_launch();
@@ -1474,11 +1304,11 @@ static int double_backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, 
     if (!table_aligned(table, nr_feat) || !aligned8(lattice_values_grad)) return PENC_ERR_MISALIGNED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (grad_grad_sliced_values) {
-        const int per_thread = gather_levels_per_thread(pos_dim);
-        const dim3 grid(tiles(nr_positions), (nr_levels + extra + per_thread - 1) / per_thread);
+        const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
+                                           slice_bytes(capacity, nr_feat, table.format));
         PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                          hipLaunchKernelGGL((grad_grad_kernel<DD, FF, TT>), grid, dim3(kBlock), 0, st,
-                                             static_cast<int>(nr_positions), nr_levels, nr_levels + extra, per_thread, static_cast<uint32_t>(capacity),
+                          hipLaunchKernelGGL((grad_grad_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st,
+                                             static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity),
                                              mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,
                                              random_shift, anneal_window, double_positions_grad, grad_grad_sliced_values));
         if (int rc = check_launch()) return rc;

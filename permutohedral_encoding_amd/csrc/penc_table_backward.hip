@@ -1,0 +1,286 @@
+// The scattering kernel of the table gradient, for the input dimension PENC_DIM (see penc_table_backward.hpp).
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "penc_lattice.hpp"
+#include "penc_scatter.hpp"
+#include "penc_table_backward.hpp"
+
+namespace penc {
+
+// ------------------------------------------------------------------------------------------
+// backward w.r.t. the table (EncodingGPU.cuh:259-414)
+
+// Wavefronts per SIMD the scattering kernel is compiled for: six (three workgroups per compute unit, at
+// most 80 vector registers) where that costs a few spilled registers at most, else four (two
+// workgroups, 128 registers).  Measured at 2^19 points, 24 levels: table backward 0.367 -> 0.338 ms
+// at D = 4 (84 -> 80 registers, 3 spilled), 0.458 -> 0.424 ms at D = 5; the second-order kernel
+// 0.577 -> 0.552 ms at D = 4, but 0.735 -> 0.754 ms at D = 5 (11 spilled), which therefore stays at
+// four; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
+// unit: held to 128, 1.334 -> 1.113 ms.
+constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins) {
+    if (wide_bins) return pos_dim <= 3 ? 6 : 4;  // (a variable bin width takes six to eight more registers: up to 30 spilled at D = 4)
+    return pos_dim <= 4 || (pos_dim == 5 && !second_order) ? 6 : 4;
+}
+
+constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins) { return pos_dim <= 3 && !wide_bins ? 6 : 4; }
+
+// kRowMajor: the upstream gradient is read as rows grad[n][2*level + feature] of `grad_row_stride`
+// floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
+// all levels of a group of points back to back, so the rows mostly come from L2 (measured: fetched
+// from memory 2.7 times, not once per level) although every level only uses 8 bytes of each.
+// With `grad_level_major` the kernel also leaves the values it read in [level][feature][n] order
+// (for the position-gradient kernel, which gathers level by level and wants its upstream gradient
+// coalesced): the layout change rides on reads this kernel makes anyway.
+// Second order: the table-gradient half of the double backward (EncodingGPU.cuh:1016-1257): the
+// vertex weights are the derivatives of the barycentric weights along `double_pos_grad` instead of
+// the barycentric weights themselves; everything else is the same scatter.
+// feat_pairs: with four or eight features per level the pairs (0,1), (2,3), ... are scattered like levels that
+// share their geometry: "levels" below (first_level, n_pass_levels, the grid, the bins) count pairs,
+// `pair_level` = level * feat_pairs + pair.  The upstream gradient needs no special case: [L][F][N]
+// is [L * F/2][2][N], and in a row the pair sits at column 2 * pair_level.
+// kWideBins: the bins span more than kBinSlots slots (tables above 2^22 slots).  A parameter of the kernel
+// rather than a value read from its arguments, because with the bin width a variable the usual instances
+// need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
+// kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
+// a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
+// gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
+// reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
+enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
+template <int D, bool kRowMajor, int kOrder, bool kWideBins>
+__device__ __forceinline__ void
+scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
+                        uint32_t capacity, uint32_t cap_mask,
+                        const float* __restrict__ positions, const float* __restrict__ scale_factor,
+                        const float* __restrict__ random_shift, const float* __restrict__ window,
+                        const float* __restrict__ grad_sliced, int64_t grad_row_stride,
+                        const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
+                        float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
+    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
+    __shared__ ScatterStateT<stage_chunk(D)> state;
+    // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
+    // workgroup of a die takes level j % levels of one group of points: a die works through all
+    // levels of a group before the next group, so the points are fetched from memory once, and
+    // compute-bound coarse levels and store-bound fine levels share the chip at all times (this
+    // kernel never reads the table: there is no slice to keep cache-resident by running a level at
+    // a time).
+    const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
+    const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
+    const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kScatterBlock;
+    if (group_base >= n_points) return;
+    const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;
+    const int level = static_cast<int>(pair_level / feat_pairs);  // the geometry's level
+    const float w_level = window[level];
+    if (w_level == 0.0f) return;
+    scatter_begin(state);
+    BinTarget bins = bins_of_level(pass_bins, level_in_pass);
+    if constexpr (!kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
+    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
+                               2 * feat_pairs, bins.direct, bins.bin_shift};
+    // Everything a thread reads lies within its group of at most 16 x 512 points, so the addresses are
+    // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets.
+    const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);
+    const float* const group_positions = positions + group_base * D;
+    const float* const group_q = kNeedsQ ? double_pos_grad + group_base * D : nullptr;
+    const float* const group_grad0 =
+        kRowMajor ? grad_sliced + group_base * grad_row_stride + 2 * pair_level
+                  : grad_sliced + (static_cast<size_t>(pair_level) * 2) * n_points + group_base;
+    const float* const group_grad1 = group_grad0 + n_points;
+    const auto load_grad = [&](uint32_t i, float& g0, float& g1) {
+        if constexpr (kRowMajor) {
+            const float2 g = *reinterpret_cast<const float2*>(group_grad0 + static_cast<int64_t>(i) * grad_row_stride);
+            g0 = g.x;
+            g1 = g.y;
+        } else {
+            g0 = group_grad0[i];
+            g1 = group_grad1[i];
+        }
+    };
+    const float* const group_second0 = kBoth ? second_grad + (static_cast<size_t>(pair_level) * 2) * n_points + group_base : nullptr;
+    const float* const group_second1 = group_second0 + n_points;
+    const auto load_group_point = [&](const float* base, uint32_t i) {
+        fvec<D> v;
+        static_for<D>(PENC_BODY(k) {
+            PENC_INDEX(k); v[k] = base[i * static_cast<uint32_t>(D) + k]; });
+        return v;
+    };
+    // A tile's inputs are fetched one tile ahead: their latency then overlaps the previous tile's
+    // scatter instead of stalling the wave at the top of every iteration.
+    const auto point_of = [&](int t) {  // the point this thread handles in tile t, within the group (clamped: the tail re-reads the last point)
+        const uint32_t i = static_cast<uint32_t>(t) * kScatterBlock + threadIdx.x;
+        return i < last_in_group ? i : last_in_group;
+    };
+    uint32_t nn = point_of(0);
+    fvec<D> pos = load_group_point(group_positions, nn);
+    fvec<D> q = 0.0f;
+    if constexpr (kNeedsQ) q = load_group_point(group_q, nn);
+    float g0, g1;
+    load_grad(nn, g0, g1);
+    float s0 = 0.0f, s1 = 0.0f;
+    if constexpr (kBoth) {
+        s0 = group_second0[nn];
+        s1 = group_second1[nn];
+    }
+    int mode = kModeCache;
+    uint32_t id_bits = 0;
+    for (int t = 0; t < tiles_per_group; ++t) {
+        const int64_t tile_base = group_base + static_cast<int64_t>(t) * kScatterBlock;
+        if (tile_base >= n_points) break;
+        const bool active = tile_base + threadIdx.x < n_points;
+        const uint32_t nn_next = point_of(t + 1);
+        const fvec<D> pos_next = load_group_point(group_positions, nn_next);
+        fvec<D> q_next = 0.0f;
+        if constexpr (kNeedsQ) q_next = load_group_point(group_q, nn_next);
+        float g0_next, g1_next;
+        load_grad(nn_next, g0_next, g1_next);
+        float s0_next = 0.0f, s1_next = 0.0f;
+        if constexpr (kBoth) {
+            s0_next = group_second0[nn_next];
+            s1_next = group_second1[nn_next];
+        }
+        if constexpr (kRowMajor) {
+            if (grad_level_major != nullptr && active) {
+                float* out = grad_level_major + (static_cast<size_t>(pair_level) * 2) * n_points + tile_base + threadIdx.x;
+                out[0] = g0;
+                out[n_points] = g1;
+            }
+        }
+        const Located<D> s = locate<D>(pos, random_shift + level * D, scale_factor + level * D);
+        uvec<D + 1> h;
+        fvec<D + 1> w;   // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
+        fvec<D + 1> w2;  // kBoth: the latter
+        bool via_lds = false;
+        if constexpr (D > kWorkgroupSortMaxDim) {
+            // Once the workgroup streams with every wave sorting on its own (stream_tile_wave), a wave's staging
+            // slice is idle between its tiles and nobody else touches it: it serves as the thread-private
+            // columns that put residuals and hash steps into rank order, in place of D(D+1) selects each
+            // (at D = 8 about 270 of 1350 vector instructions per point and level).
+            via_lds = mode == kModeStream && bins.n_bins <= static_cast<uint32_t>(kStageBins);
+        }
+        if (via_lds) {
+            constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D)>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
+            static_assert((D + 1) * 64 <= kSliceCells, "a wave's staging slice holds a column of D+1 cells per lane");
+            uint2* const column = reinterpret_cast<uint2*>(state.val) + (threadIdx.x >> 6) * kSliceCells + (threadIdx.x & 63);
+            fvec<D + 1> sorted;
+            if constexpr (kBoth) {
+                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
+                w = barycentric_of_sorted<D>(sorted) * w_level;
+                wave_lds_fence();
+                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
+                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
+            } else if constexpr (kOrder == kSecondOrder) {
+                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
+                w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
+            } else {
+                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
+                w = barycentric_of_sorted<D>(sorted) * w_level;
+            }
+            wave_lds_fence();  // the slice is staging space again from here on
+        } else {
+            h = vertex_hashes<D>(s.rank, s.hash0);
+            if constexpr (kBoth) {
+                w = barycentric<D>(s.rank, s.delta) * w_level;
+                w2 = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
+            } else if constexpr (kOrder == kSecondOrder) {
+                w = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
+            } else {
+                w = barycentric<D>(s.rank, s.delta) * w_level;
+            }
+        }
+        uvec<D + 1> slot;
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            slot[r] = to_slot(h[r], capacity, cap_mask);
+        });
+        if (t == 0) {
+            // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
+            // (its point is already here)
+            const auto slots_of_next_tile = [&]() {
+                const Located<D> s1 = locate<D>(pos_next, random_shift + level * D, scale_factor + level * D);
+                const uvec<D + 1> h1 = vertex_hashes<D>(s1.rank, s1.hash0);
+                uvec<D + 1> slot1;
+                static_for<D + 1>(PENC_BODY(r) {
+                    PENC_INDEX(r);
+                    slot1[r] = to_slot(h1[r], capacity, cap_mask);
+                });
+                return slot1;
+            };
+            const bool next_active = tile_base + kScatterBlock + threadIdx.x < n_points && tiles_per_group > 1;
+            mode = scatter_mode_decide<D>(state, bins, active, slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
+        }
+        fvec<D + 1> a0 = w * g0, a1 = w * g1;  // g_f * (b_r * w_level), :405-410
+        if constexpr (kBoth) {
+            a0 += w2 * s0;
+            a1 += w2 * s1;
+        }
+        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1);
+        // the first tile finds the lines its own look-up has claimed: no evidence of reuse
+        if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
+        pos = pos_next;
+        q = q_next;
+        g0 = g0_next;
+        g1 = g1_next;
+        s0 = s0_next;
+        s1 = s1_next;
+    }
+    scatter_end(state, level_grad, bins, group, mode, id_bits);
+}
+
+#define PENC_TABLE_PARAMETERS                                                                                                          \
+    int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group, uint32_t capacity, \
+        uint32_t cap_mask, const float *__restrict__ positions, const float *__restrict__ scale_factor,                                \
+        const float *__restrict__ random_shift, const float *__restrict__ window, const float *__restrict__ grad_sliced,               \
+        int64_t grad_row_stride, const float *__restrict__ double_pos_grad, const float *__restrict__ second_grad,                     \
+        float *__restrict__ table_grad, float *__restrict__ grad_level_major, BinTarget pass_bins
+#define PENC_TABLE_ARGUMENTS                                                                                                        \
+    n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
+        random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
+template <int D, bool kRowMajor, bool kSecond, bool kWideBins>
+__global__ void __launch_bounds__(kScatterBlock, scatter_waves_per_simd(D, kSecond, kWideBins))
+backward_table_kernel(PENC_TABLE_PARAMETERS) {
+    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins>(PENC_TABLE_ARGUMENTS);
+}
+template <int D, bool kRowMajor, bool kWideBins>
+__global__ void __launch_bounds__(kScatterBlock, both_orders_waves_per_simd(D, kWideBins))
+backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
+    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins>(PENC_TABLE_ARGUMENTS);
+}
+#undef PENC_TABLE_PARAMETERS
+#undef PENC_TABLE_ARGUMENTS
+
+template <int D>
+void launch_table_backward(const TableLaunch& t) {
+#define PENC_LAUNCH(...)                                                                                                              \
+    hipLaunchKernelGGL((__VA_ARGS__), t.grid, dim3(kScatterBlock), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,            \
+                       t.feat_pairs, t.dies, t.tiles_per_group, t.capacity, t.cap_mask, t.positions, t.scale_factor, t.random_shift,  \
+                       t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad, t.table_grad, t.grad_level_major, t.bins)
+#define PENC_LAUNCH_WIDTH(KERNEL, ...)           \
+    if (t.wide_bins) {                           \
+        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, true>);   \
+    } else {                                     \
+        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false>);  \
+    }
+    if (t.second_grad != nullptr) {
+        if (t.rows) {
+            PENC_LAUNCH_WIDTH(backward_table_both_kernel, true);
+        } else {
+            PENC_LAUNCH_WIDTH(backward_table_both_kernel, false);
+        }
+    } else if (t.second_order) {
+        if (t.rows) {
+            PENC_LAUNCH_WIDTH(backward_table_kernel, true, true);
+        } else {
+            PENC_LAUNCH_WIDTH(backward_table_kernel, false, true);
+        }
+    } else if (t.rows) {
+        PENC_LAUNCH_WIDTH(backward_table_kernel, true, false);
+    } else {
+        PENC_LAUNCH_WIDTH(backward_table_kernel, false, false);
+    }
+#undef PENC_LAUNCH_WIDTH
+#undef PENC_LAUNCH
+}
+
+template void launch_table_backward<PENC_DIM>(const TableLaunch& t);
+
+}  // namespace penc

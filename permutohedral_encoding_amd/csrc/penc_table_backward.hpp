@@ -1,0 +1,29 @@
+// The launch of the scattering kernel, one translation unit per input dimension (penc_table_backward.hip compiled
+// with -DPENC_DIM=2 ... 8): the kernel has a dozen instances per dimension, and the units compile side by side.
+#pragma once
+
+#include "penc_scatter.hpp"
+
+namespace penc {
+
+struct TableLaunch {
+    dim3 grid;
+    hipStream_t stream;
+    bool rows;          // the upstream gradient is read as rows
+    bool second_order;  // double_pos_grad is given; with second_grad too, both orders
+    bool wide_bins;
+    int n_points, first_level;
+    uint32_t n_pass_levels, feat_pairs, dies;
+    int tiles_per_group;
+    uint32_t capacity, cap_mask;
+    const float *positions, *scale_factor, *random_shift, *window, *grad;
+    int64_t grad_row_stride;
+    const float *double_pos_grad, *second_grad;
+    float *table_grad, *grad_level_major;
+    BinTarget bins;
+};
+
+template <int D>
+void launch_table_backward(const TableLaunch& t);
+
+}  // namespace penc
