@@ -297,6 +297,12 @@ int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, in
                               const float* double_positions_grad, const float* first_grad, float* lattice_values_grad,
                               uint32_t* touched, float* positions_grad, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Copies n values from HOST memory to dst as part of the enqueued work: the values travel in the launch (128 at a time), so the
+ * call neither waits for the device nor needs the host array afterwards, where a copy from pageable memory
+ * does both.  For the few values that change from step to step (the window of a coarse-to-fine schedule).
+ * Replaces: the blocking `anneal_window.cuda()` of src/pytorch_modules/modules.py:77. */
+int penc_upload(const float* host_values, float* dst, int n, void* stream);
+
 /* dst[c][r] = src[r][c] for a dense row-major rows x cols matrix with cols <= 255 (2 * levels):
  * turns the row-major upstream gradient (N, 2(L+E)) into the grad_sliced_values layout
  * [L+E][2][N] at streaming speed.

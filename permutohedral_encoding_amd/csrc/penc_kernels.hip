@@ -520,6 +520,16 @@ transpose_to_rows_kernel(const float* __restrict__ src, float* __restrict__ dst,
     }
 }
 
+// A few host values into device memory, carried by the launch itself (penc_upload).
+constexpr int kUploadValues = 128;
+struct UploadValues {
+    float v[kUploadValues];
+};
+__global__ void __launch_bounds__(kUploadValues) upload_kernel(UploadValues values, int n, float* __restrict__ dst) {
+    const int i = threadIdx.x;
+    if (i < n) dst[i] = values.v[i];
+}
+
 // Clears two arrays (the second may be empty): n2 and m2 count 8-byte units.
 __global__ void __launch_bounds__(kBlock) fill_zero_kernel(float2* __restrict__ p, size_t n2, float2* __restrict__ q, size_t m2) {
     const size_t stride = static_cast<size_t>(gridDim.x) * kBlock, first = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x;
@@ -1502,6 +1512,19 @@ int penc_adamw_step_sparse(float* params, float* grads, float* exp_avg, float* e
 int penc_clear_touched(float* grads, int nr_feat, int nr_levels, int capacity, uint32_t* touched, void* stream) {
     return launch_touched_ranges(false, nullptr, grads, nullptr, nullptr, nr_feat, nr_levels, capacity, touched, AdamWStep{}, 1,
                                  stream);
+}
+
+int penc_upload(const float* host_values, float* dst, int n, void* stream) {
+    if (!host_values || !dst) return PENC_ERR_NULL_POINTER;
+    if (n <= 0) return PENC_ERR_BAD_SIZE;
+    for (int first = 0; first < n; first += kUploadValues) {
+        UploadValues values;
+        const int count = n - first < kUploadValues ? n - first : kUploadValues;
+        __builtin_memcpy(values.v, host_values + first, static_cast<size_t>(count) * sizeof(float));
+        hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(kUploadValues), 0, static_cast<hipStream_t>(stream), values, count, dst + first);
+        if (int rc = check_launch()) return rc;
+    }
+    return PENC_OK;
 }
 
 int penc_transpose(const float* src, float* dst, int64_t rows, int cols, void* stream) {

@@ -63,6 +63,7 @@ struct Api {
     PENC_FN(adamw_step);
     PENC_FN(adamw_step_sparse);
     PENC_FN(transpose);
+    PENC_FN(upload);
 #undef PENC_FN
 } api;
 
@@ -563,6 +564,17 @@ void prepare_call(Call& c, const Tensor& positions, const Tensor& window) {
     c.extra = api.extra_levels(c.pos_dim, c.feat, c.concat);
 }
 
+// A schedule hands its window over in host memory, once per step: copied by a launch, without waiting for the device.
+Tensor window_on_device(const Tensor& window, const at::Device& device) {
+    constexpr int64_t kMost = 1024;
+    if (!window.device().is_cpu() || window.dim() != 1 || window.numel() == 0 || window.numel() > kMost) return window.to(device, at::kFloat);
+    const Tensor host = window.to(at::kFloat).contiguous();
+    const c10::DeviceGuard guard(device);
+    Tensor out = at::empty({host.numel()}, host.options().device(device));
+    check(api.upload(data(host), mutable_data(out), static_cast<int>(host.numel()), current_stream(device)), "upload");
+    return out;
+}
+
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
 //        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None) -> (N, F(L+E))
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
@@ -594,7 +606,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         {
             NoGil no_gil;
             at::NoGradGuard no_grad;
-            if (positions.is_cuda()) window = window.to(positions.device(), at::kFloat);
+            if (positions.is_cuda()) window = window_on_device(window, positions.device());
             prepare_call(c, positions, window);
             const c10::DeviceGuard device(c.device());
             out = compute_forward(c);
@@ -681,6 +693,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(adamw_step);
         PENC_FN(adamw_step_sparse);
         PENC_FN(transpose);
+        PENC_FN(upload);
 #undef PENC_FN
         Py_RETURN_NONE;
     });

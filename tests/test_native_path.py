@@ -168,3 +168,13 @@ def test_both_orders_in_one_scatter_match_the_oracle(d, n, levels, cap, rows, fe
     assert_sum_close(tg.cpu().numpy(), a["grad64"] + b["grad64"], a["abs64"] + b["abs64"], 1e-4, "both table gradients")
     wp = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], p["window"], p["grad"])
     assert np.all(np.abs(pg.cpu().numpy() - wp["grad64"]) <= 1e-6 * wp["abs64"] + 1e-30)
+
+
+@pytest.mark.parametrize("n", [1, 24, 128, 129, 300])
+def test_upload_carries_host_values_in_the_launch(n):
+    from permutohedral_encoding_amd import _native
+    host = torch.randn(n)
+    want, dst = host.clone(), torch.full((n + 1,), 7.0, device="cuda")
+    rc = _native.lib().penc_upload(host.data_ptr(), dst.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+    host.zero_()  # the caller's array is its own again
+    assert rc == 0 and torch.equal(dst[:n].cpu(), want) and dst[n].item() == 7.0
