@@ -25,6 +25,13 @@ class AdamW(torch.optim.Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay,
                                       skip_zero_gradients=bool(skip_zero_gradients)))
 
+    def zero_grad(self, set_to_none=True):
+        if not set_to_none:
+            return super().zero_grad(set_to_none=False)
+        for group in self.param_groups:
+            for p in group["params"]:
+                p.grad = None
+
     @torch.no_grad()
     def step(self, closure=None):
         loss = None
