@@ -116,6 +116,12 @@ struct LevelMap {
     uint32_t segment;  // (row, tile) pairs per segment; 0: the grid is (tile, row)
     uint32_t dies;
 };
+// Whether any level of a row (row, row + rows, ...) has a window weight other than 0.
+__device__ __forceinline__ bool row_has_level(const float* __restrict__ window, uint32_t row, uint32_t rows, int n_levels) {
+    for (uint32_t level = row; level < static_cast<uint32_t>(n_levels); level += rows)
+        if (window[level] != 0.0f) return true;
+    return false;
+}
 __device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile, uint32_t& row) {
     if (map.segment == 0u) {
         tile = blockIdx.x;
@@ -218,6 +224,8 @@ backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity,
     if (!locate_work(map, tile, row)) return;
     const int n = tile * kBlock + threadIdx.x;
     if (n >= n_points) return;
+    // (with a coarse-to-fine window half the groups can be masked: nothing is stored for them, and the reduction skips them)
+    if (map.rows > 1u && !row_has_level(window, row, map.rows, n_levels)) return;
     const fvec<D> pos = load_point<D>(positions, n);
     fvec<D> total = 0.0f;
     // The levels of a group are `rows` apart, not adjacent: with the usual coarse-to-fine level list a
@@ -248,13 +256,42 @@ backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity,
     });
 }
 
+// Sums the partial position gradients of the groups in ascending order, one value to a thread.  What it waits for at small sizes
+// is its chain of loads: those of kTogether groups are issued together, the groups that have stored anything (a masked one has
+// not) being known beforehand (2^15 points, 12 groups: 11.5 -> 3.9 us; large sums are bound by the memory, 2^20 points 31 us).
+// (16 bytes to a lane are slower, 50 us: the groups' sums lie a multiple of the memory's interleave apart, and loads of
+// several groups from the same few waves meet on one channel.)
 __global__ void __launch_bounds__(kBlock)
-reduce_level_groups_kernel(const float* __restrict__ partial, int n_groups, size_t n_values, float* __restrict__ out) {
+reduce_level_groups_kernel(const float* __restrict__ partial, const float* __restrict__ window, int n_groups, int n_levels,
+                           size_t n_values, float* __restrict__ out) {
+    constexpr int kTogether = 8;
     const size_t stride = static_cast<size_t>(gridDim.x) * kBlock;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < n_values; i += stride) {
-        float acc = partial[i];
-        for (int g = 1; g < n_groups; ++g) acc += partial[static_cast<size_t>(g) * n_values + i];
-        out[i] = acc;
+    for (size_t first_value = static_cast<size_t>(blockIdx.x) * kBlock; first_value < n_values; first_value += stride) {
+        const size_t i = first_value + threadIdx.x, at = i < n_values ? i : n_values - 1;
+        float acc = 0.0f;
+        bool first = true;
+        for (int base = 0; base < n_groups; base += 64) {
+            const int mine = base + static_cast<int>(threadIdx.x & 63);  // (all 64 lanes are here, also those past the last value)
+            unsigned long long live = __ballot(
+                mine < n_groups && row_has_level(window, static_cast<uint32_t>(mine), static_cast<uint32_t>(n_groups), n_levels));
+            while (live != 0ull) {
+                const int count = __popcll(live);
+                float v[kTogether];
+#pragma unroll
+                for (int u = 0; u < kTogether; ++u) {
+                    v[u] = 0.0f;
+                    if (live != 0ull) v[u] = partial[static_cast<size_t>(base + __builtin_ctzll(live)) * n_values + at];
+                    live &= live - 1ull;
+                }
+#pragma unroll
+                for (int u = 0; u < kTogether; ++u) {
+                    if (u >= count) break;
+                    acc = first ? v[u] : acc + v[u];
+                    first = false;
+                }
+            }
+        }
+        if (i < n_values) out[i] = acc;
     }
 }
 
@@ -994,9 +1031,11 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
                                          grad_level_major, partial));
     if (int rc = check_launch()) return rc;
     if (groups > 1) {
-        const size_t want = (n_values + kBlock * 4 - 1) / (kBlock * 4);
-        hipLaunchKernelGGL(reduce_level_groups_kernel, dim3(static_cast<unsigned>(want < 8192 ? want : 8192)), dim3(kBlock),
-                           0, st, partial, groups, n_values, positions_grad);
+        // four values to a thread where that still fills the chip
+        const size_t per_block = kBlock * (n_values >= size_t{1} << 19 ? 4 : 1);
+        const size_t want = (n_values + per_block - 1) / per_block;
+        hipLaunchKernelGGL(reduce_level_groups_kernel, dim3(static_cast<unsigned>(want < 8192 ? want : 8192)), dim3(kBlock), 0, st, partial,
+                           anneal_window, groups, nr_levels, n_values, positions_grad);
         if (int rc = check_launch()) return rc;
     }
     return PENC_OK;
