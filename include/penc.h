@@ -282,6 +282,26 @@ int penc_adamw_step_sparse(float* params, float* grads, float* exp_avg, float* e
                            double weight_decay, int64_t step, int clear, void* stream);
 int penc_clear_touched(float* grads, int nr_feat, int nr_levels, int capacity, uint32_t* touched, void* stream);
 
+/* The two halves of a double backward for an upstream gradient that is rows, where the caller keeps the level-major copy:
+ * penc_backward_positions_rowmajor is penc_backward_rowmajor for the position gradient alone, with the [L][F][N] copy of
+ * the upstream gradient left in grad_level_major (for the scattering half of the double backward, which reads it a level at a
+ * time); `workspace` as in penc_backward (penc_positions_workspace_bytes).  penc_grad_grad_rowmajor is the gathering half of
+ * penc_double_backward_from_positions with its result as rows grad_grad_rows[n][F*level + feature] of row_stride floats;
+ * `workspace` must hold the [L+E][F][N] array (penc_forward_rowmajor_workspace_bytes).
+ * table_format: 0 for an fp32 table, else as in the *_half entry points.
+ * Replaces: funcs.py:47's copy, backward_gpu_only_pos (EncodingGPU.cuh:530-769) and double_backward_from_positions_gpu_2
+ * (EncodingGPU.cuh:1260-1493) with the transpose its result takes on the way into row-major storage. */
+int penc_backward_positions_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                                     const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                                     const float* random_shift, const float* anneal_window, const float* grad_rows,
+                                     int64_t grad_row_stride, float* grad_level_major, float* positions_grad, void* workspace,
+                                     size_t workspace_bytes, void* stream);
+int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                            const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                            const float* random_shift, const float* anneal_window, const float* double_positions_grad,
+                            float* grad_grad_rows, int64_t row_stride, int concat_points, void* workspace, size_t workspace_bytes,
+                            void* stream);
+
 /* The two table gradients of a training step on an SDF in one pass: that of a loss on the encoded values, whose
  * upstream gradient is `grad` (grad_row_stride 0 or a row stride, as in penc_backward_half), plus that of a loss on the position
  * gradient a first backward has returned (double_positions_grad; `first_grad` [L+E][F][N] is what that backward was

@@ -350,6 +350,121 @@ grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uin
 }
 
 // ------------------------------------------------------------------------------------------
+// all levels of a block of points in one workgroup
+//
+// A workgroup takes 64 points and all their levels: lane = point, wave w takes levels w, w + kBlockWaves, ...  What needs
+// several launches at a level a time is one here: the sum of the position gradient over the levels happens in LDS, and rows
+// (of a result, or of an upstream gradient) pass through an LDS tile, so no transpose precedes or follows.  Every die then gathers
+// from every level, which is why this is for tables an L2 holds as a whole and for batches whose time is launches and latency
+// (takes_point_blocks says where the lines lie).
+constexpr int kBlockWaves = 8, kBlockPoints = 64, kPointBlock = kBlockWaves * kBlockPoints;
+
+// Position gradient.  The upstream gradient is [level][feature][n], or (kRows) rows of `grad_row_stride` floats, of which the
+// [level][feature][n] copy is left in grad_level_major when the caller wants it.
+template <int D, int F, typename T, bool kRows>
+__global__ void __launch_bounds__(kPointBlock)
+block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
+                          const T* __restrict__ table, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
+                          const float* __restrict__ window, const float* __restrict__ grad, int64_t grad_row_stride,
+                          float* __restrict__ grad_level_major, float* __restrict__ out) {
+    extern __shared__ float tile[];  // rows: kBlockPoints x (columns | 1)
+    __shared__ float partial[kBlockWaves][kBlockPoints * D];
+    const int base = blockIdx.x * kBlockPoints, count = n_points - base < kBlockPoints ? n_points - base : kBlockPoints;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int columns = n_levels * F, pitch = columns | 1;
+    const int n = base + (lane < count ? lane : count - 1);
+    const fvec<D> pos = load_point<D>(positions, n);
+    if constexpr (kRows) {
+        const float* const rows = grad + static_cast<int64_t>(base) * grad_row_stride;
+        for (int r = wave; r < count; r += kBlockWaves)
+            for (int c = lane; c < columns; c += 64) tile[r * pitch + c] = rows[r * grad_row_stride + c];
+        __syncthreads();
+        if (grad_level_major != nullptr && lane < count)
+            for (int c = wave; c < columns; c += kBlockWaves) grad_level_major[static_cast<size_t>(c) * n_points + n] = tile[lane * pitch + c];
+    }
+    const int row = n - base;
+    fvec<D> total = 0.0f;
+    for (int level = wave; level < n_levels; level += kBlockWaves) {
+        const float w_level = window[level];
+        if (w_level == 0.0f) continue;
+        const float* sf = scale_factor + level * D;
+        const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
+        const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
+        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+        const auto upstream = [&](int k) {
+            if constexpr (kRows) return tile[row * pitch + level * F + k];
+            else return grad[(static_cast<size_t>(level) * F + k) * n_points + n];
+        };
+        fvec<D + 1> dB = (v.f[0] * w_level) * upstream(0);  // :688-689, feature by feature
+        static_for<F - 1>(PENC_BODY(kk) {
+            PENC_INDEX(kk);
+            dB += (v.f[kk + 1] * w_level) * upstream(kk + 1);
+        });
+        total += bary_grad_to_pos_grad<D>(s.rank, dB, sf);
+    }
+    static_for<D>(PENC_BODY(i) {
+        PENC_INDEX(i);
+        partial[wave][lane * D + i] = total[i];
+    });
+    __syncthreads();
+    for (int i = threadIdx.x; i < count * D; i += kPointBlock) {
+        float acc = partial[0][i];
+#pragma unroll
+        for (int w = 1; w < kBlockWaves; ++w) acc += partial[w][i];
+        out[static_cast<size_t>(base) * D + i] = acc;
+    }
+}
+
+// The forward (kSecond = false) or the gradient w.r.t. the upstream gradient (kSecond = true) as rows of `row_stride` floats.
+template <int D, int F, typename T, bool kSecond>
+__global__ void __launch_bounds__(kPointBlock)
+block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
+                  const T* __restrict__ table, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
+                  const float* __restrict__ window, const float* __restrict__ double_pos_grad, float points_scaling,
+                  float* __restrict__ rows, int64_t row_stride) {
+    extern __shared__ float tile[];  // kBlockPoints x (columns | 1)
+    const int base = blockIdx.x * kBlockPoints, count = n_points - base < kBlockPoints ? n_points - base : kBlockPoints;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int columns = n_all_levels * F, pitch = columns | 1;
+    const int n = base + (lane < count ? lane : count - 1);
+    const fvec<D> pos = load_point<D>(positions, n);
+    fvec<D> q = 0.0f;
+    if constexpr (kSecond) q = load_point<D>(double_pos_grad, n);
+    float* const mine = tile + lane * pitch;
+    for (int level = wave; level < n_all_levels; level += kBlockWaves) {
+        if (level >= n_levels) {  // extra levels: the raw positions (:106-121), or zeros (:1290-1295)
+            const int src = (level - n_levels) * F;
+            const float* p = positions + static_cast<size_t>(n) * D;
+            static_for<F>(PENC_BODY(k) {
+                PENC_INDEX(k);
+                mine[level * F + k] = !kSecond && src + k < D ? p[src + k] * points_scaling : 0.0f;
+            });
+            continue;
+        }
+        const float w_level = window[level];
+        fvec<F> acc = 0.0f;
+        if (w_level != 0.0f) {
+            const float* sf = scale_factor + level * D;
+            const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
+            const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
+            const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+            const fvec<D + 1> w = kSecond ? pos_grad_grad_to_bary<D>(s.rank, q, sf) * w_level : barycentric<D>(s.rank, s.delta) * w_level;
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r);
+                static_for<F>(PENC_BODY(k) {
+                    PENC_INDEX(k); acc[k] = acc[k] + v.f[k][r] * w[r]; });
+            });
+        }
+        static_for<F>(PENC_BODY(k) {
+            PENC_INDEX(k); mine[level * F + k] = acc[k]; });
+    }
+    __syncthreads();
+    float* const to = rows + static_cast<int64_t>(base) * row_stride;
+    for (int r = wave; r < count; r += kBlockWaves)
+        for (int c = lane; c < columns; c += 64) to[r * row_stride + c] = tile[r * pitch + c];
+}
+
+// ------------------------------------------------------------------------------------------
 // optimiser step on the table
 
 // One fused AdamW update (decoupled weight decay, no amsgrad) in the order torch.optim.AdamW applies
@@ -1004,6 +1119,56 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     return PENC_OK;
 }
 
+// Whether a call takes the kernels that keep all levels of 64 points in a workgroup, where the LDS holds their rows.  Always
+// when an L2 of 4 MiB holds most of the table (position gradient, D = 3, 17 levels of 2^14 slots, 2^20 points: 246 -> 174 us,
+// 2^16 points 21.5 -> 13.1; forward in rows 223 -> 171 and 21.2 -> 14.3); up to 12 M gathers where it holds a third (D = 4, 16
+// levels of 2^16 slots: position gradient from rows 2^17 points 50.5 -> 44.8 us, 2^20 points 316 -> 352); else as long as every
+// die fetching the slices it needs of the whole table costs less than the launches saved (D = 3, 24 levels of 2^18 slots:
+// 4097 points 13.2 -> 9.6 us, 2^14 points 18.4 -> 16.0, 2^15 points 25.5 -> 26.1).
+constexpr size_t kBlocksTableBytes = size_t{6} << 20, kBlocksMidTableBytes = size_t{12} << 20;
+constexpr int64_t kBlocksMaxGathers = 1500000, kBlocksMidMaxGathers = 12000000;
+constexpr int kBlocksMaxColumns = 255;
+static bool takes_point_blocks(int pos_dim, int64_t n, int levels, int capacity, int nr_feat, int columns, int table_format) {
+    if (columns > kBlocksMaxColumns) return false;
+    const size_t table = static_cast<size_t>(levels) * slice_bytes(capacity, nr_feat, table_format);
+    if (table <= kBlocksTableBytes) return true;
+    return n * levels * (pos_dim + 1) <= (table <= kBlocksMidTableBytes ? kBlocksMidMaxGathers : kBlocksMaxGathers);
+}
+static size_t block_tile_bytes(int columns) { return static_cast<size_t>(kBlockPoints) * (columns | 1) * sizeof(float); }
+static unsigned point_blocks(int64_t n) { return static_cast<unsigned>((n + kBlockPoints - 1) / kBlockPoints); }
+
+static int block_positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                                    const TableRef& table, const float* scale_factor, const float* random_shift,
+                                    const float* anneal_window, const float* grad, int64_t grad_row_stride, float* grad_level_major,
+                                    float* positions_grad, hipStream_t st) {
+#define PENC_LAUNCH_BLOCKS(ROWS, LDS)                                                                                                       \
+    PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,                                                                                      \
+                      hipLaunchKernelGGL((block_backward_pos_kernel<DD, FF, TT, ROWS>), dim3(point_blocks(nr_positions)),                  \
+                                         dim3(kPointBlock), LDS, st, static_cast<int>(nr_positions), nr_levels,                            \
+                                         static_cast<uint32_t>(capacity), mask_of(capacity), positions, static_cast<const TT*>(table.values), \
+                                         scale_factor, random_shift, anneal_window, grad, grad_row_stride, grad_level_major, positions_grad))
+    if (grad_row_stride != 0) {
+        PENC_LAUNCH_BLOCKS(true, block_tile_bytes(nr_levels * nr_feat));
+    } else {
+        PENC_LAUNCH_BLOCKS(false, 0);
+    }
+#undef PENC_LAUNCH_BLOCKS
+    return check_launch();
+}
+
+template <bool kSecond>
+static int block_rows(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int extra, int capacity, const float* positions,
+                      const TableRef& table, const float* scale_factor, const float* random_shift, const float* anneal_window,
+                      const float* double_positions_grad, float points_scaling, float* rows, int64_t row_stride, hipStream_t st) {
+    PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
+                      hipLaunchKernelGGL((block_rows_kernel<DD, FF, TT, kSecond>), dim3(point_blocks(nr_positions)), dim3(kPointBlock),
+                                         block_tile_bytes((nr_levels + extra) * nr_feat), st, static_cast<int>(nr_positions), nr_levels,
+                                         nr_levels + extra, static_cast<uint32_t>(capacity), mask_of(capacity), positions,
+                                         static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
+                                         double_positions_grad, points_scaling, rows, row_stride));
+    return check_launch();
+}
+
 // The position gradient of penc_backward / penc_backward_rowmajor from a level-major upstream gradient:
 // levels in groups of pos_levels_per_group() when the workspace can hold the partial sums, else one
 // thread per point walks all levels.
@@ -1011,6 +1176,9 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
                               const TableRef& table, const float* scale_factor, const float* random_shift,
                               const float* anneal_window, const float* grad_level_major, float* positions_grad,
                               void* workspace, size_t workspace_bytes, hipStream_t st) {
+    if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, nr_levels * nr_feat, table.format))
+        return block_positions_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
+                                        anneal_window, grad_level_major, 0, nullptr, positions_grad, st);
     const int n = static_cast<int>(nr_positions);
     const uint32_t cap = static_cast<uint32_t>(capacity), mask = mask_of(capacity);
     const size_t n_values = static_cast<size_t>(nr_positions) * pos_dim;
@@ -1189,6 +1357,13 @@ int penc_forward_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
     const size_t need = static_cast<size_t>(cols) * static_cast<size_t>(nr_positions) * sizeof(float);
     if (workspace == nullptr || workspace_bytes < (base - reinterpret_cast<uintptr_t>(workspace)) + need) return PENC_ERR_WORKSPACE_TOO_SMALL;
+    if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, 0)) {
+        if (!positions || !lattice_values || !scale_factor || !random_shift || !anneal_window) return PENC_ERR_NULL_POINTER;
+        const TableRef table{lattice_values, 0};
+        if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+        return block_rows<false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                 anneal_window, nullptr, points_scaling, sliced_rows, row_stride, static_cast<hipStream_t>(stream));
+    }
     float* level_major = reinterpret_cast<float*>(base);
     if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values, 0}, scale_factor,
                               random_shift, anneal_window, level_major, concat_points, points_scaling, stream))
@@ -1296,6 +1471,9 @@ static int backward_rowmajor_impl(int pos_dim, int nr_feat, int64_t nr_positions
             return rc;
     } else {
         const int cols = nr_feat * nr_levels;
+        if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format))  // straight from the rows
+            return block_positions_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
+                                            random_shift, anneal_window, grad_rows, grad_row_stride, nullptr, positions_grad, st);
         if (cols > 255) return PENC_ERR_BAD_SIZE;
         if (int rc = transpose_rows(grad_rows, grad_row_stride, level_major, nr_positions, cols, st)) return rc;
     }
@@ -1430,6 +1608,57 @@ int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, in
     return backward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
                          anneal_window, grad, lattice_values_grad, positions_grad, workspace, workspace_bytes, stream, touched,
                          second);
+}
+
+int penc_backward_positions_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                                     const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                                     const float* random_shift, const float* anneal_window, const float* grad_rows,
+                                     int64_t grad_row_stride, float* grad_level_major, float* positions_grad, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0)) return rc;
+    const TableRef table{lattice_values, table_format};
+    if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !grad_level_major || !positions_grad)
+        return PENC_ERR_NULL_POINTER;
+    if (int rc = check_rows(grad_rows, grad_row_stride, nr_positions, nr_levels, nr_feat)) return rc;
+    if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int cols = nr_feat * nr_levels;
+    if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format))
+        return block_positions_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
+                                        anneal_window, grad_rows, grad_row_stride, grad_level_major, positions_grad, st);
+    if (int rc = transpose_rows(grad_rows, grad_row_stride, grad_level_major, nr_positions, cols, st)) return rc;
+    return positions_backward(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
+                              anneal_window, grad_level_major, positions_grad, workspace, workspace_bytes, st);
+}
+
+int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
+                            const float* positions, const void* lattice_values, int table_format, const float* scale_factor,
+                            const float* random_shift, const float* anneal_window, const float* double_positions_grad,
+                            float* grad_grad_rows, int64_t row_stride, int concat_points, void* workspace, size_t workspace_bytes,
+                            void* stream) {
+    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points);
+    if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
+    const TableRef table{lattice_values, table_format};
+    if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !double_positions_grad || !grad_grad_rows)
+        return PENC_ERR_NULL_POINTER;
+    const int cols = nr_feat * (nr_levels + extra);
+    if (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31)) return PENC_ERR_BAD_SIZE;
+    if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format))
+        return block_rows<true>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                anneal_window, double_positions_grad, 1.0f, grad_grad_rows, row_stride, st);
+    const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
+    const size_t need = static_cast<size_t>(cols) * static_cast<size_t>(nr_positions) * sizeof(float);
+    if (workspace == nullptr || workspace_bytes < (base - reinterpret_cast<uintptr_t>(workspace)) + need) return PENC_ERR_WORKSPACE_TOO_SMALL;
+    float* const level_major = reinterpret_cast<float*>(base);
+    if (int rc = double_backward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift,
+                                      anneal_window, double_positions_grad, /* read by the table half only */ level_major, 0, nullptr,
+                                      level_major, concat_points, nullptr, 0, stream))
+        return rc;
+    return transpose_to_rows(level_major, grad_grad_rows, row_stride, nr_positions, cols, st);
 }
 
 // The scalars of one AdamW step as torch.optim.AdamW forms them (in double), rounded once for the kernel.

@@ -19,6 +19,7 @@
 #include <dlfcn.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/graph_task.h>
+#include <torch/csrc/autograd/functions/accumulate_grad.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -65,6 +66,8 @@ struct Api {
     PENC_FN(adamw_step_sparse);
     PENC_FN(transpose);
     PENC_FN(upload);
+    PENC_FN(backward_positions_rowmajor);
+    PENC_FN(grad_grad_rowmajor);
 #undef PENC_FN
 } api;
 
@@ -307,16 +310,47 @@ Gradients compute_backward(const Call& c, const Upstream& up, bool want_table, b
     return g;
 }
 
+Tensor checked_double_positions_grad(const Call& c, const Tensor& double_positions_grad) {
+    require_f32_gpu(double_positions_grad, "double_positions_grad", 2);
+    PENC_REQUIRE(double_positions_grad.size(0) == c.n && double_positions_grad.size(1) == c.pos_dim,
+                 "double_positions_grad should be nr_positions x pos_dim");
+    return double_positions_grad.detach().contiguous();
+}
+
+// The position gradient alone, from rows, whose level-major copy outlives the call: the double backward's scatter reads it too
+// (coalesced, where rows cost it a sixth of its time) and can be deferred.
+Gradients compute_positions_backward(const Call& c, Upstream& up) {
+    Gradients g;
+    g.positions = at::empty({c.n, c.pos_dim}, c.positions.options());
+    Tensor level_major = level_major_array(c);
+    const Tensor ws = gradient_workspace(c, false, true, 0);
+    check(api.backward_positions_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(),
+                                          c.table_format, data(c.scale_factor), data(c.shift), data(c.window), data(up.values),
+                                          up.row_stride, mutable_data(level_major), mutable_data(g.positions), workspace_of(ws),
+                                          workspace_size(ws), current_stream(c.device())),
+          "backward_positions");
+    up = {level_major, 0};
+    return g;
+}
+
+// The gradient w.r.t. an upstream gradient, as dense rows.
+Tensor compute_grad_grad_rows(const Call& c, const Tensor& double_positions_grad) {
+    Tensor rows = at::empty({c.n, c.columns()}, c.positions.options());
+    const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
+    check(api.grad_grad_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                                 data(c.scale_factor), data(c.shift), data(c.window), data(double_positions_grad), mutable_data(rows),
+                                 c.columns(), c.concat, workspace_of(ws), workspace_size(ws), current_stream(c.device())),
+          "grad_grad");
+    return rows;
+}
+
 struct SecondOrder {
     Tensor table, upstream;  // gradients w.r.t. the table (undefined as above) and w.r.t. the upstream gradient
 };
 
 SecondOrder compute_double_backward(const Call& c, const Tensor& double_positions_grad, const Upstream& up, bool want_table,
                                     bool want_upstream) {
-    require_f32_gpu(double_positions_grad, "double_positions_grad", 2);
-    PENC_REQUIRE(double_positions_grad.size(0) == c.n && double_positions_grad.size(1) == c.pos_dim,
-                 "double_positions_grad should be nr_positions x pos_dim");
-    const Tensor dpos = double_positions_grad.contiguous();
+    const Tensor dpos = checked_double_positions_grad(c, double_positions_grad);
     void* const stream = current_stream(c.device());
     SecondOrder s;
     if (want_upstream) s.upstream = level_major_array(c);
@@ -361,6 +395,14 @@ SecondOrder compute_double_backward(const Call& c, const Tensor& double_position
 constexpr const char* kSecondTime =
     "Trying to backward through the graph a second time (or directly access saved tensors after they have already been freed). "
     "Specify retain_graph=True if you need to backward through the graph a second time.";
+
+// Whether a gradient sent along this edge ends in the .grad of a row-major leaf, which keeps the leaf's layout: autograd
+// would bring a level-major gradient into it with a strided copy, at a third of the speed of the library's transpose.  (Any other
+// consumer, such as the products of a network's double backward, takes the strided view as it is.)
+bool goes_into_row_major_leaf(const torch::autograd::Edge& edge) {
+    const auto* const leaf = dynamic_cast<const torch::autograd::AccumulateGrad*>(edge.function.get());
+    return leaf != nullptr && leaf->variable.dim() == 2 && leaf->variable.is_contiguous();
+}
 
 // Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
 // consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
@@ -425,13 +467,17 @@ struct EncodeBackNode : public Node {
         // (with create_graph the pass stays as it is written: EncodeNode's gradients are then differentiated once more, this one's not)
         if (want_table && !grad_mode && up.row_stride == 0 && task_should_compute_output(2) &&
             current_stream(c.device()) == slicing->forward_stream) {
-            slicing->leave({torch::autograd::get_current_graph_task_id(), grads[1].detach().contiguous(), up});
+            slicing->leave({torch::autograd::get_current_graph_task_id(), checked_double_positions_grad(c, grads[1]), up});
             want_table = false;
         }
-        const bool want_upstream = task_should_compute_output(0);
+        bool want_upstream = task_should_compute_output(0);
+        if (want_upstream && goes_into_row_major_leaf(next_edge(0)) && c.columns() <= 255) {
+            out[0] = compute_grad_grad_rows(c, checked_double_positions_grad(c, grads[1]));
+            want_upstream = false;
+        }
         if (!want_table && !want_upstream) return out;
         SecondOrder s = compute_double_backward(c, grads[1].detach(), up, want_table, want_upstream);
-        out[0] = std::move(s.upstream);
+        if (want_upstream) out[0] = std::move(s.upstream);
         out[1] = std::move(s.table);
         return out;
     }
@@ -455,16 +501,13 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         const SecondOrderTerm* fused = nullptr;
         if (first_order) {
             up = upstream_of(c, grads[0].detach());
-            if (differentiable && want_positions && up.row_stride == c.columns() && c.columns() <= 255) {
-                // The position gradient needs its upstream gradient level by level; that copy outlives the call, so that the
-                // double backward's scatter reads it too (coalesced, where rows cost it a sixth of its time) and can be deferred.
-                Tensor level_major = level_major_array(c);
-                check(api.transpose(data(up.values), mutable_data(level_major), c.n, static_cast<int>(c.columns()), current_stream(c.device())),
-                      "transpose");
-                up = {level_major, 0};
+            // (columns of concatenated points carry no gradient: the copy's last rows stay unwritten and are never read)
+            if (differentiable && want_positions && !want_table && up.row_stride != 0 && c.columns() <= 255) {
+                g = compute_positions_backward(c, up);
+            } else {
+                if (want_table && !terms.empty()) fused = &terms.back();
+                g = compute_backward(c, up, want_table, want_positions, fused);
             }
-            if (want_table && !terms.empty()) fused = &terms.back();
-            g = compute_backward(c, up, want_table, want_positions, fused);
         }
         for (const SecondOrderTerm& t : terms) {
             if (&t == fused || !want_table) continue;
@@ -719,6 +762,8 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(adamw_step_sparse);
         PENC_FN(transpose);
         PENC_FN(upload);
+        PENC_FN(backward_positions_rowmajor);
+        PENC_FN(grad_grad_rowmajor);
 #undef PENC_FN
         Py_RETURN_NONE;
     });

@@ -178,3 +178,39 @@ def test_upload_carries_host_values_in_the_launch(n):
     rc = _native.lib().penc_upload(host.data_ptr(), dst.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
     host.zero_()  # the caller's array is its own again
     assert rc == 0 and torch.equal(dst[:n].cpu(), want) and dst[n].item() == 7.0
+
+
+@pytest.mark.parametrize("d,n,levels,cap,feat,concat", [(3, 1, 5, 64, 2, True), (2, 63, 9, 1 << 10, 4, True), (3, 64, 24, 1 << 18, 2, False), (4, 65, 8, 1000, 8, False),
+                                                        (8, 1003, 31, 1 << 10, 8, False), (5, 20001, 7, 1 << 12, 2, True), (6, 9001, 8, 1 << 18, 2, True)])
+def test_all_levels_of_a_block_of_points(d, n, levels, cap, feat, concat):
+    """Dense rows from the forward and from the grad-grad bit for bit, the position gradient of rows within its bound and its level-major
+    copy bit for bit: one point, remainders of a block, fewer and more levels than waves, 248 columns, tables inside and beyond an L2."""
+    from helpers import make_encoding, random_problem, to_gpu
+    from oracle import api as orc
+    from permutohedral_encoding_amd import _native
+    p = random_problem(d, n, levels, cap, seed=80 + d, sigma_range=(1.0, 1e-3), nr_feat=feat)
+    p["window"][levels // 2] = 0.0
+    _, fp = make_encoding(d, p["sigmas"], p["shift"], concat_points=concat, nr_feat=feat)
+    table, pos, win, dpos = (to_gpu(p[k]) for k in ("table", "pos", "window", "dpos"))
+    extra = _native.extra_levels(d, feat, concat)
+    cols, stride = feat * (levels + extra), feat * (levels + extra) + 2
+    grad_rows = torch.zeros(n, stride, device="cuda")
+    grad_rows[:, :feat * levels] = to_gpu(p["grad"].transpose(2, 0, 1).reshape(n, -1))
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    head = (d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr())
+    params = (fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(), win.data_ptr())
+    ws = torch.empty(4 * cols * n + lib.penc_positions_workspace_bytes(d, n, levels) + 512, dtype=torch.uint8, device="cuda")
+    sf = orc.scale_factors(d, p["sigmas"])
+    rows = torch.full((n, stride), 7.0, device="cuda")
+    assert lib.penc_forward_rowmajor(*head, *params, rows.data_ptr(), stride, int(concat), 0.5, ws.data_ptr(), ws.numel(), st) == 0
+    want = orc.forward(p["pos"], p["table"], sf, p["shift"], p["window"], concat_points=concat, points_scaling=0.5)
+    assert np.array_equal(rows[:, :cols].cpu().numpy(), want.transpose(2, 0, 1).reshape(n, cols)) and torch.all(rows[:, cols:] == 7.0)
+    assert lib.penc_grad_grad_rowmajor(*head, 0, *params, dpos.data_ptr(), rows.data_ptr(), stride, int(concat), ws.data_ptr(), ws.numel(), st) == 0
+    wd = orc.double_backward(p["pos"], p["table"], sf, p["shift"], p["window"], p["dpos"], p["grad"], concat_points=concat, want32=False, want64=False)
+    assert np.array_equal(rows[:, :cols].cpu().numpy(), wd["ggs"].transpose(2, 0, 1).reshape(n, cols)) and torch.all(rows[:, cols:] == 7.0)
+    copy, pg = torch.empty(feat * levels, n, device="cuda"), torch.empty_like(pos)
+    assert lib.penc_backward_positions_rowmajor(*head, 0, *params, grad_rows.data_ptr(), stride, copy.data_ptr(), pg.data_ptr(),
+                                                ws.data_ptr(), ws.numel(), st) == 0
+    assert torch.equal(copy, grad_rows[:, :feat * levels].t())
+    wp = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], p["window"], p["grad"])
+    assert np.all(np.abs(pg.cpu().numpy() - wp["grad64"]) <= 1e-6 * wp["abs64"] + 1e-30)
