@@ -23,6 +23,7 @@
 
 #include "../../include/penc.h"
 #include "penc_lattice.hpp"
+#include "penc_group_sort.hpp"
 #include "penc_reduce.hpp"
 #include "penc_scatter.hpp"
 #include "penc_table_backward.hpp"
@@ -871,6 +872,65 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, int t
     return p;
 }
 
+// When a table gradient takes the sorted groups of penc_group_sort.hpp, and how they cut its workspace.
+//
+// Up to 2^22 looked-up slots (points x vertices x levels): there the scatter, its fill and its reduction are latency, beyond it the
+// records of the coarse levels, which the scatter absorbs, cost more (us, scatter -> sorted groups; L = 16 unless given):
+//   D = 3, L = 24, 2^18 slots  500 points 23.2 -> 19.9, 2^13 points 56.8 -> 30.0, 2^15 53.6 -> 43.8 (3.1 M slots), 2^16 63.7 -> 68.7 (6.3 M)
+//   D = 3, 2^16 slots          2^12 points 29.6 -> 16.9, 2^16 points 68.0 -> 55.6 (4.2 M), 2^17 points 80.8 -> 94.3 (8.4 M)
+//   D = 8, 2^18 slots          2000 points 40.1 -> 22.6, 2^14 points 56.8 -> 54.9 (2.4 M), 2^15 points 69.2 -> 85 (4.7 M)
+//   D = 2, F = 4, 2^16 slots   2^12 points 34.5 -> 19.5, 2^16 points 73.3 -> 47.9;  D = 4, F = 8, 2^18 slots  2^15 points 123.9 -> 92.7
+// Writing every slot once is what a dense gradient costs either way; a batch that leaves most of a large table empty is better served
+// by a fill and a few direct adds (24 levels: 2^20 slots, 500 points 43 -> 47, 2^12 points 55 -> 57; 2^22 slots, 2^12 points 211 -> 232,
+// 2^14 points 290 -> 261).  Sparse gradients have no fill to save and pay for every range that got one record: 2^20
+// slots, 2^12 points 55 -> 88, 2^14 points 126 -> 101; 2^18 slots, 2000 points 29 -> 36, 2^15 points 56 -> 54.5.
+constexpr int64_t kGroupSortMaxLookups = int64_t{1} << 22, kGroupSortSlotsPerLookup = 64, kGroupSortSparseSlotsPerLookup = 16;
+constexpr uint32_t kRangeSlotsLog2 = 12, kRangeMinSlotsLog2 = 9, kRangeWorkgroupsWanted = 512, kRangeManyGroups = 32;
+constexpr size_t kGroupSortAnyFillBytes = size_t{64} << 20;
+inline bool group_sort_serves(int pos_dim, int64_t n, int levels, int feat_pairs, int capacity, bool sparse) {
+    const int64_t lookups = n * (pos_dim + 1);
+    if (lookups * levels > kGroupSortMaxLookups || capacity > (kGroupMaxRanges << kBinSlotsLog2)) return false;
+    if (sparse) return capacity <= kGroupSortSparseSlotsPerLookup * lookups;
+    return static_cast<size_t>(capacity) * levels * feat_pairs * sizeof(float2) <= kGroupSortAnyFillBytes || capacity <= kGroupSortSlotsPerLookup * lookups;
+}
+struct GroupSortPlan {
+    bool enabled = false;
+    GroupSort sort{};
+};
+// Bytes of the arrays for `pair_levels` pairs of features (for levels of several pairs a little more than they need).
+inline size_t group_sort_bytes(int pos_dim, int64_t n, int pair_levels) {
+    const size_t groups = static_cast<size_t>((n + kGroupPoints - 1) / kGroupPoints), records = static_cast<size_t>(pos_dim + 1) * kGroupPoints;
+    return static_cast<size_t>(pair_levels) * groups * (records * (sizeof(RecordValues) + sizeof(uint16_t)) + (kGroupMaxRanges + 2) * sizeof(uint16_t)) + 1024;
+}
+inline GroupSortPlan plan_group_sort(int pos_dim, int64_t n, int levels, int feat_pairs, int capacity, bool sparse, void* workspace,
+                                     size_t bytes) {
+    GroupSortPlan p;
+    const int pair_levels = levels * feat_pairs;
+    if (workspace == nullptr || !group_sort_serves(pos_dim, n, levels, feat_pairs, capacity, sparse)) return p;
+    const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
+    if (bytes < group_sort_bytes(pos_dim, n, pair_levels) + (base - reinterpret_cast<uintptr_t>(workspace))) return p;
+    GroupSort& g = p.sort;
+    g.n_groups = static_cast<uint32_t>((n + kGroupPoints - 1) / kGroupPoints);
+    g.records = static_cast<uint32_t>((pos_dim + 1) * kGroupPoints);
+    // ranges of 4096 slots (two workgroups per compute unit, and all of a wave's stores to one stretch), narrower ones where they
+    // leave compute units idle: two workgroups per unit, four where every workgroup sums many groups (D = 4, 16 levels of
+    // 2^16 slots, 2^15 points: 64.7 -> 53.4 us; D = 3, 2^12 points: 19.2 with four, 16.8 with two)
+    const uint32_t wanted = g.n_groups >= kRangeManyGroups ? 2 * kRangeWorkgroupsWanted : kRangeWorkgroupsWanted;
+    const auto ranges = [&](uint32_t shift) { return static_cast<uint32_t>((static_cast<int64_t>(capacity) + (int64_t{1} << shift) - 1) >> shift); };
+    g.range_shift = kRangeSlotsLog2;
+    while (ranges(g.range_shift) > static_cast<uint32_t>(kGroupMaxRanges)) ++g.range_shift;  // at most kBinSlotsLog2: see group_sort_serves
+    while (g.range_shift > kRangeMinSlotsLog2 && ranges(g.range_shift) * static_cast<uint32_t>(pair_levels) < wanted &&
+           ranges(g.range_shift - 1) <= static_cast<uint32_t>(kGroupMaxRanges))
+        --g.range_shift;
+    g.n_ranges = ranges(g.range_shift);
+    const size_t all = static_cast<size_t>(g.n_groups) * g.records;
+    g.values = reinterpret_cast<RecordValues*>(base);
+    g.slots = reinterpret_cast<uint16_t*>(base + static_cast<size_t>(pair_levels) * all * sizeof(RecordValues));
+    g.starts = g.slots + static_cast<size_t>(levels) * all;
+    p.enabled = true;
+    return p;
+}
+
 // Running consecutive passes on two streams (scatter pass p+1 while pass p is reduced) was tried and
 // measured 10-15% slower than one pass over all levels on one stream; hence a single stream.
 constexpr unsigned kReduceWorkgroupsWanted = 512;  // two per compute unit
@@ -1065,6 +1125,44 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     // every pair of features is scattered like a level of its own (see backward_table_kernel)
     const uint32_t feat_pairs = static_cast<uint32_t>(nr_feat / 2);
     const int pair_levels = nr_levels * static_cast<int>(feat_pairs);
+    TableLaunch t{};
+    t.stream = st;
+    t.rows = grad_row_stride != 0;
+    t.second_order = second.double_pos_grad != nullptr;
+    t.n_points = n;
+    t.feat_pairs = feat_pairs;
+    t.capacity = cap;
+    t.cap_mask = mask;
+    t.positions = positions;
+    t.scale_factor = scale_factor;
+    t.random_shift = random_shift;
+    t.window = anneal_window;
+    t.grad = grad;
+    t.grad_row_stride = grad_row_stride;
+    t.double_pos_grad = second.double_pos_grad;
+    t.second_grad = second.upstream;
+    t.table_grad = lattice_values_grad;
+    t.grad_level_major = grad_level_major;
+    const uint32_t dies = dies_of_current_device();
+    const GroupSortPlan sorted = plan_group_sort(pos_dim, nr_positions, nr_levels, static_cast<int>(feat_pairs), capacity, touched != nullptr,
+                                                 workspace, workspace_bytes);
+    if (sorted.enabled) {
+        const GroupSort& g = sorted.sort;
+        // (few groups: spread over the dies rather than kept together on one)
+        t.dies = g.n_groups >= 2 * dies ? dies : 0u;
+        const uint32_t padded = t.dies != 0u ? (g.n_groups + dies - 1) / dies * dies : g.n_groups;
+        t.grid = dim3(padded * static_cast<uint32_t>(nr_levels));
+        PENC_DISPATCH_D(pos_dim, launch_group_sort<DD>(t, g, static_cast<uint32_t>(nr_levels)));
+        if (int rc = check_launch()) return rc;
+        // a reader per group, of 16 to 256 threads
+        uint32_t lanes_log2 = 4;
+        while (lanes_log2 < 8 && (static_cast<uint32_t>(kRangeBlock) >> (lanes_log2 + 1)) >= g.n_groups) ++lanes_log2;
+        const uint32_t items = (static_cast<uint32_t>(nr_levels) * g.n_ranges + dies - 1) / dies * dies * feat_pairs;
+        hipLaunchKernelGGL(range_sum_kernel, dim3(items), dim3(kRangeBlock),
+                           (size_t{2} << g.range_shift) * sizeof(double), st, g, anneal_window, cap, feat_pairs, static_cast<uint32_t>(nr_levels),
+                           lanes_log2, dies, touched, bins_for_capacity(capacity), bin_shift_for_capacity(capacity), lattice_values_grad);
+        return check_launch();
+    }
     int tiles_per_group = table_backward_tiles(nr_positions, pair_levels);
     BinPlan plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, workspace, workspace_bytes);
     if (!plan.enabled && tiles_per_group > kScatterTiles) {  // wide bins need short segments: smaller groups of points
@@ -1081,35 +1179,16 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     }
     uint32_t* const direct_flags = plan.target.direct;
     const int per_pass = plan.enabled ? plan.levels_per_pass : pair_levels;
-    const uint32_t dies = dies_of_current_device();
     for (int first = 0; first < pair_levels; first += per_pass) {
         const int count = pair_levels - first < per_pass ? pair_levels - first : per_pass;
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
-        TableLaunch t{};
         t.grid = dim3(padded_groups * static_cast<unsigned>(count));
-        t.stream = st;
-        t.rows = grad_row_stride != 0;
-        t.second_order = second.double_pos_grad != nullptr;
         t.wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
-        t.n_points = n;
         t.first_level = first;
         t.n_pass_levels = static_cast<uint32_t>(count);
-        t.feat_pairs = feat_pairs;
         t.dies = dies;
         t.tiles_per_group = tiles_per_group;
-        t.capacity = cap;
-        t.cap_mask = mask;
-        t.positions = positions;
-        t.scale_factor = scale_factor;
-        t.random_shift = random_shift;
-        t.window = anneal_window;
-        t.grad = grad;
-        t.grad_row_stride = grad_row_stride;
-        t.double_pos_grad = second.double_pos_grad;
-        t.second_grad = second.upstream;
-        t.table_grad = lattice_values_grad;
-        t.grad_level_major = grad_level_major;
         t.bins = plan.target;
         PENC_DISPATCH_D(pos_dim, launch_table_backward<DD>(t));
         if (int rc = check_launch()) return rc;
@@ -1307,7 +1386,11 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
                                                 wanted_segment_capacity(pos_dim, n_bins, tiles));
         per_level = need > per_level ? need : per_level;
     }
-    return per_level * static_cast<size_t>(levels_per_pass) + direct_flag_bytes(nr_levels, n_bins) + 1024;
+    const size_t binned = per_level * static_cast<size_t>(levels_per_pass) + direct_flag_bytes(nr_levels, n_bins) + 1024;
+    // (how many pairs of features share a level is not known here: up to four)
+    const bool may_sort = levels_per_pass == nr_levels && nr_positions * (pos_dim + 1) * ((nr_levels + 3) / 4) <= kGroupSortMaxLookups;
+    const size_t sorted = may_sort ? group_sort_bytes(pos_dim, nr_positions, nr_levels) + 256 : 0;
+    return sorted > binned ? sorted : binned;
 }
 
 size_t penc_positions_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels) {

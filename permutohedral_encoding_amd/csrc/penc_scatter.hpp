@@ -254,6 +254,15 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// A barrier that orders the workgroup's LDS accesses only.  __syncthreads() also makes the global stores
+// issued so far visible, i.e. waits for the counter that loads share with them: after a store, it
+// would wait for every load that is still on its way.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Stage 3.  Lanes are paired (2p, 2p+1): first both lanes of a pair add the two features of the
 // even lane's slot, then those of the odd lane's slot, so that each 8-byte slot is one request.
 // Must be called with all 64 lanes of the wave active.
@@ -321,6 +330,33 @@ __device__ __forceinline__ uint32_t fold_adjacent_runs(uint32_t slot, bool& live
     const bool was_live = live;
     live = live && last_of_run;
     return __popcll(__ballot(was_live && !live));
+}
+
+// Folds the contributions of lanes that share a slot, wherever they are in the wave.  At the coarsest levels the 64 lanes of a
+// wave hit two to six distinct slots, and LDS atomics on one address serialise (about 5 clocks per lane): so up to
+// kWaveGroups times, take the slot of the first pending lane, sum the contributions of
+// all lanes that share it with DPP, and leave the sum with that lane alone.  A group
+// of fewer than kMinWaveGroup lanes means the wave's slots are spread out: stop.  Returns the number of lanes folded away.
+__device__ __forceinline__ uint32_t fold_shared_slots(uint32_t slot, bool& live, float& x0, float& x1) {
+    uint32_t folded = 0;
+    unsigned long long pending = __ballot(live);
+#pragma unroll 1
+    for (int round = 0; round < kWaveGroups && pending != 0ull; ++round) {
+        const int leader = __builtin_ctzll(pending);
+        const uint32_t leader_slot = __builtin_amdgcn_readlane(slot, leader);
+        const bool in_group = live && slot == leader_slot;
+        const unsigned long long members = __ballot(in_group);
+        if (__popcll(members) < kMinWaveGroup) break;
+        const float s0 = lane_value(wave_sum_to_last_lane(in_group ? x0 : 0.0f), 63);
+        const float s1 = lane_value(wave_sum_to_last_lane(in_group ? x1 : 0.0f), 63);
+        const bool is_leader = static_cast<int>(threadIdx.x & 63) == leader;
+        x0 = is_leader ? s0 : x0;
+        x1 = is_leader ? s1 : x1;
+        live = live && (!in_group || is_leader);
+        folded += __popcll(members) - 1;
+        pending &= ~members;
+    }
+    return folded;
 }
 
 // LDS state of a scattering workgroup.  The accumulate cache sums in fp64 with ds_add_f64: its
@@ -850,30 +886,9 @@ __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& leve
         float x0 = a0[r], x1 = a1[r];
         bool miss = active;
         if (use_cache) {
-            // stage 1.  At the coarsest levels the 64 lanes of a wave hit two to six distinct slots,
-            // and LDS atomics on one address serialise (about 5 clocks per lane): so first, up to
-            // kWaveGroups times, take the slot of the first pending lane, sum the contributions of
-            // all lanes that share it with DPP, and leave the sum with that lane alone.  A group
-            // of fewer than kMinWaveGroup lanes means the wave's slots are spread out: stop.
             // neighbouring lanes on one slot first (points that follow each other in space), then the slots most of the wave shares
             if (ordered) hits += fold_adjacent_runs(slot[r], miss, x0, x1);
-            unsigned long long pending = __ballot(miss);
-#pragma unroll 1
-            for (int round = 0; round < kWaveGroups && pending != 0ull; ++round) {
-                const int leader = __builtin_ctzll(pending);
-                const uint32_t leader_slot = __builtin_amdgcn_readlane(slot[r], leader);
-                const bool in_group = miss && slot[r] == leader_slot;
-                const unsigned long long members = __ballot(in_group);
-                if (__popcll(members) < kMinWaveGroup) break;
-                const float s0 = lane_value(wave_sum_to_last_lane(in_group ? x0 : 0.0f), 63);
-                const float s1 = lane_value(wave_sum_to_last_lane(in_group ? x1 : 0.0f), 63);
-                const bool is_leader = static_cast<int>(threadIdx.x & 63) == leader;
-                x0 = is_leader ? s0 : x0;
-                x1 = is_leader ? s1 : x1;
-                miss = miss && (!in_group || is_leader);
-                hits += __popcll(members) - 1;  // absorbed without touching the cache
-                pending &= ~members;
-            }
+            hits += fold_shared_slots(slot[r], miss, x0, x1);
             bool found = false;
             if (miss) {
                 // From D = 4 on a third candidate line: every contribution of a slot that finds no line becomes

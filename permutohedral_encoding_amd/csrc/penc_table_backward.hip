@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "penc_group_sort.hpp"
 #include "penc_lattice.hpp"
 #include "penc_scatter.hpp"
 #include "penc_table_backward.hpp"
@@ -247,6 +248,271 @@ backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
 }
 #undef PENC_TABLE_PARAMETERS
 #undef PENC_TABLE_ARGUMENTS
+
+// ------------------------------------------------------------------------------------------
+// the same for batches that do not fill the chip for long (see penc_group_sort.hpp)
+
+// Levels whose points share a hundred slots or so are summed in an LDS table first (lines of a tag and two fp64 sums, kept
+// where the records are staged later) and leave one record per line: else every group leaves hundreds of records on the same
+// few slots, which the one range_sum_kernel workgroup that owns those slots adds one after the other (2 to 3 clocks per lane and add).
+// A level with a handful of slots spreads each over several lines, by lane, so that the lanes of a wave rarely meet.
+constexpr uint32_t kGroupLinesLog2 = 9, kGroupLines = 1u << kGroupLinesLog2, kGroupProbes = 8;
+// Not for a few thousand points, whose records on one slot are a few hundred at most: the table's barriers cost more.
+constexpr int kGroupLinesMinPoints = 4096;
+static_assert(kGroupLines == kGroupPoints, "a thread per line");
+constexpr int group_sort_waves_per_simd(int pos_dim) { return pos_dim <= 3 ? 6 : (pos_dim == 4 ? 5 : 4); }
+
+template <int D, bool kRowMajor, int kOrder>
+__global__ void __launch_bounds__(kGroupPoints, group_sort_waves_per_simd(D))
+group_sort_kernel(int n_points, uint32_t n_levels, uint32_t feat_pairs, uint32_t dies, uint32_t capacity, uint32_t cap_mask,
+                  const float* __restrict__ positions, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
+                  const float* __restrict__ window, const float* __restrict__ grad, int64_t grad_row_stride,
+                  const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad, float* __restrict__ grad_level_major,
+                  GroupSort sort) {
+    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
+    constexpr int kRecords = (D + 1) * kGroupPoints, kWaves = kGroupPoints / 64;
+    __shared__ RecordValues stage_values[kRecords];
+    __shared__ uint16_t stage_slots[kRecords];
+    __shared__ uint32_t count[kGroupMaxRanges + 1];  // records per range, then where each range starts
+    __shared__ uint32_t wave_total[kWaves];
+    __shared__ uint32_t repeats;
+    struct Lines {
+        double sum[2][kGroupLines];
+        int tag[kGroupLines];
+    };
+    static_assert(sizeof(Lines) <= sizeof(stage_values), "the table of lines lives where the values are staged");
+    static_assert(kGroupMaxRanges == kGroupPoints, "a thread per range");
+    Lines& lines = *reinterpret_cast<Lines*>(stage_values);
+    // all levels of a group of points on one die, as in the scatter: rows then come from its L2 after the first level
+    uint32_t level, group;
+    if (dies != 0u) {
+        const uint32_t j = blockIdx.x / dies;
+        level = j % n_levels;
+        group = j / n_levels * dies + blockIdx.x % dies;
+    } else {
+        level = blockIdx.x % n_levels;
+        group = blockIdx.x / n_levels;
+    }
+    if (group >= sort.n_groups) return;
+    const float w_level = window[level];
+    if (w_level == 0.0f) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t mine = static_cast<int64_t>(group) * kGroupPoints + tid;
+    const bool active = mine < n_points;
+    const int64_t n = active ? mine : n_points - 1;
+    const auto load_vector = [&](const float* base) {
+        fvec<D> v;
+        static_for<D>(PENC_BODY(k) {
+            PENC_INDEX(k); v[k] = base[n * D + k]; });
+        return v;
+    };
+    const auto load_upstream = [&](size_t pair_level, float& g0, float& g1, float& s0, float& s1) {
+        if constexpr (kRowMajor) {
+            const float2 g = *reinterpret_cast<const float2*>(grad + n * grad_row_stride + 2 * pair_level);
+            g0 = g.x;
+            g1 = g.y;
+        } else {
+            g0 = grad[2 * pair_level * n_points + n];
+            g1 = grad[(2 * pair_level + 1) * n_points + n];
+        }
+        if constexpr (kBoth) {
+            s0 = second_grad[2 * pair_level * n_points + n];
+            s1 = second_grad[(2 * pair_level + 1) * n_points + n];
+        }
+    };
+    const fvec<D> pos = load_vector(positions);
+    fvec<D> q = 0.0f;
+    if constexpr (kNeedsQ) q = load_vector(double_pos_grad);
+    float g0, g1, s0 = 0.0f, s1 = 0.0f;
+    load_upstream(static_cast<size_t>(level) * feat_pairs, g0, g1, s0, s1);
+    count[tid] = 0u;
+    if (tid == 0) repeats = 0u;
+    lines.tag[tid] = -1;
+    lines.sum[0][tid] = 0.0;
+    lines.sum[1][tid] = 0.0;
+    const float* const sf = scale_factor + level * D;
+    uvec<D + 1> slot;
+    fvec<D + 1> w, w2;
+    {
+        const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
+        const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
+        if constexpr (kOrder == kSecondOrder) {
+            w = pos_grad_grad_to_bary<D>(s.rank, q, sf) * w_level;
+        } else {
+            w = barycentric<D>(s.rank, s.delta) * w_level;
+            if constexpr (kBoth) w2 = pos_grad_grad_to_bary<D>(s.rank, q, sf) * w_level;
+        }
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            slot[r] = to_slot(h[r], capacity, cap_mask);
+        });
+    }
+    const bool ordered = neighbours_share_slots(slot[0], active);
+    const uint32_t across = static_cast<uint32_t>(__shfl_xor(static_cast<int>(slot[0]), 32));
+    const uint32_t same = __popcll(__ballot(lane < 32 && mine + 32 < n_points && across == slot[0]));
+    __syncthreads();  // the counters and lines are cleared
+    if (lane == 0 && same != 0u) atomicAdd(&repeats, same);
+    __syncthreads();
+    // of 256 pairs of lanes half a wave apart, about 256 / (distinct slots) meet
+    const uint32_t met = repeats;
+    const bool few = met >= 2u && n_points > kGroupLinesMinPoints;
+    const uint32_t copies_log2 = met >= 16u ? 4u : (met >= 4u ? 2u : 1u);
+    const uint32_t my_copy = lane & ((1u << copies_log2) - 1u);
+    // where each contribution goes: kNone (it has none), kLine | its line, or its place among the group's records
+    constexpr uint32_t kNone = 0xFFFFFFFFu, kLine = 0x80000000u;
+    uvec<D + 1> to = kNone;
+    uint32_t total = 0, line_slot = 0, line_to = kNone;
+    const size_t group_at = static_cast<size_t>(level) * sort.n_groups + group;
+    const uint32_t slot_mask = (1u << sort.range_shift) - 1u;
+#pragma unroll 1
+    for (uint32_t pair = 0; pair < feat_pairs; ++pair) {
+        const size_t pair_level = static_cast<size_t>(level) * feat_pairs + pair;
+        if (pair != 0) {
+            load_upstream(pair_level, g0, g1, s0, s1);
+            if (few) {
+                lines.sum[0][tid] = 0.0;
+                lines.sum[1][tid] = 0.0;
+                __syncthreads();
+            }
+        }
+        if constexpr (kRowMajor) {
+            if (grad_level_major != nullptr && active) {
+                grad_level_major[2 * pair_level * n_points + n] = g0;
+                grad_level_major[(2 * pair_level + 1) * n_points + n] = g1;
+            }
+        }
+        fvec<D + 1> a0 = w * g0, a1 = w * g1;
+        if constexpr (kBoth) {
+            a0 += w2 * s0;
+            a1 += w2 * s1;
+        }
+        // (which lanes are folded into which, and which line takes a slot, depends on the slots alone: the same for every pair)
+        if (ordered) {
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r);
+                float x0 = a0[r], x1 = a1[r];
+                bool keep = active;
+                fold_adjacent_runs(slot[r], keep, x0, x1);
+                a0[r] = x0;
+                a1[r] = x1;
+                if (pair == 0) to[r] = keep ? 0u : kNone;
+            });
+        } else if (pair == 0) {
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r); to[r] = active ? 0u : kNone; });
+        }
+        float line0 = 0.0f, line1 = 0.0f;
+        if (few) {
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r);
+                if (pair == 0 && to[r] != kNone) {
+                    const int want = static_cast<int>((slot[r] << copies_log2) | my_copy);  // slots stay below 2^22
+                    uint32_t e = (static_cast<uint32_t>(want) * 0x9E3779B1u) >> (32 - kGroupLinesLog2);
+#pragma unroll 1
+                    for (uint32_t probe = 0; probe < kGroupProbes; ++probe) {
+                        int owner = lines.tag[e];
+                        if (owner == -1) owner = atomicCAS(&lines.tag[e], -1, want);
+                        if (owner == -1 || owner == want) {
+                            to[r] = kLine | e;
+                            break;
+                        }
+                        e = (e + 1u) & (kGroupLines - 1u);
+                    }
+                }
+                if (to[r] != kNone && (to[r] & kLine) != 0u) {
+                    const uint32_t e = to[r] & ~kLine;
+                    __hip_atomic_fetch_add(&lines.sum[0][e], static_cast<double>(a0[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(&lines.sum[1][e], static_cast<double>(a1[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            });
+            __syncthreads();  // all contributions are in
+            if (pair == 0) {
+                const int tag = lines.tag[tid];
+                if (tag != -1) {
+                    line_slot = static_cast<uint32_t>(tag) >> copies_log2;
+                    line_to = atomicAdd(&count[line_slot >> sort.range_shift], 1u);
+                }
+            }
+            line0 = static_cast<float>(lines.sum[0][tid]);
+            line1 = static_cast<float>(lines.sum[1][tid]);
+        }
+        if (pair == 0) {
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r);
+                if ((to[r] & kLine) == 0u) to[r] = atomicAdd(&count[slot[r] >> sort.range_shift], 1u);
+            });
+        }
+        __syncthreads();  // the records are counted, the lines read
+        if (pair == 0) {
+            const uint32_t records = count[tid];
+            uint32_t in_wave;
+            uint32_t before = wave_exclusive_scan(records, in_wave);
+            if (lane == 0) wave_total[wave] = in_wave;
+            __syncthreads();
+#pragma unroll
+            for (uint32_t v = 0; v < kWaves; ++v) {
+                const uint32_t t = wave_total[v];
+                before += v < wave ? t : 0u;
+                total += t;
+            }
+            count[tid] = before;
+            uint16_t* const starts = sort.starts + group_at * (sort.n_ranges + 1);
+            if (tid < sort.n_ranges) starts[tid] = static_cast<uint16_t>(before);
+            if (tid == 0) starts[sort.n_ranges] = static_cast<uint16_t>(total);
+            __syncthreads();
+        }
+        const auto stage = [&](uint32_t& at, uint32_t of_slot, float v0, float v1) {
+            if (pair == 0) {
+                at += count[of_slot >> sort.range_shift];
+                stage_slots[at] = static_cast<uint16_t>(of_slot & slot_mask);
+            }
+            RecordValues v;
+            v.x = v0;
+            v.y = v1;
+            stage_values[at] = v;
+        };
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            uint32_t at = to[r];
+            if ((at & kLine) == 0u) stage(at, slot[r], a0[r], a1[r]);
+            to[r] = at;
+        });
+        if (line_to != kNone) stage(line_to, line_slot, line0, line1);
+        __syncthreads();
+        RecordValues* const values_out = sort.values + (pair_level * sort.n_groups + group) * sort.records;
+        for (uint32_t i = tid; i < total; i += kGroupPoints) values_out[i] = stage_values[i];
+        if (pair == 0) {
+            uint16_t* const slots_out = sort.slots + group_at * sort.records;
+            for (uint32_t i = tid; i < total; i += kGroupPoints) slots_out[i] = stage_slots[i];
+        }
+        if (pair + 1 < feat_pairs) __syncthreads();  // the staged values are read
+    }
+}
+
+template <int D>
+void launch_group_sort(const TableLaunch& t, const GroupSort& sort, uint32_t n_levels) {
+#define PENC_LAUNCH(ROWS, ORDER)                                                                                                     \
+    hipLaunchKernelGGL((group_sort_kernel<D, ROWS, ORDER>), t.grid, dim3(kGroupPoints), 0, t.stream, t.n_points, n_levels, t.feat_pairs, \
+                       t.dies, t.capacity, t.cap_mask, t.positions, t.scale_factor, t.random_shift, t.window, t.grad, t.grad_row_stride, \
+                       t.double_pos_grad, t.second_grad, t.grad_level_major, sort)
+#define PENC_LAUNCH_ORDER(ROWS)                \
+    if (t.second_grad != nullptr) {            \
+        PENC_LAUNCH(ROWS, kBothOrders);        \
+    } else if (t.second_order) {               \
+        PENC_LAUNCH(ROWS, kSecondOrder);       \
+    } else {                                   \
+        PENC_LAUNCH(ROWS, kFirstOrder);        \
+    }
+    if (t.rows) {
+        PENC_LAUNCH_ORDER(true)
+    } else {
+        PENC_LAUNCH_ORDER(false)
+    }
+#undef PENC_LAUNCH_ORDER
+#undef PENC_LAUNCH
+}
+
+template void launch_group_sort<PENC_DIM>(const TableLaunch& t, const GroupSort& sort, uint32_t n_levels);
 
 template <int D>
 void launch_table_backward(const TableLaunch& t) {

@@ -26,4 +26,16 @@ struct TableLaunch {
 template <int D>
 void launch_table_backward(const TableLaunch& t);
 
+// Where group_sort_kernel leaves the records of a group of points (see penc_group_sort.hpp).
+struct GroupSort {
+    RecordValues* values;  // [level][pair][group][records]
+    uint16_t* slots;       // [level][group][records]: the slot within its range
+    uint16_t* starts;      // [level][group][n_ranges + 1]: where each range's records start
+    uint32_t n_groups, n_ranges, range_shift;
+    uint32_t records;      // room per group: its points times (D + 1)
+};
+
+template <int D>
+void launch_group_sort(const TableLaunch& t, const GroupSort& sort, uint32_t n_levels);
+
 }  // namespace penc

@@ -214,3 +214,38 @@ def test_all_levels_of_a_block_of_points(d, n, levels, cap, feat, concat):
     assert torch.equal(copy, grad_rows[:, :feat * levels].t())
     wp = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], p["window"], p["grad"])
     assert np.all(np.abs(pg.cpu().numpy() - wp["grad64"]) <= 1e-6 * wp["abs64"] + 1e-30)
+
+
+@pytest.mark.parametrize("d,n,levels,cap,feat,finest", [(3, 1, 24, 64, 2, 1e-3), (2, 511, 3, (1 << 12) + 1, 8, 1e-3), (3, 512, 9, 1 << 18, 2, 1e-3), (4, 513, 5, 50001, 4, 1e-3),
+                                                        (8, 1025, 4, 1 << 20, 2, 1e-3), (3, 9001, 24, 1 << 16, 2, 0.5), (2, 20001, 4, 1000, 4, 0.3), (3, 65536, 16, 1 << 12, 2, 1e-2),
+                                                        (5, 17000, 3, (1 << 22) - 3, 2, 1e-3)])
+def test_sorted_groups_give_the_table_gradient(d, n, levels, cap, feat, finest):
+    """Table gradients of small batches, dense (over what the memory held) and added twice into a sparse one: edges of groups and of slot
+    ranges, one range and 512, ranges narrower than a range of the touched map, levels of a few slots, a masked level; within the bound
+    of any sum in another order, 1e-4 of the sum of magnitudes.  The position gradient goes through the level-major copy."""
+    from helpers import assert_sum_close, make_encoding, random_problem, to_gpu
+    from oracle import api as orc
+    from permutohedral_encoding_amd import _native
+    p = random_problem(d, n, levels, cap, seed=90 + d, sigma_range=(1.0, finest), nr_feat=feat)
+    p["window"][levels // 2] = 0.0
+    _, fp = make_encoding(d, p["sigmas"], p["shift"], nr_feat=feat)
+    table, pos, win = (to_gpu(p[k]) for k in ("table", "pos", "window"))
+    rows = to_gpu(p["grad"].transpose(2, 0, 1).reshape(n, -1))
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    args = (d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr(), fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(),
+            win.data_ptr(), rows.data_ptr(), feat * levels)
+    ws = torch.empty(lib.penc_backward_rowmajor_workspace_bytes(d, feat, n, levels, cap, 1, 1), dtype=torch.uint8, device="cuda")
+    tg, pg = torch.full_like(table, float("nan")), torch.empty_like(pos)
+    assert lib.penc_backward_rowmajor(*args, tg.data_ptr(), pg.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
+    sf = orc.scale_factors(d, p["sigmas"])
+    want = orc.backward_table(p["pos"], sf, p["shift"], p["window"], p["grad"], cap, want_abs=True)
+    assert_sum_close(tg.cpu().numpy(), want["grad64"], want["abs64"], 1e-4, "dense")
+    wp = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], p["window"], p["grad"])
+    assert np.all(np.abs(pg.cpu().numpy() - wp["grad64"]) <= 1e-6 * wp["abs64"] + 1e-30)
+    sums = torch.zeros_like(table)
+    touched = torch.zeros(lib.penc_touched_map_entries(feat, levels, cap), dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        assert lib.penc_backward_sparse(*args, sums.data_ptr(), touched.data_ptr(), None, ws.data_ptr(), ws.numel(), st) == 0
+    assert_sum_close(sums.cpu().numpy(), 2 * want["grad64"], 2 * want["abs64"], 1e-4, "sparse")
+    assert lib.penc_clear_touched(sums.data_ptr(), feat, levels, cap, touched.data_ptr(), st) == 0
+    assert not sums.any() and not touched.any()
