@@ -12,7 +12,8 @@ def cosine_easing_window(num_freqs, alpha):
     ``win[k] = 0.5 * (1 + cos(pi * clip(alpha - k, 0, 1) + pi))``: exactly 1 for fully eased-in
     levels, exactly 0 for levels not yet started (reference: utils.py:5-16).
     """
-    if isinstance(num_freqs, int) and isinstance(alpha, (int, float)):
+    # (a torch-function mode, such as the one that sets a default device, has to see the tensor operations)
+    if isinstance(num_freqs, int) and isinstance(alpha, (int, float)) and torch._C._len_torch_function_stack() == 0:
         return bridge().cosine_window(num_freqs, alpha)  # the same, natively
     x = torch.clip(alpha - torch.arange(num_freqs, dtype=torch.float32), 0.0, 1.0)
     return 0.5 * (1 + torch.cos(math.pi * x + math.pi))
