@@ -16,14 +16,18 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <dlfcn.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/functions/accumulate_grad.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <memory>
@@ -149,7 +153,12 @@ std::pair<Tensor, Tensor> sparse_gradient(const Call& c) {
         Py_DECREF(sparse);
     }
     Py_XDECREF(lv);
-    if (PyErr_Occurred()) PyErr_Clear();
+    if (PyErr_Occurred()) {
+        python_error error;  // (such as the allocator's, as the interpreter would raise it)
+        error.persist();
+        PyGILState_Release(gil);
+        throw error;
+    }
     PyGILState_Release(gil);
     TORCH_CHECK(grad.defined() && touched.defined(), "the sparse table gradient could not be created");
     return {grad, touched};
@@ -159,14 +168,6 @@ std::pair<Tensor, Tensor> sparse_gradient(const Call& c) {
 struct Upstream {
     Tensor values;
     int64_t row_stride = 0;
-    int64_t version = -1;  // of the values when they were kept for a later pass
-
-    void keep() { version = values.is_inference() ? -1 : static_cast<int64_t>(values._version()); }
-    void check_unmodified() const {
-        TORCH_CHECK(version < 0 || version == static_cast<int64_t>(values._version()),
-                    "one of the variables needed for gradient computation has been modified by an inplace operation: the upstream gradient "
-                    "of the encoding is at version ", values._version(), "; expected version ", version, " instead");
-    }
 };
 
 Upstream upstream_of(const Call& c, const Tensor& grad) {
@@ -410,6 +411,10 @@ bool goes_into_row_major_leaf(const torch::autograd::Edge& edge) {
 struct EncodeNode : public Node {
     std::shared_ptr<const Call> call;
     void* forward_stream = nullptr;
+    // The result counts as saved, as it does in funcs.py: changing it in place, or a second pass through a freed graph, is refused.
+    c10::VariableVersion result_version;
+    uint32_t expected_version = 0;
+    bool released = false;
 
     // A training step on an SDF asks for two table gradients in one pass, through the encoded values and through the
     // position gradient.  The node that meets the second one (EncodeBackNode) runs first, because it names this node as one
@@ -418,6 +423,17 @@ struct EncodeNode : public Node {
     std::vector<SecondOrderTerm> second_order;
 
     std::string name() const override { return "PermutoEncodingBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        released = true;
+    }
+    void check_saved() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        TORCH_CHECK(!released, kSecondTime);
+        TORCH_CHECK(result_version.current_version() == expected_version,
+                    "one of the variables needed for gradient computation has been modified by an inplace operation: the encoding is at version ",
+                    result_version.current_version(), "; expected version ", expected_version, " instead");
+    }
 
     void leave(SecondOrderTerm term) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -433,6 +449,13 @@ struct EncodeNode : public Node {
     variable_list apply(variable_list&& grads) override;
 };
 
+// What the result's grad_fn is: hands its gradient to the EncodeNode.  Hooks on the result live here, so that a pass that
+// reaches the EncodeNode from an EncodeBackNode alone does not run them on a gradient that does not exist.
+struct ResultNode : public Node {
+    std::string name() const override { return "PermutoEncodingResultBackward"; }
+    variable_list apply(variable_list&& grads) override { return std::move(grads); }
+};
+
 // Gradient of the gradients of the slicing.  Inputs (in the graph's sense): what EncodeNode produced, i.e. the
 // gradients w.r.t. the table and w.r.t. the positions; only the path through the latter is differentiated (as in the
 // reference, funcs.py:57-72).  Outputs: gradients w.r.t. the upstream gradient, w.r.t. the table, and nothing for the
@@ -440,29 +463,26 @@ struct EncodeNode : public Node {
 struct EncodeBackNode : public Node {
     std::shared_ptr<const Call> call;
     std::shared_ptr<EncodeNode> slicing;
-    Upstream upstream;
-    bool released = false;
+    torch::autograd::SavedVariable upstream;  // saved as autograd saves: version checks, hooks, freed with the graph
 
     std::string name() const override { return "PermutoEncodingBackward2"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        upstream.values.reset();
-        released = true;
+        upstream.reset_data();
     }
     variable_list apply(variable_list&& grads) override {
         variable_list out(3);
         if (grads.size() < 2 || !grads[1].defined()) return out;
-        Upstream up;
+        Tensor saved;
         {
             std::lock_guard<std::mutex> lock(mutex_);
-            TORCH_CHECK(!released, kSecondTime);
-            up = upstream;
+            saved = upstream.unpack();
         }
-        up.check_unmodified();
         const Call& c = *call;
         const bool grad_mode = c10::GradMode::is_enabled();
         at::NoGradGuard no_grad;
         const c10::DeviceGuard device(c.device());
+        const Upstream up = upstream_of(c, saved);  // (a hook may have brought it back in another layout)
         bool want_table = c.want_table && task_should_compute_output(1);
         // (with create_graph the pass stays as it is written: EncodeNode's gradients are then differentiated once more, this one's not)
         if (want_table && !grad_mode && up.row_stride == 0 && task_should_compute_output(2) &&
@@ -500,6 +520,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         const c10::DeviceGuard device(c.device());
         const SecondOrderTerm* fused = nullptr;
         if (first_order) {
+            check_saved();
             up = upstream_of(c, grads[0].detach());
             // (columns of concatenated points carry no gradient: the copy's last rows stay unwritten and are never read)
             if (differentiable && want_positions && !want_table && up.row_stride != 0 && c.columns() <= 255) {
@@ -523,8 +544,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
         back->add_next_edge(torch::autograd::Edge(back->slicing, 0));
         back->call = call;
-        back->upstream = std::move(up);
-        back->upstream.keep();
+        back->upstream = torch::autograd::SavedVariable(up.values, false);
         torch::autograd::set_history(g.table, back);
         torch::autograd::set_history(g.positions, back);
     }
@@ -546,6 +566,8 @@ template <typename F>
 PyObject* guarded(F&& body) {
     try {
         return body();
+    } catch (python_error& e) {
+        e.restore();
     } catch (const c10::ValueError& e) {
         PyErr_SetString(PyExc_ValueError, e.what_without_backtrace());
     } catch (const c10::OutOfMemoryError& e) {
@@ -612,21 +634,33 @@ void prepare_call(Call& c, const Tensor& positions, const Tensor& window) {
 Tensor window_on_device(const Tensor& window, const at::Device& device) {
     constexpr int64_t kMost = 1024;
     if (!window.device().is_cpu() || window.dim() != 1 || window.numel() == 0 || window.numel() > kMost) return window.to(device, at::kFloat);
-    const Tensor host = window.to(at::kFloat).contiguous();
     const c10::DeviceGuard guard(device);
+    // (a graph would replay the window of the step that captured it)
+    TORCH_CHECK(c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None,
+                "anneal_window is in host memory: a call that is captured in a graph needs it in GPU memory");
+    const Tensor host = window.to(at::kFloat).contiguous();
     Tensor out = at::empty({host.numel()}, host.options().device(device));
     check(api.upload(data(host), mutable_data(out), static_cast<int>(host.numel()), current_stream(device)), "upload");
     return out;
 }
 
+// Whether something has to see the autograd functions of funcs.py: a functorch transform or a forward-mode tangent, which they
+// refuse, or a trace, which records them.
+bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positions) {
+    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing() ||
+           lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined();
+}
+
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
-//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None) -> (N, F(L+E))
+//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None)
+//   -> (N, F(L+E)), or None where the autograd functions are needed
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
         TORCH_CHECK(n_args == 14, "encode takes 14 arguments");
         TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
         const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
         const Tensor& positions = tensor_arg(args[2], "positions");
+        if (needs_autograd_functions(lattice_values, positions)) Py_RETURN_NONE;
         auto call = std::make_shared<Call>();
         Call& c = *call;
         c.lattice_values = lattice_values;
@@ -660,7 +694,11 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             node->set_next_edges(torch::autograd::collect_next_edges(lattice_values, positions));
             node->forward_stream = current_stream(call->device());
             node->call = std::move(call);
-            torch::autograd::set_history(out, node);
+            node->result_version = torch::autograd::impl::version_counter(out);
+            node->expected_version = node->result_version.current_version();
+            auto result = std::shared_ptr<ResultNode>(new ResultNode(), torch::autograd::deleteNode);
+            result->add_next_edge(torch::autograd::Edge(node, node->add_input_metadata(out)));
+            torch::autograd::set_history(out, result);
         }
         return THPVariable_Wrap(std::move(out));
     });

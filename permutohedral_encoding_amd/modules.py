@@ -133,7 +133,9 @@ class PermutoEncoding(torch.nn.Module):
 
     def forward(self, positions, anneal_window=None):
         if not self.lattice.calls_replaced():
-            return self.lattice.encode(self.lattice_values, positions, self.anneal_window if anneal_window is None else anneal_window)
+            out = self.lattice.encode(self.lattice_values, positions, self.anneal_window if anneal_window is None else anneal_window)
+            if out is not None:
+                return out
         nr_positions = positions.shape[0]
         if anneal_window is None:
             anneal_window = self.anneal_window

@@ -130,6 +130,75 @@ def test_losses_on_values_and_on_position_gradients_in_one_pass(kw, normals):
     assert torch.equal(pa, pb) and all(torch.equal(x, y) for x, y in zip(ua, ub))
 
 
+def test_native_path_refuses_what_the_autograd_functions_refuse():
+    pts = torch.rand(300, 3, device="cuda")
+    for m in modules():
+        out = m(pts)
+        out.sum().backward()
+        with pytest.raises(RuntimeError, match="second time"):
+            out.sum().backward()
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            m(pts).mul_(2.0).sum().backward()
+        with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError, match="jvp|forward"):
+            m(torch.autograd.forward_ad.make_dual(pts, torch.ones_like(pts)))
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda x: m(x).sum())(pts)
+        with pytest.raises(RuntimeError):
+            torch.vmap(m)(pts[None])
+
+
+def test_hooks_on_the_encoding_do_not_run_in_a_pass_through_its_position_gradient_alone():
+    results = []
+    for m in modules():
+        p = torch.full((40, 3), 0.3, device="cuda", requires_grad=True)
+        u = torch.ones(40, m.output_dims(), device="cuda", requires_grad=True)
+        seen = []
+        out = m(p)
+        out.register_hook(lambda g: seen.append(1) or 2 * g)
+        normal, = torch.autograd.grad(out, p, u, create_graph=True)
+        assert seen == [1]
+        normal.square().sum().backward()
+        assert seen == [1]
+        results.append((normal.detach(), u.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("rows", [True, False])
+def test_saved_tensor_hooks_see_the_upstream_gradient(rows):
+    native, _ = modules()
+    p = torch.rand(500, 3, device="cuda", requires_grad=True)
+    u = torch.randn(500, native.output_dims(), device="cuda")
+    u = u if rows else u.t().contiguous().t()
+    results, packed = [], []
+    for hooks in (False, True):
+        native.lattice_values.grad = None
+        out = native(p)
+        if hooks:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t.cpu().contiguous(), lambda t: t.cuda()):
+                normal, = torch.autograd.grad(out, p, u, create_graph=True)
+        else:
+            normal, = torch.autograd.grad(out, p, u, create_graph=True)
+        normal.square().sum().backward()
+        results.append(native.lattice_values.grad)
+    assert packed
+    close_sums(*results)
+
+
+def test_a_window_in_host_memory_is_not_captured():
+    native, _ = modules()
+    pts, stream = torch.rand(300, 3, device="cuda"), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(stream):
+        native(pts, torch.ones(5))
+        graph = torch.cuda.CUDAGraph()
+        graph.capture_begin()
+        with pytest.raises(RuntimeError, match="host memory"):
+            native(pts, torch.ones(5))
+        native(pts)
+        graph.capture_end()
+    torch.cuda.synchronize()
+
+
 def test_upstream_gradient_modified_before_the_double_backward_is_refused():
     native, _ = modules()
     p = torch.rand(100, 3, device="cuda", requires_grad=True)
