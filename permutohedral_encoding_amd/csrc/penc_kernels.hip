@@ -30,10 +30,7 @@
 
 namespace penc {
 
-// Levels one position-gradient thread sums in registers (measured: 2 is fastest up to D = 5, 1
-// from D = 6 on, where a thread's arithmetic per level is long enough; 3 and 4 are slower everywhere,
-// also with all their gathers issued up front: more levels at a time overflow L2).
-constexpr int pos_levels_per_group(int pos_dim) { return pos_dim >= 6 ? 1 : 2; }
+constexpr int kPosLevelsPerGroup = 2;  // levels a position-gradient thread sums in registers (figures at backward_pos_kernel)
 
 constexpr int kDefaultLevelsPerPass = 1 << 20;  // by default the suggested workspace bins all levels in one pass (measured fastest)
 
@@ -117,11 +114,16 @@ struct LevelMap {
     uint32_t segment;  // (row, tile) pairs per segment; 0: the grid is (tile, row)
     uint32_t dies;
 };
-// Whether any level of a row (row, row + rows, ...) has a window weight other than 0.
-__device__ __forceinline__ bool row_has_level(const float* __restrict__ window, uint32_t row, uint32_t rows, int n_levels) {
-    for (uint32_t level = row; level < static_cast<uint32_t>(n_levels); level += rows)
-        if (window[level] != 0.0f) return true;
-    return false;
+// The levels whose window weight is not 0, of up to 64; of more, all of them.  (For every lane of a wave at once.)
+__device__ __forceinline__ unsigned long long live_levels(const float* __restrict__ window, int n_levels) {
+    const int lane = static_cast<int>(threadIdx.x & 63);
+    return __ballot(lane < n_levels && window[lane] != 0.0f);
+}
+constexpr int kMostLiveLevels = 64;
+// Into how many groups of `per_group` the position gradient puts its levels.
+__device__ __forceinline__ int live_groups(unsigned long long live, int n_levels, int per_group) {
+    const int count = n_levels <= kMostLiveLevels ? __popcll(live) : n_levels;
+    return (count + per_group - 1) / per_group;
 }
 __device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile, uint32_t& row) {
     if (map.segment == 0u) {
@@ -214,9 +216,15 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
 // the whole chip on the same few levels at a time (their table slices stay in L2) and give the
 // launch many more, shorter waves than one thread per point walking all levels.  (Doing this
 // kernel's rank permutations through LDS, as the forward does, was measured: no gain.)
+//
+// Groups are made of the levels that the window leaves: with half of them masked there are half as many groups, whose sums are
+// stored and read back, where a grouping of all levels left groups of one (2^20 points, 16 of 24 levels of 2^22 slots: 418 ->
+// 385 us).  Two levels to a group: one, two, three, four at 2^20 points, D = 3, 24 levels of 2^18 slots 499 / 458 / 449 / 467 us,
+// of 2^22 slots 1026 / 887 / 946 / 975; D = 4 632 / 547 / 557 / 588; D = 6, 16 levels, 2^19 points 305 / 270 / 269 / 277;
+// D = 8, 2^19 slots 444 / 420 / 459 / 487.
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
+backward_pos_kernel(int n_points, int n_levels, int per_group, LevelMap map, uint32_t capacity, uint32_t cap_mask,
                     const float* __restrict__ positions, const T* __restrict__ table,
                     const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                     const float* __restrict__ window, const float* __restrict__ grad_sliced,
@@ -224,16 +232,25 @@ backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity,
     uint32_t tile, row;
     if (!locate_work(map, tile, row)) return;
     const int n = tile * kBlock + threadIdx.x;
-    if (n >= n_points) return;
-    // (with a coarse-to-fine window half the groups can be masked: nothing is stored for them, and the reduction skips them)
-    if (map.rows > 1u && !row_has_level(window, row, map.rows, n_levels)) return;
-    const fvec<D> pos = load_point<D>(positions, n);
+    const fvec<D> pos = load_point<D>(positions, n < n_points ? n : n_points - 1);  // (on its way while the window is looked at)
+    unsigned long long live = live_levels(window, n_levels);
+    const int groups = map.rows > 1u ? live_groups(live, n_levels, per_group) : 1;
+    if (static_cast<int>(row) >= groups || n >= n_points) return;
     fvec<D> total = 0.0f;
-    // The levels of a group are `rows` apart, not adjacent: with the usual coarse-to-fine level list a
+    // The levels of a group are `groups` apart, not adjacent: with the usual coarse-to-fine level list a
     // group then pairs a coarse level, whose points share few slots, with a fine one, and the table slices
     // a die gathers from at any time fit its L2 (two adjacent fine levels are 4 MiB at 2^18 slots,
     // an L2's whole capacity).
-    for (int level = static_cast<int>(row); level < n_levels; level += static_cast<int>(map.rows)) {
+    const int left = __popcll(live);
+    const bool masked = n_levels <= kMostLiveLevels && left < n_levels;  // `live` names the levels, else their numbers do
+    const int count = masked ? left : n_levels;
+    int passed = 0;  // of `live`
+    for (int k = static_cast<int>(row); k < count; k += groups) {
+        int level = k;
+        if (masked) {
+            for (; passed < k; ++passed) live &= live - 1ull;
+            level = __builtin_ctzll(live);
+        }
         const float w_level = window[level];
         if (w_level == 0.0f) continue;
         const float* sf = scale_factor + level * D;
@@ -258,41 +275,27 @@ backward_pos_kernel(int n_points, int n_levels, LevelMap map, uint32_t capacity,
 }
 
 // Sums the partial position gradients of the groups in ascending order, one value to a thread.  What it waits for at small sizes
-// is its chain of loads: those of kTogether groups are issued together, the groups that have stored anything (a masked one has
-// not) being known beforehand (2^15 points, 12 groups: 11.5 -> 3.9 us; large sums are bound by the memory, 2^20 points 31 us).
+// is its chain of loads: those of kTogether groups are issued together (2^15 points, 12 groups: 11.5 -> 3.9 us; large sums are
+// bound by the memory, 2^20 points 31 us).
 // (16 bytes to a lane are slower, 50 us: the groups' sums lie a multiple of the memory's interleave apart, and loads of
 // several groups from the same few waves meet on one channel.)
 __global__ void __launch_bounds__(kBlock)
-reduce_level_groups_kernel(const float* __restrict__ partial, const float* __restrict__ window, int n_groups, int n_levels,
+reduce_level_groups_kernel(const float* __restrict__ partial, const float* __restrict__ window, int per_group, int n_levels,
                            size_t n_values, float* __restrict__ out) {
     constexpr int kTogether = 8;
+    const int groups = live_groups(live_levels(window, n_levels), n_levels, per_group);
     const size_t stride = static_cast<size_t>(gridDim.x) * kBlock;
-    for (size_t first_value = static_cast<size_t>(blockIdx.x) * kBlock; first_value < n_values; first_value += stride) {
-        const size_t i = first_value + threadIdx.x, at = i < n_values ? i : n_values - 1;
-        float acc = 0.0f;
-        bool first = true;
-        for (int base = 0; base < n_groups; base += 64) {
-            const int mine = base + static_cast<int>(threadIdx.x & 63);  // (all 64 lanes are here, also those past the last value)
-            unsigned long long live = __ballot(
-                mine < n_groups && row_has_level(window, static_cast<uint32_t>(mine), static_cast<uint32_t>(n_groups), n_levels));
-            while (live != 0ull) {
-                const int count = __popcll(live);
-                float v[kTogether];
+    for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < n_values; i += stride) {
+        float acc = groups > 0 ? partial[i] : 0.0f;
+        for (int base = 1; base < groups; base += kTogether) {
+            float v[kTogether];
 #pragma unroll
-                for (int u = 0; u < kTogether; ++u) {
-                    v[u] = 0.0f;
-                    if (live != 0ull) v[u] = partial[static_cast<size_t>(base + __builtin_ctzll(live)) * n_values + at];
-                    live &= live - 1ull;
-                }
+            for (int u = 0; u < kTogether; ++u) v[u] = base + u < groups ? partial[static_cast<size_t>(base + u) * n_values + i] : 0.0f;
 #pragma unroll
-                for (int u = 0; u < kTogether; ++u) {
-                    if (u >= count) break;
-                    acc = first ? v[u] : acc + v[u];
-                    first = false;
-                }
-            }
+            for (int u = 0; u < kTogether; ++u)
+                if (base + u < groups) acc += v[u];
         }
-        if (i < n_values) out[i] = acc;
+        out[i] = acc;
     }
 }
 
@@ -1249,7 +1252,7 @@ static int block_rows(int pos_dim, int nr_feat, int64_t nr_positions, int nr_lev
 }
 
 // The position gradient of penc_backward / penc_backward_rowmajor from a level-major upstream gradient:
-// levels in groups of pos_levels_per_group() when the workspace can hold the partial sums, else one
+// levels in groups of kPosLevelsPerGroup when the workspace can hold the partial sums, else one
 // thread per point walks all levels.
 static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
                               const TableRef& table, const float* scale_factor, const float* random_shift,
@@ -1264,16 +1267,16 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
     int per_group = nr_levels, groups = 1;
     float* partial = positions_grad;
     const uintptr_t ws = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
-    const int want_groups = (nr_levels + pos_levels_per_group(pos_dim) - 1) / pos_levels_per_group(pos_dim);
+    const int want_groups = (nr_levels + kPosLevelsPerGroup - 1) / kPosLevelsPerGroup;
     if (workspace != nullptr && want_groups > 1 &&
         workspace_bytes >= (ws - reinterpret_cast<uintptr_t>(workspace)) + want_groups * n_values * sizeof(float)) {
-        per_group = pos_levels_per_group(pos_dim);
+        per_group = kPosLevelsPerGroup;
         groups = want_groups;
         partial = reinterpret_cast<float*>(ws);
     }
     const GatherLaunch g = plan_gather(nr_positions, nr_levels, per_group, slice_bytes(capacity, nr_feat, table.format), kLargeGather / 2);
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st, n, nr_levels, g.map, cap, mask, positions,
+                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st, n, nr_levels, per_group, g.map, cap, mask, positions,
                                          static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
                                          grad_level_major, partial));
     if (int rc = check_launch()) return rc;
@@ -1282,7 +1285,7 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
         const size_t per_block = kBlock * (n_values >= size_t{1} << 19 ? 4 : 1);
         const size_t want = (n_values + per_block - 1) / per_block;
         hipLaunchKernelGGL(reduce_level_groups_kernel, dim3(static_cast<unsigned>(want < 8192 ? want : 8192)), dim3(kBlock), 0, st, partial,
-                           anneal_window, groups, nr_levels, n_values, positions_grad);
+                           anneal_window, per_group, nr_levels, n_values, positions_grad);
         if (int rc = check_launch()) return rc;
     }
     return PENC_OK;
@@ -1394,8 +1397,8 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
 }
 
 size_t penc_positions_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels) {
-    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= pos_levels_per_group(pos_dim)) return 0;
-    const size_t groups = static_cast<size_t>((nr_levels + pos_levels_per_group(pos_dim) - 1) / pos_levels_per_group(pos_dim));
+    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= kPosLevelsPerGroup) return 0;
+    const size_t groups = static_cast<size_t>((nr_levels + kPosLevelsPerGroup - 1) / kPosLevelsPerGroup);
     return groups * static_cast<size_t>(nr_positions) * pos_dim * sizeof(float) + 256;
 }
 

@@ -318,3 +318,29 @@ def test_sorted_groups_give_the_table_gradient(d, n, levels, cap, feat, finest):
     assert_sum_close(sums.cpu().numpy(), 2 * want["grad64"], 2 * want["abs64"], 1e-4, "sparse")
     assert lib.penc_clear_touched(sums.data_ptr(), feat, levels, cap, touched.data_ptr(), st) == 0
     assert not sums.any() and not touched.any()
+
+
+@pytest.mark.parametrize("d,n,levels,cap,feat", [(3, 16001, 24, 1 << 17, 2), (2, 40009, 13, 1 << 18, 4), (8, 10501, 16, 1 << 17, 2), (6, 6007, 65, 1 << 15, 2),
+                                                 (3, 301, 130, 64, 2), (4, 255, 64, 128, 4)])
+def test_position_gradient_groups_the_levels_a_window_leaves(d, n, levels, cap, feat):
+    """Groups of the levels that are left: all, none, the last alone, every third, the coarse half; at 64 levels, beyond them, and as
+    one group without a workspace; against the oracle within the bound of its 32-bit sums, 1e-6 of the sum of magnitudes."""
+    from helpers import make_encoding, random_problem, to_gpu
+    from oracle import api as orc
+    from permutohedral_encoding_amd import _native
+    p = random_problem(d, n, levels, cap, seed=110 + d, sigma_range=(1.0, 1e-2), nr_feat=feat)
+    _, fp = make_encoding(d, p["sigmas"], p["shift"], nr_feat=feat)
+    table, pos, grad = (to_gpu(p[k]) for k in ("table", "pos", "grad"))
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    ws = torch.full((lib.penc_positions_workspace_bytes(d, n, levels),), 0xFF, dtype=torch.uint8, device="cuda")
+    sf, k = orc.scale_factors(d, p["sigmas"]), np.arange(levels)
+    for keep in (k >= 0, k < 0, k == levels - 1, k % 3 == 1, k < levels // 2):
+        window = np.where(keep, p["window"], 0).astype(np.float32)
+        win = to_gpu(window)
+        want = orc.backward_pos(p["pos"], p["table"], sf, p["shift"], window, p["grad"])
+        for memory in (ws, None):
+            pg = torch.full_like(pos, float("nan"))
+            assert lib.penc_backward(d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr(), fp.m_scale_factor.data_ptr(),
+                                     fp.m_random_shift_per_level.data_ptr(), win.data_ptr(), grad.data_ptr(), None, pg.data_ptr(),
+                                     memory.data_ptr() if memory is not None else None, memory.numel() if memory is not None else 0, st) == 0
+            assert np.all(np.abs(pg.cpu().numpy() - want["grad64"]) <= 1e-6 * want["abs64"] + 1e-30)
