@@ -877,22 +877,31 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, int t
 
 // When a table gradient takes the sorted groups of penc_group_sort.hpp, and how they cut its workspace.
 //
-// Up to 2^22 looked-up slots (points x vertices x levels): there the scatter, its fill and its reduction are latency, beyond it the
-// records of the coarse levels, which the scatter absorbs, cost more (us, scatter -> sorted groups; L = 16 unless given):
-//   D = 3, L = 24, 2^18 slots  500 points 23.2 -> 19.9, 2^13 points 56.8 -> 30.0, 2^15 53.6 -> 43.8 (3.1 M slots), 2^16 63.7 -> 68.7 (6.3 M)
-//   D = 3, 2^16 slots          2^12 points 29.6 -> 16.9, 2^16 points 68.0 -> 55.6 (4.2 M), 2^17 points 80.8 -> 94.3 (8.4 M)
-//   D = 8, 2^18 slots          2000 points 40.1 -> 22.6, 2^14 points 56.8 -> 54.9 (2.4 M), 2^15 points 69.2 -> 85 (4.7 M)
-//   D = 2, F = 4, 2^16 slots   2^12 points 34.5 -> 19.5, 2^16 points 73.3 -> 47.9;  D = 4, F = 8, 2^18 slots  2^15 points 123.9 -> 92.7
+// Up to 2^22 looked-up slots (points x vertices x levels), 6 x 2^20 at three and four dimensions: there the scatter, its fill and its
+// reduction are latency, beyond it the records of the coarse levels, which the scatter absorbs, cost more (us, scatter ->
+// sorted groups; L = 16 unless given):
+//   D = 3, L = 24, 2^18 slots  500 points 23.2 -> 19.9, 2^14 points 51.0 -> 36.8, 2^15 56.9 -> 44.8 (3.1 M slots), 2^16 67.0 -> 61.4 (6.3 M),
+//                              along rays 69.8 -> 56.9, 125000 points 98 -> 95, 250000 points 141 -> 185
+//   D = 3, 2^16 slots          2^12 points 29.6 -> 16.9, 2^16 points 70.5 -> 49.9 (4.2 M)
+//   D = 4, L = 24, 2^18 slots  34000 points 69.1 -> 53.9, 50000 points 77.8 -> 64.0 (6 M), 92000 points 102 -> 107
+//   D = 5, 2^18 slots          31250 points 58.7 -> 43.8 (3 M), 42700 points 63.8 -> 62.0, 52000 points 74.3 -> 79.8 (5 M)
+//   D = 8, 2^18 slots          2000 points 40.1 -> 22.6, 2^15 points 71.1 -> 66.6 (4.7 M), 2^16 points 101 -> 137
+//   D = 2, F = 4, 2^16 slots   2^12 points 34.5 -> 19.5;  D = 4, F = 8, 2^18 slots  2^16 points 171 -> 142 (5.2 M), 2^17 points 259 -> 272
+// And up to 4096 points to a level and pair of features: a level's records are summed by as many workgroups as it has ranges,
+// and with many points on few levels those with a coarse level's slots end last (six levels of 2^12 slots, D = 2, 83000
+// points 26.7 -> 32.9, 228000 points 44.8 -> 71.6; of 2^18 slots, D = 3, 62500 points 36.4 -> 42.3; eight of 2^14, D = 5, 31000 points
+// 52.5 -> 36.9, 85000 points 65.5 -> 93.4).
 // Writing every slot once is what a dense gradient costs either way; a batch that leaves most of a large table empty is better served
 // by a fill and a few direct adds (24 levels: 2^20 slots, 500 points 43 -> 47, 2^12 points 55 -> 57; 2^22 slots, 2^12 points 211 -> 232,
 // 2^14 points 290 -> 261).  Sparse gradients have no fill to save and pay for every range that got one record: 2^20
 // slots, 2^12 points 55 -> 88, 2^14 points 126 -> 101; 2^18 slots, 2000 points 29 -> 36, 2^15 points 56 -> 54.5.
-constexpr int64_t kGroupSortMaxLookups = int64_t{1} << 22, kGroupSortSlotsPerLookup = 64, kGroupSortSparseSlotsPerLookup = 16;
+constexpr int64_t group_sort_max_lookups(int pos_dim) { return pos_dim == 3 || pos_dim == 4 ? int64_t{6} << 20 : int64_t{4} << 20; }
+constexpr int64_t kGroupSortPointsPerLevel = 4096, kGroupSortSlotsPerLookup = 64, kGroupSortSparseSlotsPerLookup = 16;
 constexpr uint32_t kRangeSlotsLog2 = 12, kRangeMinSlotsLog2 = 9, kRangeWorkgroupsWanted = 512, kRangeManyGroups = 32;
 constexpr size_t kGroupSortAnyFillBytes = size_t{64} << 20;
 inline bool group_sort_serves(int pos_dim, int64_t n, int levels, int feat_pairs, int capacity, bool sparse) {
     const int64_t lookups = n * (pos_dim + 1);
-    if (lookups * levels > kGroupSortMaxLookups || capacity > (kGroupMaxRanges << kBinSlotsLog2)) return false;
+    if (lookups * levels > group_sort_max_lookups(pos_dim) || n > kGroupSortPointsPerLevel * levels * feat_pairs || capacity > (kGroupMaxRanges << kBinSlotsLog2)) return false;
     if (sparse) return capacity <= kGroupSortSparseSlotsPerLookup * lookups;
     return static_cast<size_t>(capacity) * levels * feat_pairs * sizeof(float2) <= kGroupSortAnyFillBytes || capacity <= kGroupSortSlotsPerLookup * lookups;
 }
@@ -1391,7 +1400,7 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
     }
     const size_t binned = per_level * static_cast<size_t>(levels_per_pass) + direct_flag_bytes(nr_levels, n_bins) + 1024;
     // (how many pairs of features share a level is not known here: up to four)
-    const bool may_sort = levels_per_pass == nr_levels && nr_positions * (pos_dim + 1) * ((nr_levels + 3) / 4) <= kGroupSortMaxLookups;
+    const bool may_sort = levels_per_pass == nr_levels && nr_positions * (pos_dim + 1) * ((nr_levels + 3) / 4) <= group_sort_max_lookups(pos_dim);
     const size_t sorted = may_sort ? group_sort_bytes(pos_dim, nr_positions, nr_levels) + 256 : 0;
     return sorted > binned ? sorted : binned;
 }

@@ -449,8 +449,13 @@ range_sum_kernel(GroupSort sort, const float* __restrict__ window, uint32_t capa
     // it reads what nobody has written, and the result is not used)
     uint32_t first, end;
     stretch(reader, first, end);
-    const bool masked = window[level] == 0.0f;
-    if (masked && touched != nullptr) return;
+    float* const out = table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2;
+    if (window[level] == 0.0f) {
+        if (touched != nullptr) return;
+        for (uint32_t s = threadIdx.x; s < slots && slot0 + s < capacity; s += kRangeBlock)
+            *reinterpret_cast<float2*>(out + static_cast<size_t>(slot0 + s) * 2 * feat_pairs) = make_float2(0.0f, 0.0f);
+        return;
+    }
     double* const acc0 = sums;
     double* const acc1 = sums + slots;
     for (uint32_t s = threadIdx.x; s < slots; s += kRangeBlock) {
@@ -459,28 +464,26 @@ range_sum_kernel(GroupSort sort, const float* __restrict__ window, uint32_t capa
     }
     bool any = false;
     __syncthreads();
-    if (!masked) {
-        for (uint32_t g = reader; g < sort.n_groups; g += readers) {
-            if (g != reader) stretch(g, first, end);
-            any = any || end > first;
-            const uint16_t* const slot_of = sort.slots + (static_cast<size_t>(level) * sort.n_groups + g) * sort.records;
-            const RecordValues* const value_of = sort.values + ((static_cast<size_t>(level) * feat_pairs + pair) * sort.n_groups + g) * sort.records;
-            constexpr uint32_t kTogether = 4;
-            for (uint32_t k = first + l; k < end; k += kTogether * lanes) {
-                uint32_t cell[kTogether];
-                RecordValues v[kTogether];
+    for (uint32_t g = reader; g < sort.n_groups; g += readers) {
+        if (g != reader) stretch(g, first, end);
+        any = any || end > first;
+        const uint16_t* const slot_of = sort.slots + (static_cast<size_t>(level) * sort.n_groups + g) * sort.records;
+        const RecordValues* const value_of = sort.values + ((static_cast<size_t>(level) * feat_pairs + pair) * sort.n_groups + g) * sort.records;
+        constexpr uint32_t kTogether = 4;
+        for (uint32_t k = first + l; k < end; k += kTogether * lanes) {
+            uint32_t cell[kTogether];
+            RecordValues v[kTogether];
 #pragma unroll
-                for (uint32_t u = 0; u < kTogether; ++u) {
-                    const uint32_t at = k + u * lanes < end ? k + u * lanes : k;
-                    cell[u] = slot_of[at];
-                    v[u] = value_of[at];
-                }
+            for (uint32_t u = 0; u < kTogether; ++u) {
+                const uint32_t at = k + u * lanes < end ? k + u * lanes : k;
+                cell[u] = slot_of[at];
+                v[u] = value_of[at];
+            }
 #pragma unroll
-                for (uint32_t u = 0; u < kTogether; ++u) {
-                    if (k + u * lanes < end) {
-                        __hip_atomic_fetch_add(&acc0[cell[u]], static_cast<double>(v[u].x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        __hip_atomic_fetch_add(&acc1[cell[u]], static_cast<double>(v[u].y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    }
+            for (uint32_t u = 0; u < kTogether; ++u) {
+                if (k + u * lanes < end) {
+                    __hip_atomic_fetch_add(&acc0[cell[u]], static_cast<double>(v[u].x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(&acc1[cell[u]], static_cast<double>(v[u].y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
             }
         }
@@ -494,7 +497,6 @@ range_sum_kernel(GroupSort sort, const float* __restrict__ window, uint32_t capa
     } else {
         __syncthreads();
     }
-    float* const out = table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2;
     for (uint32_t s = threadIdx.x; s < slots; s += kRangeBlock) {
         if (slot0 + s >= capacity) break;
         float2* const cell = reinterpret_cast<float2*>(out + static_cast<size_t>(slot0 + s) * 2 * feat_pairs);

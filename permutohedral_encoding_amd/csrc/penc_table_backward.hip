@@ -348,15 +348,23 @@ group_sort_kernel(int n_points, uint32_t n_levels, uint32_t feat_pairs, uint32_t
         });
     }
     const bool ordered = neighbours_share_slots(slot[0], active);
-    const uint32_t across = static_cast<uint32_t>(__shfl_xor(static_cast<int>(slot[0]), 32));
-    const uint32_t same = __popcll(__ballot(lane < 32 && mine + 32 < n_points && across == slot[0]));
+    // (each lane but the last points' against those 16, 32 and 48 away)
+    uint32_t same = 0;
+#pragma unroll
+    for (int away = 16; away < 64; away += 16) {
+        const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(slot[0]), away));
+        same += __popcll(__ballot((lane & (away == 16 ? 16u : 32u)) == 0u && mine + 48 < n_points && other == slot[0]));
+    }
     __syncthreads();  // the counters and lines are cleared
     if (lane == 0 && same != 0u) atomicAdd(&repeats, same);
     __syncthreads();
-    // of 256 pairs of lanes half a wave apart, about 256 / (distinct slots) meet
+    // of 768 pairs of lanes, about 768 / (distinct slots) meet, and the level's other vertices have as many slots each: lines for
+    // up to 384 slots of a group, which then fit, and as many copies of a slot as leave its lines room (about 300 of 512)
     const uint32_t met = repeats;
-    const bool few = met >= 2u && n_points > kGroupLinesMinPoints;
-    const uint32_t copies_log2 = met >= 16u ? 4u : (met >= 4u ? 2u : 1u);
+    const bool few = met >= 2u * (D + 1) && n_points > kGroupLinesMinPoints;
+    uint32_t copies_log2 = 0;
+#pragma unroll
+    for (uint32_t c = 1; c <= 4; ++c) copies_log2 += 2u * met >= (5u * (D + 1) << c) ? 1u : 0u;
     const uint32_t my_copy = lane & ((1u << copies_log2) - 1u);
     // where each contribution goes: kNone (it has none), kLine | its line, or its place among the group's records
     constexpr uint32_t kNone = 0xFFFFFFFFu, kLine = 0x80000000u;

@@ -287,7 +287,8 @@ def test_all_levels_of_a_block_of_points(d, n, levels, cap, feat, concat):
 
 @pytest.mark.parametrize("d,n,levels,cap,feat,finest", [(3, 1, 24, 64, 2, 1e-3), (2, 511, 3, (1 << 12) + 1, 8, 1e-3), (3, 512, 9, 1 << 18, 2, 1e-3), (4, 513, 5, 50001, 4, 1e-3),
                                                         (8, 1025, 4, 1 << 20, 2, 1e-3), (3, 9001, 24, 1 << 16, 2, 0.5), (2, 20001, 4, 1000, 4, 0.3), (3, 65536, 16, 1 << 12, 2, 1e-2),
-                                                        (5, 17000, 3, (1 << 22) - 3, 2, 1e-3)])
+                                                        (5, 17000, 3, (1 << 22) - 3, 2, 1e-3), (5, 12000, 3, (1 << 22) - 3, 2, 1e-3), (4, 12289, 4, 1 << 14, 2, 0.2),
+                                                        (3, 65537, 17, 1 << 14, 2, 1e-2), (8, 4101, 2, 1 << 12, 4, 0.4)])
 def test_sorted_groups_give_the_table_gradient(d, n, levels, cap, feat, finest):
     """Table gradients of small batches, dense (over what the memory held) and added twice into a sparse one: edges of groups and of slot
     ranges, one range and 512, ranges narrower than a range of the touched map, levels of a few slots, a masked level; within the bound
