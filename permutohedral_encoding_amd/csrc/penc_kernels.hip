@@ -619,8 +619,14 @@ simplex_debug_kernel(int n_points, uint32_t capacity, uint32_t cap_mask, const f
 // kernels read (the reference does this with a strided `.contiguous()` copy,
 // src/pytorch_modules/funcs.py:47).  Each workgroup moves kTransposeRows rows through LDS: the
 // read is one contiguous chunk, every write a run of 64 consecutive floats.
+// A thread issues the loads of kTogether values together, as many as it has up to eight: with one load per trip a workgroup
+// waited a dozen times (2^20 rows of 48 columns 98.1 -> 78.7 us, a copy of the array takes 74; 100000 of 96 22.2 -> 13.7;
+// 200001 of 48 16.9 -> 15.4; fewer for few columns, of which a thread has one value to every four: 2^20 rows of 12 19.9 with one,
+// 18.0 with four, 25.8 with eight).
 constexpr int kTransposeRows = 64;  // rows per workgroup: one wavefront-wide run per written column
+constexpr int kTransposeManyColumns = 32;
 
+template <int kTogether>
 __global__ void __launch_bounds__(kBlock)
 transpose_kernel(const float* __restrict__ src, int64_t src_row_stride, float* __restrict__ dst, int64_t rows, int cols) {
     extern __shared__ float tile[];  // kTransposeRows x (cols | 1)
@@ -631,14 +637,24 @@ transpose_kernel(const float* __restrict__ src, int64_t src_row_stride, float* _
     const int n_values = n_rows * cols;
     int r = threadIdx.x / cols, c = threadIdx.x % cols;
     const int dr = kBlock / cols, dc = kBlock % cols;
-    for (int i = threadIdx.x; i < n_values; i += kBlock) {
-        tile[r * stride + c] = chunk[r * src_row_stride + c];
-        r += dr;
-        c += dc;
-        if (c >= cols) {
-            c -= cols;
-            ++r;
+    for (int i = threadIdx.x; i < n_values; i += kTogether * kBlock) {
+        float v[kTogether];
+        int at[kTogether];
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u) {
+            const bool in = i + u * kBlock < n_values;
+            at[u] = in ? r * stride + c : -1;
+            v[u] = chunk[in ? r * src_row_stride + c : 0];
+            r += dr;
+            c += dc;
+            if (c >= cols) {
+                c -= cols;
+                ++r;
+            }
         }
+#pragma unroll
+        for (int u = 0; u < kTogether; ++u)
+            if (at[u] >= 0) tile[at[u]] = v[u];
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -650,6 +666,7 @@ transpose_kernel(const float* __restrict__ src, int64_t src_row_stride, float* _
 // dst[n][F * level + feature] of `dst_row_stride` floats (what a layer that wants contiguous rows reads; the
 // reference's permute + reshape, src/pytorch_modules/modules.py:87, leaves that copy to the consumer).  Every
 // read is a run of 64 consecutive floats, the write one contiguous chunk when the rows are dense.
+template <int kTogether>
 __global__ void __launch_bounds__(kBlock)
 transpose_to_rows_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t dst_row_stride, int64_t rows, int cols) {
     extern __shared__ float tile[];  // kTransposeRows x (cols | 1)
@@ -658,8 +675,17 @@ transpose_to_rows_kernel(const float* __restrict__ src, float* __restrict__ dst,
     const int stride = cols | 1;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane < n_rows)
-        for (int col = wave; col < cols; col += kBlock / 64)
-            tile[lane * stride + col] = __builtin_nontemporal_load(src + static_cast<int64_t>(col) * rows + row0 + lane);
+        for (int first = wave; first < cols; first += kTogether * (kBlock / 64)) {
+            float v[kTogether];
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) {
+                const int col = first + u * (kBlock / 64) < cols ? first + u * (kBlock / 64) : first;
+                v[u] = __builtin_nontemporal_load(src + static_cast<int64_t>(col) * rows + row0 + lane);
+            }
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u)
+                if (first + u * (kBlock / 64) < cols) tile[lane * stride + first + u * (kBlock / 64)] = v[u];
+        }
     __syncthreads();
     float* chunk = dst + row0 * dst_row_stride;
     const int n_values = n_rows * cols;
@@ -1304,7 +1330,7 @@ static int transpose_rows(const float* src, int64_t src_row_stride, float* dst, 
     const size_t lds = static_cast<size_t>(kTransposeRows) * (cols | 1) * sizeof(float);
     if (cols <= 0 || cols > 255 || lds > 64 * 1024) return PENC_ERR_BAD_SIZE;
     const unsigned blocks = static_cast<unsigned>((rows + kTransposeRows - 1) / kTransposeRows);
-    hipLaunchKernelGGL(transpose_kernel, dim3(blocks), dim3(kBlock), lds, st, src, src_row_stride, dst, rows, cols);
+    hipLaunchKernelGGL(cols <= 8 ? transpose_kernel<2> : cols < kTransposeManyColumns ? transpose_kernel<4> : transpose_kernel<8>, dim3(blocks), dim3(kBlock), lds, st, src, src_row_stride, dst, rows, cols);
     return check_launch();
 }
 
@@ -1312,7 +1338,7 @@ static int transpose_to_rows(const float* src, float* dst, int64_t dst_row_strid
     const size_t lds = static_cast<size_t>(kTransposeRows) * (cols | 1) * sizeof(float);
     if (cols <= 0 || cols > 255 || lds > 64 * 1024) return PENC_ERR_BAD_SIZE;
     const unsigned blocks = static_cast<unsigned>((rows + kTransposeRows - 1) / kTransposeRows);
-    hipLaunchKernelGGL(transpose_to_rows_kernel, dim3(blocks), dim3(kBlock), lds, st, src, dst, dst_row_stride, rows, cols);
+    hipLaunchKernelGGL(cols <= 8 ? transpose_to_rows_kernel<2> : cols < kTransposeManyColumns ? transpose_to_rows_kernel<4> : transpose_to_rows_kernel<8>, dim3(blocks), dim3(kBlock), lds, st, src, dst, dst_row_stride, rows, cols);
     return check_launch();
 }
 

@@ -345,3 +345,22 @@ def test_position_gradient_groups_the_levels_a_window_leaves(d, n, levels, cap, 
                                      fp.m_random_shift_per_level.data_ptr(), win.data_ptr(), grad.data_ptr(), None, pg.data_ptr(),
                                      memory.data_ptr() if memory is not None else None, memory.numel() if memory is not None else 0, st) == 0
             assert np.all(np.abs(pg.cpu().numpy() - want["grad64"]) <= 1e-6 * want["abs64"] + 1e-30)
+
+
+@pytest.mark.parametrize("levels,n", [(4, 95001), (5, 78063), (6, 65537), (15, 26240), (16, 25001), (33, 12353)])
+def test_rows_and_levels_change_places(levels, n):
+    """8 to 66 columns (two, four and eight loads of a thread together, with and without remainders), odd row counts: the level-major
+    copy of rows and back, and rows of a forward whose table is too large for the kernels that need no transpose, bit for bit."""
+    from permutohedral_encoding_amd import _native
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    cols, cap = 2 * levels, 1 << 19
+    rows, back = torch.randn(n, cols, device="cuda"), torch.empty(cols, n, device="cuda")
+    assert lib.penc_transpose(rows.data_ptr(), back.data_ptr(), n, cols, st) == 0 and torch.equal(back, rows.t())
+    fp = _native.EncodingFixedParams(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels).astype(np.float32), torch.randn(levels, 3, device="cuda"), False, 1.0)
+    pos, table, win = torch.rand(n, 3, device="cuda"), torch.randn(levels, cap, 2, device="cuda"), torch.ones(levels, device="cuda")
+    args = (3, 2, n, levels, cap, pos.data_ptr(), table.data_ptr(), fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(), win.data_ptr())
+    ws = torch.empty(lib.penc_forward_rowmajor_workspace_bytes(3, 2, n, levels, 0), dtype=torch.uint8, device="cuda")
+    out, dense = torch.empty(cols, n, device="cuda"), torch.full((n, cols + 2), 7.0, device="cuda")
+    assert lib.penc_forward(*args, out.data_ptr(), 0, 1.0, st) == 0
+    assert lib.penc_forward_rowmajor(*args, dense.data_ptr(), cols + 2, 0, 1.0, ws.data_ptr(), ws.numel(), st) == 0
+    assert torch.equal(dense[:, :cols], out.t()) and torch.all(dense[:, cols:] == 7.0)
