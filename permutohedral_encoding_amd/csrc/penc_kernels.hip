@@ -1426,7 +1426,8 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
     }
     const size_t binned = per_level * static_cast<size_t>(levels_per_pass) + direct_flag_bytes(nr_levels, n_bins) + 1024;
     // (how many pairs of features share a level is not known here: up to four)
-    const bool may_sort = levels_per_pass == nr_levels && nr_positions * (pos_dim + 1) * ((nr_levels + 3) / 4) <= group_sort_max_lookups(pos_dim);
+    const bool may_sort = levels_per_pass == nr_levels && nr_positions * (pos_dim + 1) * ((nr_levels + 3) / 4) <= group_sort_max_lookups(pos_dim) &&
+                          nr_positions <= kGroupSortPointsPerLevel * nr_levels;
     const size_t sorted = may_sort ? group_sort_bytes(pos_dim, nr_positions, nr_levels) + 256 : 0;
     return sorted > binned ? sorted : binned;
 }
