@@ -143,6 +143,14 @@ def bridge():
     return _bridge
 
 
+def bridge_if_built():
+    """``bridge()``, or None where it cannot be loaded: for what can be computed without it, on a host without a GPU too."""
+    try:
+        return bridge()
+    except (RuntimeError, OSError, AttributeError):
+        return None
+
+
 def _check(status, what):
     if status != 0:
         msg = lib().penc_status_string(status).decode()

@@ -13,9 +13,11 @@
 // difference in form: the result is the (N, F(L+E)) view the module hands out rather than the (L+E, F, N)
 // array behind it (reference: src/pytorch_modules/modules.py:87), so that the permute and reshape need no nodes.
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
@@ -745,14 +747,25 @@ PyObject* adamw(PyObject* const* args, Py_ssize_t n_args, bool sparse) {
 PyObject* py_adamw_step(PyObject*, PyObject* const* args, Py_ssize_t n) { return adamw(args, n, false); }
 PyObject* py_adamw_step_sparse(PyObject*, PyObject* const* args, Py_ssize_t n) { return adamw(args, n, true); }
 
+// Whether something has to see tensor operations instead of values written through a pointer: a trace records them, a
+// torch-dispatch mode (fake tensors, which have no memory, among them), a functorch transform and a torch-function mode (such
+// as the one that sets a default device) run something else in their place.
+bool operations_are_observed() {
+    return torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           at::impl::PythonTorchFunctionTLS::stack_len() > 0;
+}
+
 // cosine_window(n, alpha) -> the window of utils.cosine_easing_window, which is what a coarse-to-fine schedule computes in every
 // step: 0.5 * (1 + cos(pi * clip(alpha - k, 0, 1) + pi)) in single precision, each operation rounded as torch rounds it (its
 // cosine is torch's own); as six tensor operations from the interpreter it cost 18 us, more than the encoding of a small batch.
+// None where those operations are observed.
 PyObject* py_cosine_window(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
         TORCH_CHECK(n_args == 2, "cosine_window takes 2 arguments");
+        if (operations_are_observed()) Py_RETURN_NONE;
         const int64_t n = PyLong_AsLongLong(args[0]);
-        const float alpha = static_cast<float>(PyFloat_AsDouble(args[1]));
+        const float alpha = PyLong_Check(args[1]) ? static_cast<float>(PyLong_AsLongLong(args[1])) : static_cast<float>(PyFloat_AsDouble(args[1]));
         if (PyErr_Occurred()) return nullptr;
         const float pi = static_cast<float>(3.14159265358979323846);
         at::NoGradGuard no_grad;

@@ -3,7 +3,7 @@ import math
 
 import torch
 
-from ._native import bridge
+from . import _native
 
 
 def cosine_easing_window(num_freqs, alpha):
@@ -12,9 +12,13 @@ def cosine_easing_window(num_freqs, alpha):
     ``win[k] = 0.5 * (1 + cos(pi * clip(alpha - k, 0, 1) + pi))``: exactly 1 for fully eased-in
     levels, exactly 0 for levels not yet started (reference: utils.py:5-16).
     """
-    # (a torch-function mode, such as the one that sets a default device, has to see the tensor operations)
-    if isinstance(num_freqs, int) and isinstance(alpha, (int, float)) and torch._C._len_torch_function_stack() == 0:
-        return bridge().cosine_window(num_freqs, alpha)  # the same, natively
+    # The same natively, for a plain step number and where nothing observes the tensor operations (None); the bools, arrays
+    # and symbols that are numbers too take the operations' own rules, and a compiler sees only these.
+    if type(num_freqs) is int and type(alpha) in (int, float) and not torch.compiler.is_compiling():
+        native = _native._bridge or _native.bridge_if_built()
+        window = native.cosine_window(num_freqs, alpha) if native is not None else None
+        if window is not None:
+            return window
     x = torch.clip(alpha - torch.arange(num_freqs, dtype=torch.float32), 0.0, 1.0)
     return 0.5 * (1 + torch.cos(math.pi * x + math.pi))
 
