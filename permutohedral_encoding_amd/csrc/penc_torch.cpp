@@ -399,6 +399,14 @@ constexpr const char* kSecondTime =
     "Trying to backward through the graph a second time (or directly access saved tensors after they have already been freed). "
     "Specify retain_graph=True if you need to backward through the graph a second time.";
 
+// The nodes compute through raw pointers: a forward-mode tangent on a gradient that reaches them would be lost, and the result
+// would come back with a derivative of zero.
+void refuse_tangents(const variable_list& grads) {
+    for (const Tensor& g : grads)
+        TORCH_CHECK_NOT_IMPLEMENTED(!g.defined() || !g._fw_grad(/*level=*/0).defined(),
+                                    "forward-mode differentiation of the encoding's gradients is not implemented: an incoming gradient has a tangent");
+}
+
 // Whether a gradient sent along this edge ends in the .grad of a row-major leaf, which keeps the leaf's layout: autograd
 // would bring a level-major gradient into it with a strided copy, at a third of the speed of the library's transpose.  (Any other
 // consumer, such as the products of a network's double backward, takes the strided view as it is.)
@@ -475,6 +483,7 @@ struct EncodeBackNode : public Node {
     variable_list apply(variable_list&& grads) override {
         variable_list out(3);
         if (grads.size() < 2 || !grads[1].defined()) return out;
+        refuse_tangents(grads);
         Tensor saved;
         {
             std::lock_guard<std::mutex> lock(mutex_);
@@ -508,6 +517,7 @@ struct EncodeBackNode : public Node {
 variable_list EncodeNode::apply(variable_list&& grads) {
     variable_list out(2);
     const Call& c = *call;
+    refuse_tangents(grads);
     std::vector<SecondOrderTerm> terms = take(torch::autograd::get_current_graph_task_id());
     const bool first_order = !grads.empty() && grads[0].defined();  // undefined: reached through a double backward alone
     const bool want_table = c.want_table && task_should_compute_output(0);
@@ -648,9 +658,9 @@ Tensor window_on_device(const Tensor& window, const at::Device& device) {
 
 // Whether something has to see the autograd functions of funcs.py: a functorch transform or a forward-mode tangent, which they
 // refuse, or a trace, which records them.
-bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positions) {
+bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positions, const Tensor& window) {
     return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing() ||
-           lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined();
+           lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined() || window._fw_grad(0).defined();
 }
 
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
@@ -662,12 +672,12 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
         const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
         const Tensor& positions = tensor_arg(args[2], "positions");
-        if (needs_autograd_functions(lattice_values, positions)) Py_RETURN_NONE;
+        Tensor window = tensor_arg(args[3], "anneal_window");
+        if (needs_autograd_functions(lattice_values, positions, window)) Py_RETURN_NONE;
         auto call = std::make_shared<Call>();
         Call& c = *call;
         c.lattice_values = lattice_values;
         c.table = tensor_arg(args[1], "lattice_values");
-        Tensor window = tensor_arg(args[3], "anneal_window");
         c.shift = tensor_arg(args[4], "random_shift_per_level");
         c.scale_factor = tensor_arg(args[5], "scale list");
         c.pos_dim = static_cast<int>(PyLong_AsLong(args[6]));

@@ -147,6 +147,34 @@ def test_native_path_refuses_what_the_autograd_functions_refuse():
             torch.vmap(m)(pts[None])
 
 
+def test_forward_mode_tangents_are_refused_and_not_dropped():
+    """On an upstream gradient (dual weights of the layers after the encoding), on what comes back through a position gradient
+    (with and without create_graph) and on the window."""
+    fa = torch.autograd.forward_ad
+    dual = lambda t: fa.make_dual(t, torch.ones_like(t))
+    refused = lambda: pytest.raises(NotImplementedError, match="jvp|forward-mode")
+    pts = torch.rand(300, 3, device="cuda")
+    for m in modules():
+        p, weights = pts.clone().requires_grad_(True), torch.randn(m.output_dims(), 1, device="cuda")
+        for graph in (False, True):
+            out = m(p)
+            with fa.dual_level(), refused():
+                torch.autograd.grad((out @ dual(weights)).sum(), p, create_graph=graph)
+            with fa.dual_level(), refused():
+                torch.autograd.grad(m(pts), m.lattice_values, dual(torch.ones_like(out)), create_graph=graph)
+        for window in (torch.ones(5, device="cuda"), torch.ones(5), torch.ones(5, dtype=torch.float64)):
+            with fa.dual_level(), refused():
+                m(pts, dual(window))
+            with fa.dual_level(), torch.no_grad(), refused():
+                m(pts, dual(window))
+    native, _ = modules()
+    for graph in (False, True):
+        for inputs in ([weights.requires_grad_(True)], [native.lattice_values], [native.lattice_values, weights]):
+            normal, = torch.autograd.grad((native(p) @ weights).sum(), p, create_graph=True)
+            with fa.dual_level(), refused():
+                torch.autograd.grad(normal, inputs, dual(torch.ones_like(normal)), create_graph=graph)
+
+
 def test_hooks_on_the_encoding_do_not_run_in_a_pass_through_its_position_gradient_alone():
     results = []
     for m in modules():
