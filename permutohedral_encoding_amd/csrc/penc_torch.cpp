@@ -30,6 +30,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <algorithm>
 #include <memory>
@@ -663,7 +664,7 @@ bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positi
            lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined() || window._fw_grad(0).defined();
 }
 
-// encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
+// encode(lattice_values, table, positions, window, random_shift, fixed_params, pos_dim, nr_feat, concat_points, points_scaling,
 //        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None)
 //   -> (N, F(L+E)), or None where the autograd functions are needed
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
@@ -679,7 +680,10 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.lattice_values = lattice_values;
         c.table = tensor_arg(args[1], "lattice_values");
         c.shift = tensor_arg(args[4], "random_shift_per_level");
-        c.scale_factor = tensor_arg(args[5], "scale list");
+        THPObjectPtr scale_factor(PyObject_GetAttrString(args[5], "m_scale_factor"));
+        if (!scale_factor) return nullptr;
+        c.scale_factor = tensor_arg(scale_factor.get(), "scale list");
+        const at::Device scale_device = c.scale_factor.device();
         c.pos_dim = static_cast<int>(PyLong_AsLong(args[6]));
         c.feat = static_cast<int>(PyLong_AsLong(args[7]));
         c.concat = PyObject_IsTrue(args[8]);
@@ -700,6 +704,10 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             prepare_call(c, positions, window);
             const c10::DeviceGuard device(c.device());
             out = compute_forward(c);
+        }
+        if (c.scale_factor.device() != scale_device) {  // the module was moved: kept where the points are, so that the next call need not copy
+            THPObjectPtr moved(THPVariable_Wrap(c.scale_factor));
+            if (!moved || PyObject_SetAttrString(args[5], "m_scale_factor", moved.get()) != 0) return nullptr;
         }
         if (c.want_table || c.want_positions) {
             auto node = std::shared_ptr<EncodeNode>(new EncodeNode(), torch::autograd::deleteNode);

@@ -227,6 +227,30 @@ def test_a_window_in_host_memory_is_not_captured():
     torch.cuda.synchronize()
 
 
+def test_a_module_moved_to_the_gpu_copies_its_scale_factors_once():
+    native, _ = modules(device="cpu")
+    assert native.fixed_params.m_scale_factor.device.type == "cpu"
+    native.cuda()
+    pts, stream = torch.rand(300, 3, device="cuda"), torch.cuda.Stream()
+    want = native(pts)
+    moved = native.fixed_params.m_scale_factor
+    assert moved.is_cuda
+    with torch.no_grad():
+        native(pts)
+    assert native.fixed_params.m_scale_factor is moved
+    # a call that copied could not be captured
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(stream):
+        native(pts)
+        graph = torch.cuda.CUDAGraph()
+        graph.capture_begin()
+        out = native(pts)
+        graph.capture_end()
+        graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 def test_upstream_gradient_modified_before_the_double_backward_is_refused():
     native, _ = modules()
     p = torch.rand(100, 3, device="cuda", requires_grad=True)
