@@ -360,7 +360,8 @@ class EncodingWrapper:
     def encode(self, lattice_values, positions, anneal_window):
         """-> the encoding (N, F(L+E)) of ``positions``, differentiable as ``funcs.py`` makes it, natively:
         one call into the extension, whose autograd nodes reach the library without entering the interpreter.
-        None under a functorch transform, with a forward-mode tangent and in a trace: those are for the functions of ``funcs.py``."""
+        None under a functorch transform, with a forward-mode tangent, with a window that requires a gradient and in a trace: those
+        are for the functions of ``funcs.py``."""
         fp = self.fixed_params
         return (_bridge or bridge()).encode(
             lattice_values, lattice_values if self.half_table is None else self.gather_table(lattice_values), positions,

@@ -658,10 +658,11 @@ Tensor window_on_device(const Tensor& window, const at::Device& device) {
 }
 
 // Whether something has to see the autograd functions of funcs.py: a functorch transform or a forward-mode tangent, which they
-// refuse, or a trace, which records them.
+// refuse, a trace, which records them, or a window that requires a gradient, which makes their result require one.
 bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positions, const Tensor& window) {
     return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing() ||
-           lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined() || window._fw_grad(0).defined();
+           lattice_values._fw_grad(0).defined() || positions._fw_grad(0).defined() || window._fw_grad(0).defined() ||
+           (window.requires_grad() && c10::GradMode::is_enabled());
 }
 
 // encode(lattice_values, table, positions, window, random_shift, fixed_params, pos_dim, nr_feat, concat_points, points_scaling,

@@ -175,6 +175,22 @@ def test_forward_mode_tangents_are_refused_and_not_dropped():
                 torch.autograd.grad(normal, inputs, dual(torch.ones_like(normal)), create_graph=graph)
 
 
+def test_a_window_that_requires_a_gradient_gets_none_and_is_not_ignored():
+    """Its result requires a gradient too, and a backward that nothing but the window asks for is refused."""
+    pts = torch.rand(300, 3, device="cuda")
+    for m in modules():
+        window = torch.ones(5, device="cuda", requires_grad=True)
+        m(pts, window).sum().backward()
+        assert window.grad is None and m.lattice_values.grad is not None
+        m.lattice_values.requires_grad_(False)
+        out = m(pts, window)
+        assert out.requires_grad
+        with pytest.raises(AssertionError, match="neither lattice_values nor positions"):
+            out.sum().backward()
+        with torch.no_grad():
+            assert not m(pts, window).requires_grad
+
+
 def test_hooks_on_the_encoding_do_not_run_in_a_pass_through_its_position_gradient_alone():
     results = []
     for m in modules():
