@@ -333,6 +333,9 @@ Gradients compute_positions_backward(const Call& c, Upstream& up) {
                                           up.row_stride, mutable_data(level_major), mutable_data(g.positions), workspace_of(ws),
                                           workspace_size(ws), current_stream(c.device())),
           "backward_positions");
+    // (the columns of concatenated points carry no gradient and are not read, but whoever saves the copy sees the whole of it)
+    const int64_t encoded = static_cast<int64_t>(c.feat) * c.levels;
+    if (c.extra != 0) level_major.narrow(1, encoded, c.columns() - encoded).copy_(up.values.narrow(1, encoded, c.columns() - encoded));
     up = {level_major, 0};
     return g;
 }
@@ -535,7 +538,6 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         if (first_order) {
             check_saved();
             up = upstream_of(c, grads[0].detach());
-            // (columns of concatenated points carry no gradient: the copy's last rows stay unwritten and are never read)
             if (differentiable && want_positions && !want_table && up.row_stride != 0 && c.columns() <= 255) {
                 g = compute_positions_backward(c, up);
             } else {

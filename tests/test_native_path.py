@@ -277,6 +277,23 @@ def test_upstream_gradient_modified_before_the_double_backward_is_refused():
         normal.sum().backward()
 
 
+@pytest.mark.parametrize("concat", [False, True])
+def test_rows_kept_as_a_copy_are_the_upstream_gradient(concat):
+    """The level-major copy that is kept of rows, as a saved-tensor hook sees it: whole, the columns of concatenated points too."""
+    for m in modules(concat_points=concat):
+        p = torch.rand(4001, 3, device="cuda", requires_grad=True)
+        up, seen = torch.randn(4001, m.output_dims(), device="cuda"), []
+        fill = torch.full((4001, m.output_dims()), float("nan"), device="cuda")  # (what the copy's memory holds before)
+        del fill
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t) or t, lambda t: t):
+            out = m(p)
+            seen.clear()
+            normal, = torch.autograd.grad(out, p, up, create_graph=True)
+        kept, = seen
+        assert torch.equal(kept.permute(2, 0, 1).reshape(up.shape) if kept.dim() == 3 else kept, up)
+        normal.sum().backward()
+
+
 @pytest.mark.parametrize("d,n,levels,cap,rows,feat", [(2, 1, 3, 64, False, 2), (3, 511, 4, 1 << 12, True, 2), (3, 4097, 3, 1 << 20, False, 4), (4, 9000, 5, 50000, True, 2),
                                                       (5, 1025, 2, 1 << 14, False, 2), (6, 700, 2, 1 << 12, True, 2), (8, 5000, 3, 1 << 13, False, 2),
                                                       (3, 600000, 1, (1 << 22) + 5, True, 2)])
