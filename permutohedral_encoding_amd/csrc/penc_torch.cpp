@@ -419,6 +419,25 @@ bool goes_into_row_major_leaf(const torch::autograd::Edge& edge) {
     return leaf != nullptr && leaf->variable.dim() == 2 && leaf->variable.is_contiguous();
 }
 
+// The version a tensor must still be at when a node that did not save the tensor itself runs.
+struct ExpectedVersion {
+    c10::VariableVersion counter;
+    uint32_t expected = 0;
+    bool set = false;
+
+    void expect(const Tensor& t) {
+        TORCH_CHECK(!t.is_inference(), "Inference tensors cannot be saved for backward: make a clone outside of inference mode");
+        counter = torch::autograd::impl::version_counter(t);
+        expected = counter.current_version();
+        set = true;
+    }
+    void check(const char* what) const {
+        TORCH_CHECK(!set || counter.current_version() == expected,
+                    "one of the variables needed for gradient computation has been modified by an inplace operation: ", what, " is at version ",
+                    counter.current_version(), "; expected version ", expected, " instead");
+    }
+};
+
 // Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
 // consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
 // table scatter.
@@ -426,8 +445,7 @@ struct EncodeNode : public Node {
     std::shared_ptr<const Call> call;
     void* forward_stream = nullptr;
     // The result counts as saved, as it does in funcs.py: changing it in place, or a second pass through a freed graph, is refused.
-    c10::VariableVersion result_version;
-    uint32_t expected_version = 0;
+    ExpectedVersion result_version;
     bool released = false;
 
     // A training step on an SDF asks for two table gradients in one pass, through the encoded values and through the
@@ -444,9 +462,7 @@ struct EncodeNode : public Node {
     void check_saved() {
         std::lock_guard<std::mutex> lock(mutex_);
         TORCH_CHECK(!released, kSecondTime);
-        TORCH_CHECK(result_version.current_version() == expected_version,
-                    "one of the variables needed for gradient computation has been modified by an inplace operation: the encoding is at version ",
-                    result_version.current_version(), "; expected version ", expected_version, " instead");
+        result_version.check("the encoding");
     }
 
     void leave(SecondOrderTerm term) {
@@ -478,6 +494,7 @@ struct EncodeBackNode : public Node {
     std::shared_ptr<const Call> call;
     std::shared_ptr<EncodeNode> slicing;
     torch::autograd::SavedVariable upstream;  // saved as autograd saves: version checks, hooks, freed with the graph
+    ExpectedVersion rows_version;             // of the rows `upstream` is a level-major copy of: changing them is refused all the same
 
     std::string name() const override { return "PermutoEncodingBackward2"; }
     void release_variables() override {
@@ -492,6 +509,7 @@ struct EncodeBackNode : public Node {
         {
             std::lock_guard<std::mutex> lock(mutex_);
             saved = upstream.unpack();
+            rows_version.check("the upstream gradient");
         }
         const Call& c = *call;
         const bool grad_mode = c10::GradMode::is_enabled();
@@ -531,6 +549,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
     const bool differentiable = c10::GradMode::is_enabled();
     Upstream up;
     Gradients g;
+    ExpectedVersion rows_version;
     {
         at::NoGradGuard no_grad;
         const c10::DeviceGuard device(c.device());
@@ -539,6 +558,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
             check_saved();
             up = upstream_of(c, grads[0].detach());
             if (differentiable && want_positions && !want_table && up.row_stride != 0 && c.columns() <= 255) {
+                if (up.values.is_alias_of(grads[0])) rows_version.expect(grads[0]);
                 g = compute_positions_backward(c, up);
             } else {
                 if (want_table && !terms.empty()) fused = &terms.back();
@@ -560,6 +580,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         back->add_next_edge(torch::autograd::Edge(back->slicing, 0));
         back->call = call;
         back->upstream = torch::autograd::SavedVariable(up.values, false);
+        back->rows_version = std::move(rows_version);
         torch::autograd::set_history(g.table, back);
         torch::autograd::set_history(g.positions, back);
     }
@@ -717,8 +738,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             node->set_next_edges(torch::autograd::collect_next_edges(lattice_values, positions));
             node->forward_stream = current_stream(call->device());
             node->call = std::move(call);
-            node->result_version = torch::autograd::impl::version_counter(out);
-            node->expected_version = node->result_version.current_version();
+            node->result_version.expect(out);
             auto result = std::shared_ptr<ResultNode>(new ResultNode(), torch::autograd::deleteNode);
             result->add_next_edge(torch::autograd::Edge(node, node->add_input_metadata(out)));
             torch::autograd::set_history(out, result);

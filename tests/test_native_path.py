@@ -279,7 +279,8 @@ def test_upstream_gradient_modified_before_the_double_backward_is_refused():
 
 @pytest.mark.parametrize("concat", [False, True])
 def test_rows_kept_as_a_copy_are_the_upstream_gradient(concat):
-    """The level-major copy that is kept of rows, as a saved-tensor hook sees it: whole, the columns of concatenated points too."""
+    """The level-major copy that is kept of rows, as a saved-tensor hook sees it: whole, the columns of concatenated points too; and
+    changing the rows, or handing over ones that cannot be tracked, before the double backward is refused as if they had been kept."""
     for m in modules(concat_points=concat):
         p = torch.rand(4001, 3, device="cuda", requires_grad=True)
         up, seen = torch.randn(4001, m.output_dims(), device="cuda"), []
@@ -292,6 +293,14 @@ def test_rows_kept_as_a_copy_are_the_upstream_gradient(concat):
         kept, = seen
         assert torch.equal(kept.permute(2, 0, 1).reshape(up.shape) if kept.dim() == 3 else kept, up)
         normal.sum().backward()
+        normal, = torch.autograd.grad(m(p), p, up, create_graph=True)
+        up.mul_(2.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            normal.sum().backward()
+        with torch.inference_mode():
+            untracked = up.clone()
+        with pytest.raises(RuntimeError, match="Inference tensors cannot be saved for backward"):
+            torch.autograd.grad(m(p), p, untracked, create_graph=True)
 
 
 @pytest.mark.parametrize("d,n,levels,cap,rows,feat", [(2, 1, 3, 64, False, 2), (3, 511, 4, 1 << 12, True, 2), (3, 4097, 3, 1 << 20, False, 4), (4, 9000, 5, 50000, True, 2),
