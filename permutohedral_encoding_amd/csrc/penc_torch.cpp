@@ -71,7 +71,6 @@ struct Api {
     PENC_FN(double_backward_from_positions_sparse);
     PENC_FN(adamw_step);
     PENC_FN(adamw_step_sparse);
-    PENC_FN(transpose);
     PENC_FN(upload);
     PENC_FN(backward_positions_rowmajor);
     PENC_FN(grad_grad_rowmajor);
@@ -852,7 +851,6 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(double_backward_from_positions_sparse);
         PENC_FN(adamw_step);
         PENC_FN(adamw_step_sparse);
-        PENC_FN(transpose);
         PENC_FN(upload);
         PENC_FN(backward_positions_rowmajor);
         PENC_FN(grad_grad_rowmajor);
