@@ -398,10 +398,6 @@ SecondOrder compute_double_backward(const Call& c, const Tensor& double_position
 // ------------------------------------------------------------------------------------------
 // autograd
 
-constexpr const char* kSecondTime =
-    "Trying to backward through the graph a second time (or directly access saved tensors after they have already been freed). "
-    "Specify retain_graph=True if you need to backward through the graph a second time.";
-
 // The nodes compute through raw pointers: a forward-mode tangent on a gradient that reaches them would be lost, and the result
 // would come back with a derivative of zero.
 void refuse_tangents(const variable_list& grads) {
@@ -460,7 +456,7 @@ struct EncodeNode : public Node {
     }
     void check_saved() {
         std::lock_guard<std::mutex> lock(mutex_);
-        TORCH_CHECK(!released, kSecondTime);
+        TORCH_CHECK(!released, torch::autograd::ERR_BACKWARD_TWICE);
         result_version.check("the encoding");
     }
 
