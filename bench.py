@@ -44,11 +44,13 @@ HBM_PEAK_GBPS = 8000.0  # MI355X published HBM3E bandwidth
 
 
 def kernel_source_digest():
-    """Identifies the kernel sources a counter summary was taken with (a summary of other sources is stale)."""
+    """Identifies the kernel sources a counter summary was taken with (a summary of other sources is stale): every
+    source of libpenc_hip.so, by name and content."""
     import hashlib
     h = hashlib.sha1()
     csrc = os.path.join(ROOT, "permutohedral_encoding_amd", "csrc")
-    for name in ("penc_kernels.hip", "penc_scatter.hpp", "penc_lattice.hpp"):
+    for name in sorted(n for n in os.listdir(csrc) if n.endswith((".hip", ".hpp")) and n != "penc_probes.hip"):
+        h.update(name.encode())
         with open(os.path.join(csrc, name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]

@@ -253,6 +253,24 @@ def test_workspace_request_is_capped_and_shrinks_when_memory_runs_out(monkeypatc
     assert requests[-1] == 1000
 
 
+def test_source_digest_follows_every_kernel_source(tmp_path, monkeypatch):
+    """A counter summary goes stale with any source of the library: those with the scattering and reducing kernels too."""
+    import shutil
+    import bench
+    csrc = tmp_path / "permutohedral_encoding_amd" / "csrc"
+    shutil.copytree(os.path.join(ROOT, "permutohedral_encoding_amd", "csrc"), csrc, ignore=shutil.ignore_patterns("build"))
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    before = bench.kernel_source_digest()
+    sources = sorted(p.name for p in csrc.iterdir() if p.suffix in (".hip", ".hpp"))
+    assert {"penc_kernels.hip", "penc_table_backward.hip", "penc_reduce.hpp", "penc_scatter.hpp", "penc_group_sort.hpp"} <= set(sources)
+    for name in sources:
+        kept = (csrc / name).read_bytes()
+        (csrc / name).write_bytes(kept + b"// changed\n")
+        assert (bench.kernel_source_digest() == before) == (name == "penc_probes.hip"), name
+        (csrc / name).write_bytes(kept)
+    assert bench.kernel_source_digest() == before
+
+
 def _counter_rows(workload):
     """(phase, kernel) -> (memory-side bytes, vector instructions) from the table of profiles/<workload>_counters.md."""
     rows = {}
