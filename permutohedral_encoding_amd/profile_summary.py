@@ -12,10 +12,10 @@ output in ``trace.log``, and one ``--pmc`` run per counter set into ``fetch/``, 
   profiles/hbm_traffic.json       per workload and phase the sums of those rows, with the rows
                                   themselves, which is what bench.py reads
 
-A dispatch belongs to a phase by what it is, not by its position in a name list: the scattering
-kernel by its second-order template argument, the kernels that serve both gradient calls (the
-fill that clears the gradient, the bin reducers) by the scattering kernel they precede or follow
-in the dispatch order.
+A dispatch belongs to a phase by what it is, not by its position in a name list: the scattering and
+the sorting kernel by their order, the kernels that serve both gradient calls (the
+fill that clears the gradient, the reducers) by the scattering or sorting kernel they precede or follow
+in the dispatch order.  The table gradient of both orders together belongs to the call that computes it, "backward".
 
 Usage: python -m permutohedral_encoding_amd.profile_summary c2 [c3 ...]   (from the repository root)
 """
@@ -46,7 +46,6 @@ COUNTER_SETS = (
     ("ea", " --no-probes", "TCC_EA0_RDREQ_sum TCC_EA0_RDREQ_32B_sum TCC_EA0_WRREQ_sum TCC_EA0_WRREQ_64B_sum"),
 )
 L2_LINE_BYTES = 128        # gfx950: an L2 request from the first-level cache moves at most one 128-byte line
-SHARED = ("fill_zero_kernel", "bin_reduce_kernel", "bin_reduce_levels_kernel", "touched_")
 
 
 def short(name):
@@ -77,35 +76,47 @@ def is_ours(kernel):
                 or "scatter_kernel" in kernel or "simplex_debug" in kernel)
 
 
+def order_of_table_gradient(kernel):
+    """Phase of a kernel that makes records of a table gradient, None for any other kernel."""
+    args = template_args(kernel)
+    if base_name(kernel) == "backward_table_kernel":  # <D, kRowMajor, kSecondOrder, kWideBins>
+        return "double_backward" if len(args) >= 3 and args[2] == "true" else "backward"
+    if base_name(kernel) == "group_sort_kernel":      # <D, kRowMajor, kOrder>: first, second, both
+        return "double_backward" if len(args) >= 3 and args[2] == "2" else "backward"
+    return "backward" if base_name(kernel) == "backward_table_both_kernel" else None
+
+
 def phase_of_dispatches(kernels):
     """Phase ("forward", "backward", "double_backward" or None) of every dispatch of a run, in order."""
     own = []
     for k in kernels:
         b = base_name(k)
-        if not is_ours(k):
+        if not is_ours(k) or b == "upload_kernel":
             own.append(None)
         elif b == "forward_kernel":
             own.append("forward")
-        elif b in ("backward_pos_kernel", "reduce_level_groups_kernel", "transpose_kernel"):
+        elif b in ("backward_pos_kernel", "block_backward_pos_kernel", "reduce_level_groups_kernel", "transpose_kernel"):
             own.append("backward")
         elif b == "grad_grad_kernel":
             own.append("double_backward")
+        elif b == "block_rows_kernel":  # <D, F, T, kSecond>
+            own.append("double_backward" if template_args(k)[-1:] == ["true"] else "forward")
         elif b == "touched_ranges_kernel":
             own.append("clear_touched")
-        elif b == "backward_table_kernel":
-            args = template_args(k)  # <D, kRowMajor, kSecondOrder, kWideBins>
-            own.append("double_backward" if len(args) >= 3 and args[2] == "true" else "backward")
         else:
-            own.append("?")  # serves whichever gradient call launched it
-    scatter_at = [i for i, k in enumerate(kernels) if base_name(k) == "backward_table_kernel"]
+            own.append(order_of_table_gradient(k) or "?")  # "?" serves whichever call launched it
+    records_at = [i for i, k in enumerate(kernels) if order_of_table_gradient(k)]
     for i, k in enumerate(kernels):
         if own[i] != "?":
             continue
         if base_name(k) == "fill_zero_kernel":   # clears the gradient before the scatter
-            after = [j for j in scatter_at if j > i]
+            after = [j for j in records_at if j > i]
             own[i] = own[after[0]] if after else None
-        else:                                     # reduces what the scatter left
-            before = [j for j in scatter_at if j < i]
+        elif base_name(k) == "transpose_to_rows_kernel":  # brings what a gathering kernel wrote into rows
+            before = [j for j in range(i) if base_name(kernels[j]) in ("forward_kernel", "grad_grad_kernel")]
+            own[i] = own[before[-1]] if before else None
+        else:                                     # reduces what the scatter, or the sort, left
+            before = [j for j in records_at if j < i]
             own[i] = own[before[-1]] if before else None
     return own
 

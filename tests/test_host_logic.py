@@ -328,4 +328,10 @@ def test_profile_summary_attributes_shared_kernels_by_dispatch_order():
          "fill_zero_kernel", "backward_table_kernel<4, false, false, false>", "bin_reduce_kernel<true>", "at::native::copy_kernel", "copy_kernel"]
     assert ps.phase_of_dispatches(k) == ["forward", "backward", "backward", "double_backward", "double_backward", "double_backward",
                                          "double_backward", "backward", "backward", "backward", None, None]
+    k = ["block_rows_kernel<3, 2, float, false>", "forward_kernel<3, 2, float>", "transpose_to_rows_kernel<8>", "upload_kernel",
+         "group_sort_kernel<3, true, 1>", "range_sum_kernel", "transpose_kernel<4>", "block_backward_pos_kernel<3, 2, float, true>",
+         "grad_grad_kernel<3, 2, float>", "transpose_to_rows_kernel<8>", "group_sort_kernel<3, false, 2>", "range_sum_kernel",
+         "block_rows_kernel<3, 2, float, true>", "fill_zero_kernel", "backward_table_both_kernel<3, true, false>", "bin_reduce_levels_kernel"]
+    assert ps.phase_of_dispatches(k) == ["forward", "forward", "forward", None, "backward", "backward", "backward", "backward", "double_backward",
+                                         "double_backward", "double_backward", "double_backward", "double_backward", "backward", "backward", "backward"]
     assert ps.short("void penc::backward_table_kernel<3, false, true, false>(int, int)") == "backward_table_kernel<3, false, true, false>"
