@@ -1,6 +1,7 @@
-"""ctypes binding over ``libpenc_hip.so`` (the C ABI declared in ``include/penc.h``).
+"""Binding over ``libpenc_hip.so`` (the C ABI declared in ``include/penc.h``): by ctypes here, and for the module's and the
+optimizers' calls by the extension ``_penc_torch`` (``csrc/penc_torch.cpp``), which ``bridge()`` loads.
 
-This is the only way the package computes anything: there is no CPU or pure-PyTorch fallback.
+This is the only way the package computes an encoding: there is no CPU or pure-PyTorch fallback.
 If the library is missing or a tensor is not on a GPU the call raises.
 
 The classes ``EncodingInput``, ``EncodingFixedParams`` and ``EncodingWrapper`` mirror the three

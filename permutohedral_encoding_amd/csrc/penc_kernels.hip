@@ -1,17 +1,22 @@
 // HIP kernels (gfx950, wave64) and C-ABI entry points of the permutohedral-lattice hash encoding.
 //
-// Work decomposition (one thread per (point, level) everywhere)
-//   forward, grad-of-grad (the gathering half of the double backward) : blockIdx.y is the level, so
-//       consecutive workgroups work on the same 8*capacity-byte slice of the table, which stays in
-//       L2, and the level's scale factors / shifts / window weight are wave-uniform (scalar loads).
-//   position backward : a thread sums a group of two levels in registers; the per-group partial
-//       sums are reduced in a fixed order, without atomics (the reference needs D atomics per
-//       point-level because it gives each level its own block,
+// Work decomposition
+//   forward, grad-of-grad (the gathering half of the double backward) : a thread takes a point at one
+//       level, or at two levels half the list apart.  Workgroups run row by row of levels, and where the
+//       slices are small enough each die keeps its own share of the rows (LevelMap), so that the slices
+//       being gathered from stay in its L2; the level's scale factors / shifts / window weight are
+//       wave-uniform (scalar loads).
+//   position backward : a thread sums a group of two of the levels the window leaves in registers; the
+//       per-group partial sums are reduced in a fixed order, without atomics (the reference needs D
+//       atomics per point-level because it gives each level its own block,
 //       kernels/permutohedral_encoding/EncodingGPU.cuh:745-750).
-//   table backward (first order and the scattering half of the double backward) : workgroups of
-//       512 threads walk groups of 8 or 16 tiles of points; neighbouring workgroups of a die take
+//   small tables and small batches : a workgroup takes 64 points and all their levels, for the position
+//       gradient and for results in rows (block_backward_pos_kernel, block_rows_kernel).
+//   table backward (first order, the scattering half of the double backward, or both) : workgroups of
+//       512 threads walk groups of 2 to 16 tiles of points; neighbouring workgroups of a die take
 //       the same points at different levels.  The scatter itself (LDS accumulate cache, slot-range
-//       bins, direct atomics) is described in penc_scatter.hpp.
+//       bins, direct atomics) is described in penc_scatter.hpp; small and ordinary batches are sorted
+//       by slot range instead (penc_group_sort.hpp).
 //   A level whose anneal-window weight is exactly 0 contributes exactly 0 everywhere (for finite
 //   table values), so such levels skip the table traffic and only store their zeros.
 #include <hip/hip_fp16.h>
@@ -301,8 +306,8 @@ reduce_level_groups_kernel(const float* __restrict__ partial, const float* __res
 
 // ------------------------------------------------------------------------------------------
 // double backward from d(loss)/d(position gradient), the half that gathers: gradient w.r.t.
-// grad_sliced_values (EncodingGPU.cuh:1260-1493).  One thread per (point, level), a level at a
-// time, like the forward.  (The other half, the scatter into the table gradient, is
+// grad_sliced_values (EncodingGPU.cuh:1260-1493).  One thread per point and one or two levels, like
+// the forward.  (The other half, the scatter into the table gradient, is
 // backward_table_kernel<D, false, true>.  One kernel doing both, with eight tiles per workgroup,
 // was measured 7-13% slower than the two: the gathering half wants small workgroups, the scattering
 // half large groups of points with the levels interleaved.)
@@ -820,7 +825,8 @@ inline unsigned scatter_groups(int64_t n, int tiles_per_group) {
 // slower otherwise).  The same rule serves the scattering half of the double backward.
 // Small batches take smaller groups, down to two tiles, until the launch has a workgroup for every slot of
 // the chip (measured at 24 levels, D = 3: 2^16 points 0.074 -> 0.064 ms with four tiles, 2^15 points
-// 0.065 -> 0.055 ms and 2^14 points 0.062 -> 0.048 ms with two; 2^17 points are best with eight).
+// 0.065 -> 0.055 ms and 2^14 points 0.062 -> 0.048 ms with two; 2^17 points are best with eight).  That is for the
+// small batches that the sorted groups below do not take: few levels, sparse or mostly empty gradients, a workspace too small.
 constexpr int64_t kMinWorkgroups = 768;  // three per compute unit
 inline int table_backward_tiles(int64_t n, int levels) {
     if (static_cast<int64_t>(scatter_groups(n, kScatterTilesLarge)) * levels >= kLargeGroupsMinWorkgroups) return kScatterTilesLarge;
