@@ -366,8 +366,8 @@ class EncodingWrapper:
         fp = self.fixed_params
         return (_bridge or bridge()).encode(
             lattice_values, lattice_values if self.half_table is None else self.gather_table(lattice_values), positions,
-            anneal_window, fp.m_random_shift_per_level, fp, self.pos_dim, self.nr_feat, fp.m_concat_points,
-            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES)
+            anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,
+            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES, fp)
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table

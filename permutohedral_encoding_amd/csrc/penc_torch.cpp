@@ -683,12 +683,12 @@ bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positi
            (window.requires_grad() && c10::GradMode::is_enabled());
 }
 
-// encode(lattice_values, table, positions, window, random_shift, fixed_params, pos_dim, nr_feat, concat_points, points_scaling,
-//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None)
+// encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
+//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params)
 //   -> (N, F(L+E)), or None where the autograd functions are needed
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
-        TORCH_CHECK(n_args == 14, "encode takes 14 arguments");
+        TORCH_CHECK(n_args == 15, "encode takes 15 arguments");
         TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
         const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
         const Tensor& positions = tensor_arg(args[2], "positions");
@@ -699,9 +699,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.lattice_values = lattice_values;
         c.table = tensor_arg(args[1], "lattice_values");
         c.shift = tensor_arg(args[4], "random_shift_per_level");
-        THPObjectPtr scale_factor(PyObject_GetAttrString(args[5], "m_scale_factor"));
-        if (!scale_factor) return nullptr;
-        c.scale_factor = tensor_arg(scale_factor.get(), "scale list");
+        c.scale_factor = tensor_arg(args[5], "scale list");
         const at::Device scale_device = c.scale_factor.device();
         c.pos_dim = static_cast<int>(PyLong_AsLong(args[6]));
         c.feat = static_cast<int>(PyLong_AsLong(args[7]));
@@ -726,7 +724,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         }
         if (c.scale_factor.device() != scale_device) {  // the module was moved: kept where the points are, so that the next call need not copy
             THPObjectPtr moved(THPVariable_Wrap(c.scale_factor));
-            if (!moved || PyObject_SetAttrString(args[5], "m_scale_factor", moved.get()) != 0) return nullptr;
+            if (!moved || PyObject_SetAttrString(args[14], "m_scale_factor", moved.get()) != 0) return nullptr;
         }
         if (c.want_table || c.want_positions) {
             auto node = std::shared_ptr<EncodeNode>(new EncodeNode(), torch::autograd::deleteNode);

@@ -14,7 +14,7 @@ def cosine_easing_window(num_freqs, alpha):
     """
     # The same natively, for a plain step number and where nothing observes the tensor operations (None); the bools, arrays
     # and symbols that are numbers too take the operations' own rules, and a compiler sees only these.
-    if type(num_freqs) is int and type(alpha) in (int, float) and not torch.compiler.is_compiling():
+    if type(num_freqs) is int and type(alpha) in (int, float) and not torch.compiler.is_dynamo_compiling():
         native = _native._bridge or _native.bridge_if_built()
         window = native.cosine_window(num_freqs, alpha) if native is not None else None
         if window is not None:
