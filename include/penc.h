@@ -317,6 +317,31 @@ int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, in
                               const float* double_positions_grad, const float* first_grad, float* lattice_values_grad,
                               uint32_t* touched, float* positions_grad, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Position derivatives without gathering from the table again.  Inside its simplex every feature of a level is an affine function of
+ * the position; penc_forward_slopes is penc_forward (penc_forward_half with a table_format) that also leaves each feature's slope in
+ * `slopes` (penc_slopes_bytes() of them; opaque, levels whose window weight is 0 are not written), with the result as rows when
+ * sliced_rows is given (row_stride >= nr_feat*(L+E); sliced_values, the [L+E][F][N] array, is then scratch).  From the slopes and
+ * the same anneal_window,
+ *   penc_backward_positions_slopes  gives the positions_grad of penc_backward (grad_row_stride 0) or penc_backward_rowmajor; for rows,
+ *                                   grad_level_major (optional, [L][F][N]) receives their level-major copy;
+ *   penc_grad_grad_slopes           gives the grad_grad_sliced_values of penc_double_backward_from_positions as [L+E][F][N], or
+ *                                   with row_stride != 0 as rows of that many floats.
+ * The same derivatives to rounding: the differences of vertex values are formed before the products.  Rows hold at most 255 columns.
+ * penc_slopes_bytes() is 0 where nothing would be gained (small batches on tables of at most 1 MiB; many features, whose slopes are as large as the
+ * vertices, on tables an L2 holds) and where rows cannot be served.  The three calls themselves take any geometry.
+ * Replaces: the second and third gather of backward_gpu_only_pos and double_backward_from_positions_gpu_2
+ * (EncodingGPU.cuh:530-769, 1260-1493). */
+size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int table_format);
+int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                        const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
+                        const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
+                        int concat_points, float points_scaling, void* stream);
+int penc_backward_positions_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, const float* slopes,
+                                   const float* anneal_window, const float* grad, int64_t grad_row_stride, float* grad_level_major,
+                                   float* positions_grad, void* stream);
+int penc_grad_grad_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, const float* slopes, const float* anneal_window,
+                          const float* double_positions_grad, float* grad_grad, int64_t row_stride, int concat_points, void* stream);
+
 /* Copies n values from HOST memory to dst as part of the enqueued work: the values travel in the launch (128 at a time), so the
  * call neither waits for the device nor needs the host array afterwards, where a copy from pageable memory
  * does both.  For the few values that change from step to step (the window of a coarse-to-fine schedule).

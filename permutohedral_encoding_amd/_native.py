@@ -99,6 +99,14 @@ _SIGNATURES = {
                                                _c_f32p, ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
                                                _c_f32p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
                                                ctypes.c_void_p]),
+    "penc_slopes_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "penc_forward_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p,
+                                           ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
+                                           ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]),
+    "penc_backward_positions_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p,
+                                                      _c_f32p, ctypes.c_int64, _c_f32p, _c_f32p, ctypes.c_void_p]),
+    "penc_grad_grad_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p,
+                                             _c_f32p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "penc_upload": (ctypes.c_int, [_c_f32p, _c_f32p, ctypes.c_int, ctypes.c_void_p]),
     "penc_transpose": (ctypes.c_int, [_c_f32p, _c_f32p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "penc_simplex_debug": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p, _c_f32p,

@@ -10,6 +10,8 @@
 //       per-group partial sums are reduced in a fixed order, without atomics (the reference needs D
 //       atomics per point-level because it gives each level its own block,
 //       kernels/permutohedral_encoding/EncodingGPU.cuh:745-750).
+//       Where the forward has kept the slopes of the features, both derivatives w.r.t. the positions read those instead of gathering
+//       (penc_slopes.hpp).
 //   small tables and small batches : a workgroup takes 64 points and all their levels, for the position
 //       gradient and for results in rows (block_backward_pos_kernel, block_rows_kernel).
 //   table backward (first order, the scattering half of the double backward, or both) : workgroups of
@@ -31,6 +33,7 @@
 #include "penc_group_sort.hpp"
 #include "penc_reduce.hpp"
 #include "penc_scatter.hpp"
+#include "penc_slopes.hpp"
 #include "penc_table_backward.hpp"
 
 namespace penc {
@@ -156,12 +159,13 @@ __device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile,
 // (compute-bound) and a fine (gather-bound) level, which takes the fine level's slice out of L2
 // (30% slower).
 
-template <int D, int F, typename T>
+// With kSlopes it also leaves the slopes of every feature behind (penc_slopes.hpp).
+template <int D, int F, typename T, bool kSlopes>
 __global__ void __launch_bounds__(kBlock)
 forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
                const float* __restrict__ positions, const T* __restrict__ table,
                const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
-               const float* __restrict__ window, float* __restrict__ sliced, float points_scaling) {
+               const float* __restrict__ window, float* __restrict__ sliced, float points_scaling, float* __restrict__ slopes) {
     uint32_t tile, row;
     if (!locate_work(map, tile, row)) return;
     const int n = tile * kBlock + threadIdx.x;
@@ -208,6 +212,8 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
             // written once and not read here: the non-temporal hint keeps it from displacing the level's table slice
             __builtin_nontemporal_store(acc[k], out + static_cast<size_t>(k) * n_points);
         });
+        if constexpr (kSlopes)
+            store_slopes<D, F>(v.f, s.rank, columns + threadIdx.x, kBlock, scale_factor + level * D, slopes + slope_offset<D, F>(n_points, level, n));
     }
 }
 
@@ -1377,7 +1383,7 @@ static int backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
 static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
                         const float* positions, const TableRef& table, const float* scale_factor,
                         const float* random_shift, const float* anneal_window, float* sliced_values,
-                        int concat_points, float points_scaling, void* stream) {
+                        int concat_points, float points_scaling, void* stream, float* slopes = nullptr) {
     const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points);
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
     if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values)
@@ -1386,11 +1392,18 @@ static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_l
     hipStream_t st = static_cast<hipStream_t>(stream);
     const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
                                        slice_bytes(capacity, nr_feat, table.format));
-    PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((forward_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st,
-                                         static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity),
-                                         mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,
-                                         random_shift, anneal_window, sliced_values, points_scaling));
+#define PENC_LAUNCH_FORWARD(SLOPES)                                                                                                      \
+    PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,                                                                                   \
+                      hipLaunchKernelGGL((forward_kernel<DD, FF, TT, SLOPES>), g.grid, dim3(kBlock), 0, st,                             \
+                                         static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity), \
+                                         mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,              \
+                                         random_shift, anneal_window, sliced_values, points_scaling, slopes))
+    if (slopes != nullptr) {
+        PENC_LAUNCH_FORWARD(true);
+    } else {
+        PENC_LAUNCH_FORWARD(false);
+    }
+#undef PENC_LAUNCH_FORWARD
     return check_launch();
 }
 
@@ -1787,6 +1800,95 @@ int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int 
                                       level_major, concat_points, nullptr, 0, stream))
         return rc;
     return transpose_to_rows(level_major, grad_grad_rows, row_stride, nr_positions, cols, st);
+}
+
+// Where a forward's slopes are worth keeping for the position gradient and the grad-grad (all three together, us, gathering -> slopes; more
+// in penc_slopes.hpp).  With two features per level also where a workgroup takes all levels of its points: D = 3, 24
+// levels of 2^18 slots, 1000 points 15.0 -> 10.8, 4097 points 24.5 -> 12.1; 16 levels of 2^13 slots, 2^16 points 44.3 -> 28.3, 2^20 575 -> 396;
+// D = 8, 16 levels of 2^12, 5001 points 23.9 -> 13.1; 6 levels of 2^12, 2^16 points 20.5 -> 15.1.  But small batches on tables of at most 1 MiB
+// wait for the host rather than for kernels (5001 points, 16 levels of 2^13 13.9 -> 10.9, with some 130 us of host work around them): they
+// are left to the gathering kernels, which give the bits of the autograd functions.
+// With four features where no such workgroups serve (D = 3, 16 levels, 2^18 points: 2^12 slots 159 -> 170, 2^14 176 -> 173, 2^15 218 -> 174, 2^16
+// 224 -> 179; D = 5, 2^14 269 -> 283).  With eight where besides no L2 holds a level (D = 3, 16 levels: 2^16 slots, 2^18 points 358 -> 347
+// but 224 -> 241 without the grad-grad, 2^18 slots 941 -> 809; 2^15 points 90 -> 56; D = 4, 2^16 slots 225 -> 233; D = 8, 2^18 slots 178 -> 117).
+constexpr size_t kSlopesSmallTableBytes = size_t{1} << 20, kSlopesMinSliceBytes = size_t{4} << 20;
+constexpr int64_t kSlopesFewPoints = 8192;
+static bool slopes_serve(int pos_dim, int nr_feat, int64_t n, int levels, int capacity, int table_format) {
+    const size_t slice = slice_bytes(capacity, nr_feat, table_format);
+    if (nr_feat == 2) return n > kSlopesFewPoints || levels * slice > kSlopesSmallTableBytes;
+    return !takes_point_blocks(pos_dim, n, levels, capacity, nr_feat, levels * nr_feat, table_format) && (nr_feat == 4 || slice > kSlopesMinSliceBytes);
+}
+
+size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int table_format) {
+    if (check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0) != PENC_OK || nr_levels * nr_feat > 255) return 0;
+    if (!slopes_serve(pos_dim, nr_feat, nr_positions, nr_levels, capacity, table_format)) return 0;
+    return static_cast<size_t>(nr_levels) * slope_tiles(nr_positions) * kSlopeTile * pos_dim * nr_feat * sizeof(float);
+}
+
+int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                        const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
+                        const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
+                        int concat_points, float points_scaling, void* stream) {
+    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!slopes) return PENC_ERR_NULL_POINTER;
+    const int cols = nr_feat * (nr_levels + penc_extra_levels(pos_dim, nr_feat, concat_points));
+    if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
+    if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values, table_format}, scale_factor,
+                              random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream, slopes))
+        return rc;
+    return sliced_rows == nullptr ? PENC_OK : transpose_to_rows(sliced_values, sliced_rows, row_stride, nr_positions, cols, static_cast<hipStream_t>(stream));
+}
+
+static size_t slope_tile_bytes(int columns) { return static_cast<size_t>(kSlopeTile) * (columns | 1) * sizeof(float); }
+
+int penc_backward_positions_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, const float* slopes,
+                                   const float* anneal_window, const float* grad, int64_t grad_row_stride, float* grad_level_major,
+                                   float* positions_grad, void* stream) {
+    if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, 1, 0)) return rc;
+    if (!slopes || !anneal_window || !grad || !positions_grad) return PENC_ERR_NULL_POINTER;
+    const int cols = nr_feat * nr_levels;
+    const bool rows = grad_row_stride != 0;
+    if (rows)
+        if (int rc = check_rows(grad, grad_row_stride, nr_positions, nr_levels, nr_feat)) return rc;
+    if (rows && cols > 255) return PENC_ERR_BAD_SIZE;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid(static_cast<unsigned>(slope_tiles(nr_positions)));
+#define PENC_LAUNCH_SLOPES(ROWS)                                                                                                       \
+    PENC_DISPATCH_DF(pos_dim, nr_feat,                                                                                                 \
+                     hipLaunchKernelGGL((positions_from_slopes_kernel<DD, FF, ROWS>), grid, dim3(kSlopeBlock),                         \
+                                        ROWS ? slope_tile_bytes(cols) : 0, st, static_cast<int>(nr_positions), nr_levels, slopes,      \
+                                        anneal_window, grad, grad_row_stride, grad_level_major, positions_grad))
+    if (rows) {
+        PENC_LAUNCH_SLOPES(true);
+    } else {
+        PENC_LAUNCH_SLOPES(false);
+    }
+#undef PENC_LAUNCH_SLOPES
+    return check_launch();
+}
+
+int penc_grad_grad_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, const float* slopes, const float* anneal_window,
+                          const float* double_positions_grad, float* grad_grad, int64_t row_stride, int concat_points, void* stream) {
+    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points);
+    if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, 1, extra)) return rc;
+    if (!slopes || !anneal_window || !double_positions_grad || !grad_grad) return PENC_ERR_NULL_POINTER;
+    const int cols = nr_feat * (nr_levels + extra);
+    const bool rows = row_stride != 0;
+    if (rows && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid(static_cast<unsigned>(slope_tiles(nr_positions)));
+#define PENC_LAUNCH_SLOPES(ROWS)                                                                                                       \
+    PENC_DISPATCH_DF(pos_dim, nr_feat,                                                                                                 \
+                     hipLaunchKernelGGL((grad_grad_from_slopes_kernel<DD, FF, ROWS>), grid, dim3(kSlopeBlock),                         \
+                                        ROWS ? slope_tile_bytes(cols) : 0, st, static_cast<int>(nr_positions), nr_levels,              \
+                                        nr_levels + extra, slopes, anneal_window, double_positions_grad, grad_grad, row_stride))
+    if (rows) {
+        PENC_LAUNCH_SLOPES(true);
+    } else {
+        PENC_LAUNCH_SLOPES(false);
+    }
+#undef PENC_LAUNCH_SLOPES
+    return check_launch();
 }
 
 // The scalars of one AdamW step as torch.optim.AdamW forms them (in double), rounded once for the kernel.

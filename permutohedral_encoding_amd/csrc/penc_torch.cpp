@@ -14,6 +14,8 @@
 // array behind it (reference: src/pytorch_modules/modules.py:87), so that the permute and reshape need no nodes.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
+#include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
@@ -33,6 +35,7 @@
 #include <torch/csrc/utils/object_ptr.h>
 
 #include <algorithm>
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -74,6 +77,10 @@ struct Api {
     PENC_FN(upload);
     PENC_FN(backward_positions_rowmajor);
     PENC_FN(grad_grad_rowmajor);
+    PENC_FN(slopes_bytes);
+    PENC_FN(forward_slopes);
+    PENC_FN(backward_positions_slopes);
+    PENC_FN(grad_grad_slopes);
 #undef PENC_FN
 } api;
 
@@ -229,11 +236,98 @@ Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t cop
 void* workspace_of(const Tensor& ws) { return ws.defined() ? ws.mutable_data_ptr() : nullptr; }
 size_t workspace_size(const Tensor& ws) { return ws.defined() ? static_cast<size_t>(ws.numel()) : 0; }
 
+// The version a tensor must still be at when a node that did not save the tensor itself runs.
+struct ExpectedVersion {
+    c10::VariableVersion counter;
+    uint32_t expected = 0;
+    bool set = false;
+
+    void expect(const Tensor& t) {
+        TORCH_CHECK(!t.is_inference(), "Inference tensors cannot be saved for backward: make a clone outside of inference mode");
+        counter = torch::autograd::impl::version_counter(t);
+        expected = counter.current_version();
+        set = true;
+    }
+    bool holds() const { return !set || counter.current_version() == expected; }
+    void check(const char* what) const {
+        TORCH_CHECK(holds(),
+                    "one of the variables needed for gradient computation has been modified by an inplace operation: ", what, " is at version ",
+                    counter.current_version(), "; expected version ", expected, " instead");
+    }
+};
+
+// The slopes of the encoded features (penc_forward_slopes), kept from the forward to the passes that differentiate w.r.t. the positions,
+// as autograd keeps the tensors a node saves: freed with the graph.  What they were computed from must still be what a gathering kernel
+// would read then; where it is not (a table stepped between forward and backward, a pass on another stream), that kernel runs.
+// Their memory is bounded: all slopes alive on a device together take at most a sixteenth of its memory, beyond which
+// forwards leave none.
+struct Slopes {
+    static constexpr int kMaxDevices = 64;
+    static std::atomic<int64_t> held[kMaxDevices];
+
+    Tensor values;
+    ExpectedVersion inputs[5];
+    void* stream;
+    int device = -1;
+    int64_t reserved = 0;
+
+    Slopes() = default;
+    Slopes(const Slopes&) = delete;
+    Slopes& operator=(const Slopes&) = delete;
+    ~Slopes() {
+        if (reserved != 0) held[device] -= reserved;
+    }
+    bool usable(const Call& c) const {
+        return current_stream(c.device()) == stream && std::all_of(std::begin(inputs), std::end(inputs), [](const ExpectedVersion& v) { return v.holds(); });
+    }
+    const float* data() const { return static_cast<const float*>(values.const_data_ptr()); }
+
+    // For the forward that is about to run; null where none are kept.  (With hooks on what a graph saves, such as those of
+    // checkpointing, which trade memory for a second computation, nothing beside what they see is kept.)
+    static std::shared_ptr<Slopes> make(const Call& c) {
+        if (!c.want_positions || c.columns() > 255 || c.levels_per_pass < 0) return nullptr;
+        const int64_t want = static_cast<int64_t>(api.slopes_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, c.table_format));
+        if (want == 0 || (c.max_workspace >= 0 && want > c.max_workspace)) return nullptr;
+        const Tensor* const from[] = {&c.table, &c.positions, &c.window, &c.shift, &c.scale_factor};
+        for (const Tensor* t : from)
+            if (t->is_inference()) return nullptr;
+        if (at::SavedTensorDefaultHooks::get_hooks().has_value()) return nullptr;
+        const int device = c.device().index();
+        if (device < 0 || device >= kMaxDevices) return nullptr;
+        const int64_t most = static_cast<int64_t>(at::cuda::getDeviceProperties(device)->totalGlobalMem / 16);
+        auto kept = std::make_shared<Slopes>();
+        kept->device = device;
+        if (held[device].fetch_add(want) + want > most) {
+            held[device] -= want;
+            return nullptr;
+        }
+        kept->reserved = want;
+        try {
+            kept->values = at::empty({want / 4}, c.positions.options().dtype(at::kFloat));
+        } catch (const c10::OutOfMemoryError&) {
+            return nullptr;
+        }
+        kept->stream = current_stream(c.device());
+        for (size_t i = 0; i < std::size(from); ++i) kept->inputs[i].expect(*from[i]);
+        return kept;
+    }
+};
+std::atomic<int64_t> Slopes::held[Slopes::kMaxDevices] = {};
+
 // ------------------------------------------------------------------------------------------
 // the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
 
-Tensor compute_forward(const Call& c) {
+Tensor compute_forward(const Call& c, const Slopes* slopes) {
     void* const stream = current_stream(c.device());
+    if (slopes != nullptr) {
+        Tensor out = level_major_array(c), rows;
+        if (c.rows_output && c.table_format == 0) rows = at::empty({c.n, c.columns()}, c.positions.options());
+        check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                                 data(c.scale_factor), data(c.shift), data(c.window), mutable_data(out), mutable_data(rows), c.columns(),
+                                 mutable_data(slopes->values), c.concat, c.scaling, stream),
+              "forward_slopes");
+        return rows.defined() ? rows : out;
+    }
     if (c.rows_output && c.table_format == 0 && c.columns() <= 255) {
         Tensor rows = at::empty({c.n, c.columns()}, c.positions.options());
         const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
@@ -320,26 +414,44 @@ Tensor checked_double_positions_grad(const Call& c, const Tensor& double_positio
     return double_positions_grad.detach().contiguous();
 }
 
-// The position gradient alone, from rows, whose level-major copy outlives the call: the double backward's scatter reads it too
-// (coalesced, where rows cost it a sixth of its time) and can be deferred.
-Gradients compute_positions_backward(const Call& c, Upstream& up) {
-    Gradients g;
-    g.positions = at::empty({c.n, c.pos_dim}, c.positions.options());
-    Tensor level_major = level_major_array(c);
-    const Tensor ws = gradient_workspace(c, false, true, 0);
-    check(api.backward_positions_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(),
-                                          c.table_format, data(c.scale_factor), data(c.shift), data(c.window), data(up.values),
-                                          up.row_stride, mutable_data(level_major), mutable_data(g.positions), workspace_of(ws),
-                                          workspace_size(ws), current_stream(c.device())),
-          "backward_positions");
+// The position gradient alone, from the slopes where the forward has kept them.  With `keep_copy`, of rows the level-major copy outlives
+// the call and takes their place: a scatter that follows, and the double backward's, reads it coalesced, where rows cost it a sixth
+// of its time.
+Tensor compute_positions_backward(const Call& c, Upstream& up, const Slopes* slopes, bool keep_copy) {
+    Tensor positions = at::empty({c.n, c.pos_dim}, c.positions.options());
+    void* const stream = current_stream(c.device());
+    Tensor level_major;
+    if (up.row_stride != 0 && keep_copy) level_major = level_major_array(c);
+    if (slopes != nullptr) {
+        check(api.backward_positions_slopes(c.pos_dim, c.feat, c.n, c.levels, slopes->data(), data(c.window), data(up.values), up.row_stride,
+                                            mutable_data(level_major), mutable_data(positions), stream),
+              "backward_positions_slopes");
+    } else {
+        const Tensor ws = gradient_workspace(c, false, true, 0);
+        check(api.backward_positions_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(),
+                                              c.table_format, data(c.scale_factor), data(c.shift), data(c.window), data(up.values),
+                                              up.row_stride, mutable_data(level_major), mutable_data(positions), workspace_of(ws),
+                                              workspace_size(ws), stream),
+              "backward_positions");
+    }
+    if (!level_major.defined()) return positions;
     // (the columns of concatenated points carry no gradient and are not read, but whoever saves the copy sees the whole of it)
     const int64_t encoded = static_cast<int64_t>(c.feat) * c.levels;
     if (c.extra != 0) level_major.narrow(1, encoded, c.columns() - encoded).copy_(up.values.narrow(1, encoded, c.columns() - encoded));
     up = {level_major, 0};
-    return g;
+    return positions;
 }
 
-// The gradient w.r.t. an upstream gradient, as dense rows.
+// The gradient w.r.t. an upstream gradient, as dense rows or in [L+E][F][N] order, from the slopes.
+Tensor compute_grad_grad(const Call& c, const Slopes& slopes, const Tensor& double_positions_grad, bool as_rows) {
+    Tensor out = as_rows ? at::empty({c.n, c.columns()}, c.positions.options()) : level_major_array(c);
+    check(api.grad_grad_slopes(c.pos_dim, c.feat, c.n, c.levels, slopes.data(), data(c.window), data(double_positions_grad), mutable_data(out),
+                               as_rows ? c.columns() : 0, c.concat, current_stream(c.device())),
+          "grad_grad_slopes");
+    return out;
+}
+
+// The same as dense rows, gathered.
 Tensor compute_grad_grad_rows(const Call& c, const Tensor& double_positions_grad) {
     Tensor rows = at::empty({c.n, c.columns()}, c.positions.options());
     const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
@@ -414,30 +526,12 @@ bool goes_into_row_major_leaf(const torch::autograd::Edge& edge) {
     return leaf != nullptr && leaf->variable.dim() == 2 && leaf->variable.is_contiguous();
 }
 
-// The version a tensor must still be at when a node that did not save the tensor itself runs.
-struct ExpectedVersion {
-    c10::VariableVersion counter;
-    uint32_t expected = 0;
-    bool set = false;
-
-    void expect(const Tensor& t) {
-        TORCH_CHECK(!t.is_inference(), "Inference tensors cannot be saved for backward: make a clone outside of inference mode");
-        counter = torch::autograd::impl::version_counter(t);
-        expected = counter.current_version();
-        set = true;
-    }
-    void check(const char* what) const {
-        TORCH_CHECK(!set || counter.current_version() == expected,
-                    "one of the variables needed for gradient computation has been modified by an inplace operation: ", what, " is at version ",
-                    counter.current_version(), "; expected version ", expected, " instead");
-    }
-};
-
 // Gradients of the slicing w.r.t. the table (0) and the positions (1).  A gradient that nothing in the running pass
 // consumes is not computed: the first half of an eikonal loss, autograd.grad(sdf, positions, create_graph=True), runs no
 // table scatter.
 struct EncodeNode : public Node {
     std::shared_ptr<const Call> call;
+    std::shared_ptr<const Slopes> slopes;  // may be null
     void* forward_stream = nullptr;
     // The result counts as saved, as it does in funcs.py: changing it in place, or a second pass through a freed graph, is refused.
     ExpectedVersion result_version;
@@ -453,6 +547,11 @@ struct EncodeNode : public Node {
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
         released = true;
+        slopes.reset();
+    }
+    std::shared_ptr<const Slopes> usable_slopes() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        return slopes != nullptr && slopes->usable(*call) ? slopes : nullptr;
     }
     void check_saved() {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -488,6 +587,7 @@ struct ResultNode : public Node {
 struct EncodeBackNode : public Node {
     std::shared_ptr<const Call> call;
     std::shared_ptr<EncodeNode> slicing;
+    std::shared_ptr<const Slopes> slopes;     // may be null
     torch::autograd::SavedVariable upstream;  // saved as autograd saves: version checks, hooks, freed with the graph
     ExpectedVersion rows_version;             // of the rows `upstream` is a level-major copy of: changing them is refused all the same
 
@@ -495,16 +595,19 @@ struct EncodeBackNode : public Node {
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
         upstream.reset_data();
+        slopes.reset();
     }
     variable_list apply(variable_list&& grads) override {
         variable_list out(3);
         if (grads.size() < 2 || !grads[1].defined()) return out;
         refuse_tangents(grads);
         Tensor saved;
+        std::shared_ptr<const Slopes> kept;
         {
             std::lock_guard<std::mutex> lock(mutex_);
             saved = upstream.unpack();
             rows_version.check("the upstream gradient");
+            if (slopes != nullptr && slopes->usable(*call)) kept = slopes;
         }
         const Call& c = *call;
         const bool grad_mode = c10::GradMode::is_enabled();
@@ -519,9 +622,11 @@ struct EncodeBackNode : public Node {
             want_table = false;
         }
         bool want_upstream = task_should_compute_output(0);
-        if (want_upstream && goes_into_row_major_leaf(next_edge(0)) && c.columns() <= 255) {
-            out[0] = compute_grad_grad_rows(c, checked_double_positions_grad(c, grads[1]));
-            want_upstream = false;
+        if (want_upstream) {
+            const bool as_rows = goes_into_row_major_leaf(next_edge(0)) && c.columns() <= 255;
+            if (kept != nullptr) out[0] = compute_grad_grad(c, *kept, checked_double_positions_grad(c, grads[1]), as_rows);
+            else if (as_rows) out[0] = compute_grad_grad_rows(c, checked_double_positions_grad(c, grads[1]));
+            want_upstream = !out[0].defined();
         }
         if (!want_table && !want_upstream) return out;
         SecondOrder s = compute_double_backward(c, grads[1].detach(), up, want_table, want_upstream);
@@ -545,19 +650,28 @@ variable_list EncodeNode::apply(variable_list&& grads) {
     Upstream up;
     Gradients g;
     ExpectedVersion rows_version;
+    std::shared_ptr<const Slopes> kept;
     {
         at::NoGradGuard no_grad;
         const c10::DeviceGuard device(c.device());
+        if (want_positions) kept = usable_slopes();
         const SecondOrderTerm* fused = nullptr;
         if (first_order) {
             check_saved();
             up = upstream_of(c, grads[0].detach());
-            if (differentiable && want_positions && !want_table && up.row_stride != 0 && c.columns() <= 255) {
-                if (up.values.is_alias_of(grads[0])) rows_version.expect(grads[0]);
-                g = compute_positions_backward(c, up);
-            } else {
+            bool gather_positions = want_positions;
+            if (want_positions &&
+                (kept != nullptr || (differentiable && !want_table && up.row_stride != 0 && c.columns() <= 255))) {
+                const bool keep_copy = differentiable || want_table;
+                if (differentiable && up.row_stride != 0 && up.values.is_alias_of(grads[0])) rows_version.expect(grads[0]);
+                g.positions = compute_positions_backward(c, up, kept.get(), keep_copy);
+                gather_positions = false;
+            }
+            if (want_table || gather_positions) {
                 if (want_table && !terms.empty()) fused = &terms.back();
-                g = compute_backward(c, up, want_table, want_positions, fused);
+                Gradients more = compute_backward(c, up, want_table, gather_positions, fused);
+                g.table = std::move(more.table);
+                if (gather_positions) g.positions = std::move(more.positions);
             }
         }
         for (const SecondOrderTerm& t : terms) {
@@ -574,6 +688,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
         back->add_next_edge(torch::autograd::Edge(back->slicing, 0));
         back->call = call;
+        back->slopes = std::move(kept);
         back->upstream = torch::autograd::SavedVariable(up.values, false);
         back->rows_version = std::move(rows_version);
         torch::autograd::set_history(g.table, back);
@@ -714,13 +829,15 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.want_positions = grad_mode && positions.requires_grad();
         if (args[10] != Py_None && (c.want_table || c.want_positions)) c.sparse_owner = std::make_shared<PyRef>(args[10]);
         Tensor out;
+        std::shared_ptr<const Slopes> slopes;
         {
             NoGil no_gil;
             at::NoGradGuard no_grad;
             if (positions.is_cuda()) window = window_on_device(window, positions.device());
             prepare_call(c, positions, window);
             const c10::DeviceGuard device(c.device());
-            out = compute_forward(c);
+            slopes = Slopes::make(c);
+            out = compute_forward(c, slopes.get());
         }
         if (c.scale_factor.device() != scale_device) {  // the module was moved: kept where the points are, so that the next call need not copy
             THPObjectPtr moved(THPVariable_Wrap(c.scale_factor));
@@ -731,6 +848,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             node->set_next_edges(torch::autograd::collect_next_edges(lattice_values, positions));
             node->forward_stream = current_stream(call->device());
             node->call = std::move(call);
+            node->slopes = std::move(slopes);
             node->result_version.expect(out);
             auto result = std::shared_ptr<ResultNode>(new ResultNode(), torch::autograd::deleteNode);
             result->add_next_edge(torch::autograd::Edge(node, node->add_input_metadata(out)));
@@ -848,6 +966,10 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(upload);
         PENC_FN(backward_positions_rowmajor);
         PENC_FN(grad_grad_rowmajor);
+        PENC_FN(slopes_bytes);
+        PENC_FN(forward_slopes);
+        PENC_FN(backward_positions_slopes);
+        PENC_FN(grad_grad_slopes);
 #undef PENC_FN
         Py_RETURN_NONE;
     });
