@@ -552,34 +552,59 @@ touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, flo
     const size_t base = (static_cast<size_t>(level) * capacity + slot0) * nr_feat;  // a multiple of kPer floats (the host checks)
     const uint32_t n_vec = slots * nr_feat / kPer;
     Vec* const g_at = reinterpret_cast<Vec*>(grads + base);
-    for (uint32_t i = threadIdx.x; i < n_vec; i += kBlock) {
-        const Vec gv = g_at[i];
-        float g[kPer];
-        __builtin_memcpy(g, &gv, sizeof(gv));
-        bool nonzero = false;
+    // What a workgroup waits for is memory, first for the gradients and then for the values of those that are not zero: both are
+    // fetched for kTogether entries of a thread at a time (24 levels of 2^22 slots, a third of the ranges touched, 445 MiB read and 78
+    // written: 145 us one by one, 135 with four).
+    constexpr uint32_t kTogether = 4;
+    for (uint32_t first = threadIdx.x; first < n_vec; first += kTogether * kBlock) {
+        Vec gv[kTogether], pv[kTogether], mv[kTogether], vv[kTogether];
+        bool nonzero[kTogether];
 #pragma unroll
-        for (uint32_t k = 0; k < kPer; ++k) nonzero = nonzero || g[k] != 0.0f;
-        if (!nonzero) continue;
-        if constexpr (kUpdate) {
-            Vec pv = reinterpret_cast<Vec*>(params + base)[i], mv = reinterpret_cast<Vec*>(exp_avg + base)[i],
-                vv = reinterpret_cast<Vec*>(exp_avg_sq + base)[i];
-            float p[kPer], m[kPer], v[kPer];
-            __builtin_memcpy(p, &pv, sizeof(pv));
-            __builtin_memcpy(m, &mv, sizeof(mv));
-            __builtin_memcpy(v, &vv, sizeof(vv));
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k) adamw_update(a, true, g[k], p[k], m[k], v[k]);
-            __builtin_memcpy(&pv, p, sizeof(pv));
-            __builtin_memcpy(&mv, m, sizeof(mv));
-            __builtin_memcpy(&vv, v, sizeof(vv));
-            reinterpret_cast<Vec*>(params + base)[i] = pv;
-            reinterpret_cast<Vec*>(exp_avg + base)[i] = mv;
-            reinterpret_cast<Vec*>(exp_avg_sq + base)[i] = vv;
+        for (uint32_t u = 0; u < kTogether; ++u) {
+            const uint32_t i = first + u * kBlock;
+            gv[u] = g_at[i < n_vec ? i : first];
         }
-        if (clear) {
-            Vec zero;
-            __builtin_memset(&zero, 0, sizeof(zero));
-            g_at[i] = zero;
+#pragma unroll
+        for (uint32_t u = 0; u < kTogether; ++u) {
+            const uint32_t i = first + u * kBlock;
+            float g[kPer];
+            __builtin_memcpy(g, &gv[u], sizeof(Vec));
+            nonzero[u] = false;
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; ++k) nonzero[u] = nonzero[u] || g[k] != 0.0f;
+            nonzero[u] = nonzero[u] && i < n_vec;
+            if constexpr (kUpdate) {
+                if (nonzero[u]) {
+                    pv[u] = reinterpret_cast<Vec*>(params + base)[i];
+                    mv[u] = reinterpret_cast<Vec*>(exp_avg + base)[i];
+                    vv[u] = reinterpret_cast<Vec*>(exp_avg_sq + base)[i];
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kTogether; ++u) {
+            const uint32_t i = first + u * kBlock;
+            if (!nonzero[u]) continue;
+            if constexpr (kUpdate) {
+                float g[kPer], p[kPer], m[kPer], v[kPer];
+                __builtin_memcpy(g, &gv[u], sizeof(Vec));
+                __builtin_memcpy(p, &pv[u], sizeof(Vec));
+                __builtin_memcpy(m, &mv[u], sizeof(Vec));
+                __builtin_memcpy(v, &vv[u], sizeof(Vec));
+#pragma unroll
+                for (uint32_t k = 0; k < kPer; ++k) adamw_update(a, true, g[k], p[k], m[k], v[k]);
+                __builtin_memcpy(&pv[u], p, sizeof(Vec));
+                __builtin_memcpy(&mv[u], m, sizeof(Vec));
+                __builtin_memcpy(&vv[u], v, sizeof(Vec));
+                reinterpret_cast<Vec*>(params + base)[i] = pv[u];
+                reinterpret_cast<Vec*>(exp_avg + base)[i] = mv[u];
+                reinterpret_cast<Vec*>(exp_avg_sq + base)[i] = vv[u];
+            }
+            if (clear) {
+                Vec zero;
+                __builtin_memset(&zero, 0, sizeof(zero));
+                g_at[i] = zero;
+            }
         }
     }
     if (clear) {
