@@ -175,7 +175,9 @@ __global__ void __launch_bounds__(kSlopeBlock)
 grad_grad_from_slopes_kernel(int n_points, int n_levels, int n_all_levels, const float* __restrict__ slopes, const float* __restrict__ window,
                              const float* __restrict__ double_pos_grad, float* __restrict__ out, int64_t row_stride) {
     extern __shared__ float tile[];  // rows: 64 x (columns | 1)
-    const int base = blockIdx.x * kSlopeTile, count = n_points - base < kSlopeTile ? n_points - base : kSlopeTile;
+    // last points first: of what the position gradient has read before, the end is what the memory-side cache still holds (D = 4, 2^20
+    // points: 189 -> 178 us; D = 3, 16 live levels: 111 -> 107)
+    const int base = (gridDim.x - 1 - blockIdx.x) * kSlopeTile, count = n_points - base < kSlopeTile ? n_points - base : kSlopeTile;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int columns = n_all_levels * F, pitch = columns | 1;
     const int n = base + (lane < count ? lane : count - 1);
