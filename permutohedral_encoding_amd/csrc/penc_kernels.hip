@@ -1028,8 +1028,12 @@ inline int reduce_bins(const BinPlan& p, const float* window, int first_level, i
         const unsigned to_fill = (kReduceWorkgroupsWanted + p.target.n_bins - 1) / p.target.n_bins;  // two workgroups per compute unit, one after the other
         if (per_bin < to_fill) per_bin = to_fill;
         if (per_bin > levels) per_bin = levels;
-        hipLaunchKernelGGL(bin_reduce_levels_kernel, dim3(p.target.n_bins, per_bin), dim3(kReduceBlock), 0, st, p.target, window,
-                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level, static_cast<uint32_t>(levels));
+#define PENC_LAUNCH_LEVELS(UNROLL)                                                                                                          \
+    hipLaunchKernelGGL(bin_reduce_levels_kernel<UNROLL>, dim3(p.target.n_bins, per_bin), dim3(kReduceBlock), 0, st, p.target, window,       \
+                       static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level, static_cast<uint32_t>(levels))
+        if (p.target.segment_capacity <= kLevelsShortSegment) PENC_LAUNCH_LEVELS(kLevelsShortUnroll);
+        else PENC_LAUNCH_LEVELS(kLevelsUnroll);
+#undef PENC_LAUNCH_LEVELS
         return check_launch();
     }
     const dim3 grid(p.target.n_bins, n_levels_in_pass, splits);

@@ -241,24 +241,30 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
 // dozen records in each of its segments and a (bin, level) has a few thousand in all, so a workgroup of
 // bin_reduce_kernel is a chain of latencies (launch, counts, records, gradient) with nothing to overlap
 // them: its 128 KiB of sums allow one workgroup per compute unit.  Here a workgroup keeps its bin and walks
-// several levels (blockIdx.y, + gridDim.y, ...): the counts of all its levels are fetched at once
+// several levels (blockIdx.y, + gridDim.y, ...): the counts of all its levels are fetched at once and kept in LDS
 // (levels that left no records cost nothing more), and over the sequence of (level, 64 segments)
-// steps that remain the counts are fetched two steps and the records one step ahead of the adds, so the
-// loads of the next level are in flight while this level's sums are added and written out
-// (measured on a 2^22-slot table, 16 levels, per call: bin_reduce_kernel 0.207 ms; this kernel 0.170 ms;
-// with every load issued unconditionally, LDS-only barriers and a store-only write-out, so that nothing
-// waits for the loads of the next step, 0.157 ms; with one workgroup per bin instead of two 0.146 ms).
-// A quarter of a wave reads a segment, kLevelsShortUnroll records per lane: needs segments of at
+// steps that remain the records are fetched two steps ahead of the adds.
+// What it would wait for otherwise is its own stores: a wait for records counts every memory operation issued after them, and how
+// many stores a write-out makes is not known when the code is compiled, so a wait that follows a write-out waits for the stores as well, a trip
+// to memory for every level.  So the next step's records are waited for before the write-out, and those of the step after it
+// are on their way over it.
+// (16 live levels of 2^22 slots, 2^20 points near a surface, 340 MB of records: 152 -> 134 us; 200001 points 80 -> 63 us; 8 levels of random
+// slots, 49 segments of 32 records 98 -> 95, 128 of 64 207 -> 212, of which the records alone 123 -> 87.)
+// A wave reads four segments at a time, their records counted through, so that every lane of a load has one (with a quarter of the
+// wave to a segment of 64 records in room for 101 half of the lanes had none).  Needs segments of at
 // most kLevelsMaxSegment records, whole (12-byte) records, at most kReduceBlock groups and
 // at most kLevelsMaxPerWorkgroup levels per workgroup (the host checks all four).
-constexpr uint32_t kLevelsShortLanes = 16, kLevelsShortUnroll = 8;
-constexpr uint32_t kLevelsMaxSegment = kLevelsShortLanes * kLevelsShortUnroll;
+constexpr uint32_t kLevelsUnroll = 6, kLevelsShortUnroll = 3;
+constexpr uint32_t kLevelsMaxSegment = 128, kLevelsShortSegment = 64;
 constexpr uint32_t kLevelsMaxPerWorkgroup = 24;
+static_assert(kLevelsMaxSegment < 256, "a segment's count is kept in a byte");
+template <uint32_t kUnroll>
 __global__ void __launch_bounds__(kReduceBlock)
 bin_reduce_levels_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs,
                          float* __restrict__ table_grad, int first_level, uint32_t n_levels_in_pass) {
-    __shared__ double acc0[kBinSlots];
-    __shared__ double acc1[kBinSlots];
+    __shared__ __align__(16) double acc0[kBinSlots];
+    __shared__ __align__(16) double acc1[kBinSlots];
+    __shared__ __align__(4) uint8_t counts[kLevelsMaxPerWorkgroup][kReduceBlock];  // records of the workgroup's i-th level in each group's segment
     __shared__ uint32_t masks[2];  // bit i: the workgroup's i-th level [0] has records in this bin, [1] got direct adds in this bin's slots
     const uint32_t bin = blockIdx.x, my_first = blockIdx.y, my_stride = gridDim.y;
     const uint32_t n_mine = (n_levels_in_pass - my_first + my_stride - 1) / my_stride;  // blockIdx.y < n_levels_in_pass
@@ -288,8 +294,10 @@ bin_reduce_levels_kernel(BinTarget pass_bins, const float* __restrict__ window, 
     __syncthreads();  // the masks are cleared
     uint32_t found = 0u;
 #pragma unroll
-    for (uint32_t i = 0; i < kLevelsMaxPerWorkgroup; ++i)
+    for (uint32_t i = 0; i < kLevelsMaxPerWorkgroup; ++i) {
+        if (i < n_mine) counts[i][threadIdx.x] = static_cast<uint8_t>(seen[i]);
         if (__ballot(seen[i] != 0u) != 0ull) found |= 1u << i;
+    }
     if (lane == 0 && found != 0u) atomicOr(&masks[0], found);
     if (direct != 0u) atomicOr(&masks[1], 1u << threadIdx.x);
     __syncthreads();
@@ -306,119 +314,129 @@ bin_reduce_levels_kernel(BinTarget pass_bins, const float* __restrict__ window, 
     };
     const uint32_t n_steps = (n_groups + 63) / 64;
     const auto after = [&](Cursor at) {
-        if (++at.step < n_steps) return at;
+        if (at.i == kEnd || ++at.step < n_steps) return at;
         at.step = 0u;
         if (++at.range < n_ranges) return at;
         const uint32_t rest = at.i + 1 < 32 ? todo >> (at.i + 1) : 0u;
         return Cursor{rest != 0u ? at.i + 1 + static_cast<uint32_t>(__builtin_ctz(rest)) : kEnd, 0u, 0u};
     };
-    const uint32_t reader = wave * 4 + lane / kLevelsShortLanes, l = lane % kLevelsShortLanes;
-    // (Every load below is issued whether or not its result is wanted, from an address that is valid
-    // either way: with loads behind branches the compiler cannot tell how many are on their way and
-    // makes every use wait for all of them, those of the next step included.)
-    const auto load_count = [&](const Cursor& at) {
-        const uint32_t g = at.step * 64 + reader;
-        const uint32_t i = at.i != kEnd ? at.i : 0u;
-        const uint32_t count = pass_bins.counts[first_segment(i) + (g < n_groups ? g : 0u)];
-        return at.i != kEnd && g < n_groups ? count : 0u;
-    };
     struct Loaded {
-        RecordWords rec[kLevelsShortUnroll];
-        uint32_t count, range;
+        RecordWords rec[kUnroll];
+        uint32_t total, range, counts4;
     };
     const BinRecord* const records = static_cast<const BinRecord*>(pass_bins.records);
-    const auto fetch = [&](const Cursor& at, uint32_t count, Loaded& got) {
-        const uint32_t g = at.step * 64 + reader;
-        const BinRecord* seg = records + (first_segment(at.i != kEnd ? at.i : 0u) + (g < n_groups ? g : 0u)) * seg_cap;
-        got.count = count;
+    // Record j of the wave's four segments, counted through, in the order of the segments.
+    const auto index_of = [&](uint32_t counts4, uint32_t j) {
+        const uint32_t c0 = counts4 & 255u, c1 = (counts4 >> 8) & 255u, c2 = (counts4 >> 16) & 255u;
+        uint32_t i = j;
+        i += j >= c0 ? seg_cap - c0 : 0u;
+        i += j >= c0 + c1 ? seg_cap - c1 : 0u;
+        i += j >= c0 + c1 + c2 ? seg_cap - c2 : 0u;
+        return i;
+    };
+    // (Every load is issued whether or not its result is wanted, from an address that is valid
+    // either way: with loads behind branches the compiler cannot tell how many are on their way and
+    // makes every use wait for all of them, those of the next step included.)
+    const auto fetch = [&](const Cursor& at, Loaded& got) {
+        const uint32_t i = at.i != kEnd ? at.i : 0u, g = at.step * 64 + wave * 4;  // (the counts reach to the end of the last step)
+        uint32_t counts4 = *reinterpret_cast<const uint32_t*>(&counts[i][g]);
+        counts4 = at.i != kEnd ? __builtin_amdgcn_readfirstlane(counts4) : 0u;
+        got.counts4 = counts4;
+        got.total = (counts4 & 255u) + ((counts4 >> 8) & 255u) + ((counts4 >> 16) & 255u) + (counts4 >> 24);
         got.range = at.range;
+        const BinRecord* seg = records + (first_segment(i) + g) * seg_cap;
 #pragma unroll
-        for (uint32_t u = 0; u < kLevelsShortUnroll; ++u) {
-            const uint32_t idx = u * kLevelsShortLanes + l;
-            // (normal loads: neighbouring short segments share cache lines); the pass's first record stands in where there is none
-            got.rec[u] = *reinterpret_cast<const RecordWords*>(idx < count ? seg + idx : records);
+        for (uint32_t u = 0; u < kUnroll; ++u) {
+            const uint32_t j = u * 64 + lane;
+            got.rec[u] = *reinterpret_cast<const RecordWords*>(j < got.total ? seg + index_of(counts4, j) : records);
         }
     };
-    const auto add = [&](const Loaded& got) {
+    // waits for a step's records
+    const auto arrive = [&](Loaded& got) {
 #pragma unroll
-        for (uint32_t u = 0; u < kLevelsShortUnroll; ++u) {
-            const RecordWords w = got.rec[u];
-            const uint32_t w0 = w.x, w1 = w.y, w2 = w.z;  // copies first: a bit cast applied directly to a vector element reads element 0
-            if (u * kLevelsShortLanes + l < got.count && (w0 >> kBinSlotsLog2) == got.range) {
-                const uint32_t cell = w0 & (kBinSlots - 1);
-                __hip_atomic_fetch_add(&acc0[cell], static_cast<double>(__builtin_bit_cast(float, w1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(&acc1[cell], static_cast<double>(__builtin_bit_cast(float, w2)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
+        for (uint32_t u = 0; u < kUnroll; ++u) asm volatile("" : "+v"(got.rec[u]));
+    };
+    const auto add_one = [&](const RecordWords& w, uint32_t range) {
+        const uint32_t w0 = w.x, w1 = w.y, w2 = w.z;  // copies first: a bit cast applied directly to a vector element reads element 0
+        if ((w0 >> kBinSlotsLog2) != range) return;
+        const uint32_t cell = w0 & (kBinSlots - 1);
+        __hip_atomic_fetch_add(&acc0[cell], static_cast<double>(__builtin_bit_cast(float, w1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(&acc1[cell], static_cast<double>(__builtin_bit_cast(float, w2)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    const auto add = [&](const Cursor& at, const Loaded& got) {
+#pragma unroll
+        for (uint32_t u = 0; u < kUnroll; ++u)
+            if (u * 64 + lane < got.total) add_one(got.rec[u], got.range);
+        // (more records than the registers take are rare: a segment's share is its mean)
+        if (got.total > kUnroll * 64) {
+            const BinRecord* seg = records + (first_segment(at.i) + at.step * 64 + wave * 4) * seg_cap;
+            for (uint32_t j = kUnroll * 64 + lane; j < got.total; j += 64)
+                add_one(*reinterpret_cast<const RecordWords*>(seg + index_of(got.counts4, j)), got.range);
         }
     };
-    // Adds the sums of one range of the bin at the workgroup's i-th level into the gradient and clears them.  Nothing else touches
-    // the bin's slots of that level while this kernel runs, so the add is a plain read-modify-write, or a
-    // store where nothing was added since the gradient was cleared.
-    const auto flush = [&](uint32_t i, uint32_t range) {
+    // Adds the sums of one range of the bin at the workgroup's i-th level into the gradient and clears them; waits for the records of
+    // `next` in between.  Nothing else touches the bin's slots of that level while this kernel runs, so the add is a plain
+    // read-modify-write, or a store where nothing was added since the gradient was cleared.  Two slots to a thread at a time.
+    typedef double Pair __attribute__((ext_vector_type(2)));
+    typedef float Quad __attribute__((ext_vector_type(4), aligned(8)));  // (the gradient is aligned to 8 bytes)
+    const auto flush = [&](uint32_t i, uint32_t range, Loaded& next) {
         lds_barrier();
         const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass(i);
         const uint32_t level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
         const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u};
         const uint32_t slot0 = (bin << pass_bins.bin_shift) + (range << kBinSlotsLog2);
         const bool untouched_so_far = ((direct_mask >> i) & 1u) == 0u;
+        constexpr int kMine = kBinSlots / kReduceBlock / 2;
+        Pair v0[kMine], v1[kMine];
+#pragma unroll
+        for (int k = 0; k < kMine; ++k) {
+            const uint32_t at = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
+            v0[k] = reinterpret_cast<const Pair*>(acc0)[at];
+            v1[k] = reinterpret_cast<const Pair*>(acc1)[at];
+        }
+        arrive(next);
         if (threadIdx.x == 0 && untouched_so_far) pass_bins.direct[static_cast<size_t>(level_in_pass(i)) * n_bins + bin] = 1u;  // this slot range now holds sums
-        constexpr int kMine = kBinSlots / kReduceBlock;
-        // (two loops, so that the usual one has no load to wait for: a wait would also be one for the
-        // records of the next step, which are on their way)
-        if (untouched_so_far) {
 #pragma unroll
-            for (int k = 0; k < kMine; ++k) {
-                const uint32_t s = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
-                const double v0 = acc0[s], v1 = acc1[s];
-                if (v0 != 0.0 || v1 != 0.0) {
-                    acc0[s] = 0.0;
-                    acc1[s] = 0.0;
-                    if (slot0 + s < capacity)
-                        *reinterpret_cast<float2*>(level_grad.at(slot0 + s)) = make_float2(static_cast<float>(v0), static_cast<float>(v1));
-                }
+        for (int k = 0; k < kMine; ++k) {
+            const uint32_t at = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x, slot = slot0 + 2 * at;
+            const bool one = v0[k].x != 0.0 || v1[k].x != 0.0, two = v0[k].y != 0.0 || v1[k].y != 0.0;
+            if (!one && !two) continue;
+            reinterpret_cast<Pair*>(acc0)[at] = Pair{0.0, 0.0};
+            reinterpret_cast<Pair*>(acc1)[at] = Pair{0.0, 0.0};
+            Quad sum = {static_cast<float>(v0[k].x), static_cast<float>(v1[k].x), static_cast<float>(v0[k].y), static_cast<float>(v1[k].y)};
+            if (untouched_so_far && feat_pairs == 1u && slot + 1 < capacity) {  // (a slot without sums holds zeros)
+                *reinterpret_cast<Quad*>(level_grad.at(slot)) = sum;
+                continue;
             }
-        } else {
-#pragma unroll
-            for (int k = 0; k < kMine; ++k) {
-                const uint32_t s = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
-                const double v0 = acc0[s], v1 = acc1[s];
-                if (v0 != 0.0 || v1 != 0.0) {
-                    acc0[s] = 0.0;
-                    acc1[s] = 0.0;
-                    if (slot0 + s < capacity) {
-                        float2* cell = reinterpret_cast<float2*>(level_grad.at(slot0 + s));
-                        float2 g = *cell;
-                        g.x += static_cast<float>(v0);
-                        g.y += static_cast<float>(v1);
-                        *cell = g;
-                    }
-                }
+            if (one && slot < capacity) {
+                float2* const cell = reinterpret_cast<float2*>(level_grad.at(slot));
+                const float2 g = untouched_so_far ? make_float2(0.0f, 0.0f) : *cell;
+                *cell = make_float2(g.x + sum.x, g.y + sum.y);
+            }
+            if (two && slot + 1 < capacity) {
+                float2* const cell = reinterpret_cast<float2*>(level_grad.at(slot + 1));
+                const float2 g = untouched_so_far ? make_float2(0.0f, 0.0f) : *cell;
+                *cell = make_float2(g.x + sum.z, g.y + sum.w);
             }
         }
         lds_barrier();
     };
-    // two sets of registers take turns for the records, two registers for the counts; past the last step the
-    // counts are zero and the loads fetch the stand-in
+    // three sets of registers take turns for the records; past the last step the loads fetch the stand-in
     Cursor it0{static_cast<uint32_t>(__builtin_ctz(todo)), 0u, 0u};
-    Cursor it1 = after(it0);
-    uint32_t count_x = load_count(it0), count_y = load_count(it1);
-    Loaded got_a, got_b;
-    fetch(it0, count_x, got_a);
-    while (true) {
-        const Cursor it2 = it1.i != kEnd ? after(it1) : it1;
-        count_x = load_count(it2);
-        fetch(it1, count_y, got_b);
-        add(got_a);
-        if (it1.i != it0.i || it1.range != it0.range) flush(it0.i, it0.range);
-        if (it1.i == kEnd) break;
-        const Cursor it3 = it2.i != kEnd ? after(it2) : it2;
-        count_y = load_count(it3);
-        fetch(it2, count_x, got_a);
-        add(got_b);
-        if (it2.i != it1.i || it2.range != it1.range) flush(it1.i, it1.range);
-        if (it2.i == kEnd) break;
-        it0 = it2;
-        it1 = it3;
+    Cursor it1 = after(it0), it2 = after(it1);
+    Loaded a, b, c;
+    fetch(it0, a);
+    fetch(it1, b);
+    const auto turn = [&](Loaded& now, Loaded& next, Loaded& last) {
+        fetch(it2, last);
+        add(it0, now);
+        if (it1.i != it0.i || it1.range != it0.range) flush(it0.i, it0.range, next);
+        it0 = it1;
+        it1 = it2;
+        it2 = after(it2);
+        return it0.i != kEnd;
+    };
+    while (turn(a, b, c) && turn(b, c, a) && turn(c, a, b)) {
     }
 }
 
