@@ -259,6 +259,34 @@ __device__ __forceinline__ void sort_by_rank_lds(uint2* column, uint32_t stride,
     });
 }
 
+// The same through columns of four-byte cells, half the LDS, one kind of value at a time.
+template <int D>
+__device__ __forceinline__ uint32_t rank_row(ivec<D + 1> rank, int c) {
+    return static_cast<uint32_t>(rank[c] < 0 ? 0 : (rank[c] > D ? D : rank[c]));  // (the clamp: as in sort_by_rank_lds)
+}
+template <int D>
+__device__ __forceinline__ fvec<D + 1> by_rank_lds(uint32_t* column, uint32_t stride, ivec<D + 1> rank, fvec<D + 1> in) {
+    static_for<D + 1>(PENC_BODY(c) {
+        PENC_INDEX(c);
+        const float x = in[c];
+        column[rank_row<D>(rank, c) * stride] = __builtin_bit_cast(uint32_t, x);
+    });
+    fvec<D + 1> out;
+    static_for<D + 1>(PENC_BODY(m) {
+        PENC_INDEX(m); out[m] = __builtin_bit_cast(float, column[m * stride]); });
+    return out;
+}
+template <int D>
+__device__ __forceinline__ uvec<D + 1> vertex_hashes_lds(uint32_t* column, uint32_t stride, ivec<D + 1> rank, uint32_t hash0) {
+    static_for<D + 1>(PENC_BODY(c) {
+        PENC_INDEX(c); column[rank_row<D>(rank, c) * stride] = hash_step<D, c>(); });
+    uvec<D + 1> hashes;
+    hashes[0] = hash0;
+    static_for<D>(PENC_BODY(r) {
+        PENC_INDEX(r); hashes[r + 1] = hashes[r] + column[(D - r) * stride]; });
+    return hashes;
+}
+
 // The three gradient chains below evaluate their sums in the same order, with the same
 // intermediate roundings, as the reference's loops, so that every term a kernel adds is the same
 // fp32 number the CPU checker computes; only the order of atomic accumulation can then differ.

@@ -62,6 +62,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                         float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
     constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
     __shared__ ScatterStateT<stage_chunk(D)> state;
+    __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kScatterBlock : 1];
     // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
     // workgroup of a die takes level j % levels of one group of points: a die works through all
     // levels of a group before the next group, so the points are fetched from memory once, and
@@ -180,6 +181,17 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                 w = barycentric_of_sorted<D>(sorted) * w_level;
             }
             wave_lds_fence();  // the slice is staging space again from here on
+        } else if constexpr (D > kWorkgroupSortMaxDim) {
+            // the other modes have no such slice: columns of their own
+            uint32_t* const column = rank_columns + threadIdx.x;
+            h = vertex_hashes_lds<D>(column, kScatterBlock, s.rank, s.hash0);
+            if constexpr (kOrder != kSecondOrder) w = barycentric_of_sorted<D>(by_rank_lds<D>(column, kScatterBlock, s.rank, s.delta)) * w_level;
+            if constexpr (kOrder != kFirstOrder) {
+                const fvec<D + 1> second = sorted_elevated_grad_to_bary<D>(by_rank_lds<D>(
+                                               column, kScatterBlock, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D))) * w_level;
+                if constexpr (kBoth) w2 = second;
+                else w = second;
+            }
         } else {
             h = vertex_hashes<D>(s.rank, s.hash0);
             if constexpr (kBoth) {
