@@ -859,6 +859,14 @@ inline unsigned scatter_groups(int64_t n, int tiles_per_group) {
 // 0.065 -> 0.055 ms and 2^14 points 0.062 -> 0.048 ms with two; 2^17 points are best with eight).  That is for the
 // small batches that the sorted groups below do not take: few levels, sparse or mostly empty gradients, a workspace too small.
 constexpr int64_t kMinWorkgroups = 768;  // three per compute unit
+// Rows of an upstream gradient are read by every level of a group, and what a die holds of them at a time should fit its L2: four
+// groups of 16 tiles are 6 MB of rows of 48 columns.  With eight the longer segments are missed less than the rows (`short_groups`; scatter
+// and reduction, us, 16 -> 8 tiles: D = 3, 24 levels of 2^18 slots, 2^20 points 515 -> 505, 2^19 280 -> 272, 16 levels of 2^16 slots 314 -> 311; D = 4,
+// 24 levels 659 -> 649; D = 5, 16 levels 324 -> 320).  Not with two dimensions (230 -> 236), four features (317 -> 320), whose rows
+// more than one pair of features reads, or more than kStageBins bins, whose runs are short as it is (2^22 slots 1212 -> 1290).
+inline bool short_groups(int pos_dim, uint32_t feat_pairs, int capacity, bool rows) {
+    return rows && pos_dim >= 3 && feat_pairs == 1u && bins_for_capacity(capacity) <= static_cast<uint32_t>(kStageBins);
+}
 inline int table_backward_tiles(int64_t n, int levels) {
     if (static_cast<int64_t>(scatter_groups(n, kScatterTilesLarge)) * levels >= kLargeGroupsMinWorkgroups) return kScatterTilesLarge;
     int tiles = kScatterTiles;
@@ -1243,6 +1251,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         return check_launch();
     }
     int tiles_per_group = table_backward_tiles(nr_positions, pair_levels);
+    if (tiles_per_group > kScatterTiles && short_groups(pos_dim, feat_pairs, capacity, t.rows)) tiles_per_group = kScatterTiles;
     BinPlan plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, workspace, workspace_bytes);
     if (!plan.enabled && tiles_per_group > kScatterTiles) {  // wide bins need short segments: smaller groups of points
         tiles_per_group = kScatterTiles;
