@@ -10,7 +10,7 @@ namespace penc {
 // Second kernel of stage 2: a workgroup sums the records of one (bin, level) in LDS (fp64,
 // ds_add_f64: a few hot slots must not serialise the whole bin, which rules out a compare-and-swap
 // loop) and adds the bin's slot range into the gradient.  gridDim.z workgroups share a bin, each
-// taking a contiguous range of the scattering workgroups' segments (a launch over few levels would
+// taking a contiguous range of the scattering workgroups' segments (a launch over few bins and levels would
 // otherwise leave most of the chip idle).  Each wavefront takes whole segments, so its loads are
 // contiguous.  With one workgroup per bin nothing else touches the bin's slots while this kernel
 // runs (the scattering kernel before it has completed, and bins do not overlap), so the final add is
@@ -227,13 +227,13 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
         return;
     }
     if (threadIdx.x == 0 && untouched_so_far) bins.direct[bin] = 1u;  // (the workgroups that share the bin all store the same value)
-    for (uint32_t s = threadIdx.x; s < static_cast<uint32_t>(kBinSlots); s += kReduceBlock) {
-        const double v0 = acc0[s], v1 = acc1[s];
-        if ((v0 != 0.0 || v1 != 0.0) && slot0 + s < capacity) {
-            float2* cell = reinterpret_cast<float2*>(level_grad.at(slot0 + s));
-            global_add(&cell->x, static_cast<float>(v0));
-            global_add(&cell->y, static_cast<float>(v1));
-        }
+    // Both features of a slot by two neighbouring lanes, so that an instruction's adds fall into half as many 64-byte segments (16 levels
+    // of 2^16 slots, four features, 2^18 points: 48 -> 34 us).
+    const double* const acc = (threadIdx.x & 1u) != 0u ? acc1 : acc0;
+#pragma unroll 4
+    for (uint32_t s = threadIdx.x >> 1; s < static_cast<uint32_t>(kBinSlots); s += kReduceBlock / 2) {
+        const double v = acc[s];
+        if (v != 0.0 && slot0 + s < capacity) global_add(level_grad.at(slot0 + s) + (threadIdx.x & 1u), static_cast<float>(v));
     }
 }
 
