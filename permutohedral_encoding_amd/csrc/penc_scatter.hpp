@@ -458,12 +458,15 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 // Stage 2 for a whole tile once the workgroup streams (see scatter_mode_decide): the cache's LDS is
 // staging space for a counting sort of the tile's records by bin, stage_chunk(D) vertices per thread
 // at a time (2048 or 2560 records).  Every wave counts its records per bin (one LDS counter per
-// bin and wave); the first wave turns the counts into run offsets (a bin's run is the waves' runs
-// one after the other) and reserves room for each bin's run in the workgroup's segment with one
-// add per bin; the waves lay their records out in that order in the staging space; and then all
+// bin and wave); then every wave, lane b looking after bin b, turns all waves' counts into the offsets of its own runs (a bin's run is the
+// waves' runs one after the other) and lays its records out in that order in the staging space; and then all
 // threads store the records in staging order: a wave instruction writes 64 consecutive records
 // of (mostly) one bin, i.e. whole cache lines, where the records of a single wave would leave in
-// runs of eight.  A staged record carries its destination (its index in the level's record
+// runs of eight.  How far the workgroup's segment of a bin is filled (`cursor`, lane b's is bin b's) every wave
+// knows from the same sums.  (With the offsets made by the first wave for all, and a cursor in LDS, the others waited for it at a
+// barrier of its own.  Scatter and reduction of the finest 12 of 24 levels of 2^18 slots, D = 3, 2^20 points: 348 -> 322 us, of the finest four
+// 149 -> 119; D = 4, second order, 12 levels 437 -> 412; with the coarse levels beside them, which keep the vector units busy, the same.)
+// A staged record carries its destination (its index in the level's record
 // array), so the store needs no search.  When a run does not fit its segment any more (rare: the
 // segments hold the mean plus three standard deviations) the chunk checks every record against
 // the room left and sends the excess to stage 3.
@@ -472,21 +475,18 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 template <int D, typename State>
 __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
-                                            fvec<D + 1> a1) {
+                                            fvec<D + 1> a1, uint32_t& cursor) {
     constexpr int kWaves = kScatterBlock / 64;
     constexpr int kStageChunk = State::kChunk;
-    static_assert(kCacheLines >= (3 * kWaves + 3) * 64, "the sort's index arrays live in the tag array");
+    static_assert(kCacheLines >= 3 * kWaves * 64, "the sort's index arrays live in the tag array");
     static_assert(offsetof(State, stage_tail) == offsetof(State, val) + sizeof(c.val) &&
                       (sizeof(c.val) + (State::kTail > 0 ? sizeof(c.stage_tail) : 0)) == kStageChunk * kScatterBlock * sizeof(uint4),
                   "val and stage_tail are one contiguous staging array");
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t* const words = reinterpret_cast<uint32_t*>(c.tag);
-    uint32_t* const count = words + wave * 64;                  // [wave][bin] records of this wave per bin
-    uint32_t* const offset = words + (kWaves + wave) * 64;      // [wave][bin] where the wave's run starts in the staging array
-    uint32_t* const dest = words + (2 * kWaves + wave) * 64;    // [wave][bin] index of the run's first record in the level's record array
-    uint32_t* const run_first = words + 3 * kWaves * 64;        // [bin] index of the workgroup's run for the bin
-    uint32_t* const room = run_first + 64;                      // [bin] records the workgroup's segment can still take
-    uint32_t* const header = room + 64;                         // [0] records staged, [1] whether every run fits
+    uint32_t* const count = words + wave * 64;  // [wave][bin] records of this wave per bin
+    // [bin] of this wave: where its run starts in the staging array, and the index of the run's first record in the level's record array
+    uint2* const run = reinterpret_cast<uint2*>(words + kWaves * 64) + wave * 64;
     uint4* const stage = reinterpret_cast<uint4*>(c.val);
     constexpr uint32_t kNoRoom = 0xFFFFFFFFu;
     constexpr int kChunks = (D + 1 + kStageChunk - 1) / kStageChunk;
@@ -501,47 +501,34 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
             PENC_INDEX(j);
             if (active) place[j] = atomicAdd(&count[slot[kFirst + j] >> kBinSlotsLog2], 1u);
         });
-        __syncthreads();
-        if (wave == 0) {  // lane b looks after bin b
-            uint32_t before[kWaves], mine = 0u;
+        __syncthreads();  // all waves have counted, and have left the staging array of the chunk before
+        uint32_t before = 0u, mine = 0u;
 #pragma unroll
-            for (int w = 0; w < kWaves; ++w) {
-                before[w] = mine;
-                mine += words[w * 64 + lane];
-            }
-            uint32_t total;
-            const uint32_t first = wave_exclusive_scan(mine, total);
-            const uint32_t taken = mine != 0u ? atomicAdd(&c.bin_count[lane], mine) : 0u;
-            const uint32_t start = (lane * bins.n_groups + group) * bins.segment_capacity + taken;
-            const bool all_fit = __all(taken + mine <= bins.segment_capacity);
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) {
-                words[(kWaves + w) * 64 + lane] = first + before[w];
-                words[(2 * kWaves + w) * 64 + lane] = start + before[w];
-            }
-            run_first[lane] = start;
-            room[lane] = taken < bins.segment_capacity ? bins.segment_capacity - taken : 0u;
-            if (lane == 0) {
-                header[0] = total;
-                header[1] = all_fit ? 1u : 0u;
-            }
+        for (int w = 0; w < kWaves; ++w) {
+            const uint32_t n = words[w * 64 + lane];
+            before += w < static_cast<int>(wave) ? n : 0u;
+            mine += n;
         }
-        __syncthreads();
-        const uint32_t total = header[0];
-        const bool all_fit = header[1] != 0u;
+        uint32_t total;
+        const uint32_t first = wave_exclusive_scan(mine, total);
+        run[lane] = make_uint2(first + before, (lane * bins.n_groups + group) * bins.segment_capacity + cursor + before);
+        cursor += mine;
+        const bool all_fit = __all(cursor <= bins.segment_capacity);
+        wave_lds_fence();
         static_for<kCount>(PENC_BODY(j) {
             PENC_INDEX(j);
             if (active) {
                 const uint32_t b = slot[kFirst + j] >> kBinSlotsLog2;
                 // copies first: a bit cast applied directly to a vector element reads element 0
                 const float v0 = a0[kFirst + j], v1 = a1[kFirst + j];
-                const uint32_t to = dest[b] + place[j];
+                const uint2 at = run[b];
+                const uint32_t to = at.y + place[j];
                 uint4 e;
                 e.x = slot[kFirst + j];
                 e.y = __builtin_bit_cast(uint32_t, v0);
                 e.z = __builtin_bit_cast(uint32_t, v1);
-                e.w = all_fit || to - run_first[b] < room[b] ? to : kNoRoom;
-                stage[offset[b] + place[j]] = e;
+                e.w = all_fit || to < (b * bins.n_groups + group + 1u) * bins.segment_capacity ? to : kNoRoom;
+                stage[at.x + place[j]] = e;
             }
         });
         __syncthreads();
@@ -561,8 +548,8 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
             if (!all_fit && __any(spill))
                 global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
         });
-        // the next chunk (or tile) writes the counters after this wave's loads above and the staging
-        // array after its next two barriers: nothing here is overwritten while another wave reads it
+        // the next chunk (or tile) writes this wave's counters, which the others have read before the barrier above, and the
+        // staging array after its own first barrier: nothing here is overwritten while another wave reads it
         wave_lds_fence();
     });
 }
@@ -863,12 +850,12 @@ __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_gr
 template <int D, typename State>
 __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                                  uint32_t group, bool active, bool use_cache, int mode, uint32_t id_bits,
-                                                 uvec<D + 1> slot, fvec<D + 1> a0, fvec<D + 1> a1) {
+                                                 uvec<D + 1> slot, fvec<D + 1> a0, fvec<D + 1> a1, uint32_t& cursor) {
     if (mode == kModeStream) {
         if (bins.n_bins > kStageBins) {
             stream_tile_many<D>(c, level_grad, bins, group, active, slot, a0, a1);
         } else if constexpr (D <= kWorkgroupSortMaxDim) {  // measured: the workgroup-wide sort wins up to D = 5, the per-wave one from D = 6 on
-            stream_tile<D>(c, level_grad, bins, group, active, slot, a0, a1);
+            stream_tile<D>(c, level_grad, bins, group, active, slot, a0, a1, cursor);
         } else {
             stream_tile_wave<D>(c, level_grad, bins, group, active, slot, a0, a1);
         }
@@ -1019,9 +1006,11 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
 // After the last tile: flushes the accumulate cache or the columns (through the bins when there are
 // any; a streaming workgroup has neither left) and publishes how many records this workgroup left in each
 // bin.  Call once, by all threads.
-template <typename State>
+template <int D, typename State>
 __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_grad, const BinTarget& bins,
-                                            uint32_t group, int mode, uint32_t id_bits) {
+                                            uint32_t group, int mode, uint32_t id_bits, uint32_t cursor) {
+    // (stream_tile keeps count in registers)
+    if (D <= kWorkgroupSortMaxDim && mode == kModeStream && bins.n_bins <= kStageBins && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
     __syncthreads();
     if (mode == kModeCache) cache_flush(c, level_grad, bins, group);
     if (mode == kModeColumns) column_flush(c, level_grad, id_bits);

@@ -127,7 +127,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s1 = group_second1[nn];
     }
     int mode = kModeCache;
-    uint32_t id_bits = 0;
+    uint32_t id_bits = 0, cursor = 0;
     for (int t = 0; t < tiles_per_group; ++t) {
         const int64_t tile_base = group_base + static_cast<int64_t>(t) * kScatterBlock;
         if (tile_base >= n_points) break;
@@ -229,7 +229,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             a0 += w2 * s0;
             a1 += w2 * s1;
         }
-        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1);
+        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1, cursor);
         // the first tile finds the lines its own look-up has claimed: no evidence of reuse
         if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
         pos = pos_next;
@@ -239,7 +239,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s0 = s0_next;
         s1 = s1_next;
     }
-    scatter_end(state, level_grad, bins, group, mode, id_bits);
+    scatter_end<D>(state, level_grad, bins, group, mode, id_bits, cursor);
 }
 
 #define PENC_TABLE_PARAMETERS                                                                                                          \
