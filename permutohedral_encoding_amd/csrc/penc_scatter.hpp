@@ -61,7 +61,7 @@ constexpr int kColumnMinIdsLog2 = 5;   // column mode: the cache's kCacheLines c
 #define PENC_COLUMN_MAX_IDS_LOG2 7
 #endif
 constexpr int kColumnMaxIdsLog2 = PENC_COLUMN_MAX_IDS_LOG2;   // ... up to 128 columns of 16 cells, by the number of distinct slots the first tile has shown
-constexpr int kColumnProbes = 16;      // linear probes before a contribution gives up on the column table
+constexpr int kColumnProbes = 16;      // entries a contribution looks at before it gives up on a column
 enum ScatterMode : int { kModeCache = 0, kModeStream = 1, kModeColumns = 2 };
 // vertices per thread a wave sorts by bin in one go (256 or 320 records): all D+1 of them up to D = 4
 constexpr int stage_chunk(int pos_dim) { return pos_dim + 1 <= 4 ? 4 : 5; }
@@ -378,6 +378,7 @@ struct ScatterStateT {
     uint32_t wanted;               // contributions of the first tile
     uint32_t lines;                // lines they claimed: the tile's distinct slots, as far as the cache could take them
     uint32_t misses;               // contributions whose slot found no line
+    uint32_t columns;              // columns given away (kModeColumns)
     uint32_t strangers;            // slots of the second tile that the first tile did not touch (counted for levels with few slots)
 };
 
@@ -395,6 +396,7 @@ __device__ __forceinline__ void scatter_begin(State& c) {
         c.lines = 0u;
         c.misses = 0u;
         c.strangers = 0u;
+        c.columns = 0u;
     }
     __syncthreads();
 }
@@ -769,28 +771,57 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
 }
 
 // Column mode of stage 1, for a level whose points share a few dozen slots.  The cache's values
-// are re-laid as 2^id_bits columns of kCacheLines >> id_bits cells; a slot owns a column (found
-// through the first 2^id_bits tags, open addressing with linear probing) and a lane adds into the
+// are re-laid as 2^id_bits columns of kCacheLines >> id_bits cells; a slot owns a column and a lane adds into the
 // cell (lane mod cells) of its slot's column.  With 64 cells a lane meets no other lane of its
 // wave, whatever the slots; with 32 or 16 cells two or four lanes share a cell.  The columns are
-// summed when the level ends (column_flush).  Returns the column of `slot`, or -1 when the probes
-// find only other slots (the contribution then takes stage 2 or 3 like any miss).
+// summed when the level ends (column_flush).
+// A slot finds its column through kColumnEntries entries, eight and more times as many as there are columns, so that nearly every
+// look-up ends at its first entry; among as many entries as columns the last lane of a wave took several probes (D = 3, 2^20 points, the six
+// coarsest of 24 levels 106 -> 96 us).  Tags, the entries' columns and the columns' slots share the tag array.
+constexpr uint32_t kColumnEntriesLog2 = 10, kColumnEntries = 1u << kColumnEntriesLog2;
+constexpr uint32_t kColumnPending = 0xFFu, kNoColumn = 0xFEu;  // in place of an entry's column: not known yet, none was left
+static_assert(kCacheLines >= static_cast<int>(kColumnEntries + kColumnEntries / 4 + (1u << kColumnMaxIdsLog2)), "they fit the tag array");
+static_assert((1u << kColumnMaxIdsLog2) <= kNoColumn, "a column's number is kept in a byte");
 template <typename State>
-__device__ __forceinline__ int column_find(State& c, uint32_t slot, uint32_t id_bits) {
+__device__ __forceinline__ uint8_t* column_of_entry(State& c) { return reinterpret_cast<uint8_t*>(c.tag + kColumnEntries); }
+template <typename State>
+__device__ __forceinline__ int* slot_of_column(State& c) { return c.tag + kColumnEntries + kColumnEntries / 4; }
+__device__ __forceinline__ uint32_t column_entry(uint32_t slot) { return (slot * 0x9E3779B1u) >> (32 - kColumnEntriesLog2); }
+
+// Looks on from entry `e` for the slot, and gives it an entry and a column where it has none.  Returns the column, or kNoColumn
+// when no entry or column is left (the contribution then takes stage 2 or 3 like any miss).  A lane that finds the slot's entry
+// just taken looks again until it says which column, a few times at most: a miss would leave a record, and a level without records
+// costs its reducers nothing.
+template <typename State>
+__device__ __forceinline__ uint32_t column_search(State& c, uint32_t slot, uint32_t e, uint32_t id_bits) {
     const int want = static_cast<int>(slot);
-    const uint32_t mask = (1u << id_bits) - 1u;
-    uint32_t e = (slot * 0x9E3779B1u) >> (32 - id_bits);
+    uint32_t column = kNoColumn;
 #pragma unroll 1
     for (int probe = 0; probe < kColumnProbes; ++probe) {
         int owner = c.tag[e];
-        if (owner == want) return static_cast<int>(e);
         if (owner == -1) {
             owner = atomicCAS(&c.tag[e], -1, want);
-            if (owner == -1 || owner == want) return static_cast<int>(e);
+            if (owner == -1) {
+                const uint32_t next = atomicAdd(&c.columns, 1u);
+                const bool left = next < (1u << id_bits);
+                if (left) slot_of_column(c)[next] = want;
+                column_of_entry(c)[e] = static_cast<uint8_t>(left ? next : kNoColumn);
+                owner = want;
+            }
         }
-        e = (e + 1u) & mask;
+        // (the lanes of a wave meet here: what one of them has written above, the others read)
+        __builtin_amdgcn_wave_barrier();
+        if (owner == want) {
+#pragma unroll 1
+            for (int look = 0; look < 64; ++look) {
+                column = __hip_atomic_load(column_of_entry(c) + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (column != kColumnPending) break;
+            }
+            break;
+        }
+        e = (e + 1u) & (kColumnEntries - 1u);
     }
-    return -1;
+    return column != kColumnPending ? column : kNoColumn;
 }
 
 template <int D, typename State>
@@ -803,9 +834,12 @@ __device__ __forceinline__ void column_tile(State& c, const GradSlice& level_gra
         PENC_INDEX(r);
         bool miss = active;
         if (active) {
-            const int e = column_find(c, slot[r], id_bits);
-            if (e >= 0) {
-                const uint32_t cell = (static_cast<uint32_t>(e) << cell_bits) | my_cell;
+            const uint32_t e = column_entry(slot[r]);
+            const int owner = c.tag[e];
+            uint32_t column = column_of_entry(c)[e];
+            if (owner != static_cast<int>(slot[r]) || column == kColumnPending) column = column_search(c, slot[r], e, id_bits);
+            if (column != kNoColumn) {
+                const uint32_t cell = (column << cell_bits) | my_cell;
                 __hip_atomic_fetch_add(&c.val[0][cell], static_cast<double>(a0[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_fetch_add(&c.val[1][cell], static_cast<double>(a1[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 miss = false;
@@ -822,7 +856,7 @@ __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_gr
     const uint32_t cell_bits = kCacheLinesLog2 - id_bits, cells = 1u << cell_bits;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (uint32_t id = wave; id < (1u << id_bits); id += kScatterBlock / 64) {
-        const int owner = c.tag[id];  // the same for all lanes of the wave
+        const int owner = slot_of_column(c)[id];  // the same for all lanes of the wave
         if (owner == -1) continue;
         double s0 = lane < cells ? c.val[0][(id << cell_bits) + lane] : 0.0;
         double s1 = lane < cells ? c.val[1][(id << cell_bits) + lane] : 0.0;
@@ -997,7 +1031,7 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
         mode = kModeColumns;
         id_bits = kColumnMinIdsLog2;
         while ((1u << (id_bits - 1)) < expected_slots && id_bits < static_cast<uint32_t>(kColumnMaxIdsLog2)) ++id_bits;
-        for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) c.tag[e] = -1;  // now the table of columns
+        for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) c.tag[e] = -1;  // now entries, without columns
         __syncthreads();
     }
     return mode;
