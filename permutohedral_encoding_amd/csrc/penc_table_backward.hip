@@ -83,7 +83,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
                                2 * feat_pairs, bins.direct, bins.bin_shift};
     // Everything a thread reads lies within its group of at most 16 x 512 points, so the addresses are
-    // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets.
+    // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets in bytes: the form the load instructions take.
     const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);
     const float* const group_positions = positions + group_base * D;
     const float* const group_q = kNeedsQ ? double_pos_grad + group_base * D : nullptr;
@@ -91,22 +91,24 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         kRowMajor ? grad_sliced + group_base * grad_row_stride + 2 * pair_level
                   : grad_sliced + (static_cast<size_t>(pair_level) * 2) * n_points + group_base;
     const float* const group_grad1 = group_grad0 + n_points;
+    const auto at_byte = [](const float* base, uint32_t offset) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + offset); };
     const auto load_grad = [&](uint32_t i, float& g0, float& g1) {
         if constexpr (kRowMajor) {
             const float2 g = *reinterpret_cast<const float2*>(group_grad0 + static_cast<int64_t>(i) * grad_row_stride);
             g0 = g.x;
             g1 = g.y;
         } else {
-            g0 = group_grad0[i];
-            g1 = group_grad1[i];
+            g0 = *at_byte(group_grad0, i * 4u);
+            g1 = *at_byte(group_grad1, i * 4u);
         }
     };
     const float* const group_second0 = kBoth ? second_grad + (static_cast<size_t>(pair_level) * 2) * n_points + group_base : nullptr;
     const float* const group_second1 = group_second0 + n_points;
     const auto load_group_point = [&](const float* base, uint32_t i) {
+        const float* const p = at_byte(base, i * static_cast<uint32_t>(D * sizeof(float)));
         fvec<D> v;
         static_for<D>(PENC_BODY(k) {
-            PENC_INDEX(k); v[k] = base[i * static_cast<uint32_t>(D) + k]; });
+            PENC_INDEX(k); v[k] = p[k]; });
         return v;
     };
     // A tile's inputs are fetched one tile ahead: their latency then overlaps the previous tile's
@@ -140,8 +142,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         load_grad(nn_next, g0_next, g1_next);
         float s0_next = 0.0f, s1_next = 0.0f;
         if constexpr (kBoth) {
-            s0_next = group_second0[nn_next];
-            s1_next = group_second1[nn_next];
+            s0_next = *at_byte(group_second0, nn_next * 4u);
+            s1_next = *at_byte(group_second1, nn_next * 4u);
         }
         if constexpr (kRowMajor) {
             if (grad_level_major != nullptr && active) {
