@@ -50,6 +50,8 @@ constexpr int kBlock = 256;            // threads per workgroup of the gather-ty
 #define PENC_CACHE_LINES_LOG2 11
 #endif
 constexpr int kScatterBlock = PENC_SCATTER_BLOCK;  // threads per scattering workgroup (its wavefronts share one accumulate cache)
+constexpr int kScatterBlockManyBins = 2 * kScatterBlock;  // ... for tables of more than kFewerOpenLinesMinBins bins (see stream_tile_many)
+constexpr uint32_t kFewerOpenLinesMinBins = 256;
 constexpr int kScatterTiles = PENC_SCATTER_TILES;  // tiles of kScatterBlock points a scattering workgroup walks (a "group" of points) ...
 constexpr int kScatterTilesLarge = PENC_SCATTER_TILES_LARGE;  // ... or this many, when the launch still has workgroups to spare
 constexpr int kCacheLinesLog2 = PENC_CACHE_LINES_LOG2;
@@ -363,10 +365,10 @@ __device__ __forceinline__ uint32_t fold_shared_slots(uint32_t slot, bool& live,
 // lines are hit by many lanes at once (that is what the cache is for), where a compare-and-swap
 // loop degrades quadratically (measured: 10-40x slower on the coarsest levels) and ds_add_f32 is
 // slow on this chip.  The fp64 partial sums are rounded to fp32 once, when the cache is flushed.
-template <int kStageChunk>
+template <int kStageChunk, int kBlockThreads>
 struct ScatterStateT {
-    static constexpr int kChunk = kStageChunk;
-    static constexpr int kTail = (kScatterBlock / 64) * kStageChunk * 64 - kCacheLines;
+    static constexpr int kChunk = kStageChunk, kThreads = kBlockThreads;
+    static constexpr int kTail = (kThreads / 64) * kStageChunk * 64 - kCacheLines;
     static_assert(kTail >= 0, "the staging slices cover the cache's values");
     int tag[kCacheLines];
     double val[2][kCacheLines];  // one array per feature: random lines then spread over all LDS bank pairs
@@ -384,12 +386,12 @@ struct ScatterStateT {
 
 template <typename State>
 __device__ __forceinline__ void scatter_begin(State& c) {
-    for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) {
+    for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) {
         c.tag[e] = -1;
         c.val[0][e] = 0.0;
         c.val[1][e] = 0.0;
     }
-    for (int b = threadIdx.x; b < kMaxBins; b += kScatterBlock) c.bin_count[b] = 0u;
+    for (int b = threadIdx.x; b < kMaxBins; b += State::kThreads) c.bin_count[b] = 0u;
     if (threadIdx.x == 0) {
         c.hits = 0u;
         c.wanted = 0u;
@@ -478,11 +480,11 @@ template <int D, typename State>
 __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
                                             fvec<D + 1> a1, uint32_t& cursor) {
-    constexpr int kWaves = kScatterBlock / 64;
+    constexpr int kWaves = State::kThreads / 64;
     constexpr int kStageChunk = State::kChunk;
     static_assert(kCacheLines >= 3 * kWaves * 64, "the sort's index arrays live in the tag array");
     static_assert(offsetof(State, stage_tail) == offsetof(State, val) + sizeof(c.val) &&
-                      (sizeof(c.val) + (State::kTail > 0 ? sizeof(c.stage_tail) : 0)) == kStageChunk * kScatterBlock * sizeof(uint4),
+                      (sizeof(c.val) + (State::kTail > 0 ? sizeof(c.stage_tail) : 0)) == kStageChunk * State::kThreads * sizeof(uint4),
                   "val and stage_tail are one contiguous staging array");
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t* const words = reinterpret_cast<uint32_t*>(c.tag);
@@ -536,7 +538,7 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
         __syncthreads();
         static_for<kCount>(PENC_BODY(j) {
             PENC_INDEX(j);
-            const uint32_t i = j * kScatterBlock + threadIdx.x;
+            const uint32_t i = j * State::kThreads + threadIdx.x;
             bool spill = false;
             uint4 e = {0u, 0u, 0u, 0u};
             if (i < total) {
@@ -563,14 +565,19 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
 // records in each, but even runs of four records are worth it: appended one at a time, every
 // 12-byte record is a store of its own to one of hundreds of open cache lines (measured on a
 // 2^22-slot table: 42 us per level against 13 us for the sorted stores of a 2^18-slot one).
+// What it waits for with the most bins is the lines the records go to: a workgroup leaves a line open in every bin, and of 512 bins and the 96
+// workgroups of a die those are 6 MB, which its L2 writes out part by part.  So workgroups of twice the threads serve them, of which
+// a compute unit holds one: a third of the open lines, and twice the records in a run.  (Scatter, reduction and fill, us: 2^22 slots, D = 3, 2^20
+// points, 24 levels 1203 -> 1046, the finest eight 664 -> 604; 200001 points 537 -> 512; D = 4, 16 levels, 2^19 points 579 -> 533; D = 8, 2^17 points
+// 427 -> 423.  With 256 bins, whose open lines nearly fit, 24 levels 855 -> 780 but 16 coarser ones from rows 502 -> 566; with 128 599 -> 661.)
 // The counters must be zero on entry (scatter_mode_decide clears them; every call leaves them so).
 template <int D, typename State>
 __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                                  uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
                                                  fvec<D + 1> a1) {
-    constexpr int kWaves = kScatterBlock / 64;
+    constexpr int kWaves = State::kThreads / 64;
     constexpr int kStageChunk = State::kChunk;
-    static_assert(kMaxBins <= kScatterBlock, "one thread per bin");
+    static_assert(kMaxBins <= State::kThreads, "one thread per bin");
     static_assert(kCacheLines >= 3 * kMaxBins + kWaves, "the sort's index arrays live in the tag array");
     const uint32_t wave = threadIdx.x >> 6;
     uint32_t* const words = reinterpret_cast<uint32_t*>(c.tag);
@@ -637,7 +644,7 @@ __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& leve
         __syncthreads();
         static_for<kCount>(PENC_BODY(j) {
             PENC_INDEX(j);
-            const uint32_t i = j * kScatterBlock + threadIdx.x;
+            const uint32_t i = j * State::kThreads + threadIdx.x;
             bool spill = false;
             uint4 e = {0u, 0u, 0u, 0u};
             if (i < total) {
@@ -674,7 +681,7 @@ template <int D, typename State>
 __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
                                             fvec<D + 1> a1) {
-    constexpr int kWaves = kScatterBlock / 64;
+    constexpr int kWaves = State::kThreads / 64;
     constexpr int kStageChunk = State::kChunk;
     static_assert(kCacheLines / kWaves >= 4 * 64, "four 64-entry arrays per wave live in the tag array");
     static_assert(offsetof(State, stage_tail) == offsetof(State, val) + sizeof(c.val) &&
@@ -855,7 +862,7 @@ template <typename State>
 __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_grad, uint32_t id_bits) {
     const uint32_t cell_bits = kCacheLinesLog2 - id_bits, cells = 1u << cell_bits;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (uint32_t id = wave; id < (1u << id_bits); id += kScatterBlock / 64) {
+    for (uint32_t id = wave; id < (1u << id_bits); id += State::kThreads / 64) {
         const int owner = slot_of_column(c)[id];  // the same for all lanes of the wave
         if (owner == -1) continue;
         double s0 = lane < cells ? c.val[0][(id << cell_bits) + lane] : 0.0;
@@ -886,7 +893,9 @@ __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& leve
                                                  uint32_t group, bool active, bool use_cache, int mode, uint32_t id_bits,
                                                  uvec<D + 1> slot, fvec<D + 1> a0, fvec<D + 1> a1, uint32_t& cursor) {
     if (mode == kModeStream) {
-        if (bins.n_bins > kStageBins) {
+        if constexpr (State::kThreads > kScatterBlock) {  // (for many bins alone)
+            stream_tile_many<D>(c, level_grad, bins, group, active, slot, a0, a1);
+        } else if (bins.n_bins > kStageBins) {
             stream_tile_many<D>(c, level_grad, bins, group, active, slot, a0, a1);
         } else if constexpr (D <= kWorkgroupSortMaxDim) {  // measured: the workgroup-wide sort wins up to D = 5, the per-wave one from D = 6 on
             stream_tile<D>(c, level_grad, bins, group, active, slot, a0, a1, cursor);
@@ -947,7 +956,7 @@ template <int D, typename State>
 __device__ __forceinline__ bool cache_pays(const State& c, int tile, uint32_t one_in = 8u) {
     const uint32_t settled = c.lines + c.misses;
     const uint32_t first_hits = c.wanted > settled ? c.wanted - settled : 0u;
-    const uint32_t seen = c.wanted + static_cast<uint32_t>(tile > 1 ? tile - 1 : 0) * kScatterBlock * (D + 1);
+    const uint32_t seen = c.wanted + static_cast<uint32_t>(tile > 1 ? tile - 1 : 0) * State::kThreads * (D + 1);
     return (first_hits + c.hits) * one_in >= seen;
 }
 
@@ -955,7 +964,7 @@ __device__ __forceinline__ bool cache_pays(const State& c, int tile, uint32_t on
 template <typename State>
 __device__ __forceinline__ void cache_flush(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group) {
-    for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) {
+    for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) {
         const int owner = c.tag[e];
         if (owner != -1) {
             const float v0 = static_cast<float>(c.val[0][e]), v1 = static_cast<float>(c.val[1][e]);
@@ -995,7 +1004,7 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
     }
     __syncthreads();  // every line the tile wants is claimed
     uint32_t used = 0;
-    for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) used += __popcll(__ballot(c.tag[e] != -1));
+    for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) used += __popcll(__ballot(c.tag[e] != -1));
     if ((threadIdx.x & 63) == 0 && used != 0u) atomicAdd(&c.lines, used);
     // Columns are for a level whose few slots the whole group shares.  The first tile shows that when the points come in no
     // particular order; where they follow each other in space (every tile another ray, or the next stretch of a space-filling
@@ -1024,14 +1033,14 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
     if (can_stream && !cache_pays<D>(c, 0, 4u)) {
         mode = kModeStream;
         if (bins.n_bins > kStageBins) {  // stream_tile_many wants its per-bin counters cleared
-            for (int e = threadIdx.x; e < kMaxBins; e += kScatterBlock) c.tag[e] = 0;
+            for (int e = threadIdx.x; e < kMaxBins; e += State::kThreads) c.tag[e] = 0;
             __syncthreads();
         }
     } else if (few_slots && expected_slots <= (3u << (kColumnMaxIdsLog2 - 2))) {  // the largest table may end up three quarters full
         mode = kModeColumns;
         id_bits = kColumnMinIdsLog2;
         while ((1u << (id_bits - 1)) < expected_slots && id_bits < static_cast<uint32_t>(kColumnMaxIdsLog2)) ++id_bits;
-        for (int e = threadIdx.x; e < kCacheLines; e += kScatterBlock) c.tag[e] = -1;  // now entries, without columns
+        for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) c.tag[e] = -1;  // now entries, without columns
         __syncthreads();
     }
     return mode;
@@ -1044,13 +1053,13 @@ template <int D, typename State>
 __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, int mode, uint32_t id_bits, uint32_t cursor) {
     // (stream_tile keeps count in registers)
-    if (D <= kWorkgroupSortMaxDim && mode == kModeStream && bins.n_bins <= kStageBins && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
+    if (D <= kWorkgroupSortMaxDim && State::kThreads == kScatterBlock && mode == kModeStream && bins.n_bins <= kStageBins && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
     __syncthreads();
     if (mode == kModeCache) cache_flush(c, level_grad, bins, group);
     if (mode == kModeColumns) column_flush(c, level_grad, id_bits);
     if (bins.records == nullptr) return;
     __syncthreads();
-    for (uint32_t b = threadIdx.x; b < bins.n_bins; b += kScatterBlock) {
+    for (uint32_t b = threadIdx.x; b < bins.n_bins; b += State::kThreads) {
         const uint32_t n = c.bin_count[b];
         bins.counts[static_cast<size_t>(b) * bins.n_groups + group] = n < bins.segment_capacity ? n : bins.segment_capacity;
     }

@@ -19,12 +19,13 @@ namespace penc {
 // 0.577 -> 0.552 ms at D = 4, but 0.735 -> 0.754 ms at D = 5 (11 spilled), which therefore stays at
 // four; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
 // unit: held to 128, 1.334 -> 1.113 ms.
-constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins) {
+constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins, int threads) {
+    if (threads > kScatterBlock) return 4;  // (one workgroup per compute unit)
     if (wide_bins) return pos_dim <= 3 ? 6 : 4;  // (a variable bin width takes six to eight more registers: up to 30 spilled at D = 4)
     return pos_dim <= 4 || (pos_dim == 5 && !second_order) ? 6 : 4;
 }
 
-constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins) { return pos_dim <= 3 && !wide_bins ? 6 : 4; }
+constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins, int threads) { return pos_dim <= 3 && !wide_bins && threads == kScatterBlock ? 6 : 4; }
 
 // kRowMajor: the upstream gradient is read as rows grad[n][2*level + feature] of `grad_row_stride`
 // floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
@@ -51,7 +52,7 @@ constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins) { return p
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
 // reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
 enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
-template <int D, bool kRowMajor, int kOrder, bool kWideBins>
+template <int D, bool kRowMajor, int kOrder, bool kWideBins, int kThreads>
 __device__ __forceinline__ void
 scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
                         uint32_t capacity, uint32_t cap_mask,
@@ -61,8 +62,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                         const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
                         float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
     constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
-    __shared__ ScatterStateT<stage_chunk(D)> state;
-    __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kScatterBlock : 1];
+    __shared__ ScatterStateT<stage_chunk(D), kThreads> state;
+    __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kThreads : 1];
     // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
     // workgroup of a die takes level j % levels of one group of points: a die works through all
     // levels of a group before the next group, so the points are fetched from memory once, and
@@ -71,7 +72,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     // a time).
     const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
     const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
-    const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kScatterBlock;
+    const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kThreads;
     if (group_base >= n_points) return;
     const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;
     const int level = static_cast<int>(pair_level / feat_pairs);  // the geometry's level
@@ -114,7 +115,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     // A tile's inputs are fetched one tile ahead: their latency then overlaps the previous tile's
     // scatter instead of stalling the wave at the top of every iteration.
     const auto point_of = [&](int t) {  // the point this thread handles in tile t, within the group (clamped: the tail re-reads the last point)
-        const uint32_t i = static_cast<uint32_t>(t) * kScatterBlock + threadIdx.x;
+        const uint32_t i = static_cast<uint32_t>(t) * kThreads + threadIdx.x;
         return i < last_in_group ? i : last_in_group;
     };
     uint32_t nn = point_of(0);
@@ -131,7 +132,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     int mode = kModeCache;
     uint32_t id_bits = 0, cursor = 0;
     for (int t = 0; t < tiles_per_group; ++t) {
-        const int64_t tile_base = group_base + static_cast<int64_t>(t) * kScatterBlock;
+        const int64_t tile_base = group_base + static_cast<int64_t>(t) * kThreads;
         if (tile_base >= n_points) break;
         const bool active = tile_base + threadIdx.x < n_points;
         const uint32_t nn_next = point_of(t + 1);
@@ -157,7 +158,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         fvec<D + 1> w;   // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
         fvec<D + 1> w2;  // kBoth: the latter
         bool via_lds = false;
-        if constexpr (D > kWorkgroupSortMaxDim) {
+        if constexpr (D > kWorkgroupSortMaxDim && kThreads == kScatterBlock) {
             // Once the workgroup streams with every wave sorting on its own (stream_tile_wave), a wave's staging
             // slice is idle between its tiles and nobody else touches it: it serves as the thread-private
             // columns that put residuals and hash steps into rank order, in place of D(D+1) selects each
@@ -165,7 +166,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             via_lds = mode == kModeStream && bins.n_bins <= static_cast<uint32_t>(kStageBins);
         }
         if (via_lds) {
-            constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D)>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
+            constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D), kThreads>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
             static_assert((D + 1) * 64 <= kSliceCells, "a wave's staging slice holds a column of D+1 cells per lane");
             uint2* const column = reinterpret_cast<uint2*>(state.val) + (threadIdx.x >> 6) * kSliceCells + (threadIdx.x & 63);
             fvec<D + 1> sorted;
@@ -186,11 +187,11 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         } else if constexpr (D > kWorkgroupSortMaxDim) {
             // the other modes have no such slice: columns of their own
             uint32_t* const column = rank_columns + threadIdx.x;
-            h = vertex_hashes_lds<D>(column, kScatterBlock, s.rank, s.hash0);
-            if constexpr (kOrder != kSecondOrder) w = barycentric_of_sorted<D>(by_rank_lds<D>(column, kScatterBlock, s.rank, s.delta)) * w_level;
+            h = vertex_hashes_lds<D>(column, kThreads, s.rank, s.hash0);
+            if constexpr (kOrder != kSecondOrder) w = barycentric_of_sorted<D>(by_rank_lds<D>(column, kThreads, s.rank, s.delta)) * w_level;
             if constexpr (kOrder != kFirstOrder) {
                 const fvec<D + 1> second = sorted_elevated_grad_to_bary<D>(by_rank_lds<D>(
-                                               column, kScatterBlock, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D))) * w_level;
+                                               column, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D))) * w_level;
                 if constexpr (kBoth) w2 = second;
                 else w = second;
             }
@@ -223,7 +224,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                 });
                 return slot1;
             };
-            const bool next_active = tile_base + kScatterBlock + threadIdx.x < n_points && tiles_per_group > 1;
+            const bool next_active = tile_base + kThreads + threadIdx.x < n_points && tiles_per_group > 1;
             mode = scatter_mode_decide<D>(state, bins, active, slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
         }
         fvec<D + 1> a0 = w * g0, a1 = w * g1;  // g_f * (b_r * w_level), :405-410
@@ -253,15 +254,15 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
 #define PENC_TABLE_ARGUMENTS                                                                                                        \
     n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
         random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
-template <int D, bool kRowMajor, bool kSecond, bool kWideBins>
-__global__ void __launch_bounds__(kScatterBlock, scatter_waves_per_simd(D, kSecond, kWideBins))
+template <int D, bool kRowMajor, bool kSecond, bool kWideBins, int kThreads>
+__global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kSecond, kWideBins, kThreads))
 backward_table_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
-template <int D, bool kRowMajor, bool kWideBins>
-__global__ void __launch_bounds__(kScatterBlock, both_orders_waves_per_simd(D, kWideBins))
+template <int D, bool kRowMajor, bool kWideBins, int kThreads>
+__global__ void __launch_bounds__(kThreads, both_orders_waves_per_simd(D, kWideBins, kThreads))
 backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
 #undef PENC_TABLE_PARAMETERS
 #undef PENC_TABLE_ARGUMENTS
@@ -541,15 +542,19 @@ template void launch_group_sort<PENC_DIM>(const TableLaunch& t, const GroupSort&
 
 template <int D>
 void launch_table_backward(const TableLaunch& t) {
+    // (a group of points is the same for both: half the tiles of twice the points)
+    const int tiles = t.threads > kScatterBlock ? t.tiles_per_group / 2 : t.tiles_per_group;
 #define PENC_LAUNCH(...)                                                                                                              \
-    hipLaunchKernelGGL((__VA_ARGS__), t.grid, dim3(kScatterBlock), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,            \
-                       t.feat_pairs, t.dies, t.tiles_per_group, t.capacity, t.cap_mask, t.positions, t.scale_factor, t.random_shift,  \
+    hipLaunchKernelGGL((__VA_ARGS__), t.grid, dim3(t.threads), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,                \
+                       t.feat_pairs, t.dies, tiles, t.capacity, t.cap_mask, t.positions, t.scale_factor, t.random_shift,  \
                        t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad, t.table_grad, t.grad_level_major, t.bins)
 #define PENC_LAUNCH_WIDTH(KERNEL, ...)           \
-    if (t.wide_bins) {                           \
-        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, true>);   \
-    } else {                                     \
-        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false>);  \
+    if (t.wide_bins) {                                                      \
+        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, true, kScatterBlockManyBins>);   \
+    } else if (t.threads > kScatterBlock) {                                 \
+        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false, kScatterBlockManyBins>);  \
+    } else {                                                                \
+        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false, kScatterBlock>);          \
     }
     if (t.second_grad != nullptr) {
         if (t.rows) {

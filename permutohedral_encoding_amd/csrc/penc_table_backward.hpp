@@ -14,7 +14,8 @@ struct TableLaunch {
     bool wide_bins;
     int n_points, first_level;
     uint32_t n_pass_levels, feat_pairs, dies;
-    int tiles_per_group;
+    int tiles_per_group;  // of kScatterBlock points; even
+    int threads;          // of a workgroup: kScatterBlock or kScatterBlockManyBins
     uint32_t capacity, cap_mask;
     const float *positions, *scale_factor, *random_shift, *window, *grad;
     int64_t grad_row_stride;
