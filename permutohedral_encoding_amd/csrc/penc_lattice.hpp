@@ -272,6 +272,31 @@ __device__ __forceinline__ void sort_by_rank_lds(uint2* column, uint32_t stride,
     });
 }
 
+// The same with the thread's cells two by two in 16-byte entries `stride` entries apart.
+template <int D>
+__device__ __forceinline__ void sort_by_rank_entries(uint2* entry, uint32_t stride, ivec<D + 1> rank, fvec<D + 1> delta, uint32_t hash0,
+                                                     fvec<D + 1>& sorted, uvec<D + 1>& hashes) {
+    static_for<D + 1>(PENC_BODY(c) {
+        PENC_INDEX(c);
+        const float d = delta[c];
+        uint2 cell;
+        cell.x = __builtin_bit_cast(uint32_t, d);
+        cell.y = hash_step<D, c>();
+        const uint32_t row = static_cast<uint32_t>(rank[c] < 0 ? 0 : (rank[c] > D ? D : rank[c]));  // (as in sort_by_rank_lds)
+        entry[row * stride - (row & 1u) * (stride - 1u)] = cell;
+    });
+    uvec<D + 1> step;
+    static_for<D + 1>(PENC_BODY(m) {
+        PENC_INDEX(m);
+        const uint2 cell = entry[(m >> 1) * 2 * stride + (m & 1)];
+        sorted[m] = __builtin_bit_cast(float, cell.x);
+        step[m] = cell.y;
+    });
+    hashes[0] = hash0;
+    static_for<D>(PENC_BODY(r) {
+        PENC_INDEX(r); hashes[r + 1] = hashes[r] + step[D - r]; });
+}
+
 // The same through columns of four-byte cells, half the LDS, one kind of value at a time.
 template <int D>
 __device__ __forceinline__ uint32_t rank_row(ivec<D + 1> rank, int c) {

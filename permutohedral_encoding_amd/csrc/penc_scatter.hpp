@@ -65,8 +65,8 @@ constexpr int kColumnMinIdsLog2 = 5;   // column mode: the cache's kCacheLines c
 constexpr int kColumnMaxIdsLog2 = PENC_COLUMN_MAX_IDS_LOG2;   // ... up to 128 columns of 16 cells, by the number of distinct slots the first tile has shown
 constexpr int kColumnProbes = 16;      // entries a contribution looks at before it gives up on a column
 enum ScatterMode : int { kModeCache = 0, kModeStream = 1, kModeColumns = 2 };
-// vertices per thread a wave sorts by bin in one go (256 or 320 records): all D+1 of them up to D = 4
-constexpr int stage_chunk(int pos_dim) { return pos_dim + 1 <= 4 ? 4 : 5; }
+// vertices per thread a wave sorts by bin in one go (256 to 384 records): all D+1 of them up to D = 5
+constexpr int stage_chunk(int pos_dim) { return pos_dim + 1 <= 4 ? 4 : (pos_dim == 5 ? 6 : 5); }
 constexpr int kStageBins = 64;         // a wave counts one bin per lane: staging needs n_bins <= 64
 constexpr int kWorkgroupSortMaxDim = 5;  // up to this input dimension a streaming workgroup sorts a tile's records across all its waves
 constexpr int kBinSlotsLog2 = 13;      // slots per bin: 8192 (128 KiB of fp64 sums in LDS)
@@ -665,8 +665,8 @@ __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& leve
 
 // The same sort with every wave on its own (no barriers), for the higher dimensions: their D+1
 // vertices take two chunks, the waves of a workgroup drift apart over their longer tiles, and
-// waiting for each other three times per chunk then costs more than the longer runs save
-// (measured: 5-7% slower at D = 6, 7, 8; D = 5, whose second chunk is a single vertex, still gains 4%).
+// waiting for each other in every chunk then costs more than the longer runs save
+// (measured: 5-7% slower at D = 6, 7, 8).
 // The staging space is a 4 or 5 KiB slice per wave.  For stage_chunk(D) vertices per thread at a time, the wave
 // counts its records per bin (one LDS counter per bin, owned by one lane), reserves room for each
 // bin's run in the workgroup's segment with one add per bin, lays the records out bin by bin in

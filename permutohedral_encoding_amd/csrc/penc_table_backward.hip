@@ -15,14 +15,14 @@ namespace penc {
 // Wavefronts per SIMD the scattering kernel is compiled for: six (three workgroups per compute unit, at
 // most 80 vector registers) where that costs a few spilled registers at most, else four (two
 // workgroups, 128 registers).  Measured at 2^19 points, 24 levels: table backward 0.367 -> 0.338 ms
-// at D = 4 (84 -> 80 registers, 3 spilled), 0.458 -> 0.424 ms at D = 5; the second-order kernel
-// 0.577 -> 0.552 ms at D = 4, but 0.735 -> 0.754 ms at D = 5 (11 spilled), which therefore stays at
-// four; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
-// unit: held to 128, 1.334 -> 1.113 ms.
+// at D = 4 (84 -> 80 registers, 3 spilled); the second-order kernel
+// 0.577 -> 0.552 ms at D = 4; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
+// unit: held to 128, 1.334 -> 1.113 ms.  At D = 5 two workgroups whose staging space takes all six vertices of a point are better than three
+// that sort a tile in two chunks (16 levels of 2^18 slots, 2^19 points, scatter and reduction 323 -> 314 us, second order 327 -> 315).
 constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins, int threads) {
     if (threads > kScatterBlock) return 4;  // (one workgroup per compute unit)
     if (wide_bins) return pos_dim <= 3 ? 6 : 4;  // (a variable bin width takes six to eight more registers: up to 30 spilled at D = 4)
-    return pos_dim <= 4 || (pos_dim == 5 && !second_order) ? 6 : 4;
+    return pos_dim <= 4 ? 6 : 4;
 }
 
 constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins, int threads) { return pos_dim <= 3 && !wide_bins && threads == kScatterBlock ? 6 : 4; }
@@ -194,6 +194,25 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                                                column, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D))) * w_level;
                 if constexpr (kBoth) w2 = second;
                 else w = second;
+            }
+        } else if (D >= 4 && mode == kModeStream) {
+            // The staging entries that a thread stores from are read by nobody else and written by others only after the tile's first
+            // barrier: until then they serve as its column.  (D = 4, 24 levels of 2^18 slots, 2^20 points, scatter and reduction 592 -> 585 us, second
+            // order 617 -> 607; with D = 3 the selects are as few as the trip through LDS.)
+            static_assert((D + 2) / 2 <= ScatterStateT<stage_chunk(D), kThreads>::kChunk, "a thread's staging entries hold its D+1 cells");
+            uint2* const entry = reinterpret_cast<uint2*>(state.val) + 2 * threadIdx.x;
+            fvec<D + 1> sorted;
+            if constexpr (kBoth) {
+                sort_by_rank_entries<D>(entry, kThreads, s.rank, s.delta, s.hash0, sorted, h);
+                w = barycentric_of_sorted<D>(sorted) * w_level;
+                sort_by_rank_entries<D>(entry, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
+                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
+            } else if constexpr (kOrder == kSecondOrder) {
+                sort_by_rank_entries<D>(entry, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
+                w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
+            } else {
+                sort_by_rank_entries<D>(entry, kThreads, s.rank, s.delta, s.hash0, sorted, h);
+                w = barycentric_of_sorted<D>(sorted) * w_level;
             }
         } else {
             h = vertex_hashes<D>(s.rank, s.hash0);
