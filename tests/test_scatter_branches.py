@@ -1,0 +1,64 @@
+"""Branches of the table gradient that depend on the size of the table or on the layout of the upstream gradient, at the sizes where they
+can go wrong."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("d,n,cap", [(3, 17 * 8192 + 777, 1 << 22), (3, 9 * 8192 + 777, 1 << 21), (2, 190001, (1 << 22) - 5), (5, 90001, 1 << 22),
+                                     (8, 60001, 1 << 22), (4, 130001, (1 << 22) + 1)])
+def test_hundreds_of_bins(d, n, cap):
+    """More than 256 bins (workgroups of 1024 threads; at 2^21 slots, 256 bins, of 512), a remainder in the last tile, bins of 2^14 slots.
+    All points of a group but its first 1024 sit in one simplex: their records crowd a few segments up to the last place, so that four
+    segments together hold more records than a reducer's registers take at a time, and the rest goes straight into the
+    gradient.  First and second order against the oracle, level by level."""
+    from helpers import assert_sum_close, gpu_input, make_encoding, random_problem, to_gpu
+    from oracle import api as orc
+    rng = np.random.default_rng(d)
+    levels = 2
+    p = random_problem(d, n, levels, 1, seed=60 + d, sigma_range=(2e-3, 1e-3))
+    crowd = (np.arange(n) % 4096) >= 1024
+    p["pos"] = np.where(crowd[:, None], (0.61 + 1e-7 * rng.standard_normal((n, d))).astype(np.float32), p["pos"])
+    sf = orc.scale_factors(d, p["sigmas"])
+    enc, _ = make_encoding(d, p["sigmas"], p["shift"])
+    inp = gpu_input(p, need_pos_grad=False)
+    inp.m_lattice_values = torch.zeros(levels, cap, 2, device="cuda")  # the table gradient does not read the table
+    tg, _ = enc.backward(inp, to_gpu(p["grad"]))
+    tg2, _ = enc.double_backward_from_positions(inp, to_gpu(p["dpos"]), to_gpu(p["grad"]))
+    for level in range(levels):
+        one = slice(level, level + 1)
+        args = (p["pos"], sf[one], p["shift"][one], p["window"][one])
+        want = orc.backward_table(*args, p["grad"][one], cap, want_abs=True)
+        assert_sum_close(tg[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"first order, level {level}")
+        want = orc.double_backward(p["pos"], np.zeros((1, cap, 2), np.float32), sf[one], p["shift"][one], p["window"][one], p["dpos"], p["grad"][one], want_abs=True)
+        assert_sum_close(tg2[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"second order, level {level}")
+
+
+@pytest.mark.parametrize("d,levels,n", [(3, 24, (1 << 20) + 5), (5, 23, (1 << 20) + 12345)])
+def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, n):
+    """Groups of eight tiles from rows, of sixteen from [L][F][N], at a size that has both, give the same sums."""
+    from helpers import make_encoding
+    from permutohedral_encoding_amd import _native
+    cap = 1 << 12
+    rng = np.random.default_rng(d)
+    _, fp = make_encoding(d, np.geomspace(1.0, 1e-4, levels).astype(np.float32), (rng.standard_normal((levels, d)) * 10).astype(np.float32))
+    pos, window = torch.rand(n, d, device="cuda"), torch.ones(levels, device="cuda")
+    rows = torch.randn(n, 2 * levels, device="cuda")
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(lib.penc_scatter_workspace_bytes(d, n, levels, cap, 0), dtype=torch.uint8, device="cuda")
+    out = []
+    for given, stride in ((rows, 2 * levels), (rows.t().contiguous(), 0), (rows.abs().t().contiguous(), 0)):
+        tg = torch.empty(levels, cap, 2, device="cuda")
+        params = (pos.data_ptr(), None, fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(), window.data_ptr(), given.data_ptr())
+        if stride:
+            rc = lib.penc_backward_rowmajor(d, 2, n, levels, cap, *params, stride, tg.data_ptr(), None, ws.data_ptr(), ws.numel(), st)
+        else:
+            rc = lib.penc_backward(d, 2, n, levels, cap, *params, tg.data_ptr(), None, ws.data_ptr(), ws.numel(), st)
+        assert rc == 0
+        out.append(tg)
+    # the weights are not negative: the third is the sum of magnitudes.  Each of up to 257 groups rounds its partial sum, and the sum it is
+    # added to, to 2^-24 of that
+    assert torch.all((out[0] - out[1]).abs() <= 2 * 2 * 257 * 2.0 ** -24 * out[2] + 1e-30)
