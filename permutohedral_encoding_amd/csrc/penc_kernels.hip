@@ -15,7 +15,7 @@
 //   small tables and small batches : a workgroup takes 64 points and all their levels, for the position
 //       gradient and for results in rows (block_backward_pos_kernel, block_rows_kernel).
 //   table backward (first order, the scattering half of the double backward, or both) : workgroups of
-//       512 threads walk groups of 2 to 16 tiles of points; neighbouring workgroups of a die take
+//       512 threads (1024 above 256 bins) walk groups of 2 to 16 tiles of points; neighbouring workgroups of a die take
 //       the same points at different levels.  The scatter itself (LDS accumulate cache, slot-range
 //       bins, direct atomics) is described in penc_scatter.hpp; small and ordinary batches are sorted
 //       by slot range instead (penc_group_sort.hpp).
@@ -537,8 +537,14 @@ adamw_step_kernel(float* __restrict__ params, const float* __restrict__ grads, f
 // cost follows what the batch touched and not the size of the table.  Within a touched range an entry
 // with a gradient of exactly 0 is left alone, as with skip_zero.  `clear` zeroes the gradients the
 // workgroup has used and the range's flags, which is what the next accumulation expects.
+// The update takes 512 threads to a range: a workgroup's time is a chain of waits, and the launch ends with the last few of them (the sizes
+// below, 128 / 256 / 512 / 1024 threads: 144 / 134 / 126 / 131 us).  Clearing alone keeps 256: it mostly finds nothing (an empty map of
+// 12288 ranges 4.7 / 7.2 / 12.9 us with 256 / 512 / 1024).
+template <bool kUpdate>
+constexpr uint32_t kTouchedBlock = kUpdate ? 512u : 256u;
+
 template <bool kUpdate, typename Vec>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kTouchedBlock<kUpdate>)
 touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, float* __restrict__ exp_avg,
                       float* __restrict__ exp_avg_sq, uint32_t capacity, uint32_t nr_feat, uint32_t n_ranges,
                       uint32_t range_shift, uint32_t* __restrict__ touched, AdamWStep a, int clear) {
@@ -554,19 +560,19 @@ touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, flo
     Vec* const g_at = reinterpret_cast<Vec*>(grads + base);
     // What a workgroup waits for is memory, first for the gradients and then for the values of those that are not zero: both are
     // fetched for kTogether entries of a thread at a time (24 levels of 2^22 slots, a third of the ranges touched, 445 MiB read and 78
-    // written: 145 us one by one, 135 with four).
+    // written: 145 us one by one, 134 with four).
     constexpr uint32_t kTogether = 4;
-    for (uint32_t first = threadIdx.x; first < n_vec; first += kTogether * kBlock) {
+    for (uint32_t first = threadIdx.x; first < n_vec; first += kTogether * kTouchedBlock<kUpdate>) {
         Vec gv[kTogether], pv[kTogether], mv[kTogether], vv[kTogether];
         bool nonzero[kTogether];
 #pragma unroll
         for (uint32_t u = 0; u < kTogether; ++u) {
-            const uint32_t i = first + u * kBlock;
+            const uint32_t i = first + u * kTouchedBlock<kUpdate>;
             gv[u] = g_at[i < n_vec ? i : first];
         }
 #pragma unroll
         for (uint32_t u = 0; u < kTogether; ++u) {
-            const uint32_t i = first + u * kBlock;
+            const uint32_t i = first + u * kTouchedBlock<kUpdate>;
             float g[kPer];
             __builtin_memcpy(g, &gv[u], sizeof(Vec));
             nonzero[u] = false;
@@ -583,7 +589,7 @@ touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, flo
         }
 #pragma unroll
         for (uint32_t u = 0; u < kTogether; ++u) {
-            const uint32_t i = first + u * kBlock;
+            const uint32_t i = first + u * kTouchedBlock<kUpdate>;
             if (!nonzero[u]) continue;
             if constexpr (kUpdate) {
                 float g[kPer], p[kPer], m[kPer], v[kPer];
@@ -2028,7 +2034,7 @@ static int launch_touched_ranges(bool update, float* params, float* grads, float
     const dim3 grid(n_ranges, static_cast<unsigned>(nr_levels));
     hipStream_t st = static_cast<hipStream_t>(stream);
 #define PENC_LAUNCH_TOUCHED(UPDATE, VEC)                                                                                   \
-    hipLaunchKernelGGL((touched_ranges_kernel<UPDATE, VEC>), grid, dim3(kBlock), 0, st, params, grads, exp_avg, exp_avg_sq, \
+    hipLaunchKernelGGL((touched_ranges_kernel<UPDATE, VEC>), grid, dim3(kTouchedBlock<UPDATE>), 0, st, params, grads, exp_avg, exp_avg_sq, \
                        static_cast<uint32_t>(capacity), static_cast<uint32_t>(nr_feat), n_ranges, shift, touched, a, clear)
     if (update && wide) PENC_LAUNCH_TOUCHED(true, float4);
     else if (update) PENC_LAUNCH_TOUCHED(true, float2);
