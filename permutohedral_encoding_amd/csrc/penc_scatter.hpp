@@ -461,7 +461,7 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 
 // Stage 2 for a whole tile once the workgroup streams (see scatter_mode_decide): the cache's LDS is
 // staging space for a counting sort of the tile's records by bin, stage_chunk(D) vertices per thread
-// at a time (2048 or 2560 records).  Every wave counts its records per bin (one LDS counter per
+// at a time (2048 to 3072 records of 512 threads).  Every wave counts its records per bin (one LDS counter per
 // bin and wave); then every wave, lane b looking after bin b, turns all waves' counts into the offsets of its own runs (a bin's run is the
 // waves' runs one after the other) and lays its records out in that order in the staging space; and then all
 // threads store the records in staging order: a wave instruction writes 64 consecutive records

@@ -31,9 +31,9 @@ constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins, int thread
 // floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
 // all levels of a group of points back to back, so that part of the rows' many reads comes from its L2, although every level only uses
 // 8 bytes of each: one L2 request per lane and level where the other layout has one per 16 lanes.  Measured at 2^20 points, 24
-// levels, D = 3 (16 tiles: the groups a die holds at a time are 6 MB of rows): 711 MiB read, the 192 MiB of rows 3.6 times, and
-// 42.9 M L2 requests, 385 us; from [level][feature][n] 220 MiB, 17.8 M, 322 us.  At 2^19 points, 16 levels, D = 8 (8 tiles, rows of 128
-// bytes) the 64 MiB of rows are read 1.7 times.
+// levels, D = 3, in groups of 16 tiles (a die holds 6 MB of rows at a time): 711 MiB read, the 192 MiB of rows 3.6 times, 42.9 M L2
+// requests, 375 us; in groups of eight 280 MiB, the rows 1.4 times, 45.2 M requests, 366 us; from [level][feature][n] 221 MiB, 17.8 M, 311 us.  At
+// 2^19 points, 16 levels, D = 8 (8 tiles, rows of 128 bytes) 328 us from rows, 316 from [level][feature][n].
 // With `grad_level_major` the kernel also leaves the values it read in [level][feature][n] order
 // (for the position-gradient kernel, which gathers level by level and wants its upstream gradient
 // coalesced): the layout change rides on reads this kernel makes anyway.

@@ -79,7 +79,7 @@ def is_ours(kernel):
 def order_of_table_gradient(kernel):
     """Phase of a kernel that makes records of a table gradient, None for any other kernel."""
     args = template_args(kernel)
-    if base_name(kernel) == "backward_table_kernel":  # <D, kRowMajor, kSecondOrder, kWideBins>
+    if base_name(kernel) == "backward_table_kernel":  # <D, kRowMajor, kSecondOrder, kWideBins, kThreads>
         return "double_backward" if len(args) >= 3 and args[2] == "true" else "backward"
     if base_name(kernel) == "group_sort_kernel":      # <D, kRowMajor, kOrder>: first, second, both
         return "double_backward" if len(args) >= 3 and args[2] == "2" else "backward"
@@ -169,7 +169,7 @@ def summarise(wl, digest, commit):
     flag = " --sparse-table-grad" if variant == "sparse" else ""
     with open(os.path.join(PROFILES, f"{wl}_kernel_trace.md"), "w") as f:
         f.write(f"# Kernel trace: bench.py, workload {wl_name}{' with the sparse table gradient' if flag else ''} ({DESCRIPTION[wl_name]}), one MI355X\n\n")
-        f.write("Command (from the repository root on the GPU box, after `cd /tmp && export TMPDIR=/tmp && cd -`):\n\n")
+        f.write("Command (from the repository root, after `cd /tmp && export TMPDIR=/tmp && cd -`):\n\n")
         f.write(f"    rocprofv3 --kernel-trace --stats -f csv -d gpurun_out/prof_{wl}/trace -o run -- python3 bench.py --workload {wl_name}{flag} --no-cpu --no-probes --no-module --steps 20 --warmup 5\n\n")
         f.write(f"Per phase of bench.py and kernel, over the run's dispatches (5 warm-up + 20 timed steps); kernel sources {digest} (commit {commit}):\n\n")
         f.write("| phase | kernel | calls | average (us) | min (us) | max (us) |\n|---|---|---|---|---|---|\n")
@@ -205,7 +205,7 @@ def summarise(wl, digest, commit):
         }
     with open(os.path.join(PROFILES, f"{wl}_counters.md"), "w") as f:
         f.write(f"# Hardware counters per dispatch: bench.py, workload {wl} ({DESCRIPTION[wl]}), one MI355X\n\n")
-        f.write("One rocprofv3 run per counter set (from the repository root on the GPU box):\n\n")
+        f.write("One rocprofv3 run per counter set (from the repository root):\n\n")
         for name, extra, ctrs in COUNTER_SETS:
             if sets[name]:
                 f.write(f"    rocprofv3 --pmc {ctrs} -f csv -d gpurun_out/prof_{wl}/{name} -o run -- python3 bench.py --workload {wl} --no-cpu --no-module{extra} --steps 3 --warmup 1\n")
