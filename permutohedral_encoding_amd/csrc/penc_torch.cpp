@@ -20,6 +20,8 @@
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
@@ -39,6 +41,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_set>
 #include <utility>
 #include <vector>
 
@@ -259,30 +262,60 @@ struct ExpectedVersion {
 // The slopes of the encoded features (penc_forward_slopes), kept from the forward to the passes that differentiate w.r.t. the positions,
 // as autograd keeps the tensors a node saves: freed with the graph.  What they were computed from must still be what a gathering kernel
 // would read then; where it is not (a table stepped between forward and backward, a pass on another stream), that kernel runs.
-// Their memory is bounded: all slopes alive on a device together take at most a sixteenth of its memory, beyond which
-// forwards leave none.
+// (A write that the version counter does not see, such as one through `.data`, is not noticed: modules.py says what to do after one.)
+// A forward that nothing differentiates w.r.t. the positions in the end has written them for nothing (penc_slopes.hpp has the times).
+// Nobody pays for them with an allocation that fails: a forward takes its result first and does without slopes where they do not fit, all
+// that are alive on a device take at most a sixteenth of the memory the process may use there, and they are given back when that
+// memory runs short (GiveBackSlopes).
 struct Slopes {
     static constexpr int kMaxDevices = 64;
     static std::atomic<int64_t> held[kMaxDevices];
 
-    Tensor values;
     ExpectedVersion inputs[5];
     void* stream;
     int device = -1;
-    int64_t reserved = 0;
+    int64_t reserved = 0;  // counted in held[device]
 
     Slopes() = default;
     Slopes(const Slopes&) = delete;
     Slopes& operator=(const Slopes&) = delete;
     ~Slopes() {
+        {
+            std::lock_guard<std::mutex> lock(mutex);
+            alive.erase(this);
+        }
         if (reserved != 0) held[device] -= reserved;
     }
-    bool usable(const Call& c) const {
-        return current_stream(c.device()) == stream && std::all_of(std::begin(inputs), std::end(inputs), [](const ExpectedVersion& v) { return v.holds(); });
+    // The slopes, or an undefined tensor where they do not stand for what a gathering kernel would read, or have been given back.
+    Tensor usable(const Call& c) const {
+        if (current_stream(c.device()) != stream || !std::all_of(std::begin(inputs), std::end(inputs), [](const ExpectedVersion& v) { return v.holds(); })) return {};
+        std::lock_guard<std::mutex> lock(mutex);
+        return values;
     }
-    const float* data() const { return static_cast<const float*>(values.const_data_ptr()); }
+    // For the forward that has just filled them.
+    void keep(Tensor filled) {
+        std::lock_guard<std::mutex> lock(mutex);
+        values = std::move(filled);
+        alive.insert(this);
+    }
 
-    // For the forward that is about to run; null where none are kept.  (With hooks on what a graph saves, such as those of
+    // What this process may use of a device's memory, and what of that is still to be had from the driver.
+    static int64_t most_memory(int device) {
+        return static_cast<int64_t>(static_cast<double>(at::cuda::getDeviceProperties(device)->totalGlobalMem) *
+                                    c10::hip::HIPCachingAllocator::getMemoryFraction(static_cast<c10::DeviceIndex>(device)));
+    }
+    static int64_t memory_left(int device) {  // (of the current device)
+        size_t free = 0, total = 0;
+        {
+            c10::hip::HIPStreamCaptureModeGuard in_a_capture_too{hipStreamCaptureModeRelaxed};
+            C10_HIP_CHECK(hipMemGetInfo(&free, &total));
+        }
+        const auto stats = c10::hip::HIPCachingAllocator::getDeviceStats(static_cast<c10::DeviceIndex>(device));
+        const int64_t taken = stats.reserved_bytes[static_cast<size_t>(c10::CachingAllocator::StatType::AGGREGATE)].current;
+        return std::min(static_cast<int64_t>(free), most_memory(device) - taken);
+    }
+
+    // For the forward that is about to run: null where none are kept.  (With hooks on what a graph saves, such as those of
     // checkpointing, which trade memory for a second computation, nothing beside what they see is kept.)
     static std::shared_ptr<Slopes> make(const Call& c) {
         if (!c.want_positions || c.columns() > 255 || c.levels_per_pass < 0) return nullptr;
@@ -294,50 +327,100 @@ struct Slopes {
         if (at::SavedTensorDefaultHooks::get_hooks().has_value()) return nullptr;
         const int device = c.device().index();
         if (device < 0 || device >= kMaxDevices) return nullptr;
-        const int64_t most = static_cast<int64_t>(at::cuda::getDeviceProperties(device)->totalGlobalMem / 16);
-        auto kept = std::make_shared<Slopes>();
-        kept->device = device;
+        const int64_t most = most_memory(device) / 16;
         if (held[device].fetch_add(want) + want > most) {
             held[device] -= want;
             return nullptr;
         }
-        kept->reserved = want;
-        try {
-            kept->values = at::empty({want / 4}, c.positions.options().dtype(at::kFloat));
-        } catch (const c10::OutOfMemoryError&) {
-            return nullptr;
-        }
-        kept->stream = current_stream(c.device());
-        for (size_t i = 0; i < std::size(from); ++i) kept->inputs[i].expect(*from[i]);
-        return kept;
+        auto slopes = std::make_shared<Slopes>();
+        slopes->device = device;
+        slopes->reserved = want;
+        slopes->stream = current_stream(c.device());
+        for (size_t i = 0; i < std::size(from); ++i) slopes->inputs[i].expect(*from[i]);
+        return slopes;
     }
+
+    // Gives back the slopes of a device that no running pass reads.  The memory itself is freed after the lock has been left: a thread that
+    // holds the lock must not wait for the allocator's, which the caller of GiveBackSlopes holds.
+    static bool give_back(int device) {
+        std::vector<Tensor> freed;
+        {
+            std::lock_guard<std::mutex> lock(mutex);
+            for (auto it = alive.begin(); it != alive.end();) {
+                Slopes* const s = *it;
+                if (s->device != device) {
+                    ++it;
+                    continue;
+                }
+                freed.push_back(std::move(s->values));
+                s->values = Tensor();
+                held[device] -= s->reserved;
+                s->reserved = 0;
+                it = alive.erase(it);
+            }
+        }
+        return !freed.empty();
+    }
+
+private:
+    static std::mutex mutex;                    // of `values` and `alive`; nothing is allocated or freed on a device under it
+    static std::unordered_set<Slopes*>& alive;  // those with values (never destroyed: a node may outlive the statics of this file)
+    Tensor values;
 };
 std::atomic<int64_t> Slopes::held[Slopes::kMaxDevices] = {};
+std::mutex Slopes::mutex;
+std::unordered_set<Slopes*>& Slopes::alive = *new std::unordered_set<Slopes*>();
+
+// What the caching allocator asks for memory, on the thread that allocates and with that device current, before it turns to the driver.  It
+// does not say how much it needs: slopes are given back as soon as the driver has less than a quarter of the process's memory left, so that
+// any smaller request finds what it would find without them.  (Once a program's blocks are all cached the allocator does not come here.)
+class GiveBackSlopes : public c10::FreeMemoryCallback {
+public:
+    bool Execute() override {
+        try {
+            const int device = c10::hip::current_device();
+            if (device < 0 || device >= Slopes::kMaxDevices || Slopes::held[device] == 0) return false;
+            if (Slopes::memory_left(device) >= Slopes::most_memory(device) / 4) return false;
+            return Slopes::give_back(device);
+        } catch (const std::exception&) {
+            return false;  // (the allocation goes on as it would)
+        }
+    }
+};
 
 // ------------------------------------------------------------------------------------------
 // the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
 
-Tensor compute_forward(const Call& c, const Slopes* slopes) {
+// With `slopes` the forward leaves them behind; where their memory is refused, it is reset and the forward is the one without.
+Tensor compute_forward(const Call& c, std::shared_ptr<Slopes>& slopes) {
     void* const stream = current_stream(c.device());
+    const bool as_rows = c.rows_output && c.table_format == 0 && c.columns() <= 255;
+    Tensor out = as_rows ? at::empty({c.n, c.columns()}, c.positions.options()) : level_major_array(c);
     if (slopes != nullptr) {
-        Tensor out = level_major_array(c), rows;
-        if (c.rows_output && c.table_format == 0) rows = at::empty({c.n, c.columns()}, c.positions.options());
-        check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
-                                 data(c.scale_factor), data(c.shift), data(c.window), mutable_data(out), mutable_data(rows), c.columns(),
-                                 mutable_data(slopes->values), c.concat, c.scaling, stream),
-              "forward_slopes");
-        return rows.defined() ? rows : out;
+        Tensor level_major = out, kept;
+        try {
+            if (as_rows) level_major = level_major_array(c);
+            kept = at::empty({slopes->reserved / 4}, c.positions.options().dtype(at::kFloat));
+        } catch (const c10::OutOfMemoryError&) {
+            slopes.reset();
+        }
+        if (slopes != nullptr) {
+            check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                                     data(c.scale_factor), data(c.shift), data(c.window), mutable_data(level_major),
+                                     as_rows ? mutable_data(out) : nullptr, c.columns(), mutable_data(kept), c.concat, c.scaling, stream),
+                  "forward_slopes");
+            slopes->keep(std::move(kept));
+            return out;
+        }
     }
-    if (c.rows_output && c.table_format == 0 && c.columns() <= 255) {
-        Tensor rows = at::empty({c.n, c.columns()}, c.positions.options());
+    if (as_rows) {
         const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
         check(api.forward_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
-                                   data(c.shift), data(c.window), mutable_data(rows), c.columns(), c.concat, c.scaling,
+                                   data(c.shift), data(c.window), mutable_data(out), c.columns(), c.concat, c.scaling,
                                    workspace_of(ws), workspace_size(ws), stream),
               "forward_rowmajor");
-        return rows;
+        return out;
     }
-    Tensor out = level_major_array(c);
     if (c.table_format != 0)
         check(api.forward_half(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
                                data(c.scale_factor), data(c.shift), data(c.window), mutable_data(out), c.concat, c.scaling, stream),
@@ -417,13 +500,13 @@ Tensor checked_double_positions_grad(const Call& c, const Tensor& double_positio
 // The position gradient alone, from the slopes where the forward has kept them.  With `keep_copy`, of rows the level-major copy outlives
 // the call and takes their place: a scatter that follows, and the double backward's, reads it coalesced, where rows cost it a sixth
 // of its time.
-Tensor compute_positions_backward(const Call& c, Upstream& up, const Slopes* slopes, bool keep_copy) {
+Tensor compute_positions_backward(const Call& c, Upstream& up, const Tensor& slopes, bool keep_copy) {
     Tensor positions = at::empty({c.n, c.pos_dim}, c.positions.options());
     void* const stream = current_stream(c.device());
     Tensor level_major;
     if (up.row_stride != 0 && keep_copy) level_major = level_major_array(c);
-    if (slopes != nullptr) {
-        check(api.backward_positions_slopes(c.pos_dim, c.feat, c.n, c.levels, slopes->data(), data(c.window), data(up.values), up.row_stride,
+    if (slopes.defined()) {
+        check(api.backward_positions_slopes(c.pos_dim, c.feat, c.n, c.levels, data(slopes), data(c.window), data(up.values), up.row_stride,
                                             mutable_data(level_major), mutable_data(positions), stream),
               "backward_positions_slopes");
     } else {
@@ -443,9 +526,9 @@ Tensor compute_positions_backward(const Call& c, Upstream& up, const Slopes* slo
 }
 
 // The gradient w.r.t. an upstream gradient, as dense rows or in [L+E][F][N] order, from the slopes.
-Tensor compute_grad_grad(const Call& c, const Slopes& slopes, const Tensor& double_positions_grad, bool as_rows) {
+Tensor compute_grad_grad(const Call& c, const Tensor& slopes, const Tensor& double_positions_grad, bool as_rows) {
     Tensor out = as_rows ? at::empty({c.n, c.columns()}, c.positions.options()) : level_major_array(c);
-    check(api.grad_grad_slopes(c.pos_dim, c.feat, c.n, c.levels, slopes.data(), data(c.window), data(double_positions_grad), mutable_data(out),
+    check(api.grad_grad_slopes(c.pos_dim, c.feat, c.n, c.levels, data(slopes), data(c.window), data(double_positions_grad), mutable_data(out),
                                as_rows ? c.columns() : 0, c.concat, current_stream(c.device())),
           "grad_grad_slopes");
     return out;
@@ -549,9 +632,9 @@ struct EncodeNode : public Node {
         released = true;
         slopes.reset();
     }
-    std::shared_ptr<const Slopes> usable_slopes() {
+    std::shared_ptr<const Slopes> kept_slopes() {
         std::lock_guard<std::mutex> lock(mutex_);
-        return slopes != nullptr && slopes->usable(*call) ? slopes : nullptr;
+        return slopes;
     }
     void check_saved() {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -602,12 +685,12 @@ struct EncodeBackNode : public Node {
         if (grads.size() < 2 || !grads[1].defined()) return out;
         refuse_tangents(grads);
         Tensor saved;
-        std::shared_ptr<const Slopes> kept;
+        Tensor kept;  // held until what reads it has been launched
         {
             std::lock_guard<std::mutex> lock(mutex_);
             saved = upstream.unpack();
             rows_version.check("the upstream gradient");
-            if (slopes != nullptr && slopes->usable(*call)) kept = slopes;
+            if (slopes != nullptr) kept = slopes->usable(*call);
         }
         const Call& c = *call;
         const bool grad_mode = c10::GradMode::is_enabled();
@@ -624,7 +707,7 @@ struct EncodeBackNode : public Node {
         bool want_upstream = task_should_compute_output(0);
         if (want_upstream) {
             const bool as_rows = goes_into_row_major_leaf(next_edge(0)) && c.columns() <= 255;
-            if (kept != nullptr) out[0] = compute_grad_grad(c, *kept, checked_double_positions_grad(c, grads[1]), as_rows);
+            if (kept.defined()) out[0] = compute_grad_grad(c, kept, checked_double_positions_grad(c, grads[1]), as_rows);
             else if (as_rows) out[0] = compute_grad_grad_rows(c, checked_double_positions_grad(c, grads[1]));
             want_upstream = !out[0].defined();
         }
@@ -650,21 +733,22 @@ variable_list EncodeNode::apply(variable_list&& grads) {
     Upstream up;
     Gradients g;
     ExpectedVersion rows_version;
-    std::shared_ptr<const Slopes> kept;
+    std::shared_ptr<const Slopes> slopes_kept;
     {
         at::NoGradGuard no_grad;
         const c10::DeviceGuard device(c.device());
-        if (want_positions) kept = usable_slopes();
+        Tensor kept;  // held until what reads it has been launched
+        if (want_positions && (slopes_kept = kept_slopes()) != nullptr && !(kept = slopes_kept->usable(c)).defined()) slopes_kept.reset();
         const SecondOrderTerm* fused = nullptr;
         if (first_order) {
             check_saved();
             up = upstream_of(c, grads[0].detach());
             bool gather_positions = want_positions;
             if (want_positions &&
-                (kept != nullptr || (differentiable && !want_table && up.row_stride != 0 && c.columns() <= 255))) {
+                (kept.defined() || (differentiable && !want_table && up.row_stride != 0 && c.columns() <= 255))) {
                 const bool keep_copy = differentiable || want_table;
                 if (differentiable && up.row_stride != 0 && up.values.is_alias_of(grads[0])) rows_version.expect(grads[0]);
-                g.positions = compute_positions_backward(c, up, kept.get(), keep_copy);
+                g.positions = compute_positions_backward(c, up, kept, keep_copy);
                 gather_positions = false;
             }
             if (want_table || gather_positions) {
@@ -688,7 +772,7 @@ variable_list EncodeNode::apply(variable_list&& grads) {
         back->set_next_edges(torch::autograd::collect_next_edges(grads[0], c.lattice_values));
         back->add_next_edge(torch::autograd::Edge(back->slicing, 0));
         back->call = call;
-        back->slopes = std::move(kept);
+        back->slopes = std::move(slopes_kept);
         back->upstream = torch::autograd::SavedVariable(up.values, false);
         back->rows_version = std::move(rows_version);
         torch::autograd::set_history(g.table, back);
@@ -829,7 +913,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.want_positions = grad_mode && positions.requires_grad();
         if (args[10] != Py_None && (c.want_table || c.want_positions)) c.sparse_owner = std::make_shared<PyRef>(args[10]);
         Tensor out;
-        std::shared_ptr<const Slopes> slopes;
+        std::shared_ptr<Slopes> slopes;
         {
             NoGil no_gil;
             at::NoGradGuard no_grad;
@@ -837,7 +921,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             prepare_call(c, positions, window);
             const c10::DeviceGuard device(c.device());
             slopes = Slopes::make(c);
-            out = compute_forward(c, slopes.get());
+            out = compute_forward(c, slopes);
         }
         if (c.scale_factor.device() != scale_device) {  // the module was moved: kept where the points are, so that the next call need not copy
             THPObjectPtr moved(THPVariable_Wrap(c.scale_factor));
@@ -987,4 +1071,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_penc_torch", "native autograd pat
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__penc_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__penc_torch() {
+    // (a key of its own for every copy of this library in the process: the registry ends the process over a name that it has already)
+    const std::string key = "penc_slopes " + std::to_string(reinterpret_cast<uintptr_t>(&module));
+    if (!c10::FreeHipMemoryCallbacksRegistry()->Has(key))
+        c10::FreeHipMemoryCallbacksRegistry()->Register(key, []() -> std::unique_ptr<c10::FreeMemoryCallback> { return std::make_unique<GiveBackSlopes>(); });
+    return PyModule_Create(&module);
+}

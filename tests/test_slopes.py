@@ -215,3 +215,57 @@ def test_slopes_are_freed_with_the_graph_and_travel_through_a_captured_graph(inp
         torch.cuda.synchronize()
         assert all(torch.equal(x, y) for x, y in zip(got[:4], want[:4])), replay
         assert torch.allclose(got[4], want[4], rtol=1e-4, atol=1e-6 * want[4].abs().max().item()), replay
+
+
+@pytest.fixture
+def little_memory():
+    """-> f(left): lets this process take `left` more bytes from the device (what it has cached is released first)."""
+    def limit(left):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + left) / torch.cuda.get_device_properties(0).total_memory)
+    yield limit
+    torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_slopes_are_given_back_where_memory_runs_short(inputs, little_memory):
+    """A tensor that fits only in the place of the slopes (11.6 MB) is allocated, and the passes over the graph then gather: the bits of the
+    autograd functions."""
+    pts, draw = inputs
+    native, python = modules()
+    up, q, g = draw(native)
+
+    def next_layer(m, p):
+        little_memory(16 << 20)
+        big = torch.empty(22 << 20, dtype=torch.uint8, device="cuda")  # noqa: F841
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    a, b = sdf_pass(native, pts, up, q, g, between=next_layer), sdf_pass(python, pts, up, q, g)
+    for x, y in zip(a[:4], b[:4]):
+        assert torch.equal(x, y)
+    assert keeps_slopes(native, pts)  # the next forward keeps them again
+
+
+@pytest.mark.parametrize("rows", [False, True])
+def test_a_forward_that_fits_without_slopes_does_not_fail_for_them(little_memory, rows):
+    """64 MB of result, 193 MB of slopes, and room for one of them; in rows the forward writes through an array of the result's size."""
+    n = 1 << 20
+    native, _ = modules(contiguous_output=rows)
+    pts = torch.rand(n, 3, device="cuda").requires_grad_(True)
+    with torch.no_grad():
+        want = native(pts)
+    little_memory((200 << 20) + (rows << 26))
+    out = native(pts)
+    assert torch.equal(out, want)
+
+
+def test_slopes_take_a_bounded_share_of_the_memory(inputs, little_memory):
+    """A sixteenth of what the process may use: here room for the slopes of one forward (11.6 MB), not of two."""
+    pts, _ = inputs
+    native, _ = modules()
+    torch.cuda.empty_cache()
+    little_memory((300 << 20) - torch.cuda.memory_reserved())
+    assert torch.cuda.memory_reserved() < 200 << 20  # (no shortage)
+    first = native(pts.clone().requires_grad_(True))
+    assert not keeps_slopes(native, pts)
+    del first
+    assert keeps_slopes(native, pts)
