@@ -33,6 +33,13 @@ class PermutoEncoding(torch.nn.Module):
     what was touched.  Neither the gradient calls nor the optimizer then walk the whole table (the
     reference clears a dense gradient in every call, src/Encoding.cu:141, 246, and its training
     protocol steps the whole table, examples/performance.py:99-101).
+
+    Where ``positions`` require a gradient the forward usually keeps what their derivatives need of the table
+    (4 * pos_dim * nr_feat bytes per point and level, until the graph is freed, given back when memory runs short).
+    The derivatives are then those of the forward as it was, unless the table, the points or the window
+    have been changed in place since, which is followed: they are computed from the present values.  A write that autograd's version
+    counter does not see (``lattice_values.data.add_(...)``, a kernel given the raw pointer) is not followed; between a
+    forward and its backward, ``torch.autograd.graph.increment_version(lattice_values)`` after it makes it so.
     """
 
     def __init__(self, pos_dim, capacity, nr_levels, nr_feat_per_level, scale_per_level,
