@@ -841,7 +841,7 @@ inline size_t direct_flag_bytes(int levels, uint32_t n_bins) {
 
 // log2 of the slots per bin: kBinSlotsLog2 (what a reducer workgroup's LDS holds) up to kMaxBins bins, wider
 // bins (summed one LDS-full after the other) for larger tables, up to kMaxBinSlotsLog2.
-inline uint32_t bin_shift_for_capacity(int capacity) {
+constexpr uint32_t bin_shift_for_capacity(int capacity) {
     uint32_t shift = kBinSlotsLog2;
     while (shift < static_cast<uint32_t>(kMaxBinSlotsLog2) &&
            ((static_cast<int64_t>(capacity) + (int64_t{1} << shift) - 1) >> shift) > kMaxBins)
@@ -850,10 +850,17 @@ inline uint32_t bin_shift_for_capacity(int capacity) {
 }
 
 // Bins per level; more than kMaxBins means the table is too large for binning.
-inline uint32_t bins_for_capacity(int capacity) {
+constexpr uint32_t bins_for_capacity(int capacity) {
     const uint32_t shift = bin_shift_for_capacity(capacity);
     return static_cast<uint32_t>((static_cast<int64_t>(capacity) + (int64_t{1} << shift) - 1) >> shift);
 }
+// A width is doubled only where it leaves more than kMaxBins bins, so wide bins are always more than half as many: their scatter is
+// that of many bins.
+static_assert(kMaxBins / 2 >= static_cast<int>(kFewerOpenLinesMinBins) && kFewerOpenLinesMinBins >= static_cast<uint32_t>(kStageBins),
+              "wide bins are many bins, and many bins are sorted by stream_tile_many");
+static_assert(bin_shift_for_capacity((kMaxBins << kBinSlotsLog2) + 1) > static_cast<uint32_t>(kBinSlotsLog2) &&
+                  bins_for_capacity((kMaxBins << kBinSlotsLog2) + 1) > kFewerOpenLinesMinBins,
+              "the smallest table with wide bins");
 
 constexpr int64_t kMinSlotsPerContribution = 8;
 constexpr int64_t kLargeGroupsMinWorkgroups = 3000;  // about four per workgroup slot of the chip (256 CUs x 3)
@@ -1285,7 +1292,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
         t.grid = dim3(padded_groups * static_cast<unsigned>(count));
-        t.threads = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins ? kScatterBlockManyBins : kScatterBlock;
+        t.many_bins = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins;
         t.wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
         t.first_level = first;
         t.n_pass_levels = static_cast<uint32_t>(count);

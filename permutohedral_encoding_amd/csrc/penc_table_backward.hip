@@ -561,19 +561,19 @@ template void launch_group_sort<PENC_DIM>(const TableLaunch& t, const GroupSort&
 
 template <int D>
 void launch_table_backward(const TableLaunch& t) {
-    // (a group of points is the same for both: half the tiles of twice the points)
-    const int tiles = t.threads > kScatterBlock ? t.tiles_per_group / 2 : t.tiles_per_group;
-#define PENC_LAUNCH(...)                                                                                                              \
-    hipLaunchKernelGGL((__VA_ARGS__), t.grid, dim3(t.threads), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,                \
-                       t.feat_pairs, t.dies, tiles, t.capacity, t.cap_mask, t.positions, t.scale_factor, t.random_shift,  \
-                       t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad, t.table_grad, t.grad_level_major, t.bins)
-#define PENC_LAUNCH_WIDTH(KERNEL, ...)           \
+    // (a group of points is the same for all instances: half the tiles of twice the points)
+#define PENC_LAUNCH(THREADS, ...)                                                                                                      \
+    hipLaunchKernelGGL((__VA_ARGS__, THREADS>), t.grid, dim3(THREADS), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,        \
+                       t.feat_pairs, t.dies, t.tiles_per_group / (THREADS / kScatterBlock), t.capacity, t.cap_mask, t.positions,       \
+                       t.scale_factor, t.random_shift, t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad,          \
+                       t.table_grad, t.grad_level_major, t.bins)
+#define PENC_LAUNCH_WIDTH(KERNEL, ...)                                      \
     if (t.wide_bins) {                                                      \
-        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, true, kScatterBlockManyBins>);   \
-    } else if (t.threads > kScatterBlock) {                                 \
-        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false, kScatterBlockManyBins>);  \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true);    \
+    } else if (t.many_bins) {                                               \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, false);   \
     } else {                                                                \
-        PENC_LAUNCH(KERNEL<D, __VA_ARGS__, false, kScatterBlock>);          \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, false);           \
     }
     if (t.second_grad != nullptr) {
         if (t.rows) {

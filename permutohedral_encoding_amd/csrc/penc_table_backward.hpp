@@ -11,11 +11,11 @@ struct TableLaunch {
     hipStream_t stream;
     bool rows;          // the upstream gradient is read as rows
     bool second_order;  // double_pos_grad is given; with second_grad too, both orders
-    bool wide_bins;
+    bool wide_bins;     // (only together with many_bins: the scatter of wide bins has no other instance)
+    bool many_bins;     // more than kFewerOpenLinesMinBins: workgroups of kScatterBlockManyBins threads, else of kScatterBlock
     int n_points, first_level;
     uint32_t n_pass_levels, feat_pairs, dies;
     int tiles_per_group;  // of kScatterBlock points; even
-    int threads;          // of a workgroup: kScatterBlock or kScatterBlockManyBins
     uint32_t capacity, cap_mask;
     const float *positions, *scale_factor, *random_shift, *window, *grad;
     int64_t grad_row_stride;

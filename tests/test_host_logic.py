@@ -77,6 +77,8 @@ def test_argument_validation_without_a_gpu():
     assert lib.penc_double_backward_from_positions_sparse(3, 2, 10, 2, 16, p, p, p, p, p, p, p, 3, p, p, p, 0, None, 0, None) == 2  # odd row stride
     assert lib.penc_touched_map_entries(2, 24, 1 << 18) == 24 * 32 and lib.penc_touched_range_slots(1 << 18) == 8192
     assert lib.penc_touched_map_entries(8, 3, 1 << 22) == 3 * 4 * 512 and lib.penc_touched_range_slots(1 << 22) == 8192
+    for capacity in [(1 << k) + extra for k in (22, 23, 24) for extra in (1, 8191, 8192, 8193)]:  # wide ranges: always hundreds of them
+        assert 256 < lib.penc_touched_map_entries(2, 1, capacity) <= 512 and lib.penc_touched_range_slots(capacity) > 8192
     assert lib.penc_touched_map_entries(2, 1, 1 << 24) == 512 and lib.penc_touched_range_slots(1 << 24) == 1 << 15
     assert lib.penc_touched_map_entries(2, 5, 100003) == 5 * 13 and lib.penc_touched_map_entries(3, 5, 100) == 0
     assert lib.penc_adamw_step_sparse(p, p, p, p, 2, 2, 16, z, 1e-3, 0.9, 0.99, 1e-8, 0.0, 1, 1, None) == 1
