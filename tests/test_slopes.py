@@ -1,5 +1,7 @@
 """Position derivatives from the slopes a forward keeps (penc_forward_slopes and what reads them), against fp64 sums over the
 oracle's simplices, and the module's rules for keeping them."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -229,6 +231,12 @@ def test_slopes_are_freed_with_the_graph_and_travel_through_a_captured_graph(inp
 @pytest.fixture
 def little_memory():
     """-> f(left): lets this process take `left` more bytes from the device (what it has cached is released first)."""
+    # (large blocks that earlier tests have left in the cache go too: what the test itself allocates would be cut from them, and what is left
+    # of such a block serves requests that are meant to find no memory)
+    gc.collect()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+
     def limit(left):
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
