@@ -658,8 +658,11 @@ __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& leve
             if (!all_fit && __any(spill))
                 global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
         });
-        // the next chunk (or tile) counts into counters this chunk has cleared, overwrites offset/dest after its
-        // first two barriers and the staging array after its third: nothing is overwritten while still read
+        // The next chunk (or tile) counts into counters this chunk has cleared, overwrites offset/dest after its
+        // first two barriers and what other threads read of the staging array after its third.  The entries a thread has stored
+        // from are its own before that (sort_by_rank_entries in the next tile writes them without a barrier): the fence
+        // keeps those writes behind the reads above.
+        wave_lds_fence();
     });
 }
 

@@ -32,6 +32,39 @@ def assert_sum_close(got, want64, abs64, rel=1e-4, what=""):
     assert worst <= 1.0, f"{what}: max err/bound = {worst:.3g} (rel {rel} of sum|terms|)"
 
 
+def scatter_plan(pos_dim, n, levels, capacity):
+    """How the scatter of a dense level-major gradient of two features is cut up: (points of a group, number of groups, bins, places in a
+    segment).  The rules of penc_kernels.hip (table_backward_tiles, bins_for_capacity, wanted_segment_capacity), so that a test can say
+    that its sizes reach the branch it is about; checked against the workspace the library asks for."""
+    from permutohedral_encoding_amd import _native
+
+    def groups(tiles):
+        return -(-n // (512 * tiles))
+
+    shift = 13
+    while -(-capacity >> shift) > 512:
+        shift += 1
+    bins = -(-capacity >> shift)
+    split = pos_dim <= 5 and bins <= 64
+
+    def places(tiles):
+        mean = (512 * tiles * (pos_dim + 1) + 2048) / bins
+        want = int(mean + 3.0 * mean ** 0.5 + 8.0)
+        return (want + 3) // 4 * 4 if split else want
+
+    if groups(16) * levels >= 3000:
+        tiles = 16
+    else:
+        tiles = 8
+        while tiles > 2 and groups(tiles) * levels < 768:
+            tiles //= 2
+    assert levels * n * (pos_dim + 1) > 6 << 20, "the sorted groups may take such a batch"
+    per_level = max(bins * groups(t) * (4 + places(t) * (10 if split else 12)) for t in (8, tiles))
+    want = per_level * levels + (levels * bins * 4 + 255) // 256 * 256 + 1024
+    assert _native.lib().penc_scatter_workspace_bytes(pos_dim, n, levels, capacity, levels) == want, "the library cuts the scatter up differently"
+    return 512 * tiles, groups(tiles), bins, places(tiles)
+
+
 # ----------------------------------------------------------------------------- GPU side
 
 def make_encoding(pos_dim, sigmas, shift, concat_points=False, points_scaling=1.0, device="cuda", nr_feat=2):

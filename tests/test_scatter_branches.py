@@ -8,19 +8,26 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-@pytest.mark.parametrize("d,n,cap", [(3, 17 * 8192 + 777, 1 << 22), (3, 9 * 8192 + 777, 1 << 21), (2, 190001, (1 << 22) - 5), (5, 90001, 1 << 22),
-                                     (8, 60001, 1 << 22), (4, 130001, (1 << 22) + 1)])
+@pytest.mark.parametrize("d,n,cap", [(3, 17 * 8192 + 777, 1 << 22), (3, 17 * 8192 + 777, 1 << 21), (2, 140001, (1 << 22) - 5), (5, 133001, 1 << 22),
+                                     (8, 131201, 1 << 22), (4, 130001, (1 << 22) + 1), (4, 16 * 8192 + 1025, 1 << 22)])
 def test_hundreds_of_bins(d, n, cap):
     """More than 256 bins (workgroups of 1024 threads; at 2^21 slots, 256 bins, of 512), a remainder in the last tile, bins of 2^14 slots.
-    All points of a group but its first 1024 sit in one simplex: their records crowd a few segments up to the last place, so that four
-    segments together hold more records than a reducer's registers take at a time, and the rest goes straight into the
-    gradient.  First and second order against the oracle, level by level."""
-    from helpers import assert_sum_close, gpu_input, make_encoding, random_problem, to_gpu
+    A third of a group's points, behind the tile by which the workgroup decides to stream, sit in one simplex: their records crowd a few
+    segments up to the last place, so that four segments together hold more records than a reducer's registers take at a time, and the rest
+    goes straight into the gradient.  First and second order against the oracle, at the first, a middle and the last level."""
+    from helpers import assert_sum_close, gpu_input, make_encoding, random_problem, scatter_plan, to_gpu
     from oracle import api as orc
     rng = np.random.default_rng(d)
-    levels = 2
+    levels = 24
+    group, n_groups, bins, places = scatter_plan(d, n, levels, cap)
+    threads = 1024 if bins > 256 else 512
+    at = np.arange(n) % group
+    crowd = (at >= group // 2) & (at < group // 2 + 1024)
+    # several tiles, the crowded ones not the first; their records do not fit the segments; those of a wave's four are more than six
+    # (up to 64 places: three) to a lane
+    assert group == 4096 and group >= 4 * threads and 1024 > places and places <= 128 and n_groups >= 32
+    assert 4 * places > 64 * (3 if places <= 64 else 6) or (d, cap) in [(5, 1 << 22), (4, 1 << 22)]
     p = random_problem(d, n, levels, 1, seed=60 + d, sigma_range=(2e-3, 1e-3))
-    crowd = (np.arange(n) % 4096) >= 1024
     p["pos"] = np.where(crowd[:, None], (0.61 + 1e-7 * rng.standard_normal((n, d))).astype(np.float32), p["pos"])
     sf = orc.scale_factors(d, p["sigmas"])
     enc, _ = make_encoding(d, p["sigmas"], p["shift"])
@@ -28,7 +35,7 @@ def test_hundreds_of_bins(d, n, cap):
     inp.m_lattice_values = torch.zeros(levels, cap, 2, device="cuda")  # the table gradient does not read the table
     tg, _ = enc.backward(inp, to_gpu(p["grad"]))
     tg2, _ = enc.double_backward_from_positions(inp, to_gpu(p["dpos"]), to_gpu(p["grad"]))
-    for level in range(levels):
+    for level in (0, 11, levels - 1):
         one = slice(level, level + 1)
         args = (p["pos"], sf[one], p["shift"][one], p["window"][one])
         want = orc.backward_table(*args, p["grad"][one], cap, want_abs=True)
