@@ -31,10 +31,10 @@ def exact_slopes(p, sf, capacity):
 
 
 @pytest.mark.parametrize("d,n,levels,cap,feat,concat,fmt", [(3, 1, 5, 64, 2, True, 0), (2, 63, 9, 1 << 10, 4, True, 0), (3, 64, 24, 1 << 18, 2, False, 0),
-                                                            (4, 65, 8, 1000, 8, False, 0), (8, 1003, 15, 1 << 10, 8, False, 0), (5, 20001, 7, 1 << 12, 2, True, 0),
+                                                            (4, 65, 8, 1000, 8, False, 0), (8, 1003, 31, 1 << 10, 8, False, 0), (5, 20001, 7, 1 << 12, 2, True, 0),
                                                             (6, 4097, 3, 1 << 12, 4, True, 0), (7, 777, 8, 1 << 14, 2, False, 1), (3, 5000, 17, 1 << 14, 2, True, 2)])
 def test_derivatives_from_slopes(d, n, levels, cap, feat, concat, fmt):
-    """One point, remainders of a tile, fewer and more levels than waves, 248 columns, a masked level, padded rows, 16-bit tables."""
+    """One point, remainders of a tile, fewer and more levels than waves, 248 columns (80 KB of LDS), a masked level, padded rows, 16-bit tables."""
     from helpers import make_encoding, random_problem, to_gpu
     from oracle import api as orc
     from permutohedral_encoding_amd import _native
