@@ -135,6 +135,7 @@ struct Call {
     Tensor scale_factor, shift, window;
     std::shared_ptr<PyRef> sparse_owner;  // the wrapper that keeps the sparse table gradient; null: dense gradients
     bool want_table, want_positions;
+    bool hooked = false;  // hooks are set on what a graph saves (looked at where slopes could be kept)
 
     int64_t columns() const { return static_cast<int64_t>(feat) * (levels + extra); }
     at::Device device() const { return positions.device(); }
@@ -315,16 +316,18 @@ struct Slopes {
         return std::min(static_cast<int64_t>(free), most_memory(device) - taken);
     }
 
-    // For the forward that is about to run: null where none are kept.  (With hooks on what a graph saves, such as those of
-    // checkpointing, which trade memory for a second computation, nothing beside what they see is kept.)
+    // Whether hooks are on what a graph saves, such as those of checkpointing, which trade memory for a second computation: nothing
+    // beside what they see is kept then.  With the GIL held: looking copies Python objects.
+    static bool hooks_are_set() { return at::SavedTensorDefaultHooks::get_hooks().has_value(); }
+
+    // For the forward that is about to run: null where none are kept.
     static std::shared_ptr<Slopes> make(const Call& c) {
-        if (!c.want_positions || c.columns() > 255 || c.levels_per_pass < 0) return nullptr;
+        if (!c.want_positions || c.hooked || c.columns() > 255 || c.levels_per_pass < 0) return nullptr;
         const int64_t want = static_cast<int64_t>(api.slopes_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, c.table_format));
         if (want == 0 || (c.max_workspace >= 0 && want > c.max_workspace)) return nullptr;
         const Tensor* const from[] = {&c.table, &c.positions, &c.window, &c.shift, &c.scale_factor};
         for (const Tensor* t : from)
             if (t->is_inference()) return nullptr;
-        if (at::SavedTensorDefaultHooks::get_hooks().has_value()) return nullptr;
         const int device = c.device().index();
         if (device < 0 || device >= kMaxDevices) return nullptr;
         const int64_t most = most_memory(device) / 16;
@@ -911,6 +914,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         const bool grad_mode = c10::GradMode::is_enabled();
         c.want_table = grad_mode && lattice_values.requires_grad();
         c.want_positions = grad_mode && positions.requires_grad();
+        if (c.want_positions) c.hooked = Slopes::hooks_are_set();
         if (args[10] != Py_None && (c.want_table || c.want_positions)) c.sparse_owner = std::make_shared<PyRef>(args[10]);
         Tensor out;
         std::shared_ptr<Slopes> slopes;

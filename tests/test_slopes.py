@@ -391,3 +391,32 @@ def test_slopes_across_streams_and_threads(inputs, where):
     assert torch.equal(out, want[0])
     for x, y in zip((normal, p.grad, u.grad, native.lattice_values.grad), want[1:]):
         close(x.detach(), y)
+
+
+def test_hooks_on_saved_tensors_are_looked_at_under_the_interpreters_lock():
+    """Forwards of several threads under the same hooks leave their reference counts as they were."""
+    import sys
+    import threading
+    native, _ = modules(levels=2, cap=1 << 18)
+    pts = torch.rand(9000, 3, device="cuda").requires_grad_(True)
+
+    def pack(t):
+        return t
+
+    def unpack(t):
+        return t
+
+    def forwards():
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            for _ in range(300):
+                native(pts)
+    before = sys.getrefcount(pack), sys.getrefcount(unpack)
+    workers = [threading.Thread(target=forwards) for _ in range(4)]
+    for w in workers:
+        w.start()
+    for w in workers:
+        w.join()
+    torch.cuda.synchronize()
+    del workers
+    gc.collect()
+    assert (sys.getrefcount(pack), sys.getrefcount(unpack)) == before
