@@ -37,6 +37,7 @@
 #include <torch/csrc/utils/object_ptr.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <memory>
 #include <mutex>
@@ -272,7 +273,22 @@ struct Slopes {
     static constexpr int kMaxDevices = 64;
     static std::atomic<int64_t> held[kMaxDevices];
 
-    ExpectedVersion inputs[5];
+    // What an input must still be: unchanged in place, and not given other memory (`lattice_values.data = ...`), which is no change in place.
+    struct Input {
+        ExpectedVersion version;
+        c10::Storage storage;  // (kept, so that no other memory can take its place)
+        int64_t offset = 0;
+
+        void expect(const Tensor& t) {
+            version.expect(t);
+            storage = t.storage();
+            offset = t.storage_offset();
+        }
+        bool holds(const Tensor& t) const {
+            return version.holds() && t.storage().unsafeGetStorageImpl() == storage.unsafeGetStorageImpl() && t.storage_offset() == offset;
+        }
+    } inputs[5];
+    static std::array<const Tensor*, 5> inputs_of(const Call& c) { return {&c.table, &c.positions, &c.window, &c.shift, &c.scale_factor}; }
     void* stream;
     int device = -1;
     int64_t reserved = 0;  // counted in held[device]
@@ -289,7 +305,10 @@ struct Slopes {
     }
     // The slopes, or an undefined tensor where they do not stand for what a gathering kernel would read, or have been given back.
     Tensor usable(const Call& c) const {
-        if (current_stream(c.device()) != stream || !std::all_of(std::begin(inputs), std::end(inputs), [](const ExpectedVersion& v) { return v.holds(); })) return {};
+        if (current_stream(c.device()) != stream) return {};
+        const auto from = inputs_of(c);
+        for (size_t i = 0; i < from.size(); ++i)
+            if (!inputs[i].holds(*from[i])) return {};
         std::lock_guard<std::mutex> lock(mutex);
         return values;
     }
@@ -325,7 +344,7 @@ struct Slopes {
         if (!c.want_positions || c.hooked || c.columns() > 255 || c.levels_per_pass < 0) return nullptr;
         const int64_t want = static_cast<int64_t>(api.slopes_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, c.table_format));
         if (want == 0 || (c.max_workspace >= 0 && want > c.max_workspace)) return nullptr;
-        const Tensor* const from[] = {&c.table, &c.positions, &c.window, &c.shift, &c.scale_factor};
+        const auto from = inputs_of(c);
         for (const Tensor* t : from)
             if (t->is_inference()) return nullptr;
         const int device = c.device().index();
@@ -339,7 +358,7 @@ struct Slopes {
         slopes->device = device;
         slopes->reserved = want;
         slopes->stream = current_stream(c.device());
-        for (size_t i = 0; i < std::size(from); ++i) slopes->inputs[i].expect(*from[i]);
+        for (size_t i = 0; i < from.size(); ++i) slopes->inputs[i].expect(*from[i]);
         return slopes;
     }
 

@@ -161,10 +161,10 @@ def test_module_keeps_slopes_and_agrees_with_the_gathering_path(inputs, kw, rows
         close(x, y)
 
 
-@pytest.mark.parametrize("what", ["table", "data", "positions", "shift", "window", "hooks", "cap"])
+@pytest.mark.parametrize("what", ["table", "data", "other_memory", "positions", "shift", "window", "hooks", "cap"])
 def test_slopes_of_changed_inputs_are_not_used(inputs, monkeypatch, what):
-    """Where an input changes in place between the passes the gathering kernels run, as in the autograd functions: the same bits.  And
-    nothing is kept beside what hooks on saved tensors see, nor over the cap on scratch memory."""
+    """Where an input changes in place, or is given other memory, between the passes the gathering kernels run, as in the autograd
+    functions: the same bits.  And nothing is kept beside what hooks on saved tensors see, nor over the cap on scratch memory."""
     from permutohedral_encoding_amd import _native
     pts, draw = inputs
     native, python = modules()
@@ -177,6 +177,8 @@ def test_slopes_of_changed_inputs_are_not_used(inputs, monkeypatch, what):
         elif what == "data":  # (the version counter does not see the write: the program says so)
             m.lattice_values.data.mul_(0.5)
             torch.autograd.graph.increment_version(m.lattice_values)
+        elif what == "other_memory":
+            m.lattice_values.data = 0.5 * m.lattice_values.data
         elif what == "positions":
             p.mul_(0.5)
         elif what == "shift":
