@@ -879,13 +879,24 @@ inline unsigned scatter_groups(int64_t n, int tiles_per_group) {
 // 0.065 -> 0.055 ms and 2^14 points 0.062 -> 0.048 ms with two; 2^17 points are best with eight).  That is for the
 // small batches that the sorted groups below do not take: few levels, sparse or mostly empty gradients, a workspace too small.
 constexpr int64_t kMinWorkgroups = 768;  // three per compute unit
-// Rows of an upstream gradient are read by every level of a group, and what a die holds of them at a time should fit its L2: four
-// groups of 16 tiles are 6 MB of rows of 48 columns.  With eight the longer segments are missed less than the rows (`short_groups`; scatter
-// and reduction, us, 16 -> 8 tiles: D = 3, 24 levels of 2^18 slots, 2^20 points 515 -> 505, 2^19 280 -> 272, 16 levels of 2^16 slots 314 -> 311; D = 4,
-// 24 levels 659 -> 649; D = 5, 16 levels 324 -> 320).  Not with two dimensions (230 -> 236), four features (317 -> 320), whose rows
-// more than one pair of features reads, or more than kStageBins bins, whose runs are short as it is (2^22 slots 1212 -> 1290).
-inline bool short_groups(int pos_dim, uint32_t feat_pairs, int capacity, bool rows) {
-    return rows && pos_dim >= 3 && feat_pairs == 1u && bins_for_capacity(capacity) <= static_cast<uint32_t>(kStageBins);
+// Rows of an upstream gradient are read by every level of a group, and what a die holds of them at a time should fit its L2: 96
+// workgroups (three to a compute unit, up to four dimensions) of 16 tiles read 6 MB of rows, however many levels those rows have.  With
+// eight tiles the longer segments are missed less than the rows.  Forward and backward of the module from rows, us, 16 -> 8 tiles, all at sizes
+// that take 16 otherwise (about 25 M points times levels):
+//   D = 3, 24 levels       2^17 slots 789 -> 764   2^18 790 -> 778   2^19 926 -> 913;  2^16 slots (8 bins, shared by reducers) 742 -> 739
+//          16 levels       2^17 826 -> 813   2^18 1072 -> 1069   2^19 915 -> 908;  2^16 slots 892 -> 907, 20 levels 1166 -> 1176
+//          few levels, which keep in step anyway   12 of 2^18 772 -> 768   10 780 -> 779;  8 1033 -> 1038   6 780 -> 788
+//   D = 4, 24 levels       2^18 1036 -> 1025   2^19 1292 -> 1288;  2^17 926 -> 929, 16 levels 1072 -> 1088, of 2^16 1238 -> 1248
+//          10 levels       2^18 1018 -> 1007;  8 1292 -> 1309
+// Not from five dimensions on, where two workgroups to a compute unit read 4 MB (D = 5, 24 levels 1294 -> 1318, 32 levels 1690 -> 1736; D = 7, 16
+// levels 2384 -> 2412; D = 8 1985 -> 1981), with two dimensions (scatter and reduction 230 -> 236), four features (317 -> 320), whose rows
+// more than one pair of features reads, or more than kStageBins bins, whose runs are short as it is (2^22 slots 1212 -> 1290).  A spectrum of
+// scales without fine levels, which the launch does not know of, has few records to gain or lose by (24 levels down to 1e-2: 552 -> 563).
+constexpr int kShortGroupsMinLevels = 10;
+inline bool short_groups(int pos_dim, uint32_t feat_pairs, int levels, int capacity, bool rows) {
+    const uint32_t bins = bins_for_capacity(capacity);
+    return rows && (pos_dim == 3 || pos_dim == 4) && feat_pairs == 1u && levels >= kShortGroupsMinLevels &&
+           bins >= (pos_dim == 3 ? 16u : 32u) && bins <= static_cast<uint32_t>(kStageBins);
 }
 inline int table_backward_tiles(int64_t n, int levels) {
     if (static_cast<int64_t>(scatter_groups(n, kScatterTilesLarge)) * levels >= kLargeGroupsMinWorkgroups) return kScatterTilesLarge;
@@ -1271,7 +1282,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         return check_launch();
     }
     int tiles_per_group = table_backward_tiles(nr_positions, pair_levels);
-    if (tiles_per_group > kScatterTiles && short_groups(pos_dim, feat_pairs, capacity, t.rows)) tiles_per_group = kScatterTiles;
+    if (tiles_per_group > kScatterTiles && short_groups(pos_dim, feat_pairs, pair_levels, capacity, t.rows)) tiles_per_group = kScatterTiles;
     BinPlan plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, workspace, workspace_bytes);
     if (!plan.enabled && tiles_per_group > kScatterTiles) {  // wide bins need short segments: smaller groups of points
         tiles_per_group = kScatterTiles;

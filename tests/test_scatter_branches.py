@@ -44,13 +44,13 @@ def test_hundreds_of_bins(d, n, cap):
         assert_sum_close(tg2[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"second order, level {level}")
 
 
-@pytest.mark.parametrize("d,levels,n", [(3, 24, (1 << 20) + 5), (5, 24, (1 << 20) + 12345)])
-def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, n):
-    """Groups of eight tiles from rows, of sixteen from [L][F][N], at a size that has both, give the same sums."""
+@pytest.mark.parametrize("d,levels,n,cap", [(3, 24, (1 << 20) + 5, 1 << 17), (4, 24, (1 << 20) + 5, 1 << 18), (5, 24, (1 << 20) + 12345, 1 << 12)])
+def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, n, cap):
+    """Groups of eight tiles from rows (of sixteen from five dimensions on), of sixteen from [L][F][N], at a size that has both, give the
+    same sums."""
     from helpers import make_encoding, scatter_plan
     from permutohedral_encoding_amd import _native
-    cap = 1 << 12
-    assert scatter_plan(d, n, levels, cap)[0] == 16 * 512  # (level-major; rows of such a size: eight)
+    assert scatter_plan(d, n, levels, cap)[0] == 16 * 512  # (level-major)
     rng = np.random.default_rng(d)
     _, fp = make_encoding(d, np.geomspace(1.0, 1e-4, levels).astype(np.float32), (rng.standard_normal((levels, d)) * 10).astype(np.float32))
     pos, window = torch.rand(n, d, device="cuda"), torch.ones(levels, device="cuda")
