@@ -304,7 +304,7 @@ bin_reduce_levels_kernel(BinTarget pass_bins, const float* __restrict__ window, 
     const uint32_t todo = masks[0], direct_mask = masks[1];
     if (todo == 0u) return;
 
-    // a step: 64 segments of one level, one per quarter wave
+    // a step: 64 segments of one level, four to a wave
     constexpr uint32_t kEnd = 32;
     // Bins wider than the LDS sums (tables above 2^22 slots) are summed one range of kBinSlots slots after
     // the other: every range walks all the bin's records and takes those that fall into it.
