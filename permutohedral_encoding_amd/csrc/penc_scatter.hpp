@@ -460,8 +460,8 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 }
 
 // Stage 2 for a whole tile once the workgroup streams (see scatter_mode_decide): the cache's LDS is
-// staging space for a counting sort of the tile's records by bin, stage_chunk(D) vertices per thread
-// at a time (2048 to 3072 records of 512 threads).  Every wave counts its records per bin (one LDS counter per
+// staging space for a counting sort of the tile's records by bin, all vertices at a time
+// (1536 to 3072 records of 512 threads).  Every wave counts its records per bin (one LDS counter per
 // bin and wave); then every wave, lane b looking after bin b, turns all waves' counts into the offsets of its own runs (a bin's run is the
 // waves' runs one after the other) and lays its records out in that order in the staging space; and then all
 // threads store the records in staging order: a wave instruction writes 64 consecutive records
@@ -472,7 +472,7 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 // 149 -> 119; D = 4, second order, 12 levels 437 -> 412; with the coarse levels beside them, which keep the vector units busy, the same.)
 // A staged record carries its destination (its index in the level's record
 // array), so the store needs no search.  When a run does not fit its segment any more (rare: the
-// segments hold the mean plus three standard deviations) the chunk checks every record against
+// segments hold the mean plus three standard deviations) the tile checks every record against
 // the room left and sends the excess to stage 3.
 // Needs bins.n_bins <= kStageBins and a level's record array below 2^32 bytes (the host plans
 // for both); all threads of the workgroup must call it together.
@@ -482,6 +482,7 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
                                             fvec<D + 1> a1, uint32_t& cursor) {
     constexpr int kWaves = State::kThreads / 64;
     constexpr int kStageChunk = State::kChunk;
+    static_assert(D + 1 <= kStageChunk, "all vertices of a tile are staged at a time");
     static_assert(kCacheLines >= 3 * kWaves * 64, "the sort's index arrays live in the tag array");
     static_assert(offsetof(State, stage_tail) == offsetof(State, val) + sizeof(c.val) &&
                       (sizeof(c.val) + (State::kTail > 0 ? sizeof(c.stage_tail) : 0)) == kStageChunk * State::kThreads * sizeof(uint4),
@@ -493,69 +494,63 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
     uint2* const run = reinterpret_cast<uint2*>(words + kWaves * 64) + wave * 64;
     uint4* const stage = reinterpret_cast<uint4*>(c.val);
     constexpr uint32_t kNoRoom = 0xFFFFFFFFu;
-    constexpr int kChunks = (D + 1 + kStageChunk - 1) / kStageChunk;
-    static_for<kChunks>(PENC_BODY(chunk) {
-        PENC_INDEX(chunk);
-        constexpr int kFirst = chunk * kStageChunk;
-        constexpr int kCount = D + 1 - kFirst < kStageChunk ? D + 1 - kFirst : kStageChunk;
-        count[lane] = 0u;
-        wave_lds_fence();
-        uvec<kStageChunk> place = 0u;  // rank of each record within its wave's run for the bin
-        static_for<kCount>(PENC_BODY(j) {
-            PENC_INDEX(j);
-            if (active) place[j] = atomicAdd(&count[slot[kFirst + j] >> kBinSlotsLog2], 1u);
-        });
-        __syncthreads();  // all waves have counted, and have left the staging array of the chunk before
-        uint32_t before = 0u, mine = 0u;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const uint32_t n = words[w * 64 + lane];
-            before += w < static_cast<int>(wave) ? n : 0u;
-            mine += n;
-        }
-        uint32_t total;
-        const uint32_t first = wave_exclusive_scan(mine, total);
-        run[lane] = make_uint2(first + before, (lane * bins.n_groups + group) * bins.segment_capacity + cursor + before);
-        cursor += mine;
-        const bool all_fit = __all(cursor <= bins.segment_capacity);
-        wave_lds_fence();
-        static_for<kCount>(PENC_BODY(j) {
-            PENC_INDEX(j);
-            if (active) {
-                const uint32_t b = slot[kFirst + j] >> kBinSlotsLog2;
-                // copies first: a bit cast applied directly to a vector element reads element 0
-                const float v0 = a0[kFirst + j], v1 = a1[kFirst + j];
-                const uint2 at = run[b];
-                const uint32_t to = at.y + place[j];
-                uint4 e;
-                e.x = slot[kFirst + j];
-                e.y = __builtin_bit_cast(uint32_t, v0);
-                e.z = __builtin_bit_cast(uint32_t, v1);
-                e.w = all_fit || to < (b * bins.n_groups + group + 1u) * bins.segment_capacity ? to : kNoRoom;
-                stage[at.x + place[j]] = e;
-            }
-        });
-        __syncthreads();
-        static_for<kCount>(PENC_BODY(j) {
-            PENC_INDEX(j);
-            const uint32_t i = j * State::kThreads + threadIdx.x;
-            bool spill = false;
-            uint4 e = {0u, 0u, 0u, 0u};
-            if (i < total) {
-                e = stage[i];
-                if (e.w != kNoRoom) {
-                    store_record(bins, e.w, e.x & (kBinSlots - 1), __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-                } else {
-                    spill = true;  // the segment is full: stage 3
-                }
-            }
-            if (!all_fit && __any(spill))
-                global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-        });
-        // the next chunk (or tile) writes this wave's counters, which the others have read before the barrier above, and the
-        // staging array after its own first barrier: nothing here is overwritten while another wave reads it
-        wave_lds_fence();
+    count[lane] = 0u;
+    wave_lds_fence();
+    uvec<D + 1> place = 0u;  // rank of each record within its wave's run for the bin
+    static_for<D + 1>(PENC_BODY(j) {
+        PENC_INDEX(j);
+        if (active) place[j] = atomicAdd(&count[slot[j] >> kBinSlotsLog2], 1u);
     });
+    __syncthreads();  // all waves have counted, and have left the staging array of the tile before
+    uint32_t before = 0u, mine = 0u;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t n = words[w * 64 + lane];
+        before += w < static_cast<int>(wave) ? n : 0u;
+        mine += n;
+    }
+    uint32_t total;
+    const uint32_t first = wave_exclusive_scan(mine, total);
+    run[lane] = make_uint2(first + before, (lane * bins.n_groups + group) * bins.segment_capacity + cursor + before);
+    cursor += mine;
+    const bool all_fit = __all(cursor <= bins.segment_capacity);
+    wave_lds_fence();
+    static_for<D + 1>(PENC_BODY(j) {
+        PENC_INDEX(j);
+        if (active) {
+            const uint32_t b = slot[j] >> kBinSlotsLog2;
+            // copies first: a bit cast applied directly to a vector element reads element 0
+            const float v0 = a0[j], v1 = a1[j];
+            const uint2 at = run[b];
+            const uint32_t to = at.y + place[j];
+            uint4 e;
+            e.x = slot[j];
+            e.y = __builtin_bit_cast(uint32_t, v0);
+            e.z = __builtin_bit_cast(uint32_t, v1);
+            e.w = all_fit || to < (b * bins.n_groups + group + 1u) * bins.segment_capacity ? to : kNoRoom;
+            stage[at.x + place[j]] = e;
+        }
+    });
+    __syncthreads();
+    static_for<D + 1>(PENC_BODY(j) {
+        PENC_INDEX(j);
+        const uint32_t i = j * State::kThreads + threadIdx.x;
+        bool spill = false;
+        uint4 e = {0u, 0u, 0u, 0u};
+        if (i < total) {
+            e = stage[i];
+            if (e.w != kNoRoom) {
+                store_record(bins, e.w, e.x & (kBinSlots - 1), __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
+            } else {
+                spill = true;  // the segment is full: stage 3
+            }
+        }
+        if (!all_fit && __any(spill))
+            global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
+    });
+    // the next tile writes this wave's counters, which the others have read before the barrier above, and the
+    // staging array after its own first barrier: nothing here is overwritten while another wave reads it
+    wave_lds_fence();
 }
 
 // The same sort for tables with more bins than a wave has lanes (up to one bin per thread of the

@@ -19,13 +19,10 @@ namespace penc {
 // 0.577 -> 0.552 ms at D = 4; at D = 8 the second-order kernel needed 130 registers and ran one workgroup per compute
 // unit: held to 128, 1.334 -> 1.113 ms.  At D = 5 two workgroups whose staging space takes all six vertices of a point are better than three
 // that sort a tile in two chunks (16 levels of 2^18 slots, 2^19 points, scatter and reduction 323 -> 314 us, second order 327 -> 315).
-constexpr int scatter_waves_per_simd(int pos_dim, bool second_order, bool wide_bins, int threads) {
-    if (threads > kScatterBlock) return 4;  // (one workgroup per compute unit)
-    if (wide_bins) return pos_dim <= 3 ? 6 : 4;  // (a variable bin width takes six to eight more registers: up to 30 spilled at D = 4)
-    return pos_dim <= 4 ? 6 : 4;
-}
+// Workgroups of 1024 threads, the wide bins' among them, are alone on their compute unit: four.
+constexpr int scatter_waves_per_simd(int pos_dim, int threads) { return pos_dim <= 4 && threads == kScatterBlock ? 6 : 4; }
 
-constexpr int both_orders_waves_per_simd(int pos_dim, bool wide_bins, int threads) { return pos_dim <= 3 && !wide_bins && threads == kScatterBlock ? 6 : 4; }
+constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_dim <= 3 && threads == kScatterBlock ? 6 : 4; }
 
 // kRowMajor: the upstream gradient is read as rows grad[n][2*level + feature] of `grad_row_stride`
 // floats (what the layer after the encoding produces) instead of [level][feature][n].  A die walks
@@ -274,12 +271,12 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
         random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
 template <int D, bool kRowMajor, bool kSecond, bool kWideBins, int kThreads>
-__global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kSecond, kWideBins, kThreads))
+__global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kThreads))
 backward_table_kernel(PENC_TABLE_PARAMETERS) {
     scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
 template <int D, bool kRowMajor, bool kWideBins, int kThreads>
-__global__ void __launch_bounds__(kThreads, both_orders_waves_per_simd(D, kWideBins, kThreads))
+__global__ void __launch_bounds__(kThreads, both_orders_waves_per_simd(D, kThreads))
 backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
     scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
