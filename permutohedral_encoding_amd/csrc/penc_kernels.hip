@@ -430,14 +430,17 @@ block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_
     }
 }
 
-// The forward (kSecond = false) or the gradient w.r.t. the upstream gradient (kSecond = true) as rows of `row_stride` floats.
-template <int D, int F, typename T, bool kSecond>
+// The forward (kSecond = false) or the gradient w.r.t. the upstream gradient (kSecond = true) as rows of `row_stride` floats.  With
+// kSlopes the forward also leaves the slopes of every feature behind (penc_slopes.hpp): a call that keeps them is the one launch that it is
+// without them.
+template <int D, int F, typename T, bool kSlopes, bool kSecond>
 __global__ void __launch_bounds__(kPointBlock)
 block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
                   const T* __restrict__ table, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                   const float* __restrict__ window, const float* __restrict__ double_pos_grad, float points_scaling,
-                  float* __restrict__ rows, int64_t row_stride) {
+                  float* __restrict__ rows, int64_t row_stride, float* __restrict__ slopes) {
     extern __shared__ float tile[];  // kBlockPoints x (columns | 1)
+    __shared__ uint2 rank_columns[kSlopes ? (D + 1) * kPointBlock : 1];
     const int base = blockIdx.x * kBlockPoints, count = n_points - base < kBlockPoints ? n_points - base : kBlockPoints;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int columns = n_all_levels * F, pitch = columns | 1;
@@ -469,6 +472,8 @@ block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacit
                 static_for<F>(PENC_BODY(k) {
                     PENC_INDEX(k); acc[k] = acc[k] + v.f[k][r] * w[r]; });
             });
+            if constexpr (kSlopes)  // (lanes without a point repeat the last one)
+                store_slopes<D, F>(v.f, s.rank, rank_columns + threadIdx.x, kPointBlock, sf, slopes + slope_offset<D, F>(n_points, level, n));
         }
         static_for<F>(PENC_BODY(k) {
             PENC_INDEX(k); mine[level * F + k] = acc[k]; });
@@ -1355,16 +1360,16 @@ static int block_positions_backward(int pos_dim, int nr_feat, int64_t nr_positio
     return check_launch();
 }
 
-template <bool kSecond>
+template <bool kSlopes, bool kSecond>
 static int block_rows(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int extra, int capacity, const float* positions,
                       const TableRef& table, const float* scale_factor, const float* random_shift, const float* anneal_window,
-                      const float* double_positions_grad, float points_scaling, float* rows, int64_t row_stride, hipStream_t st) {
+                      const float* double_positions_grad, float points_scaling, float* rows, int64_t row_stride, float* slopes, hipStream_t st) {
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((block_rows_kernel<DD, FF, TT, kSecond>), dim3(point_blocks(nr_positions)), dim3(kPointBlock),
+                      hipLaunchKernelGGL((block_rows_kernel<DD, FF, TT, kSlopes, kSecond>), dim3(point_blocks(nr_positions)), dim3(kPointBlock),
                                          block_tile_bytes((nr_levels + extra) * nr_feat), st, static_cast<int>(nr_positions), nr_levels,
                                          nr_levels + extra, static_cast<uint32_t>(capacity), mask_of(capacity), positions,
                                          static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
-                                         double_positions_grad, points_scaling, rows, row_stride));
+                                         double_positions_grad, points_scaling, rows, row_stride, slopes));
     return check_launch();
 }
 
@@ -1572,8 +1577,8 @@ int penc_forward_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         if (!positions || !lattice_values || !scale_factor || !random_shift || !anneal_window) return PENC_ERR_NULL_POINTER;
         const TableRef table{lattice_values, 0};
         if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
-        return block_rows<false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
-                                 anneal_window, nullptr, points_scaling, sliced_rows, row_stride, static_cast<hipStream_t>(stream));
+        return block_rows<false, false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                        anneal_window, nullptr, points_scaling, sliced_rows, row_stride, nullptr, static_cast<hipStream_t>(stream));
     }
     float* level_major = reinterpret_cast<float*>(base);
     if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values, 0}, scale_factor,
@@ -1859,8 +1864,8 @@ int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int 
     if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format))
-        return block_rows<true>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
-                                anneal_window, double_positions_grad, 1.0f, grad_grad_rows, row_stride, st);
+        return block_rows<false, true>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                       anneal_window, double_positions_grad, 1.0f, grad_grad_rows, row_stride, nullptr, st);
     const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
     const size_t need = static_cast<size_t>(cols) * static_cast<size_t>(nr_positions) * sizeof(float);
     if (workspace == nullptr || workspace_bytes < (base - reinterpret_cast<uintptr_t>(workspace)) + need) return PENC_ERR_WORKSPACE_TOO_SMALL;
@@ -1895,14 +1900,34 @@ size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
     return static_cast<size_t>(nr_levels) * slope_tiles(nr_positions) * kSlopeTile * pos_dim * nr_feat * sizeof(float);
 }
 
+// Whether a forward in rows that keeps slopes takes the kernel that keeps all levels of 64 points in a workgroup, as the one without slopes does
+// there; else it is forward_kernel and a transpose, whose launch alone costs a pass that waits for the host 4 to 5 us (D = 3, 16 levels of 2^14
+// slots, forward and position gradient through the module, 16384 points 62.3 -> 58.1 us, 56 without slopes).  Where the device is what is waited
+// for (two launches -> one; forward and position gradient, then the pass of an SDF): D = 3, 16 levels of 2^14 slots, 2^17 points 58.7 -> 57.1,
+// 169 -> 164, 2^19 points 164 -> 147, 516 -> 489; D = 5, 10 levels 165 -> 152, 519 -> 503; D = 6, 24 levels of 2^11 slots 338 -> 340, 995 -> 973.
+// From seven dimensions on the columns that bring the slopes into the order of the coordinates leave room for too few workgroups (D = 7, the same
+// 375 -> 392, 1272 -> 1264; D = 8 425 -> 466, 1330 -> 1353, 16 levels of 2^12 slots, 2^17 points 82.7 -> 88.4 and 2^16 60.1 -> 54.9 and 58.9 -> 61.1).
+static bool slopes_in_point_blocks(int pos_dim, int64_t n, int levels, int capacity, int nr_feat, int columns, int table_format) {
+    return takes_point_blocks(pos_dim, n, levels, capacity, nr_feat, columns, table_format) &&
+           (pos_dim <= 6 || n * levels * (pos_dim + 1) <= kBlocksMidMaxGathers);
+}
+
 int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
                         const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
                         const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
                         int concat_points, float points_scaling, void* stream) {
     if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (!slopes) return PENC_ERR_NULL_POINTER;
-    const int cols = nr_feat * (nr_levels + penc_extra_levels(pos_dim, nr_feat, concat_points));
+    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points), cols = nr_feat * (nr_levels + extra);
     if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
+    if (sliced_rows != nullptr && slopes_in_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table_format)) {
+        if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
+        const TableRef table{lattice_values, table_format};
+        if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values) return PENC_ERR_NULL_POINTER;
+        if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+        return block_rows<true, false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                       anneal_window, nullptr, points_scaling, sliced_rows, row_stride, slopes, static_cast<hipStream_t>(stream));
+    }
     if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values, table_format}, scale_factor,
                               random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream, slopes))
         return rc;

@@ -99,7 +99,7 @@ def phase_of_dispatches(kernels):
             own.append("backward")
         elif b == "grad_grad_kernel":
             own.append("double_backward")
-        elif b == "block_rows_kernel":  # <D, F, T, kSecond>
+        elif b == "block_rows_kernel":  # <D, F, T, kSlopes, kSecond>
             own.append("double_backward" if template_args(k)[-1:] == ["true"] else "forward")
         elif b == "touched_ranges_kernel":
             own.append("clear_touched")

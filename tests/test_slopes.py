@@ -32,9 +32,11 @@ def exact_slopes(p, sf, capacity):
 
 @pytest.mark.parametrize("d,n,levels,cap,feat,concat,fmt", [(3, 1, 5, 64, 2, True, 0), (2, 63, 9, 1 << 10, 4, True, 0), (3, 64, 24, 1 << 18, 2, False, 0),
                                                             (4, 65, 8, 1000, 8, False, 0), (8, 1003, 31, 1 << 10, 8, False, 0), (5, 20001, 7, 1 << 12, 2, True, 0),
-                                                            (6, 4097, 3, 1 << 12, 4, True, 0), (7, 777, 8, 1 << 14, 2, False, 1), (3, 5000, 17, 1 << 14, 2, True, 2)])
+                                                            (6, 4097, 3, 1 << 12, 4, True, 0), (7, 777, 8, 1 << 14, 2, False, 1), (3, 5000, 17, 1 << 14, 2, True, 2),
+                                                            (8, 56001, 24, 1 << 10, 2, False, 0), (3, 30001, 24, 1 << 16, 2, True, 0)])
 def test_derivatives_from_slopes(d, n, levels, cap, feat, concat, fmt):
-    """One point, remainders of a tile, fewer and more levels than waves, 248 columns (80 KB of LDS), a masked level, padded rows, 16-bit tables."""
+    """One point, remainders of a tile, fewer and more levels than waves, 248 columns (80 and 102 KB of LDS), a masked level, padded rows, 16-bit
+    tables; the result level by level and in rows, which a forward of these sizes brings out of workgroups of 64 points, or by a transpose."""
     from helpers import make_encoding, random_problem, to_gpu
     from oracle import api as orc
     from permutohedral_encoding_amd import _native
@@ -52,12 +54,16 @@ def test_derivatives_from_slopes(d, n, levels, cap, feat, concat, fmt):
     lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
     slopes = torch.full((levels * -(-n // 64) * 64 * d * feat,), float("nan"), device="cuda")  # what is not written must not be read
     out, rows = torch.empty(cols, n, device="cuda"), torch.full((n, stride), 7.0, device="cuda")
+    kept = []
     for to_rows in (None, rows.data_ptr()):
+        slopes.fill_(float("nan"))
         assert lib.penc_forward_slopes(d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr(), fmt, fp.m_scale_factor.data_ptr(),
                                        fp.m_random_shift_per_level.data_ptr(), win.data_ptr(), out.data_ptr(), to_rows, stride,
                                        slopes.data_ptr(), int(concat), 0.5, st) == 0
         want = orc.forward(p["pos"], p["table"], sf, p["shift"], p["window"], concat_points=concat, points_scaling=0.5).reshape(cols, n)
         assert np.array_equal(out.cpu().numpy(), want)
+        kept.append(slopes.clone())
+    assert torch.allclose(*kept, rtol=0, atol=0, equal_nan=True)
     assert np.array_equal(rows[:, :cols].cpu().numpy(), want.T) and torch.all(rows[:, cols:] == 7.0)
 
     slope, mag = exact_slopes(p, sf, cap)
