@@ -327,8 +327,8 @@ int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, in
  *   penc_grad_grad_slopes           gives the grad_grad_sliced_values of penc_double_backward_from_positions as [L+E][F][N], or
  *                                   with row_stride != 0 as rows of that many floats.
  * The same derivatives to rounding: the differences of vertex values are formed before the products.  Rows hold at most 255 columns.
- * penc_slopes_bytes() is 0 where nothing would be gained (small batches on tables of at most 1 MiB; many features, whose slopes are as large as the
- * vertices, on tables an L2 holds) and where rows cannot be served.  The three calls themselves take any geometry.
+ * penc_slopes_bytes() is 0 where nothing would be gained (small batches, whose passes wait for the host; many features, whose slopes are as large as
+ * the vertices, on tables an L2 holds) and where rows cannot be served.  The three calls themselves take any geometry.
  * Replaces: the second and third gather of backward_gpu_only_pos and double_backward_from_positions_gpu_2
  * (EncodingGPU.cuh:530-769, 1260-1493). */
 size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int table_format);

@@ -1878,20 +1878,25 @@ int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int 
 }
 
 // Where a forward's slopes are worth keeping for the position gradient and the grad-grad (all three together, us, gathering -> slopes; more
-// in penc_slopes.hpp).  With two features per level also where a workgroup takes all levels of its points: D = 3, 24
-// levels of 2^18 slots, 1000 points 15.0 -> 10.8, 4097 points 24.5 -> 12.1; 16 levels of 2^13 slots, 2^16 points 44.3 -> 28.3, 2^20 575 -> 396;
-// D = 8, 16 levels of 2^12, 5001 points 23.9 -> 13.1; 6 levels of 2^12, 2^16 points 20.5 -> 15.1.  But small batches on tables of at most 1 MiB
-// wait for the host rather than for kernels (5001 points, 16 levels of 2^13 13.9 -> 10.9, with some 130 us of host work around them): they
-// are left to the gathering kernels, which give the bits of the autograd functions.
+// in penc_slopes.hpp).  With two features per level where no workgroup takes all levels of its points (takes_point_blocks), and there too once
+// the batch is large enough: D = 3, 16 levels of 2^13 slots, 2^16 points 44.3 -> 28.3, 2^20 575 -> 396; D = 8, 16 levels of 2^12, 5001
+// points 23.9 -> 13.1.  But a pass on fewer points waits for the host, which keeping slopes costs some 3 us (an allocation more, and what is looked
+// at before they are used), so the line lies where the kernels take as long as the host does: at 3.2 M points times levels times dimensions.
+// Passes of an SDF, and forward and position gradient alone, through the module:
+//   D = 3, 16 levels of 2^14 slots   2^14 points 122.6 -> 126.4, 54.5 -> 57.6   2^16 (3.1 M) 130 -> 130, 56 -> 58   2^17 194 -> 161, 55 -> 57
+//   D = 5, 10 levels of 2^14         2^15 points 124.7 -> 127.6, 55.0 -> 57.6   2^16 (3.3 M) 138 -> 136, 54 -> 55   2^17 212 -> 168, 58 -> 56
+//   D = 8, 16 levels of 2^12         2^14 points 128 -> 128                     2^15 (4.2 M) 131 -> 131             2^16 196 -> 168
+//   D = 3, 24 levels of 2^18 slots   2048 points 122.8 -> 125.5, 54.1 -> 57.1   2^14, the first without blocks, 132.9 -> 124.5, 60.6 -> 56.8
+// (A captured graph, which waits for no host, would gain below the line too.)
 // With four features where no such workgroups serve (D = 3, 16 levels, 2^18 points: 2^12 slots 159 -> 170, 2^14 176 -> 173, 2^15 218 -> 174, 2^16
 // 224 -> 179; D = 5, 2^14 269 -> 283).  With eight where besides no L2 holds a level (D = 3, 16 levels: 2^16 slots, 2^18 points 358 -> 347
 // but 224 -> 241 without the grad-grad, 2^18 slots 941 -> 809; 2^15 points 90 -> 56; D = 4, 2^16 slots 225 -> 233; D = 8, 2^18 slots 178 -> 117).
-constexpr size_t kSlopesSmallTableBytes = size_t{1} << 20, kSlopesMinSliceBytes = size_t{4} << 20;
-constexpr int64_t kSlopesFewPoints = 8192;
+constexpr size_t kSlopesMinSliceBytes = size_t{4} << 20;
+constexpr int64_t kSlopesMinWork = 3200000;
 static bool slopes_serve(int pos_dim, int nr_feat, int64_t n, int levels, int capacity, int table_format) {
-    const size_t slice = slice_bytes(capacity, nr_feat, table_format);
-    if (nr_feat == 2) return n > kSlopesFewPoints || levels * slice > kSlopesSmallTableBytes;
-    return !takes_point_blocks(pos_dim, n, levels, capacity, nr_feat, levels * nr_feat, table_format) && (nr_feat == 4 || slice > kSlopesMinSliceBytes);
+    const bool blocks = takes_point_blocks(pos_dim, n, levels, capacity, nr_feat, levels * nr_feat, table_format);
+    if (nr_feat == 2) return !blocks || n * levels * pos_dim >= kSlopesMinWork;
+    return !blocks && (nr_feat == 4 || slice_bytes(capacity, nr_feat, table_format) > kSlopesMinSliceBytes);
 }
 
 size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int table_format) {

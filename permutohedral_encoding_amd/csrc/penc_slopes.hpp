@@ -21,7 +21,9 @@
 //   D = 3, 24 levels of 2^18 slots, 2^15 points   13.4 -> 15   24.5 -> 7.7  19.8 -> 7.7  57.7 -> 30.4
 // Many features make the slopes as large as the vertices (D = 3, F = 8, 16 levels of 2^18 slots, 2^19 points: 96 bytes against four gathers
 // of 32, 231 -> 353   366 -> 255   344 -> 202   941 -> 809); slopes_serve says where they are kept.  A position gradient that is not
-// differentiated again gains less (D = 3, F = 2: 735 -> 520; F = 4: 672 -> 575; D = 4, F = 8: 415 -> 409; D = 3, F = 8: 597 -> 607).
+// differentiated again gains less (kernels: D = 3, F = 2: 735 -> 520; F = 4: 672 -> 575; D = 4, F = 8: 415 -> 409; D = 3, F = 8: 597 -> 607, through
+// the module 513 -> 505) or loses, where the gathers hit the first-level cache (D = 6, 24 levels of 2^11 slots, 2^19 points 287 -> 340, the pass of
+// an SDF 1047 -> 978; 16 levels of 2^12 242 -> 250 and 889 -> 767).
 // Error against 64 bits (2-norm, D = 2 to 8): position gradient 7.3e-8 - 9.9e-8 -> 5.9e-8 - 7.3e-8, grad-grad 6.5e-8 - 9.4e-8 -> 5.4e-8 - 7.1e-8.
 //
 // slopes[level][tile of 64 points][f * D + k][64]: what a wave of the forward writes for a level, and a wave here reads, is one contiguous

@@ -34,7 +34,7 @@ class PermutoEncoding(torch.nn.Module):
     reference clears a dense gradient in every call, src/Encoding.cu:141, 246, and its training
     protocol steps the whole table, examples/performance.py:99-101).
 
-    Where ``positions`` require a gradient the forward usually keeps what their derivatives need of the table
+    Where ``positions`` require a gradient the forward of all but small batches keeps what their derivatives need of the table
     (4 * pos_dim * nr_feat bytes per point and level, until the graph is freed, given back when memory runs short).
     The derivatives are then those of the forward as it was, unless the table, the points or the window
     have been changed in place since, which is followed: they are computed from the present values.  A write that autograd's version
