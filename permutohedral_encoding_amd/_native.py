@@ -99,10 +99,17 @@ _SIGNATURES = {
                                                _c_f32p, ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
                                                _c_f32p, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
                                                ctypes.c_void_p]),
+    "penc_table_cells_points": (ctypes.c_int64, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "penc_table_cells_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "penc_table_cells": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
+                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "penc_slopes_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "penc_forward_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p,
                                            ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
                                            ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]),
+    "penc_forward_table": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p,
+                                          ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
+                                          ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]),
     "penc_backward_positions_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p,
                                                       _c_f32p, ctypes.c_int64, _c_f32p, _c_f32p, ctypes.c_void_p]),
     "penc_grad_grad_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p,
@@ -372,15 +379,18 @@ class EncodingWrapper:
         None under a functorch transform, with a forward-mode tangent, with a window that requires a gradient and in a trace: those
         are for the functions of ``funcs.py``."""
         fp = self.fixed_params
+        table, in_cells = (lattice_values, False) if self.half_table is None else self._copy_to_gather(lattice_values, positions)
         return (_bridge or bridge()).encode(
-            lattice_values, lattice_values if self.half_table is None else self.gather_table(lattice_values), positions,
+            lattice_values, table, positions,
             anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,
-            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES, fp)
+            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES, fp, in_cells)
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table
     _half_copy = None
     _half_copy_of = None
+    _cells = None      # (key, copy): the 16-bit copy in cells (penc_table_cells), where enough points have been gathered for it
+    _gathered = None   # (key, points): how many were, without it, since the table was last modified
     # set by the module (sparse_table_grad=True): table gradients are added into `sparse_grad`, a SparseTableGrad the
     # wrapper keeps across calls, and the gradient calls return None for them
     sparse_table_grad = False
@@ -393,17 +403,53 @@ class EncodingWrapper:
             self.sparse_grad = SparseTableGrad(lattice_values)
         return self.sparse_grad
 
+    def _half_key(self, lattice_values):
+        return (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, tuple(lattice_values.shape), self.half_table)
+
     def gather_table(self, lattice_values):
         """The tensor the gathering kernels read for ``lattice_values``: the tensor itself, or, with
         ``half_table``, its 16-bit copy, made again whenever the tensor has been modified in place."""
         if self.half_table is None or lattice_values.dtype != torch.float32:
             return lattice_values
-        key = (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, tuple(lattice_values.shape),
-               self.half_table)
+        key = self._half_key(lattice_values)
         if self._half_copy_of != key:
             self._half_copy = lattice_values.detach().to(self.half_table)
             self._half_copy_of = key
         return self._half_copy
+
+    def _copy_to_gather(self, lattice_values, positions):
+        """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
+        is made once the points gathered since the table was last modified are enough (penc_table_cells_points; four times as many while
+        the table is trained, whose next version may be a step away), from the 16-bit copy if there is one."""
+        if lattice_values.dtype != torch.float32 or lattice_values.dim() != 3 or not lattice_values.is_cuda or not lattice_values.is_contiguous():
+            return self.gather_table(lattice_values), False
+        key = self._half_key(lattice_values)
+        cells = self._cells
+        if cells is not None:
+            if cells[0] == key:
+                return cells[1], True
+            self._cells = cells = None
+        points = lib().penc_table_cells_points(self.nr_feat, lattice_values.shape[1], TABLE_FORMATS[self.half_table])
+        if points < 0 or lattice_values.shape[2] != self.nr_feat or positions.dim() != 2:
+            return self.gather_table(lattice_values), False
+        if lattice_values.requires_grad and torch.is_grad_enabled():
+            points *= 4
+        gathered = self._gathered
+        so_far = positions.shape[0] + (gathered[1] if gathered is not None and gathered[0] == key else 0)
+        self._gathered = (key, so_far)
+        if so_far < points:
+            return self.gather_table(lattice_values), False
+        if torch.cuda.is_current_stream_capturing():  # (a copy whose making is captured holds nothing before the graph runs)
+            return self.gather_table(lattice_values), False
+        rounded = self._half_copy_of == key  # it stays: a captured graph may read it
+        try:
+            copy = (_bridge or bridge()).table_in_cells(self._half_copy if rounded else lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
+        except torch.cuda.OutOfMemoryError:
+            return self.gather_table(lattice_values), False
+        if not rounded:
+            self._half_copy = self._half_copy_of = None
+        self._cells = (key, copy)
+        return copy, True
 
     def invalidate_half_table(self):
         """Forgets the 16-bit copy, so that the next call converts the table again.  The copy follows the
@@ -412,6 +458,8 @@ class EncodingWrapper:
         and must be followed by this call."""
         self._half_copy = None
         self._half_copy_of = None
+        self._cells = None
+        self._gathered = None
 
     def _check_common(self, inp):
         fp = self.fixed_params

@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "../../include/penc.h"
+#include "penc_cells.hpp"
 #include "penc_lattice.hpp"
 #include "penc_group_sort.hpp"
 #include "penc_reduce.hpp"
@@ -55,9 +56,6 @@ __device__ __forceinline__ fvec<D> load_point(const float* __restrict__ position
 // bytes for eight floats), fetched back to back so that all loads are in flight together.
 // f[k][r] is feature k of vertex r.  T is the table's element type: float, or __half / bfloat16_bits
 // for a table kept in 16 bits (the values are widened exactly; all arithmetic stays fp32).
-struct bfloat16_bits {
-    uint16_t bits;  // the upper half of the fp32 with the same value
-};
 template <int D, int F>
 struct Vertices {
     fvec<D + 1> f[F];
@@ -162,7 +160,7 @@ __device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile,
 // With kSlopes it also leaves the slopes of every feature behind (penc_slopes.hpp).
 template <int D, int F, typename T, bool kSlopes>
 __global__ void __launch_bounds__(kBlock)
-forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
+forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells,
                const float* __restrict__ positions, const T* __restrict__ table,
                const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                const float* __restrict__ window, float* __restrict__ sliced, float points_scaling, float* __restrict__ slopes) {
@@ -199,7 +197,8 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
         fvec<D + 1> sorted;
         sort_by_rank_lds<D>(columns + threadIdx.x, kBlock, s.rank, s.delta, s.hash0, sorted, h);
         const fvec<D + 1> w = barycentric_of_sorted<D>(sorted);
-        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
+                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
         fvec<F> acc = 0.0f;
         static_for<D + 1>(PENC_BODY(r) {
             PENC_INDEX(r);
@@ -235,7 +234,7 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
 // D = 8, 2^19 slots 444 / 420 / 459 / 487.
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-backward_pos_kernel(int n_points, int n_levels, int per_group, LevelMap map, uint32_t capacity, uint32_t cap_mask,
+backward_pos_kernel(int n_points, int n_levels, int per_group, LevelMap map, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells,
                     const float* __restrict__ positions, const T* __restrict__ table,
                     const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                     const float* __restrict__ window, const float* __restrict__ grad_sliced,
@@ -267,7 +266,8 @@ backward_pos_kernel(int n_points, int n_levels, int per_group, LevelMap map, uin
         const float* sf = scale_factor + level * D;
         const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
         const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
-        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
+                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
         const float* gp = grad_sliced + (static_cast<size_t>(level) * F) * n_points + n;
         // the upstream gradient is read once (non-temporal: it should not displace the table slices)
         fvec<D + 1> dB = (v.f[0] * w_level) * __builtin_nontemporal_load(gp);  // :688-689, feature by feature
@@ -320,7 +320,7 @@ reduce_level_groups_kernel(const float* __restrict__ partial, const float* __res
 
 template <int D, int F, typename T>
 __global__ void __launch_bounds__(kBlock)
-grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask,
+grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells,
                  const float* __restrict__ positions, const T* __restrict__ table,
                  const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                  const float* __restrict__ window, const float* __restrict__ double_pos_grad,
@@ -350,7 +350,8 @@ grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uin
         uvec<D + 1> h;
         fvec<D + 1> sorted;
         sort_by_rank_lds<D>(columns + threadIdx.x, kBlock, s.rank, pos_grad_grad_to_elevated<D>(q, sf), s.hash0, sorted, h);
-        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
+                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
         // dB[r] * w_level, then times the vertex value (:1484-1485)
         const fvec<D + 1> wr = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
         fvec<F> gg = 0.0f;
@@ -378,7 +379,7 @@ constexpr int kBlockWaves = 8, kBlockPoints = 64, kPointBlock = kBlockWaves * kB
 // [level][feature][n] copy is left in grad_level_major when the caller wants it.
 template <int D, int F, typename T, bool kRows>
 __global__ void __launch_bounds__(kPointBlock)
-block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
+block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells, const float* __restrict__ positions,
                           const T* __restrict__ table, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                           const float* __restrict__ window, const float* __restrict__ grad, int64_t grad_row_stride,
                           float* __restrict__ grad_level_major, float* __restrict__ out) {
@@ -405,7 +406,8 @@ block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_
         const float* sf = scale_factor + level * D;
         const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
         const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
-        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
+                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
         const auto upstream = [&](int k) {
             if constexpr (kRows) return tile[row * pitch + level * F + k];
             else return grad[(static_cast<size_t>(level) * F + k) * n_points + n];
@@ -435,7 +437,7 @@ block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_
 // without them.
 template <int D, int F, typename T, bool kSlopes, bool kSecond>
 __global__ void __launch_bounds__(kPointBlock)
-block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
+block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells, const float* __restrict__ positions,
                   const T* __restrict__ table, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
                   const float* __restrict__ window, const float* __restrict__ double_pos_grad, float points_scaling,
                   float* __restrict__ rows, int64_t row_stride, float* __restrict__ slopes) {
@@ -465,7 +467,8 @@ block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacit
             const float* sf = scale_factor + level * D;
             const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
             const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
-            const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
+            const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
+                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
             const fvec<D + 1> w = kSecond ? pos_grad_grad_to_bary<D>(s.rank, q, sf) * w_level : barycentric<D>(s.rank, s.delta) * w_level;
             static_for<D + 1>(PENC_BODY(r) {
                 PENC_INDEX(r);
@@ -808,7 +811,25 @@ inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7
 struct TableRef {
     const void* values;
     int format;
+    bool cells = false;  // PENC_TABLE_CELLS (penc_cells.hpp)
 };
+inline int slots_per_line(int nr_feat, int format) { return kLineBytes / (nr_feat * (format != 0 ? 2 : 4)); }
+inline bool cells_possible(int nr_feat, int capacity, int format) {
+    return capacity >= slots_per_line(nr_feat, format) && (capacity & (capacity - 1)) == 0;
+}
+inline int strip_cells(int table_format) { return table_format & ~PENC_TABLE_CELLS; }
+inline bool known_format(int table_format) {
+    const int format = strip_cells(table_format);
+    return format == 0 || format == PENC_TABLE_FP16 || format == PENC_TABLE_BF16;
+}
+inline bool known_half_format(int table_format) { return known_format(table_format) && strip_cells(table_format) != 0; }
+// (nr_feat is checked by the caller's check_geometry: whatever it refuses is none of this function's)
+inline bool cells_fit(int table_format, int nr_feat, int capacity) {
+    return (table_format & PENC_TABLE_CELLS) == 0 || nr_feat < 2 || nr_feat > 8 || cells_possible(nr_feat, capacity, strip_cells(table_format));
+}
+inline TableRef table_ref(const void* values, int table_format) {
+    return TableRef{values, strip_cells(table_format), (table_format & PENC_TABLE_CELLS) != 0};
+}
 // a slot is gathered with one load (two of 16 bytes for eight floats): 4 to 16 bytes
 inline bool table_aligned(const TableRef& t, int nr_feat) {
     const unsigned slot_bytes = static_cast<unsigned>(nr_feat) * (t.format != 0 ? 2u : 4u);
@@ -1345,11 +1366,12 @@ static int block_positions_backward(int pos_dim, int nr_feat, int64_t nr_positio
                                     const TableRef& table, const float* scale_factor, const float* random_shift,
                                     const float* anneal_window, const float* grad, int64_t grad_row_stride, float* grad_level_major,
                                     float* positions_grad, hipStream_t st) {
+    const uint32_t in_cells = table.cells ? 1u : 0u;
 #define PENC_LAUNCH_BLOCKS(ROWS, LDS)                                                                                                       \
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,                                                                                      \
                       hipLaunchKernelGGL((block_backward_pos_kernel<DD, FF, TT, ROWS>), dim3(point_blocks(nr_positions)),                  \
                                          dim3(kPointBlock), LDS, st, static_cast<int>(nr_positions), nr_levels,                            \
-                                         static_cast<uint32_t>(capacity), mask_of(capacity), positions, static_cast<const TT*>(table.values), \
+                                         static_cast<uint32_t>(capacity), mask_of(capacity), in_cells, positions, static_cast<const TT*>(table.values), \
                                          scale_factor, random_shift, anneal_window, grad, grad_row_stride, grad_level_major, positions_grad))
     if (grad_row_stride != 0) {
         PENC_LAUNCH_BLOCKS(true, block_tile_bytes(nr_levels * nr_feat));
@@ -1364,10 +1386,11 @@ template <bool kSlopes, bool kSecond>
 static int block_rows(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int extra, int capacity, const float* positions,
                       const TableRef& table, const float* scale_factor, const float* random_shift, const float* anneal_window,
                       const float* double_positions_grad, float points_scaling, float* rows, int64_t row_stride, float* slopes, hipStream_t st) {
+    const uint32_t in_cells = table.cells ? 1u : 0u;
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
                       hipLaunchKernelGGL((block_rows_kernel<DD, FF, TT, kSlopes, kSecond>), dim3(point_blocks(nr_positions)), dim3(kPointBlock),
                                          block_tile_bytes((nr_levels + extra) * nr_feat), st, static_cast<int>(nr_positions), nr_levels,
-                                         nr_levels + extra, static_cast<uint32_t>(capacity), mask_of(capacity), positions,
+                                         nr_levels + extra, static_cast<uint32_t>(capacity), mask_of(capacity), in_cells, positions,
                                          static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
                                          double_positions_grad, points_scaling, rows, row_stride, slopes));
     return check_launch();
@@ -1397,8 +1420,9 @@ static int positions_backward(int pos_dim, int nr_feat, int64_t nr_positions, in
         partial = reinterpret_cast<float*>(ws);
     }
     const GatherLaunch g = plan_gather(nr_positions, nr_levels, per_group, slice_bytes(capacity, nr_feat, table.format), kLargeGather / 2);
+    const uint32_t in_cells = table.cells ? 1u : 0u;
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
-                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st, n, nr_levels, per_group, g.map, cap, mask, positions,
+                      hipLaunchKernelGGL((backward_pos_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st, n, nr_levels, per_group, g.map, cap, mask, in_cells, positions,
                                          static_cast<const TT*>(table.values), scale_factor, random_shift, anneal_window,
                                          grad_level_major, partial));
     if (int rc = check_launch()) return rc;
@@ -1467,11 +1491,12 @@ static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_l
     hipStream_t st = static_cast<hipStream_t>(stream);
     const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
                                        slice_bytes(capacity, nr_feat, table.format));
+    const uint32_t in_cells = table.cells ? 1u : 0u;
 #define PENC_LAUNCH_FORWARD(SLOPES)                                                                                                      \
     PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,                                                                                   \
                       hipLaunchKernelGGL((forward_kernel<DD, FF, TT, SLOPES>), g.grid, dim3(kBlock), 0, st,                             \
                                          static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity), \
-                                         mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,              \
+                                         mask_of(capacity), in_cells, positions, static_cast<const TT*>(table.values), scale_factor,              \
                                          random_shift, anneal_window, sliced_values, points_scaling, slopes))
     if (slopes != nullptr) {
         PENC_LAUNCH_FORWARD(true);
@@ -1494,7 +1519,7 @@ const char* penc_status_string(int status) {
         case PENC_ERR_MISALIGNED: return "lattice_values must be aligned to one slot (at most 16 bytes), lattice_values_grad and gradient rows to 8 bytes";
         case PENC_ERR_LAUNCH: return "the HIP runtime rejected a kernel launch";
         case PENC_ERR_WORKSPACE_TOO_SMALL: return "the workspace cannot hold the level-major array the call needs (penc_backward_rowmajor_workspace_bytes, penc_forward_rowmajor_workspace_bytes)";
-        case PENC_ERR_UNSUPPORTED_TABLE_FORMAT: return "table_format must be PENC_TABLE_FP16 or PENC_TABLE_BF16";
+        case PENC_ERR_UNSUPPORTED_TABLE_FORMAT: return "table_format must be PENC_TABLE_FP16 or PENC_TABLE_BF16, with PENC_TABLE_CELLS for capacities that are powers of two and fill a line";
         case PENC_ERR_SCRATCH_TOO_SMALL: return "the problem is too large for the library's static scratch (penc_static_scratch_bytes): use penc_backward with a workspace";
         default: return "unknown status";
     }
@@ -1591,8 +1616,8 @@ int penc_forward_half(int pos_dim, int nr_feat, int64_t nr_positions, int nr_lev
                       const float* positions, const void* lattice_values_half, int table_format,
                       const float* scale_factor, const float* random_shift, const float* anneal_window,
                       float* sliced_values, int concat_points, float points_scaling, void* stream) {
-    if (table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
-    return forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values_half, table_format},
+    if (!known_half_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    return forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table_ref(lattice_values_half, table_format),
                         scale_factor, random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream);
 }
 
@@ -1712,8 +1737,8 @@ int penc_backward_half(int pos_dim, int nr_feat, int64_t nr_positions, int nr_le
                        const float* scale_factor, const float* random_shift, const float* anneal_window,
                        const float* grad, int64_t grad_row_stride, float* lattice_values_grad, float* positions_grad,
                        void* workspace, size_t workspace_bytes, void* stream) {
-    if (table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
-    const TableRef table{lattice_values_half, table_format};
+    if (!known_half_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    const TableRef table = table_ref(lattice_values_half, table_format);
     if (grad_row_stride != 0)
         return backward_rowmajor_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
                                       random_shift, anneal_window, grad, grad_row_stride, lattice_values_grad, positions_grad,
@@ -1749,10 +1774,11 @@ static int double_backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, 
     if (grad_grad_sliced_values) {
         const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
                                            slice_bytes(capacity, nr_feat, table.format));
+        const uint32_t in_cells = table.cells ? 1u : 0u;
         PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,
                           hipLaunchKernelGGL((grad_grad_kernel<DD, FF, TT>), g.grid, dim3(kBlock), 0, st,
                                              static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity),
-                                             mask_of(capacity), positions, static_cast<const TT*>(table.values), scale_factor,
+                                             mask_of(capacity), in_cells, positions, static_cast<const TT*>(table.values), scale_factor,
                                              random_shift, anneal_window, double_positions_grad, grad_grad_sliced_values));
         if (int rc = check_launch()) return rc;
     }
@@ -1799,11 +1825,11 @@ int penc_double_backward_from_positions_half(int pos_dim, int nr_feat, int64_t n
                                              const float* grad, int64_t grad_row_stride, float* lattice_values_grad,
                                              float* grad_grad_sliced_values, int concat_points, void* workspace,
                                              size_t workspace_bytes, void* stream) {
-    if (table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!known_half_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (grad_row_stride != 0 && nr_levels > 0 && nr_positions > 0)
         if (int rc = check_rows(grad, grad_row_stride, nr_positions, nr_levels, nr_feat)) return rc;
     return double_backward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions,
-                                TableRef{lattice_values_half, table_format}, scale_factor, random_shift, anneal_window,
+                                table_ref(lattice_values_half, table_format), scale_factor, random_shift, anneal_window,
                                 double_positions_grad, grad, grad_row_stride, lattice_values_grad, grad_grad_sliced_values,
                                 concat_points, workspace, workspace_bytes, stream);
 }
@@ -1813,9 +1839,9 @@ int penc_backward_both_orders(int pos_dim, int nr_feat, int64_t nr_positions, in
                               const float* random_shift, const float* anneal_window, const float* grad, int64_t grad_row_stride,
                               const float* double_positions_grad, const float* first_grad, float* lattice_values_grad,
                               uint32_t* touched, float* positions_grad, void* workspace, size_t workspace_bytes, void* stream) {
-    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!known_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (!lattice_values_grad || !double_positions_grad || !first_grad) return PENC_ERR_NULL_POINTER;
-    const TableRef table{lattice_values, table_format};
+    const TableRef table = table_ref(lattice_values, table_format);
     const SecondGradient second{double_positions_grad, first_grad};
     if (grad_row_stride != 0)
         return backward_rowmajor_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
@@ -1831,9 +1857,9 @@ int penc_backward_positions_rowmajor(int pos_dim, int nr_feat, int64_t nr_positi
                                      const float* random_shift, const float* anneal_window, const float* grad_rows,
                                      int64_t grad_row_stride, float* grad_level_major, float* positions_grad, void* workspace,
                                      size_t workspace_bytes, void* stream) {
-    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!known_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0)) return rc;
-    const TableRef table{lattice_values, table_format};
+    const TableRef table = table_ref(lattice_values, table_format);
     if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !grad_level_major || !positions_grad)
         return PENC_ERR_NULL_POINTER;
     if (int rc = check_rows(grad_rows, grad_row_stride, nr_positions, nr_levels, nr_feat)) return rc;
@@ -1853,10 +1879,10 @@ int penc_grad_grad_rowmajor(int pos_dim, int nr_feat, int64_t nr_positions, int 
                             const float* random_shift, const float* anneal_window, const float* double_positions_grad,
                             float* grad_grad_rows, int64_t row_stride, int concat_points, void* workspace, size_t workspace_bytes,
                             void* stream) {
-    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!known_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points);
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
-    const TableRef table{lattice_values, table_format};
+    const TableRef table = table_ref(lattice_values, table_format);
     if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !double_positions_grad || !grad_grad_rows)
         return PENC_ERR_NULL_POINTER;
     const int cols = nr_feat * (nr_levels + extra);
@@ -1901,7 +1927,7 @@ static bool slopes_serve(int pos_dim, int nr_feat, int64_t n, int levels, int ca
 
 size_t penc_slopes_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int table_format) {
     if (check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0) != PENC_OK || nr_levels * nr_feat > 255) return 0;
-    if (!slopes_serve(pos_dim, nr_feat, nr_positions, nr_levels, capacity, table_format)) return 0;
+    if (!slopes_serve(pos_dim, nr_feat, nr_positions, nr_levels, capacity, strip_cells(table_format))) return 0;
     return static_cast<size_t>(nr_levels) * slope_tiles(nr_positions) * kSlopeTile * pos_dim * nr_feat * sizeof(float);
 }
 
@@ -1917,26 +1943,37 @@ static bool slopes_in_point_blocks(int pos_dim, int64_t n, int levels, int capac
            (pos_dim <= 6 || n * levels * (pos_dim + 1) <= kBlocksMidMaxGathers);
 }
 
+int penc_forward_table(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                       const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
+                       const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
+                       int concat_points, float points_scaling, void* stream) {
+    if (!known_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points), cols = nr_feat * (nr_levels + extra);
+    if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
+    const TableRef table = table_ref(lattice_values, table_format);
+    if (sliced_rows != nullptr &&
+        (slopes != nullptr ? slopes_in_point_blocks : takes_point_blocks)(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format)) {
+        if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
+        if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values) return PENC_ERR_NULL_POINTER;
+        if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+        return (slopes != nullptr ? block_rows<true, false> : block_rows<false, false>)(
+            pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift, anneal_window, nullptr,
+            points_scaling, sliced_rows, row_stride, slopes, static_cast<hipStream_t>(stream));
+    }
+    if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
+                              random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream, slopes))
+        return rc;
+    return sliced_rows == nullptr ? PENC_OK : transpose_to_rows(sliced_values, sliced_rows, row_stride, nr_positions, cols, static_cast<hipStream_t>(stream));
+}
+
 int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
                         const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
                         const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
                         int concat_points, float points_scaling, void* stream) {
-    if (table_format != 0 && table_format != PENC_TABLE_FP16 && table_format != PENC_TABLE_BF16) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!known_format(table_format)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (!slopes) return PENC_ERR_NULL_POINTER;
-    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points), cols = nr_feat * (nr_levels + extra);
-    if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
-    if (sliced_rows != nullptr && slopes_in_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table_format)) {
-        if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
-        const TableRef table{lattice_values, table_format};
-        if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values) return PENC_ERR_NULL_POINTER;
-        if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
-        return block_rows<true, false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
-                                       anneal_window, nullptr, points_scaling, sliced_rows, row_stride, slopes, static_cast<hipStream_t>(stream));
-    }
-    if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, TableRef{lattice_values, table_format}, scale_factor,
-                              random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream, slopes))
-        return rc;
-    return sliced_rows == nullptr ? PENC_OK : transpose_to_rows(sliced_values, sliced_rows, row_stride, nr_positions, cols, static_cast<hipStream_t>(stream));
+    return penc_forward_table(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, lattice_values, table_format, scale_factor,
+                              random_shift, anneal_window, sliced_values, sliced_rows, row_stride, slopes, concat_points, points_scaling, stream);
 }
 
 static size_t slope_tile_bytes(int columns) { return static_cast<size_t>(kSlopeTile) * (columns | 1) * sizeof(float); }
@@ -2110,6 +2147,85 @@ int penc_adamw_step_sparse(float* params, float* grads, float* exp_avg, float* e
 int penc_clear_touched(float* grads, int nr_feat, int nr_levels, int capacity, uint32_t* touched, void* stream) {
     return launch_touched_ranges(false, nullptr, grads, nullptr, nullptr, nr_feat, nr_levels, capacity, touched, AdamWStep{}, 1,
                                  stream);
+}
+
+// Levels of the column-major copy that are made at a time: what stays in the memory-side cache until it is read (24 levels of 2^22 slots in
+// bfloat16, 32 / 64 / 128 / 384 MiB at a time 386 / 361 / 337 / 365 us, fp32 64 / 128 / 256 568 / 513 / 590).
+constexpr size_t kCellChunkBytes = size_t{128} << 20;
+
+size_t penc_table_cells_workspace_bytes(int nr_feat, int nr_levels, int capacity, int table_format) {
+    if ((nr_feat != 2 && nr_feat != 4 && nr_feat != 8) || nr_levels <= 0 || capacity <= 0) return 0;
+    if (strip_cells(table_format) != table_format || !known_format(table_format) || !cells_possible(nr_feat, capacity, table_format)) return 0;
+    const size_t slice = slice_bytes(capacity, nr_feat, table_format);
+    size_t levels = kCellChunkBytes / slice;
+    if (levels < 1) levels = 1;
+    if (levels > static_cast<size_t>(nr_levels)) levels = static_cast<size_t>(nr_levels);
+    return levels * slice + 256;
+}
+
+// Gathers from a copy of at least 64 KiB a level are faster in cells by 2 to 15 ps a point and level (forward, 12 levels in binary16, 2^18
+// points, table -> copy: D = 2, 2^16 slots 28.7 -> 19.5 us; D = 3, 2^16 39.4 -> 27.1, 2^20 54.8 -> 40.8, with four features 80.0 -> 51.3; D = 5,
+// 2^20 84.0 -> 73.2; D = 8, 2^16 87.4 -> 79.8, with eight features 2^20 285 -> 247; 24 levels of 2^22 slots in bfloat16, 500003 points near a
+// surface 315 -> 160), from a smaller one, which the first-level cache holds, slower (2^12 slots: D = 3 19.5 -> 19.8, D = 8 41.6 -> 43.8).  Making
+// it takes longer than rounding the table does (24 levels, 2^18 slots 22.5 and 11.7 us, 2^20 87 and 48, 2^22 337 and 206); the line is where
+// the points make up for that, which larger levels, whose lines come from beyond the L2, do sooner.
+int64_t penc_table_cells_points(int nr_feat, int capacity, int table_format) {
+    if ((nr_feat != 2 && nr_feat != 4 && nr_feat != 8) || capacity <= 0 || !known_half_format(table_format) ||
+        strip_cells(table_format) != table_format || !cells_possible(nr_feat, capacity, table_format))
+        return -1;
+    const size_t slice = slice_bytes(capacity, nr_feat, table_format);
+    if (slice < (size_t{64} << 10)) return -1;
+    return static_cast<int64_t>(slice / (slice <= (size_t{4} << 20) ? 8 : 40));
+}
+
+int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, const void* lattice_values, int source_format, int table_format,
+                     void* cells, void* workspace, size_t workspace_bytes, void* stream) {
+    if (int rc = check_geometry(pos_dim, nr_feat, 1, nr_levels, capacity, 0)) return rc;
+    if (strip_cells(table_format) != table_format || !known_format(table_format) || !cells_possible(nr_feat, capacity, table_format) ||
+        (source_format != 0 && source_format != table_format))
+        return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!lattice_values || !cells) return PENC_ERR_NULL_POINTER;
+    if (!table_aligned(TableRef{lattice_values, source_format}, nr_feat) || (reinterpret_cast<uintptr_t>(cells) & 15u) != 0) return PENC_ERR_MISALIGNED;
+    const size_t slice = slice_bytes(capacity, nr_feat, table_format);
+    const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
+    const size_t lost = base - reinterpret_cast<uintptr_t>(workspace);
+    if (workspace == nullptr || workspace_bytes < lost + slice) return PENC_ERR_WORKSPACE_TOO_SMALL;
+    void* const columns = reinterpret_cast<void*>(base);
+    const size_t room = (workspace_bytes - lost) / slice;
+    const int slots = slots_per_line(nr_feat, table_format), most = room < static_cast<size_t>(nr_levels) ? static_cast<int>(room) : nr_levels;
+    const uint32_t lines = static_cast<uint32_t>(capacity / slots);
+    const CellMap map = cell_map(pos_dim, slots);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    for (int level = 0; level < nr_levels; level += most) {
+        const dim3 grid((lines + kCellLines - 1) / kCellLines, nr_levels - level < most ? nr_levels - level : most);
+        const void* const from = static_cast<const char*>(lattice_values) + static_cast<size_t>(level) * slice_bytes(capacity, nr_feat, source_format);
+        void* const to = static_cast<char*>(cells) + static_cast<size_t>(level) * slice;
+#define PENC_LAUNCH_COLUMNS(F_, T_, RAW_) hipLaunchKernelGGL((cell_columns_kernel<F_, T_, RAW_>), grid, dim3(kCellBlock), 0, st, from, lines, columns)
+#define PENC_LAUNCH_COLUMNS_OF(T_, RAW_)                     \
+    if (nr_feat == 2) PENC_LAUNCH_COLUMNS(2, T_, RAW_);      \
+    else if (nr_feat == 4) PENC_LAUNCH_COLUMNS(4, T_, RAW_); \
+    else PENC_LAUNCH_COLUMNS(8, T_, RAW_)
+        if (table_format == 0) {
+            PENC_LAUNCH_COLUMNS_OF(float, true);
+        } else if (source_format != 0) {
+            PENC_LAUNCH_COLUMNS_OF(bfloat16_bits, true);  // (either format: the bits are moved)
+        } else if (table_format == PENC_TABLE_BF16) {
+            PENC_LAUNCH_COLUMNS_OF(bfloat16_bits, false);
+        } else {
+            PENC_LAUNCH_COLUMNS_OF(__half, false);
+        }
+#undef PENC_LAUNCH_COLUMNS_OF
+#undef PENC_LAUNCH_COLUMNS
+        if (int rc = check_launch()) return rc;
+        switch (kLineBytes / slots / 4) {
+            case 1: hipLaunchKernelGGL(cell_lines_kernel<1>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
+            case 2: hipLaunchKernelGGL(cell_lines_kernel<2>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
+            case 4: hipLaunchKernelGGL(cell_lines_kernel<4>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
+            default: hipLaunchKernelGGL(cell_lines_kernel<8>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
+        }
+        if (int rc = check_launch()) return rc;
+    }
+    return PENC_OK;
 }
 
 int penc_upload(const float* host_values, float* dst, int n, void* stream) {

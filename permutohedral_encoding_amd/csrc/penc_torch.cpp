@@ -82,6 +82,8 @@ struct Api {
     PENC_FN(backward_positions_rowmajor);
     PENC_FN(grad_grad_rowmajor);
     PENC_FN(slopes_bytes);
+    PENC_FN(table_cells);
+    PENC_FN(table_cells_workspace_bytes);
     PENC_FN(forward_slopes);
     PENC_FN(backward_positions_slopes);
     PENC_FN(grad_grad_slopes);
@@ -127,7 +129,8 @@ struct PyRef {
 struct Call {
     int pos_dim, feat, levels, capacity, extra, concat;
     float scaling;
-    int table_format;  // 0: fp32, else PENC_TABLE_FP16 / PENC_TABLE_BF16
+    int table_format;  // 0: fp32, else PENC_TABLE_FP16 / PENC_TABLE_BF16, with PENC_TABLE_CELLS where in_cells
+    bool in_cells;     // the table is a 16-bit copy in cells (table_in_cells)
     bool rows_output;
     int64_t n, levels_per_pass, max_workspace;  // the binding's LEVELS_PER_PASS, MAX_WORKSPACE_BYTES (< 0: no cap)
     Tensor positions;                           // contiguous
@@ -852,7 +855,7 @@ void prepare_call(Call& c, const Tensor& positions, const Tensor& window) {
     if (type == at::kHalf || type == at::kBFloat16) {
         PENC_REQUIRE(c.table.is_cuda(), "lattice_values should be in GPU memory. Please call .cuda() on the tensor");
         PENC_REQUIRE(c.table.dim() == 3, "lattice_values should have 3 dimensions, however it has sizes ", c.table.sizes());
-        c.table_format = type == at::kHalf ? PENC_TABLE_FP16 : PENC_TABLE_BF16;
+        c.table_format = (type == at::kHalf ? PENC_TABLE_FP16 : PENC_TABLE_BF16) | (c.in_cells ? PENC_TABLE_CELLS : 0);
     } else {
         require_f32_gpu(c.table, "lattice_values", 3);
         c.table_format = 0;
@@ -905,11 +908,11 @@ bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positi
 }
 
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
-//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params)
+//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params, in_cells)
 //   -> (N, F(L+E)), or None where the autograd functions are needed
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
-        TORCH_CHECK(n_args == 15, "encode takes 15 arguments");
+        TORCH_CHECK(n_args == 16, "encode takes 16 arguments");
         TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
         const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
         const Tensor& positions = tensor_arg(args[2], "positions");
@@ -927,6 +930,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.concat = PyObject_IsTrue(args[8]);
         c.scaling = static_cast<float>(PyFloat_AsDouble(args[9]));
         c.rows_output = PyObject_IsTrue(args[11]);
+        c.in_cells = PyObject_IsTrue(args[15]);
         c.levels_per_pass = PyLong_AsLongLong(args[12]);
         c.max_workspace = args[13] == Py_None ? -1 : PyLong_AsLongLong(args[13]);
         if (PyErr_Occurred()) return nullptr;
@@ -962,6 +966,34 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             torch::autograd::set_history(out, result);
         }
         return THPVariable_Wrap(std::move(out));
+    });
+}
+
+// table_in_cells(table, table_format, pos_dim) -> the table (fp32, or already of that format) as a 16-bit copy in cells
+PyObject* py_table_in_cells(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 3, "table_in_cells takes 3 arguments");
+        TORCH_CHECK(api.table_cells != nullptr, "bind() has not been called");
+        const Tensor& table = tensor_arg(args[0], "lattice_values");
+        const int format = static_cast<int>(PyLong_AsLong(args[1])), pos_dim = static_cast<int>(PyLong_AsLong(args[2]));
+        if (PyErr_Occurred()) return nullptr;
+        const bool fp32 = table.scalar_type() == at::kFloat;
+        const auto type = format == PENC_TABLE_FP16 ? at::kHalf : at::kBFloat16;
+        PENC_REQUIRE(table.is_cuda() && table.is_contiguous() && table.dim() == 3 && (fp32 || table.scalar_type() == type), "bad table");
+        const int levels = static_cast<int>(table.size(0)), capacity = static_cast<int>(table.size(1)), feat = static_cast<int>(table.size(2));
+        Tensor cells;
+        {
+            NoGil no_gil;
+            at::NoGradGuard no_grad;
+            const c10::DeviceGuard device(table.device());
+            cells = at::empty(table.sizes(), table.options().dtype(type));
+            const size_t n = api.table_cells_workspace_bytes(feat, levels, capacity, format);
+            const Tensor ws = at::empty({static_cast<int64_t>(n)}, table.options().dtype(at::kByte));
+            check(api.table_cells(pos_dim, feat, levels, capacity, table.const_data_ptr(), fp32 ? 0 : format, format, cells.mutable_data_ptr(),
+                                  ws.mutable_data_ptr(), n, current_stream(table.device())),
+                  "table_cells");
+        }
+        return THPVariable_Wrap(std::move(cells));
     });
 }
 
@@ -1074,6 +1106,8 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(backward_positions_rowmajor);
         PENC_FN(grad_grad_rowmajor);
         PENC_FN(slopes_bytes);
+        PENC_FN(table_cells);
+        PENC_FN(table_cells_workspace_bytes);
         PENC_FN(forward_slopes);
         PENC_FN(backward_positions_slopes);
         PENC_FN(grad_grad_slopes);
@@ -1085,6 +1119,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
     {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},
     {"cosine_window", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_cosine_window)), METH_FASTCALL, "a coarse-to-fine window"},
     {"adamw_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step)), METH_FASTCALL, "one AdamW step"},
     {"adamw_step_sparse", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step_sparse)), METH_FASTCALL,

@@ -19,7 +19,8 @@ class PermutoEncoding(torch.nn.Module):
     kernels gather from a 16-bit copy of ``lattice_values`` (the switch the reference carries
     disabled, EncodingGPU.cuh:12).  The parameter itself and every gradient stay fp32; the copy is
     refreshed whenever the parameter has been modified in place (optimizer steps), so it pays for
-    large tables and for inference.  float16 resolves the reference's initial values (about 1e-5)
+    large tables and for inference.  Once enough points have been gathered from one version of the table its copy is
+    laid out anew, in an order of its own that needs fewer cache lines (``EncodingWrapper._copy_to_gather``); the results are the same.  float16 resolves the reference's initial values (about 1e-5)
     only to 6e-8; bfloat16 keeps three significant digits at any magnitude.
 
     ``contiguous_output=True`` returns the (N, F(L+E)) result as a contiguous array instead of the strided

@@ -1,0 +1,202 @@
+"""Tables in cells (csrc/penc_cells.hpp): a gather from a permuted copy reads the values of the table it was made from."""
+import numpy as np
+import pytest
+import torch
+
+CELLS = 0x100
+HALF = {0: torch.float32, 1: torch.float16, 2: torch.bfloat16}
+
+
+def make_cells(table, pos_dim, fmt, workspace_levels=None):
+    from permutohedral_encoding_amd import _native
+    lib, (levels, cap, feat) = _native.lib(), table.shape
+    source = {v: k for k, v in HALF.items()}[table.dtype]
+    cells = torch.full((levels, cap, feat), float("nan"), dtype=HALF[fmt], device="cuda")
+    nbytes = lib.penc_table_cells_workspace_bytes(feat, levels, cap, fmt)
+    if workspace_levels is not None:
+        nbytes = workspace_levels * cap * feat * cells.element_size() + 256
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    assert lib.penc_table_cells(pos_dim, feat, levels, cap, table.data_ptr(), source, fmt, cells.data_ptr(), ws.data_ptr(), nbytes,
+                                torch.cuda.current_stream().cuda_stream) == 0
+    return cells
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("feat", [2, 4, 8])
+@pytest.mark.parametrize("d", range(2, 9))
+def test_every_gather_from_cells_equals_the_gather_from_the_table(d, feat, fmt):
+    """One line, two, less than a workgroup's lines, as many, a few workgroups'; levels one and several at a time through the workspace, a masked
+    one; results bit for bit, from workgroups of 64 points and all levels and from launches a level at a time."""
+    from helpers import make_encoding, random_problem, to_gpu
+    from permutohedral_encoding_amd import _native
+    line = 128 // (feat * (2 if fmt else 4))
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    for cap, levels, n in ((line, 3, 100), (2 * line, 3, 65), (64 * line, 5, 1003), (128 * line, 5, 1003), (1 << 14, 5, 2001), (1 << 18, 24 // feat * 2, 30001)):
+        p = random_problem(d, n, levels, cap, seed=d, sigma_range=(1.0, 1e-3), nr_feat=feat)
+        p["window"][levels // 2] = 0.0
+        _, fp = make_encoding(d, p["sigmas"], p["shift"], nr_feat=feat)
+        table, pos, win, dpos, grad = (to_gpu(p[k]) for k in ("table", "pos", "window", "dpos", "grad"))
+        plain = table.to(HALF[fmt])
+        cells = make_cells(table, d, fmt, workspace_levels=2 if cap == 1 << 14 else None)
+        assert torch.equal(cells, make_cells(plain, d, fmt))  # from a table already rounded
+        assert torch.equal(cells.reshape(levels, -1, feat).float().sort(1).values, plain.reshape(levels, -1, feat).float().sort(1).values)
+        sf, shift = fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr()
+        cols = feat * levels
+        rows = grad.reshape(cols, n).t().contiguous()
+        ws = torch.empty(lib.penc_positions_workspace_bytes(d, n, levels) + 4 * cols * n + 1024, dtype=torch.uint8, device="cuda")
+
+        def results(values, table_format):
+            common = (d, feat, n, levels, cap, pos.data_ptr(), values.data_ptr(), table_format, sf, shift, win.data_ptr())
+            out, as_rows, positions_grad = torch.empty(cols, n, device="cuda"), torch.empty(n, cols, device="cuda"), torch.empty(n, d, device="cuda")
+            slopes = torch.zeros(levels * -(-n // 64) * 64 * d * feat, device="cuda")
+            got = []
+            for keep in (None, slopes.data_ptr()):
+                for to_rows in (None, as_rows.data_ptr()):
+                    assert lib.penc_forward_table(*common, out.data_ptr(), to_rows, cols, keep, 0, 1.0, st) == 0
+                    got += [out.clone(), as_rows.clone()] if to_rows is None else [as_rows.clone()]
+            got = [got[0], got[2], got[3], got[5], slopes]
+            level_major = torch.empty(cols, n, device="cuda")
+            assert lib.penc_backward_positions_rowmajor(*common, rows.data_ptr(), cols, level_major.data_ptr(), positions_grad.data_ptr(),
+                                                        ws.data_ptr(), ws.numel(), st) == 0
+            got.append(positions_grad)
+            grad_grad = torch.empty(n, cols, device="cuda")
+            assert lib.penc_grad_grad_rowmajor(*common, dpos.data_ptr(), grad_grad.data_ptr(), cols, 0, ws.data_ptr(), ws.numel(), st) == 0
+            got.append(grad_grad)
+            if table_format != 0 and table_format != CELLS:
+                out2, positions_grad2, grad_grad2 = torch.empty(cols, n, device="cuda"), torch.empty(n, d, device="cuda"), torch.empty(cols, n, device="cuda")
+                assert lib.penc_forward_half(*common, out2.data_ptr(), 0, 1.0, st) == 0
+                assert lib.penc_backward_half(*common, grad.data_ptr(), 0, None, positions_grad2.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
+                assert lib.penc_double_backward_from_positions_half(*common, dpos.data_ptr(), grad.data_ptr(), 0, None, grad_grad2.data_ptr(), 0,
+                                                                    ws.data_ptr(), ws.numel(), st) == 0
+                got += [out2, positions_grad2, grad_grad2]
+            return got
+
+        for k, (want, got) in enumerate(zip(results(plain, fmt), results(cells, fmt | CELLS))):
+            assert torch.equal(want, got), (cap, levels, n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [1, 2])
+def test_conversion_rounds_as_torch_does(fmt):
+    """Ties, subnormals, overflow, infinities, NaN, signed zeros: a line of them each."""
+    bits = torch.cat([torch.arange(0, 1 << 32, 65521, dtype=torch.int64), torch.tensor([0x7F800000, 0xFF800000, 0x7FC00000, 0x7F800001, 0x80000000, 0x33000000,
+                      0x33000001, 0x387FE000, 0x477FF000, 0x477FEFFF, 0x3F808000, 0x3F818000, 0x7F7FFFFF])])
+    bits = torch.cat([bits, bits[: (1 << 17) - len(bits) % (1 << 17)]])
+    values = bits.to(torch.int32).view(torch.float32)[: 1 << 17].reshape(1, 1 << 16, 2).cuda()
+    plain, cells = values.to(HALF[fmt]), make_cells(values, 3, fmt)
+    as_bits = lambda t: torch.where(torch.isnan(t), torch.full_like(t, float("nan")), t).view(torch.int16).reshape(-1).sort().values
+    assert torch.equal(as_bits(plain), as_bits(cells))
+
+
+def test_cells_are_refused_where_they_are_not_possible():
+    import ctypes
+    from permutohedral_encoding_amd import _native
+    lib, p = _native.lib(), ctypes.c_void_p(1 << 20)
+    assert lib.penc_table_cells_workspace_bytes(2, 4, 32, 1) > 0 and lib.penc_table_cells_workspace_bytes(2, 4, 16, 0) > 0
+    for feat, cap, fmt in ((2, 16, 1), (2, 8, 0), (2, 1000, 0), (8, 4, 1), (3, 64, 0), (2, 64, 3), (2, 64, 1 | CELLS)):
+        assert lib.penc_table_cells_workspace_bytes(feat, 4, cap, fmt) == 0
+        assert lib.penc_table_cells(3, feat, 4, cap, p, 0, fmt, p, p, 1 << 20, None) != 0
+    for cap, fmt in ((16, 1), (1000, 1), (8, 0), (1000, 0)):  # neither is a table said to be in cells
+        assert lib.penc_forward_table(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, None, 0, None, 0, 1.0, None) == 9
+        if fmt:
+            assert lib.penc_forward_half(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, 0, 1.0, None) == 9
+    assert lib.penc_forward_half(3, 2, 10, 4, 64, p, p, CELLS, p, p, p, p, 0, 1.0, None) == 9
+    assert lib.penc_table_cells(3, 2, 4, 64, p, 1, 2, p, p, 1 << 20, None) == 9
+    assert lib.penc_table_cells(3, 2, 4, 64, None, 0, 1, p, p, 1 << 20, None) == 1
+    assert lib.penc_table_cells(3, 2, 4, 64, p, 0, 1, ctypes.c_void_p((1 << 20) + 8), p, 1 << 20, None) == 5
+    assert lib.penc_table_cells(3, 2, 4, 64, p, 0, 1, p, p, 64, None) == 8
+
+
+def test_cells_cover_the_lattice_once():
+    """The rule of the head comment in Python's integers: for every dimension and line the offsets found by another search give a permutation."""
+    mul = 2531011
+    for d in (2, 3, 5, 8):
+        step = [(sum(mul ** (d - i) for i in range(d)) - ((d + 1) * mul ** (d - c) if c < d else 0)) % (1 << 32) for c in range(d + 1)]
+        for line in (4, 8, 16, 32):
+            offset, frontier = {0: 0}, [0]
+            while frontier:  # breadth first over the steps
+                frontier = [h for f in frontier for s in step for h in ((f + s) % (1 << 32), (f - s) % (1 << 32))
+                            if h % line not in offset and offset.setdefault(h % line, h) == h]
+            assert len(offset) == line
+            cap = 64 * line
+            slots = {((h - offset[h % line]) | (h % line)) % cap for h in range(cap)}
+            assert slots == set(range(cap))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,feat,cap,dtype", [(3, 2, 1 << 16, torch.bfloat16), (2, 4, 1 << 14, torch.float16), (5, 8, 1 << 12, torch.bfloat16)])
+def test_module_gathers_from_cells_once_enough_points_were_gathered(d, feat, cap, dtype):
+    """Results are those of the table in its own order throughout: before, at and after the call that makes the copy, in both derivatives, after
+    an in-place change, in a graph captured before the copy was made, and where its making is refused."""
+    import permutohedral_encoding_amd as pe
+    from permutohedral_encoding_amd import _native
+    levels = 6
+    line = _native.lib().penc_table_cells_points(feat, cap, _native.TABLE_FORMATS[dtype])
+    assert line > 0
+    m = pe.PermutoEncoding(d, cap, levels, feat, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=dtype)
+    plain = pe.PermutoEncoding(d, cap, levels, feat, np.geomspace(1.0, 1e-3, levels))  # of the rounded values, gathered in fp32
+    plain.load_state_dict(m.state_dict())
+
+    def follow():
+        with torch.no_grad():
+            plain.lattice_values.copy_(m.lattice_values.to(dtype).float())
+    follow()
+    few, many = torch.rand(line // 2, d, device="cuda"), torch.rand(line, d, device="cuda")
+    with torch.no_grad():
+        assert torch.equal(m(few), plain(few)) and m.lattice._cells is None
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            m(few[:100])
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = m(many)  # enough by now, but not while a graph is captured
+        assert m.lattice._cells is None
+        assert torch.equal(m(few), plain(few)) and m.lattice._cells is not None
+        assert torch.equal(m(many), plain(many)) and torch.equal(m(many[:1]), plain(many[:1]))
+        for _ in range(2):
+            captured.zero_()
+            graph.replay()
+            assert torch.equal(captured, plain(many))
+
+        m.lattice_values.mul_(0.5)
+        follow()
+        assert torch.equal(m(many), plain(many)) and m.lattice._cells is not None and m.lattice._half_copy is None
+
+    def derivatives(enc, pos):
+        pos = pos.clone().requires_grad_(True)
+        out = enc(pos)
+        normal, = torch.autograd.grad(out, pos, torch.ones_like(out).requires_grad_(True), create_graph=True)
+        enc.lattice_values.grad = None
+        (normal * pos.detach()).sum().backward()
+        return out.detach(), normal.detach(), enc.lattice_values.grad
+    for pos in (few, many):
+        for a, b in zip(derivatives(m, pos), derivatives(plain, pos)):
+            assert (a - b).norm() <= 1e-6 * b.norm()
+
+    # a table in training: four times the points before the next version is laid out
+    with torch.no_grad():
+        m.lattice_values.mul_(2.0)
+    follow()
+    assert torch.equal(m(many).detach(), plain(many).detach()) and m.lattice._cells is None
+    for _ in range(3):
+        m(many)
+    assert m.lattice._cells is not None and torch.equal(m(many).detach(), plain(many).detach())
+
+    # no memory for it: the copy in the table's own order serves
+    m.invalidate_half_table()
+
+    class Refusing:
+        def __getattr__(self, name):
+            return getattr(_native_bridge, name)
+
+        def table_in_cells(self, *args):
+            raise torch.cuda.OutOfMemoryError("refused")
+    _native_bridge, _native._bridge = _native._bridge, Refusing()
+    try:
+        with torch.no_grad():
+            assert torch.equal(m(many), plain(many)) and m.lattice._cells is None
+    finally:
+        _native._bridge = _native_bridge
