@@ -220,8 +220,8 @@ int penc_double_backward_from_positions_rowmajor(int pos_dim, int nr_feat, int64
 
 /* A copy of the table in cells: capacities that are powers of two and fill a 128-byte line can be permuted so that a line
  * holds the slots of neighbouring lattice points, and the D+1 vertices of a simplex lie on about half as many lines
- * (csrc/penc_cells.hpp).  penc_table_cells makes such a copy of a table that is fp32 (source_format 0: rounded to nearest even where
- * table_format is PENC_TABLE_FP16 or PENC_TABLE_BF16) or already in table_format: `cells` has the table's [L][C][F] values in another order within every level, 16-byte aligned (128 for
+ * (csrc/penc_cells.hpp).  penc_table_cells makes such a copy, as table_format PENC_TABLE_FP16 or PENC_TABLE_BF16, of a table that is fp32
+ * (source_format 0: rounded to nearest even) or already in table_format: `cells` has the table's [L][C][F] values in another order within every level, 16-byte aligned (128 for
  * whole lines), for the same pos_dim only.  A call takes it in place of the table with table_format | PENC_TABLE_CELLS where it has
  * a table_format, and returns what it returns for the table.  The order is the library's own: a copy is not to be stored.
  * The workspace holds at least one level of the copy; the suggested size is what stays in the memory-side cache. */
@@ -350,11 +350,14 @@ int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_l
                         const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
                         const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
                         int concat_points, float points_scaling, void* stream);
-/* The same with slopes optional (NULL: none are left): the one forward that takes every table_format and gives rows. */
-int penc_forward_table(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
-                       const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
-                       const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
-                       int concat_points, float points_scaling, void* stream);
+/* penc_forward (sliced_rows NULL) or penc_forward_rowmajor (sliced_values is then scratch), without slopes (NULL) or as penc_forward_slopes, by way
+ * of a copy in cells of the levels whose gathers gain by it: two or four features, a capacity that is a power of two and fills a line.  penc_forward_cells_workspace_bytes() is 0 where the copy costs as much as it gives (row_columns: nr_feat*(L+E)
+ * when rows are wanted, else 0). */
+size_t penc_forward_cells_workspace_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int row_columns);
+int penc_forward_cells(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                       const float* lattice_values, const float* scale_factor, const float* random_shift, const float* anneal_window,
+                       float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes, int concat_points, float points_scaling,
+                       void* workspace, size_t workspace_bytes, void* stream);
 int penc_backward_positions_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, const float* slopes,
                                    const float* anneal_window, const float* grad, int64_t grad_row_stride, float* grad_level_major,
                                    float* positions_grad, void* stream);

@@ -107,9 +107,10 @@ _SIGNATURES = {
     "penc_forward_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p,
                                            ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
                                            ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]),
-    "penc_forward_table": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p,
-                                          ctypes.c_void_p, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
-                                          ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]),
+    "penc_forward_cells_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "penc_forward_cells": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p,
+                                          _c_f32p, _c_f32p, _c_f32p, _c_f32p, ctypes.c_int64, _c_f32p, ctypes.c_int, ctypes.c_float,
+                                          ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "penc_backward_positions_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p,
                                                       _c_f32p, ctypes.c_int64, _c_f32p, _c_f32p, ctypes.c_void_p]),
     "penc_grad_grad_slopes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, _c_f32p, _c_f32p, _c_f32p,
@@ -379,7 +380,9 @@ class EncodingWrapper:
         None under a functorch transform, with a forward-mode tangent, with a window that requires a gradient and in a trace: those
         are for the functions of ``funcs.py``."""
         fp = self.fixed_params
-        table, in_cells = (lattice_values, False) if self.half_table is None else self._copy_to_gather(lattice_values, positions)
+        table, in_cells = lattice_values, False
+        if self.half_table is not None:
+            table, in_cells = self._copy_to_gather(lattice_values, positions)
         return (_bridge or bridge()).encode(
             lattice_values, table, positions,
             anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,

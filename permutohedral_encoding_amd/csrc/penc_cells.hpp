@@ -22,6 +22,7 @@
 #include <utility>
 
 #include "penc_lattice.hpp"
+#include "penc_scatter.hpp"
 
 namespace penc {
 
@@ -100,8 +101,7 @@ static __device__ const CellOffsets cell_offsets = kCells<D>;
 
 // Raw hashes whose low bits are slots of the table in cells.  (A wave's look-ups fall into one line, which the first-level cache holds.)
 template <int D, int kSlots>
-__device__ __forceinline__ uvec<D + 1> hashes_in_cells(uint32_t in_cells, uvec<D + 1> h) {
-    if (in_cells == 0u) return h;
+__device__ __forceinline__ uvec<D + 1> hashes_in_cells(uvec<D + 1> h) {
     uvec<D + 1> moved;
     static_for<D + 1>(PENC_BODY(r) {
         PENC_INDEX(r);
@@ -109,6 +109,14 @@ __device__ __forceinline__ uvec<D + 1> hashes_in_cells(uint32_t in_cells, uvec<D
         moved[r] = (h[r] - cell_offsets<D>.t[cells_at(kSlots) + i]) | i;  // (the difference is a multiple of kSlots)
     });
     return moved;
+}
+// The same for a 16-bit copy that may be in cells.
+template <int D, int F, typename T>
+__device__ __forceinline__ uvec<D + 1> hashes_in_copy(uint32_t in_cells, uvec<D + 1> h) {
+    if constexpr (sizeof(T) == 2) {
+        if (in_cells != 0u) h = hashes_in_cells<D, line_slots<F, T>()>(h);
+    }
+    return h;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -239,6 +247,85 @@ cell_lines_kernel(const void* __restrict__ columns, uint32_t lines, CellMap map,
     for (int k = 0; k < kEach; ++k) {
         const uint32_t e = k * kCellBlock + threadIdx.x;
         if (e < count * kSlots) to[e] = tile[(e / kSlots) * kPitch + e % kSlots];
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// a copy for one forward
+//
+// The table of a training step is another one in every step, so a copy of an fp32 table serves one forward, and what it costs must be less than
+// what that forward gains: for levels that an L2 holds, one die to a level, so that the columns can be read where they are (a request for every
+// slot, as in a gather), and of those only the levels where most gathers of a wave are lines of their own.  (Where lanes share lines the
+// first-level cache serves them, from either copy alike: the coarse half of 24 levels for unordered points, all but the finest for samples along
+// rays.)  Every workgroup of a level looks at the same points, a stretch of 64 from the beginning of each quarter of the batch, and counts a wave's
+// lines as bits of a small map; the first says what they found.
+// Forward of 2^20 unordered points, 24 levels of 2^18 slots, D = 3: 280 -> 237 us with 16 levels chosen (all of them, or the 16 in two passes through
+// columns, 246 and 244; one, two, four times kCellLines lines to a workgroup 241 / 237 / 239), D = 4 377 -> 344.
+constexpr int kCellsPerWorkgroup = 2;   // times kCellLines lines
+constexpr uint32_t kSampleBits = 4096;  // of a wave's map: up to 8 x 64 lines
+template <int D, int F>
+__global__ void __launch_bounds__(kCellBlock)
+chosen_cells_kernel(const float* __restrict__ table, uint32_t lines, uint32_t n_levels, uint32_t per_level, uint32_t dies, CellMap map, int64_t n_points,
+                    const float* __restrict__ positions, const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
+                    const float* __restrict__ window, uint32_t* __restrict__ chosen, float* __restrict__ cells) {
+    constexpr int kWaves = kCellBlock / 64, kSlots = line_slots<F, float>(), kPitch = kSlots + 1;
+    using Slot = CellSlot<F>;
+    __shared__ Slot tile[kCellLines * kPitch];
+    __shared__ uint32_t seen[kWaves][kSampleBits / 32];
+    __shared__ uint32_t distinct;
+    const uint32_t j = blockIdx.x / dies, level = j / per_level * dies + blockIdx.x % dies, part = j % per_level;
+    if (level >= n_levels) return;
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    bool mine = false;
+    if (window[level] != 0.0f) {
+        int64_t n = n_points / kWaves * wave + lane;
+        n = n < n_points ? n : n_points - 1;
+        const float* const p = positions + n * D;
+        fvec<D> pos;
+        static_for<D>(PENC_BODY(k) {
+            PENC_INDEX(k); pos[k] = p[k]; });
+        for (uint32_t i = lane; i < kSampleBits / 32; i += 64) seen[wave][i] = 0u;
+        if (threadIdx.x == 0) distinct = 0u;
+        const Located<D> at = locate<D>(pos, random_shift + level * D, scale_factor + level * D);
+        const uvec<D + 1> h = vertex_hashes<D>(at.rank, at.hash0);
+        __syncthreads();
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            const uint32_t line = (h[r] / kSlots) & (lines - 1u), bit = (line * 0x9E3779B1u) / (0xFFFFFFFFu / kSampleBits + 1u);
+            atomicOr(&seen[wave][bit / 32], 1u << (bit % 32));
+        });
+        wave_lds_fence();
+        uint32_t count = 0u;
+        for (uint32_t i = lane; i < kSampleBits / 32; i += 64) count += __popc(seen[wave][i]);
+        if (count != 0u) atomicAdd(&distinct, count);
+        __syncthreads();
+        mine = distinct * 8u >= static_cast<uint32_t>(5 * (D + 1) * kCellBlock);
+    }
+    if (part == 0u && threadIdx.x == 0) chosen[level] = mine ? 1u : 0u;
+    if (!mine) return;
+    const Slot* const from = reinterpret_cast<const Slot*>(table) + static_cast<size_t>(level) * lines * kSlots;
+    Slot* const to = reinterpret_cast<Slot*>(cells) + static_cast<size_t>(level) * lines * kSlots;
+    constexpr int kEach = kCellLines * kSlots / kCellBlock;
+    for (uint32_t first = part * (kCellsPerWorkgroup * kCellLines), end = first + kCellsPerWorkgroup * kCellLines; first < end && first < lines; first += kCellLines) {
+        Slot slot[kEach];
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const uint32_t e = k * kCellBlock + threadIdx.x, line = e % kCellLines;
+            const uint32_t i = __builtin_amdgcn_readfirstlane(e / kCellLines);  // (a wave is in one column)
+            slot[k] = from[((first + line + map.t[i] / kSlots) & (lines - 1u)) * kSlots + i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const uint32_t e = k * kCellBlock + threadIdx.x;
+            tile[(e % kCellLines) * kPitch + e / kCellLines] = slot[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const uint32_t e = k * kCellBlock + threadIdx.x;
+            if (first + e / kSlots < lines) to[static_cast<size_t>(first) * kSlots + e] = tile[(e / kSlots) * kPitch + e % kSlots];
+        }
     }
 }
 

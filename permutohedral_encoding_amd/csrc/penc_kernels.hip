@@ -157,13 +157,15 @@ __device__ __forceinline__ bool locate_work(const LevelMap& map, uint32_t& tile,
 // (compute-bound) and a fine (gather-bound) level, which takes the fine level's slice out of L2
 // (30% slower).
 
-// With kSlopes it also leaves the slopes of every feature behind (penc_slopes.hpp).
-template <int D, int F, typename T, bool kSlopes>
+// With kSlopes it also leaves the slopes of every feature behind (penc_slopes.hpp).  With kChosen the levels that `chosen` names are gathered from
+// `cells` (chosen_cells_kernel).
+template <int D, int F, typename T, bool kSlopes, bool kChosen>
 __global__ void __launch_bounds__(kBlock)
 forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint32_t capacity, uint32_t cap_mask, uint32_t in_cells,
                const float* __restrict__ positions, const T* __restrict__ table,
                const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
-               const float* __restrict__ window, float* __restrict__ sliced, float points_scaling, float* __restrict__ slopes) {
+               const float* __restrict__ window, float* __restrict__ sliced, float points_scaling, float* __restrict__ slopes,
+               const T* __restrict__ cells, const uint32_t* __restrict__ chosen) {
     uint32_t tile, row;
     if (!locate_work(map, tile, row)) return;
     const int n = tile * kBlock + threadIdx.x;
@@ -185,6 +187,8 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
     for (int level = static_cast<int>(row); level < n_levels; level += static_cast<int>(map.rows)) {
         float* out = sliced + (static_cast<size_t>(level) * F) * n_points + n;  // feature k at out[k * n_points]
         const float w_level = window[level];
+        uint32_t here = 0u;
+        if constexpr (kChosen) here = chosen[level];  // (before it is waited for)
         if (w_level == 0.0f) {
             static_for<F>(PENC_BODY(k) {
                 PENC_INDEX(k); out[static_cast<size_t>(k) * n_points] = 0.0f; });
@@ -197,8 +201,16 @@ forward_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uint3
         fvec<D + 1> sorted;
         sort_by_rank_lds<D>(columns + threadIdx.x, kBlock, s.rank, s.delta, s.hash0, sorted, h);
         const fvec<D + 1> w = barycentric_of_sorted<D>(sorted);
-        const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
-                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
+        const T* slice = table;
+        if constexpr (kChosen) {
+            if (here != 0u) {
+                slice = cells;
+                h = hashes_in_cells<D, line_slots<F, T>()>(h);
+            }
+        } else {
+            h = hashes_in_copy<D, F, T>(in_cells, h);
+        }
+        const Vertices<D, F> v = load_vertices<D, F, T>(slice + static_cast<size_t>(level) * capacity * F, h, capacity, cap_mask);
         fvec<F> acc = 0.0f;
         static_for<D + 1>(PENC_BODY(r) {
             PENC_INDEX(r);
@@ -267,7 +279,7 @@ backward_pos_kernel(int n_points, int n_levels, int per_group, LevelMap map, uin
         const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
         const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
         const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
-                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
+                                                         hashes_in_copy<D, F, T>(in_cells, h), capacity, cap_mask);
         const float* gp = grad_sliced + (static_cast<size_t>(level) * F) * n_points + n;
         // the upstream gradient is read once (non-temporal: it should not displace the table slices)
         fvec<D + 1> dB = (v.f[0] * w_level) * __builtin_nontemporal_load(gp);  // :688-689, feature by feature
@@ -351,7 +363,7 @@ grad_grad_kernel(int n_points, int n_levels, int n_all_levels, LevelMap map, uin
         fvec<D + 1> sorted;
         sort_by_rank_lds<D>(columns + threadIdx.x, kBlock, s.rank, pos_grad_grad_to_elevated<D>(q, sf), s.hash0, sorted, h);
         const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
-                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
+                                                         hashes_in_copy<D, F, T>(in_cells, h), capacity, cap_mask);
         // dB[r] * w_level, then times the vertex value (:1484-1485)
         const fvec<D + 1> wr = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
         fvec<F> gg = 0.0f;
@@ -407,7 +419,7 @@ block_backward_pos_kernel(int n_points, int n_levels, uint32_t capacity, uint32_
         const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
         const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
         const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
-                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
+                                                         hashes_in_copy<D, F, T>(in_cells, h), capacity, cap_mask);
         const auto upstream = [&](int k) {
             if constexpr (kRows) return tile[row * pitch + level * F + k];
             else return grad[(static_cast<size_t>(level) * F + k) * n_points + n];
@@ -468,7 +480,7 @@ block_rows_kernel(int n_points, int n_levels, int n_all_levels, uint32_t capacit
             const Located<D> s = locate<D>(pos, random_shift + level * D, sf);
             const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
             const Vertices<D, F> v = load_vertices<D, F, T>(table + static_cast<size_t>(level) * capacity * F,
-                                                         hashes_in_cells<D, line_slots<F, T>()>(in_cells, h), capacity, cap_mask);
+                                                         hashes_in_copy<D, F, T>(in_cells, h), capacity, cap_mask);
             const fvec<D + 1> w = kSecond ? pos_grad_grad_to_bary<D>(s.rank, q, sf) * w_level : barycentric<D>(s.rank, s.delta) * w_level;
             static_for<D + 1>(PENC_BODY(r) {
                 PENC_INDEX(r);
@@ -820,7 +832,7 @@ inline bool cells_possible(int nr_feat, int capacity, int format) {
 inline int strip_cells(int table_format) { return table_format & ~PENC_TABLE_CELLS; }
 inline bool known_format(int table_format) {
     const int format = strip_cells(table_format);
-    return format == 0 || format == PENC_TABLE_FP16 || format == PENC_TABLE_BF16;
+    return table_format == 0 || format == PENC_TABLE_FP16 || format == PENC_TABLE_BF16;
 }
 inline bool known_half_format(int table_format) { return known_format(table_format) && strip_cells(table_format) != 0; }
 // (nr_feat is checked by the caller's check_geometry: whatever it refuses is none of this function's)
@@ -1479,10 +1491,16 @@ static int backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
     return PENC_OK;
 }
 
+// The levels of an fp32 table that a forward gathers from cells made for it (chosen_columns_kernel).
+struct ChosenCells {
+    const void* cells = nullptr;
+    const uint32_t* levels = nullptr;
+};
+
 static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity,
                         const float* positions, const TableRef& table, const float* scale_factor,
                         const float* random_shift, const float* anneal_window, float* sliced_values,
-                        int concat_points, float points_scaling, void* stream, float* slopes = nullptr) {
+                        int concat_points, float points_scaling, void* stream, float* slopes = nullptr, const ChosenCells& chosen = {}) {
     const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points);
     if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
     if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values)
@@ -1492,16 +1510,25 @@ static int forward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_l
     const GatherLaunch g = plan_gather(nr_positions, nr_levels, gather_levels_per_thread(pos_dim, nr_positions, nr_levels),
                                        slice_bytes(capacity, nr_feat, table.format));
     const uint32_t in_cells = table.cells ? 1u : 0u;
-#define PENC_LAUNCH_FORWARD(SLOPES)                                                                                                      \
-    PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format,                                                                                   \
-                      hipLaunchKernelGGL((forward_kernel<DD, FF, TT, SLOPES>), g.grid, dim3(kBlock), 0, st,                             \
-                                         static_cast<int>(nr_positions), nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity), \
-                                         mask_of(capacity), in_cells, positions, static_cast<const TT*>(table.values), scale_factor,              \
-                                         random_shift, anneal_window, sliced_values, points_scaling, slopes))
-    if (slopes != nullptr) {
-        PENC_LAUNCH_FORWARD(true);
+#define PENC_LAUNCH_FORWARD(FEAT, TYPE, SLOPES, CHOSEN)                                                                                  \
+    hipLaunchKernelGGL((forward_kernel<DD, FEAT, TYPE, SLOPES, CHOSEN>), g.grid, dim3(kBlock), 0, st, static_cast<int>(nr_positions),     \
+                       nr_levels, nr_levels + extra, g.map, static_cast<uint32_t>(capacity), mask_of(capacity), in_cells, positions,     \
+                       static_cast<const TYPE*>(table.values), scale_factor, random_shift, anneal_window, sliced_values, points_scaling, \
+                       slopes, static_cast<const TYPE*>(chosen.cells), chosen.levels)
+    if (chosen.levels != nullptr) {  // (two or four features)
+        if (nr_feat == 4 && slopes != nullptr) {
+            PENC_DISPATCH_D(pos_dim, PENC_LAUNCH_FORWARD(4, float, true, true))
+        } else if (nr_feat == 4) {
+            PENC_DISPATCH_D(pos_dim, PENC_LAUNCH_FORWARD(4, float, false, true))
+        } else if (slopes != nullptr) {
+            PENC_DISPATCH_D(pos_dim, PENC_LAUNCH_FORWARD(2, float, true, true))
+        } else {
+            PENC_DISPATCH_D(pos_dim, PENC_LAUNCH_FORWARD(2, float, false, true))
+        }
+    } else if (slopes != nullptr) {
+        PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format, PENC_LAUNCH_FORWARD(FF, TT, true, false));
     } else {
-        PENC_LAUNCH_FORWARD(false);
+        PENC_DISPATCH_DFT(pos_dim, nr_feat, table.format, PENC_LAUNCH_FORWARD(FF, TT, false, false));
     }
 #undef PENC_LAUNCH_FORWARD
     return check_launch();
@@ -1943,37 +1970,26 @@ static bool slopes_in_point_blocks(int pos_dim, int64_t n, int levels, int capac
            (pos_dim <= 6 || n * levels * (pos_dim + 1) <= kBlocksMidMaxGathers);
 }
 
-int penc_forward_table(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
-                       const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
-                       const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
-                       int concat_points, float points_scaling, void* stream) {
+int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                        const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
+                        const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
+                        int concat_points, float points_scaling, void* stream) {
     if (!known_format(table_format) || !cells_fit(table_format, nr_feat, capacity)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!slopes) return PENC_ERR_NULL_POINTER;
     const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points), cols = nr_feat * (nr_levels + extra);
     if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
     const TableRef table = table_ref(lattice_values, table_format);
-    if (sliced_rows != nullptr &&
-        (slopes != nullptr ? slopes_in_point_blocks : takes_point_blocks)(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format)) {
+    if (sliced_rows != nullptr && slopes_in_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, cols, table.format)) {
         if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
         if (!positions || !table.values || !scale_factor || !random_shift || !anneal_window || !sliced_values) return PENC_ERR_NULL_POINTER;
         if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
-        return (slopes != nullptr ? block_rows<true, false> : block_rows<false, false>)(
-            pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift, anneal_window, nullptr,
-            points_scaling, sliced_rows, row_stride, slopes, static_cast<hipStream_t>(stream));
+        return block_rows<true, false>(pos_dim, nr_feat, nr_positions, nr_levels, extra, capacity, positions, table, scale_factor, random_shift,
+                                       anneal_window, nullptr, points_scaling, sliced_rows, row_stride, slopes, static_cast<hipStream_t>(stream));
     }
     if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor,
                               random_shift, anneal_window, sliced_values, concat_points, points_scaling, stream, slopes))
         return rc;
     return sliced_rows == nullptr ? PENC_OK : transpose_to_rows(sliced_values, sliced_rows, row_stride, nr_positions, cols, static_cast<hipStream_t>(stream));
-}
-
-int penc_forward_slopes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
-                        const void* lattice_values, int table_format, const float* scale_factor, const float* random_shift,
-                        const float* anneal_window, float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes,
-                        int concat_points, float points_scaling, void* stream) {
-    if (!known_format(table_format)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
-    if (!slopes) return PENC_ERR_NULL_POINTER;
-    return penc_forward_table(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, lattice_values, table_format, scale_factor,
-                              random_shift, anneal_window, sliced_values, sliced_rows, row_stride, slopes, concat_points, points_scaling, stream);
 }
 
 static size_t slope_tile_bytes(int columns) { return static_cast<size_t>(kSlopeTile) * (columns | 1) * sizeof(float); }
@@ -2155,7 +2171,7 @@ constexpr size_t kCellChunkBytes = size_t{128} << 20;
 
 size_t penc_table_cells_workspace_bytes(int nr_feat, int nr_levels, int capacity, int table_format) {
     if ((nr_feat != 2 && nr_feat != 4 && nr_feat != 8) || nr_levels <= 0 || capacity <= 0) return 0;
-    if (strip_cells(table_format) != table_format || !known_format(table_format) || !cells_possible(nr_feat, capacity, table_format)) return 0;
+    if (strip_cells(table_format) != table_format || !known_half_format(table_format) || !cells_possible(nr_feat, capacity, table_format)) return 0;
     const size_t slice = slice_bytes(capacity, nr_feat, table_format);
     size_t levels = kCellChunkBytes / slice;
     if (levels < 1) levels = 1;
@@ -2181,7 +2197,7 @@ int64_t penc_table_cells_points(int nr_feat, int capacity, int table_format) {
 int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, const void* lattice_values, int source_format, int table_format,
                      void* cells, void* workspace, size_t workspace_bytes, void* stream) {
     if (int rc = check_geometry(pos_dim, nr_feat, 1, nr_levels, capacity, 0)) return rc;
-    if (strip_cells(table_format) != table_format || !known_format(table_format) || !cells_possible(nr_feat, capacity, table_format) ||
+    if (strip_cells(table_format) != table_format || !known_half_format(table_format) || !cells_possible(nr_feat, capacity, table_format) ||
         (source_format != 0 && source_format != table_format))
         return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
     if (!lattice_values || !cells) return PENC_ERR_NULL_POINTER;
@@ -2205,9 +2221,7 @@ int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, cons
     if (nr_feat == 2) PENC_LAUNCH_COLUMNS(2, T_, RAW_);      \
     else if (nr_feat == 4) PENC_LAUNCH_COLUMNS(4, T_, RAW_); \
     else PENC_LAUNCH_COLUMNS(8, T_, RAW_)
-        if (table_format == 0) {
-            PENC_LAUNCH_COLUMNS_OF(float, true);
-        } else if (source_format != 0) {
+        if (source_format != 0) {
             PENC_LAUNCH_COLUMNS_OF(bfloat16_bits, true);  // (either format: the bits are moved)
         } else if (table_format == PENC_TABLE_BF16) {
             PENC_LAUNCH_COLUMNS_OF(bfloat16_bits, false);
@@ -2220,12 +2234,78 @@ int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, cons
         switch (kLineBytes / slots / 4) {
             case 1: hipLaunchKernelGGL(cell_lines_kernel<1>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
             case 2: hipLaunchKernelGGL(cell_lines_kernel<2>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
-            case 4: hipLaunchKernelGGL(cell_lines_kernel<4>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
-            default: hipLaunchKernelGGL(cell_lines_kernel<8>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
+            default: hipLaunchKernelGGL(cell_lines_kernel<4>, grid, dim3(kCellBlock), 0, st, columns, lines, map, to); break;
         }
         if (int rc = check_launch()) return rc;
     }
     return PENC_OK;
+}
+
+// Where one forward is worth a copy of the fp32 table in cells: from 16 M points times levels on (the copy's launch takes 5 us, all that is to be
+// lost), on levels of 64 KiB to 2 MiB with at most a slot for every two or three points.  Forward without -> with, us, two features, finest scale
+// 1e-4 / 1e-3 / 1e-2:
+//   D = 3, 24 levels, 2^20 points   2^18 slots, unordered 280 -> 237, 261 -> 206, 171 -> 170   along rays 179 -> 175, 132 -> 137, 111 -> 116
+//                                   2^19 slots 360 -> 375, 286 -> 299, 173 -> 203 (an L2 holds no such level beside what it gathers)
+//          2^19 points              2^14 slots 122 -> 103   2^16 138 -> 119   2^17 141 -> 125   along rays, 1e-2, 2^14 55 -> 63
+//   16 levels, 1e-3, 2^18 slots     D = 2 115 -> 101   D = 4 230 -> 204   D = 5 291 -> 277   D = 6 337 -> 325   D = 7 387 -> 376   (D = 8, 2^19 271 -> 309)
+// Four features, D = 3, 16 levels: 2^14 slots 163 -> 144, 2^16 176 -> 152, 2^17 179 -> 172, 2^18 217 -> 235; eight: 2^16 243 -> 267.
+constexpr int64_t kForwardCellsMinWork = 16000000;
+constexpr size_t kForwardCellsMaxSlice = size_t{2} << 20;
+static bool forward_cells_serve(int pos_dim, int nr_feat, int64_t n, int levels, int capacity) {
+    if (pos_dim > 7 || nr_feat == 8 || !cells_possible(nr_feat, capacity, 0) || n * levels < kForwardCellsMinWork) return false;
+    const size_t slice = slice_bytes(capacity, nr_feat, 0);
+    return slice >= (size_t{64} << 10) && slice <= kForwardCellsMaxSlice && slice <= static_cast<size_t>(n) * 3;
+}
+// What the workspace holds: the flags of the levels, then the copy.
+static size_t forward_cells_flags(int levels) { return (static_cast<size_t>(levels) * sizeof(uint32_t) + 255u) & ~size_t{255}; }
+
+size_t penc_forward_cells_workspace_bytes(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, int row_columns) {
+    if (check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, 0) != PENC_OK) return 0;
+    // (rows that a workgroup of 64 points and all levels writes need no transpose)
+    if (row_columns != 0 && takes_point_blocks(pos_dim, nr_positions, nr_levels, capacity, nr_feat, row_columns, 0)) return 0;
+    if (!forward_cells_serve(pos_dim, nr_feat, nr_positions, nr_levels, capacity)) return 0;
+    return forward_cells_flags(nr_levels) + slice_bytes(capacity, nr_feat, 0) * static_cast<size_t>(nr_levels) + 256;
+}
+
+int penc_forward_cells(int pos_dim, int nr_feat, int64_t nr_positions, int nr_levels, int capacity, const float* positions,
+                       const float* lattice_values, const float* scale_factor, const float* random_shift, const float* anneal_window,
+                       float* sliced_values, float* sliced_rows, int64_t row_stride, float* slopes, int concat_points, float points_scaling,
+                       void* workspace, size_t workspace_bytes, void* stream) {
+    const int extra = penc_extra_levels(pos_dim, nr_feat, concat_points), cols = nr_feat * (nr_levels + extra);
+    if (int rc = check_geometry(pos_dim, nr_feat, nr_positions, nr_levels, capacity, extra)) return rc;
+    if (sliced_rows != nullptr && (cols > 255 || row_stride < cols || row_stride * nr_positions >= (int64_t{1} << 31))) return PENC_ERR_BAD_SIZE;
+    if (nr_feat == 8 || !cells_possible(nr_feat, capacity, 0)) return PENC_ERR_UNSUPPORTED_TABLE_FORMAT;
+    if (!positions || !lattice_values || !scale_factor || !random_shift || !anneal_window || !sliced_values) return PENC_ERR_NULL_POINTER;
+    const TableRef table{lattice_values, 0};
+    if (!table_aligned(table, nr_feat)) return PENC_ERR_MISALIGNED;
+    const size_t flags = forward_cells_flags(nr_levels);
+    const uintptr_t base = (reinterpret_cast<uintptr_t>(workspace) + 255u) & ~uintptr_t{255};
+    if (workspace == nullptr || workspace_bytes < (base - reinterpret_cast<uintptr_t>(workspace)) + flags +
+                                                      slice_bytes(capacity, nr_feat, 0) * static_cast<size_t>(nr_levels))
+        return PENC_ERR_WORKSPACE_TOO_SMALL;
+    uint32_t* const chosen = reinterpret_cast<uint32_t*>(base);
+    float* const cells = reinterpret_cast<float*>(base + flags);
+    const int slots = slots_per_line(nr_feat, 0);
+    const uint32_t lines = static_cast<uint32_t>(capacity / slots), levels = static_cast<uint32_t>(nr_levels), dies = dies_of_current_device();
+    const uint32_t per_level = (lines + kCellLines * kCellsPerWorkgroup - 1) / (kCellLines * kCellsPerWorkgroup);
+    const CellMap map = cell_map(pos_dim, slots);
+    const dim3 grid(dies * per_level * ((levels + dies - 1) / dies));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+#define PENC_LAUNCH_CHOSEN(F_)                                                                                                              \
+    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((chosen_cells_kernel<DD, F_>), grid, dim3(kCellBlock), 0, st, lattice_values, lines, levels, \
+                                                per_level, dies, map, nr_positions, positions, scale_factor, random_shift, anneal_window,    \
+                                                chosen, cells))
+    if (nr_feat == 4) {
+        PENC_LAUNCH_CHOSEN(4);
+    } else {
+        PENC_LAUNCH_CHOSEN(2);
+    }
+#undef PENC_LAUNCH_CHOSEN
+    if (int rc = check_launch()) return rc;
+    if (int rc = forward_impl(pos_dim, nr_feat, nr_positions, nr_levels, capacity, positions, table, scale_factor, random_shift, anneal_window,
+                              sliced_values, concat_points, points_scaling, stream, slopes, ChosenCells{cells, chosen}))
+        return rc;
+    return sliced_rows == nullptr ? PENC_OK : transpose_to_rows(sliced_values, sliced_rows, row_stride, nr_positions, cols, st);
 }
 
 int penc_upload(const float* host_values, float* dst, int n, void* stream) {

@@ -82,6 +82,8 @@ struct Api {
     PENC_FN(backward_positions_rowmajor);
     PENC_FN(grad_grad_rowmajor);
     PENC_FN(slopes_bytes);
+    PENC_FN(forward_cells);
+    PENC_FN(forward_cells_workspace_bytes);
     PENC_FN(table_cells);
     PENC_FN(table_cells_workspace_bytes);
     PENC_FN(forward_slopes);
@@ -416,6 +418,26 @@ public:
 // ------------------------------------------------------------------------------------------
 // the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
 
+// The forward by way of a copy of the table in cells, where that pays and there is memory for it; false: not done.  `rows` is undefined where
+// the result is `level_major`, which else is scratch and may be undefined; `slopes` where none are kept.
+bool forward_in_cells(const Call& c, Tensor level_major, const Tensor& rows, const Tensor& slopes) {
+    if (c.table_format != 0) return false;
+    const size_t n = api.forward_cells_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, rows.defined() ? static_cast<int>(c.columns()) : 0);
+    if (n == 0) return false;
+    Tensor ws;
+    try {
+        if (!level_major.defined()) level_major = level_major_array(c);
+        ws = bytes(c, n);
+    } catch (const c10::OutOfMemoryError&) {
+        return false;
+    }
+    check(api.forward_cells(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor), data(c.shift),
+                            data(c.window), mutable_data(level_major), mutable_data(rows), c.columns(), mutable_data(slopes), c.concat, c.scaling,
+                            ws.mutable_data_ptr(), n, current_stream(c.device())),
+          "forward_cells");
+    return true;
+}
+
 // With `slopes` the forward leaves them behind; where their memory is refused, it is reset and the forward is the one without.
 Tensor compute_forward(const Call& c, std::shared_ptr<Slopes>& slopes) {
     void* const stream = current_stream(c.device());
@@ -430,14 +452,16 @@ Tensor compute_forward(const Call& c, std::shared_ptr<Slopes>& slopes) {
             slopes.reset();
         }
         if (slopes != nullptr) {
-            check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
-                                     data(c.scale_factor), data(c.shift), data(c.window), mutable_data(level_major),
-                                     as_rows ? mutable_data(out) : nullptr, c.columns(), mutable_data(kept), c.concat, c.scaling, stream),
-                  "forward_slopes");
+            if (!forward_in_cells(c, level_major, as_rows ? out : Tensor(), kept))
+                check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
+                                         data(c.scale_factor), data(c.shift), data(c.window), mutable_data(level_major),
+                                         as_rows ? mutable_data(out) : nullptr, c.columns(), mutable_data(kept), c.concat, c.scaling, stream),
+                      "forward_slopes");
             slopes->keep(std::move(kept));
             return out;
         }
     }
+    if (as_rows ? forward_in_cells(c, {}, out, {}) : forward_in_cells(c, out, {}, {})) return out;
     if (as_rows) {
         const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
         check(api.forward_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
@@ -1106,6 +1130,8 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(backward_positions_rowmajor);
         PENC_FN(grad_grad_rowmajor);
         PENC_FN(slopes_bytes);
+        PENC_FN(forward_cells);
+        PENC_FN(forward_cells_workspace_bytes);
         PENC_FN(table_cells);
         PENC_FN(table_cells_workspace_bytes);
         PENC_FN(forward_slopes);

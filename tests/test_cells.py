@@ -4,13 +4,13 @@ import pytest
 import torch
 
 CELLS = 0x100
-HALF = {0: torch.float32, 1: torch.float16, 2: torch.bfloat16}
+HALF = {1: torch.float16, 2: torch.bfloat16}
 
 
 def make_cells(table, pos_dim, fmt, workspace_levels=None):
     from permutohedral_encoding_amd import _native
     lib, (levels, cap, feat) = _native.lib(), table.shape
-    source = {v: k for k, v in HALF.items()}[table.dtype]
+    source = 0 if table.dtype == torch.float32 else fmt
     cells = torch.full((levels, cap, feat), float("nan"), dtype=HALF[fmt], device="cuda")
     nbytes = lib.penc_table_cells_workspace_bytes(feat, levels, cap, fmt)
     if workspace_levels is not None:
@@ -22,7 +22,7 @@ def make_cells(table, pos_dim, fmt, workspace_levels=None):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("feat", [2, 4, 8])
 @pytest.mark.parametrize("d", range(2, 9))
 def test_every_gather_from_cells_equals_the_gather_from_the_table(d, feat, fmt):
@@ -30,7 +30,7 @@ def test_every_gather_from_cells_equals_the_gather_from_the_table(d, feat, fmt):
     one; results bit for bit, from workgroups of 64 points and all levels and from launches a level at a time."""
     from helpers import make_encoding, random_problem, to_gpu
     from permutohedral_encoding_amd import _native
-    line = 128 // (feat * (2 if fmt else 4))
+    line = 128 // (feat * 2)
     lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
     for cap, levels, n in ((line, 3, 100), (2 * line, 3, 65), (64 * line, 5, 1003), (128 * line, 5, 1003), (1 << 14, 5, 2001), (1 << 18, 24 // feat * 2, 30001)):
         p = random_problem(d, n, levels, cap, seed=d, sigma_range=(1.0, 1e-3), nr_feat=feat)
@@ -50,12 +50,11 @@ def test_every_gather_from_cells_equals_the_gather_from_the_table(d, feat, fmt):
             common = (d, feat, n, levels, cap, pos.data_ptr(), values.data_ptr(), table_format, sf, shift, win.data_ptr())
             out, as_rows, positions_grad = torch.empty(cols, n, device="cuda"), torch.empty(n, cols, device="cuda"), torch.empty(n, d, device="cuda")
             slopes = torch.zeros(levels * -(-n // 64) * 64 * d * feat, device="cuda")
-            got = []
-            for keep in (None, slopes.data_ptr()):
-                for to_rows in (None, as_rows.data_ptr()):
-                    assert lib.penc_forward_table(*common, out.data_ptr(), to_rows, cols, keep, 0, 1.0, st) == 0
-                    got += [out.clone(), as_rows.clone()] if to_rows is None else [as_rows.clone()]
-            got = [got[0], got[2], got[3], got[5], slopes]
+            assert lib.penc_forward_half(*common, out.data_ptr(), 0, 1.0, st) == 0
+            got = [out.clone()]
+            for to_rows in (None, as_rows.data_ptr()):
+                assert lib.penc_forward_slopes(*common, out.data_ptr(), to_rows, cols, slopes.data_ptr(), 0, 1.0, st) == 0
+                got += [slopes.clone(), out.clone() if to_rows is None else as_rows]
             level_major = torch.empty(cols, n, device="cuda")
             assert lib.penc_backward_positions_rowmajor(*common, rows.data_ptr(), cols, level_major.data_ptr(), positions_grad.data_ptr(),
                                                         ws.data_ptr(), ws.numel(), st) == 0
@@ -63,13 +62,11 @@ def test_every_gather_from_cells_equals_the_gather_from_the_table(d, feat, fmt):
             grad_grad = torch.empty(n, cols, device="cuda")
             assert lib.penc_grad_grad_rowmajor(*common, dpos.data_ptr(), grad_grad.data_ptr(), cols, 0, ws.data_ptr(), ws.numel(), st) == 0
             got.append(grad_grad)
-            if table_format != 0 and table_format != CELLS:
-                out2, positions_grad2, grad_grad2 = torch.empty(cols, n, device="cuda"), torch.empty(n, d, device="cuda"), torch.empty(cols, n, device="cuda")
-                assert lib.penc_forward_half(*common, out2.data_ptr(), 0, 1.0, st) == 0
-                assert lib.penc_backward_half(*common, grad.data_ptr(), 0, None, positions_grad2.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
-                assert lib.penc_double_backward_from_positions_half(*common, dpos.data_ptr(), grad.data_ptr(), 0, None, grad_grad2.data_ptr(), 0,
-                                                                    ws.data_ptr(), ws.numel(), st) == 0
-                got += [out2, positions_grad2, grad_grad2]
+            positions_grad2, grad_grad2 = torch.empty(n, d, device="cuda"), torch.empty(cols, n, device="cuda")
+            assert lib.penc_backward_half(*common, grad.data_ptr(), 0, None, positions_grad2.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
+            assert lib.penc_double_backward_from_positions_half(*common, dpos.data_ptr(), grad.data_ptr(), 0, None, grad_grad2.data_ptr(), 0,
+                                                                ws.data_ptr(), ws.numel(), st) == 0
+            got += [positions_grad2, grad_grad2]
             return got
 
         for k, (want, got) in enumerate(zip(results(plain, fmt), results(cells, fmt | CELLS))):
@@ -93,19 +90,31 @@ def test_cells_are_refused_where_they_are_not_possible():
     import ctypes
     from permutohedral_encoding_amd import _native
     lib, p = _native.lib(), ctypes.c_void_p(1 << 20)
-    assert lib.penc_table_cells_workspace_bytes(2, 4, 32, 1) > 0 and lib.penc_table_cells_workspace_bytes(2, 4, 16, 0) > 0
-    for feat, cap, fmt in ((2, 16, 1), (2, 8, 0), (2, 1000, 0), (8, 4, 1), (3, 64, 0), (2, 64, 3), (2, 64, 1 | CELLS)):
-        assert lib.penc_table_cells_workspace_bytes(feat, 4, cap, fmt) == 0
+    assert lib.penc_table_cells_workspace_bytes(2, 4, 32, 1) > 0 and lib.penc_table_cells_workspace_bytes(8, 4, 8, 2) > 0
+    for feat, cap, fmt in ((2, 16, 1), (2, 64, 0), (2, 1000, 2), (8, 4, 1), (3, 64, 1), (2, 64, 3), (2, 64, 1 | CELLS)):
+        assert lib.penc_table_cells_workspace_bytes(feat, 4, cap, fmt) == 0 and lib.penc_table_cells_points(feat, cap, fmt) == -1
         assert lib.penc_table_cells(3, feat, 4, cap, p, 0, fmt, p, p, 1 << 20, None) != 0
-    for cap, fmt in ((16, 1), (1000, 1), (8, 0), (1000, 0)):  # neither is a table said to be in cells
-        assert lib.penc_forward_table(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, None, 0, None, 0, 1.0, None) == 9
-        if fmt:
-            assert lib.penc_forward_half(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, 0, 1.0, None) == 9
-    assert lib.penc_forward_half(3, 2, 10, 4, 64, p, p, CELLS, p, p, p, p, 0, 1.0, None) == 9
+    for cap, fmt in ((16, 1), (1000, 2), (64, 0)):  # neither is a table said to be in cells
+        assert lib.penc_forward_slopes(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, None, 0, p, 0, 1.0, None) == 9
+        assert lib.penc_forward_half(3, 2, 10, 4, cap, p, p, fmt | CELLS, p, p, p, p, 0, 1.0, None) == 9
     assert lib.penc_table_cells(3, 2, 4, 64, p, 1, 2, p, p, 1 << 20, None) == 9
     assert lib.penc_table_cells(3, 2, 4, 64, None, 0, 1, p, p, 1 << 20, None) == 1
     assert lib.penc_table_cells(3, 2, 4, 64, p, 0, 1, ctypes.c_void_p((1 << 20) + 8), p, 1 << 20, None) == 5
     assert lib.penc_table_cells(3, 2, 4, 64, p, 0, 1, p, p, 64, None) == 8
+    for feat, cap, bad in ((8, 64, 9), (2, 8, 9), (2, 1000, 9)):
+        assert lib.penc_forward_cells(3, feat, 10, 4, cap, p, p, p, p, p, p, None, 0, None, 0, 1.0, p, 1 << 20, None) == bad
+    assert lib.penc_forward_cells(3, 2, 10, 4, 64, p, None, p, p, p, p, None, 0, None, 0, 1.0, p, 1 << 20, None) == 1
+    assert lib.penc_forward_cells(3, 2, 10, 4, 64, p, p, p, p, p, p, None, 0, None, 0, 1.0, p, 64, None) == 8
+    assert lib.penc_forward_cells(3, 2, 10, 4, 64, p, p, p, p, p, p, p, 7, None, 0, 1.0, p, 1 << 20, None) == 2  # rows of seven floats
+
+
+def test_where_a_forward_goes_by_way_of_cells():
+    from permutohedral_encoding_amd import _native
+    serves = lambda *geometry: _native.lib().penc_forward_cells_workspace_bytes(*geometry) > 0
+    assert serves(3, 2, 1 << 20, 24, 1 << 18, 0) and serves(3, 2, 1 << 20, 24, 1 << 18, 48) and not serves(3, 8, 1 << 20, 24, 1 << 14, 0)
+    assert not serves(8, 2, 1 << 20, 24, 1 << 18, 0) and not serves(3, 2, 1 << 20, 24, 1 << 19, 0) and not serves(3, 2, 1 << 20, 24, 200000, 0)
+    assert not serves(3, 2, 1 << 18, 24, 1 << 14, 0) and not serves(3, 2, 1 << 20, 24, 1 << 12, 0)
+    assert serves(3, 2, 1 << 20, 24, 1 << 14, 0) and not serves(3, 2, 1 << 20, 24, 1 << 14, 48)  # rows without a transpose
 
 
 def test_cells_cover_the_lattice_once():
@@ -200,3 +209,40 @@ def test_module_gathers_from_cells_once_enough_points_were_gathered(d, feat, cap
             assert torch.equal(m(many), plain(many)) and m.lattice._cells is None
     finally:
         _native._bridge = _native_bridge
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("feat", [2, 4])
+@pytest.mark.parametrize("d", range(2, 9))
+def test_forward_by_way_of_cells_equals_the_forward(d, feat):
+    """Levels that are chosen for the copy and levels that are not in one call, a masked one among them, fewer levels than dies and more, one line,
+    part of a workgroup's and several workgroups' lines, a batch of one point and one that ends in the middle of a wave; level by level, in rows,
+    with and without slopes."""
+    from helpers import make_encoding, random_problem, to_gpu
+    from permutohedral_encoding_amd import _native
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    line, kinds = 128 // (4 * feat), set()
+    for cap, levels, n, finest in ((line, 2, 1, 1e-3), (4 * line, 3, 65, 1e-3), (1 << 14, 6, 5003, 1e-4), (1 << 16, 19, 3001, 1e-4)):
+        p = random_problem(d, n, levels, cap, seed=d, sigma_range=(1.0, finest), nr_feat=feat)
+        p["window"][levels // 3] = 0.0
+        _, fp = make_encoding(d, p["sigmas"], p["shift"], nr_feat=feat)
+        table, pos, win = to_gpu(p["table"]), to_gpu(p["pos"]), to_gpu(p["window"])
+        cols, slope_floats = feat * levels, levels * -(-n // 64) * 64 * d * feat
+        nbytes = 512 + cap * feat * 4 * levels
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        common = (d, feat, n, levels, cap, pos.data_ptr(), table.data_ptr())
+        geometry = (fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(), win.data_ptr())
+        want, kept = torch.empty(cols, n, device="cuda"), torch.zeros(slope_floats, device="cuda")
+        assert lib.penc_forward_slopes(*common, 0, *geometry, want.data_ptr(), None, 0, kept.data_ptr(), 0, 1.0, st) == 0
+        for as_rows in (False, True):
+            for keep in (False, True):
+                out, rows, slopes = torch.zeros(cols, n, device="cuda"), torch.zeros(n, cols, device="cuda"), torch.zeros(slope_floats, device="cuda")
+                assert lib.penc_forward_cells(*common, *geometry, out.data_ptr(), rows.data_ptr() if as_rows else None, cols,
+                                              slopes.data_ptr() if keep else None, 0, 1.0, ws.data_ptr(), nbytes, st) == 0
+                assert torch.equal(rows.t() if as_rows else out, want)
+                assert not keep or torch.equal(slopes, kept)
+                first = (ws.data_ptr() + 255) // 256 * 256 - ws.data_ptr()
+                chosen = ws[first:first + 4 * levels].view(torch.int32)
+                assert chosen[levels // 3] == 0
+                kinds.update(chosen.tolist())
+    assert kinds == {0, 1}
