@@ -1341,7 +1341,8 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
         t.grid = dim3(padded_groups * static_cast<unsigned>(count));
-        t.many_bins = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins;
+        t.many_bins = plan.target.records != nullptr && plan.target.n_bins > static_cast<uint32_t>(kStageBins);
+        t.most_bins = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins;
         t.wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
         t.first_level = first;
         t.n_pass_levels = static_cast<uint32_t>(count);

@@ -149,6 +149,15 @@ __device__ __forceinline__ void store_record(const BinTarget& bins, uint32_t i, 
     }
 }
 
+// Writes a staged record {slot in its bin, values, index of the record in the level's array}, where records are whole.
+__device__ __forceinline__ void store_whole_record(const BinTarget& bins, uint4 e) {
+    BinRecord rec;
+    rec.slot_in_bin = e.x;
+    rec.a0 = __builtin_bit_cast(float, e.y);
+    rec.a1 = __builtin_bit_cast(float, e.z);
+    *reinterpret_cast<BinRecord*>(static_cast<char*>(bins.records) + e.w * static_cast<uint32_t>(sizeof(BinRecord))) = rec;
+}
+
 // Record `i` of a bin whose first record is `first` (of the level's arrays), with ordinary loads.
 template <bool kSplit>
 __device__ __forceinline__ BinRecord load_record(const BinTarget& bins, size_t first, uint32_t i) {
@@ -461,10 +470,9 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 
 // Stage 2 for a whole tile once the workgroup streams (see scatter_mode_decide): the cache's LDS is
 // staging space for a counting sort of the tile's records by bin, all vertices at a time
-// (1536 to 3072 records of 512 threads).  Every wave counts its records per bin (one LDS counter per
-// bin and wave); then every wave, lane b looking after bin b, turns all waves' counts into the offsets of its own runs (a bin's run is the
-// waves' runs one after the other) and lays its records out in that order in the staging space; and then all
-// threads store the records in staging order: a wave instruction writes 64 consecutive records
+// (1536 to 3072 records of 512 threads).  The workgroup counts its records per bin; then every wave, lane b looking after bin b, turns the
+// counts into where each bin's run starts in the staging space and in the workgroup's segment, and lays its records out in that order;
+// and then all threads store the records in staging order: a wave instruction writes 64 consecutive records
 // of (mostly) one bin, i.e. whole cache lines, where the records of a single wave would leave in
 // runs of eight.  How far the workgroup's segment of a bin is filled (`cursor`, lane b's is bin b's) every wave
 // knows from the same sums.  (With the offsets made by the first wave for all, and a cursor in LDS, the others waited for it at a
@@ -473,83 +481,117 @@ __device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
 // A staged record carries its destination (its index in the level's record
 // array), so the store needs no search.  When a run does not fit its segment any more (rare: the
 // segments hold the mean plus three standard deviations) the tile checks every record against
-// the room left and sends the excess to stage 3.
-// Needs bins.n_bins <= kStageBins and a level's record array below 2^32 bytes (the host plans
-// for both); all threads of the workgroup must call it together.
+// the room left and sends the excess to stage 3, in code of its own: without a branch in them, a thread's trips to the LDS
+// for its D+1 records are made together, not one after the other.
+// Two arrays of counters take turns (`tile` says which): the other one is cleared between this tile's barriers.  Both are
+// zero before the first tile.
+// Needs bins.n_bins <= kStageBins, split records and a level's record array below 2^32 bytes (the host plans
+// for all three); all threads of the workgroup must call it together.
 template <int D, typename State>
 __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_grad, const BinTarget& bins,
-                                            uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
+                                            uint32_t group, uint32_t tile, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
                                             fvec<D + 1> a1, uint32_t& cursor) {
     constexpr int kWaves = State::kThreads / 64;
     constexpr int kStageChunk = State::kChunk;
     static_assert(D + 1 <= kStageChunk, "all vertices of a tile are staged at a time");
-    static_assert(kCacheLines >= 3 * kWaves * 64, "the sort's index arrays live in the tag array");
+    static_assert(kCacheLines >= 2 * kStageBins + 2 * kWaves * kStageBins, "the sort's index arrays live in the tag array");
     static_assert(offsetof(State, stage_tail) == offsetof(State, val) + sizeof(c.val) &&
                       (sizeof(c.val) + (State::kTail > 0 ? sizeof(c.stage_tail) : 0)) == kStageChunk * State::kThreads * sizeof(uint4),
                   "val and stage_tail are one contiguous staging array");
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t* const words = reinterpret_cast<uint32_t*>(c.tag);
-    uint32_t* const count = words + wave * 64;  // [wave][bin] records of this wave per bin
-    // [bin] of this wave: where its run starts in the staging array, and the index of the run's first record in the level's record array
-    uint2* const run = reinterpret_cast<uint2*>(words + kWaves * 64) + wave * 64;
+    uint32_t* const count = words + (tile & 1u) * kStageBins;  // [bin] records of this tile
+    uint32_t* const next_count = words + (~tile & 1u) * kStageBins;
+    // [bin], every wave's own: where the bin's run starts in the staging array, and the index of the run's first record in the level's record array
+    uint2* const run = reinterpret_cast<uint2*>(words + 2 * kStageBins) + wave * kStageBins;
     uint4* const stage = reinterpret_cast<uint4*>(c.val);
-    constexpr uint32_t kNoRoom = 0xFFFFFFFFu;
-    count[lane] = 0u;
-    wave_lds_fence();
-    uvec<D + 1> place = 0u;  // rank of each record within its wave's run for the bin
-    static_for<D + 1>(PENC_BODY(j) {
-        PENC_INDEX(j);
-        if (active) place[j] = atomicAdd(&count[slot[j] >> kBinSlotsLog2], 1u);
-    });
-    __syncthreads();  // all waves have counted, and have left the staging array of the tile before
-    uint32_t before = 0u, mine = 0u;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-        const uint32_t n = words[w * 64 + lane];
-        before += w < static_cast<int>(wave) ? n : 0u;
-        mine += n;
+    constexpr int kTogether = D == 4 ? 3 : D + 1;
+    uvec<D + 1> place = 0u;  // rank of each record within its bin's run
+    if (active) {
+        static_for<D + 1>(PENC_BODY(j) {
+            PENC_INDEX(j); place[j] = atomicAdd(&count[slot[j] >> kBinSlotsLog2], 1u); });
     }
+    __syncthreads();  // all waves have counted, and have left the staging array of the tile before
+    const uint32_t mine = count[lane];
+    if (wave == 0u) next_count[lane] = 0u;  // (last read before the last tile's second barrier, counted in after the next one here)
     uint32_t total;
     const uint32_t first = wave_exclusive_scan(mine, total);
-    run[lane] = make_uint2(first + before, (lane * bins.n_groups + group) * bins.segment_capacity + cursor + before);
+    run[lane] = make_uint2(first, (lane * bins.n_groups + group) * bins.segment_capacity + cursor);
     cursor += mine;
     const bool all_fit = __all(cursor <= bins.segment_capacity);
     wave_lds_fence();
-    static_for<D + 1>(PENC_BODY(j) {
-        PENC_INDEX(j);
+    RecordValues* const values_out = static_cast<RecordValues*>(bins.records);
+    const auto record_of = [&](uint32_t slot_in_bin, float v0, float v1, uint32_t to) {
+        uint4 e;
+        e.x = slot_in_bin;
+        e.y = __builtin_bit_cast(uint32_t, v0);
+        e.z = __builtin_bit_cast(uint32_t, v1);
+        e.w = to;
+        return e;
+    };
+    const auto store = [&](const uint4& e) {
+        RecordValues v;
+        v.x = __builtin_bit_cast(float, e.y);
+        v.y = __builtin_bit_cast(float, e.z);
+        *reinterpret_cast<RecordValues*>(reinterpret_cast<char*>(values_out) + e.w * static_cast<uint32_t>(sizeof(RecordValues))) = v;
+        *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(bins.slots) + e.w * 2u) = static_cast<uint16_t>(e.x);
+    };
+    if (all_fit) {
         if (active) {
-            const uint32_t b = slot[j] >> kBinSlotsLog2;
-            // copies first: a bit cast applied directly to a vector element reads element 0
-            const float v0 = a0[j], v1 = a1[j];
-            const uint2 at = run[b];
-            const uint32_t to = at.y + place[j];
-            uint4 e;
-            e.x = slot[j];
-            e.y = __builtin_bit_cast(uint32_t, v0);
-            e.z = __builtin_bit_cast(uint32_t, v1);
-            e.w = all_fit || to < (b * bins.n_groups + group + 1u) * bins.segment_capacity ? to : kNoRoom;
-            stage[at.x + place[j]] = e;
+            static_for<(D + kTogether) / kTogether>(PENC_BODY(part) {
+                PENC_INDEX(part);
+                constexpr int kFirst = part * kTogether, kCount = D + 1 - kFirst < kTogether ? D + 1 - kFirst : kTogether;
+                uint2 at[kCount];
+                static_for<kCount>(PENC_BODY(k) {
+                    PENC_INDEX(k); at[k] = run[slot[kFirst + k] >> kBinSlotsLog2]; });
+                static_for<kCount>(PENC_BODY(k) {
+                    PENC_INDEX(k);
+                    constexpr int j = kFirst + k;
+                    const float v0 = a0[j], v1 = a1[j];  // copies first: a bit cast applied directly to a vector element reads element 0
+                    stage[at[k].x + place[j]] = record_of(slot[j] & (kBinSlots - 1), v0, v1, at[k].y + place[j]);
+                });
+            });
         }
-    });
-    __syncthreads();
-    static_for<D + 1>(PENC_BODY(j) {
-        PENC_INDEX(j);
-        const uint32_t i = j * State::kThreads + threadIdx.x;
-        bool spill = false;
-        uint4 e = {0u, 0u, 0u, 0u};
-        if (i < total) {
-            e = stage[i];
-            if (e.w != kNoRoom) {
-                store_record(bins, e.w, e.x & (kBinSlots - 1), __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-            } else {
-                spill = true;  // the segment is full: stage 3
+        __syncthreads();
+        static_for<(D + kTogether) / kTogether>(PENC_BODY(part) {
+            PENC_INDEX(part);
+            constexpr int kFirst = part * kTogether, kCount = D + 1 - kFirst < kTogether ? D + 1 - kFirst : kTogether;
+            uint4 e[kCount];  // (past the tile's last record: what an earlier one left there)
+            static_for<kCount>(PENC_BODY(k) {
+                PENC_INDEX(k); e[k] = stage[(kFirst + k) * State::kThreads + threadIdx.x]; });
+            static_for<kCount>(PENC_BODY(k) {
+                PENC_INDEX(k);
+                if ((kFirst + k) * State::kThreads + threadIdx.x < total) store(e[k]);
+            });
+        });
+    } else {
+        constexpr uint32_t kNoRoom = 0xFFFFFFFFu;
+        if (active) {
+            static_for<D + 1>(PENC_BODY(j) {
+                PENC_INDEX(j);
+                const uint32_t b = slot[j] >> kBinSlotsLog2;
+                const float v0 = a0[j], v1 = a1[j];
+                const uint2 at = run[b];
+                const uint32_t to = at.y + place[j];
+                stage[at.x + place[j]] = record_of(slot[j], v0, v1, to < (b * bins.n_groups + group + 1u) * bins.segment_capacity ? to : kNoRoom);
+            });
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int j = 0; j <= D; ++j) {
+            const uint32_t i = j * State::kThreads + threadIdx.x;
+            bool spill = false;
+            uint4 e = {0u, 0u, 0u, 0u};
+            if (i < total) {
+                e = stage[i];
+                spill = e.w == kNoRoom;  // the segment is full: stage 3
+                if (!spill) store(make_uint4(e.x & (kBinSlots - 1), e.y, e.z, e.w));
             }
+            if (__any(spill)) global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
         }
-        if (!all_fit && __any(spill))
-            global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-    });
-    // the next tile writes this wave's counters, which the others have read before the barrier above, and the
-    // staging array after its own first barrier: nothing here is overwritten while another wave reads it
+    }
+    // the next tile counts in the other array, and writes the staging array after its own first barrier: nothing here is
+    // overwritten while another wave reads it
     wave_lds_fence();
 }
 
@@ -673,8 +715,8 @@ __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& leve
 // store needs no search.  When a run does not fit its segment any more (rare: the segments hold
 // the mean plus three standard deviations) the whole chunk takes the careful path, which checks
 // every record against the room left and sends the excess to stage 3.
-// Needs bins.n_bins <= kStageBins and a level's record array below 2^32 bytes (the host plans
-// for both); all 64 lanes of the wave must call it together.
+// Needs bins.n_bins <= kStageBins, whole records and a level's record array below 2^32 bytes (the host plans
+// for all three); all 64 lanes of the wave must call it together.
 template <int D, typename State>
 __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, bool active, uvec<D + 1> slot, fvec<D + 1> a0,
@@ -687,8 +729,7 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
                   "val and stage_tail are one contiguous array of staging slices");
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t* count = reinterpret_cast<uint32_t*>(c.tag) + wave * (kCacheLines / kWaves);  // records per bin
-    uint32_t* offset = count + 64;  // where a bin's run starts in the wave's slice
-    uint32_t* start = count + 128;  // index of the run's first record in the level's record array
+    uint2* run = reinterpret_cast<uint2*>(count + 64);  // where a bin's run starts in the wave's slice, and the index of its first record in the level's record array
     uint32_t* room = count + 192;   // records the workgroup's segment of the bin can still take
     uint4* stage = reinterpret_cast<uint4*>(c.val) + wave * (kStageChunk * 64);
     constexpr uint32_t kNoRoom = 0xFFFFFFFFu;
@@ -700,42 +741,43 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
         count[lane] = 0u;
         wave_lds_fence();
         uvec<kStageChunk> place = 0u;  // rank of each record within its bin's run
-        static_for<kCount>(PENC_BODY(j) {
-            PENC_INDEX(j);
-            if (active) place[j] = atomicAdd(&count[slot[kFirst + j] >> kBinSlotsLog2], 1u);
-        });
+        if (active) {
+            static_for<kCount>(PENC_BODY(j) {
+                PENC_INDEX(j); place[j] = atomicAdd(&count[slot[kFirst + j] >> kBinSlotsLog2], 1u); });
+        }
         wave_lds_fence();
         // lane b looks after bin b: one reservation and one index computation per bin, not per record
         const uint32_t mine = count[lane];
-        uint32_t total;
-        offset[lane] = wave_exclusive_scan(mine, total);
         const uint32_t taken = mine != 0u ? atomicAdd(&c.bin_count[lane], mine) : 0u;
-        start[lane] = (lane * bins.n_groups + group) * bins.segment_capacity + taken;
+        uint32_t total;
+        const uint32_t before = wave_exclusive_scan(mine, total);
+        run[lane] = make_uint2(before, (lane * bins.n_groups + group) * bins.segment_capacity + taken);
         const bool fits = taken + mine <= bins.segment_capacity;
-        if (__all(fits)) {
+        if (__all(fits)) {  // (no branch for single records: a thread's trips to the LDS are made together)
             wave_lds_fence();
-            static_for<kCount>(PENC_BODY(j) {
-                PENC_INDEX(j);
-                if (active) {
-                    const uint32_t b = slot[kFirst + j] >> kBinSlotsLog2;
+            if (active) {
+                uint2 at[kCount];
+                static_for<kCount>(PENC_BODY(j) {
+                    PENC_INDEX(j); at[j] = run[slot[kFirst + j] >> kBinSlotsLog2]; });
+                static_for<kCount>(PENC_BODY(j) {
+                    PENC_INDEX(j);
                     // copies first: a bit cast applied directly to a vector element reads element 0
                     const float v0 = a0[kFirst + j], v1 = a1[kFirst + j];
                     uint4 e;
                     e.x = slot[kFirst + j] & (kBinSlots - 1);
                     e.y = __builtin_bit_cast(uint32_t, v0);
                     e.z = __builtin_bit_cast(uint32_t, v1);
-                    e.w = start[b] + place[j];
-                    stage[offset[b] + place[j]] = e;
-                }
-            });
+                    e.w = at[j].y + place[j];
+                    stage[at[j].x + place[j]] = e;
+                });
+            }
             wave_lds_fence();
+            uint4 e[kCount];  // (past the chunk's last record: what an earlier one left there)
+            static_for<kCount>(PENC_BODY(j) {
+                PENC_INDEX(j); e[j] = stage[j * 64 + lane]; });
             static_for<kCount>(PENC_BODY(j) {
                 PENC_INDEX(j);
-                const uint32_t i = j * 64 + lane;
-                if (i < total) {
-                    const uint4 e = stage[i];
-                    store_record(bins, e.w, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-                }
+                if (j * 64 + lane < total) store_whole_record(bins, e[j]);
             });
         } else {
             room[lane] = taken < bins.segment_capacity ? bins.segment_capacity - taken : 0u;
@@ -749,8 +791,8 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
                     e.x = slot[kFirst + j];
                     e.y = __builtin_bit_cast(uint32_t, v0);
                     e.z = __builtin_bit_cast(uint32_t, v1);
-                    e.w = place[j] < room[b] ? start[b] + place[j] : kNoRoom;
-                    stage[offset[b] + place[j]] = e;
+                    e.w = place[j] < room[b] ? run[b].y + place[j] : kNoRoom;
+                    stage[run[b].x + place[j]] = e;
                 }
             });
             wave_lds_fence();
@@ -761,11 +803,8 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
                 uint4 e = {0u, 0u, 0u, 0u};
                 if (i < total) {
                     e = stage[i];
-                    if (e.w != kNoRoom) {
-                        store_record(bins, e.w, e.x & (kBinSlots - 1), __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
-                    } else {
-                        spill = true;  // the segment is full: stage 3
-                    }
+                    spill = e.w == kNoRoom;  // the segment is full: stage 3
+                    if (!spill) store_whole_record(bins, make_uint4(e.x & (kBinSlots - 1), e.y, e.z, e.w));
                 }
                 if (__any(spill))
                     global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
@@ -886,17 +925,15 @@ __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_gr
 // only take part in the wave-wide steps.  `use_cache` (wave-uniform) is false once the workgroup
 // has seen that the cache does not hit at this level; `mode` and `id_bits` are what
 // scatter_mode_decide decided.  The return value is the number of hits of this wave in this tile.
-template <int D, typename State>
+template <int D, bool kManyBins, typename State>
 __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& level_grad, const BinTarget& bins,
-                                                 uint32_t group, bool active, bool use_cache, int mode, uint32_t id_bits,
+                                                 uint32_t group, uint32_t tile, bool active, bool use_cache, int mode, uint32_t id_bits,
                                                  uvec<D + 1> slot, fvec<D + 1> a0, fvec<D + 1> a1, uint32_t& cursor) {
     if (mode == kModeStream) {
-        if constexpr (State::kThreads > kScatterBlock) {  // (for many bins alone)
-            stream_tile_many<D>(c, level_grad, bins, group, active, slot, a0, a1);
-        } else if (bins.n_bins > kStageBins) {
+        if constexpr (kManyBins) {
             stream_tile_many<D>(c, level_grad, bins, group, active, slot, a0, a1);
         } else if constexpr (D <= kWorkgroupSortMaxDim) {  // measured: the workgroup-wide sort wins up to D = 5, the per-wave one from D = 6 on
-            stream_tile<D>(c, level_grad, bins, group, active, slot, a0, a1, cursor);
+            stream_tile<D>(c, level_grad, bins, group, tile, active, slot, a0, a1, cursor);
         } else {
             stream_tile_wave<D>(c, level_grad, bins, group, active, slot, a0, a1);
         }
@@ -1030,10 +1067,8 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
         c.lines + (2u * c.lines * c.strangers * static_cast<uint32_t>(tiles_per_group - 1)) / (c.wanted != 0u ? c.wanted : 1u);
     if (can_stream && !cache_pays<D>(c, 0, 4u)) {
         mode = kModeStream;
-        if (bins.n_bins > kStageBins) {  // stream_tile_many wants its per-bin counters cleared
-            for (int e = threadIdx.x; e < kMaxBins; e += State::kThreads) c.tag[e] = 0;
-            __syncthreads();
-        }
+        for (int e = threadIdx.x; e < kMaxBins; e += State::kThreads) c.tag[e] = 0;  // stream_tile and stream_tile_many count there
+        __syncthreads();
     } else if (few_slots && expected_slots <= (3u << (kColumnMaxIdsLog2 - 2))) {  // the largest table may end up three quarters full
         mode = kModeColumns;
         id_bits = kColumnMinIdsLog2;
@@ -1047,11 +1082,11 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
 // After the last tile: flushes the accumulate cache or the columns (through the bins when there are
 // any; a streaming workgroup has neither left) and publishes how many records this workgroup left in each
 // bin.  Call once, by all threads.
-template <int D, typename State>
+template <int D, bool kManyBins, typename State>
 __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_grad, const BinTarget& bins,
                                             uint32_t group, int mode, uint32_t id_bits, uint32_t cursor) {
     // (stream_tile keeps count in registers)
-    if (D <= kWorkgroupSortMaxDim && State::kThreads == kScatterBlock && mode == kModeStream && bins.n_bins <= kStageBins && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
+    if (D <= kWorkgroupSortMaxDim && !kManyBins && mode == kModeStream && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
     __syncthreads();
     if (mode == kModeCache) cache_flush(c, level_grad, bins, group);
     if (mode == kModeColumns) column_flush(c, level_grad, id_bits);

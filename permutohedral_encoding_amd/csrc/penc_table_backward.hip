@@ -41,6 +41,8 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // share their geometry: "levels" below (first_level, n_pass_levels, the grid, the bins) count pairs,
 // `pair_level` = level * feat_pairs + pair.  The upstream gradient needs no special case: [L][F][N]
 // is [L * F/2][2][N], and in a row the pair sits at column 2 * pair_level.
+// kManyBins: the records go to more than kStageBins bins (stream_tile_many).  Instances of their own, so that neither sort's registers are spilled for
+// the other's sake.
 // kWideBins: the bins span more than kBinSlots slots (tables above 2^22 slots).  A parameter of the kernel
 // rather than a value read from its arguments, because with the bin width a variable the usual instances
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
@@ -49,7 +51,7 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
 // reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
 enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
-template <int D, bool kRowMajor, int kOrder, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, int kOrder, bool kManyBins, bool kWideBins, int kThreads>
 __device__ __forceinline__ void
 scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
                         uint32_t capacity, uint32_t cap_mask,
@@ -160,7 +162,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             // slice is idle between its tiles and nobody else touches it: it serves as the thread-private
             // columns that put residuals and hash steps into rank order, in place of D(D+1) selects each
             // (at D = 8 about 270 of 1350 vector instructions per point and level).
-            via_lds = mode == kModeStream && bins.n_bins <= static_cast<uint32_t>(kStageBins);
+            via_lds = !kManyBins && mode == kModeStream;
         }
         if (via_lds) {
             constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D), kThreads>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
@@ -223,10 +225,12 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             }
         }
         uvec<D + 1> slot;
-        static_for<D + 1>(PENC_BODY(r) {
-            PENC_INDEX(r);
-            slot[r] = to_slot(h[r], capacity, cap_mask);
-        });
+        if (cap_mask != 0u) {  // (to_slot, asked once)
+            slot = h & cap_mask;
+        } else {
+            static_for<D + 1>(PENC_BODY(r) {
+                PENC_INDEX(r); slot[r] = h[r] % capacity; });
+        }
         if (t == 0) {
             // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
             // (its point is already here)
@@ -248,7 +252,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             a0 += w2 * s0;
             a1 += w2 * s1;
         }
-        const uint32_t hits = scatter_tile<D>(state, level_grad, bins, group, active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1, cursor);
+        const uint32_t hits = scatter_tile<D, kManyBins>(state, level_grad, bins, group, static_cast<uint32_t>(t), active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1, cursor);
         // the first tile finds the lines its own look-up has claimed: no evidence of reuse
         if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
         pos = pos_next;
@@ -258,7 +262,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s0 = s0_next;
         s1 = s1_next;
     }
-    scatter_end<D>(state, level_grad, bins, group, mode, id_bits, cursor);
+    scatter_end<D, kManyBins>(state, level_grad, bins, group, mode, id_bits, cursor);
 }
 
 #define PENC_TABLE_PARAMETERS                                                                                                          \
@@ -270,15 +274,15 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
 #define PENC_TABLE_ARGUMENTS                                                                                                        \
     n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
         random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
-template <int D, bool kRowMajor, bool kSecond, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, bool kSecond, bool kManyBins, bool kWideBins, int kThreads>
 __global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kThreads))
 backward_table_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kManyBins, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
-template <int D, bool kRowMajor, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, bool kManyBins, bool kWideBins, int kThreads>
 __global__ void __launch_bounds__(kThreads, both_orders_waves_per_simd(D, kThreads))
 backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kBothOrders, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kBothOrders, kManyBins, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
 #undef PENC_TABLE_PARAMETERS
 #undef PENC_TABLE_ARGUMENTS
@@ -564,13 +568,15 @@ void launch_table_backward(const TableLaunch& t) {
                        t.feat_pairs, t.dies, t.tiles_per_group / (THREADS / kScatterBlock), t.capacity, t.cap_mask, t.positions,       \
                        t.scale_factor, t.random_shift, t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad,          \
                        t.table_grad, t.grad_level_major, t.bins)
-#define PENC_LAUNCH_WIDTH(KERNEL, ...)                                      \
-    if (t.wide_bins) {                                                      \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true);    \
-    } else if (t.many_bins) {                                               \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, false);   \
-    } else {                                                                \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, false);           \
+#define PENC_LAUNCH_WIDTH(KERNEL, ...)                                            \
+    if (t.wide_bins) {                                                            \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true, true);    \
+    } else if (t.most_bins) {                                                     \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true, false);   \
+    } else if (t.many_bins) {                                                     \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, true, false);           \
+    } else {                                                                      \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, false, false);          \
     }
     if (t.second_grad != nullptr) {
         if (t.rows) {

@@ -11,8 +11,9 @@ struct TableLaunch {
     hipStream_t stream;
     bool rows;          // the upstream gradient is read as rows
     bool second_order;  // double_pos_grad is given; with second_grad too, both orders
-    bool wide_bins;     // (only together with many_bins: the scatter of wide bins has no other instance)
-    bool many_bins;     // more than kFewerOpenLinesMinBins: workgroups of kScatterBlockManyBins threads, else of kScatterBlock
+    bool many_bins;     // records go to more than kStageBins bins
+    bool most_bins;     // more than kFewerOpenLinesMinBins (many_bins too, where there are records): workgroups of kScatterBlockManyBins threads, else of kScatterBlock
+    bool wide_bins;     // (only together with most_bins: the scatter of wide bins has no other instance)
     int n_points, first_level;
     uint32_t n_pass_levels, feat_pairs, dies;
     int tiles_per_group;  // of kScatterBlock points; even

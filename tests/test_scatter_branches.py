@@ -44,6 +44,37 @@ def test_hundreds_of_bins(d, n, cap):
         assert_sum_close(tg2[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"second order, level {level}")
 
 
+@pytest.mark.parametrize("d,n,cap", [(2, 17 * 8192 + 777, 1 << 19), (3, 17 * 8192 + 777, 1 << 18), (4, 130001, 200001), (5, 133001, 1 << 18), (8, 131201, 1 << 18)])
+def test_segments_of_few_bins_run_over(d, n, cap):
+    """At most 64 bins: tiles whose records all fit their segments take turns with tiles whose do not.  Of every group, 1024 points behind the tile
+    by which it decides to stream sit in one simplex, and the rest of the group fills what their segments have left; the last tile ends early, and from
+    non-powers of two slots are remainders.  First and second order against the oracle."""
+    from helpers import assert_sum_close, gpu_input, make_encoding, random_problem, scatter_plan, to_gpu
+    from oracle import api as orc
+    rng = np.random.default_rng(d)
+    levels = 24
+    group, _, bins, places = scatter_plan(d, n, levels, cap)
+    at = np.arange(n) % group
+    crowd = (at >= group // 2) & (at < group // 2 + 1024)
+    assert group == 4096 and bins <= 64 and n % 512 != 0
+    assert 1024 + (group - 1024) * (d + 1) // bins > places
+    p = random_problem(d, n, levels, 1, seed=80 + d, sigma_range=(2e-3, 1e-3))
+    p["pos"] = np.where(crowd[:, None], (0.61 + 1e-7 * rng.standard_normal((n, d))).astype(np.float32), p["pos"])
+    sf = orc.scale_factors(d, p["sigmas"])
+    enc, _ = make_encoding(d, p["sigmas"], p["shift"])
+    inp = gpu_input(p, need_pos_grad=False)
+    inp.m_lattice_values = torch.zeros(levels, cap, 2, device="cuda")  # the table gradient does not read the table
+    tg, _ = enc.backward(inp, to_gpu(p["grad"]))
+    tg2, _ = enc.double_backward_from_positions(inp, to_gpu(p["dpos"]), to_gpu(p["grad"]))
+    for level in (0, levels - 1):
+        one = slice(level, level + 1)
+        args = (p["pos"], sf[one], p["shift"][one], p["window"][one])
+        want = orc.backward_table(*args, p["grad"][one], cap, want_abs=True)
+        assert_sum_close(tg[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"first order, level {level}")
+        want = orc.double_backward(p["pos"], np.zeros((1, cap, 2), np.float32), sf[one], p["shift"][one], p["window"][one], p["dpos"], p["grad"][one], want_abs=True)
+        assert_sum_close(tg2[level].cpu().numpy()[None], want["grad64"], want["abs64"], 1e-4, f"second order, level {level}")
+
+
 @pytest.mark.parametrize("d,levels,n,cap", [(3, 24, (1 << 20) + 5, 1 << 17), (4, 24, (1 << 20) + 5, 1 << 18), (5, 24, (1 << 20) + 12345, 1 << 12)])
 def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, n, cap):
     """Groups of eight tiles from rows (of sixteen from five dimensions on), of sixteen from [L][F][N], at a size that has both, give the
