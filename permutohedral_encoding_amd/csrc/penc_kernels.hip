@@ -870,6 +870,7 @@ struct BinPlan {
     int levels_per_pass = 0;
     BinTarget target{};       // of the first pass; target.direct covers all levels, a pass starts at its first level's flags
     size_t direct_bytes = 0;  // size of target.direct (to be cleared with the gradient)
+    uintptr_t end = 0;        // of what is used of the workspace
 };
 
 // Bytes of the `direct` flags of all levels (one 4-byte flag per level and bin), padded to the workspace's alignment.
@@ -1011,8 +1012,39 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, int t
     const size_t records_per_pass = static_cast<size_t>(p.levels_per_pass) * segments * cap;
     p.target.records = reinterpret_cast<void*>(counts_at + counts_bytes);
     p.target.slots = split ? reinterpret_cast<uint16_t*>(counts_at + counts_bytes + records_per_pass * sizeof(RecordValues)) : nullptr;
+    p.end = counts_at + counts_bytes + records_per_pass * record_bytes(pos_dim, n_bins);
     p.enabled = true;
     return p;
+}
+
+// Fill, scatter, reduction and late adds, us, fill apart -> in the scatter (24 levels unless given):
+//   D = 3, 2^22 slots  2^20 points 1050 -> 986, near a surface with 16 levels live 609 -> 521, 200001 points 506 -> 425;  2^23 slots, 2^19 points 1039 -> 984
+//          2^21        200001 points 303 -> 253
+//          2^20        2^20 points 620 -> 606, from rows 663 -> 664, 200001 points 200 -> 190;  9 levels (75 MB) 2^18 points 91 -> 90
+//   D = 2, 16 levels of 2^20, 2^18 points 135 -> 127;  D = 4, 16 levels of 2^22, 2^19 points 625 -> 572, of 2^21 423 -> 391;  D = 8, of 2^22, 2^17 points 454 -> 395
+// A smaller gradient takes no longer to fill than the lists take to be added, and the instances for few bins stay without the code.
+constexpr size_t kClearInScatterBytes = size_t{64} << 20;
+inline bool clears_in_scatter(uint32_t n_bins, int pair_levels, int capacity) {
+    return n_bins > static_cast<uint32_t>(kStageBins) && static_cast<size_t>(pair_levels) * capacity * sizeof(float2) >= kClearInScatterBytes;
+}
+// What the lists of deferred adds (BinTarget) take behind the bins, for all levels at once.
+inline size_t deferred_bytes(int pos_dim, int pair_levels, uint32_t n_groups, int tiles_per_group) {
+    return static_cast<size_t>(pair_levels) * n_groups * (deferred_room(pos_dim, tiles_per_group) * sizeof(BinRecord) + sizeof(uint32_t)) + 512;
+}
+// Gives the plan of a dense gradient such lists where its scatter has the instance that clears, takes all levels in one launch, and the workspace has room
+// for them.
+inline bool plan_deferred(BinPlan& p, int pos_dim, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
+                          size_t bytes) {
+    if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity) || p.levels_per_pass < pair_levels) return false;
+    if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0 || (static_cast<int64_t>(pair_levels) * capacity) % 2 != 0) return false;
+    const uintptr_t base = (p.end + 255u) & ~uintptr_t{255};
+    if (base + deferred_bytes(pos_dim, pair_levels, p.target.n_groups, tiles_per_group) > reinterpret_cast<uintptr_t>(workspace) + bytes) return false;
+    p.target.deferred_room = deferred_room(pos_dim, tiles_per_group);
+    p.target.deferred = reinterpret_cast<BinRecord*>(base);
+    p.target.deferred_counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.target.deferred_room * sizeof(BinRecord));
+    p.target.clear_quads = static_cast<uint64_t>(pair_levels) * capacity / 2;
+    p.target.clear_flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
+    return true;
 }
 
 // When a table gradient takes the sorted groups of penc_group_sort.hpp, and how they cut its workspace.
@@ -1330,6 +1362,8 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         plan.target.direct = touched;
         plan.target.n_bins = bins_for_capacity(capacity);
         plan.target.bin_shift = bin_shift_for_capacity(capacity);
+    } else if (plan_deferred(plan, pos_dim, pair_levels, capacity, tiles_per_group, lattice_values_grad, workspace, workspace_bytes)) {
+        // the scattering kernel clears
     } else if (int rc = clear_table_grad(lattice_values_grad, pair_levels, capacity, plan.enabled ? plan.target.direct : nullptr,
                                          plan.direct_bytes, st)) {
         return rc;
@@ -1353,6 +1387,11 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         if (int rc = check_launch()) return rc;
         if (plan.enabled)
             if (int rc = reduce_bins(plan, anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
+    }
+    if (plan.target.deferred != nullptr) {
+        hipLaunchKernelGGL(add_deferred_kernel, dim3(plan.target.n_groups, static_cast<unsigned>(pair_levels)), dim3(kBlock), 0, st, plan.target, anneal_window,
+                           cap, feat_pairs, lattice_values_grad);
+        return check_launch();
     }
     return PENC_OK;
 }
@@ -1577,6 +1616,18 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
                           nr_positions <= kGroupSortPointsPerLevel * nr_levels;
     const size_t sorted = may_sort ? group_sort_bytes(pos_dim, nr_positions, nr_levels) + 256 : 0;
     return sorted > binned ? sorted : binned;
+}
+
+size_t penc_scatter_deferred_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
+    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
+    const uint32_t n_bins = bins_for_capacity(capacity);
+    if (n_bins > static_cast<uint32_t>(kMaxBins) || !clears_in_scatter(n_bins, nr_levels, capacity) || nr_positions * (pos_dim + 1) * kMinSlotsPerContribution <= capacity) return 0;
+    size_t most = 0;
+    for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {
+        const size_t need = deferred_bytes(pos_dim, nr_levels, scatter_groups(nr_positions, tiles), tiles);
+        most = need > most ? need : most;
+    }
+    return most + 256;
 }
 
 size_t penc_positions_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels) {

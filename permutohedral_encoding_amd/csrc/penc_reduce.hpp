@@ -193,7 +193,7 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // thread 0 sets the flag at the end.
     const bool untouched_so_far = bins.direct[bin] == 0u;
     __syncthreads();
-    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u};
+    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
     const uint32_t slot0 = bin << kBinSlotsLog2;  // (this kernel serves bins of kBinSlots slots only)
     const bool alone = gridDim.z == 1;
     if (alone) {
@@ -234,6 +234,23 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     for (uint32_t s = threadIdx.x >> 1; s < static_cast<uint32_t>(kBinSlots); s += kReduceBlock / 2) {
         const double v = acc[s];
         if (v != 0.0 && slot0 + s < capacity) global_add(level_grad.at(slot0 + s) + (threadIdx.x & 1u), static_cast<float>(v));
+    }
+}
+
+// Adds what a scattering kernel that cleared the gradient has kept (BinTarget::deferred): a workgroup to a group of points and a level.
+__global__ void __launch_bounds__(kBlock)
+add_deferred_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs, float* __restrict__ table_grad) {
+    const uint32_t group = blockIdx.x, pair_level = blockIdx.y, level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
+    if (window[level] == 0.0f) return;  // masked level: its scattering workgroups wrote no counts
+    const BinTarget bins = bins_of_level(pass_bins, pair_level);
+    const uint32_t count = bins.deferred_counts[group];
+    const BinRecord* const kept = bins.deferred + static_cast<size_t>(group) * bins.deferred_room;
+    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
+    for (uint32_t first = 0; first < count; first += kBlock) {
+        const uint32_t i = first + threadIdx.x;
+        BinRecord rec{0u, 0.0f, 0.0f};
+        if (i < count) rec = kept[i];
+        global_add_pairs(level_grad, i < count, rec.slot_in_bin, rec.a0, rec.a1);
     }
 }
 
@@ -383,7 +400,7 @@ bin_reduce_levels_kernel(BinTarget pass_bins, const float* __restrict__ window, 
         lds_barrier();
         const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass(i);
         const uint32_t level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
-        const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u};
+        const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
         const uint32_t slot0 = (bin << pass_bins.bin_shift) + (range << kBinSlotsLog2);
         const bool untouched_so_far = ((direct_mask >> i) & 1u) == 0u;
         constexpr int kMine = kBinSlots / kReduceBlock / 2;

@@ -106,6 +106,14 @@ constexpr size_t kSplitRecordBytes = sizeof(RecordValues) + sizeof(uint16_t);
 //                                                  for a caller who keeps gradient and flags across calls (the sparse
 //                                                  entry points), the caller's map of touched slot ranges.
 // `records` == nullptr disables binning (`direct`, `n_bins` and `bin_shift` may still be set: flags without bins).
+//
+// Large tables (`deferred` set; more than kStageBins bins, all levels in one launch): the scattering kernel clears the gradient and the flags
+// itself, each workgroup a share of them when it starts, because those writes pass while it waits for other things (2^22 slots, 24 levels,
+// 16 of them live, 2^20 points: fill 134 and scatter 329 us apart, 373 together; 200001 points 163 and 90, 184).  Nothing may
+// be added to a gradient that another workgroup is still to clear, so what would go straight into it is kept until the reducers have ended, and
+// add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
+//   deferred         [level_in_pass][group][deferred_room]   {slot in the level, values}; there is room for all a group can leave
+//   deferred_counts  [level_in_pass][group]
 struct BinTarget {
     void* records;
     uint16_t* slots;
@@ -115,7 +123,16 @@ struct BinTarget {
     uint32_t n_groups;
     uint32_t segment_capacity;
     uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records)
+    uint32_t deferred_room;
+    BinRecord* deferred;
+    uint32_t* deferred_counts;
+    uint64_t clear_quads;   // 16-byte units of the gradient, where the scattering kernel clears it,
+    uint32_t clear_flags;   // and its flags
 };
+// What a group of points can leave for later at a level: all its contributions, and the lines its cache claimed.
+constexpr uint32_t deferred_room(int pos_dim, int tiles_per_group) {
+    return static_cast<uint32_t>(tiles_per_group * kScatterBlock * (pos_dim + 1) + kCacheLines);
+}
 
 // `pass` describes the first level of a launch; level k of the launch follows k bin arrays later.
 __device__ __forceinline__ BinTarget bins_of_level(const BinTarget& pass, uint32_t k) {
@@ -128,6 +145,10 @@ __device__ __forceinline__ BinTarget bins_of_level(const BinTarget& pass, uint32
         t.counts += segments;
     }
     if (pass.direct != nullptr) t.direct += static_cast<size_t>(k) * pass.n_bins;
+    if (pass.deferred != nullptr) {
+        t.deferred += static_cast<size_t>(k) * pass.n_groups * pass.deferred_room;
+        t.deferred_counts += static_cast<size_t>(k) * pass.n_groups;
+    }
     return t;
 }
 
@@ -208,6 +229,8 @@ struct GradSlice {
     uint32_t slot_floats;
     uint32_t* direct;
     uint32_t bin_shift;  // of the bins `direct` belongs to
+    BinRecord* deferred;       // nullptr: adds go into the gradient; else the workgroup's list of them (see BinTarget),
+    uint32_t* deferred_count;  // in LDS: how many are in it
     __device__ __forceinline__ float* at(uint32_t slot) const { return base + static_cast<size_t>(slot) * slot_floats; }
     // A plain store on purpose: many workgroups may set the same flag at once, all to 1, and nobody reads it before the
     // kernel has ended.  (As a relaxed atomic store of device scope, a store that writes through the L2, the levels that
@@ -215,6 +238,7 @@ struct GradSlice {
     __device__ __forceinline__ void mark_direct(uint32_t slot) const {
         if (direct != nullptr) direct[slot >> bin_shift] = 1u;
     }
+    __device__ __forceinline__ void defer(uint32_t slot, float a0, float a1) const { deferred[atomicAdd(deferred_count, 1u)] = BinRecord{slot, a0, a1}; }
 };
 
 __device__ __forceinline__ void global_add(float* addr, float v) {
@@ -281,6 +305,10 @@ __device__ __forceinline__ void global_add_pairs(const GradSlice& level_grad, bo
                                                  float a0, float a1) {
     constexpr int kFromEven = 0xA0;  // quad_perm:[0,0,2,2]
     constexpr int kFromOdd = 0xF5;   // quad_perm:[1,1,3,3]
+    if (level_grad.deferred != nullptr) {
+        if (need) level_grad.defer(slot, a0, a1);
+        return;
+    }
     if (need) level_grad.mark_direct(slot);
     const int odd = threadIdx.x & 1;
     const int slot_i = static_cast<int>(slot), need_i = need ? 1 : 0;
@@ -390,6 +418,7 @@ struct ScatterStateT {
     uint32_t lines;                // lines they claimed: the tile's distinct slots, as far as the cache could take them
     uint32_t misses;               // contributions whose slot found no line
     uint32_t columns;              // columns given away (kModeColumns)
+    uint32_t deferred;             // entries of the workgroup's list of deferred adds
     uint32_t strangers;            // slots of the second tile that the first tile did not touch (counted for levels with few slots)
 };
 
@@ -408,6 +437,7 @@ __device__ __forceinline__ void scatter_begin(State& c) {
         c.misses = 0u;
         c.strangers = 0u;
         c.columns = 0u;
+        c.deferred = 0u;
     }
     __syncthreads();
 }
@@ -912,6 +942,10 @@ __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_gr
         if (lane == 0) {
             // straight into the gradient: a level in column mode leaves a few dozen sums per workgroup, and
             // as records they would only make every bin's reducer workgroup run for a handful of them
+            if (level_grad.deferred != nullptr) {
+                level_grad.defer(static_cast<uint32_t>(owner), static_cast<float>(s0), static_cast<float>(s1));
+                continue;
+            }
             float* g = level_grad.at(static_cast<uint32_t>(owner));
             level_grad.mark_direct(static_cast<uint32_t>(owner));
             global_add(g, static_cast<float>(s0));
@@ -1004,7 +1038,9 @@ __device__ __forceinline__ void cache_flush(State& c, const GradSlice& level_gra
         if (owner != -1) {
             const float v0 = static_cast<float>(c.val[0][e]), v1 = static_cast<float>(c.val[1][e]);
             const bool binned = bins.records != nullptr && append_record(c, bins, group, static_cast<uint32_t>(owner), v0, v1);
-            if (!binned) {
+            if (!binned && level_grad.deferred != nullptr) {
+                level_grad.defer(static_cast<uint32_t>(owner), v0, v1);
+            } else if (!binned) {
                 float* g = level_grad.at(static_cast<uint32_t>(owner));
                 level_grad.mark_direct(static_cast<uint32_t>(owner));
                 global_add(g, v0);
@@ -1096,6 +1132,7 @@ __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_gra
         const uint32_t n = c.bin_count[b];
         bins.counts[static_cast<size_t>(b) * bins.n_groups + group] = n < bins.segment_capacity ? n : bins.segment_capacity;
     }
+    if (level_grad.deferred != nullptr && threadIdx.x == 0) bins.deferred_counts[group] = c.deferred;
 }
 
 }  // namespace penc

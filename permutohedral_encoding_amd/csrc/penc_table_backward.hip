@@ -71,6 +71,17 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     // a time).
     const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
     const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
+    constexpr bool kMayDefer = kManyBins;
+    if constexpr (kMayDefer) {
+        if (pass_bins.deferred != nullptr) {
+            typedef float Quad __attribute__((ext_vector_type(4)));
+            const uint64_t share = (pass_bins.clear_quads + gridDim.x - 1) / gridDim.x, from = share * blockIdx.x;
+            const uint64_t to = from + share < pass_bins.clear_quads ? from + share : pass_bins.clear_quads;
+            for (uint64_t i = from + threadIdx.x; i < to; i += kThreads) __builtin_nontemporal_store(Quad(0.0f), reinterpret_cast<Quad*>(table_grad) + i);
+            const uint32_t flag = blockIdx.x * kThreads + threadIdx.x;
+            if (flag < pass_bins.clear_flags) pass_bins.direct[flag] = 0u;
+        }
+    }
     const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kThreads;
     if (group_base >= n_points) return;
     const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;
@@ -81,7 +92,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     if constexpr (!kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
-                               2 * feat_pairs, bins.direct, bins.bin_shift};
+                               2 * feat_pairs, bins.direct, bins.bin_shift,
+                               kMayDefer && bins.deferred != nullptr ? bins.deferred + static_cast<size_t>(group) * bins.deferred_room : nullptr, &state.deferred};
     // Everything a thread reads lies within its group of at most 16 x 512 points, so the addresses are
     // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets in bytes: the form the load instructions take.
     const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);

@@ -101,3 +101,64 @@ def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, 
     # the weights are not negative: the third is the sum of magnitudes.  Each of up to 257 groups rounds its partial sum, and the sum it is
     # added to, to 2^-24 of that
     assert torch.all((out[0] - out[1]).abs() <= 2 * 2 * 257 * 2.0 ** -24 * out[2] + 1e-30)
+
+
+@pytest.mark.parametrize("d,feat,levels,n,cap", [(3, 2, 24, 17 * 8192 + 777, 1 << 22), (2, 4, 12, 200003, (1 << 22) - 6), (4, 2, 24, 130001, (1 << 22) + 2),
+                                                 (8, 2, 8, 131201, 1 << 22), (3, 2, 24, 17 * 8192 + 777, 1 << 20), (3, 2, 5, (1 << 19) + 3, (1 << 21) + 8192)])
+def test_scatter_that_clears_the_gradient(d, feat, levels, n, cap):
+    """With lists of deferred adds in the workspace the scatter clears the gradient, whatever it held, masked levels too, and what would go straight into
+    it follows later: column sums of the coarse levels, and what segments have no room for (a third of the points sit in one simplex).  Both
+    orders, rows and level-major, against the call without lists."""
+    from helpers import make_encoding
+    from permutohedral_encoding_amd import _native
+    rng = np.random.default_rng(d)
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    _, fp = make_encoding(d, np.geomspace(1.0, 1e-3, levels).astype(np.float32), (rng.standard_normal((levels, d)) * 10).astype(np.float32), nr_feat=feat)
+    torch.manual_seed(d)
+    pos = torch.rand(n, d, device="cuda")
+    crowd = (torch.arange(n, device="cuda") % 4096 >= 2048) & (torch.arange(n, device="cuda") % 4096 < 3400)
+    pos[crowd] = 0.61 + 1e-7 * torch.randn(int(crowd.sum()), d, device="cuda")
+    window = torch.ones(levels, device="cuda")
+    window[1] = 0.0
+    rows, q = torch.randn(n, feat * levels, device="cuda"), torch.randn(n, d, device="cuda")
+    pairs = levels * feat // 2
+    table = torch.zeros(levels, cap, feat, device="cuda")  # (not read by a table gradient)
+    plain, lists = lib.penc_scatter_workspace_bytes(d, n, pairs, cap, pairs), lib.penc_scatter_deferred_bytes(d, n, pairs, cap)
+    assert lists > pairs * n * (d + 1) * 12
+    ws = torch.empty(plain + lists, dtype=torch.uint8, device="cuda")
+
+    def gradient(size, order, as_rows, up):
+        up = up.contiguous() if as_rows else up.t().contiguous()
+        tg = torch.full((levels, cap, feat), float("nan"), device="cuda")
+        ws.fill_(0xAB)
+        common = (pos.data_ptr(), table.data_ptr(), fp.m_scale_factor.data_ptr(), fp.m_random_shift_per_level.data_ptr(), window.data_ptr())
+        end = (tg.data_ptr(), None)
+        if order == 1:
+            rc = (lib.penc_backward_rowmajor(d, feat, n, levels, cap, *common, up.data_ptr(), feat * levels, *end, ws.data_ptr(), size, st) if as_rows else
+                  lib.penc_backward(d, feat, n, levels, cap, *common, up.data_ptr(), *end, ws.data_ptr(), size, st))
+        elif as_rows:
+            rc = lib.penc_double_backward_from_positions_rowmajor(d, feat, n, levels, cap, *common, q.data_ptr(), up.data_ptr(), feat * levels, *end, 0,
+                                                                  ws.data_ptr(), size, st)
+        else:
+            rc = lib.penc_double_backward_from_positions(d, feat, n, levels, cap, *common, q.data_ptr(), up.data_ptr(), *end, 0, ws.data_ptr(), size, st)
+        assert rc == 0
+        return tg
+
+    # Weights of the first order are not negative but for 2^-24 of rounding, so their sum with |gradient| is that of magnitudes.  A slot's groups round their partial sums, and what
+    # these are added to, to 2^-24 of that: all but the slots of the crowd's simplex (a few more where its 1e-7 reach over a face), whose
+    # contributions are added one by one.
+    magnitude = gradient(plain, 1, False, rows.abs()).abs()
+    each, one_by_one = -(-n // 4096), int(crowd.sum())
+    want = gradient(plain, 1, False, rows)
+    for as_rows in (False, True):
+        got = gradient(plain + lists, 1, as_rows, rows)
+        assert torch.all(got[1] == 0.0) and not torch.any(torch.isnan(got))
+        off = (got - want).abs()
+        assert torch.all(off <= 4 * (each + one_by_one) * 2.0 ** -24 * magnitude + 1e-12)
+        assert int((off > 4 * each * 2.0 ** -24 * magnitude + 1e-12).sum()) <= levels * feat * 4 * (d + 1)
+    for as_rows in (False, True):
+        got, want = gradient(plain + lists, 2, as_rows, rows).double(), gradient(plain, 2, as_rows, rows).double()
+        assert torch.all(got[1] == 0.0)
+        # 2-norm, level by level: the two round the same sums in another order, those of the crowd's slots at random and `one_by_one` times
+        for level in range(levels):
+            assert (got[level] - want[level]).norm() <= 4 * one_by_one ** 0.5 * 2.0 ** -24 * (want[level].norm() + want[level].abs().max() * (d + 1) ** 0.5)
