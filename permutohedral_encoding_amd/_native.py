@@ -393,7 +393,7 @@ class EncodingWrapper:
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table
     _half_copy = None
     _half_copy_of = None
-    _cells = None      # (key, copy): the 16-bit copy in cells (penc_table_cells), where enough points have been gathered for it
+    _cells = None      # (key, copy, stream, event): the 16-bit copy in cells (penc_table_cells), where enough points have been gathered for it
     _gathered = None   # (key, points): how many were, without it, since the table was last modified
     # set by the module (sparse_table_grad=True): table gradients are added into `sparse_grad`, a SparseTableGrad the
     # wrapper keeps across calls, and the gradient calls return None for them
@@ -431,6 +431,11 @@ class EncodingWrapper:
         cells = self._cells
         if cells is not None:
             if cells[0] == key:
+                # it was made in the middle of a program, by a call on some stream: one on another stream waits for it, and keeps it from reuse
+                if cells[2] != torch._C._cuda_getCurrentRawStream(lattice_values.get_device()) and not torch.cuda.is_current_stream_capturing():
+                    stream = torch.cuda.current_stream(lattice_values.device)
+                    stream.wait_event(cells[3])
+                    cells[1].record_stream(stream)
                 return cells[1], True
             self._cells = cells = None
         points = lib().penc_table_cells_points(self.nr_feat, lattice_values.shape[1], TABLE_FORMATS[self.half_table])
@@ -452,7 +457,8 @@ class EncodingWrapper:
             return self.gather_table(lattice_values), False
         if not rounded:
             self._half_copy = self._half_copy_of = None
-        self._cells = (key, copy)
+        stream = torch.cuda.current_stream(lattice_values.device)
+        self._cells = (key, copy, stream.cuda_stream, stream.record_event())
         return copy, True
 
     def invalidate_half_table(self):

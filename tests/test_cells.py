@@ -246,3 +246,25 @@ def test_forward_by_way_of_cells_equals_the_forward(d, feat):
                 assert chosen[levels // 3] == 0
                 kinds.update(chosen.tolist())
     assert kinds == {0, 1}
+
+
+@pytest.mark.gpu
+def test_copy_made_on_one_stream_is_waited_for_on_another():
+    """The copy is made in the middle of a program, behind what its stream has to do; a call on another stream that finds it made waits for it."""
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 20, 12, 2, np.geomspace(1.0, 1e-3, 12), lattice_half_precision=torch.bfloat16)
+    line = pe._native.lib().penc_table_cells_points(2, 1 << 20, 2)
+    few, many = torch.rand(1000, 3, device="cuda"), torch.rand(line, 3, device="cuda")
+    work = torch.randn(4096, 4096, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        want = m(few)
+        torch.cuda.synchronize()
+        for _ in range(20):
+            work = (work @ work).clamp(-1, 1)
+        m(many)
+        assert m.lattice._cells is not None
+        with torch.cuda.stream(side):
+            got = m(few)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
