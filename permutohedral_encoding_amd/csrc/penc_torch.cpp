@@ -430,7 +430,7 @@ public:
 bool forward_in_cells(const Call& c, Tensor level_major, const Tensor& rows, const Tensor& slopes) {
     if (c.table_format != 0) return false;
     const size_t n = api.forward_cells_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, rows.defined() ? static_cast<int>(c.columns()) : 0);
-    if (n == 0) return false;
+    if (n == 0 || (c.max_workspace >= 0 && static_cast<int64_t>(n) > c.max_workspace)) return false;
     Tensor ws;
     try {
         if (!level_major.defined()) level_major = level_major_array(c);

@@ -268,3 +268,27 @@ def test_copy_made_on_one_stream_is_waited_for_on_another():
             got = m(few)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [False, True])
+def test_forward_by_way_of_cells_keeps_to_the_workspace_cap(monkeypatch, rows):
+    import permutohedral_encoding_amd as pe
+    from permutohedral_encoding_amd import _native
+    levels, cap, n = 16, 1 << 18, 1 << 20
+    m = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels), contiguous_output=rows)
+    assert _native.lib().penc_forward_cells_workspace_bytes(3, 2, n, levels, cap, 2 * levels if rows else 0) > m.lattice_values.numel() * 4
+    pos = torch.rand(n, 3, device="cuda")
+
+    def taken():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        with torch.no_grad():
+            out = m(pos)
+        return out, torch.cuda.max_memory_allocated() - before
+
+    want, free = taken()
+    monkeypatch.setattr(_native, "MAX_WORKSPACE_BYTES", m.lattice_values.numel() * 4)
+    got, capped = taken()
+    assert torch.equal(got, want) and capped <= free - m.lattice_values.numel() * 4
