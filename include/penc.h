@@ -84,10 +84,10 @@ int penc_scale_factors(int pos_dim, int nr_levels, const float* sigmas, float* s
  * atomicAdd per value, EncodingGPU.cuh:409-410). */
 size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity,
                                     int levels_per_pass);
-/* What a workspace for all levels may hold besides, for a dense gradient of 64 MiB and more of a table of more than 2^19 slots: lists that
- * let the scatter clear the gradient while it works (csrc/penc_scatter.hpp); 0 where there are none.  12 * (pos_dim + 1) bytes per point and level, little of which is
- * ever written. */
-size_t penc_scatter_deferred_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity);
+/* What the scatter of a dense gradient can use on top of penc_scatter_workspace_bytes() for all levels: for a gradient of 64 MiB and more of a table of
+ * more than 2^19 slots, lists that let the scatter clear the gradient while it works (12 * (pos_dim + 1) bytes per point and level, little of which
+ * is ever written; csrc/penc_scatter.hpp); for small tables and few levels, the slack of more and narrower bins (a few percent); else 0. */
+size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity);
 
 /* Size of `workspace` that lets penc_backward compute positions_grad in groups of a few levels
  * (partial sums in the workspace, then one deterministic reduction) instead of one thread walking

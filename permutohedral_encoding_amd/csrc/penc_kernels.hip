@@ -888,10 +888,32 @@ constexpr uint32_t bin_shift_for_capacity(int capacity) {
     return shift;
 }
 
-// Bins per level; more than kMaxBins means the table is too large for binning.
-constexpr uint32_t bins_for_capacity(int capacity) {
-    const uint32_t shift = bin_shift_for_capacity(capacity);
+constexpr uint32_t bins_of_shift(int capacity, uint32_t shift) {
     return static_cast<uint32_t>((static_cast<int64_t>(capacity) + (int64_t{1} << shift) - 1) >> shift);
+}
+// Bins per level; more than kMaxBins means the table is too large for binning.
+constexpr uint32_t bins_for_capacity(int capacity) { return bins_of_shift(capacity, bin_shift_for_capacity(capacity)); }
+
+// The width of the bins of a dense gradient whose workspace has room for the slack of more segments (penc_scatter_extra_bytes): where there are fewer
+// (bin, level) pairs than reducers wanted, so that several would share a bin and add into the gradient with atomics (60 ns each), bins of half the width
+// and less, down to 2^10 slots, until there are kFineBinsWanted pairs, each reduced by one workgroup of a part of a compute unit's LDS.  Scatter and
+// reduction, us:
+//   D = 3, 24 levels   2^16 slots, 2^20 points 517 -> 481   2^14 598 -> 488   2^12, 2^19 points 408 -> 270;  6 levels of 2^16, 2^20 points 145 -> 128
+//          16 levels   2^18 points, 2^16 slots 105 -> 98   2^14 131 -> 101   100003 slots 108 -> 98;  12 levels of 2^18, 2^19 points 134 -> 125
+//   D = 2, 16 levels   2^16 slots, 2^18 points 83 -> 73, four features 125 -> 117;  2^17, 2^19 points 124 -> 123
+//   D = 5, 16 levels   2^16 slots, 2^18 points 177 -> 160;  D = 6 of 2^14 217 -> 204;  D = 8 of 2^16 255 -> 250, 8 levels of 2^18, 2^17 points 97 -> 91
+// With four dimensions the accumulate cache leaves some slots of the coarse levels out, whose records several reducers of a bin share
+// better than one (16 levels, 2^18 points: 2^16 slots 130 -> 137, 2^17 126 -> 132; 2^15 131 -> 122).
+constexpr uint32_t kReduceWorkgroupsWanted = 512;  // two per compute unit
+constexpr uint32_t kFineBinsWanted = 768, kFineBinsMostPairs4d = 128;
+constexpr uint32_t fine_bin_shift(int pos_dim, int capacity, int pair_levels) {
+    uint32_t shift = bin_shift_for_capacity(capacity);
+    const uint32_t levels = static_cast<uint32_t>(pair_levels), pairs = bins_of_shift(capacity, shift) * levels;
+    if (shift != static_cast<uint32_t>(kBinSlotsLog2) || pairs >= (pos_dim == 4 ? kFineBinsMostPairs4d : kReduceWorkgroupsWanted)) return shift;
+    while (shift > static_cast<uint32_t>(kFinestBinSlotsLog2) && bins_of_shift(capacity, shift) * levels < kFineBinsWanted &&
+           bins_of_shift(capacity, shift - 1) <= static_cast<uint32_t>(kStageBins))
+        --shift;
+    return shift;
 }
 // A width is doubled only where it leaves more than kMaxBins bins, so wide bins are always more than half as many: their scatter is
 // that of many bins.
@@ -965,10 +987,10 @@ inline size_t bin_bytes_per_level(int pos_dim, uint32_t n_bins, uint32_t n_group
     return segments * (sizeof(uint32_t) + static_cast<size_t>(segment_capacity) * record_bytes(pos_dim, n_bins));
 }
 
-inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, int tiles_per_group, void* workspace,
+inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, uint32_t bin_shift, int tiles_per_group, void* workspace,
                          size_t bytes) {
     BinPlan p;
-    const uint32_t n_bins = bins_for_capacity(capacity);
+    const uint32_t n_bins = bins_of_shift(capacity, bin_shift);
     const uint32_t n_groups = scatter_groups(n, tiles_per_group);
     if (workspace == nullptr || n_bins > static_cast<uint32_t>(kMaxBins)) return p;
     // few contributions per slot: the reducer's fixed cost per bin (clearing and flushing 128 KiB of
@@ -997,13 +1019,13 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, int t
     const size_t fit = bytes / bin_bytes_per_level(pos_dim, n_bins, n_groups, cap);
     p.levels_per_pass = static_cast<int>(fit < static_cast<size_t>(levels) ? fit : static_cast<size_t>(levels));
     // wide bins are served by bin_reduce_levels_kernel only
-    if (bin_shift_for_capacity(capacity) != static_cast<uint32_t>(kBinSlotsLog2) &&
+    if (bin_shift > static_cast<uint32_t>(kBinSlotsLog2) &&
         (cap > kLevelsMaxSegment || n_groups > static_cast<uint32_t>(kReduceBlock)))
         return p;
     p.target.n_bins = n_bins;
     p.target.n_groups = n_groups;
     p.target.segment_capacity = cap;
-    p.target.bin_shift = bin_shift_for_capacity(capacity);
+    p.target.bin_shift = bin_shift;
     p.target.direct = reinterpret_cast<uint32_t*>(base);
     p.direct_bytes = flag_bytes;
     const uintptr_t counts_at = base + flag_bytes;
@@ -1117,19 +1139,20 @@ inline GroupSortPlan plan_group_sort(int pos_dim, int64_t n, int levels, int fea
 
 // Running consecutive passes on two streams (scatter pass p+1 while pass p is reduced) was tried and
 // measured 10-15% slower than one pass over all levels on one stream; hence a single stream.
-constexpr unsigned kReduceWorkgroupsWanted = 512;  // two per compute unit
+constexpr unsigned kReduceWorkgroupsWantedFine = 128;  // of narrow bins, which end sooner
 constexpr unsigned kMaxReduceSplits = 16;
 
 inline int reduce_bins(const BinPlan& p, const float* window, int first_level, int n_levels_in_pass, int capacity,
                        uint32_t feat_pairs, float* table_grad, hipStream_t st) {
     // enough workgroups for every compute unit, by letting several share a bin when bins*levels is small
     const unsigned pairs = p.target.n_bins * static_cast<unsigned>(n_levels_in_pass);
-    unsigned splits = pairs >= kReduceWorkgroupsWanted ? 1u : (kReduceWorkgroupsWanted + pairs - 1) / pairs;
+    const bool fine = p.target.bin_shift < static_cast<uint32_t>(kBinSlotsLog2);
+    unsigned splits = pairs >= (fine ? kReduceWorkgroupsWantedFine : kReduceWorkgroupsWanted) ? 1u : (kReduceWorkgroupsWanted + pairs - 1) / pairs;
     if (splits > p.target.n_groups) splits = p.target.n_groups;
     if (splits > kMaxReduceSplits) splits = kMaxReduceSplits;
     // many bins with a few thousand records each: workgroups that keep their bin and walk several levels
     // (bins wider than kBinSlots are planned only where this kernel can serve them)
-    const bool wide = p.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
+    const bool wide = p.target.bin_shift > static_cast<uint32_t>(kBinSlotsLog2);
     if (wide || (p.target.slots == nullptr && p.target.n_bins > static_cast<uint32_t>(kStageBins) && splits == 1 &&
                  p.target.segment_capacity <= kLevelsMaxSegment && p.target.n_groups <= static_cast<uint32_t>(kReduceBlock))) {
         const unsigned levels = static_cast<unsigned>(n_levels_in_pass);
@@ -1146,12 +1169,23 @@ inline int reduce_bins(const BinPlan& p, const float* window, int first_level, i
         return check_launch();
     }
     const dim3 grid(p.target.n_bins, n_levels_in_pass, splits);
-    if (p.target.slots != nullptr)
-        hipLaunchKernelGGL(bin_reduce_kernel<true>, grid, dim3(kReduceBlock), 0, st, p.target, window,
-                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level);
-    else
-        hipLaunchKernelGGL(bin_reduce_kernel<false>, grid, dim3(kReduceBlock), 0, st, p.target, window,
-                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level);
+#define PENC_LAUNCH_REDUCE(SPLIT, SLOTS_LOG2)                                                                                                       \
+    case SLOTS_LOG2:                                                                                                                                \
+        hipLaunchKernelGGL((bin_reduce_kernel<SPLIT, SLOTS_LOG2>), grid, dim3(reduce_threads(SLOTS_LOG2)), 0, st, p.target, window,                 \
+                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level);                                                  \
+        break;
+#define PENC_LAUNCH_REDUCE_ALL(SPLIT)                                                                                                               \
+    switch (p.target.bin_shift) {                                                                                                                   \
+        PENC_LAUNCH_REDUCE(SPLIT, 10) PENC_LAUNCH_REDUCE(SPLIT, 11) PENC_LAUNCH_REDUCE(SPLIT, 12) PENC_LAUNCH_REDUCE(SPLIT, 13)                     \
+    }
+    static_assert(kFinestBinSlotsLog2 == 10 && kBinSlotsLog2 == 13, "an instance for every width");
+    if (p.target.slots != nullptr) {
+        PENC_LAUNCH_REDUCE_ALL(true)
+    } else {
+        PENC_LAUNCH_REDUCE_ALL(false)
+    }
+#undef PENC_LAUNCH_REDUCE_ALL
+#undef PENC_LAUNCH_REDUCE
     return check_launch();
 }
 
@@ -1353,10 +1387,14 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
     }
     int tiles_per_group = table_backward_tiles(nr_positions, pair_levels);
     if (tiles_per_group > kScatterTiles && short_groups(pos_dim, feat_pairs, pair_levels, capacity, t.rows)) tiles_per_group = kScatterTiles;
-    BinPlan plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, workspace, workspace_bytes);
+    const uint32_t bin_shift = bin_shift_for_capacity(capacity), fine_shift = touched == nullptr ? fine_bin_shift(pos_dim, capacity, pair_levels) : bin_shift;
+    BinPlan plan;
+    if (fine_shift != bin_shift) plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, fine_shift, tiles_per_group, workspace, workspace_bytes);
+    if (!plan.enabled || plan.levels_per_pass < pair_levels)
+        plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, bin_shift, tiles_per_group, workspace, workspace_bytes);
     if (!plan.enabled && tiles_per_group > kScatterTiles) {  // wide bins need short segments: smaller groups of points
         tiles_per_group = kScatterTiles;
-        plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, workspace, workspace_bytes);
+        plan = plan_bins(pos_dim, nr_positions, pair_levels, capacity, bin_shift, tiles_per_group, workspace, workspace_bytes);
     }
     if (touched != nullptr) {
         plan.target.direct = touched;
@@ -1377,7 +1415,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         t.grid = dim3(padded_groups * static_cast<unsigned>(count));
         t.many_bins = plan.target.records != nullptr && plan.target.n_bins > static_cast<uint32_t>(kStageBins);
         t.most_bins = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins;
-        t.wide_bins = direct_flags != nullptr && plan.target.bin_shift != static_cast<uint32_t>(kBinSlotsLog2);
+        t.wide_bins = direct_flags != nullptr && plan.target.bin_shift > static_cast<uint32_t>(kBinSlotsLog2);
         t.first_level = first;
         t.n_pass_levels = static_cast<uint32_t>(count);
         t.dies = dies;
@@ -1618,9 +1656,19 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
     return sorted > binned ? sorted : binned;
 }
 
-size_t penc_scatter_deferred_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
+size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
     if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
-    const uint32_t n_bins = bins_for_capacity(capacity);
+    const uint32_t n_bins = bins_for_capacity(capacity), fine_shift = fine_bin_shift(pos_dim, capacity, nr_levels);
+    if (fine_shift != bin_shift_for_capacity(capacity)) {
+        const uint32_t fine = bins_of_shift(capacity, fine_shift);
+        size_t most = 0;
+        for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {
+            const size_t need = bin_bytes_per_level(pos_dim, fine, scatter_groups(nr_positions, tiles), wanted_segment_capacity(pos_dim, fine, tiles)) * nr_levels;
+            most = need > most ? need : most;
+        }
+        const size_t want = most + direct_flag_bytes(nr_levels, fine) + 8192, have = penc_scatter_workspace_bytes(pos_dim, nr_positions, nr_levels, capacity, nr_levels);
+        return want > have ? want - have : 0;
+    }
     if (n_bins > static_cast<uint32_t>(kMaxBins) || !clears_in_scatter(n_bins, nr_levels, capacity) || nr_positions * (pos_dim + 1) * kMinSlotsPerContribution <= capacity) return 0;
     size_t most = 0;
     for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {

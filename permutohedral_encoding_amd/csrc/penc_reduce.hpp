@@ -16,14 +16,16 @@ namespace penc {
 // runs (the scattering kernel before it has completed, and bins do not overlap), so the final add is
 // a plain coalesced read-modify-write; workgroups that share a bin add with atomics (consecutive
 // addresses: one request per 64 bytes).
-template <bool kSplit>  // whether the records are split (the host knows: BinTarget::slots)
-__global__ void __launch_bounds__(kReduceBlock)
+constexpr int reduce_threads(int slots_log2) { return slots_log2 >= 12 ? kReduceBlock : kReduceBlock / 2; }
+template <bool kSplit, int kSlotsLog2>  // whether the records are split (the host knows: BinTarget::slots), and the slots per bin
+__global__ void __launch_bounds__(reduce_threads(kSlotsLog2))
 bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs,
                   float* __restrict__ table_grad, int first_level) {
+    constexpr int kSlots = 1 << kSlotsLog2, kThreads = reduce_threads(kSlotsLog2);
     // one array per feature: lanes that hit different slots then spread over all bank pairs (interleaved
     // features would leave every other pair idle in each of the two adds)
-    __shared__ double acc0[kBinSlots];
-    __shared__ double acc1[kBinSlots];
+    __shared__ double acc0[kSlots];
+    __shared__ double acc1[kSlots];
     const uint32_t bin = blockIdx.x;
     // last level first: with the usual coarse-to-fine level list the bins with the most records are
     // started first and the nearly empty ones fill the tail of the launch
@@ -33,7 +35,7 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     const uint32_t level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
     if (window[level] == 0.0f) return;  // masked level: its scattering workgroups wrote no counts
     const BinTarget bins = bins_of_level(pass_bins, level_in_pass);
-    constexpr uint32_t kWaves = kReduceBlock / 64;
+    constexpr uint32_t kWaves = kThreads / 64;
     constexpr uint32_t kUnroll = 4;  // even
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t per_split = (bins.n_groups + gridDim.z - 1) / gridDim.z;
@@ -45,8 +47,8 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // range no point touches) ends here: the look at the counts overlaps the clearing of the sums,
     // and the barrier that follows the clearing carries the vote.
     bool any = false;
-    for (uint32_t g = group_begin + threadIdx.x; g < group_end; g += kReduceBlock) any = any || counts[g] != 0u;
-    for (int s = threadIdx.x; s < kBinSlots; s += kReduceBlock) {
+    for (uint32_t g = group_begin + threadIdx.x; g < group_end; g += kThreads) any = any || counts[g] != 0u;
+    for (int s = threadIdx.x; s < kSlots; s += kThreads) {
         acc0[s] = 0.0;
         acc1[s] = 0.0;
     }
@@ -194,29 +196,29 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     const bool untouched_so_far = bins.direct[bin] == 0u;
     __syncthreads();
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
-    const uint32_t slot0 = bin << kBinSlotsLog2;  // (this kernel serves bins of kBinSlots slots only)
+    const uint32_t slot0 = bin << kSlotsLog2;
     const bool alone = gridDim.z == 1;
     if (alone) {
         // all of a thread's read-modify-writes at once: the loads are issued together, not one per trip
-        constexpr int kMine = kBinSlots / kReduceBlock;
+        constexpr int kMine = kSlots / kThreads;
         float2 sum[kMine], g[kMine];
         bool touched[kMine];
 #pragma unroll
         for (int k = 0; k < kMine; ++k) {
-            const uint32_t s = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
+            const uint32_t s = static_cast<uint32_t>(k) * kThreads + threadIdx.x;
             const double v0 = acc0[s], v1 = acc1[s];
             sum[k] = make_float2(static_cast<float>(v0), static_cast<float>(v1));
             touched[k] = (v0 != 0.0 || v1 != 0.0) && slot0 + s < capacity;
         }
 #pragma unroll
         for (int k = 0; k < kMine; ++k) {
-            const uint32_t s = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
+            const uint32_t s = static_cast<uint32_t>(k) * kThreads + threadIdx.x;
             g[k] = make_float2(0.0f, 0.0f);
             if (touched[k] && !untouched_so_far) g[k] = *reinterpret_cast<const float2*>(level_grad.at(slot0 + s));
         }
 #pragma unroll
         for (int k = 0; k < kMine; ++k) {
-            const uint32_t s = static_cast<uint32_t>(k) * kReduceBlock + threadIdx.x;
+            const uint32_t s = static_cast<uint32_t>(k) * kThreads + threadIdx.x;
             if (touched[k]) {
                 g[k].x += sum[k].x;
                 g[k].y += sum[k].y;
@@ -231,7 +233,7 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // of 2^16 slots, four features, 2^18 points: 48 -> 34 us).
     const double* const acc = (threadIdx.x & 1u) != 0u ? acc1 : acc0;
 #pragma unroll 4
-    for (uint32_t s = threadIdx.x >> 1; s < static_cast<uint32_t>(kBinSlots); s += kReduceBlock / 2) {
+    for (uint32_t s = threadIdx.x >> 1; s < static_cast<uint32_t>(kSlots); s += kThreads / 2) {
         const double v = acc[s];
         if (v != 0.0 && slot0 + s < capacity) global_add(level_grad.at(slot0 + s) + (threadIdx.x & 1u), static_cast<float>(v));
     }

@@ -71,6 +71,7 @@ constexpr int kStageBins = 64;         // a wave counts one bin per lane: stagin
 constexpr int kWorkgroupSortMaxDim = 5;  // up to this input dimension a streaming workgroup sorts a tile's records across all its waves
 constexpr int kBinSlotsLog2 = 13;      // slots per bin: 8192 (128 KiB of fp64 sums in LDS)
 constexpr int kBinSlots = 1 << kBinSlotsLog2;
+constexpr int kFinestBinSlotsLog2 = 10;  // small tables get narrower bins, down to this
 constexpr int kMaxBins = 512;          // bins per level
 constexpr int kMaxBinSlotsLog2 = 16;   // tables of more than kMaxBins * kBinSlots slots (2^22) get bins of up to 2^16 slots, which their
                                        // reducer sums one range of kBinSlots slots after the other; above 2^25 slots nothing is binned
@@ -122,7 +123,7 @@ struct BinTarget {
     uint32_t n_bins;
     uint32_t n_groups;
     uint32_t segment_capacity;
-    uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records)
+    uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records), less for small tables
     uint32_t deferred_room;
     BinRecord* deferred;
     uint32_t* deferred_counts;
@@ -539,7 +540,7 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
     uvec<D + 1> place = 0u;  // rank of each record within its bin's run
     if (active) {
         static_for<D + 1>(PENC_BODY(j) {
-            PENC_INDEX(j); place[j] = atomicAdd(&count[slot[j] >> kBinSlotsLog2], 1u); });
+            PENC_INDEX(j); place[j] = atomicAdd(&count[slot[j] >> bins.bin_shift], 1u); });
     }
     __syncthreads();  // all waves have counted, and have left the staging array of the tile before
     const uint32_t mine = count[lane];
@@ -573,12 +574,12 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
                 constexpr int kFirst = part * kTogether, kCount = D + 1 - kFirst < kTogether ? D + 1 - kFirst : kTogether;
                 uint2 at[kCount];
                 static_for<kCount>(PENC_BODY(k) {
-                    PENC_INDEX(k); at[k] = run[slot[kFirst + k] >> kBinSlotsLog2]; });
+                    PENC_INDEX(k); at[k] = run[slot[kFirst + k] >> bins.bin_shift]; });
                 static_for<kCount>(PENC_BODY(k) {
                     PENC_INDEX(k);
                     constexpr int j = kFirst + k;
                     const float v0 = a0[j], v1 = a1[j];  // copies first: a bit cast applied directly to a vector element reads element 0
-                    stage[at[k].x + place[j]] = record_of(slot[j] & (kBinSlots - 1), v0, v1, at[k].y + place[j]);
+                    stage[at[k].x + place[j]] = record_of(slot[j] & ((1u << bins.bin_shift) - 1u), v0, v1, at[k].y + place[j]);
                 });
             });
         }
@@ -599,7 +600,7 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
         if (active) {
             static_for<D + 1>(PENC_BODY(j) {
                 PENC_INDEX(j);
-                const uint32_t b = slot[j] >> kBinSlotsLog2;
+                const uint32_t b = slot[j] >> bins.bin_shift;
                 const float v0 = a0[j], v1 = a1[j];
                 const uint2 at = run[b];
                 const uint32_t to = at.y + place[j];
@@ -615,7 +616,7 @@ __device__ __forceinline__ void stream_tile(State& c, const GradSlice& level_gra
             if (i < total) {
                 e = stage[i];
                 spill = e.w == kNoRoom;  // the segment is full: stage 3
-                if (!spill) store(make_uint4(e.x & (kBinSlots - 1), e.y, e.z, e.w));
+                if (!spill) store(make_uint4(e.x & ((1u << bins.bin_shift) - 1u), e.y, e.z, e.w));
             }
             if (__any(spill)) global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
         }
@@ -773,7 +774,7 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
         uvec<kStageChunk> place = 0u;  // rank of each record within its bin's run
         if (active) {
             static_for<kCount>(PENC_BODY(j) {
-                PENC_INDEX(j); place[j] = atomicAdd(&count[slot[kFirst + j] >> kBinSlotsLog2], 1u); });
+                PENC_INDEX(j); place[j] = atomicAdd(&count[slot[kFirst + j] >> bins.bin_shift], 1u); });
         }
         wave_lds_fence();
         // lane b looks after bin b: one reservation and one index computation per bin, not per record
@@ -788,13 +789,13 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
             if (active) {
                 uint2 at[kCount];
                 static_for<kCount>(PENC_BODY(j) {
-                    PENC_INDEX(j); at[j] = run[slot[kFirst + j] >> kBinSlotsLog2]; });
+                    PENC_INDEX(j); at[j] = run[slot[kFirst + j] >> bins.bin_shift]; });
                 static_for<kCount>(PENC_BODY(j) {
                     PENC_INDEX(j);
                     // copies first: a bit cast applied directly to a vector element reads element 0
                     const float v0 = a0[kFirst + j], v1 = a1[kFirst + j];
                     uint4 e;
-                    e.x = slot[kFirst + j] & (kBinSlots - 1);
+                    e.x = slot[kFirst + j] & ((1u << bins.bin_shift) - 1u);
                     e.y = __builtin_bit_cast(uint32_t, v0);
                     e.z = __builtin_bit_cast(uint32_t, v1);
                     e.w = at[j].y + place[j];
@@ -815,7 +816,7 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
             static_for<kCount>(PENC_BODY(j) {
                 PENC_INDEX(j);
                 if (active) {
-                    const uint32_t b = slot[kFirst + j] >> kBinSlotsLog2;
+                    const uint32_t b = slot[kFirst + j] >> bins.bin_shift;
                     const float v0 = a0[kFirst + j], v1 = a1[kFirst + j];
                     uint4 e;
                     e.x = slot[kFirst + j];
@@ -834,7 +835,7 @@ __device__ __forceinline__ void stream_tile_wave(State& c, const GradSlice& leve
                 if (i < total) {
                     e = stage[i];
                     spill = e.w == kNoRoom;  // the segment is full: stage 3
-                    if (!spill) store_whole_record(bins, make_uint4(e.x & (kBinSlots - 1), e.y, e.z, e.w));
+                    if (!spill) store_whole_record(bins, make_uint4(e.x & ((1u << bins.bin_shift) - 1u), e.y, e.z, e.w));
                 }
                 if (__any(spill))
                     global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));

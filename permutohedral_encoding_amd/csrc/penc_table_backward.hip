@@ -90,7 +90,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     if (w_level == 0.0f) return;
     scatter_begin(state);
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
-    if constexpr (!kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
+    if constexpr (kManyBins && !kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
                                2 * feat_pairs, bins.direct, bins.bin_shift,
                                kMayDefer && bins.deferred != nullptr ? bins.deferred + static_cast<size_t>(group) * bins.deferred_room : nullptr, &state.deferred};

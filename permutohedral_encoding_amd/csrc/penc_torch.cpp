@@ -66,7 +66,7 @@ struct Api {
     PENC_FN(forward_rowmajor);
     PENC_FN(forward_rowmajor_workspace_bytes);
     PENC_FN(scatter_workspace_bytes);
-    PENC_FN(scatter_deferred_bytes);
+    PENC_FN(scatter_extra_bytes);
     PENC_FN(positions_workspace_bytes);
     PENC_FN(backward);
     PENC_FN(backward_half);
@@ -220,15 +220,15 @@ Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t cop
     const int64_t pair_levels = static_cast<int64_t>(c.levels) * (c.feat / 2);
     int64_t per_pass = c.levels_per_pass <= 0 ? pair_levels : std::min(c.levels_per_pass, pair_levels);
     if (!table || c.levels_per_pass < 0) per_pass = 0;
-    // (asked for once, with all levels in a pass: a dense gradient's lists of deferred adds)
-    int64_t lists = per_pass == pair_levels && c.sparse_owner == nullptr
-                        ? static_cast<int64_t>(api.scatter_deferred_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels), c.capacity))
+    // (asked for once, with all levels in a pass: what a dense gradient can use besides)
+    int64_t extra = per_pass == pair_levels && c.sparse_owner == nullptr
+                        ? static_cast<int64_t>(api.scatter_extra_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels), c.capacity))
                         : 0;
     while (true) {
         int64_t want = per_pass > 0 ? static_cast<int64_t>(api.scatter_workspace_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels),
                                                                                       c.capacity, static_cast<int>(per_pass)))
                                     : 0;
-        want = std::max(want, pos_bytes) + copy_bytes + lists;
+        want = std::max(want, pos_bytes) + copy_bytes + extra;
         if (c.max_workspace < 0 || want <= c.max_workspace) {
             if (want == 0) return {};
             try {
@@ -236,8 +236,8 @@ Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t cop
             } catch (const c10::OutOfMemoryError&) {
             }
         }
-        if (lists > 0) {
-            lists = 0;
+        if (extra > 0) {
+            extra = 0;
         } else if (per_pass > 1) {
             per_pass /= 2;
         } else if (per_pass == 1 || pos_bytes > 0) {
@@ -1121,7 +1121,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(forward_rowmajor);
         PENC_FN(forward_rowmajor_workspace_bytes);
         PENC_FN(scatter_workspace_bytes);
-        PENC_FN(scatter_deferred_bytes);
+        PENC_FN(scatter_extra_bytes);
         PENC_FN(positions_workspace_bytes);
         PENC_FN(backward);
         PENC_FN(backward_half);
