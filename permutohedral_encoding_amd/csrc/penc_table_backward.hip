@@ -41,17 +41,17 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // share their geometry: "levels" below (first_level, n_pass_levels, the grid, the bins) count pairs,
 // `pair_level` = level * feat_pairs + pair.  The upstream gradient needs no special case: [L][F][N]
 // is [L * F/2][2][N], and in a row the pair sits at column 2 * pair_level.
-// kManyBins: the records go to more than kStageBins bins (stream_tile_many).  Instances of their own, so that neither sort's registers are spilled for
-// the other's sake.
-// kWideBins: the bins span more than kBinSlots slots (tables above 2^22 slots).  A parameter of the kernel
+// kBins: what the bins are.  Many: the records go to more than kStageBins bins (stream_tile_many), so that neither sort's registers are spilled
+// for the other's sake.  Wide: of more than kBinSlots slots (tables above 2^22 slots), narrow: of fewer (small tables).  A parameter of the kernel
 // rather than a value read from its arguments, because with the bin width a variable the usual instances
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
+enum BinKind : int { kBinsFew = 0, kBinsNarrow = 1, kBinsMany = 2, kBinsWide = 3 };
 // kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
 // a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
 // reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
 enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
-template <int D, bool kRowMajor, int kOrder, bool kManyBins, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, int kOrder, int kBins, int kThreads>
 __device__ __forceinline__ void
 scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
                         uint32_t capacity, uint32_t cap_mask,
@@ -60,7 +60,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                         const float* __restrict__ grad_sliced, int64_t grad_row_stride,
                         const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
                         float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
-    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders;
+    constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders, kManyBins = kBins >= kBinsMany;
     __shared__ ScatterStateT<stage_chunk(D), kThreads> state;
     __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kThreads : 1];
     // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
@@ -90,7 +90,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     if (w_level == 0.0f) return;
     scatter_begin(state);
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
-    if constexpr (kManyBins && !kWideBins) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
+    if constexpr (kBins == kBinsFew || kBins == kBinsMany) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
                                2 * feat_pairs, bins.direct, bins.bin_shift,
                                kMayDefer && bins.deferred != nullptr ? bins.deferred + static_cast<size_t>(group) * bins.deferred_room : nullptr, &state.deferred};
@@ -286,15 +286,15 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
 #define PENC_TABLE_ARGUMENTS                                                                                                        \
     n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
         random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
-template <int D, bool kRowMajor, bool kSecond, bool kManyBins, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, bool kSecond, int kBins, int kThreads>
 __global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kThreads))
 backward_table_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kManyBins, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kSecond ? kSecondOrder : kFirstOrder, kBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
-template <int D, bool kRowMajor, bool kManyBins, bool kWideBins, int kThreads>
+template <int D, bool kRowMajor, int kBins, int kThreads>
 __global__ void __launch_bounds__(kThreads, both_orders_waves_per_simd(D, kThreads))
 backward_table_both_kernel(PENC_TABLE_PARAMETERS) {
-    scatter_group_of_points<D, kRowMajor, kBothOrders, kManyBins, kWideBins, kThreads>(PENC_TABLE_ARGUMENTS);
+    scatter_group_of_points<D, kRowMajor, kBothOrders, kBins, kThreads>(PENC_TABLE_ARGUMENTS);
 }
 #undef PENC_TABLE_PARAMETERS
 #undef PENC_TABLE_ARGUMENTS
@@ -580,15 +580,17 @@ void launch_table_backward(const TableLaunch& t) {
                        t.feat_pairs, t.dies, t.tiles_per_group / (THREADS / kScatterBlock), t.capacity, t.cap_mask, t.positions,       \
                        t.scale_factor, t.random_shift, t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad,          \
                        t.table_grad, t.grad_level_major, t.bins)
-#define PENC_LAUNCH_WIDTH(KERNEL, ...)                                            \
-    if (t.wide_bins) {                                                            \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true, true);    \
-    } else if (t.most_bins) {                                                     \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, true, false);   \
-    } else if (t.many_bins) {                                                     \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, true, false);           \
-    } else {                                                                      \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, false, false);          \
+#define PENC_LAUNCH_WIDTH(KERNEL, ...)                                          \
+    if (t.wide_bins) {                                                          \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, kBinsWide);   \
+    } else if (t.most_bins) {                                                   \
+        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, kBinsMany);   \
+    } else if (t.many_bins) {                                                   \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsMany);           \
+    } else if (t.bins.records != nullptr && t.bins.bin_shift < static_cast<uint32_t>(kBinSlotsLog2)) { \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsNarrow);         \
+    } else {                                                                    \
+        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsFew);            \
     }
     if (t.second_grad != nullptr) {
         if (t.rows) {

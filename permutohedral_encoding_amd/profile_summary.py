@@ -79,7 +79,7 @@ def is_ours(kernel):
 def order_of_table_gradient(kernel):
     """Phase of a kernel that makes records of a table gradient, None for any other kernel."""
     args = template_args(kernel)
-    if base_name(kernel) == "backward_table_kernel":  # <D, kRowMajor, kSecondOrder, kManyBins, kWideBins, kThreads>
+    if base_name(kernel) == "backward_table_kernel":  # <D, kRowMajor, kSecondOrder, kBins, kThreads>
         return "double_backward" if len(args) >= 3 and args[2] == "true" else "backward"
     if base_name(kernel) == "group_sort_kernel":      # <D, kRowMajor, kOrder>: first, second, both
         return "double_backward" if len(args) >= 3 and args[2] == "2" else "backward"
