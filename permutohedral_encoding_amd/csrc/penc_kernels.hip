@@ -1569,7 +1569,7 @@ static int backward_impl(int pos_dim, int nr_feat, int64_t nr_positions, int nr_
     return PENC_OK;
 }
 
-// The levels of an fp32 table that a forward gathers from cells made for it (chosen_columns_kernel).
+// The levels of an fp32 table that a forward gathers from cells made for it (chosen_cells_kernel).
 struct ChosenCells {
     const void* cells = nullptr;
     const uint32_t* levels = nullptr;
