@@ -394,6 +394,7 @@ class EncodingWrapper:
     _half_copy = None
     _half_copy_of = None
     _cells = None      # (key, copy, stream, event): the 16-bit copy in cells (penc_table_cells), where enough points have been gathered for it
+    _cells_line = None  # (capacity, half_table, penc_table_cells_points of them)
     _gathered = None   # (key, points): how many were, without it, since the table was last modified
     # set by the module (sparse_table_grad=True): table gradients are added into `sparse_grad`, a SparseTableGrad the
     # wrapper keeps across calls, and the gradient calls return None for them
@@ -410,12 +411,13 @@ class EncodingWrapper:
     def _half_key(self, lattice_values):
         return (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, tuple(lattice_values.shape), self.half_table)
 
-    def gather_table(self, lattice_values):
+    def gather_table(self, lattice_values, key=None):
         """The tensor the gathering kernels read for ``lattice_values``: the tensor itself, or, with
         ``half_table``, its 16-bit copy, made again whenever the tensor has been modified in place."""
         if self.half_table is None or lattice_values.dtype != torch.float32:
             return lattice_values
-        key = self._half_key(lattice_values)
+        if key is None:
+            key = self._half_key(lattice_values)
         if self._half_copy_of != key:
             self._half_copy = lattice_values.detach().to(self.half_table)
             self._half_copy_of = key
@@ -425,7 +427,7 @@ class EncodingWrapper:
         """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
         is made once the points gathered since the table was last modified are enough (penc_table_cells_points; four times as many while
         the table is trained, whose next version may be a step away), from the 16-bit copy if there is one."""
-        if lattice_values.dtype != torch.float32 or lattice_values.dim() != 3 or not lattice_values.is_cuda or not lattice_values.is_contiguous():
+        if lattice_values.dtype != torch.float32 or not lattice_values.is_contiguous():
             return self.gather_table(lattice_values), False
         key = self._half_key(lattice_values)
         cells = self._cells
@@ -438,23 +440,29 @@ class EncodingWrapper:
                     cells[1].record_stream(stream)
                 return cells[1], True
             self._cells = cells = None
-        points = lib().penc_table_cells_points(self.nr_feat, lattice_values.shape[1], TABLE_FORMATS[self.half_table])
-        if points < 0 or lattice_values.shape[2] != self.nr_feat or positions.dim() != 2:
-            return self.gather_table(lattice_values), False
+        if not lattice_values.is_cuda or lattice_values.dim() != 3:
+            return self.gather_table(lattice_values, key), False
+        _, capacity, feat = key[3]
+        line = self._cells_line
+        if line is None or line[0] != capacity or line[1] != self.half_table:
+            line = self._cells_line = (capacity, self.half_table, lib().penc_table_cells_points(self.nr_feat, capacity, TABLE_FORMATS[self.half_table]))
+        points = line[2]
+        if points < 0 or feat != self.nr_feat or positions.dim() != 2:
+            return self.gather_table(lattice_values, key), False
         if lattice_values.requires_grad and torch.is_grad_enabled():
             points *= 4
         gathered = self._gathered
         so_far = positions.shape[0] + (gathered[1] if gathered is not None and gathered[0] == key else 0)
         self._gathered = (key, so_far)
         if so_far < points:
-            return self.gather_table(lattice_values), False
+            return self.gather_table(lattice_values, key), False
         if torch.cuda.is_current_stream_capturing():  # (a copy whose making is captured holds nothing before the graph runs)
-            return self.gather_table(lattice_values), False
+            return self.gather_table(lattice_values, key), False
         rounded = self._half_copy_of == key  # it stays: a captured graph may read it
         try:
             copy = (_bridge or bridge()).table_in_cells(self._half_copy if rounded else lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
         except torch.cuda.OutOfMemoryError:
-            return self.gather_table(lattice_values), False
+            return self.gather_table(lattice_values, key), False
         if not rounded:
             self._half_copy = self._half_copy_of = None
         stream = torch.cuda.current_stream(lattice_values.device)

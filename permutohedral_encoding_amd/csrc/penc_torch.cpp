@@ -428,7 +428,7 @@ public:
 // The forward by way of a copy of the table in cells, where that pays and there is memory for it; false: not done.  `rows` is undefined where
 // the result is `level_major`, which else is scratch and may be undefined; `slopes` where none are kept.
 bool forward_in_cells(const Call& c, Tensor level_major, const Tensor& rows, const Tensor& slopes) {
-    if (c.table_format != 0) return false;
+    if (c.table_format != 0 || c.n * c.levels < (int64_t{1} << 20)) return false;  // (far below where it pays: such calls wait for the host)
     const size_t n = api.forward_cells_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, rows.defined() ? static_cast<int>(c.columns()) : 0);
     if (n == 0 || (c.max_workspace >= 0 && static_cast<int64_t>(n) > c.max_workspace)) return false;
     Tensor ws;
