@@ -426,7 +426,7 @@ class EncodingWrapper:
     def _copy_to_gather(self, lattice_values, positions):
         """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
         is made once the points gathered since the table was last modified are enough (penc_table_cells_points; four times as many while
-        the table is trained, whose next version may be a step away), from the 16-bit copy if there is one."""
+        the table is trained, whose next version may be a step away)."""
         if lattice_values.dtype != torch.float32 or not lattice_values.is_contiguous():
             return self.gather_table(lattice_values), False
         key = self._half_key(lattice_values)
@@ -458,12 +458,12 @@ class EncodingWrapper:
             return self.gather_table(lattice_values, key), False
         if torch.cuda.is_current_stream_capturing():  # (a copy whose making is captured holds nothing before the graph runs)
             return self.gather_table(lattice_values, key), False
-        rounded = self._half_copy_of == key  # it stays: a captured graph may read it
         try:
-            copy = (_bridge or bridge()).table_in_cells(self._half_copy if rounded else lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
+            # (never from the 16-bit copy: another stream may still be filling it, or a captured graph that has not run)
+            copy = (_bridge or bridge()).table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
         except torch.cuda.OutOfMemoryError:
             return self.gather_table(lattice_values, key), False
-        if not rounded:
+        if self._half_copy_of != key:  # (one of this version stays: a captured graph may read it)
             self._half_copy = self._half_copy_of = None
         stream = torch.cuda.current_stream(lattice_values.device)
         self._cells = (key, copy, stream.cuda_stream, stream.record_event())

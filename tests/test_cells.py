@@ -270,6 +270,43 @@ def test_copy_made_on_one_stream_is_waited_for_on_another():
     assert torch.equal(got, want)
 
 
+def busy(work, times=20):
+    for _ in range(times):
+        work = (work @ work).clamp(-1, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("captured", [False, True])
+def test_cells_are_made_of_the_table_where_its_16_bit_copy_is_not_filled_yet(captured):
+    """The 16-bit copy waits for what its stream has to do, or for the first replay of the graph that makes it, when a call on another stream gathers
+    enough for cells: they hold the table's values all the same, then and later."""
+    import permutohedral_encoding_amd as pe
+    levels, cap = 12, 1 << 20
+    m = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=torch.bfloat16)
+    plain = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels))
+    plain.load_state_dict(m.state_dict())
+    few, many = torch.rand(1000, 3, device="cuda"), torch.rand(pe._native.lib().penc_table_cells_points(2, cap, 2), 3, device="cuda")
+    work, side, graph = torch.randn(4096, 4096, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.no_grad():
+        plain.lattice_values.copy_(plain.lattice_values.bfloat16().float())
+        want_few, want_many = plain(few), plain(many)
+        plain(few[:10])
+        torch.cuda.synchronize()
+        if captured:
+            with torch.cuda.graph(graph):
+                first = m(few)
+        else:
+            with torch.cuda.stream(side):
+                busy(work)
+                first = m(few)
+        got = m(many)
+        assert m.lattice._cells is not None
+        torch.cuda.synchronize()
+        if captured:
+            graph.replay()
+        assert torch.equal(got, want_many) and torch.equal(first, want_few) and torch.equal(m(few), want_few)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [False, True])
 def test_forward_by_way_of_cells_keeps_to_the_workspace_cap(monkeypatch, rows):
