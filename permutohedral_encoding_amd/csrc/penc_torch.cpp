@@ -1017,11 +1017,14 @@ PyObject* py_table_in_cells(PyObject*, PyObject* const* args, Py_ssize_t n_args)
             NoGil no_gil;
             at::NoGradGuard no_grad;
             const c10::DeviceGuard device(table.device());
+            // The library reads a slot at a time.  A table that begins elsewhere, such as a view into flattened parameters, is rounded first.
+            const bool in_slots = (reinterpret_cast<uintptr_t>(table.const_data_ptr()) & (std::min<size_t>(feat * table.element_size(), 16) - 1)) == 0;
+            const Tensor from = in_slots ? table : table.to(type, /*non_blocking=*/false, /*copy=*/true);
             cells = at::empty(table.sizes(), table.options().dtype(type));
             const size_t n = api.table_cells_workspace_bytes(feat, levels, capacity, format);
             const Tensor ws = at::empty({static_cast<int64_t>(n)}, table.options().dtype(at::kByte));
-            check(api.table_cells(pos_dim, feat, levels, capacity, table.const_data_ptr(), fp32 ? 0 : format, format, cells.mutable_data_ptr(),
-                                  ws.mutable_data_ptr(), n, current_stream(table.device())),
+            check(api.table_cells(pos_dim, feat, levels, capacity, from.const_data_ptr(), fp32 && in_slots ? 0 : format, format,
+                                  cells.mutable_data_ptr(), ws.mutable_data_ptr(), n, current_stream(table.device())),
                   "table_cells");
         }
         return THPVariable_Wrap(std::move(cells));

@@ -308,6 +308,24 @@ def test_cells_are_made_of_the_table_where_its_16_bit_copy_is_not_filled_yet(cap
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("feat", [2, 4, 8])
+def test_cells_of_a_table_that_does_not_begin_at_a_slot(feat):
+    """A view into flattened parameters, one float into them: its 16-bit copy has always served, and so do the cells made of it."""
+    import permutohedral_encoding_amd as pe
+    levels, cap = 4, 1 << 14
+    m = pe.PermutoEncoding(3, cap, levels, feat, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=torch.bfloat16)
+    flat = torch.randn(m.lattice_values.numel() + 1, device="cuda")
+    m.lattice_values = torch.nn.Parameter(flat[1:].view(levels, cap, feat))
+    many = torch.rand(pe._native.lib().penc_table_cells_points(feat, cap, 2), 3, device="cuda")
+    with torch.no_grad():
+        few = m(many[:100])
+        assert m.lattice._cells is None
+        m.invalidate_half_table()
+        got = m(many)
+    assert m.lattice._cells is not None and torch.equal(got[:100], few)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [False, True])
 def test_forward_by_way_of_cells_keeps_to_the_workspace_cap(monkeypatch, rows):
     import permutohedral_encoding_amd as pe
