@@ -391,9 +391,11 @@ class EncodingWrapper:
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table
-    _half_copy = None
-    _half_copy_of = None
-    _cells = None      # (key, copy, stream, event): the 16-bit copy in cells (penc_table_cells), where enough points have been gathered for it
+    # Copies kept with what they were made of and when: (key, copy, stream, event).  One attribute each, so that threads never see one's
+    # copy with another's key.
+    _half_copy = None  # in 16 bits
+    _cells = None      # in 16 bits and in cells (penc_table_cells), where enough points have been gathered for it
+    _captured = None   # ((key, capture, stream), copy): in 16 bits, made by a call that is captured: for that capture's calls alone
     _cells_line = None  # (capacity, half_table, penc_table_cells_points of them)
     _gathered = None   # (key, points): how many were, without it, since the table was last modified
     # set by the module (sparse_table_grad=True): table gradients are added into `sparse_grad`, a SparseTableGrad the
@@ -418,10 +420,41 @@ class EncodingWrapper:
             return lattice_values
         if key is None:
             key = self._half_key(lattice_values)
-        if self._half_copy_of != key:
-            self._half_copy = lattice_values.detach().to(self.half_table)
-            self._half_copy_of = key
-        return self._half_copy
+        kept = self._half_copy
+        if kept is not None and kept[0] == key:
+            return self._for_this_stream(kept)
+        if not lattice_values.is_cuda:
+            return lattice_values.detach().to(self.half_table)  # (for the checks, which refuse it)
+        capture = (_bridge or bridge()).capture_id(lattice_values.get_device())
+        if capture:
+            # what is recorded now holds nothing until the graph runs, and then only for what the same graph runs after it
+            made_for = (key, capture, torch._C._cuda_getCurrentRawStream(lattice_values.get_device()))
+            captured = self._captured
+            if captured is None or captured[0] != made_for:
+                captured = self._captured = (made_for, lattice_values.detach().to(self.half_table))
+            return captured[1]
+        copy = lattice_values.detach().to(self.half_table)
+        self._half_copy = self._made_now(key, copy)
+        return copy
+
+    @staticmethod
+    def _made_now(key, copy):
+        with torch.cuda.device(copy.device):
+            event = torch.cuda.Event()
+            event.record()
+            return (key, copy, torch._C._cuda_getCurrentRawStream(copy.get_device()), event)
+
+    @staticmethod
+    def _for_this_stream(kept):
+        """The copy of a ``_made_now``.  It was made in the middle of a program, by a call on some stream: one on another stream waits for it, and
+        keeps its memory from reuse."""
+        copy = kept[1]
+        if kept[2] != torch._C._cuda_getCurrentRawStream(copy.get_device()):
+            stream = torch.cuda.current_stream(copy.device)
+            if not (_bridge or bridge()).capture_id(copy.get_device()):
+                stream.wait_event(kept[3])
+                copy.record_stream(stream)
+        return copy
 
     def _copy_to_gather(self, lattice_values, positions):
         """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
@@ -433,12 +466,7 @@ class EncodingWrapper:
         cells = self._cells
         if cells is not None:
             if cells[0] == key:
-                # it was made in the middle of a program, by a call on some stream: one on another stream waits for it, and keeps it from reuse
-                if cells[2] != torch._C._cuda_getCurrentRawStream(lattice_values.get_device()) and not torch.cuda.is_current_stream_capturing():
-                    stream = torch.cuda.current_stream(lattice_values.device)
-                    stream.wait_event(cells[3])
-                    cells[1].record_stream(stream)
-                return cells[1], True
+                return self._for_this_stream(cells), True
             self._cells = cells = None
         if not lattice_values.is_cuda or lattice_values.dim() != 3:
             return self.gather_table(lattice_values, key), False
@@ -456,17 +484,17 @@ class EncodingWrapper:
         self._gathered = (key, so_far)
         if so_far < points:
             return self.gather_table(lattice_values, key), False
-        if torch.cuda.is_current_stream_capturing():  # (a copy whose making is captured holds nothing before the graph runs)
+        if (_bridge or bridge()).capture_id(lattice_values.get_device()):  # (a copy whose making is captured holds nothing before the graph runs)
             return self.gather_table(lattice_values, key), False
         try:
-            # (never from the 16-bit copy: another stream may still be filling it, or a captured graph that has not run)
+            # (never from the 16-bit copy, which another stream may still be filling)
             copy = (_bridge or bridge()).table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
         except torch.cuda.OutOfMemoryError:
             return self.gather_table(lattice_values, key), False
-        if self._half_copy_of != key:  # (one of this version stays: a captured graph may read it)
-            self._half_copy = self._half_copy_of = None
-        stream = torch.cuda.current_stream(lattice_values.device)
-        self._cells = (key, copy, stream.cuda_stream, stream.record_event())
+        kept = self._half_copy
+        if kept is not None and kept[0] != key:  # (one of this version stays: a captured graph may read it)
+            self._half_copy = None
+        self._cells = self._made_now(key, copy)
         return copy, True
 
     def invalidate_half_table(self):
@@ -475,8 +503,8 @@ class EncodingWrapper:
         advance; a write that bypasses it (``p.data.add_(...)``, a kernel given the raw pointer) does not,
         and must be followed by this call."""
         self._half_copy = None
-        self._half_copy_of = None
         self._cells = None
+        self._captured = None
         self._gathered = None
 
     def _check_common(self, inp):

@@ -1000,6 +1000,22 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     });
 }
 
+// capture_id(device) -> the id of the capture that the device's current stream takes part in, 0 where it takes part in none
+PyObject* py_capture_id(PyObject*, PyObject* device) {
+    return guarded([&]() -> PyObject* {
+        const long index = PyLong_AsLong(device);
+        if (PyErr_Occurred()) return nullptr;
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(static_cast<c10::DeviceIndex>(index)).stream();
+        if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {  // (the default stream while another is captured)
+            (void)hipGetLastError();
+            status = hipStreamCaptureStatusNone;
+        }
+        return PyLong_FromUnsignedLongLong(status == hipStreamCaptureStatusNone ? 0 : id + 1);
+    });
+}
+
 // table_in_cells(table, table_format, pos_dim) -> the table (fp32, or already of that format) as a 16-bit copy in cells
 PyObject* py_table_in_cells(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
@@ -1156,6 +1172,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
     {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},
     {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},
     {"cosine_window", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_cosine_window)), METH_FASTCALL, "a coarse-to-fine window"},
     {"adamw_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step)), METH_FASTCALL, "one AdamW step"},

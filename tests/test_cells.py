@@ -308,6 +308,67 @@ def test_cells_are_made_of_the_table_where_its_16_bit_copy_is_not_filled_yet(cap
 
 
 @pytest.mark.gpu
+def test_a_16_bit_copy_made_on_one_stream_is_waited_for_on_another():
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 20, 12, 2, np.geomspace(1.0, 1e-3, 12), lattice_half_precision=torch.float16)
+    few = torch.rand(1000, 3, device="cuda")
+    work, side = torch.randn(4096, 4096, device="cuda"), torch.cuda.Stream()
+    with torch.no_grad():
+        want = m(few)
+        m.invalidate_half_table()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            busy(work)
+            m(few)
+        got = m(few)  # beside the other stream's work, but for the copy
+        again = m(few)
+    torch.cuda.synchronize()
+    assert m.lattice._half_copy[2] == side.cuda_stream and torch.equal(got, want) and torch.equal(again, want)
+
+
+@pytest.mark.gpu
+def test_a_16_bit_copy_that_a_capture_makes_is_that_captures_alone():
+    """Neither a call outside, before the graph has run, nor another graph reads it; the calls of one capture share it."""
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 16, 6, 2, np.geomspace(1.0, 1e-3, 6), lattice_half_precision=torch.bfloat16)
+    few, other = torch.rand(1000, 3, device="cuda"), torch.rand(1000, 3, device="cuda")
+    with torch.no_grad():
+        want, want_other = m(few), m(other)
+        first, second = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+        m.invalidate_half_table()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(first):
+            a = m(few)
+            made = m.lattice._captured[1]
+            b = m(other)
+            assert m.lattice._captured[1] is made
+        assert m.lattice._half_copy is None
+        with torch.cuda.graph(second):
+            c = m(few)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):  # (never run) a stream that takes part in a capture begun on another
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                m(few)
+            torch.cuda.current_stream().wait_stream(side)
+        third = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(third):
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                d = m(few)
+            torch.cuda.current_stream().wait_stream(side)
+        assert torch.equal(m(few), want)
+        for graph, outs, wants in ((second, (c,), (want,)), (third, (d,), (want,)), (first, (a, b), (want, want_other))):
+            for _ in range(3):
+                for out in outs:
+                    out.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert all(torch.equal(x, y) for x, y in zip(outs, wants))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("feat", [2, 4, 8])
 def test_cells_of_a_table_that_does_not_begin_at_a_slot(feat):
     """A view into flattened parameters, one float into them: its 16-bit copy has always served, and so do the cells made of it."""
