@@ -450,8 +450,10 @@ class EncodingWrapper:
         keeps its memory from reuse."""
         copy = kept[1]
         if kept[2] != torch._C._cuda_getCurrentRawStream(copy.get_device()):
-            stream = torch.cuda.current_stream(copy.device)
-            if not (_bridge or bridge()).capture_id(copy.get_device()):
+            if (_bridge or bridge()).capture_id(copy.get_device()):
+                _bridge.wait_for_event(kept[3].cuda_event)  # (a graph cannot wait for what is outside it: the host does, before the graph can run)
+            else:
+                stream = torch.cuda.current_stream(copy.device)
                 stream.wait_event(kept[3])
                 copy.record_stream(stream)
         return copy

@@ -1016,6 +1016,20 @@ PyObject* py_capture_id(PyObject*, PyObject* device) {
     });
 }
 
+// wait_for_event(handle): on the host, also while this thread captures a graph
+PyObject* py_wait_for_event(PyObject*, PyObject* handle) {
+    return guarded([&]() -> PyObject* {
+        const auto event = static_cast<hipEvent_t>(PyLong_AsVoidPtr(handle));
+        if (PyErr_Occurred()) return nullptr;
+        {
+            NoGil no_gil;
+            c10::hip::HIPStreamCaptureModeGuard in_a_capture_too{hipStreamCaptureModeRelaxed};
+            C10_HIP_CHECK(hipEventSynchronize(event));
+        }
+        Py_RETURN_NONE;
+    });
+}
+
 // table_in_cells(table, table_format, pos_dim) -> the table (fp32, or already of that format) as a 16-bit copy in cells
 PyObject* py_table_in_cells(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
@@ -1173,6 +1187,7 @@ PyMethodDef methods[] = {
     {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
     {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
     {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},
+    {"wait_for_event", py_wait_for_event, METH_O, "waits on the host for an event"},
     {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},
     {"cosine_window", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_cosine_window)), METH_FASTCALL, "a coarse-to-fine window"},
     {"adamw_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step)), METH_FASTCALL, "one AdamW step"},

@@ -327,6 +327,34 @@ def test_a_16_bit_copy_made_on_one_stream_is_waited_for_on_another():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cells", [False, True])
+def test_a_capture_waits_for_a_copy_made_on_another_stream(cells):
+    """A graph captured and replayed while the stream that makes the copy is busy with other things."""
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 20, 12, 2, np.geomspace(1.0, 1e-3, 12), lattice_half_precision=torch.bfloat16)
+    few, many = torch.rand(1000, 3, device="cuda"), torch.rand(pe._native.lib().penc_table_cells_points(2, 1 << 20, 2), 3, device="cuda")
+    work, side, graph = torch.randn(4096, 4096, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.no_grad():
+        want = m(few)
+        m.invalidate_half_table()
+        torch.cuda.synchronize()
+        busy(work)
+        m(many if cells else few)
+        with torch.cuda.stream(side):
+            graph.capture_begin()
+            got = m(few)
+            graph.capture_end()
+            graph.replay()
+        side.synchronize()
+        assert (m.lattice._cells is not None) == cells and m.lattice._captured is None and torch.equal(got, want)
+        for _ in range(2):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 def test_a_16_bit_copy_that_a_capture_makes_is_that_captures_alone():
     """Neither a call outside, before the graph has run, nor another graph reads it; the calls of one capture share it."""
     import permutohedral_encoding_amd as pe
