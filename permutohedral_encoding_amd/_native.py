@@ -383,7 +383,7 @@ class EncodingWrapper:
         fp = self.fixed_params
         table, in_cells = lattice_values, False
         if self.half_table is not None:
-            table, in_cells = self._copy_to_gather(lattice_values, positions)
+            table, in_cells = self._copy_to_gather(lattice_values, positions, anneal_window)
         return (_bridge or bridge()).encode(
             lattice_values, table, positions,
             anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,
@@ -458,7 +458,7 @@ class EncodingWrapper:
                 copy.record_stream(stream)
         return copy
 
-    def _copy_to_gather(self, lattice_values, positions):
+    def _copy_to_gather(self, lattice_values, positions, anneal_window):
         """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
         is made once the points gathered since the table was last modified are enough (penc_table_cells_points; four times as many while
         the table is trained, whose next version may be a step away)."""
@@ -487,6 +487,8 @@ class EncodingWrapper:
         if so_far < points:
             return self.gather_table(lattice_values, key), False
         if (_bridge or bridge()).capture_id(lattice_values.get_device()):  # (a copy whose making is captured holds nothing before the graph runs)
+            return self.gather_table(lattice_values, key), False
+        if (_bridge or bridge()).needs_autograd_functions(lattice_values, positions, anneal_window):  # (they gather from the copy in the table's order)
             return self.gather_table(lattice_values, key), False
         try:
             # (never from the 16-bit copy, which another stream may still be filling)

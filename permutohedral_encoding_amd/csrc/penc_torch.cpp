@@ -938,6 +938,15 @@ bool needs_autograd_functions(const Tensor& lattice_values, const Tensor& positi
            (window.requires_grad() && c10::GradMode::is_enabled());
 }
 
+// needs_autograd_functions(lattice_values, positions, window) -> whether encode() would return None
+PyObject* py_needs_autograd_functions(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 3, "needs_autograd_functions takes 3 arguments");
+        return PyBool_FromLong(needs_autograd_functions(tensor_arg(args[0], "lattice_values"), tensor_arg(args[1], "positions"),
+                                                        tensor_arg(args[2], "anneal_window")));
+    });
+}
+
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
 //        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params, in_cells)
 //   -> (N, F(L+E)), or None where the autograd functions are needed
@@ -1186,6 +1195,8 @@ PyObject* py_bind(PyObject*, PyObject* path) {
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
     {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"needs_autograd_functions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_needs_autograd_functions)), METH_FASTCALL,
+     "whether a call is for the autograd functions of funcs.py"},
     {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},
     {"wait_for_event", py_wait_for_event, METH_O, "waits on the host for an event"},
     {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},

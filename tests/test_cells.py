@@ -327,6 +327,22 @@ def test_a_16_bit_copy_made_on_one_stream_is_waited_for_on_another():
 
 
 @pytest.mark.gpu
+def test_no_cells_are_made_for_a_call_that_would_not_gather_from_them():
+    """A window that requires a gradient is for the autograd functions, which gather from the copy in the table's order."""
+    import permutohedral_encoding_amd as pe
+    levels, cap = 6, 1 << 16
+    m = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=torch.bfloat16)
+    m.lattice_values.requires_grad_(False)
+    many = torch.rand(pe._native.lib().penc_table_cells_points(2, cap, 2), 3, device="cuda")
+    window = torch.ones(levels, device="cuda", requires_grad=True)
+    with torch.no_grad():
+        want = m(many, window)
+    m.invalidate_half_table()
+    got = m(many, window)
+    assert m.lattice._cells is None and m.lattice._half_copy is not None and torch.equal(got.detach(), want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cells", [False, True])
 def test_a_capture_waits_for_a_copy_made_on_another_stream(cells):
     """A graph captured and replayed while the stream that makes the copy is busy with other things."""
