@@ -477,7 +477,7 @@ class EncodingWrapper:
         if line is None or line[0] != capacity or line[1] != self.half_table:
             line = self._cells_line = (capacity, self.half_table, lib().penc_table_cells_points(self.nr_feat, capacity, TABLE_FORMATS[self.half_table]))
         points = line[2]
-        if points < 0 or feat != self.nr_feat or positions.dim() != 2:
+        if points < 0 or feat != self.nr_feat or not isinstance(positions, torch.Tensor) or positions.dim() != 2:  # (refused later)
             return self.gather_table(lattice_values, key), False
         if lattice_values.requires_grad and torch.is_grad_enabled():
             points *= 4

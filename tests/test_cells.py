@@ -343,6 +343,17 @@ def test_no_cells_are_made_for_a_call_that_would_not_gather_from_them():
 
 
 @pytest.mark.gpu
+def test_positions_that_are_no_tensor_are_refused_as_ever():
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 16, 4, 2, np.geomspace(1.0, 1e-3, 4), lattice_half_precision=torch.bfloat16)
+    for bad in ([[0.0, 0.0, 0.0]], np.zeros((4, 3), np.float32), 1.0):
+        with pytest.raises(ValueError, match="must be a torch.Tensor"):
+            m(bad)
+    with pytest.raises(ValueError, match="should have 2 dimensions"):
+        m(torch.rand(3, device="cuda"))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cells", [False, True])
 def test_a_capture_waits_for_a_copy_made_on_another_stream(cells):
     """A graph captured and replayed while the stream that makes the copy is busy with other things."""
