@@ -243,6 +243,7 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
 TABLE_FORMATS = {torch.float16: 1, torch.bfloat16: 2}  # PENC_TABLE_FP16, PENC_TABLE_BF16 (include/penc.h)
 
 
@@ -380,24 +381,24 @@ class EncodingWrapper:
         one call into the extension, whose autograd nodes reach the library without entering the interpreter.
         None under a functorch transform, with a forward-mode tangent, with a window that requires a gradient and in a trace: those
         are for the functions of ``funcs.py``."""
-        fp = self.fixed_params
-        table, in_cells = lattice_values, False
+        fp, table, encode = self.fixed_params, lattice_values, (_bridge or bridge()).encode
         if self.half_table is not None:
             table, in_cells = self._copy_to_gather(lattice_values, positions, anneal_window)
-        return (_bridge or bridge()).encode(
+            if in_cells:
+                encode = _bridge.encode_from_cells
+        return encode(
             lattice_values, table, positions,
             anneal_window, fp.m_random_shift_per_level, fp.m_scale_factor, self.pos_dim, self.nr_feat, fp.m_concat_points,
-            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES, fp, in_cells)
+            fp.m_points_scaling, self if self.sparse_table_grad else None, self.rows_output, LEVELS_PER_PASS, MAX_WORKSPACE_BYTES, fp)
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table
-    # Copies kept with what they were made of and when: (key, copy, stream, event).  One attribute each, so that threads never see one's
+    # Copies kept with what they were made of and when: (key, copy, device, stream, event).  One attribute each, so that threads never see one's
     # copy with another's key.
-    _half_copy = None  # in 16 bits
+    _half_copy = None  # in 16 bits; behind the event the points from which cells are worth having (< 0: never) and a list of the points gathered so far
     _cells = None      # in 16 bits and in cells (penc_table_cells), where enough points have been gathered for it
     _captured = None   # ((key, capture, stream), copy): in 16 bits, made by a call that is captured: for that capture's calls alone
-    _cells_line = None  # (capacity, half_table, penc_table_cells_points of them)
-    _gathered = None   # (key, points): how many were, without it, since the table was last modified
+    _cells_line = None  # ((capacity, half_table), penc_table_cells_points of them)
     # set by the module (sparse_table_grad=True): table gradients are added into `sparse_grad`, a SparseTableGrad the
     # wrapper keeps across calls, and the gradient calls return None for them
     sparse_table_grad = False
@@ -411,11 +412,12 @@ class EncodingWrapper:
         return self.sparse_grad
 
     def _half_key(self, lattice_values):
-        return (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, tuple(lattice_values.shape), self.half_table)
+        return (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, lattice_values.shape, self.half_table)
 
-    def gather_table(self, lattice_values, key=None):
+    def gather_table(self, lattice_values, key=None, points=0):
         """The tensor the gathering kernels read for ``lattice_values``: the tensor itself, or, with
-        ``half_table``, its 16-bit copy, made again whenever the tensor has been modified in place."""
+        ``half_table``, its 16-bit copy, made again whenever the tensor has been modified in place (``points``: what the call that
+        makes it gathers)."""
         if self.half_table is None or lattice_values.dtype != torch.float32:
             return lattice_values
         if key is None:
@@ -428,78 +430,97 @@ class EncodingWrapper:
         capture = (_bridge or bridge()).capture_id(lattice_values.get_device())
         if capture:
             # what is recorded now holds nothing until the graph runs, and then only for what the same graph runs after it
-            made_for = (key, capture, torch._C._cuda_getCurrentRawStream(lattice_values.get_device()))
+            made_for = (key, capture, _raw_stream(lattice_values.get_device()))
             captured = self._captured
             if captured is None or captured[0] != made_for:
                 captured = self._captured = (made_for, lattice_values.detach().to(self.half_table))
             return captured[1]
         copy = lattice_values.detach().to(self.half_table)
-        self._half_copy = self._made_now(key, copy)
+        self._half_copy = self._made_now(key, copy) + (self._points_for_cells(lattice_values), [points])
         return copy
 
     @staticmethod
     def _made_now(key, copy):
-        with torch.cuda.device(copy.device):
+        device = copy.get_device()
+        with torch.cuda.device(device):
             event = torch.cuda.Event()
             event.record()
-            return (key, copy, torch._C._cuda_getCurrentRawStream(copy.get_device()), event)
+            return (key, copy, device, _raw_stream(device), event)
 
     @staticmethod
     def _for_this_stream(kept):
         """The copy of a ``_made_now``.  It was made in the middle of a program, by a call on some stream: one on another stream waits for it, and
         keeps its memory from reuse."""
-        copy = kept[1]
-        if kept[2] != torch._C._cuda_getCurrentRawStream(copy.get_device()):
-            if (_bridge or bridge()).capture_id(copy.get_device()):
-                _bridge.wait_for_event(kept[3].cuda_event)  # (a graph cannot wait for what is outside it: the host does, before the graph can run)
+        _, copy, device, stream, event, *_ = kept
+        if stream != _raw_stream(device):
+            if (_bridge or bridge()).capture_id(device):
+                _bridge.wait_for_event(event.cuda_event)  # (a graph cannot wait for what is outside it: the host does, before the graph can run)
             else:
-                stream = torch.cuda.current_stream(copy.device)
-                stream.wait_event(kept[3])
-                copy.record_stream(stream)
+                here = torch.cuda.current_stream(device)
+                here.wait_event(event)
+                copy.record_stream(here)
         return copy
+
+    def _points_for_cells(self, lattice_values):
+        """From how many points a copy of ``lattice_values`` is worth having in cells; < 0: never."""
+        if (lattice_values.dtype != torch.float32 or not lattice_values.is_cuda or lattice_values.dim() != 3 or not lattice_values.is_contiguous()
+                or lattice_values.shape[2] != self.nr_feat):
+            return -1
+        line, of = self._cells_line, (lattice_values.shape[1], self.half_table)
+        if line is None or line[0] != of:
+            line = self._cells_line = (of, lib().penc_table_cells_points(self.nr_feat, of[0], TABLE_FORMATS[self.half_table]))
+        return line[1]
 
     def _copy_to_gather(self, lattice_values, positions, anneal_window):
         """-> (``gather_table`` or the same values in cells, whether in cells).  A copy in cells takes longer to make and less to gather from: it
         is made once the points gathered since the table was last modified are enough (penc_table_cells_points; four times as many while
-        the table is trained, whose next version may be a step away)."""
-        if lattice_values.dtype != torch.float32 or not lattice_values.is_contiguous():
-            return self.gather_table(lattice_values), False
-        key = self._half_key(lattice_values)
-        cells = self._cells
-        if cells is not None:
-            if cells[0] == key:
-                return self._for_this_stream(cells), True
-            self._cells = cells = None
-        if not lattice_values.is_cuda or lattice_values.dim() != 3:
-            return self.gather_table(lattice_values, key), False
-        _, capacity, feat = key[3]
-        line = self._cells_line
-        if line is None or line[0] != capacity or line[1] != self.half_table:
-            line = self._cells_line = (capacity, self.half_table, lib().penc_table_cells_points(self.nr_feat, capacity, TABLE_FORMATS[self.half_table]))
-        points = line[2]
-        if points < 0 or feat != self.nr_feat or not isinstance(positions, torch.Tensor) or positions.dim() != 2:  # (refused later)
-            return self.gather_table(lattice_values, key), False
-        if lattice_values.requires_grad and torch.is_grad_enabled():
-            points *= 4
-        gathered = self._gathered
-        so_far = positions.shape[0] + (gathered[1] if gathered is not None and gathered[0] == key else 0)
-        self._gathered = (key, so_far)
-        if so_far < points:
-            return self.gather_table(lattice_values, key), False
-        if (_bridge or bridge()).capture_id(lattice_values.get_device()):  # (a copy whose making is captured holds nothing before the graph runs)
-            return self.gather_table(lattice_values, key), False
-        if (_bridge or bridge()).needs_autograd_functions(lattice_values, positions, anneal_window):  # (they gather from the copy in the table's order)
-            return self.gather_table(lattice_values, key), False
+        the table is trained, whose next version may be a step away).  A small batch waits for what is done here: the question whether a table can
+        be in cells at all is asked once per copy."""
+        key = (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, lattice_values.shape, self.half_table)  # (_half_key)
+        kept = self._cells
+        if kept is not None:
+            if kept[0] == key and lattice_values.is_contiguous():
+                return kept[1] if kept[3] == _raw_stream(kept[2]) else self._for_this_stream(kept), True
+            self._cells = None
+        half = self._half_copy
+        if half is not None and half[0] == key:
+            points = half[5]
+            if points < 0:
+                return half[1] if half[3] == _raw_stream(half[2]) else self._for_this_stream(half), False
+        else:
+            half, points = None, self._points_for_cells(lattice_values)
+        try:
+            so_far = len(positions)
+        except TypeError:  # (what is no tensor of points is refused later)
+            so_far = 0
+        if points >= 0:
+            if half is not None:
+                half[6][0] += so_far
+                so_far = half[6][0]
+            if so_far >= points:
+                cells = self._make_cells(lattice_values, positions, anneal_window, key, so_far, points)
+                if cells is not None:
+                    return cells, True
+        return (self.gather_table(lattice_values, key, so_far) if half is None else self._for_this_stream(half)), False
+
+    def _make_cells(self, lattice_values, positions, anneal_window, key, so_far, points):
+        if lattice_values.requires_grad and torch.is_grad_enabled() and so_far < 4 * points:
+            return None
+        native = _bridge or bridge()
+        if native.capture_id(lattice_values.get_device()):  # (a copy whose making is captured holds nothing before the graph runs)
+            return None
+        if native.needs_autograd_functions(lattice_values, positions, anneal_window):  # (they gather from the copy in the table's order)
+            return None
         try:
             # (never from the 16-bit copy, which another stream may still be filling)
-            copy = (_bridge or bridge()).table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
+            copy = native.table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
         except torch.cuda.OutOfMemoryError:
-            return self.gather_table(lattice_values, key), False
+            return None
         kept = self._half_copy
         if kept is not None and kept[0] != key:  # (one of this version stays: a captured graph may read it)
             self._half_copy = None
         self._cells = self._made_now(key, copy)
-        return copy, True
+        return copy
 
     def invalidate_half_table(self):
         """Forgets the 16-bit copy, so that the next call converts the table again.  The copy follows the
@@ -509,7 +530,6 @@ class EncodingWrapper:
         self._half_copy = None
         self._cells = None
         self._captured = None
-        self._gathered = None
 
     def _check_common(self, inp):
         fp = self.fixed_params

@@ -425,10 +425,12 @@ public:
 // ------------------------------------------------------------------------------------------
 // the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
 
+// Whether forward_in_cells is worth a call: small batches, far below where it pays, wait for the host.
+bool may_go_by_cells(const Call& c) { return c.table_format == 0 && c.n * c.levels >= (int64_t{1} << 20); }
+
 // The forward by way of a copy of the table in cells, where that pays and there is memory for it; false: not done.  `rows` is undefined where
 // the result is `level_major`, which else is scratch and may be undefined; `slopes` where none are kept.
 bool forward_in_cells(const Call& c, Tensor level_major, const Tensor& rows, const Tensor& slopes) {
-    if (c.table_format != 0 || c.n * c.levels < (int64_t{1} << 20)) return false;  // (far below where it pays: such calls wait for the host)
     const size_t n = api.forward_cells_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, rows.defined() ? static_cast<int>(c.columns()) : 0);
     if (n == 0 || (c.max_workspace >= 0 && static_cast<int64_t>(n) > c.max_workspace)) return false;
     Tensor ws;
@@ -459,7 +461,7 @@ Tensor compute_forward(const Call& c, std::shared_ptr<Slopes>& slopes) {
             slopes.reset();
         }
         if (slopes != nullptr) {
-            if (!forward_in_cells(c, level_major, as_rows ? out : Tensor(), kept))
+            if (!may_go_by_cells(c) || !forward_in_cells(c, level_major, as_rows ? out : Tensor(), kept))
                 check(api.forward_slopes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), c.table.const_data_ptr(), c.table_format,
                                          data(c.scale_factor), data(c.shift), data(c.window), mutable_data(level_major),
                                          as_rows ? mutable_data(out) : nullptr, c.columns(), mutable_data(kept), c.concat, c.scaling, stream),
@@ -468,7 +470,7 @@ Tensor compute_forward(const Call& c, std::shared_ptr<Slopes>& slopes) {
             return out;
         }
     }
-    if (as_rows ? forward_in_cells(c, {}, out, {}) : forward_in_cells(c, out, {}, {})) return out;
+    if (may_go_by_cells(c) && (as_rows ? forward_in_cells(c, {}, out, {}) : forward_in_cells(c, out, {}, {}))) return out;
     if (as_rows) {
         const Tensor ws = bytes(c, api.forward_rowmajor_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.concat));
         check(api.forward_rowmajor(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor),
@@ -948,11 +950,13 @@ PyObject* py_needs_autograd_functions(PyObject*, PyObject* const* args, Py_ssize
 }
 
 // encode(lattice_values, table, positions, window, random_shift, scale_factor, pos_dim, nr_feat, concat_points, points_scaling,
-//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params, in_cells)
+//        sparse_owner or None, rows_output, levels_per_pass, max_workspace_bytes or None, fixed_params)
 //   -> (N, F(L+E)), or None where the autograd functions are needed
+// encode_from_cells: the same from a table that is a copy in cells (table_in_cells)
+template <bool kInCells>
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
-        TORCH_CHECK(n_args == 16, "encode takes 16 arguments");
+        TORCH_CHECK(n_args == 15, "encode takes 15 arguments");
         TORCH_CHECK(api.forward != nullptr, "bind() has not been called");
         const Tensor& lattice_values = tensor_arg(args[0], "lattice_values");
         const Tensor& positions = tensor_arg(args[2], "positions");
@@ -970,7 +974,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         c.concat = PyObject_IsTrue(args[8]);
         c.scaling = static_cast<float>(PyFloat_AsDouble(args[9]));
         c.rows_output = PyObject_IsTrue(args[11]);
-        c.in_cells = PyObject_IsTrue(args[15]);
+        c.in_cells = kInCells;
         c.levels_per_pass = PyLong_AsLongLong(args[12]);
         c.max_workspace = args[13] == Py_None ? -1 : PyLong_AsLongLong(args[13]);
         if (PyErr_Occurred()) return nullptr;
@@ -1194,7 +1198,8 @@ PyObject* py_bind(PyObject*, PyObject* path) {
 
 PyMethodDef methods[] = {
     {"bind", py_bind, METH_O, "takes the C ABI from the library at the given path"},
-    {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"encode", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode<false>)), METH_FASTCALL, "the encoding of a batch, differentiable"},
+    {"encode_from_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_encode<true>)), METH_FASTCALL, "the same from a copy in cells"},
     {"needs_autograd_functions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_needs_autograd_functions)), METH_FASTCALL,
      "whether a call is for the autograd functions of funcs.py"},
     {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},

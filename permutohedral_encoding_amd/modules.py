@@ -141,7 +141,10 @@ class PermutoEncoding(torch.nn.Module):
 
     def forward(self, positions, anneal_window=None):
         if not self.lattice.calls_replaced():
-            out = self.lattice.encode(self.lattice_values, positions, self.anneal_window if anneal_window is None else anneal_window)
+            # (a small batch waits for the host: 0.4 us less than the attribute, which a module finds after everything else)
+            lattice_values = self._parameters.get("lattice_values")
+            out = self.lattice.encode(self.lattice_values if lattice_values is None else lattice_values, positions,
+                                      self.anneal_window if anneal_window is None else anneal_window)
             if out is not None:
                 return out
         nr_positions = positions.shape[0]

@@ -323,7 +323,7 @@ def test_a_16_bit_copy_made_on_one_stream_is_waited_for_on_another():
         got = m(few)  # beside the other stream's work, but for the copy
         again = m(few)
     torch.cuda.synchronize()
-    assert m.lattice._half_copy[2] == side.cuda_stream and torch.equal(got, want) and torch.equal(again, want)
+    assert m.lattice._half_copy[3] == side.cuda_stream and torch.equal(got, want) and torch.equal(again, want)
 
 
 @pytest.mark.gpu
