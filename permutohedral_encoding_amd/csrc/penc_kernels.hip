@@ -869,6 +869,7 @@ struct BinPlan {
     bool enabled = false;
     int levels_per_pass = 0;
     BinTarget target{};       // of the first pass; target.direct covers all levels, a pass starts at its first level's flags
+    ClearTarget clear{};      // (plan_deferred)
     size_t direct_bytes = 0;  // size of target.direct (to be cleared with the gradient)
     uintptr_t end = 0;        // of what is used of the workspace
 };
@@ -1049,7 +1050,7 @@ constexpr size_t kClearInScatterBytes = size_t{64} << 20;
 inline bool clears_in_scatter(uint32_t n_bins, int pair_levels, int capacity) {
     return n_bins > static_cast<uint32_t>(kStageBins) && static_cast<size_t>(pair_levels) * capacity * sizeof(float2) >= kClearInScatterBytes;
 }
-// What the lists of deferred adds (BinTarget) take behind the bins, for all levels at once.
+// What the lists of deferred adds (ClearTarget) take behind the bins, for all levels at once.
 inline size_t deferred_bytes(int pos_dim, int pair_levels, uint32_t n_groups, int tiles_per_group) {
     return static_cast<size_t>(pair_levels) * n_groups * (deferred_room(pos_dim, tiles_per_group) * sizeof(BinRecord) + sizeof(uint32_t)) + 512;
 }
@@ -1061,11 +1062,11 @@ inline bool plan_deferred(BinPlan& p, int pos_dim, int pair_levels, int capacity
     if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0 || (static_cast<int64_t>(pair_levels) * capacity) % 2 != 0) return false;
     const uintptr_t base = (p.end + 255u) & ~uintptr_t{255};
     if (base + deferred_bytes(pos_dim, pair_levels, p.target.n_groups, tiles_per_group) > reinterpret_cast<uintptr_t>(workspace) + bytes) return false;
-    p.target.deferred_room = deferred_room(pos_dim, tiles_per_group);
-    p.target.deferred = reinterpret_cast<BinRecord*>(base);
-    p.target.deferred_counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.target.deferred_room * sizeof(BinRecord));
-    p.target.clear_quads = static_cast<uint64_t>(pair_levels) * capacity / 2;
-    p.target.clear_flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
+    p.clear.room = deferred_room(pos_dim, tiles_per_group);
+    p.clear.kept = reinterpret_cast<BinRecord*>(base);
+    p.clear.counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.clear.room * sizeof(BinRecord));
+    p.clear.quads = static_cast<uint64_t>(pair_levels) * capacity / 2;
+    p.clear.flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
     return true;
 }
 
@@ -1421,13 +1422,14 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         t.dies = dies;
         t.tiles_per_group = tiles_per_group;
         t.bins = plan.target;
+        t.clear = plan.clear;
         PENC_DISPATCH_D(pos_dim, launch_table_backward<DD>(t));
         if (int rc = check_launch()) return rc;
         if (plan.enabled)
             if (int rc = reduce_bins(plan, anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
     }
-    if (plan.target.deferred != nullptr) {
-        hipLaunchKernelGGL(add_deferred_kernel, dim3(plan.target.n_groups, static_cast<unsigned>(pair_levels)), dim3(kBlock), 0, st, plan.target, anneal_window,
+    if (plan.clear.kept != nullptr) {
+        hipLaunchKernelGGL(add_deferred_kernel, dim3(plan.target.n_groups, static_cast<unsigned>(pair_levels)), dim3(kBlock), 0, st, plan.clear, anneal_window,
                            cap, feat_pairs, lattice_values_grad);
         return check_launch();
     }

@@ -239,14 +239,14 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     }
 }
 
-// Adds what a scattering kernel that cleared the gradient has kept (BinTarget::deferred): a workgroup to a group of points and a level.
+// Adds what a scattering kernel that cleared the gradient has kept (ClearTarget::kept): a workgroup to a group of points and a level.
 __global__ void __launch_bounds__(kBlock)
-add_deferred_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs, float* __restrict__ table_grad) {
+add_deferred_kernel(ClearTarget clear, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs, float* __restrict__ table_grad) {
     const uint32_t group = blockIdx.x, pair_level = blockIdx.y, level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
     if (window[level] == 0.0f) return;  // masked level: its scattering workgroups wrote no counts
-    const BinTarget bins = bins_of_level(pass_bins, pair_level);
-    const uint32_t count = bins.deferred_counts[group];
-    const BinRecord* const kept = bins.deferred + static_cast<size_t>(group) * bins.deferred_room;
+    const size_t list = static_cast<size_t>(pair_level) * gridDim.x + group;
+    const uint32_t count = clear.counts[list];
+    const BinRecord* const kept = clear.kept + list * clear.room;
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
     for (uint32_t first = 0; first < count; first += kBlock) {
         const uint32_t i = first + threadIdx.x;

@@ -107,14 +107,8 @@ constexpr size_t kSplitRecordBytes = sizeof(RecordValues) + sizeof(uint16_t);
 //                                                  for a caller who keeps gradient and flags across calls (the sparse
 //                                                  entry points), the caller's map of touched slot ranges.
 // `records` == nullptr disables binning (`direct`, `n_bins` and `bin_shift` may still be set: flags without bins).
-//
-// Large tables (`deferred` set; more than kStageBins bins, all levels in one launch): the scattering kernel clears the gradient and the flags
-// itself, each workgroup a share of them when it starts, because those writes pass while it waits for other things (2^22 slots, 24 levels,
-// 16 of them live, 2^20 points: fill 134 and scatter 329 us apart, 373 together; 200001 points 163 and 90, 184).  Nothing may
-// be added to a gradient that another workgroup is still to clear, so what would go straight into it is kept until the reducers have ended, and
-// add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
-//   deferred         [level_in_pass][group][deferred_room]   {slot in the level, values}; there is room for all a group can leave
-//   deferred_counts  [level_in_pass][group]
+// (Every kernel of a small batch begins with a fetch of its arguments, a cache line at a time: with the fields of ClearTarget in here too, a third
+// line for the same code, bin_reduce_kernel took 14.4 us where it takes 14.1, and the table gradient of 131007 points along rays 0.6 us longer in all.)
 struct BinTarget {
     void* records;
     uint16_t* slots;
@@ -124,11 +118,25 @@ struct BinTarget {
     uint32_t n_groups;
     uint32_t segment_capacity;
     uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records), less for small tables
-    uint32_t deferred_room;
-    BinRecord* deferred;
-    uint32_t* deferred_counts;
-    uint64_t clear_quads;   // 16-byte units of the gradient, where the scattering kernel clears it,
-    uint32_t clear_flags;   // and its flags
+};
+// Large tables (more than kStageBins bins, all levels in one launch; kept == nullptr: not): the scattering kernel clears the gradient and the flags
+// itself, each workgroup a share of them when it starts, because those writes pass while it waits for other things (2^22 slots, 24 levels,
+// 16 of them live, 2^20 points: fill 134 and scatter 329 us apart, 373 together; 200001 points 163 and 90, 184).  Nothing may
+// be added to a gradient that another workgroup is still to clear, so what would go straight into it is kept until the reducers have ended, and
+// add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
+//   kept    [level_in_pass][group][room]   {slot in the level, values}; there is room for all a group can leave
+//   counts  [level_in_pass][group]
+struct ClearTarget {
+    BinRecord* kept;
+    uint32_t* counts;
+    uint64_t quads;   // 16-byte units of the gradient,
+    uint32_t flags;   // and its flags
+    uint32_t room;
+};
+// What instances for few bins are given instead.
+struct NoClearTarget {
+    NoClearTarget() = default;
+    explicit NoClearTarget(const ClearTarget&) {}
 };
 // What a group of points can leave for later at a level: all its contributions, and the lines its cache claimed.
 constexpr uint32_t deferred_room(int pos_dim, int tiles_per_group) {
@@ -146,10 +154,6 @@ __device__ __forceinline__ BinTarget bins_of_level(const BinTarget& pass, uint32
         t.counts += segments;
     }
     if (pass.direct != nullptr) t.direct += static_cast<size_t>(k) * pass.n_bins;
-    if (pass.deferred != nullptr) {
-        t.deferred += static_cast<size_t>(k) * pass.n_groups * pass.deferred_room;
-        t.deferred_counts += static_cast<size_t>(k) * pass.n_groups;
-    }
     return t;
 }
 
@@ -230,7 +234,7 @@ struct GradSlice {
     uint32_t slot_floats;
     uint32_t* direct;
     uint32_t bin_shift;  // of the bins `direct` belongs to
-    BinRecord* deferred;       // nullptr: adds go into the gradient; else the workgroup's list of them (see BinTarget),
+    BinRecord* deferred;       // nullptr: adds go into the gradient; else the workgroup's list of them (see ClearTarget),
     uint32_t* deferred_count;  // in LDS: how many are in it
     __device__ __forceinline__ float* at(uint32_t slot) const { return base + static_cast<size_t>(slot) * slot_floats; }
     // A plain store on purpose: many workgroups may set the same flag at once, all to 1, and nobody reads it before the
@@ -438,7 +442,6 @@ __device__ __forceinline__ void scatter_begin(State& c) {
         c.misses = 0u;
         c.strangers = 0u;
         c.columns = 0u;
-        c.deferred = 0u;
     }
     __syncthreads();
 }
@@ -1137,7 +1140,6 @@ __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_gra
         const uint32_t n = c.bin_count[b];
         bins.counts[static_cast<size_t>(b) * bins.n_groups + group] = n < bins.segment_capacity ? n : bins.segment_capacity;
     }
-    if (level_grad.deferred != nullptr && threadIdx.x == 0) bins.deferred_counts[group] = c.deferred;
 }
 
 }  // namespace penc

@@ -2,6 +2,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "penc_group_sort.hpp"
 #include "penc_lattice.hpp"
 #include "penc_scatter.hpp"
@@ -46,6 +48,8 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // rather than a value read from its arguments, because with the bin width a variable the usual instances
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
 enum BinKind : int { kBinsFew = 0, kBinsNarrow = 1, kBinsMany = 2, kBinsWide = 3 };
+template <int kBins>
+using ClearTargetOf = std::conditional_t<(kBins >= kBinsMany), ClearTarget, NoClearTarget>;
 // kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
 // a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
@@ -59,7 +63,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                         const float* __restrict__ random_shift, const float* __restrict__ window,
                         const float* __restrict__ grad_sliced, int64_t grad_row_stride,
                         const float* __restrict__ double_pos_grad, const float* __restrict__ second_grad,
-                        float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins) {
+                        float* __restrict__ table_grad, float* __restrict__ grad_level_major, const BinTarget& pass_bins,
+                        const ClearTargetOf<kBins>& clear) {
     constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders, kManyBins = kBins >= kBinsMany;
     __shared__ ScatterStateT<stage_chunk(D), kThreads> state;
     __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kThreads : 1];
@@ -71,15 +76,14 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     // a time).
     const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
     const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
-    constexpr bool kMayDefer = kManyBins;
-    if constexpr (kMayDefer) {
-        if (pass_bins.deferred != nullptr) {
+    if constexpr (kManyBins) {
+        if (clear.kept != nullptr) {
             typedef float Quad __attribute__((ext_vector_type(4)));
-            const uint64_t share = (pass_bins.clear_quads + gridDim.x - 1) / gridDim.x, from = share * blockIdx.x;
-            const uint64_t to = from + share < pass_bins.clear_quads ? from + share : pass_bins.clear_quads;
+            const uint64_t share = (clear.quads + gridDim.x - 1) / gridDim.x, from = share * blockIdx.x;
+            const uint64_t to = from + share < clear.quads ? from + share : clear.quads;
             for (uint64_t i = from + threadIdx.x; i < to; i += kThreads) __builtin_nontemporal_store(Quad(0.0f), reinterpret_cast<Quad*>(table_grad) + i);
             const uint32_t flag = blockIdx.x * kThreads + threadIdx.x;
-            if (flag < pass_bins.clear_flags) pass_bins.direct[flag] = 0u;
+            if (flag < clear.flags) pass_bins.direct[flag] = 0u;
         }
     }
     const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kThreads;
@@ -88,12 +92,16 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     const int level = static_cast<int>(pair_level / feat_pairs);  // the geometry's level
     const float w_level = window[level];
     if (w_level == 0.0f) return;
+    BinRecord* deferred = nullptr;
+    if constexpr (kManyBins) {
+        if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
+        if (threadIdx.x == 0) state.deferred = 0u;
+    }
     scatter_begin(state);
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     if constexpr (kBins == kBinsFew || kBins == kBinsMany) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
-                               2 * feat_pairs, bins.direct, bins.bin_shift,
-                               kMayDefer && bins.deferred != nullptr ? bins.deferred + static_cast<size_t>(group) * bins.deferred_room : nullptr, &state.deferred};
+                               2 * feat_pairs, bins.direct, bins.bin_shift, deferred, &state.deferred};
     // Everything a thread reads lies within its group of at most 16 x 512 points, so the addresses are
     // wave-uniform 64-bit bases (scalar registers) plus 32-bit per-thread offsets in bytes: the form the load instructions take.
     const uint32_t last_in_group = static_cast<uint32_t>(n_points - 1 - group_base);
@@ -275,6 +283,9 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s1 = s1_next;
     }
     scatter_end<D, kManyBins>(state, level_grad, bins, group, mode, id_bits, cursor);
+    if constexpr (kManyBins) {
+        if (deferred != nullptr && threadIdx.x == 0) clear.counts[static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group] = state.deferred;
+    }
 }
 
 #define PENC_TABLE_PARAMETERS                                                                                                          \
@@ -282,10 +293,10 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         uint32_t cap_mask, const float *__restrict__ positions, const float *__restrict__ scale_factor,                                \
         const float *__restrict__ random_shift, const float *__restrict__ window, const float *__restrict__ grad_sliced,               \
         int64_t grad_row_stride, const float *__restrict__ double_pos_grad, const float *__restrict__ second_grad,                     \
-        float *__restrict__ table_grad, float *__restrict__ grad_level_major, BinTarget pass_bins
+        float *__restrict__ table_grad, float *__restrict__ grad_level_major, BinTarget pass_bins, ClearTargetOf<kBins> clear
 #define PENC_TABLE_ARGUMENTS                                                                                                        \
     n_points, first_level, n_pass_levels, feat_pairs, dies, tiles_per_group, capacity, cap_mask, positions, scale_factor,           \
-        random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins
+        random_shift, window, grad_sliced, grad_row_stride, double_pos_grad, second_grad, table_grad, grad_level_major, pass_bins, clear
 template <int D, bool kRowMajor, bool kSecond, int kBins, int kThreads>
 __global__ void __launch_bounds__(kThreads, scatter_waves_per_simd(D, kThreads))
 backward_table_kernel(PENC_TABLE_PARAMETERS) {
@@ -575,22 +586,22 @@ template void launch_group_sort<PENC_DIM>(const TableLaunch& t, const GroupSort&
 template <int D>
 void launch_table_backward(const TableLaunch& t) {
     // (a group of points is the same for all instances: half the tiles of twice the points)
-#define PENC_LAUNCH(THREADS, ...)                                                                                                      \
-    hipLaunchKernelGGL((__VA_ARGS__, THREADS>), t.grid, dim3(THREADS), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,        \
+#define PENC_LAUNCH(THREADS, BINS, ...)                                                                                                \
+    hipLaunchKernelGGL((__VA_ARGS__, BINS, THREADS>), t.grid, dim3(THREADS), 0, t.stream, t.n_points, t.first_level, t.n_pass_levels,  \
                        t.feat_pairs, t.dies, t.tiles_per_group / (THREADS / kScatterBlock), t.capacity, t.cap_mask, t.positions,       \
                        t.scale_factor, t.random_shift, t.window, t.grad, t.grad_row_stride, t.double_pos_grad, t.second_grad,          \
-                       t.table_grad, t.grad_level_major, t.bins)
+                       t.table_grad, t.grad_level_major, t.bins, ClearTargetOf<BINS>(t.clear))
 #define PENC_LAUNCH_WIDTH(KERNEL, ...)                                          \
     if (t.wide_bins) {                                                          \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, kBinsWide);   \
+        PENC_LAUNCH(kScatterBlockManyBins, kBinsWide, KERNEL<D, __VA_ARGS__);   \
     } else if (t.most_bins) {                                                   \
-        PENC_LAUNCH(kScatterBlockManyBins, KERNEL<D, __VA_ARGS__, kBinsMany);   \
+        PENC_LAUNCH(kScatterBlockManyBins, kBinsMany, KERNEL<D, __VA_ARGS__);   \
     } else if (t.many_bins) {                                                   \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsMany);           \
+        PENC_LAUNCH(kScatterBlock, kBinsMany, KERNEL<D, __VA_ARGS__);           \
     } else if (t.bins.records != nullptr && t.bins.bin_shift < static_cast<uint32_t>(kBinSlotsLog2)) { \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsNarrow);         \
+        PENC_LAUNCH(kScatterBlock, kBinsNarrow, KERNEL<D, __VA_ARGS__);         \
     } else {                                                                    \
-        PENC_LAUNCH(kScatterBlock, KERNEL<D, __VA_ARGS__, kBinsFew);            \
+        PENC_LAUNCH(kScatterBlock, kBinsFew, KERNEL<D, __VA_ARGS__);            \
     }
     if (t.second_grad != nullptr) {
         if (t.rows) {

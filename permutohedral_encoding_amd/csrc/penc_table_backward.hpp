@@ -23,6 +23,7 @@ struct TableLaunch {
     const float *double_pos_grad, *second_grad;
     float *table_grad, *grad_level_major;
     BinTarget bins;
+    ClearTarget clear;
 };
 
 template <int D>
