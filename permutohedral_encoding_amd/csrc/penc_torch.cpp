@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -210,6 +211,16 @@ Upstream upstream_of(const Call& c, const Tensor& grad) {
     return {level_major, 0};
 }
 
+// Memory of `size` bytes that a call does better with and can do without: whether `take`, which allocates it, has found it.  A request in vain makes
+// the allocator release all it has cached, for the driver to be asked again by whatever follows; so once a device has refused, as much is not
+// asked for again until the process could have a sixteenth of it more than then.  Slopes are not given back for it.
+bool take_optional(const at::Device& device, int64_t size, const std::function<void()>& take);
+Tensor optional_bytes(const Call& c, int64_t n) {
+    Tensor t;
+    take_optional(c.device(), n, [&] { t = bytes(c, static_cast<size_t>(n)); });
+    return t;
+}
+
 // Scratch memory of one gradient call, undefined when the library would not use any.  The scatter counts every
 // pair of features as a level.  `copy_bytes`: the level-major copy of a row-major upstream gradient, which the call
 // cannot do without.  A request over the cap, or one the allocator cannot serve, is made again for fewer levels per
@@ -231,9 +242,14 @@ Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t cop
         want = std::max(want, pos_bytes) + copy_bytes + extra;
         if (c.max_workspace < 0 || want <= c.max_workspace) {
             if (want == 0) return {};
-            try {
-                return bytes(c, static_cast<size_t>(want));
-            } catch (const c10::OutOfMemoryError&) {
+            if (extra > 0) {
+                const Tensor ws = optional_bytes(c, want);
+                if (ws.defined()) return ws;
+            } else {
+                try {
+                    return bytes(c, static_cast<size_t>(want));
+                } catch (const c10::OutOfMemoryError&) {
+                }
             }
         }
         if (extra > 0) {
@@ -410,7 +426,9 @@ std::unordered_set<Slopes*>& Slopes::alive = *new std::unordered_set<Slopes*>();
 // any smaller request finds what it would find without them.  (Once a program's blocks are all cached the allocator does not come here.)
 class GiveBackSlopes : public c10::FreeMemoryCallback {
 public:
+    static thread_local bool not_for_this;  // the thread asks for memory that it can do without
     bool Execute() override {
+        if (not_for_this) return false;
         try {
             const int device = c10::hip::current_device();
             if (device < 0 || device >= Slopes::kMaxDevices || Slopes::held[device] == 0) return false;
@@ -421,6 +439,49 @@ public:
         }
     }
 };
+thread_local bool GiveBackSlopes::not_for_this = false;
+
+bool take_optional(const at::Device& device, int64_t size, const std::function<void()>& take) {
+    struct Refusal {
+        std::mutex mutex;
+        int64_t size = 0, available = 0;  // the last request in vain (0: none since one as large was served), and what there was to be had after it
+    };
+    static Refusal refusals[Slopes::kMaxDevices];
+    const int index = device.index();
+    if (index < 0 || index >= Slopes::kMaxDevices) return false;
+    Refusal& last = refusals[index];
+    // what the allocator has cached and what the driver still has for this process
+    const auto available = [&] {
+        const auto stats = c10::hip::HIPCachingAllocator::getDeviceStats(static_cast<c10::DeviceIndex>(index));
+        constexpr auto kAll = static_cast<size_t>(c10::CachingAllocator::StatType::AGGREGATE);
+        return Slopes::memory_left(index) + stats.reserved_bytes[kAll].current - stats.allocated_bytes[kAll].current;
+    };
+    int64_t wanted = 0;
+    {
+        std::lock_guard<std::mutex> lock(last.mutex);
+        if (last.size != 0 && size >= last.size) wanted = last.available + size / 16;
+    }
+    if (wanted != 0 && available() < wanted) return false;
+    struct Asking {
+        Asking() { GiveBackSlopes::not_for_this = true; }
+        ~Asking() { GiveBackSlopes::not_for_this = false; }
+    };
+    try {
+        const Asking asking;
+        take();
+    } catch (const c10::OutOfMemoryError&) {
+        const int64_t left = available();
+        std::lock_guard<std::mutex> lock(last.mutex);
+        last.size = size;
+        last.available = left;
+        return false;
+    }
+    if (wanted != 0) {
+        std::lock_guard<std::mutex> lock(last.mutex);
+        last.size = 0;
+    }
+    return true;
+}
 
 // ------------------------------------------------------------------------------------------
 // the three computations (reference: Encoding<D,F>::forward, ::backward, ::double_backward_from_positions, src/Encoding.cu:55-334)
@@ -433,13 +494,9 @@ bool may_go_by_cells(const Call& c) { return c.table_format == 0 && c.n * c.leve
 bool forward_in_cells(const Call& c, Tensor level_major, const Tensor& rows, const Tensor& slopes) {
     const size_t n = api.forward_cells_workspace_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity, rows.defined() ? static_cast<int>(c.columns()) : 0);
     if (n == 0 || (c.max_workspace >= 0 && static_cast<int64_t>(n) > c.max_workspace)) return false;
-    Tensor ws;
-    try {
-        if (!level_major.defined()) level_major = level_major_array(c);
-        ws = bytes(c, n);
-    } catch (const c10::OutOfMemoryError&) {
-        return false;
-    }
+    if (!level_major.defined()) level_major = level_major_array(c);  // (a forward in rows needs as much either way)
+    const Tensor ws = optional_bytes(c, static_cast<int64_t>(n));
+    if (!ws.defined()) return false;
     check(api.forward_cells(c.pos_dim, c.feat, c.n, c.levels, c.capacity, data(c.positions), data(c.table), data(c.scale_factor), data(c.shift),
                             data(c.window), mutable_data(level_major), mutable_data(rows), c.columns(), mutable_data(slopes), c.concat, c.scaling,
                             ws.mutable_data_ptr(), n, current_stream(c.device())),
