@@ -513,8 +513,10 @@ class EncodingWrapper:
             return None
         try:
             # (never from the 16-bit copy, which another stream may still be filling)
-            copy = native.table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim)
+            copy = native.table_in_cells(lattice_values.detach(), TABLE_FORMATS[self.half_table], self.pos_dim, MAX_WORKSPACE_BYTES)
         except torch.cuda.OutOfMemoryError:
+            return None
+        if copy is None:  # (no memory)
             return None
         kept = self._half_copy
         if kept is not None and kept[0] != key:  # (one of this version stays: a captured graph may read it)

@@ -1100,33 +1100,47 @@ PyObject* py_wait_for_event(PyObject*, PyObject* handle) {
     });
 }
 
-// table_in_cells(table, table_format, pos_dim) -> the table (fp32, or already of that format) as a 16-bit copy in cells
+// table_in_cells(table, table_format, pos_dim, max_workspace_bytes or None) -> the table (fp32, or already of that format) as a 16-bit copy in cells;
+// None where there is no memory for it, or none for a level of it under the cap
 PyObject* py_table_in_cells(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return guarded([&]() -> PyObject* {
-        TORCH_CHECK(n_args == 3, "table_in_cells takes 3 arguments");
+        TORCH_CHECK(n_args == 4, "table_in_cells takes 4 arguments");
         TORCH_CHECK(api.table_cells != nullptr, "bind() has not been called");
         const Tensor& table = tensor_arg(args[0], "lattice_values");
         const int format = static_cast<int>(PyLong_AsLong(args[1])), pos_dim = static_cast<int>(PyLong_AsLong(args[2]));
+        const int64_t cap = args[3] == Py_None ? -1 : PyLong_AsLongLong(args[3]);
         if (PyErr_Occurred()) return nullptr;
         const bool fp32 = table.scalar_type() == at::kFloat;
         const auto type = format == PENC_TABLE_FP16 ? at::kHalf : at::kBFloat16;
         PENC_REQUIRE(table.is_cuda() && table.is_contiguous() && table.dim() == 3 && (fp32 || table.scalar_type() == type), "bad table");
         const int levels = static_cast<int>(table.size(0)), capacity = static_cast<int>(table.size(1)), feat = static_cast<int>(table.size(2));
+        // (a few levels at a time go through the workspace, which holds at least one)
+        int64_t n = static_cast<int64_t>(api.table_cells_workspace_bytes(feat, levels, capacity, format));
+        const int64_t one_level = static_cast<int64_t>(api.table_cells_workspace_bytes(feat, 1, capacity, format));
+        if (cap >= 0 && n > cap) n = cap;
+        if (n < one_level) Py_RETURN_NONE;
+        // The library reads a slot at a time.  A table that begins elsewhere, such as a view into flattened parameters, is rounded first.
+        const bool in_slots = (reinterpret_cast<uintptr_t>(table.const_data_ptr()) & (std::min<size_t>(feat * table.element_size(), 16) - 1)) == 0;
+        const int64_t copy_bytes = 2 * table.numel();
         Tensor cells;
         {
             NoGil no_gil;
             at::NoGradGuard no_grad;
             const c10::DeviceGuard device(table.device());
-            // The library reads a slot at a time.  A table that begins elsewhere, such as a view into flattened parameters, is rounded first.
-            const bool in_slots = (reinterpret_cast<uintptr_t>(table.const_data_ptr()) & (std::min<size_t>(feat * table.element_size(), 16) - 1)) == 0;
-            const Tensor from = in_slots ? table : table.to(type, /*non_blocking=*/false, /*copy=*/true);
-            cells = at::empty(table.sizes(), table.options().dtype(type));
-            const size_t n = api.table_cells_workspace_bytes(feat, levels, capacity, format);
-            const Tensor ws = at::empty({static_cast<int64_t>(n)}, table.options().dtype(at::kByte));
-            check(api.table_cells(pos_dim, feat, levels, capacity, from.const_data_ptr(), fp32 && in_slots ? 0 : format, format,
-                                  cells.mutable_data_ptr(), ws.mutable_data_ptr(), n, current_stream(table.device())),
-                  "table_cells");
+            Tensor from = table, ws;
+            const bool taken = take_optional(table.device(), (in_slots ? 1 : 2) * copy_bytes + n, [&] {
+                cells = at::empty(table.sizes(), table.options().dtype(type));
+                ws = at::empty({n}, table.options().dtype(at::kByte));
+                if (!in_slots) from = table.to(type, /*non_blocking=*/false, /*copy=*/true);
+            });
+            if (taken)
+                check(api.table_cells(pos_dim, feat, levels, capacity, from.const_data_ptr(), fp32 && in_slots ? 0 : format, format,
+                                      cells.mutable_data_ptr(), ws.mutable_data_ptr(), static_cast<size_t>(n), current_stream(table.device())),
+                      "table_cells");
+            else
+                cells = Tensor();
         }
+        if (!cells.defined()) Py_RETURN_NONE;
         return THPVariable_Wrap(std::move(cells));
     });
 }

@@ -89,6 +89,47 @@ def test_a_forward_that_is_refused_its_copy_in_cells(room_for, rows):
     refused_once(call, check, pe._native.lib().penc_forward_cells_workspace_bytes(3, 2, n, levels, cap, 2 * levels if rows else 0), room_for)
 
 
+def half_table(levels, cap):
+    """-> (an encoding with a 16-bit table, its call on points enough for a copy in cells over a number of calls)"""
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=torch.bfloat16)
+    pos = torch.rand(pe._native.lib().penc_table_cells_points(2, cap, 2), 3, device="cuda")
+
+    def call(of=1):
+        with torch.no_grad():
+            return m(pos[:len(pos) // of])
+    return m, call
+
+
+def test_a_table_that_is_refused_its_copy_in_cells(room_for):
+    m, call = half_table(16, 1 << 20)
+    want = call(8)
+    room_for(60 << 20)  # a result of 8 MB, not a copy of 64 MB
+    before = torch.cuda.memory_stats()["num_alloc_retries"]
+    for _ in range(12):
+        got = call(8)
+        assert torch.equal(got, want) and m.lattice._cells is None
+    assert torch.cuda.memory_stats()["num_alloc_retries"] == before + 1
+    torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(call(8), want) and m.lattice._cells is not None
+
+
+def test_a_copy_in_cells_keeps_to_the_workspace_cap(monkeypatch):
+    """Some levels at a time through a smaller workspace, or, with no room for one, the copy in the table's order."""
+    from permutohedral_encoding_amd import _native
+    levels, cap = 16, 1 << 20
+    m, call = half_table(levels, cap)
+    slice_bytes = 4 * cap
+    want = call()
+    assert m.lattice._cells is not None
+    for most, made in ((3 * slice_bytes + 300, True), (slice_bytes + 256, True), (slice_bytes + 255, False), (0, False)):
+        m.invalidate_half_table()
+        monkeypatch.setattr(_native, "MAX_WORKSPACE_BYTES", most)
+        got, taken = peak_of(call)
+        assert torch.equal(got, want) and (m.lattice._cells is not None) == made
+        assert taken <= got.numel() * 4 + levels * slice_bytes + most
+
+
 def test_slopes_are_not_given_back_for_memory_that_a_call_can_do_without(room_for):
     """A forward finds room for its result, but for its copy in cells only in the place of another graph's slopes."""
     import permutohedral_encoding_amd as pe
