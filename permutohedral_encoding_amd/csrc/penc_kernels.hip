@@ -2285,15 +2285,23 @@ size_t penc_table_cells_workspace_bytes(int nr_feat, int nr_levels, int capacity
 // points, table -> copy: D = 2, 2^16 slots 28.7 -> 19.5 us; D = 3, 2^16 39.4 -> 27.1, 2^20 54.8 -> 40.8, with four features 80.0 -> 51.3; D = 5,
 // 2^20 84.0 -> 73.2; D = 8, 2^16 87.4 -> 79.8, with eight features 2^20 285 -> 247; 24 levels of 2^22 slots in bfloat16, 500003 points near a
 // surface 315 -> 160), from a smaller one, which the first-level cache holds, slower (2^12 slots: D = 3 19.5 -> 19.8, D = 8 41.6 -> 43.8).  Making
-// it takes longer than rounding the table does (24 levels, 2^18 slots 22.5 and 11.7 us, 2^20 87 and 48, 2^22 337 and 206); the line is where
-// the points make up for that, which larger levels, whose lines come from beyond the L2, do sooner.
+// it takes longer than rounding the table does (24 levels, 2^18 slots 22.5 and 11.7 us, 2^20 87 and 48, 2^22 337 and 206).  The line is where a
+// first pass on a new table, its copy made, takes as long either way; from 1.5 to 14 MiB a level that is about the same number of points.  24 levels in
+// bfloat16, D = 3, the copy in the table's order -> in cells, us:
+//   2^16 slots   32768 points 30.7 -> 34.8   65536 40.0 -> 40.3   131072 56.7 -> 52.9
+//   2^18         131072 73.8 -> 78.7, along rays 62.7 -> 69.1   262144 108 -> 105, 85.0 -> 86.4   524288 179 -> 156, 131 -> 123
+//   2^20         262144 190 -> 205, near a surface 184 -> 202   524288 282 -> 272, 272 -> 262
+//   2^21         299593 329 -> 331, 305 -> 325   419430 395 -> 370, 363 -> 358   599186 498 -> 422, 455 -> 410
+//   2^22         419430 552 -> 577, 520 -> 563   599186 678 -> 639, 626 -> 619   838860 834 -> 724, 767 -> 708
+//   (16 levels: D = 4, 2^22 slots 299593 388 -> 404   419430 466 -> 447;  D = 2, four features, 2^20 419430 219 -> 222   599186 259 -> 248)
 int64_t penc_table_cells_points(int nr_feat, int capacity, int table_format) {
     if ((nr_feat != 2 && nr_feat != 4 && nr_feat != 8) || capacity <= 0 || !known_half_format(table_format) ||
         strip_cells(table_format) != table_format || !cells_possible(nr_feat, capacity, table_format))
         return -1;
     const size_t slice = slice_bytes(capacity, nr_feat, table_format);
     if (slice < (size_t{64} << 10)) return -1;
-    return static_cast<int64_t>(slice / (slice <= (size_t{4} << 20) ? 8 : 40));
+    const size_t points = slice / 3 < (size_t{1} << 19) ? slice / 3 : size_t{1} << 19;
+    return static_cast<int64_t>(points > slice / 28 ? points : slice / 28);
 }
 
 int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, const void* lattice_values, int source_format, int table_format,
@@ -2343,13 +2351,20 @@ int penc_table_cells(int pos_dim, int nr_feat, int nr_levels, int capacity, cons
     return PENC_OK;
 }
 
-// Where one forward is worth a copy of the fp32 table in cells: from 16 M points times levels on (the copy's launch takes 5 us, all that is to be
-// lost), on levels of 64 KiB to 2 MiB with at most a slot for every two or three points.  Forward without -> with, us, two features, finest scale
-// 1e-4 / 1e-3 / 1e-2:
-//   D = 3, 24 levels, 2^20 points   2^18 slots, unordered 280 -> 237, 261 -> 206, 171 -> 170   along rays 179 -> 175, 132 -> 137, 111 -> 116
-//                                   2^19 slots 360 -> 375, 286 -> 299, 173 -> 203 (an L2 holds no such level beside what it gathers)
-//          2^19 points              2^14 slots 122 -> 103   2^16 138 -> 119   2^17 141 -> 125   along rays, 1e-2, 2^14 55 -> 63
-//   16 levels, 1e-3, 2^18 slots     D = 2 115 -> 101   D = 4 230 -> 204   D = 5 291 -> 277   D = 6 337 -> 325   D = 7 387 -> 376   (D = 8, 2^19 271 -> 309)
+// Where one forward is worth a copy of the fp32 table in cells: from 16 M points times levels on, on levels of 64 KiB to 2 MiB with at most a slot for
+// every two or three points.  What is gained depends on the points, which only the device sees: a call whose levels are not worth a copy has
+// looked in vain (5 us, 9 with 2^18 slots), and one along rays to a coarse finest level loses 4 to 10%, at the line up to 15%, where unordered points, and
+// points near a surface, gain up to 28%.  Below the line the loss is a larger share (up to a third) and the gain a smaller one.  Forward without -> with, us, D = 3, 24
+// levels, two features, at 6.3 / 12.6 / 16.8 / 25.2 M (2^18 to 2^20 points):
+//   2^14 slots, finest scale 1e-4   unordered 71 -> 63  123 -> 104  164 -> 134  241 -> 192   along rays 50 -> 50  78 -> 76  101 ->  97  147 -> 139
+//                            1e-2             43 -> 48   79 ->  81  106 -> 104  154 -> 149              27 -> 31  50 -> 55   66 ->  72   96 -> 102
+//   2^16                     1e-4             75 -> 69  139 -> 117  185 -> 149  273 -> 212              48 -> 52  88 -> 85  116 -> 107  170 -> 150
+//                            1e-2             50 -> 53   88 ->  84  117 -> 106  170 -> 151              27 -> 32  48 -> 56   68 ->  72   97 -> 102
+//   2^18                     1e-4             83 -> 91  145 -> 139  193 -> 173  283 -> 239              51 -> 65  94 -> 102 123 -> 128  179 -> 175
+//                            1e-3             76 -> 81  134 -> 120  176 -> 149  261 -> 203              38 -> 54  69 -> 81   90 -> 100  133 -> 137
+//                            1e-2             53 -> 70   90 -> 100  118 -> 123  172 -> 167              27 -> 36  51 -> 59   69 ->  75   98 -> 106
+//   2^19         2^20 points, unordered 360 -> 375, 1e-3 286 -> 299, 1e-2 173 -> 203 (an L2 holds no such level beside what it gathers)
+//   16 levels, 1e-3, 2^18 slots, 2^20 points     D = 2 115 -> 101   D = 4 230 -> 204   D = 5 291 -> 277   D = 6 337 -> 325   D = 7 387 -> 376   (D = 8, 2^19 271 -> 309)
 // Four features, D = 3, 16 levels: 2^14 slots 163 -> 144, 2^16 176 -> 152, 2^17 179 -> 172, 2^18 217 -> 235; eight: 2^16 243 -> 267.
 constexpr int64_t kForwardCellsMinWork = 16000000;
 constexpr size_t kForwardCellsMaxSlice = size_t{2} << 20;

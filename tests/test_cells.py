@@ -117,6 +117,15 @@ def test_where_a_forward_goes_by_way_of_cells():
     assert serves(3, 2, 1 << 20, 24, 1 << 14, 0) and not serves(3, 2, 1 << 20, 24, 1 << 14, 48)  # rows without a transpose
 
 
+def test_from_how_many_points_a_16_bit_table_is_laid_out_in_cells():
+    """Where a first pass on a new table takes as long either way: a third of a slice in points, half a million from 1.5 MiB on, a 28th of a slice."""
+    from permutohedral_encoding_amd import _native
+    points = _native.lib().penc_table_cells_points
+    assert points(2, 1 << 14, 2) == (1 << 16) // 3 and points(2, 1 << 13, 2) == -1 and points(2, 1 << 18, 1) == (1 << 20) // 3
+    assert points(2, 1 << 19, 2) == points(2, 1 << 20, 2) == points(4, 1 << 20, 2) == 1 << 19
+    assert points(2, 1 << 22, 2) == (1 << 24) // 28 > 500003 and points(8, 1 << 22, 1) == (1 << 26) // 28
+
+
 def test_cells_cover_the_lattice_once():
     """The rule of the head comment in Python's integers: for every dimension and line the offsets found by another search give a permutation."""
     mul = 2531011
