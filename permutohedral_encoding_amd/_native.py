@@ -442,10 +442,7 @@ class EncodingWrapper:
     @staticmethod
     def _made_now(key, copy):
         device = copy.get_device()
-        with torch.cuda.device(device):
-            event = torch.cuda.Event()
-            event.record()
-            return (key, copy, device, _raw_stream(device), event)
+        return (key, copy, device, _raw_stream(device), (_bridge or bridge()).record_event(device))
 
     @staticmethod
     def _for_this_stream(kept):
@@ -453,12 +450,10 @@ class EncodingWrapper:
         keeps its memory from reuse."""
         _, copy, device, stream, event, *_ = kept
         if stream != _raw_stream(device):
-            if (_bridge or bridge()).capture_id(device):
-                _bridge.wait_for_event(event.cuda_event)  # (a graph cannot wait for what is outside it: the host does, before the graph can run)
-            else:
-                here = torch.cuda.current_stream(device)
-                here.wait_event(event)
-                copy.record_stream(here)
+            native = _bridge or bridge()
+            native.wait_for_event(event, device)
+            if not native.capture_id(device):
+                copy.record_stream(torch.cuda.current_stream(device))
         return copy
 
     def _points_for_cells(self, lattice_values):

@@ -1070,28 +1070,56 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     });
 }
 
-// capture_id(device) -> the id of the capture that the device's current stream takes part in, 0 where it takes part in none
+// The capture that a stream takes part in, 0 where it takes part in none.
+uint64_t capture_of(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {  // (the default stream while another is captured)
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusNone ? 0 : id + 1;
+}
+
+// capture_id(device) -> that of the device's current stream
 PyObject* py_capture_id(PyObject*, PyObject* device) {
     return guarded([&]() -> PyObject* {
         const long index = PyLong_AsLong(device);
         if (PyErr_Occurred()) return nullptr;
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        unsigned long long id = 0;
-        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(static_cast<c10::DeviceIndex>(index)).stream();
-        if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {  // (the default stream while another is captured)
-            (void)hipGetLastError();
-            status = hipStreamCaptureStatusNone;
-        }
-        return PyLong_FromUnsignedLongLong(status == hipStreamCaptureStatusNone ? 0 : id + 1);
+        return PyLong_FromUnsignedLongLong(capture_of(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(static_cast<c10::DeviceIndex>(index)).stream()));
     });
 }
 
-// wait_for_event(handle): on the host, also while this thread captures a graph
-PyObject* py_wait_for_event(PyObject*, PyObject* handle) {
+// record_event(device) -> a capsule: what the device's current stream has been given so far.  For the device's own streams alone: a fence for the host, which
+// an event of torch's has, would stand between the launches before it and after it.
+constexpr const char* kEventCapsule = "penc.event";
+PyObject* py_record_event(PyObject*, PyObject* device) {
     return guarded([&]() -> PyObject* {
-        const auto event = static_cast<hipEvent_t>(PyLong_AsVoidPtr(handle));
+        const auto index = static_cast<c10::DeviceIndex>(PyLong_AsLong(device));
         if (PyErr_Occurred()) return nullptr;
-        {
+        const c10::DeviceGuard guard(at::Device(at::kCUDA, index));
+        hipEvent_t event = nullptr;
+        C10_HIP_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming | hipEventDisableSystemFence));
+        const hipError_t recorded = hipEventRecord(event, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(index).stream());
+        if (recorded != hipSuccess) (void)hipEventDestroy(event);
+        C10_HIP_CHECK(recorded);
+        return PyCapsule_New(event, kEventCapsule, [](PyObject* capsule) {
+            (void)hipEventDestroy(static_cast<hipEvent_t>(PyCapsule_GetPointer(capsule, kEventCapsule)));
+        });
+    });
+}
+
+// wait_for_event(event, device): the device's current stream does, or, where it takes part in a capture, which cannot wait for what is outside it, the host
+PyObject* py_wait_for_event(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 2, "wait_for_event takes 2 arguments");
+        const auto event = static_cast<hipEvent_t>(PyCapsule_GetPointer(args[0], kEventCapsule));
+        const auto index = static_cast<c10::DeviceIndex>(PyLong_AsLong(args[1]));
+        if (PyErr_Occurred()) return nullptr;
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(index).stream();
+        if (capture_of(stream) == 0) {
+            C10_HIP_CHECK(hipStreamWaitEvent(stream, event, 0));
+        } else {
             NoGil no_gil;
             c10::hip::HIPStreamCaptureModeGuard in_a_capture_too{hipStreamCaptureModeRelaxed};
             C10_HIP_CHECK(hipEventSynchronize(event));
@@ -1274,7 +1302,8 @@ PyMethodDef methods[] = {
     {"needs_autograd_functions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_needs_autograd_functions)), METH_FASTCALL,
      "whether a call is for the autograd functions of funcs.py"},
     {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},
-    {"wait_for_event", py_wait_for_event, METH_O, "waits on the host for an event"},
+    {"record_event", py_record_event, METH_O, "an event of a device's current stream"},
+    {"wait_for_event", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_wait_for_event)), METH_FASTCALL, "waits for such an event"},
     {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},
     {"cosine_window", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_cosine_window)), METH_FASTCALL, "a coarse-to-fine window"},
     {"adamw_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_adamw_step)), METH_FASTCALL, "one AdamW step"},
