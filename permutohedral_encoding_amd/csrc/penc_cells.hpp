@@ -9,8 +9,8 @@
 //     line(h) = (h - T[h mod B]) / B,   place in the line = h mod B
 // gives all points of a cell one line.  It is a permutation of the slots whatever the points, so a gather from the
 // permuted copy reads the values it would read from the table.  Lines per simplex, with 16 slots (32) to a line, mean over all
-// simplices: D = 2 1.5 of 3 (1.36), D = 3 2.23 of 4 (2.03), D = 4 3.1 of 5 (2.8), D = 5 4.4 of 6 (3.9), D = 6 5.2 of 7 (4.9), D = 8 7.4 of 9
-// (6.9); and at levels whose points share vertices, a line holds many that are used.  Forward of 500003 points near a surface, 24 levels of 2^22
+// simplices: D = 2 1.5 of 3 (1.36), D = 3 2.23 of 4 (2.03), D = 4 3.1 of 5 (2.8), D = 5 4.35 of 6 (3.9), D = 6 5.2 of 7 (4.85), D = 7 6.3 of 8
+// (5.75), D = 8 7.4 of 9 (7.0); and at levels whose points share vertices, a line holds many that are used.  Forward of 500003 points near a surface, 24 levels of 2^22
 // slots in bfloat16, of which the L2s miss every other line: 313 -> 160 us; of 2^20 unordered points, 2^18 slots 276 -> 194, 2^14 194 -> 149.
 #pragma once
 
