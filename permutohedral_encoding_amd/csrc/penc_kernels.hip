@@ -905,6 +905,9 @@ constexpr uint32_t bins_for_capacity(int capacity) { return bins_of_shift(capaci
 //   D = 5, 16 levels   2^16 slots, 2^18 points 177 -> 160;  D = 6 of 2^14 217 -> 204;  D = 8 of 2^16 255 -> 250, 8 levels of 2^18, 2^17 points 97 -> 91
 // With four dimensions the accumulate cache leaves some slots of the coarse levels out, whose records several reducers of a bin share
 // better than one (16 levels, 2^18 points: 2^16 slots 130 -> 137, 2^17 126 -> 132; 2^15 131 -> 122).
+// A table that is one bin has room there for everything a group leaves; of narrower ones one can run over, where points that hardly share slots
+// crowd a range of them, and what finds no room is added to the gradient in fp32 one by one, as it is for any table of several bins, instead of in
+// the reducer's sums in fp64.
 constexpr uint32_t kReduceWorkgroupsWanted = 512;  // two per compute unit
 constexpr uint32_t kFineBinsWanted = 768, kFineBinsMostPairs4d = 128;
 constexpr uint32_t fine_bin_shift(int pos_dim, int capacity, int pair_levels) {

@@ -224,7 +224,7 @@ Tensor optional_bytes(const Call& c, int64_t n) {
 // Scratch memory of one gradient call, undefined when the library would not use any.  The scatter counts every
 // pair of features as a level.  `copy_bytes`: the level-major copy of a row-major upstream gradient, which the call
 // cannot do without.  A request over the cap, or one the allocator cannot serve, is made again for fewer levels per
-// pass and in the end without the scatter's part (the library then adds directly): _native.scatter_workspace.
+// pass and in the end without the scatter's part (the library then adds directly), as in _native.scatter_workspace, which does not ask for `extra`.
 Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t copy_bytes) {
     if (c.levels_per_pass < 0 && copy_bytes == 0) return {};
     int64_t pos_bytes = positions ? static_cast<int64_t>(api.positions_workspace_bytes(c.pos_dim, c.n, c.levels)) : 0;
