@@ -354,6 +354,7 @@ class EncodingFixedParams:
         self.m_points_scaling = float(points_scaling)
         sf = scale_factors(self.m_pos_dim, self.m_sigmas_list)
         self.m_scale_factor = torch.from_numpy(sf).to(random_shift_per_level.device)
+        self.m_captured_copy = None  # address of the 16-bit copy of the table that a graph was last captured with
 
 
 _WRAPPER_CALLS = frozenset(("forward", "backward", "double_backward_from_positions"))
@@ -428,6 +429,8 @@ class EncodingWrapper:
             key = self._half_key(lattice_values)
         kept = self._half_copy
         if kept is not None and kept[0] == key:
+            if (_bridge or bridge()).capture_id(kept[2]):
+                self.fixed_params.m_captured_copy = kept[1].data_ptr()
             return self._for_this_stream(kept)
         if not lattice_values.is_cuda:
             return lattice_values.detach().to(self.half_table)  # (for the checks, which refuse it)
@@ -518,7 +521,7 @@ class EncodingWrapper:
         if copy is None:  # (no memory)
             return None
         kept = self._half_copy
-        if kept is not None and kept[0] != key:  # (one of this version stays: a captured graph may read it)
+        if kept is not None and (kept[0] != key or kept[1].data_ptr() != self.fixed_params.m_captured_copy):  # (a graph would read what takes its place)
             self._half_copy = None
         self._cells = self._made_now(key, copy)
         return copy

@@ -110,6 +110,17 @@ void* current_stream(const at::Device& device) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream();
 }
 
+// The capture that a stream takes part in, 0 where it takes part in none.
+uint64_t capture_of(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {  // (the default stream while another is captured)
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusNone ? 0 : id + 1;
+}
+
 const float* data(const Tensor& t) { return static_cast<const float*>(t.const_data_ptr()); }
 float* mutable_data(const Tensor& t) { return t.defined() ? static_cast<float*>(t.mutable_data_ptr()) : nullptr; }
 
@@ -1042,6 +1053,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         if (args[10] != Py_None && (c.want_table || c.want_positions)) c.sparse_owner = std::make_shared<PyRef>(args[10]);
         Tensor out;
         std::shared_ptr<Slopes> slopes;
+        bool captured = false;
         {
             NoGil no_gil;
             at::NoGradGuard no_grad;
@@ -1050,6 +1062,11 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
             const c10::DeviceGuard device(c.device());
             slopes = Slopes::make(c);
             out = compute_forward(c, slopes);
+            if (!kInCells && c.table_format != 0) captured = capture_of(static_cast<hipStream_t>(current_stream(c.device()))) != 0;
+        }
+        if (captured) {  // (a graph reads this copy from now on)
+            THPObjectPtr copy(PyLong_FromVoidPtr(const_cast<void*>(c.table.const_data_ptr())));
+            if (!copy || PyObject_SetAttrString(args[14], "m_captured_copy", copy.get()) != 0) return nullptr;
         }
         if (c.scale_factor.device() != scale_device) {  // the module was moved: kept where the points are, so that the next call need not copy
             THPObjectPtr moved(THPVariable_Wrap(c.scale_factor));
@@ -1068,17 +1085,6 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
         }
         return THPVariable_Wrap(std::move(out));
     });
-}
-
-// The capture that a stream takes part in, 0 where it takes part in none.
-uint64_t capture_of(hipStream_t stream) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    unsigned long long id = 0;
-    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {  // (the default stream while another is captured)
-        (void)hipGetLastError();
-        return 0;
-    }
-    return status == hipStreamCaptureStatusNone ? 0 : id + 1;
 }
 
 // capture_id(device) -> that of the device's current stream

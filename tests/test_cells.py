@@ -368,6 +368,34 @@ def test_a_16_bit_copy_made_on_one_stream_is_waited_for_on_another():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("captured", ["not", "on its stream", "on another"])
+def test_the_copy_in_the_tables_order_goes_once_there_are_cells(captured):
+    """One 16-bit copy of a table in the end, as ever, unless a graph has been captured with the first one."""
+    import permutohedral_encoding_amd as pe
+    levels, cap = 6, 1 << 20
+    m = pe.PermutoEncoding(3, cap, levels, 2, np.geomspace(1.0, 1e-3, levels), lattice_half_precision=torch.bfloat16)
+    few, many = torch.rand(1000, 3, device="cuda"), torch.rand(pe._native.lib().penc_table_cells_points(2, cap, 2), 3, device="cuda")
+    before, side, graph = torch.cuda.memory_allocated(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.no_grad():
+        with torch.cuda.stream(side if captured == "on its stream" else torch.cuda.current_stream()):
+            want = m(few)
+        torch.cuda.synchronize()
+        if captured != "not":
+            with torch.cuda.graph(graph, stream=side):
+                got = m(few)
+        m(many)
+        assert m.lattice._cells is not None and (m.lattice._half_copy is None) == (captured == "not")
+        if captured == "not":
+            assert torch.cuda.memory_allocated() - before <= 2 * m.lattice_values.numel() + 4 * want.numel() + 4096
+        else:
+            torch.empty(m.lattice_values.numel(), dtype=torch.bfloat16, device="cuda").fill_(7.0)
+            got.zero_()
+            graph.replay()
+            assert torch.equal(got, want)
+        assert torch.equal(m(few), want)
+
+
+@pytest.mark.gpu
 def test_no_cells_are_made_for_a_call_that_would_not_gather_from_them():
     """A window that requires a gradient is for the autograd functions, which gather from the copy in the table's order."""
     import permutohedral_encoding_amd as pe
