@@ -535,6 +535,10 @@ class EncodingWrapper:
         self._cells = None
         self._captured = None
 
+    def __getstate__(self):
+        """(copy.deepcopy, pickle) Without the copies of the table, whose events are this process's."""
+        return {name: value for name, value in self.__dict__.items() if name not in ("_half_copy", "_cells", "_captured")}
+
     def _check_common(self, inp):
         fp = self.fixed_params
         pos, lv, win = inp.m_positions_raw, inp.m_lattice_values, inp.m_anneal_window

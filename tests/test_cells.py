@@ -412,6 +412,23 @@ def test_no_cells_are_made_for_a_call_that_would_not_gather_from_them():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("points", [1000, 1 << 19])
+def test_a_wrapper_that_keeps_copies_can_be_copied(points):
+    """As it could when the 16-bit copy was a tensor alone: (1000 points: in the table's order, else in cells)"""
+    import copy
+    import permutohedral_encoding_amd as pe
+    m = pe.PermutoEncoding(3, 1 << 16, 12, 2, np.geomspace(1.0, 1e-3, 12), lattice_half_precision=torch.bfloat16)
+    pos = torch.rand(points, 3, device="cuda")
+    with torch.no_grad():
+        want = m(pos)
+        assert (m.lattice._cells is None) == (points == 1000)
+        other = copy.deepcopy(m.lattice)
+        assert other.half_table == torch.bfloat16 and other._half_copy is None and other._cells is None
+        assert torch.equal(other.encode(m.lattice_values, pos, m.anneal_window), want)
+        assert torch.equal(copy.deepcopy(m)(pos), want) and torch.equal(m(pos), want)
+
+
+@pytest.mark.gpu
 def test_positions_that_are_no_tensor_are_refused_as_ever():
     import permutohedral_encoding_amd as pe
     m = pe.PermutoEncoding(3, 1 << 16, 4, 2, np.geomspace(1.0, 1e-3, 4), lattice_half_precision=torch.bfloat16)
