@@ -398,7 +398,7 @@ class EncodingWrapper:
 
     # -- checks shared by the three calls (reference: src/Encoding.cu:38-45, 57-66, 119-125)
     half_table = None  # set by the module: torch.float16 or torch.bfloat16 to gather from such a copy of the fp32 table
-    # Copies kept with what they were made of and when: (key, copy, device, stream, event).  One attribute each, so that threads never see one's
+    # Copies kept with what they were made of and when: (key, copy, device, stream, [event]).  One attribute each, so that threads never see one's
     # copy with another's key.
     _half_copy = None  # in 16 bits; behind the event the points from which cells are worth having (< 0: never) and a list of the points gathered so far
     _cells = None      # in 16 bits and in cells (penc_table_cells), where enough points have been gathered for it
@@ -419,10 +419,10 @@ class EncodingWrapper:
     def _half_key(self, lattice_values):
         return (lattice_values.data_ptr(), lattice_values._version, lattice_values.device, lattice_values.shape, self.half_table)
 
-    def gather_table(self, lattice_values, key=None, points=0):
+    def gather_table(self, lattice_values, key=None, points=0, line=None):
         """The tensor the gathering kernels read for ``lattice_values``: the tensor itself, or, with
         ``half_table``, its 16-bit copy, made again whenever the tensor has been modified in place (``points``: what the call that
-        makes it gathers)."""
+        makes it gathers; ``line``: _points_for_cells, where it is known)."""
         if self.half_table is None or lattice_values.dtype != torch.float32:
             return lattice_values
         if key is None:
@@ -442,14 +442,15 @@ class EncodingWrapper:
             if captured is None or captured[0] != made_for:
                 captured = self._captured = (made_for, lattice_values.detach().to(self.half_table))
             return captured[1]
-        copy = lattice_values.detach().to(self.half_table)
-        self._half_copy = self._made_now(key, copy) + (self._points_for_cells(lattice_values), [points])
-        return copy
+        if line is None:
+            line = self._points_for_cells(lattice_values)
+        kept = self._half_copy = _bridge.rounded_copy(key, lattice_values, TABLE_FORMATS[self.half_table], line, points)
+        return kept[1]
 
     @staticmethod
     def _made_now(key, copy):
         device = copy.get_device()
-        return (key, copy, device, _raw_stream(device), (_bridge or bridge()).record_event(device))
+        return (key, copy, device, _raw_stream(device), (_bridge or bridge()).event_behind(device))
 
     @staticmethod
     def _for_this_stream(kept):
@@ -458,7 +459,9 @@ class EncodingWrapper:
         _, copy, device, stream, event, *_ = kept
         if stream != _raw_stream(device):
             native = _bridge or bridge()
-            native.wait_for_event(event, device)
+            if event[0] is None:  # (made on the default stream)
+                event[0] = native.record_event(device)
+            native.wait_for_event(event[0], device)
             if not native.capture_id(device):
                 copy.record_stream(torch.cuda.current_stream(device))
         return copy
@@ -503,7 +506,7 @@ class EncodingWrapper:
                 cells = self._make_cells(lattice_values, positions, anneal_window, key, so_far, points)
                 if cells is not None:
                     return cells, True
-        return (self.gather_table(lattice_values, key, so_far) if half is None else self._for_this_stream(half)), False
+        return (self.gather_table(lattice_values, key, so_far, points) if half is None else self._for_this_stream(half)), False
 
     def _make_cells(self, lattice_values, positions, anneal_window, key, so_far, points):
         if lattice_values.requires_grad and torch.is_grad_enabled() and so_far < 4 * points:

@@ -1096,22 +1096,63 @@ PyObject* py_capture_id(PyObject*, PyObject* device) {
     });
 }
 
-// record_event(device) -> a capsule: what the device's current stream has been given so far.  For the device's own streams alone: a fence for the host, which
+// record_event(device) -> a capsule: what the device's default stream has been given so far.  For the device's own streams alone: a fence for the host, which
 // an event of torch's has, would stand between the launches before it and after it.
 constexpr const char* kEventCapsule = "penc.event";
+PyObject* event_of_stream(hipStream_t stream) {
+    hipEvent_t event = nullptr;
+    C10_HIP_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming | hipEventDisableSystemFence));
+    const hipError_t recorded = hipEventRecord(event, stream);
+    if (recorded != hipSuccess) (void)hipEventDestroy(event);
+    C10_HIP_CHECK(recorded);
+    return PyCapsule_New(event, kEventCapsule, [](PyObject* capsule) {
+        (void)hipEventDestroy(static_cast<hipEvent_t>(PyCapsule_GetPointer(capsule, kEventCapsule)));
+    });
+}
 PyObject* py_record_event(PyObject*, PyObject* device) {
     return guarded([&]() -> PyObject* {
         const auto index = static_cast<c10::DeviceIndex>(PyLong_AsLong(device));
         if (PyErr_Occurred()) return nullptr;
         const c10::DeviceGuard guard(at::Device(at::kCUDA, index));
-        hipEvent_t event = nullptr;
-        C10_HIP_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming | hipEventDisableSystemFence));
-        const hipError_t recorded = hipEventRecord(event, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(index).stream());
-        if (recorded != hipSuccess) (void)hipEventDestroy(event);
-        C10_HIP_CHECK(recorded);
-        return PyCapsule_New(event, kEventCapsule, [](PyObject* capsule) {
-            (void)hipEventDestroy(static_cast<hipEvent_t>(PyCapsule_GetPointer(capsule, kEventCapsule)));
-        });
+        c10::hip::HIPStreamCaptureModeGuard in_a_capture_too{hipStreamCaptureModeRelaxed};
+        return event_of_stream(nullptr);
+    });
+}
+
+// A list of an event of the device's current stream.  Of None where that is the default stream, which is never destroyed nor captured: the event is recorded
+// by the first call on another stream, if there is one (a program that trains a 16-bit table makes a copy in every step, and its event 2 to 4 us).
+PyObject* event_behind(const at::Device& device) {
+    const auto stream = static_cast<hipStream_t>(current_stream(device));
+    if (stream == nullptr) return Py_BuildValue("[O]", Py_None);
+    const c10::DeviceGuard guard(device);
+    THPObjectPtr event(event_of_stream(stream));
+    return event ? Py_BuildValue("[N]", event.release()) : nullptr;
+}
+PyObject* py_event_behind(PyObject*, PyObject* device) {
+    return guarded([&]() -> PyObject* {
+        const auto index = static_cast<c10::DeviceIndex>(PyLong_AsLong(device));
+        return PyErr_Occurred() ? nullptr : event_behind(at::Device(at::kCUDA, index));
+    });
+}
+
+// rounded_copy(key, table, table_format, points, so_far) -> (key, the table in 16 bits, device, stream, [event], points, [so_far]): what the wrapper keeps of a
+// copy it has just made.  (In the interpreter, call by call, 1 us more.)
+PyObject* py_rounded_copy(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+    return guarded([&]() -> PyObject* {
+        TORCH_CHECK(n_args == 5, "rounded_copy takes 5 arguments");
+        const Tensor& table = tensor_arg(args[1], "lattice_values");
+        const long format = PyLong_AsLong(args[2]);
+        if (PyErr_Occurred()) return nullptr;
+        Tensor copy;
+        {
+            NoGil no_gil;
+            at::NoGradGuard no_grad;
+            copy = table.to(format == PENC_TABLE_FP16 ? at::kHalf : at::kBFloat16);
+        }
+        THPObjectPtr event(event_behind(copy.device()));
+        if (!event) return nullptr;
+        return Py_BuildValue("(ONiNNO[O])", args[0], THPVariable_Wrap(copy), static_cast<int>(copy.get_device()),
+                             PyLong_FromVoidPtr(current_stream(copy.device())), event.release(), args[3], args[4]);
     });
 }
 
@@ -1308,7 +1349,9 @@ PyMethodDef methods[] = {
     {"needs_autograd_functions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_needs_autograd_functions)), METH_FASTCALL,
      "whether a call is for the autograd functions of funcs.py"},
     {"capture_id", py_capture_id, METH_O, "the capture a device's current stream takes part in"},
-    {"record_event", py_record_event, METH_O, "an event of a device's current stream"},
+    {"rounded_copy", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_rounded_copy)), METH_FASTCALL, "a 16-bit copy of a table, as it is kept"},
+    {"event_behind", py_event_behind, METH_O, "an event of a device's current stream, where it has to be recorded now"},
+    {"record_event", py_record_event, METH_O, "an event of a device's default stream"},
     {"wait_for_event", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_wait_for_event)), METH_FASTCALL, "waits for such an event"},
     {"table_in_cells", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_table_in_cells)), METH_FASTCALL, "a 16-bit copy of a table in cells"},
     {"cosine_window", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_cosine_window)), METH_FASTCALL, "a coarse-to-fine window"},

@@ -304,11 +304,13 @@ def test_copy_made_on_one_stream_is_waited_for_on_another():
         for _ in range(20):
             work = (work @ work).clamp(-1, 1)
         m(many)
-        assert m.lattice._cells is not None
+        assert m.lattice._cells[4] == [None]  # (the default stream's: the event is recorded when one is needed, and kept)
         with torch.cuda.stream(side):
             got = m(few)
+            event, = m.lattice._cells[4]
+            again = m(few)
     torch.cuda.synchronize()
-    assert torch.equal(got, want)
+    assert event is not None and m.lattice._cells[4] == [event] and torch.equal(got, want) and torch.equal(again, want)
 
 
 def busy(work, times=20):
