@@ -1043,25 +1043,33 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, uint3
     return p;
 }
 
-// Fill, scatter, reduction and late adds, us, fill apart -> in the scatter (24 levels unless given):
-//   D = 3, 2^22 slots  2^20 points 1050 -> 986, near a surface with 16 levels live 609 -> 521, 200001 points 506 -> 425;  2^23 slots, 2^19 points 1039 -> 984
-//          2^21        200001 points 303 -> 253
-//          2^20        2^20 points 620 -> 606, from rows 663 -> 664, 200001 points 200 -> 190;  9 levels (75 MB) 2^18 points 91 -> 90
-//   D = 2, 16 levels of 2^20, 2^18 points 135 -> 127;  D = 4, 16 levels of 2^22, 2^19 points 625 -> 572, of 2^21 423 -> 391;  D = 8, of 2^22, 2^17 points 454 -> 395
-// A smaller gradient takes no longer to fill than the lists take to be added, and the instances for few bins stay without the code.
+// Fill, scatter, reduction and late adds, us, fill apart -> in the scatter (24 levels unless given; more beside ClearTarget):
+//   D = 3, 2^22 slots  2^20 points 1081 -> 1012, near a surface with 16 levels live 600 -> 530;  2^23 slots, 2^19 points 1039 -> 984
+//          2^20        2^20 points from rows 652 -> 650;  16 levels 424 -> 425
+//   D = 2, 16 levels of 2^20, 2^18 points 133 -> 121;  D = 4, 16 levels of 2^20, 2^18 points 186 -> 173;  D = 8, of 2^22, 2^17 points 465 -> 360
+// A smaller gradient takes no longer to fill than the lists take to be added, and the instances for few bins stay without the code.  With workgroups of 512
+// threads, not for less than one round of them, which the clearing ones put off (D = 8, 2^20 slots: 480 workgroups 80 -> 85, 89 -> 93, 111 -> 121;  588
+// of them 95 -> 89, 600 120 -> 107).
 constexpr size_t kClearInScatterBytes = size_t{64} << 20;
-inline bool clears_in_scatter(uint32_t n_bins, int pair_levels, int capacity) {
-    return n_bins > static_cast<uint32_t>(kStageBins) && static_cast<size_t>(pair_levels) * capacity * sizeof(float2) >= kClearInScatterBytes;
+constexpr int64_t kClearMinWorkgroups = 512;  // two to a compute unit
+inline bool clears_in_scatter(uint32_t n_bins, int pair_levels, int capacity, int64_t workgroups) {
+    return n_bins > static_cast<uint32_t>(kStageBins) && static_cast<size_t>(pair_levels) * capacity * sizeof(float2) >= kClearInScatterBytes &&
+           (n_bins > kFewerOpenLinesMinBins || workgroups >= kClearMinWorkgroups);
 }
+// Threads to a die that clear and do nothing else, and up to how many points times levels.  Beyond, a share each -> rows apart, 2^20 points, us: 2^22 slots 1014 ->
+// 987, along rays 900 -> 890, 1e-3 774 -> 763, 1e-2 597 -> 623, near a surface with 16 levels live 530 -> 543;  2^21 830 -> 804, along rays, 1e-2, 463 ->
+// 478;  2^20 650 -> 639, 388 -> 400, 16 levels 426 -> 430.
+constexpr uint32_t kClearingThreads = 4096;
+constexpr int64_t kClearApartMaxWork = 16000000;
 // What the lists of deferred adds (ClearTarget) take behind the bins, for all levels at once.
 inline size_t deferred_bytes(int pos_dim, int pair_levels, uint32_t n_groups, int tiles_per_group) {
     return static_cast<size_t>(pair_levels) * n_groups * (deferred_room(pos_dim, tiles_per_group) * sizeof(BinRecord) + sizeof(uint32_t)) + 512;
 }
 // Gives the plan of a dense gradient such lists where its scatter has the instance that clears, takes all levels in one launch, and the workspace has room
 // for them.
-inline bool plan_deferred(BinPlan& p, int pos_dim, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
+inline bool plan_deferred(BinPlan& p, int pos_dim, int64_t nr_positions, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
                           size_t bytes) {
-    if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity) || p.levels_per_pass < pair_levels) return false;
+    if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity, static_cast<int64_t>(p.target.n_groups) * pair_levels) || p.levels_per_pass < pair_levels) return false;
     if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0 || (static_cast<int64_t>(pair_levels) * capacity) % 2 != 0) return false;
     const uintptr_t base = (p.end + 255u) & ~uintptr_t{255};
     if (base + deferred_bytes(pos_dim, pair_levels, p.target.n_groups, tiles_per_group) > reinterpret_cast<uintptr_t>(workspace) + bytes) return false;
@@ -1070,6 +1078,8 @@ inline bool plan_deferred(BinPlan& p, int pos_dim, int pair_levels, int capacity
     p.clear.counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.clear.room * sizeof(BinRecord));
     p.clear.quads = static_cast<uint64_t>(pair_levels) * capacity / 2;
     p.clear.flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
+    const uint32_t threads = p.target.n_bins > kFewerOpenLinesMinBins ? kScatterBlockManyBins : kScatterBlock;
+    p.clear.rows = nr_positions * pair_levels < kClearApartMaxWork ? kClearingThreads / threads : 0u;
     return true;
 }
 
@@ -1404,7 +1414,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         plan.target.direct = touched;
         plan.target.n_bins = bins_for_capacity(capacity);
         plan.target.bin_shift = bin_shift_for_capacity(capacity);
-    } else if (plan_deferred(plan, pos_dim, pair_levels, capacity, tiles_per_group, lattice_values_grad, workspace, workspace_bytes)) {
+    } else if (plan_deferred(plan, pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, lattice_values_grad, workspace, workspace_bytes)) {
         // the scattering kernel clears
     } else if (int rc = clear_table_grad(lattice_values_grad, pair_levels, capacity, plan.enabled ? plan.target.direct : nullptr,
                                          plan.direct_bytes, st)) {
@@ -1416,7 +1426,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         const int count = pair_levels - first < per_pass ? pair_levels - first : per_pass;
         const unsigned padded_groups = (scatter_groups(nr_positions, tiles_per_group) + dies - 1) / dies * dies;
         if (direct_flags != nullptr) plan.target.direct = direct_flags + static_cast<size_t>(first) * plan.target.n_bins;
-        t.grid = dim3(padded_groups * static_cast<unsigned>(count));
+        t.grid = dim3(padded_groups * static_cast<unsigned>(count) + plan.clear.rows * dies);
         t.many_bins = plan.target.records != nullptr && plan.target.n_bins > static_cast<uint32_t>(kStageBins);
         t.most_bins = direct_flags != nullptr && plan.target.n_bins > kFewerOpenLinesMinBins;
         t.wide_bins = direct_flags != nullptr && plan.target.bin_shift > static_cast<uint32_t>(kBinSlotsLog2);
@@ -1674,7 +1684,10 @@ size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels
         const size_t want = most + direct_flag_bytes(nr_levels, fine) + 8192, have = penc_scatter_workspace_bytes(pos_dim, nr_positions, nr_levels, capacity, nr_levels);
         return want > have ? want - have : 0;
     }
-    if (n_bins > static_cast<uint32_t>(kMaxBins) || !clears_in_scatter(n_bins, nr_levels, capacity) || nr_positions * (pos_dim + 1) * kMinSlotsPerContribution <= capacity) return 0;
+    const int64_t workgroups = static_cast<int64_t>(scatter_groups(nr_positions, table_backward_tiles(nr_positions, nr_levels))) * nr_levels;
+    if (n_bins > static_cast<uint32_t>(kMaxBins) || !clears_in_scatter(n_bins, nr_levels, capacity, workgroups) ||
+        nr_positions * (pos_dim + 1) * kMinSlotsPerContribution <= capacity)
+        return 0;
     size_t most = 0;
     for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {
         const size_t need = deferred_bytes(pos_dim, nr_levels, scatter_groups(nr_positions, tiles), tiles);

@@ -120,8 +120,17 @@ struct BinTarget {
     uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records), less for small tables
 };
 // Large tables (more than kStageBins bins, all levels in one launch; kept == nullptr: not): the scattering kernel clears the gradient and the flags
-// itself, each workgroup a share of them when it starts, because those writes pass while it waits for other things (2^22 slots, 24 levels,
-// 16 of them live, 2^20 points: fill 134 and scatter 329 us apart, 373 together; 200001 points 163 and 90, 184).  Nothing may
+// itself, because those writes pass while it waits for other things.  The first `rows` rows of its grid, a workgroup to a die, do nothing else; rows == 0: every
+// workgroup clears a share when it starts.  So many rows that they write at about half of the memory's rate: with more the loads of
+// the others wait behind them, and where a share each is cleared by little more than one round of workgroups at once, fill and scatter might as
+// well be apart (table gradient with a fill / a share each / rows, D = 3, 24 levels unless given, us):
+//   2^21 slots  95077 points 227 / 201 / 167, 19 levels 158 / 161 / 133;  70000 points 196 / 192 / 155;  200001 points along rays, 1e-2, 208 / 185 / 145;  400000
+//               459 / 428 / 400
+//   2^20        70000 points 122 / 112 / 103, 16 levels 88 / 87 / 83;  200001 points 204 / 189 / 179;  D = 8, 50000 points 161 / 153 / 152
+//   2^22        200001 points 524 / 431 / 383, near a surface with 16 levels live 324 / 246 / 246;  500003 points 784 / 719 / 666, near a surface, 1e-2,
+//               498 / 414 / 423, 1e-3 631 / 566 / 523
+// (4, 6, 8 and 12 rows of 512 threads for 95077 points 190 / 175 / 167 / 174; 3, 4, 6, 8 of 1024 for 500003 686 / 666 / 683 / 678.)  With many points the two are
+// as good on average and apart by point order (kClearApartMaxWork).  Nothing may
 // be added to a gradient that another workgroup is still to clear, so what would go straight into it is kept until the reducers have ended, and
 // add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
 //   kept    [level_in_pass][group][room]   {slot in the level, values}; there is room for all a group can leave
@@ -132,6 +141,7 @@ struct ClearTarget {
     uint64_t quads;   // 16-byte units of the gradient,
     uint32_t flags;   // and its flags
     uint32_t room;
+    uint32_t rows;    // of workgroups that clear and do nothing else
 };
 // What instances for few bins are given instead.
 struct NoClearTarget {

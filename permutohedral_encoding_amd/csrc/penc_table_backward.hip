@@ -74,18 +74,23 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     // compute-bound coarse levels and store-bound fine levels share the chip at all times (this
     // kernel never reads the table: there is no slice to keep cache-resident by running a level at
     // a time).
-    const uint32_t die = blockIdx.x % dies, j = blockIdx.x / dies;
-    const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
+    const uint32_t die = blockIdx.x % dies;
+    uint32_t j = blockIdx.x / dies;
     if constexpr (kManyBins) {
         if (clear.kept != nullptr) {
-            typedef float Quad __attribute__((ext_vector_type(4)));
-            const uint64_t share = (clear.quads + gridDim.x - 1) / gridDim.x, from = share * blockIdx.x;
-            const uint64_t to = from + share < clear.quads ? from + share : clear.quads;
-            for (uint64_t i = from + threadIdx.x; i < to; i += kThreads) __builtin_nontemporal_store(Quad(0.0f), reinterpret_cast<Quad*>(table_grad) + i);
-            const uint32_t flag = blockIdx.x * kThreads + threadIdx.x;
-            if (flag < clear.flags) pass_bins.direct[flag] = 0u;
+            const uint32_t workgroups = clear.rows != 0u ? clear.rows * dies : gridDim.x;
+            if (blockIdx.x < workgroups) {
+                typedef float Quad __attribute__((ext_vector_type(4)));
+                const uint64_t share = (clear.quads + workgroups - 1) / workgroups, from = share * blockIdx.x;
+                const uint64_t to = from + share < clear.quads ? from + share : clear.quads;
+                for (uint64_t i = from + threadIdx.x; i < to; i += kThreads) __builtin_nontemporal_store(Quad(0.0f), reinterpret_cast<Quad*>(table_grad) + i);
+                for (uint32_t flag = blockIdx.x * kThreads + threadIdx.x; flag < clear.flags; flag += workgroups * kThreads) pass_bins.direct[flag] = 0u;
+                if (clear.rows != 0u) return;
+            }
+            j -= clear.rows;
         }
     }
+    const uint32_t level_in_pass = j % n_pass_levels, group = (j / n_pass_levels) * dies + die;
     const int64_t group_base = static_cast<int64_t>(group) * tiles_per_group * kThreads;
     if (group_base >= n_points) return;
     const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;

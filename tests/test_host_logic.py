@@ -122,6 +122,14 @@ def test_argument_validation_without_a_gpu():
     assert lib.penc_scatter_workspace_bytes(3, 1 << 20, 24, 1 << 18, 0) == lib.penc_scatter_workspace_bytes(3, 1 << 20, 24, 1 << 18, 24)
 
 
+def test_clearing_in_the_scatter_is_offered_from_a_round_of_workgroups_on():
+    """Workgroups of 1024 points: 504 and 516 of them for twelve levels; more than 256 bins (workgroups twice as large) whatever the number."""
+    from permutohedral_encoding_amd import _native
+    extra = _native.lib().penc_scatter_extra_bytes
+    assert extra(8, 42 * 1024, 12, 1 << 20) == 0 and extra(8, 43 * 1024, 12, 1 << 20) > 12 * 9 * 43 * 1024 * 12
+    assert extra(8, 70 * 1024, 4, 1 << 22) > 12 * 9 * 70 * 1024 * 4
+
+
 @pytest.mark.parametrize("d", range(2, 9))
 def test_scale_factors_match_oracle_and_closed_form(d):
     sig = np.geomspace(1.0, 1e-4, 24).astype(np.float32)
