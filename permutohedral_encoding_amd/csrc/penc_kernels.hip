@@ -897,7 +897,8 @@ constexpr uint32_t bins_for_capacity(int capacity) { return bins_of_shift(capaci
 
 // The width of the bins of a dense gradient whose workspace has room for the slack of more segments (penc_scatter_extra_bytes): where there are fewer
 // (bin, level) pairs than reducers wanted, so that several would share a bin and add into the gradient with atomics (60 ns each), bins of half the width
-// and less, down to 2^10 slots, until there are kFineBinsWanted pairs, each reduced by one workgroup of a part of a compute unit's LDS.  Scatter and
+// and less, down to 2^10 slots, until there are kFineBinsWanted pairs, each reduced by one workgroup of a part of a compute unit's LDS (a few where
+// there are fewer pairs all the same, kFineBinsShared).  Scatter and
 // reduction, us:
 //   D = 3, 24 levels   2^16 slots, 2^20 points 517 -> 481   2^14 598 -> 488   2^12, 2^19 points 408 -> 270;  6 levels of 2^16, 2^20 points 145 -> 128
 //          16 levels   2^18 points, 2^16 slots 105 -> 98   2^14 131 -> 101   100003 slots 108 -> 98;  12 levels of 2^18, 2^19 points 134 -> 125
@@ -1153,15 +1154,25 @@ inline GroupSortPlan plan_group_sort(int pos_dim, int64_t n, int levels, int fea
 
 // Running consecutive passes on two streams (scatter pass p+1 while pass p is reduced) was tried and
 // measured 10-15% slower than one pass over all levels on one stream; hence a single stream.
-constexpr unsigned kReduceWorkgroupsWantedFine = 128;  // of narrow bins, which end sooner
+// Narrow bins, which end sooner, are shared up to one pair of bin and level to a compute unit, and up to kFineBinsSharedCrowded pairs where a slot of at most 2^11
+// has eight contributions and more.  Scatter and reduction, alone -> shared (as wide bins), 2^19 points, us:
+//   128 pairs  D = 3, 16 levels of 2^13 slots 235 -> 182 (246), along rays 246 -> 195 (237)   D = 8, 8 levels of 2^14 295 -> 245 (253), 364 -> 290 (292)
+//   192        D = 2, 24 of 2^13 198 -> 160 (208), 217 -> 172 (200);  D = 4, 6 of 2^15 96 -> 88 (109), 111 -> 93 (103);  D = 3, 24 of 2^13 282 -> 247 (402)
+//   384        D = 3, 12 of 2^15 125 -> 126 (159), 140 -> 130 (144);  6 of 2^17, four contributions to a slot 35.1 -> 36.8 (48)
+//              bins of 2^12: D = 5, 6 of 2^18 141 -> 147 (151), along rays 148 -> 146 (145)
+constexpr unsigned kFineBinsShared = 256, kFineBinsSharedCrowded = 448;
 constexpr unsigned kMaxReduceSplits = 16;
 
-inline int reduce_bins(const BinPlan& p, const float* window, int first_level, int n_levels_in_pass, int capacity,
+inline int reduce_bins(const BinPlan& p, int64_t lookups, const float* window, int first_level, int n_levels_in_pass, int capacity,
                        uint32_t feat_pairs, float* table_grad, hipStream_t st) {
     // enough workgroups for every compute unit, by letting several share a bin when bins*levels is small
     const unsigned pairs = p.target.n_bins * static_cast<unsigned>(n_levels_in_pass);
-    const bool fine = p.target.bin_shift < static_cast<uint32_t>(kBinSlotsLog2);
-    unsigned splits = pairs >= (fine ? kReduceWorkgroupsWantedFine : kReduceWorkgroupsWanted) ? 1u : (kReduceWorkgroupsWanted + pairs - 1) / pairs;
+    unsigned enough = kReduceWorkgroupsWanted;
+    if (p.target.bin_shift < static_cast<uint32_t>(kBinSlotsLog2)) {
+        const bool crowded = p.target.bin_shift <= 11u && lookups >= static_cast<int64_t>(p.target.n_bins) << (p.target.bin_shift + 3);
+        enough = (crowded ? kFineBinsSharedCrowded : kFineBinsShared) + 1;
+    }
+    unsigned splits = pairs >= enough ? 1u : (kReduceWorkgroupsWanted + pairs - 1) / pairs;
     if (splits > p.target.n_groups) splits = p.target.n_groups;
     if (splits > kMaxReduceSplits) splits = kMaxReduceSplits;
     // many bins with a few thousand records each: workgroups that keep their bin and walk several levels
@@ -1439,7 +1450,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         PENC_DISPATCH_D(pos_dim, launch_table_backward<DD>(t));
         if (int rc = check_launch()) return rc;
         if (plan.enabled)
-            if (int rc = reduce_bins(plan, anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
+            if (int rc = reduce_bins(plan, nr_positions * (pos_dim + 1), anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
     }
     if (plan.clear.kept != nullptr) {
         hipLaunchKernelGGL(add_deferred_kernel, dim3(plan.target.n_groups, static_cast<unsigned>(pair_levels)), dim3(kBlock), 0, st, plan.clear, anneal_window,

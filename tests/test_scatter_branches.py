@@ -108,12 +108,13 @@ def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, 
                                                  (8, 2, 8, 65537, 1 << 18), (4, 2, 5, 120001, 1 << 14), (3, 2, 3, 60001, 700),
                                                  (8, 2, 8, 131201, 1 << 22), (3, 2, 24, 17 * 8192 + 777, 1 << 20), (3, 2, 5, (1 << 19) + 3, (1 << 21) + 8192),
                                                  (3, 2, 19, 95077, 1 << 21), (6, 2, 17, 60013, 600002), (8, 2, 24, 25003, 1 << 20),
-                                                 (2, 2, 24, 700001, 1 << 20), (3, 2, 24, 700001, (1 << 21) + 8192)])
+                                                 (2, 2, 24, 700001, 1 << 20), (3, 2, 24, 700001, (1 << 21) + 8192),
+                                                 (3, 2, 8, 200003, 1 << 14), (2, 2, 12, 300007, 30001)])
 def test_scatter_with_more_workspace(d, feat, levels, n, cap):
     """Large tables: with lists of deferred adds in the workspace the scatter clears the gradient (in rows of workgroups that do nothing else, for
     16 M points times levels in shares of all), whatever it held, masked levels too, and what would go straight into it follows later: column sums of the
     coarse levels, and what segments have no room for (a third of the points sit in one simplex).  Small tables: bins of 2^10 to 2^12 slots, the
-    last one not full, tables of less than one bin.  Both orders, rows and level-major, against the call without the extra bytes."""
+    last one not full, tables of less than one bin, summed by one workgroup or by several.  Both orders, rows and level-major, against the call without the extra bytes."""
     from helpers import make_encoding
     from permutohedral_encoding_amd import _native
     rng = np.random.default_rng(d)
