@@ -1071,13 +1071,13 @@ inline size_t deferred_bytes(int pos_dim, int pair_levels, uint32_t n_groups, in
 inline bool plan_deferred(BinPlan& p, int pos_dim, int64_t nr_positions, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
                           size_t bytes) {
     if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity, static_cast<int64_t>(p.target.n_groups) * pair_levels) || p.levels_per_pass < pair_levels) return false;
-    if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0 || (static_cast<int64_t>(pair_levels) * capacity) % 2 != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0) return false;
     const uintptr_t base = (p.end + 255u) & ~uintptr_t{255};
     if (base + deferred_bytes(pos_dim, pair_levels, p.target.n_groups, tiles_per_group) > reinterpret_cast<uintptr_t>(workspace) + bytes) return false;
     p.clear.room = deferred_room(pos_dim, tiles_per_group);
     p.clear.kept = reinterpret_cast<BinRecord*>(base);
     p.clear.counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.clear.room * sizeof(BinRecord));
-    p.clear.quads = static_cast<uint64_t>(pair_levels) * capacity / 2;
+    p.clear.pairs = static_cast<uint64_t>(pair_levels) * capacity;
     p.clear.flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
     const uint32_t threads = p.target.n_bins > kFewerOpenLinesMinBins ? kScatterBlockManyBins : kScatterBlock;
     p.clear.rows = nr_positions * pair_levels < kClearApartMaxWork ? kClearingThreads / threads : 0u;

@@ -138,7 +138,7 @@ struct BinTarget {
 struct ClearTarget {
     BinRecord* kept;
     uint32_t* counts;
-    uint64_t quads;   // 16-byte units of the gradient,
+    uint64_t pairs;   // 8-byte units of the gradient,
     uint32_t flags;   // and its flags
     uint32_t room;
     uint32_t rows;    // of workgroups that clear and do nothing else

@@ -81,9 +81,10 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
             const uint32_t workgroups = clear.rows != 0u ? clear.rows * dies : gridDim.x;
             if (blockIdx.x < workgroups) {
                 typedef float Quad __attribute__((ext_vector_type(4)));
-                const uint64_t share = (clear.quads + workgroups - 1) / workgroups, from = share * blockIdx.x;
-                const uint64_t to = from + share < clear.quads ? from + share : clear.quads;
+                const uint64_t quads = clear.pairs / 2, share = (quads + workgroups - 1) / workgroups, from = share * blockIdx.x;
+                const uint64_t to = from + share < quads ? from + share : quads;
                 for (uint64_t i = from + threadIdx.x; i < to; i += kThreads) __builtin_nontemporal_store(Quad(0.0f), reinterpret_cast<Quad*>(table_grad) + i);
+                if ((clear.pairs & 1u) != 0u && blockIdx.x == 0 && threadIdx.x == 0) reinterpret_cast<float2*>(table_grad)[clear.pairs - 1] = make_float2(0.0f, 0.0f);
                 for (uint32_t flag = blockIdx.x * kThreads + threadIdx.x; flag < clear.flags; flag += workgroups * kThreads) pass_bins.direct[flag] = 0u;
                 if (clear.rows != 0u) return;
             }

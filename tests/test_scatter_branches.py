@@ -109,7 +109,7 @@ def test_rows_take_other_groups_of_points_than_level_major_gradients(d, levels, 
                                                  (8, 2, 8, 131201, 1 << 22), (3, 2, 24, 17 * 8192 + 777, 1 << 20), (3, 2, 5, (1 << 19) + 3, (1 << 21) + 8192),
                                                  (3, 2, 19, 95077, 1 << 21), (6, 2, 17, 60013, 600002), (8, 2, 24, 25003, 1 << 20),
                                                  (2, 2, 24, 700001, 1 << 20), (3, 2, 24, 700001, (1 << 21) + 8192),
-                                                 (3, 2, 8, 200003, 1 << 14), (2, 2, 12, 300007, 30001)])
+                                                 (3, 2, 8, 200003, 1 << 14), (2, 2, 12, 300007, 30001), (2, 2, 21, 100003, 1342081), (2, 2, 21, 800003, 1342081)])
 def test_scatter_with_more_workspace(d, feat, levels, n, cap):
     """Large tables: with lists of deferred adds in the workspace the scatter clears the gradient (in rows of workgroups that do nothing else, for
     16 M points times levels in shares of all), whatever it held, masked levels too, and what would go straight into it follows later: column sums of the
