@@ -429,9 +429,11 @@ class EncodingWrapper:
             key = self._half_key(lattice_values)
         kept = self._half_copy
         if kept is not None and kept[0] == key:
-            if (_bridge or bridge()).capture_id(kept[2]):
-                self.fixed_params.m_captured_copy = kept[1].data_ptr()
-            return self._for_this_stream(kept)
+            copy = self._for_this_stream(kept)
+            if copy is not None:
+                if (_bridge or bridge()).capture_id(kept[2]):
+                    self.fixed_params.m_captured_copy = copy.data_ptr()
+                return copy
         if not lattice_values.is_cuda:
             return lattice_values.detach().to(self.half_table)  # (for the checks, which refuse it)
         capture = (_bridge or bridge()).capture_id(lattice_values.get_device())
@@ -455,12 +457,15 @@ class EncodingWrapper:
     @staticmethod
     def _for_this_stream(kept):
         """The copy of a ``_made_now``.  It was made in the middle of a program, by a call on some stream: one on another stream waits for it, and
-        keeps its memory from reuse."""
+        keeps its memory from reuse.  None for a call that is captured and cannot wait."""
         _, copy, device, stream, event, *_ = kept
         if stream != _raw_stream(device):
             native = _bridge or bridge()
             if event[0] is None:  # (made on the default stream)
-                event[0] = native.record_event(device)
+                recorded = native.record_event(device)
+                if recorded is None:
+                    return None
+                event[0] = recorded
             native.wait_for_event(event[0], device)
             if not native.capture_id(device):
                 copy.record_stream(torch.cuda.current_stream(device))
@@ -485,13 +490,16 @@ class EncodingWrapper:
         kept = self._cells
         if kept is not None:
             if kept[0] == key and lattice_values.is_contiguous():
-                return kept[1] if kept[3] == _raw_stream(kept[2]) else self._for_this_stream(kept), True
-            self._cells = None
+                copy = kept[1] if kept[3] == _raw_stream(kept[2]) else self._for_this_stream(kept)
+                if copy is not None:
+                    return copy, True
+            else:
+                self._cells = None
         half = self._half_copy
         if half is not None and half[0] == key:
             points = half[5]
             if points < 0:
-                return half[1] if half[3] == _raw_stream(half[2]) else self._for_this_stream(half), False
+                return half[1] if half[3] == _raw_stream(half[2]) else self.gather_table(lattice_values, key, 0, points), False
         else:
             half, points = None, self._points_for_cells(lattice_values)
         try:
@@ -506,7 +514,9 @@ class EncodingWrapper:
                 cells = self._make_cells(lattice_values, positions, anneal_window, key, so_far, points)
                 if cells is not None:
                     return cells, True
-        return (self.gather_table(lattice_values, key, so_far, points) if half is None else self._for_this_stream(half)), False
+        if half is not None and half[3] == _raw_stream(half[2]):
+            return half[1], False
+        return self.gather_table(lattice_values, key, so_far, points), False
 
     def _make_cells(self, lattice_values, positions, anneal_window, key, so_far, points):
         if lattice_values.requires_grad and torch.is_grad_enabled() and so_far < 4 * points:

@@ -1096,7 +1096,8 @@ PyObject* py_capture_id(PyObject*, PyObject* device) {
     });
 }
 
-// record_event(device) -> a capsule: what the device's default stream has been given so far.  For the device's own streams alone: a fence for the host, which
+// record_event(device) -> a capsule: what the device's default stream has been given so far; None where the current stream is captured and
+// the default stream would wait for it (torch's streams are none of these).  For the device's own streams alone: a fence for the host, which
 // an event of torch's has, would stand between the launches before it and after it.
 constexpr const char* kEventCapsule = "penc.event";
 PyObject* event_of_stream(hipStream_t stream) {
@@ -1114,6 +1115,12 @@ PyObject* py_record_event(PyObject*, PyObject* device) {
         const auto index = static_cast<c10::DeviceIndex>(PyLong_AsLong(device));
         if (PyErr_Occurred()) return nullptr;
         const c10::DeviceGuard guard(at::Device(at::kCUDA, index));
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(index).stream();
+        unsigned flags = hipStreamNonBlocking;
+        if (capture_of(stream) != 0 && (hipStreamGetFlags(stream, &flags) != hipSuccess || (flags & hipStreamNonBlocking) == 0)) {
+            (void)hipGetLastError();
+            Py_RETURN_NONE;
+        }
         c10::hip::HIPStreamCaptureModeGuard in_a_capture_too{hipStreamCaptureModeRelaxed};
         return event_of_stream(nullptr);
     });

@@ -470,6 +470,41 @@ def test_a_capture_waits_for_a_copy_made_on_another_stream(cells):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cells", [False, True])
+def test_a_capture_on_a_stream_the_default_stream_waits_for(cells):
+    """No event can be recorded on the default stream, which made the copy, while such a stream is captured: the graph makes its own."""
+    import ctypes
+    import permutohedral_encoding_amd as pe
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipStreamCreate.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    m = pe.PermutoEncoding(3, 1 << 16, 6, 2, np.geomspace(1.0, 1e-3, 6), lattice_half_precision=torch.bfloat16)
+    few, many = torch.rand(1000, 3, device="cuda"), torch.rand(pe._native.lib().penc_table_cells_points(2, 1 << 16, 2), 3, device="cuda")
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    stream, graph = torch.cuda.ExternalStream(handle.value), torch.cuda.CUDAGraph()
+    with torch.no_grad():
+        want = m(many if cells else few)[:1000]
+        points = many[:1000].contiguous() if cells else few
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.capture_begin()
+            got = m(points)
+            graph.capture_end()
+        assert (m.lattice._cells is not None) == cells and m.lattice._captured is not None
+        for _ in range(3):
+            got.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(m(points), want)
+    del graph, got
+    torch.cuda.synchronize()
+    assert hip.hipStreamDestroy(handle) == 0
+
+
+@pytest.mark.gpu
 def test_a_16_bit_copy_that_a_capture_makes_is_that_captures_alone():
     """Neither a call outside, before the graph has run, nor another graph reads it; the calls of one capture share it."""
     import permutohedral_encoding_amd as pe
