@@ -385,10 +385,11 @@ int penc_transpose(const float* src, float* dst, int64_t rows, int cols, void* s
  *   rem0, rank : the remainder-0 lattice point and the residual ranks after the hyperplane wrap
  *   slot       : hashed table index of each of the D+1 vertices
  *   barycentric: the D+1 interpolation weights
- * The kernels share one routine for rem0 and rank and have two equivalent routines for slots and
- * weights; gather_path picks which one is reported: 0 = the compare-and-select chains of the
- * scattering and position-gradient kernels, 1 = the rank sort through LDS of the forward and
- * grad-of-grad kernels (reference: EncodingGPU.cuh:130-223). */
+ * There is one routine for rem0 and rank, and several equivalent ones for slots and weights;
+ * gather_path picks which is reported: 0 = the compare-and-select chains of the position-gradient
+ * and group-sorting kernels, 1 = the rank sort through LDS of the forward and grad-of-grad kernels,
+ * 2 and 3 = the sorting network of the scatter, first order and both (reference: EncodingGPU.cuh:130-223). With 2,
+ * where D+1 is a power of two, equal residuals may leave a vertex whose weight is 0 open: its slot may be that of either. */
 int penc_simplex_debug(int pos_dim, int64_t nr_positions, int nr_levels, int capacity,
                        const float* positions, const float* scale_factor, const float* random_shift,
                        int gather_path, int* rem0, int* rank, int* slot, float* barycentric, void* stream);

@@ -749,8 +749,8 @@ class EncodingWrapper:
         """Introspection: dict(rem0, rank, slot (int32), barycentric) each of shape (L, N, D+1).
 
         ``gather_path`` picks the device routine whose slots and weights are reported: False for the
-        select chains of the scattering and position-gradient kernels, True for the LDS rank sort of
-        the forward and grad-of-grad kernels."""
+        select chains of the position-gradient and group-sorting kernels, True for the LDS rank sort of
+        the forward and grad-of-grad kernels, 2 and 3 for the sorting network of the scatter (first order, both)."""
         fp = self.fixed_params
         _check_f32_gpu(positions, "positions", 2)
         pos = positions.contiguous()
@@ -761,7 +761,7 @@ class EncodingWrapper:
         shift = fp.m_random_shift_per_level.contiguous()
         with torch.cuda.device(pos.device):
             _check(lib().penc_simplex_debug(self.pos_dim, n, levels, int(capacity), _ptr(pos),
-                                            _ptr(fp.m_scale_factor.to(pos.device)), _ptr(shift), int(bool(gather_path)),
+                                            _ptr(fp.m_scale_factor.to(pos.device)), _ptr(shift), int(gather_path),
                                             _ptr(out["rem0"]),
                                             _ptr(out["rank"]), _ptr(out["slot"]), _ptr(out["barycentric"]), _stream()),
                    "simplex_debug")

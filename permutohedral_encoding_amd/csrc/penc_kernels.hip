@@ -649,10 +649,11 @@ touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, flo
 // ------------------------------------------------------------------------------------------
 // introspection
 
-// kViaLds selects which of the two equivalent device routines produce the slots and weights: the
-// compare-and-select chains (vertex_hashes / barycentric: table backward, position backward) or
-// the thread-private LDS column (sort_by_rank_lds: forward, grad-of-grad).
-template <int D, bool kViaLds>
+// kRoutine selects which of the equivalent device routines produces the slots and weights: the
+// compare-and-select chains (vertex_hashes / barycentric: position backward, sorted groups), the thread-private LDS column
+// (sort_by_rank_lds: forward, grad-of-grad), or the sorting network (cyclic_simplex: the scatter, of the first order or of both).
+enum SimplexRoutine : int { kBySelects = 0, kByLds = 1, kByNetwork = 2, kByNetworkBothOrders = 3 };
+template <int D, int kRoutine>
 __global__ void __launch_bounds__(kBlock)
 simplex_debug_kernel(int n_points, uint32_t capacity, uint32_t cap_mask, const float* __restrict__ positions,
                      const float* __restrict__ scale_factor, const float* __restrict__ random_shift,
@@ -664,7 +665,13 @@ simplex_debug_kernel(int n_points, uint32_t capacity, uint32_t cap_mask, const f
     const Located<D> s = locate<D>(load_point<D>(positions, n), random_shift + level * D, scale_factor + level * D);
     uvec<D + 1> h;
     fvec<D + 1> w;
-    if constexpr (kViaLds) {
+    if constexpr (kRoutine >= kByNetwork) {
+        const fvec<D> point = load_point<D>(positions, n);
+        const CyclicSimplex<D> c = cyclic_simplex<D, true, kRoutine == kByNetworkBothOrders>(point, point, random_shift + level * D,
+                                                                                             scale_factor + level * D, capacity, cap_mask);
+        h = turn_back<D + 1>(c.slot, c.turned);
+        w = turn_back<D + 1>(c.w, c.turned);
+    } else if constexpr (kRoutine == kByLds) {
         __shared__ uint2 columns[(D + 1) * kBlock];
         fvec<D + 1> sorted;
         sort_by_rank_lds<D>(columns + threadIdx.x, kBlock, s.rank, s.delta, s.hash0, sorted, h);
@@ -678,7 +685,7 @@ simplex_debug_kernel(int n_points, uint32_t capacity, uint32_t cap_mask, const f
         PENC_INDEX(i);
         if (rem0) rem0[o + i] = s.rem0[i];
         if (rank) rank[o + i] = s.rank[i];
-        if (slot) slot[o + i] = static_cast<int>(to_slot(h[i], capacity, cap_mask));
+        if (slot) slot[o + i] = static_cast<int>(kRoutine >= kByNetwork ? h[i] : to_slot(h[i], capacity, cap_mask));
         if (bary) bary[o + i] = w[i];
     });
 }
@@ -2479,15 +2486,16 @@ int penc_simplex_debug(int pos_dim, int64_t nr_positions, int nr_levels, int cap
     if (!positions || !scale_factor || !random_shift) return PENC_ERR_NULL_POINTER;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid(tiles(nr_positions), nr_levels);
-#define PENC_LAUNCH_DEBUG(VIA_LDS)                                                                                   \
-    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((simplex_debug_kernel<DD, VIA_LDS>), grid, dim3(kBlock), 0, st,       \
+#define PENC_LAUNCH_DEBUG(ROUTINE)                                                                                   \
+    PENC_DISPATCH_D(pos_dim, hipLaunchKernelGGL((simplex_debug_kernel<DD, ROUTINE>), grid, dim3(kBlock), 0, st,       \
                                                 static_cast<int>(nr_positions), static_cast<uint32_t>(capacity),     \
                                                 mask_of(capacity), positions, scale_factor, random_shift, rem0, rank, \
                                                 slot, barycentric))
-    if (gather_path) {
-        PENC_LAUNCH_DEBUG(true);
-    } else {
-        PENC_LAUNCH_DEBUG(false);
+    switch (gather_path) {
+        case kBySelects: PENC_LAUNCH_DEBUG(kBySelects); break;
+        case kByNetwork: PENC_LAUNCH_DEBUG(kByNetwork); break;
+        case kByNetworkBothOrders: PENC_LAUNCH_DEBUG(kByNetworkBothOrders); break;
+        default: PENC_LAUNCH_DEBUG(kByLds); break;
     }
 #undef PENC_LAUNCH_DEBUG
     return check_launch();

@@ -97,11 +97,20 @@ struct Located {
     uint32_t hash0;      // raw hash of vertex 0
 };
 
-// Elevate, round, rank, wrap (EncodingGPU.cuh:130-186) for one point at one level.
-// `shift` and `sf` point at this level's D random shifts and D scale factors.
 template <int D>
-__device__ __forceinline__ Located<D> locate(fvec<D> pos, const float* __restrict__ shift,
-                                             const float* __restrict__ sf) {
+struct Rounded {
+    fvec<D + 1> resid;     // (elevated - rounded) / kUnit: exact in fp32 (the two are within (D+1)/2 of each other)
+    ivec<D + 1> multiple;  // rounded / kUnit
+    int sum;               // of the rounded coordinates, in units of D+1
+    // Where D+1 is a power of two, dividing by it is exact and everything is kept divided (kUnit is what resid and `multiple` count in).
+    static constexpr bool kExactInverse = ((D + 1) & D) == 0;
+    static constexpr float kUnit = kExactInverse ? static_cast<float>(D + 1) : 1.0f;
+};
+
+// Elevate and round (EncodingGPU.cuh:130-158) for one point at one level.
+// `shift` and `sf` point at this level's D random shifts and D scale factors.
+template <int D, bool kLowerAtTies = true>
+__device__ __forceinline__ Rounded<D> elevate_and_round(fvec<D> pos, const float* __restrict__ shift, const float* __restrict__ sf) {
     constexpr int D1 = D + 1;
     constexpr float kInv = 1.0f / D1;
     fvec<D1> elevated;
@@ -118,32 +127,43 @@ __device__ __forceinline__ Located<D> locate(fvec<D> pos, const float* __restric
     // Round every coordinate to the nearer multiple of D+1, the lower one at a tie (:149-158).  The
     // upper candidate is formed as down + (D+1) instead of ceil(v)*(D+1): the two differ only when v
     // is an integer, where the reference's candidates coincide and the lower one is chosen here too.
-    // Where D+1 is a power of two, dividing by it is exact and everything below is kept divided (kUnit is what resid and `multiple` count
-    // in): the nearer integer is then one instruction, which takes the even one at a tie, and the lower one has to be put right
-    // where that was the upper.  (D = 3: 20 of 300 vector instructions per point and level of the scatter.)
-    constexpr bool kExactInverse = (D1 & (D1 - 1)) == 0;
-    constexpr float kUnit = kExactInverse ? static_cast<float>(D1) : 1.0f;
-    fvec<D1> resid;     // (elevated - rounded) / kUnit: exact in fp32 (the two are within (D+1)/2 of each other)
-    ivec<D1> multiple;  // rounded / kUnit
-    int sum = 0;        // of the rounded coordinates, in units of D+1
+    // Where D+1 is a power of two the nearer integer is one instruction, which takes the even one at a tie, and the lower one has to be put right
+    // where that was the upper (unless a caller may do without: see cyclic_simplex).
+    Rounded<D> o;
+    o.sum = 0;
     static_for<D1>(PENC_BODY(i) {
         PENC_INDEX(i);
         const float e = elevated[i];
-        if constexpr (kExactInverse) {
+        if constexpr (Rounded<D>::kExactInverse) {
             const float v = e * kInv, nearest = __builtin_rintf(v), r = v - nearest;
-            const bool lower = r == -0.5f;
-            multiple[i] = static_cast<int>(nearest) - (lower ? 1 : 0);
-            resid[i] = lower ? 0.5f : r;
+            const bool lower = kLowerAtTies && r == -0.5f;
+            o.multiple[i] = static_cast<int>(nearest) - (lower ? 1 : 0);
+            o.resid[i] = lower ? 0.5f : r;
         } else {
             const float down = __builtin_floorf(e * kInv) * static_cast<float>(D1);
             const float up = down + static_cast<float>(D1);
             const float b = (up - e < e - down) ? up : down;
-            multiple[i] = static_cast<int>(b);
-            resid[i] = e - b;
+            o.multiple[i] = static_cast<int>(b);
+            o.resid[i] = e - b;
         }
-        sum += multiple[i];
+        o.sum += o.multiple[i];
     });
-    if constexpr (!kExactInverse) sum /= D1;
+    if constexpr (!Rounded<D>::kExactInverse) o.sum /= D1;
+    return o;
+}
+
+// Elevate, round, rank, wrap (EncodingGPU.cuh:130-186) for one point at one level.
+template <int D>
+__device__ __forceinline__ Located<D> locate(fvec<D> pos, const float* __restrict__ shift,
+                                             const float* __restrict__ sf) {
+    constexpr int D1 = D + 1;
+    constexpr float kInv = 1.0f / D1;
+    constexpr bool kExactInverse = Rounded<D>::kExactInverse;
+    constexpr float kUnit = Rounded<D>::kUnit;
+    const Rounded<D> rounded = elevate_and_round<D>(pos, shift, sf);
+    const fvec<D1> resid = rounded.resid;
+    const ivec<D1> multiple = rounded.multiple;
+    const int sum = rounded.sum;
 
     ivec<D1> rank = 0;
     static_for<D>(PENC_BODY(i) {
@@ -272,59 +292,6 @@ __device__ __forceinline__ void sort_by_rank_lds(uint2* column, uint32_t stride,
     });
 }
 
-// The same with the thread's cells two by two in 16-byte entries `stride` entries apart.
-template <int D>
-__device__ __forceinline__ void sort_by_rank_entries(uint2* entry, uint32_t stride, ivec<D + 1> rank, fvec<D + 1> delta, uint32_t hash0,
-                                                     fvec<D + 1>& sorted, uvec<D + 1>& hashes) {
-    static_for<D + 1>(PENC_BODY(c) {
-        PENC_INDEX(c);
-        const float d = delta[c];
-        uint2 cell;
-        cell.x = __builtin_bit_cast(uint32_t, d);
-        cell.y = hash_step<D, c>();
-        const uint32_t row = static_cast<uint32_t>(rank[c] < 0 ? 0 : (rank[c] > D ? D : rank[c]));  // (as in sort_by_rank_lds)
-        entry[row * stride - (row & 1u) * (stride - 1u)] = cell;
-    });
-    uvec<D + 1> step;
-    static_for<D + 1>(PENC_BODY(m) {
-        PENC_INDEX(m);
-        const uint2 cell = entry[(m >> 1) * 2 * stride + (m & 1)];
-        sorted[m] = __builtin_bit_cast(float, cell.x);
-        step[m] = cell.y;
-    });
-    hashes[0] = hash0;
-    static_for<D>(PENC_BODY(r) {
-        PENC_INDEX(r); hashes[r + 1] = hashes[r] + step[D - r]; });
-}
-
-// The same through columns of four-byte cells, half the LDS, one kind of value at a time.
-template <int D>
-__device__ __forceinline__ uint32_t rank_row(ivec<D + 1> rank, int c) {
-    return static_cast<uint32_t>(rank[c] < 0 ? 0 : (rank[c] > D ? D : rank[c]));  // (the clamp: as in sort_by_rank_lds)
-}
-template <int D>
-__device__ __forceinline__ fvec<D + 1> by_rank_lds(uint32_t* column, uint32_t stride, ivec<D + 1> rank, fvec<D + 1> in) {
-    static_for<D + 1>(PENC_BODY(c) {
-        PENC_INDEX(c);
-        const float x = in[c];
-        column[rank_row<D>(rank, c) * stride] = __builtin_bit_cast(uint32_t, x);
-    });
-    fvec<D + 1> out;
-    static_for<D + 1>(PENC_BODY(m) {
-        PENC_INDEX(m); out[m] = __builtin_bit_cast(float, column[m * stride]); });
-    return out;
-}
-template <int D>
-__device__ __forceinline__ uvec<D + 1> vertex_hashes_lds(uint32_t* column, uint32_t stride, ivec<D + 1> rank, uint32_t hash0) {
-    static_for<D + 1>(PENC_BODY(c) {
-        PENC_INDEX(c); column[rank_row<D>(rank, c) * stride] = hash_step<D, c>(); });
-    uvec<D + 1> hashes;
-    hashes[0] = hash0;
-    static_for<D>(PENC_BODY(r) {
-        PENC_INDEX(r); hashes[r + 1] = hashes[r] + column[(D - r) * stride]; });
-    return hashes;
-}
-
 // The three gradient chains below evaluate their sums in the same order, with the same
 // intermediate roundings, as the reference's loops, so that every term a kernel adds is the same
 // fp32 number the CPU checker computes; only the order of atomic accumulation can then differ.
@@ -442,6 +409,224 @@ template <int D>
 __device__ __forceinline__ fvec<D + 1> pos_grad_grad_to_bary(ivec<D + 1> rank, fvec<D> q,
                                                              const float* __restrict__ sf) {
     return sorted_elevated_grad_to_bary<D>(by_rank<D>(rank, pos_grad_grad_to_elevated<D>(q, sf)));
+}
+
+// ------------------------------------------------------------------------------------------
+// the same simplex, its vertices in cyclic order
+//
+// A scatter adds every vertex's contribution on its own, so it needs the vertices' weights and slots but not which of them is which.
+// Then the residuals can be sorted as they are, before the wrap, and neither ranks nor the selects that bring D+1 values into
+// rank order are needed: with m the place in descending order, s[m] the residual and c_m its coordinate, and everything modulo D+1,
+//     place m wraps by q_m = floor((m + sum) / (D+1))                    (-1, 0 or 1: the reference's rank + sum beyond 0..D)
+//     d[m]   = (s[m] + (D+1) q_m) / (D+1)                                (its delta after the wrap)
+//     w_k    = d[D-k] - d[D+1-k], and 1 more where between the two the wrap begins, or does not and k = 0
+//     h_0    = sum_i rounded_i M^(D-i) - sum * sum_i M^(D-i),   h_{k+1} = h_k + hash step of c_{D-k}
+// are weight and raw hash of remainder vertex r = k - sum, the same fp32 numbers as those of the functions above (the steps of all
+// coordinates add up to zero, so the chain closes: it may begin at any vertex).  `turned` is sum modulo D+1: turn_back() brings them into the order of r.
+//
+// The sort is a network of compare-exchanges, each two instructions (v_max_f64, v_min_f64, at the rate of an fp32 comparison on gfx950): a key is a double
+// whose upper word is the residual's fp32 bits, which order doubles as they order floats, and whose lower word, the hash step, comes along.
+// Equal residuals have to be taken in the order of their coordinates (the lower first): the upper four bits of the lower word see to that, reversed
+// for negative residuals, whose order by magnitude is the reverse; the steps then count modulo 2^28, which capacities that are powers of two up to that
+// hide, and for others the upper bits are put back.  Where D+1 is a power of two and only barycentric weights are wanted, the vertex that two equal residuals
+// leave open has the weight 0 exactly, and a residual of a half is as good on either side: neither is looked after (kOpenTies).
+// Against ranks, selects and trips through the LDS: the scatter of 2^20 points, 24 levels of 2^18 slots, D = 3 issues 94 M vector instructions instead of 120 M
+// (2^19 points, 16 levels of 2^19 slots, D = 8: 100 M of 113 M, and 18 KB of LDS less); it is bound by them at the coarse levels only, so a training step with it
+// goes 726 -> 722 us (D = 8: 715 -> 701; the gradient of both orders, 2^22 slots, 1239 -> 1230).
+template <int N> using dvec = double __attribute__((ext_vector_type(N)));
+
+// Compare-exchanges (place of the larger, place of the smaller) that sort N keys.
+struct SortingNetwork {
+    int count;
+    int a[25], b[25];
+};
+template <int N>
+constexpr SortingNetwork sorting_network() {
+    static_assert(N >= 3 && N <= 9, "networks for 3 to 9 keys");
+    if constexpr (N == 3) return {3, {0, 0, 1}, {2, 1, 2}};
+    else if constexpr (N == 4) return {5, {0, 1, 0, 2, 1}, {2, 3, 1, 3, 2}};
+    else if constexpr (N == 5) return {9, {0, 1, 0, 1, 0, 2, 1, 3, 2}, {3, 4, 2, 3, 1, 4, 2, 4, 3}};
+    else if constexpr (N == 6) return {12, {0, 1, 2, 1, 3, 0, 2, 0, 2, 4, 1, 3}, {5, 3, 4, 2, 4, 3, 5, 1, 3, 5, 2, 4}};
+    else if constexpr (N == 7) return {16, {0, 2, 4, 0, 1, 3, 0, 2, 3, 1, 4, 2, 4, 1, 3, 5}, {6, 3, 5, 2, 4, 6, 1, 5, 4, 2, 6, 3, 5, 2, 4, 6}};
+    else if constexpr (N == 8)
+        return {19, {0, 1, 4, 5, 0, 1, 2, 3, 0, 2, 4, 6, 2, 3, 1, 3, 1, 3, 5}, {2, 3, 6, 7, 4, 5, 6, 7, 1, 3, 5, 7, 4, 5, 4, 6, 2, 4, 6}};
+    else
+        return {25, {0, 1, 2, 4, 0, 2, 3, 5, 0, 1, 4, 7, 1, 3, 5, 0, 2, 3, 6, 2, 4, 6, 1, 3, 5},
+                {3, 7, 5, 8, 7, 4, 8, 6, 2, 3, 5, 8, 4, 6, 7, 1, 4, 5, 8, 3, 5, 7, 2, 4, 6}};
+}
+// (a network that sorts all sequences of zeros and ones sorts everything)
+template <int N>
+constexpr bool sorts_everything() {
+    const SortingNetwork net = sorting_network<N>();
+    for (uint32_t keys = 0; keys < (1u << N); ++keys) {
+        uint32_t k = keys;
+        for (int e = 0; e < net.count; ++e) {
+            const uint32_t larger = (k >> net.a[e]) & 1u, smaller = (k >> net.b[e]) & 1u;
+            if (larger < smaller) k ^= (1u << net.a[e]) | (1u << net.b[e]);
+        }
+        if ((k & (k + 1u)) != 0u) return false;  // the ones are the first places
+    }
+    return true;
+}
+template <int N>
+constexpr SortingNetwork kNetwork = sorting_network<N>();
+static_assert(sorts_everything<3>() && sorts_everything<4>() && sorts_everything<5>() && sorts_everything<6>() && sorts_everything<7>() &&
+                  sorts_everything<8>() && sorts_everything<9>(),
+              "every network sorts");
+
+// v_max_f64 and v_min_f64 as they are: the builtins would first quiet operands that might be signalling NaNs.  No key is one: it would take an fp32 NaN with a
+// payload of its own (the hardware's has none); such a point's slots are as meaningless as any NaN's, and within the table.
+__device__ __forceinline__ double larger_key(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double smaller_key(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double make_key(uint32_t lower, float upper) {
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(__builtin_bit_cast(uint32_t, upper)) << 32) | lower);
+}
+
+constexpr uint32_t kKeyStepBits = 28;
+template <int D, int... C>
+constexpr uint64_t upper_step_bits(std::integer_sequence<int, C...>) {  // the upper four bits of coordinate c's hash step at 4 (D - c)
+    return ((static_cast<uint64_t>(hash_step<D, C>() >> kKeyStepBits) << (4 * (D - C))) | ...);
+}
+
+template <int D>
+struct CyclicSimplex {
+    fvec<D + 1> w;         // barycentric weights (kFirst)
+    fvec<D + 1> dB;        // derivatives of the weights along the direction given (kSecond; see pos_grad_grad_to_bary)
+    uvec<D + 1> slot;
+    int turned;
+};
+
+template <int D, bool kFirst, bool kSecond>
+__device__ __forceinline__ CyclicSimplex<D> cyclic_simplex(fvec<D> pos, fvec<D> q, const float* __restrict__ shift, const float* __restrict__ sf,
+                                                           uint32_t capacity, uint32_t cap_mask) {
+    constexpr int D1 = D + 1;
+    constexpr float kInv = 1.0f / D1;
+    constexpr bool kExactInverse = Rounded<D>::kExactInverse;
+    constexpr bool kOpenTies = kExactInverse && !kSecond;
+    constexpr uint32_t kOrderBits = ~((1u << kKeyStepBits) - 1u);
+    const Rounded<D> rounded = elevate_and_round<D, !kOpenTies>(pos, shift, sf);
+    const int sum = rounded.sum;
+
+    uint32_t h0 = 0u;
+    dvec<D1> key;
+    static_for<D1>(PENC_BODY(c) {
+        PENC_INDEX(c);
+        const float r = rounded.resid[c];
+        if constexpr (c < D) h0 += static_cast<uint32_t>(rounded.multiple[c]) * (static_cast<uint32_t>(Rounded<D>::kUnit) * hash_pow(D - c));
+        if constexpr (kOpenTies) {
+            key[c] = make_key(hash_step<D, c>(), r);
+        } else {
+            constexpr uint32_t kLower = (static_cast<uint32_t>(D - c) << kKeyStepBits) | (hash_step<D, c>() & ~kOrderBits);
+            key[c] = make_key(kLower ^ (static_cast<uint32_t>(__builtin_bit_cast(int, r) >> 31) & kOrderBits), r);
+        }
+    });
+    h0 -= static_cast<uint32_t>(sum) * hash_pow_sum<D>();
+    fvec<D1> along = 0.0f;  // d(weights)/d(elevated coordinates) along the direction, in the order of the keys
+    if constexpr (kSecond) along = pos_grad_grad_to_elevated<D>(q, sf);
+
+    static_for<kNetwork<D1>.count>(PENC_BODY(e) {
+        PENC_INDEX(e);
+        constexpr int a = kNetwork<D1>.a[e], b = kNetwork<D1>.b[e];
+        const double x = key[a], y = key[b];
+        if constexpr (kSecond) {
+            const float u = along[a], v = along[b];
+            const bool swap = x < y;
+            along[a] = swap ? v : u;
+            along[b] = swap ? u : v;
+        }
+        key[a] = larger_key(x, y);
+        key[b] = smaller_key(x, y);
+    });
+    if constexpr (kSecond) {  // (moved behind the next branch, the exchanges would keep every stage of the keys in registers)
+        static_for<D1>(PENC_BODY(m) {
+            PENC_INDEX(m);
+            float x = along[m];
+            asm volatile("" : "+v"(x));
+            along[m] = x;
+        });
+    }
+    fvec<D1> sorted;
+    uvec<D1> step;
+    static_for<D1>(PENC_BODY(m) {
+        PENC_INDEX(m);
+        const double k = key[m];
+        const uint64_t bits = __builtin_bit_cast(uint64_t, k);
+        sorted[m] = __builtin_bit_cast(float, static_cast<uint32_t>(bits >> 32));
+        step[m] = static_cast<uint32_t>(bits);
+    });
+    if constexpr (!kOpenTies) {
+        if (cap_mask == 0u || cap_mask >= (1u << kKeyStepBits)) {
+            constexpr uint64_t kUpper = upper_step_bits<D>(std::make_integer_sequence<int, D1>{});
+            static_for<D1>(PENC_BODY(m) {
+                PENC_INDEX(m);
+                const float r = sorted[m];
+                const uint32_t order = (step[m] ^ static_cast<uint32_t>(__builtin_bit_cast(int, r) >> 31)) >> kKeyStepBits;
+                step[m] = (step[m] & ~kOrderBits) | (static_cast<uint32_t>(kUpper >> (4u * order)) << kKeyStepBits);
+            });
+        }
+    }
+
+    CyclicSimplex<D> o;
+    uvec<D1> h;
+    h[0] = h0;
+    static_for<D>(PENC_BODY(k) {
+        PENC_INDEX(k); h[k + 1] = h[k] + step[D - k]; });
+    if (cap_mask != 0u) {  // (to_slot, asked once)
+        o.slot = h & cap_mask;
+    } else {
+        static_for<D1>(PENC_BODY(k) {
+            PENC_INDEX(k); o.slot[k] = h[k] % capacity; });
+    }
+    o.turned = kExactInverse ? (sum & D) : (sum < 0 ? sum + D1 : sum);
+    if constexpr (kFirst) {
+        fvec<D1> d, wrap;
+        static_for<D1>(PENC_BODY(m) {
+            PENC_INDEX(m);
+            if constexpr (kExactInverse) {
+                constexpr int kLog2 = __builtin_ctz(D1);
+                wrap[m] = static_cast<float>((sum + m) >> kLog2);
+                d[m] = sorted[m] + wrap[m];
+            } else {
+                wrap[m] = (sum > D - m ? 1.0f : 0.0f) - (sum < -m ? 1.0f : 0.0f);
+                d[m] = __builtin_fmaf(wrap[m], static_cast<float>(D1), sorted[m]) * kInv;
+            }
+        });
+        o.w[0] = d[D] + ((1.0f + wrap[0] - wrap[D]) - d[0]);
+        static_for<D>(PENC_BODY(kk) {
+            PENC_INDEX(kk);
+            constexpr int k = kk + 1;
+            o.w[k] = d[D - k] + ((wrap[D1 - k] - wrap[D - k]) - d[D1 - k]);
+        });
+    }
+    if constexpr (kSecond) o.dB = sorted_elevated_grad_to_bary<D>(along);
+    return o;
+}
+
+// in[k] of a CyclicSimplex in the order of the remainder vertices.
+template <int N, typename V>
+__device__ __forceinline__ V turn_back(V in, int turned) {
+    static_for<4>(PENC_BODY(bit) {
+        PENC_INDEX(bit);
+        constexpr int kBy = 1 << bit;
+        if constexpr (kBy < N) {
+            const bool by = (turned & kBy) != 0;
+            const V from = in;
+            static_for<N>(PENC_BODY(r) {
+                PENC_INDEX(r);
+                const auto stay = from[r], other = from[(r + kBy) % N];
+                in[r] = by ? other : stay;
+            });
+        }
+    });
+    return in;
 }
 
 }  // namespace penc

@@ -67,7 +67,6 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                         const ClearTargetOf<kBins>& clear) {
     constexpr bool kNeedsQ = kOrder != kFirstOrder, kBoth = kOrder == kBothOrders, kManyBins = kBins >= kBinsMany;
     __shared__ ScatterStateT<stage_chunk(D), kThreads> state;
-    __shared__ uint32_t rank_columns[D > kWorkgroupSortMaxDim ? (D + 1) * kThreads : 1];
     // Workgroups are dealt round-robin to the chip's `dies` dies, each with an L2 of its own.  The j-th
     // workgroup of a die takes level j % levels of one group of points: a die works through all
     // levels of a group before the next group, so the points are fetched from memory once, and
@@ -178,107 +177,31 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                 out[n_points] = g1;
             }
         }
-        const Located<D> s = locate<D>(pos, random_shift + level * D, scale_factor + level * D);
-        uvec<D + 1> h;
-        fvec<D + 1> w;   // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
-        fvec<D + 1> w2;  // kBoth: the latter
-        bool via_lds = false;
-        if constexpr (D > kWorkgroupSortMaxDim && kThreads == kScatterBlock) {
-            // Once the workgroup streams with every wave sorting on its own (stream_tile_wave), a wave's staging
-            // slice is idle between its tiles and nobody else touches it: it serves as the thread-private
-            // columns that put residuals and hash steps into rank order, in place of D(D+1) selects each
-            // (at D = 8 about 270 of 1350 vector instructions per point and level).
-            via_lds = !kManyBins && mode == kModeStream;
-        }
-        if (via_lds) {
-            constexpr uint32_t kSliceCells = ScatterStateT<stage_chunk(D), kThreads>::kChunk * 64 * 2;  // 8-byte cells of a wave's slice
-            static_assert((D + 1) * 64 <= kSliceCells, "a wave's staging slice holds a column of D+1 cells per lane");
-            uint2* const column = reinterpret_cast<uint2*>(state.val) + (threadIdx.x >> 6) * kSliceCells + (threadIdx.x & 63);
-            fvec<D + 1> sorted;
-            if constexpr (kBoth) {
-                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-                wave_lds_fence();
-                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else if constexpr (kOrder == kSecondOrder) {
-                sort_by_rank_lds<D>(column, 64, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else {
-                sort_by_rank_lds<D>(column, 64, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-            }
-            wave_lds_fence();  // the slice is staging space again from here on
-        } else if constexpr (D > kWorkgroupSortMaxDim) {
-            // the other modes have no such slice: columns of their own
-            uint32_t* const column = rank_columns + threadIdx.x;
-            h = vertex_hashes_lds<D>(column, kThreads, s.rank, s.hash0);
-            if constexpr (kOrder != kSecondOrder) w = barycentric_of_sorted<D>(by_rank_lds<D>(column, kThreads, s.rank, s.delta)) * w_level;
-            if constexpr (kOrder != kFirstOrder) {
-                const fvec<D + 1> second = sorted_elevated_grad_to_bary<D>(by_rank_lds<D>(
-                                               column, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D))) * w_level;
-                if constexpr (kBoth) w2 = second;
-                else w = second;
-            }
-        } else if (D >= 4 && mode == kModeStream) {
-            // The staging entries that a thread stores from are read by nobody else and written by others only after the tile's first
-            // barrier: until then they serve as its column.  (D = 4, 24 levels of 2^18 slots, 2^20 points, scatter and reduction 592 -> 585 us, second
-            // order 617 -> 607; with D = 3 the selects are as few as the trip through LDS.)
-            static_assert((D + 2) / 2 <= ScatterStateT<stage_chunk(D), kThreads>::kChunk, "a thread's staging entries hold its D+1 cells");
-            uint2* const entry = reinterpret_cast<uint2*>(state.val) + 2 * threadIdx.x;
-            fvec<D + 1> sorted;
-            if constexpr (kBoth) {
-                sort_by_rank_entries<D>(entry, kThreads, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-                sort_by_rank_entries<D>(entry, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w2 = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else if constexpr (kOrder == kSecondOrder) {
-                sort_by_rank_entries<D>(entry, kThreads, s.rank, pos_grad_grad_to_elevated<D>(q, scale_factor + level * D), s.hash0, sorted, h);
-                w = sorted_elevated_grad_to_bary<D>(sorted) * w_level;
-            } else {
-                sort_by_rank_entries<D>(entry, kThreads, s.rank, s.delta, s.hash0, sorted, h);
-                w = barycentric_of_sorted<D>(sorted) * w_level;
-            }
-        } else {
-            h = vertex_hashes<D>(s.rank, s.hash0);
-            if constexpr (kBoth) {
-                w = barycentric<D>(s.rank, s.delta) * w_level;
-                w2 = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
-            } else if constexpr (kOrder == kSecondOrder) {
-                w = pos_grad_grad_to_bary<D>(s.rank, q, scale_factor + level * D) * w_level;
-            } else {
-                w = barycentric<D>(s.rank, s.delta) * w_level;
-            }
-        }
-        uvec<D + 1> slot;
-        if (cap_mask != 0u) {  // (to_slot, asked once)
-            slot = h & cap_mask;
-        } else {
-            static_for<D + 1>(PENC_BODY(r) {
-                PENC_INDEX(r); slot[r] = h[r] % capacity; });
-        }
+        CyclicSimplex<D> s = cyclic_simplex<D, kOrder != kSecondOrder, kNeedsQ>(pos, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask);
         if (t == 0) {
             // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
             // (its point is already here)
             const auto slots_of_next_tile = [&]() {
-                const Located<D> s1 = locate<D>(pos_next, random_shift + level * D, scale_factor + level * D);
-                const uvec<D + 1> h1 = vertex_hashes<D>(s1.rank, s1.hash0);
-                uvec<D + 1> slot1;
-                static_for<D + 1>(PENC_BODY(r) {
-                    PENC_INDEX(r);
-                    slot1[r] = to_slot(h1[r], capacity, cap_mask);
-                });
-                return slot1;
+                return cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
             };
             const bool next_active = tile_base + kThreads + threadIdx.x < n_points && tiles_per_group > 1;
-            mode = scatter_mode_decide<D>(state, bins, active, slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
+            mode = scatter_mode_decide<D>(state, bins, active, s.slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
+        }
+        // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
+        fvec<D + 1> w = (kOrder == kSecondOrder ? s.dB : s.w) * w_level;
+        fvec<D + 1> w2 = 0.0f;
+        if constexpr (kBoth) w2 = s.dB * w_level;
+        if (mode == kModeCache) {  // which folds lanes by vertex: the same vertex of a simplex in the same place in all lanes
+            s.slot = turn_back<D + 1>(s.slot, s.turned);
+            w = turn_back<D + 1>(w, s.turned);
+            if constexpr (kBoth) w2 = turn_back<D + 1>(w2, s.turned);
         }
         fvec<D + 1> a0 = w * g0, a1 = w * g1;  // g_f * (b_r * w_level), :405-410
         if constexpr (kBoth) {
             a0 += w2 * s0;
             a1 += w2 * s1;
         }
-        const uint32_t hits = scatter_tile<D, kManyBins>(state, level_grad, bins, group, static_cast<uint32_t>(t), active, cache_pays<D>(state, t), mode, id_bits, slot, a0, a1, cursor);
+        const uint32_t hits = scatter_tile<D, kManyBins>(state, level_grad, bins, group, static_cast<uint32_t>(t), active, cache_pays<D>(state, t), mode, id_bits, s.slot, a0, a1, cursor);
         // the first tile finds the lines its own look-up has claimed: no evidence of reuse
         if ((threadIdx.x & 63) == 0 && hits && t > 0) atomicAdd(&state.hits, hits);
         pos = pos_next;
