@@ -428,28 +428,32 @@ struct ScatterStateT {
     uint4 stage_tail[kTail > 0 ? kTail : 1];
     uint32_t bin_count[kMaxBins];  // records this workgroup has appended to each bin so far
     uint32_t hits;                 // contributions the cache has absorbed into existing lines since the first tile
-    // what the look-ups of the first tile's slots showed (see scatter_mode_decide)
-    uint32_t wanted;               // contributions of the first tile
-    uint32_t lines;                // lines they claimed: the tile's distinct slots, as far as the cache could take them
-    uint32_t misses;               // contributions whose slot found no line
+    // what the look at the first tile's slots showed (see scatter_mode_decide)
+    uint32_t distinct;             // of them, as far as the bits they were marked in tell them apart
+    uint32_t wanted;               // contributions of the first tile,
+    uint32_t first_hits;           // and how many of them find a line that an earlier one has claimed
     uint32_t columns;              // columns given away (kModeColumns)
     uint32_t deferred;             // entries of the workgroup's list of deferred adds
     uint32_t strangers;            // slots of the second tile that the first tile did not touch (counted for levels with few slots)
 };
 
+// The bits in which the first tile's slots are marked: 128 to a thread of the workgroup (2^16 or 2^17 of them), where the values will be.
+template <typename State>
+__device__ __forceinline__ uint32_t* seen_bits(State& c) { return reinterpret_cast<uint32_t*>(c.val); }
+template <typename State>
+__device__ __forceinline__ uint32_t seen_bit(uint32_t slot) {
+    return (slot * 0x9E3779B1u) >> (32 - __builtin_ctz(static_cast<unsigned>(State::kThreads) * 128u));
+}
+
+// Clears what the look at the first tile needs, and the bins' cursors.
 template <typename State>
 __device__ __forceinline__ void scatter_begin(State& c) {
-    for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) {
-        c.tag[e] = -1;
-        c.val[0][e] = 0.0;
-        c.val[1][e] = 0.0;
-    }
+    static_assert(State::kThreads * sizeof(uint4) <= sizeof(c.val), "the bits fit");
+    reinterpret_cast<uint4*>(seen_bits(c))[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
     for (int b = threadIdx.x; b < kMaxBins; b += State::kThreads) c.bin_count[b] = 0u;
     if (threadIdx.x == 0) {
         c.hits = 0u;
-        c.wanted = 0u;
-        c.lines = 0u;
-        c.misses = 0u;
+        c.distinct = 0u;
         c.strangers = 0u;
         c.columns = 0u;
     }
@@ -468,6 +472,16 @@ __device__ __forceinline__ bool append_record(State& c, const BinTarget& bins, u
     return true;
 }
 
+// From D = 4 on a third candidate line: every contribution of a slot that finds no line becomes
+// a record, and tens of thousands of records on a handful of slots serialise in the LDS of
+// the one reducer workgroup that owns their bin.  At D = 3 the low 11 bits of a coarse level's
+// slots are all distinct and two candidates leave no slot out while the level fits; at D = 4
+// they collide (levels 6 and 7 of 24: 350 and 1000 slots, 4 and 110 of them left out; those
+// levels' reducer workgroups took 0.05-0.11 ms each, and with a third candidate the
+// double backward's table half went from 0.73 to 0.65 ms; at D = 3 it would add 2% to the
+// scattering kernel for nothing).
+constexpr int cache_probes(int pos_dim) { return pos_dim >= 4 ? 3 : 2; }
+
 // Looks `slot` up in the accumulate cache, claiming a free line if there is one.  Two candidate
 // lines per slot (two-choice hashing): with one, a level with a few hundred distinct slots already
 // loses several of them to collisions, and those are exactly the slots every wave keeps hitting.
@@ -475,7 +489,7 @@ __device__ __forceinline__ bool append_record(State& c, const BinTarget& bins, u
 // line already held the slot (a hit, as opposed to a claim).
 // (Spreading the lanes that share a slot over replicated sub-tables, instead of folding them in
 // registers first, was measured 30% slower on the coarse levels, and no faster on top of folding.)
-template <int kProbes = 2, typename State>
+template <int kProbes, typename State>
 __device__ __forceinline__ int cache_find(State& c, uint32_t slot, bool& found) {
     const int want = static_cast<int>(slot);
     int e = static_cast<int>(slot & (kCacheLines - 1));
@@ -496,20 +510,6 @@ __device__ __forceinline__ int cache_find(State& c, uint32_t slot, bool& found) 
         if (probe + 1 < kProbes) e = static_cast<int>((slot * kMix[probe]) >> (32 - kCacheLinesLog2));
     }
     return -1;
-}
-
-// Whether `slot` holds a line of the cache, without claiming one.
-template <int kProbes = 2, typename State>
-__device__ __forceinline__ bool cache_holds(const State& c, uint32_t slot) {
-    const int want = static_cast<int>(slot);
-    int e = static_cast<int>(slot & (kCacheLines - 1));
-    constexpr uint32_t kMix[3] = {0x9E3779B1u, 0x85EBCA6Bu, 0xC2B2AE35u};
-#pragma unroll
-    for (int probe = 0; probe < kProbes; ++probe) {
-        if (c.tag[e] == want) return true;
-        if (probe + 1 < kProbes) e = static_cast<int>((slot * kMix[probe]) >> (32 - kCacheLinesLog2));
-    }
-    return false;
 }
 
 // Stage 2 for a whole tile once the workgroup streams (see scatter_mode_decide): the cache's LDS is
@@ -744,10 +744,7 @@ __device__ __forceinline__ void stream_tile_many(State& c, const GradSlice& leve
                 global_add_pairs(level_grad, spill, e.x, __builtin_bit_cast(float, e.y), __builtin_bit_cast(float, e.z));
         });
         // The next chunk (or tile) counts into counters this chunk has cleared, overwrites offset/dest after its
-        // first two barriers and what other threads read of the staging array after its third.  The entries a thread has stored
-        // from are its own before that (sort_by_rank_entries in the next tile writes them without a barrier): the fence
-        // keeps those writes behind the reads above.
-        wave_lds_fence();
+        // first two barriers and what other threads read of the staging array after its third.
     });
 }
 
@@ -1008,16 +1005,7 @@ __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& leve
             hits += fold_shared_slots(slot[r], miss, x0, x1);
             bool found = false;
             if (miss) {
-                // From D = 4 on a third candidate line: every contribution of a slot that finds no line becomes
-                // a record, and tens of thousands of records on a handful of slots serialise in the LDS of
-                // the one reducer workgroup that owns their bin.  At D = 3 the low 11 bits of a coarse level's
-                // slots are all distinct and two candidates leave no slot out while the level fits; at D = 4
-                // they collide (levels 6 and 7 of 24: 350 and 1000 slots, 4 and 110 of them left out; those
-                // levels' reducer workgroups took 0.05-0.11 ms each, and with a third candidate the
-                // double backward's table half went from 0.73 to 0.65 ms; at D = 3 it would add 2% to the
-                // scattering kernel for nothing).
-                constexpr int kProbes = D >= 4 ? 3 : 2;
-                const int e = cache_find<kProbes>(c, slot[r], found);
+                const int e = cache_find<cache_probes(D)>(c, slot[r], found);
                 if (e >= 0) {
                     __hip_atomic_fetch_add(&c.val[0][e], static_cast<double>(x0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     __hip_atomic_fetch_add(&c.val[1][e], static_cast<double>(x1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1035,16 +1023,13 @@ __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& leve
 
 // The workgroup-wide decision whether stage 1 is worth its LDS traffic at this level: keep using the
 // cache only while at least one contribution in `one_in` hits.  The evidence before tile `tile` is
-// the look-up of the first tile's slots (a contribution that neither claimed a line nor missed
-// would have hit) and the hits of the tiles processed since.  Against appending every miss to its
+// the look at the first tile's slots and the hits of the tiles processed since.  Against appending every miss to its
 // bin on its own, one hit in eight pays; against sorting the tile's records by bin (stream_tile),
 // which is cheaper than the cache's look-ups, it takes one in four.
 template <int D, typename State>
-__device__ __forceinline__ bool cache_pays(const State& c, int tile, uint32_t one_in = 8u) {
-    const uint32_t settled = c.lines + c.misses;
-    const uint32_t first_hits = c.wanted > settled ? c.wanted - settled : 0u;
+__device__ __forceinline__ bool cache_pays(const State& c, int tile) {
     const uint32_t seen = c.wanted + static_cast<uint32_t>(tile > 1 ? tile - 1 : 0) * State::kThreads * (D + 1);
-    return (first_hits + c.hits) * one_in >= seen;
+    return (c.first_hits + c.hits) * 8u >= seen;
 }
 
 // Sends every line of the accumulate cache on to stage 2 (or 3).  By all threads, between barriers.
@@ -1069,46 +1054,52 @@ __device__ __forceinline__ void cache_flush(State& c, const GradSlice& level_gra
 }
 
 // Before the first tile is scattered (all threads call it, with the tile's slots): decides for the
-// whole workgroup how the level goes.  The slots are looked up in the (empty) cache, which claims a
-// line for every distinct slot as far as it can; the counts tell what the cache is good for.  One
-// that would not hit is never filled: its LDS becomes staging space (kModeStream, see
-// stream_tile; needs bins).  One that hits on at most 64 lines, and whose group of points is not expected to
+// whole workgroup how the level goes, and clears the LDS for it.  Every slot is marked in a bit of its own, nearly, and a bit that was not set
+// yet is a slot more: the tile's distinct slots tell what the accumulate cache would be good for.  One
+// that would not hit is not used: its LDS becomes staging space (kModeStream, see
+// stream_tile; needs bins).  One that would hit on at most 64 lines, and whose group of points is not expected to
 // touch more than 96 slots in all, becomes columns (kModeColumns, `id_bits` says how many).  Otherwise the
-// cache serves, with the lines already claimed.
+// cache serves.
+// (One LDS operation for a contribution, all of a thread's made together.  Claiming the slots' lines in the cache itself to find out took a workgroup 5700 clocks,
+// up to 14000 among others, and all of its LDS had to be cleared before; a tile takes 4000 to 12000.  Scatter, us: D = 3, 2^20 points, 24 levels of 2^18 slots from
+// rows 348 -> 337; D = 8, 2^19 points, 16 levels of 2^19 306 -> 267; 2^22 slots, 200001 points, both orders 91.5 -> 86.)
 template <int D, typename State, typename NextSlots>
-__device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bins, bool active, uvec<D + 1> slot,
+__device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bins, bool active, uint32_t points, uvec<D + 1> slot,
                                                    uint32_t& id_bits, bool next_active, NextSlots&& slots_of_next_tile,
                                                    int tiles_per_group) {
-    uint32_t wanted = 0, missed = 0;  // over the wave
-    static_for<D + 1>(PENC_BODY(r) {
-        PENC_INDEX(r);
-        bool found = false;
-        const bool miss = active && cache_find(c, slot[r], found) < 0;
-        wanted += __popcll(__ballot(active));
-        missed += __popcll(__ballot(miss));
-    });
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&c.wanted, wanted);
-        if (missed != 0u) atomicAdd(&c.misses, missed);
+    uint32_t* const seen = seen_bits(c);
+    uvec<D + 1> before = 0xFFFFFFFFu;
+    if (active) {
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            const uint32_t bit = seen_bit<State>(slot[r]);
+            before[r] = atomicOr(&seen[bit >> 5], 1u << (bit & 31u)) >> (bit & 31u);
+        });
     }
-    __syncthreads();  // every line the tile wants is claimed
-    uint32_t used = 0;
-    for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) used += __popcll(__ballot(c.tag[e] != -1));
-    if ((threadIdx.x & 63) == 0 && used != 0u) atomicAdd(&c.lines, used);
+    uint32_t fresh = 0;  // over the wave
+    static_for<D + 1>(PENC_BODY(r) {
+        PENC_INDEX(r); fresh += __popcll(__ballot((before[r] & 1u) == 0u)); });
+    if ((threadIdx.x & 63) == 0) atomicAdd(&c.distinct, fresh);
+    __syncthreads();
+    const uint32_t wanted = points * (D + 1), distinct = c.distinct;
+    // Of u slots that each look for one of N lines at two places, N tanh(u/N) find one, and as large a part of the repeats does.
+    const float load = static_cast<float>(distinct) * (1.0f / kCacheLines), load2 = load * load;
+    const float held = (27.0f + load2) / (27.0f + 9.0f * load2);  // tanh(load) / load, within 2% up to twice as many slots as lines
+    const uint32_t first_hits = wanted > distinct ? static_cast<uint32_t>(static_cast<float>(wanted - distinct) * held) : 0u;
     // Columns are for a level whose few slots the whole group shares.  The first tile shows that when the points come in no
     // particular order; where they follow each other in space (every tile another ray, or the next stretch of a space-filling
     // curve) each tile brings slots of its own, the table of columns fills up, and every contribution that then finds no
     // column probes in vain and leaves one record.  The second tile's slots tell the two apart: how many of its contributions
     // go to slots the first tile did not touch?  (Asked only of a level that is a candidate for columns: the look at the
     // second tile costs a simplex search.)
-    __syncthreads();
-    const bool few_slots = cache_pays<D>(c, 0) && c.lines <= (1u << (kColumnMaxIdsLog2 - 1));  // the table of columns starts at most half full
+    const bool few_slots = first_hits * 8u >= wanted && distinct <= (1u << (kColumnMaxIdsLog2 - 1));  // the table of columns starts at most half full
     if (few_slots && tiles_per_group > 1) {
         const uvec<D + 1> next_slot = slots_of_next_tile();
         uint32_t strangers = 0;
         static_for<D + 1>(PENC_BODY(r) {
             PENC_INDEX(r);
-            strangers += __popcll(__ballot(next_active && !cache_holds(c, next_slot[r])));
+            const uint32_t bit = seen_bit<State>(next_slot[r]);
+            strangers += __popcll(__ballot(next_active && ((seen[bit >> 5] >> (bit & 31u)) & 1u) == 0u));
         });
         if ((threadIdx.x & 63) == 0 && strangers != 0u) atomicAdd(&c.strangers, strangers);
         __syncthreads();
@@ -1117,17 +1108,37 @@ __device__ __forceinline__ int scatter_mode_decide(State& c, const BinTarget& bi
     const bool can_stream = bins.records != nullptr && bins.n_bins <= static_cast<uint32_t>(kMaxBins);
     // The slots the group will have touched in the end: the first tile's, and from every later tile as many new ones as the
     // second tile brought, counted twice (a slot at the rim of what a tile covers gets fewer contributions than one inside).
-    const uint32_t expected_slots =
-        c.lines + (2u * c.lines * c.strangers * static_cast<uint32_t>(tiles_per_group - 1)) / (c.wanted != 0u ? c.wanted : 1u);
-    if (can_stream && !cache_pays<D>(c, 0, 4u)) {
+    const uint32_t expected_slots = distinct + (2u * distinct * c.strangers * static_cast<uint32_t>(tiles_per_group - 1)) / (wanted != 0u ? wanted : 1u);
+    if (can_stream && first_hits * 4u < wanted) {
         mode = kModeStream;
         for (int e = threadIdx.x; e < kMaxBins; e += State::kThreads) c.tag[e] = 0;  // stream_tile and stream_tile_many count there
-        __syncthreads();
-    } else if (few_slots && expected_slots <= (3u << (kColumnMaxIdsLog2 - 2))) {  // the largest table may end up three quarters full
-        mode = kModeColumns;
-        id_bits = kColumnMinIdsLog2;
-        while ((1u << (id_bits - 1)) < expected_slots && id_bits < static_cast<uint32_t>(kColumnMaxIdsLog2)) ++id_bits;
-        for (int e = threadIdx.x; e < kCacheLines; e += State::kThreads) c.tag[e] = -1;  // now entries, without columns
+    } else {
+        if (few_slots && expected_slots <= (3u << (kColumnMaxIdsLog2 - 2))) {  // the largest table may end up three quarters full
+            mode = kModeColumns;
+            id_bits = kColumnMinIdsLog2;
+            while ((1u << (id_bits - 1)) < expected_slots && id_bits < static_cast<uint32_t>(kColumnMaxIdsLog2)) ++id_bits;
+        }
+        // lines without a slot, or entries without columns; no sums yet
+        const uint32_t kNone = 0xFFFFFFFFu;
+        static_assert(kCacheLines % (2 * State::kThreads) == 0, "whole entries to a thread");
+#pragma unroll
+        for (int e = 0; e < kCacheLines / 2; e += State::kThreads) reinterpret_cast<uint2*>(c.tag)[e + threadIdx.x] = make_uint2(kNone, kNone);
+#pragma unroll
+        for (int e = 0; e < kCacheLines; e += State::kThreads) reinterpret_cast<uint4*>(c.val)[e + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
+        if (threadIdx.x == 0) {
+            c.wanted = wanted;
+            c.first_hits = first_hits;
+        }
+    }
+    __syncthreads();
+    if (mode == kModeCache) {
+        // The tile's slots claim their lines before any later tile's do: the slots that come often are among them, and every contribution of a slot
+        // that finds no line is a record.  (Waves that claimed as they came: reducers of two such levels, D = 8, 22 -> 29 and 34 -> 46 us.)
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r);
+            bool found = false;
+            if (active) cache_find<cache_probes(D)>(c, slot[r], found);
+        });
         __syncthreads();
     }
     return mode;

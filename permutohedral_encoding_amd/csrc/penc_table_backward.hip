@@ -102,7 +102,6 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
         if (threadIdx.x == 0) state.deferred = 0u;
     }
-    scatter_begin(state);
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     if constexpr (kBins == kBinsFew || kBins == kBinsMany) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
@@ -153,6 +152,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s0 = group_second0[nn];
         s1 = group_second1[nn];
     }
+    scatter_begin(state);  // (while the first tile is on its way)
     int mode = kModeCache;
     uint32_t id_bits = 0, cursor = 0;
     for (int t = 0; t < tiles_per_group; ++t) {
@@ -185,7 +185,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                 return cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
             };
             const bool next_active = tile_base + kThreads + threadIdx.x < n_points && tiles_per_group > 1;
-            mode = scatter_mode_decide<D>(state, bins, active, s.slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
+            const uint32_t points = last_in_group < static_cast<uint32_t>(kThreads) ? last_in_group + 1u : kThreads;
+            mode = scatter_mode_decide<D>(state, bins, active, points, s.slot, id_bits, next_active, slots_of_next_tile, tiles_per_group);
         }
         // b_r * w_level (:405), or dB[r] * w_level (:1244-1245)
         fvec<D + 1> w = (kOrder == kSecondOrder ? s.dB : s.w) * w_level;
