@@ -84,9 +84,11 @@ int penc_scale_factors(int pos_dim, int nr_levels, const float* sigmas, float* s
  * atomicAdd per value, EncodingGPU.cuh:409-410). */
 size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity,
                                     int levels_per_pass);
-/* What the scatter of a dense gradient can use on top of penc_scatter_workspace_bytes() for all levels: for a gradient of 64 MiB and more of a table of
- * more than 2^19 slots and more than a few workgroups, lists that let the scatter clear the gradient while it works (12 * (pos_dim + 1) bytes per point and level, room for
- * everything, of which a few MB are written: 1.3 GB for 2^20 points, 24 levels, pos_dim 3; csrc/penc_scatter.hpp); for small tables and few levels, the slack of more and narrower bins (a few percent); else 0. */
+/* What the scatter of a dense gradient can use on top of penc_scatter_workspace_bytes() for all levels, so that the gradient need not be cleared
+ * before: lists of 12 * (pos_dim + 1) bytes per point and level with room for everything, of which a few MB are written at most (1.3 GB for 2^20 points, 24 levels,
+ * pos_dim 3).  With them the reducers of a table of up to 64 slot ranges write its gradient whole, where each has a range to itself, and the scatter of a gradient of 64 MiB and
+ * more, of a table of more than 2^19 slots and more than a few workgroups, clears it while it works (csrc/penc_scatter.hpp).  For small tables and few
+ * levels also the slack of more and narrower bins (a few percent).  Else 0. */
 size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity);
 
 /* Size of `workspace` that lets penc_backward compute positions_grad in groups of a few levels

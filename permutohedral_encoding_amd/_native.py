@@ -193,8 +193,8 @@ def scale_factors(pos_dim, sigmas):
 # levels, pos_dim 3): MAX_WORKSPACE_BYTES caps the request, and a request the allocator cannot serve
 # is retried with fewer levels per pass and finally without a workspace; the library computes the
 # same sums either way (more passes over the levels, or direct atomics).
-# The native path asks for more where it makes a call faster, under the same cap: for dense gradients of large tables (more than 2^19 slots,
-# 64 MiB) the lists of penc_scatter_extra_bytes, 1.2 GiB beside those 1.4; for forwards of 16 M points times levels and more, a copy of a table of up to
+# The native path asks for more where it makes a call faster, under the same cap: for dense gradients the lists of
+# penc_scatter_extra_bytes, 1.2 GiB beside those 1.4; for forwards of 16 M points times levels and more, a copy of a table of up to
 # 2 MiB a level; for a 16-bit table laid out in cells, up to 128 MiB.  A cap below such a sum means the call without it.
 LEVELS_PER_PASS = 0
 MAX_WORKSPACE_BYTES = None

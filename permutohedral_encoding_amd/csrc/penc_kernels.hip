@@ -1073,17 +1073,20 @@ constexpr int64_t kClearApartMaxWork = 16000000;
 inline size_t deferred_bytes(int pos_dim, int pair_levels, uint32_t n_groups, int tiles_per_group) {
     return static_cast<size_t>(pair_levels) * n_groups * (deferred_room(pos_dim, tiles_per_group) * sizeof(BinRecord) + sizeof(uint32_t)) + 512;
 }
-// Gives the plan of a dense gradient such lists where its scatter has the instance that clears, takes all levels in one launch, and the workspace has room
-// for them.
-inline bool plan_deferred(BinPlan& p, int pos_dim, int64_t nr_positions, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
-                          size_t bytes) {
-    if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity, static_cast<int64_t>(p.target.n_groups) * pair_levels) || p.levels_per_pass < pair_levels) return false;
-    if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0) return false;
+inline bool place_lists(BinPlan& p, int pos_dim, int pair_levels, int tiles_per_group, const void* workspace, size_t bytes) {
     const uintptr_t base = (p.end + 255u) & ~uintptr_t{255};
     if (base + deferred_bytes(pos_dim, pair_levels, p.target.n_groups, tiles_per_group) > reinterpret_cast<uintptr_t>(workspace) + bytes) return false;
     p.clear.room = deferred_room(pos_dim, tiles_per_group);
     p.clear.kept = reinterpret_cast<BinRecord*>(base);
     p.clear.counts = reinterpret_cast<uint32_t*>(base + static_cast<size_t>(pair_levels) * p.target.n_groups * p.clear.room * sizeof(BinRecord));
+    return true;
+}
+// Gives the plan of a dense gradient such lists where its scatter has the instance that clears, takes all levels in one launch, and the workspace has room
+// for them.
+inline bool plan_deferred(BinPlan& p, int pos_dim, int64_t nr_positions, int pair_levels, int capacity, int tiles_per_group, const float* table_grad, const void* workspace,
+                          size_t bytes) {
+    if (!p.enabled || !clears_in_scatter(p.target.n_bins, pair_levels, capacity, static_cast<int64_t>(p.target.n_groups) * pair_levels) || p.levels_per_pass < pair_levels) return false;
+    if ((reinterpret_cast<uintptr_t>(table_grad) & 15u) != 0 || !place_lists(p, pos_dim, pair_levels, tiles_per_group, workspace, bytes)) return false;
     p.clear.pairs = static_cast<uint64_t>(pair_levels) * capacity;
     p.clear.flags = static_cast<uint32_t>(p.direct_bytes / sizeof(uint32_t));
     const uint32_t threads = p.target.n_bins > kFewerOpenLinesMinBins ? kScatterBlockManyBins : kScatterBlock;
@@ -1170,18 +1173,31 @@ inline GroupSortPlan plan_group_sort(int pos_dim, int64_t n, int levels, int fea
 constexpr unsigned kFineBinsShared = 256, kFineBinsSharedCrowded = 448;
 constexpr unsigned kMaxReduceSplits = 16;
 
-inline int reduce_bins(const BinPlan& p, int64_t lookups, const float* window, int first_level, int n_levels_in_pass, int capacity,
-                       uint32_t feat_pairs, float* table_grad, hipStream_t st) {
-    // enough workgroups for every compute unit, by letting several share a bin when bins*levels is small
-    const unsigned pairs = p.target.n_bins * static_cast<unsigned>(n_levels_in_pass);
+// How many workgroups share a bin: enough for every compute unit.
+inline unsigned reduce_splits(uint32_t n_bins, uint32_t bin_shift, uint32_t n_groups, int64_t lookups, int n_levels_in_pass) {
+    const unsigned pairs = n_bins * static_cast<unsigned>(n_levels_in_pass);
     unsigned enough = kReduceWorkgroupsWanted;
-    if (p.target.bin_shift < static_cast<uint32_t>(kBinSlotsLog2)) {
-        const bool crowded = p.target.bin_shift <= 11u && lookups >= static_cast<int64_t>(p.target.n_bins) << (p.target.bin_shift + 3);
+    if (bin_shift < static_cast<uint32_t>(kBinSlotsLog2)) {
+        const bool crowded = bin_shift <= 11u && lookups >= static_cast<int64_t>(n_bins) << (bin_shift + 3);
         enough = (crowded ? kFineBinsSharedCrowded : kFineBinsShared) + 1;
     }
     unsigned splits = pairs >= enough ? 1u : (kReduceWorkgroupsWanted + pairs - 1) / pairs;
-    if (splits > p.target.n_groups) splits = p.target.n_groups;
-    if (splits > kMaxReduceSplits) splits = kMaxReduceSplits;
+    if (splits > n_groups) splits = n_groups;
+    return splits > kMaxReduceSplits ? kMaxReduceSplits : splits;
+}
+
+// The gradient of a table of few bins is written whole by its reducers (LateTarget) where each has a bin to itself and all levels are one pass.
+inline bool written_whole(uint32_t n_bins, uint32_t bin_shift, uint32_t n_groups, int64_t lookups, int pair_levels) {
+    return n_bins <= static_cast<uint32_t>(kStageBins) && reduce_splits(n_bins, bin_shift, n_groups, lookups, pair_levels) == 1u;
+}
+inline bool plan_late(BinPlan& p, int pos_dim, int64_t lookups, int pair_levels, int tiles_per_group, const void* workspace, size_t bytes) {
+    if (!p.enabled || p.levels_per_pass < pair_levels || !written_whole(p.target.n_bins, p.target.bin_shift, p.target.n_groups, lookups, pair_levels)) return false;
+    return place_lists(p, pos_dim, pair_levels, tiles_per_group, workspace, bytes);
+}
+
+inline int reduce_bins(const BinPlan& p, int64_t lookups, const float* window, int first_level, int n_levels_in_pass, int capacity,
+                       uint32_t feat_pairs, float* table_grad, hipStream_t st) {
+    const unsigned splits = reduce_splits(p.target.n_bins, p.target.bin_shift, p.target.n_groups, lookups, n_levels_in_pass);
     // many bins with a few thousand records each: workgroups that keep their bin and walk several levels
     // (bins wider than kBinSlots are planned only where this kernel can serve them)
     const bool wide = p.target.bin_shift > static_cast<uint32_t>(kBinSlotsLog2);
@@ -1201,10 +1217,11 @@ inline int reduce_bins(const BinPlan& p, int64_t lookups, const float* window, i
         return check_launch();
     }
     const dim3 grid(p.target.n_bins, n_levels_in_pass, splits);
+    const LateTarget late = p.target.n_bins <= static_cast<uint32_t>(kStageBins) ? LateTarget(p.clear) : LateTarget{};
 #define PENC_LAUNCH_REDUCE(SPLIT, SLOTS_LOG2)                                                                                                       \
     case SLOTS_LOG2:                                                                                                                                \
         hipLaunchKernelGGL((bin_reduce_kernel<SPLIT, SLOTS_LOG2>), grid, dim3(reduce_threads(SLOTS_LOG2)), 0, st, p.target, window,                 \
-                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level);                                                  \
+                           static_cast<uint32_t>(capacity), feat_pairs, table_grad, first_level, late);                                            \
         break;
 #define PENC_LAUNCH_REDUCE_ALL(SPLIT)                                                                                                               \
     switch (p.target.bin_shift) {                                                                                                                   \
@@ -1434,6 +1451,8 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         plan.target.bin_shift = bin_shift_for_capacity(capacity);
     } else if (plan_deferred(plan, pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, lattice_values_grad, workspace, workspace_bytes)) {
         // the scattering kernel clears
+    } else if (plan_late(plan, pos_dim, nr_positions * (pos_dim + 1), pair_levels, tiles_per_group, workspace, workspace_bytes)) {
+        // the reducers write all of it
     } else if (int rc = clear_table_grad(lattice_values_grad, pair_levels, capacity, plan.enabled ? plan.target.direct : nullptr,
                                          plan.direct_bytes, st)) {
         return rc;
@@ -1459,7 +1478,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         if (plan.enabled)
             if (int rc = reduce_bins(plan, nr_positions * (pos_dim + 1), anneal_window, first, count, capacity, feat_pairs, lattice_values_grad, st)) return rc;
     }
-    if (plan.clear.kept != nullptr) {
+    if (plan.clear.pairs != 0u) {
         hipLaunchKernelGGL(add_deferred_kernel, dim3(plan.target.n_groups, static_cast<unsigned>(pair_levels)), dim3(kBlock), 0, st, plan.clear, anneal_window,
                            cap, feat_pairs, lattice_values_grad);
         return check_launch();
@@ -1691,27 +1710,24 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
 
 size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
     if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
-    const uint32_t n_bins = bins_for_capacity(capacity), fine_shift = fine_bin_shift(pos_dim, capacity, nr_levels);
-    if (fine_shift != bin_shift_for_capacity(capacity)) {
-        const uint32_t fine = bins_of_shift(capacity, fine_shift);
-        size_t most = 0;
-        for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {
-            const size_t need = bin_bytes_per_level(pos_dim, fine, scatter_groups(nr_positions, tiles), wanted_segment_capacity(pos_dim, fine, tiles)) * nr_levels;
-            most = need > most ? need : most;
-        }
-        const size_t want = most + direct_flag_bytes(nr_levels, fine) + 8192, have = penc_scatter_workspace_bytes(pos_dim, nr_positions, nr_levels, capacity, nr_levels);
-        return want > have ? want - have : 0;
+    const uint32_t n_bins = bins_for_capacity(capacity), shift = bin_shift_for_capacity(capacity), fine_shift = fine_bin_shift(pos_dim, capacity, nr_levels);
+    const int64_t lookups = nr_positions * (pos_dim + 1);
+    const int most_tiles = table_backward_tiles(nr_positions, nr_levels);
+    if (n_bins > static_cast<uint32_t>(kMaxBins) || lookups * kMinSlotsPerContribution <= capacity) return 0;
+    size_t lists = 0, narrow = 0;
+    for (const int tiles : {kScatterTiles, most_tiles}) {
+        const uint32_t groups = scatter_groups(nr_positions, tiles), fine = bins_of_shift(capacity, fine_shift);
+        const size_t need = deferred_bytes(pos_dim, nr_levels, groups, tiles), bins = bin_bytes_per_level(pos_dim, fine, groups, wanted_segment_capacity(pos_dim, fine, tiles)) * nr_levels;
+        if (clears_in_scatter(n_bins, nr_levels, capacity, static_cast<int64_t>(scatter_groups(nr_positions, most_tiles)) * nr_levels) ||
+            written_whole(fine, fine_shift, groups, lookups, nr_levels))
+            lists = need > lists ? need : lists;
+        if (fine_shift != shift) narrow = bins > narrow ? bins : narrow;
     }
-    const int64_t workgroups = static_cast<int64_t>(scatter_groups(nr_positions, table_backward_tiles(nr_positions, nr_levels))) * nr_levels;
-    if (n_bins > static_cast<uint32_t>(kMaxBins) || !clears_in_scatter(n_bins, nr_levels, capacity, workgroups) ||
-        nr_positions * (pos_dim + 1) * kMinSlotsPerContribution <= capacity)
-        return 0;
-    size_t most = 0;
-    for (const int tiles : {kScatterTiles, table_backward_tiles(nr_positions, nr_levels)}) {
-        const size_t need = deferred_bytes(pos_dim, nr_levels, scatter_groups(nr_positions, tiles), tiles);
-        most = need > most ? need : most;
-    }
-    return most + 256;
+    if (lists != 0) lists += 256;
+    if (narrow == 0) return lists;
+    const size_t want = narrow + direct_flag_bytes(nr_levels, bins_of_shift(capacity, fine_shift)) + 8192 + lists;
+    const size_t have = penc_scatter_workspace_bytes(pos_dim, nr_positions, nr_levels, capacity, nr_levels);
+    return want > have ? want - have : 0;
 }
 
 size_t penc_positions_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels) {

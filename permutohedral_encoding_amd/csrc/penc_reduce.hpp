@@ -20,12 +20,13 @@ constexpr int reduce_threads(int slots_log2) { return slots_log2 >= 12 ? kReduce
 template <bool kSplit, int kSlotsLog2>  // whether the records are split (the host knows: BinTarget::slots), and the slots per bin
 __global__ void __launch_bounds__(reduce_threads(kSlotsLog2))
 bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_t capacity, uint32_t feat_pairs,
-                  float* __restrict__ table_grad, int first_level) {
+                  float* __restrict__ table_grad, int first_level, LateTarget late) {
     constexpr int kSlots = 1 << kSlotsLog2, kThreads = reduce_threads(kSlotsLog2);
     // one array per feature: lanes that hit different slots then spread over all bank pairs (interleaved
     // features would leave every other pair idle in each of the two adds)
     __shared__ double acc0[kSlots];
     __shared__ double acc1[kSlots];
+    __shared__ uint32_t wave_late[kThreads / 64];
     const uint32_t bin = blockIdx.x;
     // last level first: with the usual coarse-to-fine level list the bins with the most records are
     // started first and the nearly empty ones fill the tail of the launch
@@ -33,7 +34,33 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // with more than two features per level, every pair of features is scattered and reduced like a level of its own
     const uint32_t pair_level = static_cast<uint32_t>(first_level) + level_in_pass;
     const uint32_t level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
-    if (window[level] == 0.0f) return;  // masked level: its scattering workgroups wrote no counts
+    // With lists of late adds (LateTarget) nobody has cleared the gradient, and nobody else adds to it: the workgroup, alone with its bin,
+    // writes all of the bin's slot range.
+    const bool whole = late.kept != nullptr;
+    const uint32_t slot0 = bin << kSlotsLog2;
+    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
+    // Its sums, two slots to a store where they lie together (16 bytes of 8-byte alignment).
+    const auto write_whole = [&](auto&& sum_of) {
+        typedef float Quad __attribute__((ext_vector_type(4), aligned(8)));
+        if (feat_pairs == 1u) {
+#pragma unroll 2
+            for (uint32_t s = 2 * threadIdx.x; s < static_cast<uint32_t>(kSlots); s += 2 * kThreads) {
+                const float2 a = sum_of(s), b = sum_of(s + 1);
+                float* const to = level_grad.at(slot0 + s);
+                if (slot0 + s + 1 < capacity) *reinterpret_cast<Quad*>(to) = Quad{a.x, a.y, b.x, b.y};
+                else if (slot0 + s < capacity) *reinterpret_cast<float2*>(to) = a;
+            }
+        } else {
+#pragma unroll 4
+            for (uint32_t s = threadIdx.x; s < static_cast<uint32_t>(kSlots); s += kThreads)
+                if (slot0 + s < capacity) *reinterpret_cast<float2*>(level_grad.at(slot0 + s)) = sum_of(s);
+        }
+    };
+    const auto write_zeros = [&]() { write_whole([](uint32_t) { return make_float2(0.0f, 0.0f); }); };
+    if (window[level] == 0.0f) {  // masked level: its scattering workgroups wrote no counts
+        if (whole) write_zeros();
+        return;
+    }
     const BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     constexpr uint32_t kWaves = kThreads / 64;
     constexpr uint32_t kUnroll = 4;  // even
@@ -48,11 +75,22 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // and the barrier that follows the clearing carries the vote.
     bool any = false;
     for (uint32_t g = group_begin + threadIdx.x; g < group_end; g += kThreads) any = any || counts[g] != 0u;
+    const uint32_t* const late_counts = late.counts + static_cast<size_t>(level_in_pass) * bins.n_groups;
+    bool any_late = false;
+    if (whole) {
+        for (uint32_t g = threadIdx.x; g < bins.n_groups; g += kThreads) any_late = any_late || late_counts[g] != 0u;
+        any = any || any_late;
+    }
+    any_late = __any(any_late);
+    if (lane == 0) wave_late[wave] = any_late ? 1u : 0u;
     for (int s = threadIdx.x; s < kSlots; s += kThreads) {
         acc0[s] = 0.0;
         acc1[s] = 0.0;
     }
-    if (!__syncthreads_or(any)) return;
+    if (!__syncthreads_or(any)) {
+        if (whole) write_zeros();
+        return;
+    }
     // segments g = group_begin + wave, + kWaves, ...; their record counts are fetched 64 at a time
     // (one per lane) so that no segment has to wait for its own count.  The records are walked in
     // chunks of kUnroll wave-widths, and the next chunk's loads are issued before the current
@@ -190,13 +228,33 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
             add(b, got_b);
         }
     }
+    if (whole) {
+        bool level_has_late = false;
+#pragma unroll
+        for (uint32_t w = 0; w < kWaves; ++w) level_has_late = level_has_late || wave_late[w] != 0u;
+        if (level_has_late) {  // (rare: segments that ran over)
+            for (uint32_t g = wave; g < bins.n_groups; g += kWaves) {
+                const uint32_t count = late_counts[g];
+                const BinRecord* const kept = late.kept + (static_cast<size_t>(level_in_pass) * bins.n_groups + g) * late.room;
+                for (uint32_t i = lane; i < count; i += 64) {
+                    const BinRecord rec = kept[i];
+                    const uint32_t cell = rec.slot_in_bin - slot0;  // (a late add's slot is that in the level)
+                    if (cell < static_cast<uint32_t>(kSlots)) {
+                        __hip_atomic_fetch_add(&acc0[cell], static_cast<double>(rec.a0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        __hip_atomic_fetch_add(&acc1[cell], static_cast<double>(rec.a1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        write_whole([&](uint32_t s) { return make_float2(static_cast<float>(acc0[s]), static_cast<float>(acc1[s])); });
+        return;
+    }
     // nothing has been added to the bin's slots since the gradient was cleared (or, for a caller who keeps the gradient
     // across calls, since that caller last cleared this slot range): the sums are the result.  Read before the barrier:
     // thread 0 sets the flag at the end.
     const bool untouched_so_far = bins.direct[bin] == 0u;
     __syncthreads();
-    const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
-    const uint32_t slot0 = bin << kSlotsLog2;
     const bool alone = gridDim.z == 1;
     if (alone) {
         // all of a thread's read-modify-writes at once: the loads are issued together, not one per trip

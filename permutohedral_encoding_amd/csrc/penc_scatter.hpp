@@ -135,18 +135,18 @@ struct BinTarget {
 // add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
 //   kept    [level_in_pass][group][room]   {slot in the level, values}; there is room for all a group can leave
 //   counts  [level_in_pass][group]
-struct ClearTarget {
+struct LateTarget {
     BinRecord* kept;
     uint32_t* counts;
+    uint32_t room;
+};
+// (Few bins have nothing cleared at all: their reducers, one to a bin, write all of its slot range, and take what was kept from the lists of their level themselves.
+// Fill, scatter and reduction, us: 24 levels of 2^18 slots, D = 3, 2^20 points 11.4 + 335 + 133 -> 335 + 139, 131007 points along rays 9 + 50 + 14.8 -> 51.5 + 20.3;
+// D = 8, 16 levels of 2^19, 2^19 points 11 + 289 + 131 -> 290 + 132;  D = 2, four features, 16 levels of 2^16, 2^18 points 6.5 + 93 + 26.5 -> 95 + 29.)
+struct ClearTarget : LateTarget {
+    uint32_t rows;    // of workgroups that clear and do nothing else
     uint64_t pairs;   // 8-byte units of the gradient,
     uint32_t flags;   // and its flags
-    uint32_t room;
-    uint32_t rows;    // of workgroups that clear and do nothing else
-};
-// What instances for few bins are given instead.
-struct NoClearTarget {
-    NoClearTarget() = default;
-    explicit NoClearTarget(const ClearTarget&) {}
 };
 // What a group of points can leave for later at a level: all its contributions, and the lines its cache claimed.
 constexpr uint32_t deferred_room(int pos_dim, int tiles_per_group) {
@@ -940,8 +940,8 @@ __device__ __forceinline__ void column_tile(State& c, const GradSlice& level_gra
 }
 
 // Sums every column in use and adds the sums to the gradient (stage 3).  By all threads, between barriers.
-template <typename State>
-__device__ __forceinline__ void column_flush(State& c, const GradSlice& level_grad, uint32_t id_bits) {
+template <bool kManyBins, typename State>
+__device__ __forceinline__ void column_flush(State& c, const GradSlice& level_grad, const BinTarget& bins, uint32_t group, uint32_t id_bits) {
     const uint32_t cell_bits = kCacheLinesLog2 - id_bits, cells = 1u << cell_bits;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (uint32_t id = wave; id < (1u << id_bits); id += State::kThreads / 64) {
@@ -956,9 +956,11 @@ __device__ __forceinline__ void column_flush(State& c, const GradSlice& level_gr
         }
         if (lane == 0) {
             // straight into the gradient: a level in column mode leaves a few dozen sums per workgroup, and
-            // as records they would only make every bin's reducer workgroup run for a handful of them
+            // as records they would only make every bin's reducer workgroup run for a handful of them.  (Where the reducers write everything they run
+            // in any case.)
             if (level_grad.deferred != nullptr) {
-                level_grad.defer(static_cast<uint32_t>(owner), static_cast<float>(s0), static_cast<float>(s1));
+                const float v0 = static_cast<float>(s0), v1 = static_cast<float>(s1);
+                if (kManyBins || !append_record(c, bins, group, static_cast<uint32_t>(owner), v0, v1)) level_grad.defer(static_cast<uint32_t>(owner), v0, v1);
                 continue;
             }
             float* g = level_grad.at(static_cast<uint32_t>(owner));
@@ -1154,7 +1156,7 @@ __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_gra
     if (D <= kWorkgroupSortMaxDim && !kManyBins && mode == kModeStream && threadIdx.x < 64) c.bin_count[threadIdx.x] = cursor;
     __syncthreads();
     if (mode == kModeCache) cache_flush(c, level_grad, bins, group);
-    if (mode == kModeColumns) column_flush(c, level_grad, id_bits);
+    if (mode == kModeColumns) column_flush<kManyBins>(c, level_grad, bins, group, id_bits);
     if (bins.records == nullptr) return;
     __syncthreads();
     for (uint32_t b = threadIdx.x; b < bins.n_bins; b += State::kThreads) {

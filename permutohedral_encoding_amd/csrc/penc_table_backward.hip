@@ -49,7 +49,7 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
 enum BinKind : int { kBinsFew = 0, kBinsNarrow = 1, kBinsMany = 2, kBinsWide = 3 };
 template <int kBins>
-using ClearTargetOf = std::conditional_t<(kBins >= kBinsMany), ClearTarget, NoClearTarget>;
+using ClearTargetOf = std::conditional_t<(kBins >= kBinsMany), ClearTarget, LateTarget>;
 // kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
 // a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
@@ -98,10 +98,8 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     const float w_level = window[level];
     if (w_level == 0.0f) return;
     BinRecord* deferred = nullptr;
-    if constexpr (kManyBins) {
-        if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
-        if (threadIdx.x == 0) state.deferred = 0u;
-    }
+    if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
+    if (threadIdx.x == 0) state.deferred = 0u;
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     if constexpr (kBins == kBinsFew || kBins == kBinsMany) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
@@ -213,9 +211,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s1 = s1_next;
     }
     scatter_end<D, kManyBins>(state, level_grad, bins, group, mode, id_bits, cursor);
-    if constexpr (kManyBins) {
-        if (deferred != nullptr && threadIdx.x == 0) clear.counts[static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group] = state.deferred;
-    }
+    if (deferred != nullptr && threadIdx.x == 0) clear.counts[static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group] = state.deferred;
 }
 
 #define PENC_TABLE_PARAMETERS                                                                                                          \
