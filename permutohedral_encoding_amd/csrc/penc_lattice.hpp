@@ -587,6 +587,14 @@ __device__ __forceinline__ CyclicSimplex<D> cyclic_simplex(fvec<D> pos, fvec<D> 
     }
     o.turned = kExactInverse ? (sum & D) : (sum < 0 ? sum + D1 : sum);
     if constexpr (kFirst) {
+        // A residual that is NaN (its point's coordinates are not finite, or overflow) loses every exchange with a number: the weights get it from here, each
+        // from one of its two deltas.  (Five vector instructions of 240 a point and level at D = 3: training step 713 -> 713 us; 13 at D = 8, 686 -> 691, between cards.)
+        float any_nan = rounded.resid[0];
+        static_for<D>(PENC_BODY(c) {
+            PENC_INDEX(c); any_nan += rounded.resid[c + 1]; });
+        static_for<D1>(PENC_BODY(m) {
+            PENC_INDEX(m);
+            if constexpr ((D - m) % 2 == 0) sorted[m] = __builtin_fmaf(any_nan, 0.0f, sorted[m]); });
         fvec<D1> d, wrap;
         static_for<D1>(PENC_BODY(m) {
             PENC_INDEX(m);

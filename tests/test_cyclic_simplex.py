@@ -52,3 +52,22 @@ def test_points_on_ties_and_faces(d):
     enc, fp = make_encoding(d, np.ones(1, np.float32), shift)
     fp.m_scale_factor = torch.ones((1, d), device="cuda")
     check(enc, pos, sf, shift, 1 << 16)
+
+
+@pytest.mark.parametrize("d", [2, 3, 4, 5, 6, 7, 8])
+def test_weights_of_points_without_a_place(d):
+    """A coordinate that is not finite, or overflows, gives weights that are NaN, as every other pass does, and slots within the table."""
+    rng = np.random.default_rng(d)
+    pos = rng.uniform(-1, 1, (4 * d + 100, d)).astype(np.float32)
+    for i in range(d):
+        pos[4 * i:4 * i + 4, i] = [np.nan, np.inf, -np.inf, 3e38]
+    levels, capacity = 2, 100003
+    shift = np.zeros((levels, d), np.float32)
+    enc, _ = make_encoding(d, np.array([1e-2, 1e-4], np.float32), shift)
+    for routine in (FIRST_ORDER, BOTH_ORDERS):
+        got = enc.simplex_debug(to_gpu(pos), capacity, gather_path=routine)
+        weights, slots = got["barycentric"].cpu().numpy(), got["slot"].cpu().numpy()
+        bad = np.isnan(weights)
+        print(d, routine, weights.shape)
+        assert bad.all(-1)[:, :4 * d].all() and not bad[:, 4 * d:].any()
+        assert slots.min() >= 0 and slots.max() < capacity
