@@ -445,6 +445,35 @@ __device__ __forceinline__ uint32_t seen_bit(uint32_t slot) {
     return (slot * 0x9E3779B1u) >> (32 - __builtin_ctz(static_cast<unsigned>(State::kThreads) * 128u));
 }
 
+// Where the weights of a thread's first point (kSets arrays of D+1) wait while the slots of its second one are found for scatter_mode_decide: in the staging
+// space past the marked bits, and in the tags, neither of which holds anything yet.  A cell is its thread's own.  With both points' values in registers at
+// once the kernels of both orders were held to 128 with up to 24 of them spilled, the next tile's point among them, which every tile then waited for
+// (scatter of both orders from [level][feature][n], 16 levels, 2^18 points, before -> with ranks, as it was -> so, us: D = 8, 2^14 slots 202 -> 188 -> 182,
+// 2^18 195 -> 178 -> 180, 2^20 235 -> 216 -> 212, 2^22 373 -> 302 -> 294;  D = 7, 2^20 231 -> 217 -> 197;  D = 3, 2^20 105 -> 101 -> 102;  first order, D = 4, 2^18 82 -> 83 -> 79).
+// With two dimensions nothing was spilled.
+constexpr int kParkMinDim = 3;
+template <int D, int kSets, typename State>
+struct ParkedWeights {
+    static constexpr int kInStage = 4 * State::kChunk - 4;  // words a thread has there
+    static_assert((kSets * (D + 1) - kInStage) * State::kThreads <= kCacheLines, "they fit");
+    State& c;
+    template <int i>
+    __device__ __forceinline__ float& cell() const {
+        if constexpr (i < kInStage) return reinterpret_cast<float*>(c.val)[(4 + i) * State::kThreads + threadIdx.x];
+        else return reinterpret_cast<float*>(c.tag)[(i - kInStage) * State::kThreads + threadIdx.x];
+    }
+    template <int kSet>
+    __device__ __forceinline__ void put(fvec<D + 1> w) const {
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r); cell<kSet * (D + 1) + r>() = w[r]; });
+    }
+    template <int kSet>
+    __device__ __forceinline__ void take(fvec<D + 1>& w) const {
+        static_for<D + 1>(PENC_BODY(r) {
+            PENC_INDEX(r); w[r] = cell<kSet * (D + 1) + r>(); });
+    }
+};
+
 // Clears what the look at the first tile needs, and the bins' cursors.
 template <typename State>
 __device__ __forceinline__ void scatter_begin(State& c) {

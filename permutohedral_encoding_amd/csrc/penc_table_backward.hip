@@ -178,9 +178,21 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         CyclicSimplex<D> s = cyclic_simplex<D, kOrder != kSecondOrder, kNeedsQ>(pos, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask);
         if (t == 0) {
             // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
-            // (its point is already here)
+            // (its point is already here).  This tile's weights wait in the LDS meanwhile (ParkedWeights).
             const auto slots_of_next_tile = [&]() {
-                return cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
+                const ParkedWeights<D, kBoth ? 2 : 1, ScatterStateT<stage_chunk(D), kThreads>> parked{state};
+                if constexpr (D >= kParkMinDim) {
+                    parked.template put<0>(kOrder == kSecondOrder ? s.dB : s.w);
+                    if constexpr (kBoth) parked.template put<1>(s.dB);
+                    wave_lds_fence();
+                }
+                const uvec<D + 1> next_slot = cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
+                if constexpr (D >= kParkMinDim) {
+                    wave_lds_fence();
+                    parked.template take<0>(kOrder == kSecondOrder ? s.dB : s.w);
+                    if constexpr (kBoth) parked.template take<1>(s.dB);
+                }
+                return next_slot;
             };
             const bool next_active = tile_base + kThreads + threadIdx.x < n_points && tiles_per_group > 1;
             const uint32_t points = last_in_group < static_cast<uint32_t>(kThreads) ? last_in_group + 1u : kThreads;
