@@ -84,12 +84,15 @@ int penc_scale_factors(int pos_dim, int nr_levels, const float* sigmas, float* s
  * atomicAdd per value, EncodingGPU.cuh:409-410). */
 size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity,
                                     int levels_per_pass);
-/* What the scatter of a dense gradient can use on top of penc_scatter_workspace_bytes() for all levels, so that the gradient need not be cleared
- * before: lists of 12 * (pos_dim + 1) bytes per point and level with room for everything, of which a few MB are written at most (1.3 GB for 2^20 points, 24 levels,
- * pos_dim 3).  With them the reducers of a table of up to 64 slot ranges write its gradient whole, where each has a range to itself, and the scatter of a gradient of 64 MiB and
- * more, of a table of more than 2^19 slots and more than a few workgroups, clears it while it works (csrc/penc_scatter.hpp).  For small tables and few
- * levels also the slack of more and narrower bins (a few percent).  Else 0. */
+/* What the scatter of a dense gradient can use at most on top of penc_scatter_workspace_bytes() for all levels, whatever the number of features (nr_levels counts pairs of them),
+ * and what a call of nr_feat_per_level features (nr_levels levels) does use; a workspace that has it is used so, one that has not serves as well, with the steps it would have saved.
+ * Lists of 12 * (pos_dim + 1) bytes per point, level and pair of features (1.3 GB for 2^20 points, 24 levels, pos_dim 3: as much again as the workspace itself), so that the gradient need
+ * not be cleared before: there is room in them for every contribution, and written is what finds no room in the segments, which hold three standard deviations
+ * more than the mean.  With them the reducers of a table of up to 64 slot ranges write its gradient whole, where each has a range of 2^13 slots to itself, there are up to four features
+ * and, with pos_dim 2, up to 2^18 points; and the scatter of a gradient of 64 MiB and more, of a table of more than 2^19 slots and more than a few workgroups, clears it while it
+ * works (csrc/penc_scatter.hpp).  For small tables and few levels instead the slack of more and narrower bins (a few percent).  Else 0. */
 size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity);
+size_t penc_scatter_useful_bytes(int pos_dim, int nr_feat_per_level, int64_t nr_positions, int nr_levels, int capacity);
 
 /* Size of `workspace` that lets penc_backward compute positions_grad in groups of a few levels
  * (partial sums in the workspace, then one deterministic reduction) instead of one thread walking

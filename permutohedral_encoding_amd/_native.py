@@ -34,6 +34,7 @@ _SIGNATURES = {
     "penc_scatter_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int,
                                                        ctypes.c_int]),
     "penc_scatter_extra_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
+    "penc_scatter_useful_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
     "penc_positions_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int64, ctypes.c_int]),
     "penc_backward": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int,
                                      _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p, _c_f32p,
@@ -194,7 +195,7 @@ def scale_factors(pos_dim, sigmas):
 # is retried with fewer levels per pass and finally without a workspace; the library computes the
 # same sums either way (more passes over the levels, or direct atomics).
 # The native path asks for more where it makes a call faster, under the same cap: for dense gradients the lists of
-# penc_scatter_extra_bytes, 1.2 GiB beside those 1.4; for forwards of 16 M points times levels and more, a copy of a table of up to
+# penc_scatter_useful_bytes, 1.2 GiB beside those 1.4; for forwards of 16 M points times levels and more, a copy of a table of up to
 # 2 MiB a level; for a 16-bit table laid out in cells, up to 128 MiB.  A cap below such a sum means the call without it.
 LEVELS_PER_PASS = 0
 MAX_WORKSPACE_BYTES = None
@@ -210,7 +211,7 @@ def scatter_workspace(pos_dim, nr_positions, nr_levels, capacity, device, table_
     """Scratch memory for one gradient call (None when the library would not use any).
 
     The scatter counts every pair of features as a level (``nr_levels * nr_feat / 2`` of them).
-    (gradient_workspace of csrc/penc_torch.cpp, but for penc_scatter_extra_bytes, which the functions of ``funcs.py`` do without.)
+    (gradient_workspace of csrc/penc_torch.cpp, but for penc_scatter_useful_bytes, which the functions of ``funcs.py`` do without.)
     ``fixed_bytes`` is added to every request (the level-major copy of a row-major upstream gradient);
     ``required_bytes`` is the part of it the call cannot do without."""
     if LEVELS_PER_PASS < 0 and not required_bytes:

@@ -1186,12 +1186,28 @@ inline unsigned reduce_splits(uint32_t n_bins, uint32_t bin_shift, uint32_t n_gr
     return splits > kMaxReduceSplits ? kMaxReduceSplits : splits;
 }
 
-// The gradient of a table of few bins is written whole by its reducers (LateTarget) where each has a bin to itself and all levels are one pass.
-inline bool written_whole(uint32_t n_bins, uint32_t bin_shift, uint32_t n_groups, int64_t lookups, int pair_levels) {
+inline bool few_bins_alone(uint32_t n_bins, uint32_t bin_shift, uint32_t n_groups, int64_t lookups, int pair_levels) {
     return n_bins <= static_cast<uint32_t>(kStageBins) && reduce_splits(n_bins, bin_shift, n_groups, lookups, pair_levels) == 1u;
 }
-inline bool plan_late(BinPlan& p, int pos_dim, int64_t lookups, int pair_levels, int tiles_per_group, const void* workspace, size_t bytes) {
-    if (!p.enabled || p.levels_per_pass < pair_levels || !written_whole(p.target.n_bins, p.target.bin_shift, p.target.n_groups, lookups, pair_levels)) return false;
+// The gradient of a table of few bins is written whole by its reducers (LateTarget) where each has a bin to itself, all levels are one pass and the bins have kBinSlots slots.
+// Fill, scatter and reduction, us: 24 levels of 2^18 slots, D = 3, 2^20 points 8 + 320 + 125 -> 317 + 124, 2^18 points 8 + 89 + 40 -> 89 + 40, 131007 points along rays
+// 9 + 50 + 14.8 -> 51.5 + 20.3;  D = 8, 16 levels of 2^19, 2^19 points 11 + 289 + 131 -> 290 + 132.
+// Narrow bins have little to fill, and short segments, which run over where few slots are hot; what does goes into the gradient one by one while the scatter does other things, but as late
+// adds it waits in the one reducer of the hot bin: D = 8, 16 levels of 2^16 slots down to 1e-2, 2^18 points near a surface 5 + 193 + 39 -> 179 + 115, 12 levels
+// 5 + 146 + 42 -> 147 + 118;  D = 2, 16 levels of 2^16 5 + 57 + 9 -> 64 + 14;  at best 1% of a pass less.
+// More than two pairs of features write every slot in parts, 8 bytes of 64 at a time (forward and table gradient, 16 levels of 2^18 slots, 131072 points along rays, the window on 0.4
+// of them: D = 3, eight features 103 -> 125, four 79 -> 77; all levels 239 -> 246, four 185 -> 178).
+// With two dimensions a level's hashes fill the bins unevenly, and a full one's reducer is what the launch waits for (24 levels of 2^18 slots: 2^20 points 9 + 279 + 80 -> 271 + 144,
+// 2^18 points 8 + 69 + 29 -> 68 + 35;  18 levels, 2^19 points 7 + 100 + 35 -> 98 + 53, 2^17 points 8 + 36 + 16 -> 37 + 19).
+constexpr int64_t kWholeMaxPoints2d = 1 << 18;
+inline bool written_whole(int pos_dim, uint32_t feat_pairs, int64_t nr_positions, uint32_t n_bins, uint32_t bin_shift, uint32_t n_groups, int pair_levels) {
+    return bin_shift == static_cast<uint32_t>(kBinSlotsLog2) && feat_pairs <= 2u && (pos_dim > 2 || nr_positions <= kWholeMaxPoints2d) &&
+           few_bins_alone(n_bins, bin_shift, n_groups, nr_positions * (pos_dim + 1), pair_levels);
+}
+inline bool plan_late(BinPlan& p, int pos_dim, uint32_t feat_pairs, int64_t nr_positions, int pair_levels, int tiles_per_group, const void* workspace, size_t bytes) {
+    if (!p.enabled || p.levels_per_pass < pair_levels ||
+        !written_whole(pos_dim, feat_pairs, nr_positions, p.target.n_bins, p.target.bin_shift, p.target.n_groups, pair_levels))
+        return false;
     return place_lists(p, pos_dim, pair_levels, tiles_per_group, workspace, bytes);
 }
 
@@ -1451,7 +1467,7 @@ static int table_backward(int pos_dim, int nr_feat, int64_t nr_positions, int nr
         plan.target.bin_shift = bin_shift_for_capacity(capacity);
     } else if (plan_deferred(plan, pos_dim, nr_positions, pair_levels, capacity, tiles_per_group, lattice_values_grad, workspace, workspace_bytes)) {
         // the scattering kernel clears
-    } else if (plan_late(plan, pos_dim, nr_positions * (pos_dim + 1), pair_levels, tiles_per_group, workspace, workspace_bytes)) {
+    } else if (plan_late(plan, pos_dim, feat_pairs, nr_positions, pair_levels, tiles_per_group, workspace, workspace_bytes)) {
         // the reducers write all of it
     } else if (int rc = clear_table_grad(lattice_values_grad, pair_levels, capacity, plan.enabled ? plan.target.direct : nullptr,
                                          plan.direct_bytes, st)) {
@@ -1708,26 +1724,40 @@ size_t penc_scatter_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_le
     return sorted > binned ? sorted : binned;
 }
 
-size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
-    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
-    const uint32_t n_bins = bins_for_capacity(capacity), shift = bin_shift_for_capacity(capacity), fine_shift = fine_bin_shift(pos_dim, capacity, nr_levels);
+// feat_pairs: of the levels that `pair_levels` counts, for what a call of so many pairs has a use for; 0: for whatever number, at most.
+static size_t scatter_extra_bytes(int pos_dim, uint32_t feat_pairs, int64_t nr_positions, int pair_levels, int capacity) {
+    const uint32_t n_bins = bins_for_capacity(capacity), shift = bin_shift_for_capacity(capacity), fine_shift = fine_bin_shift(pos_dim, capacity, pair_levels);
     const int64_t lookups = nr_positions * (pos_dim + 1);
-    const int most_tiles = table_backward_tiles(nr_positions, nr_levels);
+    const int most_tiles = table_backward_tiles(nr_positions, pair_levels);
     if (n_bins > static_cast<uint32_t>(kMaxBins) || lookups * kMinSlotsPerContribution <= capacity) return 0;
     size_t lists = 0, narrow = 0;
     for (const int tiles : {kScatterTiles, most_tiles}) {
         const uint32_t groups = scatter_groups(nr_positions, tiles), fine = bins_of_shift(capacity, fine_shift);
-        const size_t need = deferred_bytes(pos_dim, nr_levels, groups, tiles), bins = bin_bytes_per_level(pos_dim, fine, groups, wanted_segment_capacity(pos_dim, fine, tiles)) * nr_levels;
-        if (clears_in_scatter(n_bins, nr_levels, capacity, static_cast<int64_t>(scatter_groups(nr_positions, most_tiles)) * nr_levels) ||
-            written_whole(fine, fine_shift, groups, lookups, nr_levels))
+        const size_t need = deferred_bytes(pos_dim, pair_levels, groups, tiles), bins = bin_bytes_per_level(pos_dim, fine, groups, wanted_segment_capacity(pos_dim, fine, tiles)) * pair_levels;
+        if (clears_in_scatter(n_bins, pair_levels, capacity, static_cast<int64_t>(scatter_groups(nr_positions, most_tiles)) * pair_levels) ||
+            (feat_pairs != 0u ? written_whole(pos_dim, feat_pairs, nr_positions, fine, fine_shift, groups, pair_levels)
+                              : few_bins_alone(fine, fine_shift, groups, lookups, pair_levels)))
             lists = need > lists ? need : lists;
         if (fine_shift != shift) narrow = bins > narrow ? bins : narrow;
     }
     if (lists != 0) lists += 256;
     if (narrow == 0) return lists;
-    const size_t want = narrow + direct_flag_bytes(nr_levels, bins_of_shift(capacity, fine_shift)) + 8192 + lists;
-    const size_t have = penc_scatter_workspace_bytes(pos_dim, nr_positions, nr_levels, capacity, nr_levels);
+    const size_t want = narrow + direct_flag_bytes(pair_levels, bins_of_shift(capacity, fine_shift)) + 8192 + lists;
+    const size_t have = penc_scatter_workspace_bytes(pos_dim, nr_positions, pair_levels, capacity, pair_levels);
     return want > have ? want - have : 0;
+}
+
+size_t penc_scatter_extra_bytes(int pos_dim, int64_t nr_positions, int nr_levels, int capacity) {
+    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
+    return scatter_extra_bytes(pos_dim, 0u, nr_positions, nr_levels, capacity);
+}
+
+size_t penc_scatter_useful_bytes(int pos_dim, int nr_feat_per_level, int64_t nr_positions, int nr_levels, int capacity) {
+    if (pos_dim < 2 || pos_dim > 8 || nr_positions <= 0 || nr_levels <= 0 || capacity <= 0) return 0;
+    if (nr_feat_per_level != 2 && nr_feat_per_level != 4 && nr_feat_per_level != 8) return 0;
+    const int feat_pairs = nr_feat_per_level / 2;
+    if (group_sort_serves(pos_dim, nr_positions, nr_levels, feat_pairs, capacity, false)) return 0;
+    return scatter_extra_bytes(pos_dim, static_cast<uint32_t>(feat_pairs), nr_positions, nr_levels * feat_pairs, capacity);
 }
 
 size_t penc_positions_workspace_bytes(int pos_dim, int64_t nr_positions, int nr_levels) {

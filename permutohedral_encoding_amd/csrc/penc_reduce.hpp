@@ -36,7 +36,7 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     const uint32_t level = pair_level / feat_pairs, pair = pair_level % feat_pairs;
     // With lists of late adds (LateTarget) nobody has cleared the gradient, and nobody else adds to it: the workgroup, alone with its bin,
     // writes all of the bin's slot range.
-    const bool whole = late.kept != nullptr;
+    const bool whole = kSlotsLog2 == kBinSlotsLog2 && late.kept != nullptr;
     const uint32_t slot0 = bin << kSlotsLog2;
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair) * 2, 2 * feat_pairs, nullptr, 0u, nullptr, nullptr};
     // Its sums, two slots to a store where they lie together (16 bytes of 8-byte alignment).

@@ -119,7 +119,23 @@ struct BinTarget {
     uint32_t segment_capacity;
     uint32_t bin_shift;  // log2 of the slots per bin: kBinSlotsLog2, more only with more than kStageBins bins (whole records), less for small tables
 };
-// Large tables (more than kStageBins bins, all levels in one launch; kept == nullptr: not): the scattering kernel clears the gradient and the flags
+// Where nothing may be added to a gradient that has not been cleared or written yet, what would go straight into it is kept:
+//   kept    [level_in_pass][group][room]   {slot in the level, values}; there is room for all a group can leave
+//   counts  [level_in_pass][group]
+// kept == nullptr: nothing is.  Few bins of kBinSlots slots (written_whole) have no gradient cleared before: their reducers, one to a bin, write all of its slot range,
+// and take what was kept from the lists of their level themselves.
+struct LateTarget {
+    BinRecord* kept;
+    uint32_t* counts;
+    uint32_t room;
+};
+// What the instances for narrow bins, which are never written whole, are given instead (for the look whether there are lists, and what follows from it, the scatter of 16
+// levels of 2^14 slots, 2^18 points, took up to 3% longer: D = 2 53.6 -> 51.9 us, D = 3 62.1 -> 60.6, D = 5 118 -> 113).
+struct NoLateTarget {
+    NoLateTarget() = default;
+    explicit NoLateTarget(const LateTarget&) {}
+};
+// Large tables (more than kStageBins bins, all levels in one launch): the scattering kernel clears the gradient and the flags
 // itself, because those writes pass while it waits for other things.  The first `rows` rows of its grid, a workgroup to a die, do nothing else; rows == 0: every
 // workgroup clears a share when it starts.  So many rows that they write at about half of the memory's rate: with more the loads of
 // the others wait behind them, and where a share each is cleared by little more than one round of workgroups at once, fill and scatter might as
@@ -132,17 +148,7 @@ struct BinTarget {
 // (4, 6, 8 and 12 rows of 512 threads for 95077 points 190 / 175 / 167 / 174; 3, 4, 6, 8 of 1024 for 500003 686 / 666 / 683 / 678.)  With many points the two are
 // as good on average and apart by point order (kClearApartMaxWork).  Nothing may
 // be added to a gradient that another workgroup is still to clear, so what would go straight into it is kept until the reducers have ended, and
-// add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over):
-//   kept    [level_in_pass][group][room]   {slot in the level, values}; there is room for all a group can leave
-//   counts  [level_in_pass][group]
-struct LateTarget {
-    BinRecord* kept;
-    uint32_t* counts;
-    uint32_t room;
-};
-// (Few bins have nothing cleared at all: their reducers, one to a bin, write all of its slot range, and take what was kept from the lists of their level themselves.
-// Fill, scatter and reduction, us: 24 levels of 2^18 slots, D = 3, 2^20 points 11.4 + 335 + 133 -> 335 + 139, 131007 points along rays 9 + 50 + 14.8 -> 51.5 + 20.3;
-// D = 8, 16 levels of 2^19, 2^19 points 11 + 289 + 131 -> 290 + 132;  D = 2, four features, 16 levels of 2^16, 2^18 points 6.5 + 93 + 26.5 -> 95 + 29.)
+// add_deferred_kernel adds it (5 to 7 us, up to 22 with more segments that have run over).
 struct ClearTarget : LateTarget {
     uint32_t rows;    // of workgroups that clear and do nothing else
     uint64_t pairs;   // 8-byte units of the gradient,
@@ -450,8 +456,6 @@ __device__ __forceinline__ uint32_t seen_bit(uint32_t slot) {
 // once the kernels of both orders were held to 128 with up to 24 of them spilled, the next tile's point among them, which every tile then waited for
 // (scatter of both orders from [level][feature][n], 16 levels, 2^18 points, before -> with ranks, as it was -> so, us: D = 8, 2^14 slots 202 -> 188 -> 182,
 // 2^18 195 -> 178 -> 180, 2^20 235 -> 216 -> 212, 2^22 373 -> 302 -> 294;  D = 7, 2^20 231 -> 217 -> 197;  D = 3, 2^20 105 -> 101 -> 102;  first order, D = 4, 2^18 82 -> 83 -> 79).
-// With two dimensions nothing was spilled.
-constexpr int kParkMinDim = 3;
 template <int D, int kSets, typename State>
 struct ParkedWeights {
     static constexpr int kInStage = 4 * State::kChunk - 4;  // words a thread has there

@@ -49,12 +49,14 @@ constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_
 // need up to eight more vector registers (at D = 4, held to 80 registers, 27 spilled instead of 5).
 enum BinKind : int { kBinsFew = 0, kBinsNarrow = 1, kBinsMany = 2, kBinsWide = 3 };
 template <int kBins>
-using ClearTargetOf = std::conditional_t<(kBins >= kBinsMany), ClearTarget, LateTarget>;
+using ClearTargetOf = std::conditional_t<(kBins >= kBinsMany), ClearTarget, std::conditional_t<kBins == kBinsFew, LateTarget, NoLateTarget>>;
 // kOrder: kFirstOrder, kSecondOrder (above), or kBothOrders: the table gradient of a loss on the encoded values and of
 // a loss on the position gradient of the same points in one pass (`second_grad`, always [level][feature][n], is the upstream
 // gradient of the latter).  Both are sums over the same simplices, so they share the search, the records and the
 // reducer; apart, the second pass and the dense sum of the two gradients were a third of an SDF training step.
 enum TableOrder : int { kFirstOrder = 1, kSecondOrder = 2, kBothOrders = 3 };
+// From which dimension on the weights are parked (ParkedWeights): below, nothing is spilled without.
+constexpr int park_min_dim(int order) { return order == kBothOrders ? 3 : (order == kFirstOrder ? 4 : 5); }
 template <int D, bool kRowMajor, int kOrder, int kBins, int kThreads>
 __device__ __forceinline__ void
 scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, uint32_t feat_pairs, uint32_t dies, int tiles_per_group,
@@ -98,8 +100,10 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
     const float w_level = window[level];
     if (w_level == 0.0f) return;
     BinRecord* deferred = nullptr;
-    if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
-    if (threadIdx.x == 0) state.deferred = 0u;
+    if constexpr (kBins != kBinsNarrow) {
+        if (clear.kept != nullptr) deferred = clear.kept + (static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group) * clear.room;
+        if (threadIdx.x == 0) state.deferred = 0u;
+    }
     BinTarget bins = bins_of_level(pass_bins, level_in_pass);
     if constexpr (kBins == kBinsFew || kBins == kBinsMany) bins.bin_shift = kBinSlotsLog2;  // a constant from here on
     const GradSlice level_grad{table_grad + (static_cast<size_t>(level) * capacity * feat_pairs + pair_level % feat_pairs) * 2,
@@ -179,15 +183,16 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         if (t == 0) {
             // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
             // (its point is already here).  This tile's weights wait in the LDS meanwhile (ParkedWeights).
+            constexpr bool kPark = D >= park_min_dim(kOrder);
             const auto slots_of_next_tile = [&]() {
                 const ParkedWeights<D, kBoth ? 2 : 1, ScatterStateT<stage_chunk(D), kThreads>> parked{state};
-                if constexpr (D >= kParkMinDim) {
+                if constexpr (kPark) {
                     parked.template put<0>(kOrder == kSecondOrder ? s.dB : s.w);
                     if constexpr (kBoth) parked.template put<1>(s.dB);
                     wave_lds_fence();
                 }
                 const uvec<D + 1> next_slot = cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
-                if constexpr (D >= kParkMinDim) {
+                if constexpr (kPark) {
                     wave_lds_fence();
                     parked.template take<0>(kOrder == kSecondOrder ? s.dB : s.w);
                     if constexpr (kBoth) parked.template take<1>(s.dB);
@@ -223,7 +228,9 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
         s1 = s1_next;
     }
     scatter_end<D, kManyBins>(state, level_grad, bins, group, mode, id_bits, cursor);
-    if (deferred != nullptr && threadIdx.x == 0) clear.counts[static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group] = state.deferred;
+    if constexpr (kBins != kBinsNarrow) {
+        if (deferred != nullptr && threadIdx.x == 0) clear.counts[static_cast<size_t>(level_in_pass) * pass_bins.n_groups + group] = state.deferred;
+    }
 }
 
 #define PENC_TABLE_PARAMETERS                                                                                                          \

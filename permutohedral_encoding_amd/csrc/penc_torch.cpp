@@ -67,7 +67,7 @@ struct Api {
     PENC_FN(forward_rowmajor);
     PENC_FN(forward_rowmajor_workspace_bytes);
     PENC_FN(scatter_workspace_bytes);
-    PENC_FN(scatter_extra_bytes);
+    PENC_FN(scatter_useful_bytes);
     PENC_FN(positions_workspace_bytes);
     PENC_FN(backward);
     PENC_FN(backward_half);
@@ -242,9 +242,9 @@ Tensor gradient_workspace(const Call& c, bool table, bool positions, int64_t cop
     const int64_t pair_levels = static_cast<int64_t>(c.levels) * (c.feat / 2);
     int64_t per_pass = c.levels_per_pass <= 0 ? pair_levels : std::min(c.levels_per_pass, pair_levels);
     if (!table || c.levels_per_pass < 0) per_pass = 0;
-    // (asked for once, with all levels in a pass: what a dense gradient can use besides)
+    // (asked for once, with all levels in a pass: what a dense gradient uses besides, lists of late adds or the slack of narrower bins)
     int64_t extra = per_pass == pair_levels && c.sparse_owner == nullptr
-                        ? static_cast<int64_t>(api.scatter_extra_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels), c.capacity))
+                        ? static_cast<int64_t>(api.scatter_useful_bytes(c.pos_dim, c.feat, c.n, c.levels, c.capacity))
                         : 0;
     while (true) {
         int64_t want = per_pass > 0 ? static_cast<int64_t>(api.scatter_workspace_bytes(c.pos_dim, c.n, static_cast<int>(pair_levels),
@@ -1320,7 +1320,7 @@ PyObject* py_bind(PyObject*, PyObject* path) {
         PENC_FN(forward_rowmajor);
         PENC_FN(forward_rowmajor_workspace_bytes);
         PENC_FN(scatter_workspace_bytes);
-        PENC_FN(scatter_extra_bytes);
+        PENC_FN(scatter_useful_bytes);
         PENC_FN(positions_workspace_bytes);
         PENC_FN(backward);
         PENC_FN(backward_half);
