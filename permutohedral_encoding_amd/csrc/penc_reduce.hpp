@@ -26,7 +26,7 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // features would leave every other pair idle in each of the two adds)
     __shared__ double acc0[kSlots];
     __shared__ double acc1[kSlots];
-    __shared__ uint32_t wave_late[kThreads / 64];
+    __shared__ uint32_t wave_ran_over[kThreads / 64];
     const uint32_t bin = blockIdx.x;
     // last level first: with the usual coarse-to-fine level list the bins with the most records are
     // started first and the nearly empty ones fill the tail of the launch
@@ -75,14 +75,11 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     // and the barrier that follows the clearing carries the vote.
     bool any = false;
     for (uint32_t g = group_begin + threadIdx.x; g < group_end; g += kThreads) any = any || counts[g] != 0u;
-    const uint32_t* const late_counts = late.counts + static_cast<size_t>(level_in_pass) * bins.n_groups;
-    bool any_late = false;
-    if (whole) {
-        for (uint32_t g = threadIdx.x; g < bins.n_groups; g += kThreads) any_late = any_late || late_counts[g] != 0u;
-        any = any || any_late;
-    }
-    any_late = __any(any_late);
-    if (lane == 0) wave_late[wave] = any_late ? 1u : 0u;
+    bool ran_over = false;
+    if (whole)
+        for (uint32_t g = threadIdx.x; g < bins.n_groups; g += kThreads) ran_over = ran_over || counts[g] > bins.segment_capacity;
+    ran_over = __any(ran_over);
+    if (lane == 0) wave_ran_over[wave] = ran_over ? 1u : 0u;
     for (int s = threadIdx.x; s < kSlots; s += kThreads) {
         acc0[s] = 0.0;
         acc1[s] = 0.0;
@@ -102,7 +99,8 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     constexpr uint32_t kShortLanes = 16, kShortUnroll = 8, kShortMax = kShortLanes * kShortUnroll;
     for (uint32_t g0 = group_begin + wave; g0 < group_end; g0 += kWaves * 64) {
         const uint32_t mine = g0 + lane * kWaves;
-        const uint32_t my_count = mine < group_end ? counts[mine] : 0u;
+        const uint32_t wanted = mine < group_end ? counts[mine] : 0u;
+        const uint32_t my_count = wanted < bins.segment_capacity ? wanted : bins.segment_capacity;
         const uint32_t n_segments = (group_end - g0 + kWaves - 1) / kWaves < 64u ? (group_end - g0 + kWaves - 1) / kWaves : 64u;
         if (__ballot(my_count > kShortMax) == 0ull) {
             const uint32_t quarter = lane / kShortLanes, l = lane % kShortLanes;
@@ -229,19 +227,34 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
         }
     }
     if (whole) {
-        bool level_has_late = false;
+        // Late adds: of this bin where its segment was to have more records than it has room for, in the list of that group, with others.  A full bin's reducer is what
+        // the launch waits for: eight loads on their way at once.  (Every list of the level by every reducer, a load at a time -> so, forward and table gradient, us: D = 3, 24 levels
+        // of 2^18 slots, a third of the points in one simplex, 2^18 points 518 -> 397, 2^20 2011 -> 1493;  D = 8, 16 levels of 2^19, three quarters of 131072 points in a small
+        // box 403 -> 349.  With a fill and direct adds 1389, 5571 and 598.)
+        bool any_ran_over = false;
 #pragma unroll
-        for (uint32_t w = 0; w < kWaves; ++w) level_has_late = level_has_late || wave_late[w] != 0u;
-        if (level_has_late) {  // (rare: segments that ran over)
+        for (uint32_t w = 0; w < kWaves; ++w) any_ran_over = any_ran_over || wave_ran_over[w] != 0u;
+        if (any_ran_over) {
+            constexpr uint32_t kAtOnce = 8;
             for (uint32_t g = wave; g < bins.n_groups; g += kWaves) {
-                const uint32_t count = late_counts[g];
-                const BinRecord* const kept = late.kept + (static_cast<size_t>(level_in_pass) * bins.n_groups + g) * late.room;
-                for (uint32_t i = lane; i < count; i += 64) {
-                    const BinRecord rec = kept[i];
-                    const uint32_t cell = rec.slot_in_bin - slot0;  // (a late add's slot is that in the level)
-                    if (cell < static_cast<uint32_t>(kSlots)) {
-                        __hip_atomic_fetch_add(&acc0[cell], static_cast<double>(rec.a0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        __hip_atomic_fetch_add(&acc1[cell], static_cast<double>(rec.a1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (counts[g] <= bins.segment_capacity) continue;
+                const size_t list = static_cast<size_t>(level_in_pass) * bins.n_groups + g;
+                const BinRecord* const kept = late.kept + list * late.room;
+                const uint32_t count = late.counts[list];
+                for (uint32_t base = 0; base < count; base += 64 * kAtOnce) {
+                    BinRecord rec[kAtOnce];
+#pragma unroll
+                    for (uint32_t u = 0; u < kAtOnce; ++u) {
+                        const uint32_t i = base + u * 64 + lane;
+                        rec[u] = kept[i < count ? i : 0u];
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < kAtOnce; ++u) {
+                        const uint32_t cell = rec[u].slot_in_bin - slot0;  // (a late add's slot is that in the level)
+                        if (base + u * 64 + lane < count && cell < static_cast<uint32_t>(kSlots)) {
+                            __hip_atomic_fetch_add(&acc0[cell], static_cast<double>(rec[u].a0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                            __hip_atomic_fetch_add(&acc1[cell], static_cast<double>(rec[u].a1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
                     }
                 }
             }

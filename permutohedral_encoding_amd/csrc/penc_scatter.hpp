@@ -100,7 +100,7 @@ constexpr size_t kSplitRecordBytes = sizeof(RecordValues) + sizeof(uint16_t);
 // bin, so appending needs no global atomics and no synchronisation: the cursor is an LDS counter.
 //   records [level_in_pass][bin][group][segment_capacity]   12-byte records, or the 8-byte values of split ones
 //   slots   [level_in_pass][bin][group][segment_capacity]   the 2-byte slots of split records; nullptr otherwise
-//   counts  [level_in_pass][bin][group]            records actually written (<= segment_capacity)
+//   counts  [level_in_pass][bin][group]            records actually written (<= segment_capacity); with late adds of few bins (LateTarget) those there were to be
 //   direct  [level_in_pass][bin]                   nonzero once anything has been added into the gradient in the
 //                                                  bin's slot range: straight from the scattering kernel (see
 //                                                  GradSlice), or by the bin's reducer.  Cleared with the gradient, or,
@@ -1200,7 +1200,9 @@ __device__ __forceinline__ void scatter_end(State& c, const GradSlice& level_gra
     __syncthreads();
     for (uint32_t b = threadIdx.x; b < bins.n_bins; b += State::kThreads) {
         const uint32_t n = c.bin_count[b];
-        bins.counts[static_cast<size_t>(b) * bins.n_groups + group] = n < bins.segment_capacity ? n : bins.segment_capacity;
+        // (a reducer that takes late adds too looks for them where a segment was to have more records than it has room for)
+        const bool as_wanted = !kManyBins && level_grad.deferred != nullptr;
+        bins.counts[static_cast<size_t>(b) * bins.n_groups + group] = as_wanted || n < bins.segment_capacity ? n : bins.segment_capacity;
     }
 }
 
