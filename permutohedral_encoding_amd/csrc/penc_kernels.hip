@@ -1194,9 +1194,9 @@ inline bool few_bins_alone(uint32_t n_bins, uint32_t bin_shift, uint32_t n_group
 // 9 + 50 + 14.8 -> 51.5 + 20.3;  D = 8, 16 levels of 2^19, 2^19 points 11 + 289 + 131 -> 290 + 132.
 // Narrow bins have little to fill, and short segments, which run over where few slots are hot; what does goes into the gradient one by one while the scatter does other things, but as late
 // adds it waits in the one reducer of the hot bin: D = 8, 16 levels of 2^16 slots down to 1e-2, 2^18 points near a surface 5 + 193 + 39 -> 179 + 115, 12 levels
-// 5 + 146 + 42 -> 147 + 118;  D = 2, 16 levels of 2^16 5 + 57 + 9 -> 64 + 14;  at best 1% of a pass less.
+// 5 + 146 + 42 -> 147 + 118;  D = 2, 16 levels of 2^16 5 + 57 + 9 -> 64 + 14;  otherwise a pass is up to 4% shorter written whole, 0.6% on average over 330 geometries.
 // More than two pairs of features write every slot in parts, 8 bytes of 64 at a time (forward and table gradient, 16 levels of 2^18 slots, 131072 points along rays, the window on 0.4
-// of them: D = 3, eight features 103 -> 125, four 79 -> 77; all levels 239 -> 246, four 185 -> 178).
+// of them: D = 3, eight features 103 -> 125, four 77 -> 77; all levels 239 -> 246, four 133 -> 128).
 // With two dimensions a level's hashes fill the bins unevenly, and a full one's reducer is what the launch waits for (24 levels of 2^18 slots: 2^20 points 9 + 279 + 80 -> 271 + 144,
 // 2^18 points 8 + 69 + 29 -> 68 + 35;  18 levels, 2^19 points 7 + 100 + 35 -> 98 + 53, 2^17 points 8 + 36 + 16 -> 37 + 19).
 constexpr int64_t kWholeMaxPoints2d = 1 << 18;

@@ -58,7 +58,17 @@ bin_reduce_kernel(BinTarget pass_bins, const float* __restrict__ window, uint32_
     };
     const auto write_zeros = [&]() { write_whole([](uint32_t) { return make_float2(0.0f, 0.0f); }); };
     if (window[level] == 0.0f) {  // masked level: its scattering workgroups wrote no counts
-        if (whole) write_zeros();
+        if (whole && feat_pairs == 2u) {
+            // half of the bin's slots to each of the level's two pairs of features, whole slots of 16 bytes (forward and table gradient, D = 3, 16 levels of 2^18 slots, the window
+            // on 0.4 of them, us: 131072 points along rays 79.0 -> 77.1, 2^18 points 99.6 -> 97.3;  with a fill 76.9 and 97.5)
+            typedef float Quad __attribute__((ext_vector_type(4), aligned(8)));
+            const uint32_t half0 = slot0 + pair * (kSlots / 2);
+            float* const to = table_grad + (static_cast<size_t>(level) * capacity + half0) * 4;
+            for (uint32_t s = threadIdx.x; s < static_cast<uint32_t>(kSlots / 2); s += kThreads)
+                if (half0 + s < capacity) *reinterpret_cast<Quad*>(to + 4 * s) = Quad{0.0f, 0.0f, 0.0f, 0.0f};
+        } else if (whole) {
+            write_zeros();
+        }
         return;
     }
     const BinTarget bins = bins_of_level(pass_bins, level_in_pass);
