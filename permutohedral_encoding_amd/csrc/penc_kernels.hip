@@ -651,7 +651,7 @@ touched_ranges_kernel(float* __restrict__ params, float* __restrict__ grads, flo
 
 // kRoutine selects which of the equivalent device routines produces the slots and weights: the
 // compare-and-select chains (vertex_hashes / barycentric: position backward, sorted groups), the thread-private LDS column
-// (sort_by_rank_lds: forward, grad-of-grad), or the sorting network (cyclic_simplex: the scatter, of the first order or of both).
+// (sort_by_rank_lds: forward, grad-of-grad), or what the scatter takes (scatter_simplex: a sorting network, of the first order or of both).
 enum SimplexRoutine : int { kBySelects = 0, kByLds = 1, kByNetwork = 2, kByNetworkBothOrders = 3 };
 template <int D, int kRoutine>
 __global__ void __launch_bounds__(kBlock)
@@ -667,7 +667,7 @@ simplex_debug_kernel(int n_points, uint32_t capacity, uint32_t cap_mask, const f
     fvec<D + 1> w;
     if constexpr (kRoutine >= kByNetwork) {
         const fvec<D> point = load_point<D>(positions, n);
-        const CyclicSimplex<D> c = cyclic_simplex<D, true, kRoutine == kByNetworkBothOrders>(point, point, random_shift + level * D,
+        const CyclicSimplex<D> c = scatter_simplex<D, true, kRoutine == kByNetworkBothOrders>(point, point, random_shift + level * D,
                                                                                              scale_factor + level * D, capacity, cap_mask);
         h = turn_back<D + 1>(c.slot, c.turned);
         w = turn_back<D + 1>(c.w, c.turned);

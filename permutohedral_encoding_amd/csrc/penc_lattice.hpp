@@ -618,6 +618,33 @@ __device__ __forceinline__ CyclicSimplex<D> cyclic_simplex(fvec<D> pos, fvec<D> 
     return o;
 }
 
+// A point's simplex as a scatter takes it.  With two dimensions by ranks, in the order of the remainder vertices: three residuals are ranked as fast as they are sorted,
+// and a coarse level, whose few slots a vertex of one remainder meets in turn, is summed faster in that order, in columns and in the accumulate cache, whose
+// lines the slots of one remainder claim without getting in each other's way.  (Forward and table gradient, 2^18 points, mean of 12 geometries, network -> ranks, us: 16 levels of 2^16 slots
+// down to 1e-2 90.5 -> 88.0, 18 levels 95.6 -> 93.8, of 29429 slots, four features, a window on 0.4 of them, 88.8 -> 87.3;  2^18 slots 90.7 -> 90.1, along rays, 2^16, 101.1 -> 102.8;
+// 2^22 slots, 2^19 points 503.0 -> 506.9.)
+template <int D, bool kFirst, bool kSecond>
+__device__ __forceinline__ CyclicSimplex<D> scatter_simplex(fvec<D> pos, fvec<D> q, const float* __restrict__ shift, const float* __restrict__ sf,
+                                                            uint32_t capacity, uint32_t cap_mask) {
+    if constexpr (D > 2) {
+        return cyclic_simplex<D, kFirst, kSecond>(pos, q, shift, sf, capacity, cap_mask);
+    } else {
+        CyclicSimplex<D> o;
+        const Located<D> s = locate<D>(pos, shift, sf);
+        const uvec<D + 1> h = vertex_hashes<D>(s.rank, s.hash0);
+        if (cap_mask != 0u) {  // (to_slot, asked once)
+            o.slot = h & cap_mask;
+        } else {
+            static_for<D + 1>(PENC_BODY(k) {
+                PENC_INDEX(k); o.slot[k] = h[k] % capacity; });
+        }
+        if constexpr (kFirst) o.w = barycentric<D>(s.rank, s.delta);
+        if constexpr (kSecond) o.dB = pos_grad_grad_to_bary<D>(s.rank, q, sf);
+        o.turned = 0;
+        return o;
+    }
+}
+
 // in[k] of a CyclicSimplex in the order of the remainder vertices.
 template <int N, typename V>
 __device__ __forceinline__ V turn_back(V in, int turned) {

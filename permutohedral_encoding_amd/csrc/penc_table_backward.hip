@@ -179,7 +179,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                 out[n_points] = g1;
             }
         }
-        CyclicSimplex<D> s = cyclic_simplex<D, kOrder != kSecondOrder, kNeedsQ>(pos, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask);
+        CyclicSimplex<D> s = scatter_simplex<D, kOrder != kSecondOrder, kNeedsQ>(pos, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask);
         if (t == 0) {
             // the next tile's slots, should the decision want to know whether its points use the slots this tile uses
             // (its point is already here).  This tile's weights wait in the LDS meanwhile (ParkedWeights).
@@ -191,7 +191,7 @@ scatter_group_of_points(int n_points, int first_level, uint32_t n_pass_levels, u
                     if constexpr (kBoth) parked.template put<1>(s.dB);
                     wave_lds_fence();
                 }
-                const uvec<D + 1> next_slot = cyclic_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
+                const uvec<D + 1> next_slot = scatter_simplex<D, false, false>(pos_next, q, random_shift + level * D, scale_factor + level * D, capacity, cap_mask).slot;
                 if constexpr (kPark) {
                     wave_lds_fence();
                     parked.template take<0>(kOrder == kSecondOrder ? s.dB : s.w);
