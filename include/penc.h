@@ -393,7 +393,7 @@ int penc_transpose(const float* src, float* dst, int64_t rows, int cols, void* s
  * There is one routine for rem0 and rank, and several equivalent ones for slots and weights;
  * gather_path picks which is reported: 0 = the compare-and-select chains of the position-gradient
  * and group-sorting kernels, 1 = the rank sort through LDS of the forward and grad-of-grad kernels,
- * 2 and 3 = the sorting network of the scatter, first order and both (reference: EncodingGPU.cuh:130-223). With 2,
+ * 2 and 3 = what the scatter takes, first order and both: a sorting network, the select chains with pos_dim 2 (reference: EncodingGPU.cuh:130-223). With 2,
  * where D+1 is a power of two, equal residuals may leave a vertex whose weight is 0 open: its slot may be that of either. */
 int penc_simplex_debug(int pos_dim, int64_t nr_positions, int nr_levels, int capacity,
                        const float* positions, const float* scale_factor, const float* random_shift,

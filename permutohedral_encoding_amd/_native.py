@@ -751,7 +751,8 @@ class EncodingWrapper:
 
         ``gather_path`` picks the device routine whose slots and weights are reported: False for the
         select chains of the position-gradient and group-sorting kernels, True for the LDS rank sort of
-        the forward and grad-of-grad kernels, 2 and 3 for the sorting network of the scatter (first order, both)."""
+        the forward and grad-of-grad kernels, 2 and 3 for what the scatter takes (first order, both): a sorting network from
+        three dimensions on."""
         fp = self.fixed_params
         _check_f32_gpu(positions, "positions", 2)
         pos = positions.contiguous()

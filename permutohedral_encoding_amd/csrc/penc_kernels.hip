@@ -876,7 +876,7 @@ struct BinPlan {
     bool enabled = false;
     int levels_per_pass = 0;
     BinTarget target{};       // of the first pass; target.direct covers all levels, a pass starts at its first level's flags
-    ClearTarget clear{};      // (plan_deferred)
+    ClearTarget clear{};      // (plan_deferred, plan_late)
     size_t direct_bytes = 0;  // size of target.direct (to be cleared with the gradient)
     uintptr_t end = 0;        // of what is used of the workspace
 };
@@ -902,7 +902,7 @@ constexpr uint32_t bins_of_shift(int capacity, uint32_t shift) {
 // Bins per level; more than kMaxBins means the table is too large for binning.
 constexpr uint32_t bins_for_capacity(int capacity) { return bins_of_shift(capacity, bin_shift_for_capacity(capacity)); }
 
-// The width of the bins of a dense gradient whose workspace has room for the slack of more segments (penc_scatter_extra_bytes): where there are fewer
+// The width of the bins of a dense gradient whose workspace has room for the slack of more segments (penc_scatter_useful_bytes): where there are fewer
 // (bin, level) pairs than reducers wanted, so that several would share a bin and add into the gradient with atomics (60 ns each), bins of half the width
 // and less, down to 2^10 slots, until there are kFineBinsWanted pairs, each reduced by one workgroup of a part of a compute unit's LDS (a few where
 // there are fewer pairs all the same, kFineBinsShared).  Scatter and
@@ -914,7 +914,7 @@ constexpr uint32_t bins_for_capacity(int capacity) { return bins_of_shift(capaci
 // With four dimensions the accumulate cache leaves some slots of the coarse levels out, whose records several reducers of a bin share
 // better than one (16 levels, 2^18 points: 2^16 slots 130 -> 137, 2^17 126 -> 132; 2^15 131 -> 122).
 // A table that is one bin has room there for everything a group leaves; of narrower ones one can run over, where points that hardly share slots
-// crowd a range of them, and what finds no room is added to the gradient in fp32 one by one, as it is for any table of several bins, instead of in
+// crowd a range of them, and what finds no room is added to the gradient in fp32 one by one, as it is for any table of several bins that is not written whole, instead of in
 // the reducer's sums in fp64.
 constexpr uint32_t kReduceWorkgroupsWanted = 512;  // two per compute unit
 constexpr uint32_t kFineBinsWanted = 768, kFineBinsMostPairs4d = 128;
@@ -1055,7 +1055,7 @@ inline BinPlan plan_bins(int pos_dim, int64_t n, int levels, int capacity, uint3
 //   D = 3, 2^22 slots  2^20 points 1081 -> 1012, near a surface with 16 levels live 600 -> 530;  2^23 slots, 2^19 points 1039 -> 984
 //          2^20        2^20 points from rows 652 -> 650;  16 levels 424 -> 425
 //   D = 2, 16 levels of 2^20, 2^18 points 133 -> 121;  D = 4, 16 levels of 2^20, 2^18 points 186 -> 173;  D = 8, of 2^22, 2^17 points 465 -> 360
-// A smaller gradient takes no longer to fill than the lists take to be added, and the instances for few bins stay without the code.  With workgroups of 512
+// A smaller gradient takes no longer to fill than the lists take to be added (few bins: written_whole).  With workgroups of 512
 // threads, not for less than one round of them, which the clearing ones put off (D = 8, 2^20 slots: 480 workgroups 80 -> 85, 89 -> 93, 111 -> 121;  588
 // of them 95 -> 89, 600 120 -> 107).
 constexpr size_t kClearInScatterBytes = size_t{64} << 20;

@@ -432,10 +432,12 @@ __device__ __forceinline__ fvec<D + 1> pos_grad_grad_to_bary(ivec<D + 1> rank, f
 // leave open has the weight 0 exactly, and a residual of a half is as good on either side: neither is looked after (kOpenTies).
 // Against ranks, selects and trips through the LDS: the scatter of 2^20 points, 24 levels of 2^18 slots, D = 3 issues 94 M vector instructions instead of 120 M
 // (2^19 points, 16 levels of 2^19 slots, D = 8: 100 M of 113 M, and 18 KB of LDS less); it is bound by them at the coarse levels only, so a training step with it
-// goes 726 -> 722 us (D = 8: 715 -> 701; the gradient of both orders, 2^22 slots, 1239 -> 1230).
+// goes 726 -> 722 us (D = 8: 715 -> 701; the gradient of both orders, 2^22 slots, 1239 -> 1230).  The values of the second order ride along, a comparison and two selects an
+// exchange: kept in LDS columns and fetched by the coordinate a key names after the sort they took as many registers, and the scatters of both orders, D = 6 to 8, 0.5% less time.
 template <int N> using dvec = double __attribute__((ext_vector_type(N)));
 
-// Compare-exchanges (place of the larger, place of the smaller) that sort N keys.
+// Compare-exchanges (place of the larger, place of the smaller) that sort N keys: networks of the fewest, as B. Dobbelaere's published list of the smallest known ones has them
+// (up to eight keys optimal by Knuth, The Art of Computer Programming 3, 5.3.4; the 25 for nine by Floyd), each checked below.
 struct SortingNetwork {
     int count;
     int a[25], b[25];
@@ -474,8 +476,8 @@ static_assert(sorts_everything<3>() && sorts_everything<4>() && sorts_everything
                   sorts_everything<8>() && sorts_everything<9>(),
               "every network sorts");
 
-// v_max_f64 and v_min_f64 as they are: the builtins would first quiet operands that might be signalling NaNs.  No key is one: it would take an fp32 NaN with a
-// payload of its own (the hardware's has none); such a point's slots are as meaningless as any NaN's, and within the table.
+// v_max_f64 and v_min_f64 as they are: the builtins would first quiet operands that might be signalling NaNs.  A key is a NaN only where its residual is one with
+// payload bits of its own (the hardware's has none but the first); such a point's slots are as meaningless as any NaN's, and within the table.
 __device__ __forceinline__ double larger_key(double a, double b) {
     double r;
     asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
@@ -587,8 +589,9 @@ __device__ __forceinline__ CyclicSimplex<D> cyclic_simplex(fvec<D> pos, fvec<D> 
     }
     o.turned = kExactInverse ? (sum & D) : (sum < 0 ? sum + D1 : sum);
     if constexpr (kFirst) {
-        // A residual that is NaN (its point's coordinates are not finite, or overflow) loses every exchange with a number: the weights get it from here, each
-        // from one of its two deltas.  (Five vector instructions of 240 a point and level at D = 3: training step 713 -> 713 us; 13 at D = 8, 686 -> 691, between cards.)
+        // A residual that is NaN (its point's coordinates are not finite, or overflow) is a key like any other where its bits are an ordinary double's upper word, as 0x7FC00000 is
+        // (2.2e307): it ends up first or last, by its sign, and in the two weights beside that end.  With its upper payload bits set (0x7FF00000 and more) it is a NaN as a key
+        // too, and vanishes from the network, which then holds another key twice.  So all weights get it from here, each from one of its two deltas.  (Five vector instructions of 240 a point and level at D = 3: training step 713 -> 713 us; 13 at D = 8, 686 -> 691, between cards.)
         float any_nan = rounded.resid[0];
         static_for<D>(PENC_BODY(c) {
             PENC_INDEX(c); any_nan += rounded.resid[c + 1]; });

@@ -108,7 +108,8 @@ constexpr size_t kSplitRecordBytes = sizeof(RecordValues) + sizeof(uint16_t);
 //                                                  entry points), the caller's map of touched slot ranges.
 // `records` == nullptr disables binning (`direct`, `n_bins` and `bin_shift` may still be set: flags without bins).
 // (Every kernel of a small batch begins with a fetch of its arguments, a cache line at a time: with the fields of ClearTarget in here too, a third
-// line for the same code, bin_reduce_kernel took 14.4 us where it takes 14.1, and the table gradient of 131007 points along rays 0.6 us longer in all.)
+// line for the same code, bin_reduce_kernel took 14.4 us where it took 14.1, and the table gradient of 131007 points along rays 0.6 us longer in all.  The lists of late adds
+// are given to the kernels that read them, bin_reduce_kernel among them, as an argument of their own.)
 struct BinTarget {
     void* records;
     uint16_t* slots;
@@ -250,7 +251,7 @@ struct GradSlice {
     uint32_t slot_floats;
     uint32_t* direct;
     uint32_t bin_shift;  // of the bins `direct` belongs to
-    BinRecord* deferred;       // nullptr: adds go into the gradient; else the workgroup's list of them (see ClearTarget),
+    BinRecord* deferred;       // nullptr: adds go into the gradient; else the workgroup's list of them (see LateTarget),
     uint32_t* deferred_count;  // in LDS: how many are in it
     __device__ __forceinline__ float* at(uint32_t slot) const { return base + static_cast<size_t>(slot) * slot_floats; }
     // A plain store on purpose: many workgroups may set the same flag at once, all to 1, and nobody reads it before the
@@ -1057,7 +1058,7 @@ __device__ __forceinline__ uint32_t scatter_tile(State& c, const GradSlice& leve
 }
 
 // The workgroup-wide decision whether stage 1 is worth its LDS traffic at this level: keep using the
-// cache only while at least one contribution in `one_in` hits.  The evidence before tile `tile` is
+// cache only while at least one contribution in eight hits.  The evidence before tile `tile` is
 // the look at the first tile's slots and the hits of the tiles processed since.  Against appending every miss to its
 // bin on its own, one hit in eight pays; against sorting the tile's records by bin (stream_tile),
 // which is cheaper than the cache's look-ups, it takes one in four.

@@ -22,6 +22,8 @@ namespace penc {
 // unit: held to 128, 1.334 -> 1.113 ms.  At D = 5 two workgroups whose staging space takes all six vertices of a point are better than three
 // that sort a tile in two chunks (16 levels of 2^18 slots, 2^19 points, scatter and reduction 323 -> 314 us, second order 327 -> 315).
 // Workgroups of 1024 threads, the wide bins' among them, are alone on their compute unit: four.
+// (The register counts are of the search by ranks.  With the sorting network the first order takes 80 at D = 4 and none is spilled, 125 at D = 8; of both orders a few
+// addresses are spilled, before the first tile, at D = 3 and from D = 6 on: ParkedWeights.)
 constexpr int scatter_waves_per_simd(int pos_dim, int threads) { return pos_dim <= 4 && threads == kScatterBlock ? 6 : 4; }
 
 constexpr int both_orders_waves_per_simd(int pos_dim, int threads) { return pos_dim <= 3 && threads == kScatterBlock ? 6 : 4; }
